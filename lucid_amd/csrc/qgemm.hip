@@ -433,6 +433,67 @@ int launch_tile_cfg(const GemmArgs& g, int conv, int groups, int tile_config, hi
     return launch_tile_shape(g, conv, groups, cfg, schedule, st);
 }
 
+// ---------------------------------------------------------------- rows of any length and alignment
+// The small-batch kernels walk K in 16-byte chunks.  Global loads on gfx950 take any byte address, so
+// a row needs no alignment; what a K that is not a multiple of 16 needs is its last chunk, which must
+// not run past the row (the last row ends where the allocation may).  That chunk is the row's LAST 16
+// bytes instead, for both operands, with the activation bytes that the chunk before already covered
+// set to zero.  (With K % 16 == 0 the chunk is an ordinary one and no byte is dropped.)  K >= 16.
+__device__ __forceinline__ v4i load16(const int8_t* p) {
+    v4i v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+__device__ __forceinline__ int chunk_at(int k, int K) { return k + 16 <= K ? k : K - 16; }
+__device__ __forceinline__ v4i act16(const int8_t* row, int k, int K) {
+    v4i v = load16(row + chunk_at(k, K));
+    const int drop = k + 16 - K;  // bytes of the previous chunk at the front of a last chunk
+    if ((K & 15) != 0 && drop > 0) {  // (the first test is uniform)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int b = drop - 4 * i;
+            v[i] &= b <= 0 ? -1 : (b >= 4 ? 0 : int(0xffffffffu << (8 * b)));
+        }
+    }
+    return v;
+}
+
+// The tile kernels' global-to-LDS loads do need aligned rows: for more than 64 activation rows both
+// operands are copied to rows of `ld` bytes (a multiple of 64: every shape is open to the problem), zeros
+// past K.  A thread moves 16 bytes.  The copy moves 2 (M + N) K bytes beside 2 M N K operations and is bound by
+// memory: at 333 x 1001 x 1000 it is 3.9 us and the product 7 us, where the one-output-per-lane kernel took
+// 1340 us (2000 x 4000 x 4090: 147 ms -> 0.06 ms for the two).
+__global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t* __restrict__ a, int M,
+                                                       const int8_t* __restrict__ w, int N, int K, int ld,
+                                                       int8_t* __restrict__ pa, int8_t* __restrict__ pw) {
+    const unsigned per_row = unsigned(ld) >> 4;
+    const size_t total = size_t(M + N) * per_row;
+    for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < total; i += size_t(gridDim.x) * 256) {
+        const unsigned row = unsigned(i / per_row), c = unsigned(i - size_t(row) * per_row);
+        const bool is_a = row < unsigned(M);
+        const size_t r = is_a ? row : row - unsigned(M);
+        const int8_t* src = (is_a ? a : w) + r * size_t(K);
+        const int k = int(c) * 16, left = K - k;
+        v4i v{0, 0, 0, 0};
+        if (left >= 16) {
+            v = load16(src + k);
+        } else if (left > 0) {
+            // the row's last 16 bytes, shifted down by the bytes that belong to the chunk before
+            const v4i t = load16(src + K - 16);
+            const int sh = 16 - left;
+            const uint64_t lo = uint32_t(t[0]) | uint64_t(uint32_t(t[1])) << 32;
+            const uint64_t hi = uint32_t(t[2]) | uint64_t(uint32_t(t[3])) << 32;
+            uint64_t o0, o1;
+            if (sh >= 8)
+                o0 = hi >> (8 * (sh - 8)), o1 = 0;
+            else
+                o0 = lo >> (8 * sh) | hi << (64 - 8 * sh), o1 = hi >> (8 * sh);
+            v = v4i{int(uint32_t(o0)), int(uint32_t(o0 >> 32)), int(uint32_t(o1)), int(uint32_t(o1 >> 32))};
+        }
+        *reinterpret_cast<v4i*>((is_a ? pa : pw) + r * size_t(ld) + k) = v;
+    }
+}
+
 // ---------------------------------------------------------------- skinny kernel
 // M <= 16*MT.  A block owns 16 weight rows; its 4 wavefronts each take a
 // quarter of K.  In load c of a 256-byte K block, lane (n = lane&15, g = lane>>4) reads
@@ -470,8 +531,7 @@ __global__ __launch_bounds__(256) void qgemm_skinny_kernel(GemmArgs g) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const int k = kbase + c * 64;
-                wf[u][c] = (kbc + u < kb1 && k < g.K) ? *reinterpret_cast<const v4i*>(wrow + k)
-                                                     : v4i{0, 0, 0, 0};
+                wf[u][c] = (kbc + u < kb1 && k < g.K) ? load16(wrow + chunk_at(k, g.K)) : v4i{0, 0, 0, 0};
             }
         }
 #pragma unroll
@@ -485,8 +545,7 @@ __global__ __launch_bounds__(256) void qgemm_skinny_kernel(GemmArgs g) {
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     const int k = kbase + c * 64;
-                    v4i af = (k < g.K && m < g.M) ? *reinterpret_cast<const v4i*>(arow + k)
-                                                  : v4i{0, 0, 0, 0};
+                    v4i af = (k < g.K && m < g.M) ? act16(arow, k, g.K) : v4i{0, 0, 0, 0};
                     acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, wf[u][c], acc[t], 0, 0, 0);
                 }
             }
@@ -546,7 +605,7 @@ __global__ __launch_bounds__(512) void qgemv1_kernel(GemmArgs g) {
     const int kchunks = (g.K + 4095) / 4096;
     // the activation row is requested first: loads return in order
     for (int k = tid * 16; k < kchunks * 4096; k += blockDim.x * 16) {
-        const v4i v = k < g.K ? *reinterpret_cast<const v4i*>(g.a + k) : v4i{0, 0, 0, 0};
+        const v4i v = k < g.K ? act16(g.a, k, g.K) : v4i{0, 0, 0, 0};
         *reinterpret_cast<v4i*>(a_lds + k) = v;
     }
     float S = 1.0f, Z = 0.0f;
@@ -573,7 +632,7 @@ __global__ __launch_bounds__(512) void qgemv1_kernel(GemmArgs g) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int k = kc * 4096 + i * 1024 + lane * 16;
-                wv[r][i] = (n < g.N && k < g.K) ? *reinterpret_cast<const v4i*>(row + k) : v4i{0, 0, 0, 0};
+                wv[r][i] = (n < g.N && k < g.K) ? load16(row + chunk_at(k, g.K)) : v4i{0, 0, 0, 0};
             }
         }
         if (kc == 0) __syncthreads();  // the activation row is in LDS (uniform: every wave runs chunk 0)
@@ -649,7 +708,7 @@ __global__ __launch_bounds__(1024) void qgemm_skinny16_kernel(GemmArgs g, int ro
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int k = kbase + c * 64;
-            af[c] = (m_ok && k < g.K) ? *reinterpret_cast<const v4i*>(arow + k) : v4i{0, 0, 0, 0};
+            af[c] = (m_ok && k < g.K) ? act16(arow, k, g.K) : v4i{0, 0, 0, 0};
         }
 #pragma unroll
         for (int j = 0; j < G; ++j) {
@@ -658,7 +717,7 @@ __global__ __launch_bounds__(1024) void qgemm_skinny16_kernel(GemmArgs g, int ro
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const int k = kbase + c * 64;
-                wf[j][c] = (n < n_end && k < g.K) ? *reinterpret_cast<const v4i*>(wrow + k) : v4i{0, 0, 0, 0};
+                wf[j][c] = (n < n_end && k < g.K) ? load16(wrow + chunk_at(k, g.K)) : v4i{0, 0, 0, 0};
             }
         }
 #pragma unroll
@@ -790,11 +849,31 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
     GemmArgs g = g_in;
     const bool vec_ok = g.K % 16 == 0 && g.K > 0 && aligned16(g.a) && aligned16(g.w);
     int path = force_path;  // 0 = choose, 1 = tile, 2 = skinny, 3 = naive
-    if (path == 0) path = !vec_ok ? 3 : (g.M <= 64 && g.range == nullptr ? 2 : 1);
+    if (path == 0) {
+        // The small-batch kernels stream the weight once whatever its alignment.  More rows than they take,
+        // or a kept range, need the tile kernel: ragged or unaligned operands are copied to padded rows
+        // first (333 x 1001 x 1000: 1340 -> 11 us; 100 x 11008 x 5001: 26.4 ms -> 50 us).  Rows shorter than one chunk stay with the plain kernel.
+        path = g.K < 16 ? 3 : (g.M <= 64 && g.range == nullptr ? 2 : 1);
+        if (path == 1 && !vec_ok) {
+            const int ld = (g.K + 63) / 64 * 64;
+            const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;
+            void* tmp = nullptr;
+            int rc = stream_buffer(4, a_bytes + w_bytes, 0, st, &tmp, nullptr);
+            if (rc) return rc;
+            int8_t* pa = static_cast<int8_t*>(tmp);
+            const size_t chunks = (a_bytes + w_bytes) / 16;
+            const size_t blocks = (chunks + 255) / 256 < 16384 ? (chunks + 255) / 256 : 16384;
+            hipLaunchKernelGGL(pad_rows_kernel, dim3(unsigned(blocks)), dim3(256), 0, st, g.a, g.M, g.w, g.N, g.K, ld,
+                               pa, pa + a_bytes);
+            LQ_CHECK_LAUNCH("pad_rows");
+            g.a = pa, g.w = pa + a_bytes, g.K = ld;
+            return run_tile_kernel(g, 0, 1, tile_config, st);
+        }
+    }
     // only the tile kernel keeps the range of what it writes
     LQ_REQUIRE(g.range == nullptr || path == 1, LQ_ERR_NOT_IMPLEMENTED,
                "qlinear_i8: a kept range needs the tile kernel (K %% 16 == 0, aligned operands)");
-    LQ_REQUIRE(path == 3 || vec_ok, LQ_ERR_VALUE,
+    LQ_REQUIRE(path == 3 || vec_ok || force_path == 0, LQ_ERR_VALUE,
                "qlinear_i8: MFMA paths need K %% 16 == 0 and 16-byte aligned operands");
     if (path == 1) {
         int rc = run_tile_kernel(g, 0, 1, tile_config, st);

@@ -133,6 +133,24 @@ def test_auto_path_matches_forced_paths():
     assert np.array_equal(_ops.qlinear_i8(hip(a), hip(w), out_mode=0).numpy(), O.igemm(a, w))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 17, 17), (1, 1001, 4097), (3, 33, 31), (16, 100, 1025), (11, 257, 2047), (20, 65, 1000),
+                                   (64, 129, 250), (65, 65, 999), (66, 10, 16 * 5 + 15), (333, 77, 1000), (300, 300, 65)])
+@pytest.mark.parametrize("shift", [(0, 0), (1, 7)])
+def test_rows_of_any_length_and_alignment(M, N, K, shift):
+    """K that is not a multiple of 16 and operands at any byte address: the small-batch kernels' last
+    chunk, and the padded copies that feed the tile kernel."""
+    rng = np.random.default_rng(M + 5 * N + K)
+    a, w = codes(rng, (M, K)), codes(rng, (N, K))
+
+    def at(v, off):
+        host = np.zeros(v.size + off, np.int8)
+        host[off:] = v.reshape(-1)
+        return L.Tensor(v.shape, L.int8, "hip", buf=hip(host)._buf, offset=off)
+
+    acc = _ops.qlinear_i8(at(a, shift[0]), at(w, shift[1]), out_mode=_ops.OUT_ACC_I32).numpy()
+    assert np.array_equal(acc, O.igemm(a, w))
+
+
 def _epilogue_case(rng, M, N, K, per_row, bias_kind):
     a, w = codes(rng, (M, K)), codes(rng, (N, K))
     a_scale = rng.uniform(0.005, 0.05, M if per_row else 1).astype(np.float32)
