@@ -187,6 +187,28 @@ int lq_lstm_cell_f32(const float* gates_x, size_t gates_x_ld, const float* gates
                      const float* c_in, int batch, int hidden, float* h_out, float* c_out, float* y,
                      size_t y_ld, lq_stream stream);
 
+/* The recurrence of one LSTM layer with int8 recurrent weights over a whole sequence (one launch per
+ * 16 batch rows that fit the device, all directions together; dynamic/rnn.py:66-84,
+ * CpuBackend.h:13394-13519).  Gate order i, f, g, o:
+ *   raw[t] = gates_x[t] + scale * (h[t-1] . codes) + (bias_ih + bias_hh)
+ *   c[t] = sigmoid(f)*c[t-1] + sigmoid(i)*tanh(g),  h[t] = sigmoid(o)*tanh(c[t])
+ * Direction 1 walks the steps backwards.  Float32 arithmetic throughout: the codes enter exactly,
+ * h as three bfloat16 parts. */
+typedef struct lq_lstm_args {
+    const float* gates_x[2];    /* per direction: x W_ih^T of every step, [4*hidden] per (step, row) in the order of y */
+    const int8_t* w_hh[2];      /* [4*hidden, hidden] codes, symmetric */
+    const float* w_hh_scale[2]; /* [4*hidden] */
+    const float* bias_ih[2];    /* [4*hidden], or NULL together with bias_hh */
+    const float* bias_hh[2];
+    const float* h0;            /* [directions, batch, hidden], or NULL for zeros */
+    const float* c0;
+    float* h_n;                 /* [directions, batch, hidden] */
+    float* c_n;
+    float* y;                   /* [steps, batch, directions*hidden], or [batch, steps, ...] when batch_first */
+    int steps, batch, hidden, directions, batch_first; /* hidden at most 1024 (LQ_ERR_NOT_IMPLEMENTED beyond) */
+} lq_lstm_args;
+int lq_lstm_sequence_f32(const lq_lstm_args* args, lq_stream stream);
+
 /* Self-test of the tile kernels' requantize arithmetic.  Their epilogue computes
  * clamp(rint(x / scale) + zp, qmin, qmax) mostly without dividing (x * (1/scale),
  * accepted when it lies clear of every rounding boundary, the IEEE quotient

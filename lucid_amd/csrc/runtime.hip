@@ -652,7 +652,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 __global__ void fill_bytes_kernel(uint8_t* x, size_t n, uint8_t v) {
     size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     size_t stride = size_t(gridDim.x) * blockDim.x;
-    for (; i < n; i += stride) x[i] = v;
+    // 16-byte stores between the unaligned ends (a byte per lane moves 1/16 of what a store can)
+    const size_t head = (16 - (reinterpret_cast<uintptr_t>(x) & 15)) & 15;
+    if (n < 64 + head) {
+        for (; i < n; i += stride) x[i] = v;
+        return;
+    }
+    const size_t n16 = (n - head) / 16;
+    const unsigned word = v * 0x01010101u;
+    uint4* x16 = reinterpret_cast<uint4*>(x + head);
+    if (i < head) x[i] = v;
+    if (i < n - head - n16 * 16) x[head + n16 * 16 + i] = v;
+    for (; i < n16; i += stride) x16[i] = uint4{word, word, word, word};
 }
 
 __global__ void copy16_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src, size_t n16) {
@@ -736,7 +747,7 @@ int lq_probe_mfma_i8_k64(const int8_t* a, const int8_t* b, size_t nbytes, int it
 int lq_fill_bytes(void* dst, int value, size_t nbytes, lq_stream stream) {
     if (nbytes == 0) return LQ_OK;
     LQ_REQUIRE(dst, LQ_ERR_VALUE, "dst is NULL");
-    hipLaunchKernelGGL(fill_bytes_kernel, dim3(blocks_for(nbytes, 256, 65536)), dim3(256), 0,
+    hipLaunchKernelGGL(fill_bytes_kernel, dim3(blocks_for(nbytes, 256 * 16, 16384)), dim3(256), 0,
                        as_stream(stream), static_cast<uint8_t*>(dst), nbytes, uint8_t(value));
     LQ_CHECK_LAUNCH("fill_bytes");
     return LQ_OK;

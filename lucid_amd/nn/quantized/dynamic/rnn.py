@@ -6,10 +6,14 @@ stored as ``<name>_int8`` codes with a per-row ``<name>_scale`` (symmetric, zero
 b_hh)``).
 
 On the device the input product of a layer is taken once over all time steps
-(float32 MFMA GEMM), then each step is one recurrent GEMM and one gate kernel.
+(float32 MFMA GEMM), then the recurrence of all steps and directions is one launch
+(``lq_lstm_sequence_f32``).  Packed sequences, projections and hidden sizes beyond 1024
+take a recurrent GEMM and a gate kernel per step instead.
 """
 
 from __future__ import annotations
+
+import ctypes as C
 
 import numpy as np
 
@@ -105,6 +109,9 @@ class LSTM(Module):
                                        f"got {h0.shape} and {c0.shape}")
         h_n = Tensor.empty((n_state, Bn, R), T.float32, "hip")
         c_n = Tensor.empty((n_state, Bn, H), T.float32, "hip")
+        # (the one-launch recurrence addresses a step's rows with 32-bit byte offsets)
+        if packed is None and P == 0 and H <= 1024 and Tn > 0 and Bn > 0 and Tn * Bn * dirs * H < 1 << 29:
+            return self._forward_sequences(x, h0, c0, h_n, c_n, Tn, Bn), (h_n, c_n)
         ragged = any(bs != Bn for bs in batch_sizes)
         layer_in = x
         for k in range(self.num_layers):
@@ -172,6 +179,29 @@ class LSTM(Module):
                     return res
                 h_n, c_n = restore(h_n, R), restore(c_n, H)
         return PackedSequence(out, packed.batch_sizes, packed.sorted_indices, packed.unsorted_indices), (h_n, c_n)
+
+    def _forward_sequences(self, x, h0, c0, h_n, c_n, Tn, Bn):
+        """Whole sequences, one launch per layer for the recurrence; fills ``h_n`` / ``c_n``."""
+        H, dirs = self.hidden_size, 2 if self.bidirectional else 1
+        bufs, state = self._buffers, Bn * H * 4
+        for k in range(self.num_layers):
+            y = Tensor.empty((Bn, Tn, dirs * H) if self.batch_first else (Tn, Bn, dirs * H), T.float32, "hip")
+            a = _C.LstmArgs()
+            gates = []
+            for d, suffix in enumerate(("", "_reverse")[:dirs]):
+                name = f"l{k}{suffix}"
+                gates.append(linear_f32(x, self._weight("weight_ih_" + name)))
+                a.gates_x[d] = gates[-1].data_ptr
+                a.w_hh[d], a.w_hh_scale[d] = bufs[f"weight_hh_{name}_int8"].data_ptr, bufs[f"weight_hh_{name}_scale"].data_ptr
+                if self.bias:
+                    a.bias_ih[d], a.bias_hh[d] = bufs["bias_ih_" + name].data_ptr, bufs["bias_hh_" + name].data_ptr
+            at = k * dirs * state
+            a.h0, a.c0 = (None, None) if h0 is None else (h0.data_ptr + at, c0.data_ptr + at)
+            a.h_n, a.c_n, a.y = h_n.data_ptr + at, c_n.data_ptr + at, y.data_ptr
+            a.steps, a.batch, a.hidden, a.directions, a.batch_first = Tn, Bn, H, dirs, int(self.batch_first)
+            _C.call("lq_lstm_sequence_f32", C.byref(a), None)
+            x = y
+        return x
 
     @classmethod
     def from_float(cls, mod, dtype: QDtype = qint8) -> "LSTM":

@@ -290,6 +290,28 @@ def test_dynamic_lstm(layers, bidir, batch_first, bias, with_state):
     assert np.abs(yf - y.numpy()).mean() / (np.abs(yf).mean() + 1e-9) < 0.03
 
 
+@pytest.mark.parametrize("I,H,Bn,Tn,bidir,batch_first",
+                         [(3, 1, 1, 3, False, False), (8, 17, 5, 4, True, True), (16, 33, 16, 2, False, True),
+                          (8, 128, 17, 3, True, False), (7, 129, 33, 2, False, False), (16, 300, 3, 1, True, True),
+                          (16, 512, 20, 3, True, False), (8, 530, 2, 3, True, False), (8, 1024, 17, 2, False, False)])
+def test_dynamic_lstm_sequence_sizes(I, H, Bn, Tn, bidir, batch_first):
+    """The one-launch recurrence at the edges of its tiles: units, batch rows and hidden columns that
+    do not fill a block, a group or an instruction, and every split of the hidden axis.  The bound is
+    the float32 sum of 4 H-wide rows in another order, H + I terms of size up to 1, seven times over
+    (both sums and the gates), at 2^-24 each."""
+    rng = np.random.default_rng(H + Bn)
+    qm = Q.quantize_dynamic(nn.LSTM(I, H, batch_first=batch_first, bidirectional=bidir))
+    x = rng.standard_normal((Bn, Tn, I) if batch_first else (Tn, Bn, I)).astype(np.float32)
+    hx = tuple(rng.standard_normal((2 if bidir else 1, Bn, H)).astype(np.float32) for _ in range(2))
+    xd, hd = hip(x), tuple(hip(v) for v in hx)
+    want = _oracle_lstm_stack(qm, x, hx, batch_first)
+    for _ in range(2):  # the second pass finds the first one's h in its output buffer
+        y, (hn, cn) = qm(xd, hd)
+        for got, ref in zip((y, hn, cn), want):
+            assert np.abs(got.numpy() - ref).max() < 7 * (H + I) ** 0.5 * 2.0 ** -24 * 8
+        del y, hn, cn
+
+
 def _deq(q, name):
     return (getattr(q, name + "_int8").numpy().astype(np.float32) *
             getattr(q, name + "_scale").numpy()[:, None]).astype(np.float32)
