@@ -14,7 +14,7 @@
 // A constant group (max == min) gets s = 1e-7-floored, so its codes are 0 and it
 // decodes to beta exactly.  The decode side takes scales and biases as given (any
 // sign), so weights packed elsewhere under the same contract load unchanged.
-#include "common.hpp"
+#include "wq_pack.hpp"
 
 using namespace lq;
 
@@ -79,88 +79,17 @@ __global__ __launch_bounds__(256) void wq_dequantize_kernel(const uint32_t* __re
     for (int j = 0; j < per_word; ++j) out[first + j] = float((word >> (j * bits)) & mask) * s + b;
 }
 
-// Decode-shaped matmul: y[m, n] = sum_k x[m, k] * (c[n, k] * s[n, g(k)] + b[n, g(k)]), m < MT.
-// A block stages the MT activation rows in LDS once and computes WQ_ROWS output
-// columns with them, four per wavefront; a lane takes 16 bytes of codes (32 int4
-// or 16 int8 codes, never straddling a group) per step, so a wavefront streams
-// 1 KiB of contiguous weight per load.  Per group: acc += s * sum(c*x) + b * sum(x).
-constexpr int WQ_ROWS = 16;
+constexpr int WQ_ROWS = 16;  // output columns per block, four per wavefront
 
-template <int BITS, int MT>
-__global__ __launch_bounds__(256) void wq_gemv_kernel(const float* __restrict__ x, const uint32_t* __restrict__ packed,
-                                                      const float* __restrict__ scales,
-                                                      const float* __restrict__ biases, int M, int N, int K, int gs,
-                                                      int m0, float* __restrict__ out) {
-    // Activation rows in LDS, permuted so that the lanes of a wavefront read
-    // consecutive 16-byte slots: k = CODES*L + 4*j + e is stored at [m][j][L][e]
-    // (lane L of a step reads quad j of its CODES-long chunk).
-    extern __shared__ __attribute__((aligned(16))) float sx[];
-    constexpr int CODES = 128 / BITS;  // codes per 16-byte load
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int rows = M - m0 < MT ? M - m0 : MT;
-    const int chunks = K / CODES;
-    for (int i = tid * 4; i < MT * K; i += 256 * 4) {
-        const int m = i / K, k = i - m * K;
-        float4 v = {0.f, 0.f, 0.f, 0.f};
-        if (m < rows) v = *reinterpret_cast<const float4*>(x + size_t(m0 + m) * K + k);
-        const int L = k / CODES, j = (k % CODES) / 4;
-        *reinterpret_cast<float4*>(sx + m * K + (j * chunks + L) * 4) = v;
-    }
-    __syncthreads();
-    const int words_per_row = K * BITS / 32, groups_per_row = K / gs;
-    for (int r = 0; r < WQ_ROWS / 4; ++r) {
-        const int n = blockIdx.x * WQ_ROWS + wave * (WQ_ROWS / 4) + r;
-        if (n >= N) break;
-        const uint32_t* wrow = packed + size_t(n) * words_per_row;
-        const float* srow = scales + size_t(n) * groups_per_row;
-        const float* brow = biases + size_t(n) * groups_per_row;
-        float acc[MT];
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m] = 0.0f;
-        for (int k = lane * CODES; k < K; k += 64 * CODES) {
-            const uint4 wv = *reinterpret_cast<const uint4*>(wrow + k * BITS / 32);
-            const int g = k / gs;
-            const float s = srow[g], b = brow[g];
-            const uint32_t words[4] = {wv.x, wv.y, wv.z, wv.w};
-            float dot[MT], sum[MT];
-#pragma unroll
-            for (int m = 0; m < MT; ++m) dot[m] = 0.0f, sum[m] = 0.0f;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-#pragma unroll
-                for (int j = 0; j < 32 / BITS; j += 4) {
-                    const int quad = (q * (32 / BITS) + j) / 4;  // quad of this lane's chunk
-                    float c[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        c[e] = float((words[q] >> ((j + e) * BITS)) & ((1u << BITS) - 1u));
-#pragma unroll
-                    for (int m = 0; m < MT; ++m) {
-                        const float4 xv =
-                            *reinterpret_cast<const float4*>(sx + m * K + (quad * chunks + k / CODES) * 4);
-                        dot[m] += c[0] * xv.x + c[1] * xv.y + c[2] * xv.z + c[3] * xv.w;
-                        sum[m] += (xv.x + xv.y) + (xv.z + xv.w);
-                    }
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < MT; ++m) acc[m] += s * dot[m] + b * sum[m];
-        }
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            float v = acc[m];
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
-            if (lane == 0 && m < rows) out[size_t(m0 + m) * N + n] = v;
-        }
-    }
-}
-
-// One activation row (decode): the same scheme with the weight stream software-pipelined.
-// A wavefront owns four weight rows and walks K in steps of 64 * CODES; the 16-byte code
+// One activation row (decode): y[n] = sum_k x[k] * (c[n, k] * s[n, g(k)] + b[n, g(k)]), per group
+// acc += s * sum(c*x) + b * sum(x).  A block stages the row in LDS once; a lane takes 16 bytes of codes
+// (32 int4 or 16 int8 codes, never straddling a group) per step, so a wavefront streams 1 KiB of
+// contiguous weight per load.  The weight stream is software-pipelined:
+// a wavefront owns four weight rows and walks K in steps of 64 * CODES; the 16-byte code
 // loads (and scale / bias) of all four rows for the next step are in flight while the current
 // step is multiplied, and the first step's loads are issued before x is staged, so the only
-// exposed memory latency is the first one.  K % (64 * CODES) == 0.
+// exposed memory latency is the first one.  K need not fill the last step: its lanes past K read
+// the row's last 16 bytes against zeros of x.
 template <int BITS>
 __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uint32_t* packed, const float* scales,
                                                        const float* biases, int N, int K, int gs, float* out) {
@@ -169,7 +98,7 @@ __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uin
     constexpr uint32_t MASK = (1u << BITS) - 1u;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int chunks = K / CODES, steps = chunks / 64;
+    const int last_chunk = K / CODES - 1, steps = last_chunk / 64 + 1, chunks = steps * 64;  // (chunks: those of whole steps)
     const int gs_shift = 31 - __builtin_clz(gs);
     const int words_per_row = K * BITS / 32, groups_per_row = K >> gs_shift;
     const uint4* wrow[RW];
@@ -193,9 +122,11 @@ __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uin
     // about the same whatever it carries.  Layout: sb[wave][array][row][64].
     const bool sb_lds = RW == 4 && groups_per_row <= 64 && groups_per_row % 4 == 0 &&
                         ((reinterpret_cast<uintptr_t>(scales) | reinterpret_cast<uintptr_t>(biases)) & 15u) == 0;
-    float* const sb = sx + K + wave * 512;
+    float* const sb = sx + chunks * CODES + wave * 512;
     auto fetch = [&](int step, Operands& o) {
-        const int L = step * 64 + lane, g = (L * CODES) >> gs_shift;  // group sizes are powers of two
+        int L = step * 64 + lane;
+        L = L < last_chunk ? L : last_chunk;
+        const int g = (L * CODES) >> gs_shift;  // group sizes are powers of two
 #pragma unroll
         for (int r = 0; r < RW; ++r) o.w[r] = wrow[r][L];
         if (!sb_lds) {
@@ -219,8 +150,10 @@ __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uin
         __builtin_amdgcn_global_load_lds((gptr)(brow[r % RW] + part), (lptr)(sb + 256), 16, 0, 0);
     }
     pin();
-    for (int i = tid * 4; i < K; i += 256 * 4) {
-        const float4 v = *reinterpret_cast<const float4*>(x + i);
+    // (in LDS the lanes of a wavefront read consecutive 16-byte slots: lane L of a step, quad j of its chunk)
+    for (int i = tid * 4; i < chunks * CODES; i += 256 * 4) {
+        float4 v{0.f, 0.f, 0.f, 0.f};
+        if (i < K) v = *reinterpret_cast<const float4*>(x + i);
         const int L = i / CODES, j = (i % CODES) / 4;
         *reinterpret_cast<float4*>(sx + (j * chunks + L) * 4) = v;
     }
@@ -234,7 +167,7 @@ __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uin
     auto compute = [&](int step, Operands& o) {
         const int L = step * 64 + lane;
         if (sb_lds) {
-            const int g = (L * CODES) >> gs_shift;
+            const int g = ((L < last_chunk ? L : last_chunk) * CODES) >> gs_shift;
 #pragma unroll
             for (int r = 0; r < RW; ++r) o.s[r] = sb[r * 64 + g], o.b[r] = sb[256 + r * 64 + g];
         }
@@ -300,44 +233,32 @@ __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uin
     }
 }
 
+constexpr int kGemv1MaxLds = 160 * 1024;
+// x of whole steps, then scales / biases per wavefront
+size_t wq_gemv1_lds(int K, int bits) {
+    const size_t step = 64 * 128 / bits;
+    return (size_t(K) + step - 1) / step * step * sizeof(float) + 4 * 512 * sizeof(float);
+}
+
 template <int BITS>
 int launch_gemv1(const float* x, const uint32_t* packed, const float* scales, const float* biases, int N, int K,
                  int gs, float* out, hipStream_t st) {
-    const size_t smem = size_t(K) * sizeof(float) + 4 * 512 * sizeof(float);  // x, then scales / biases per wavefront
-    const void* fn = reinterpret_cast<const void*>(wq_gemv1_kernel<BITS>);
-    static size_t attr = 0;
-    if (smem > attr) {
-        LQ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(smem)));
-        attr = smem;
-    }
+    const size_t smem = wq_gemv1_lds(K, BITS);
+    static DeviceOnce once;
+    if (const int rc = allow_dynamic_lds(once, reinterpret_cast<const void*>(wq_gemv1_kernel<BITS>), kGemv1MaxLds)) return rc;
     hipLaunchKernelGGL((wq_gemv1_kernel<BITS>), dim3(unsigned((N + WQ_ROWS - 1) / WQ_ROWS)), dim3(256), smem, st, x,
                        packed, scales, biases, N, K, gs, out);
     LQ_CHECK_LAUNCH("wq_gemv1");
     return LQ_OK;
 }
 
-template <int BITS, int MT>
-int launch_gemv(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
-                int K, int gs, int m0, float* out, hipStream_t st) {
-    const size_t smem = size_t(MT) * K * sizeof(float);
-    const void* fn = reinterpret_cast<const void*>(wq_gemv_kernel<BITS, MT>);
-    static size_t attr = 0;
-    if (smem > attr) {
-        LQ_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(smem)));
-        attr = smem;
-    }
-    hipLaunchKernelGGL((wq_gemv_kernel<BITS, MT>), dim3(unsigned((N + WQ_ROWS - 1) / WQ_ROWS)), dim3(256), smem, st, x,
-                       packed, scales, biases, M, N, K, gs, m0, out);
-    LQ_CHECK_LAUNCH("wq_gemv");
-    return LQ_OK;
-}
-
-// Small-batch matmul on the matrix cores (2 .. 64 activation rows, 16 per block row).
+// Small-batch matmul on the matrix cores (16 activation rows per block row; up to about a hundred rows, more
+// where the weight is small: wq_gemm_beats_small_batch).
 //
 // y[m, n] = sum over groups g of  s[n, g] * (sum_{k in g} c[n, k] x[m, k])  +  b[n, g] * (sum_{k in g} x[m, k]):
 // the inner sums run on v_mfma_f32_16x16x32_bf16 with the codes themselves as one operand -
-// an 8-bit code is exact in bfloat16, a 4-bit code c is formed as the bit pattern 0x4300 | c
-// = 128 + c (one AND-OR per two codes) and the 128 goes into the bias term - and x as the
+// an 8-bit code is exact in bfloat16, a 4-bit code c is formed as the bit pattern of OFF + c
+// (wq_codes) and the OFF goes into the bias term - and x as the
 // other, split into three bfloat16 parts x = hi + mid + lo (exact: 8 + 8 + 8 significant
 // bits, wq_split3x2), one MFMA each.  Products are exact and accumulate in float32, so nothing of x or
 // of the weight is rounded before the sums.
@@ -369,64 +290,8 @@ int launch_gemv(const float* x, const uint32_t* packed, const float* scales, con
 // writes its partial sums to a slab, and the last one to arrive (an arrival counter per row
 // tile, reset by that block) adds the slabs in index order - the result does not depend on
 // the order of arrival - and stores.  One launch, no workspace besides the slabs.
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
 // LDS a block may ask for: 48 KiB of x fragments and the tables of 256 rows x 16 groups
 constexpr int kWqMaxLds = 512 / 32 * 3 * 64 * 16 + 2 * 256 * 17 * 4;
-
-template <int BITS>
-struct WqGeom {
-    static constexpr int CODES = 128 / BITS;  // codes per 16-byte load: 32 or 16
-    static constexpr int WK = 4 * CODES;      // k per window: 128 or 64
-    static constexpr int NI = WK / 32;        // instructions (k steps of 32) per window: 4 or 2
-};
-
-// How the registers are exchanged for a group size: 0 = not at all, 1 = between lane halves,
-// 2 = transposed; the window then holds 1, 2 or 4 group segments.
-__host__ __device__ inline int wq_swap_mode(int bits, int gs) {
-    const int window = 512 / bits;
-    return gs >= window ? 0 : (gs * 2 == window ? 1 : 2);
-}
-
-// After the exchange, register rho of quarter q holds what quarter q_src loaded as register j_src.
-__host__ __device__ inline void wq_source(int sw, int rho, int q, int& q_src, int& j_src) {
-    q_src = q, j_src = rho;
-    if (sw == 1 && (rho < 2) != (q < 2)) {
-        q_src = rho < 2 ? q - 2 : q + 2;
-        j_src = rho < 2 ? rho + 2 : rho - 2;
-    } else if (sw == 2) {
-        q_src = rho, j_src = q;
-    }
-}
-
-// upper lane half of a <-> lower lane half of b
-__device__ __forceinline__ void wq_swap32(uint32_t& a, uint32_t& b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = r[0], b = r[1];
-}
-// odd 16-lane rows of a <-> even 16-lane rows of b
-__device__ __forceinline__ void wq_swap16(uint32_t& a, uint32_t& b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    a = r[0], b = r[1];
-}
-
-// (e0, e1) = h + m + l part by part, each part a pair of bfloat16 (e0's in the low half): the
-// packed conversion rounds to nearest, the remainders are exact (8 + 8 + 8 significant bits with
-// signed remainders).  A NaN stays a NaN in every part; an infinity turns into a NaN in the
-// lower parts, so a non-finite x gives a non-finite y.
-typedef __bf16 wq_bf2 __attribute__((ext_vector_type(2)));
-typedef float wq_f2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t wq_pk(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(wq_f2{a, b}, wq_bf2));
-}
-__device__ __forceinline__ void wq_split3x2(float e0, float e1, uint32_t& h, uint32_t& m, uint32_t& l) {
-    h = wq_pk(e0, e1);
-    e0 -= __uint_as_float(h << 16), e1 -= __uint_as_float(h & 0xffff0000u);
-    m = wq_pk(e0, e1);
-    e0 -= __uint_as_float(m << 16), e1 -= __uint_as_float(m & 0xffff0000u);
-    l = wq_pk(e0, e1);
-}
 
 constexpr int kWqRows = 256;    // weight rows per block
 constexpr int kWqSliceK = 512;  // k per block
@@ -439,7 +304,7 @@ constexpr int kWqSliceK = 512;  // k per block
 // stay conflict-free.
 __device__ __forceinline__ int wq_x_slot(int m, int qd, int blk) { return ((m + 4 * qd + blk) & 15) + 16 * qd; }
 
-template <int BITS, int SW>
+template <int BITS, int SW, int OFF>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void wq_mfma_kernel(
     const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N, int K,
     int gs_shift, float* out, float* slabs, int* counters) {
@@ -465,12 +330,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int tile = blockIdx.y, ks = blockIdx.x, mb = blockIdx.z, slices = gridDim.x;
     const int n_base = tile * kWqRows + wave * (RB * 16), m0 = mb * 16;
     const int words_per_row = K * BITS / 32, groups_per_row = K >> gs_shift;
-    const int windows = K / WK;
+    const int windows = (K + WK - 1) / WK;  // the last one may be partial (K is a multiple of 32: whole 16-byte loads)
     const int w0 = ks * WPS;
     const int nw = windows - w0 < WPS ? windows - w0 : WPS;  // at least 1: the host sizes grid.y so
     // groups of this block's windows, and the row stride of the tables
     const int g0 = (w0 * WK) >> gs_shift;
-    const int ng = (((w0 + nw) * WK - 1) >> gs_shift) - g0 + 1;
+    const int k_end = (w0 + nw) * WK < K ? (w0 + nw) * WK : K;
+    const int ng = ((k_end - 1) >> gs_shift) - g0 + 1;
     const int gmax = kWqSliceK >> gs_shift, gp = (gmax < 1 ? 1 : gmax) + 1;
 
     // Every global load of the block is requested before anything is consumed, in the order of
@@ -514,7 +380,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     for (int u = 0; u < UNITS / 512; ++u) {
         const int unit = u * 512 + threadIdx.x, m = m0 + unit / OCTS, kl = (unit % OCTS) * 8;
         raw[u][0] = raw[u][1] = float4{0.f, 0.f, 0.f, 0.f};
-        if (m < M && kl < nw * WK) {
+        if (m < M && w0 * WK + kl < k_end) {
             const float* src = x + size_t(m) * K + w0 * WK + kl;
             raw[u][0] = *reinterpret_cast<const float4*>(src);
             raw[u][1] = *reinterpret_cast<const float4*>(src + 4);
@@ -533,8 +399,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         const uint32_t* row = packed + size_t(n) * words_per_row + (lane & 3) * (CODES * BITS / 32);
 #pragma unroll
         for (int wi = 0; wi < WPS; ++wi)
-            // past the last window every lane reads the same 16 bytes: one cache line, dropped later
-            wv[wi][rb] = *reinterpret_cast<const uint4*>(wi < nw ? row + (w0 + wi) * (WK * BITS / 32) : packed);
+            // past K every lane reads the same 16 bytes: one cache line, dropped later or multiplied by zeros of x
+            wv[wi][rb] = *reinterpret_cast<const uint4*>(
+                (w0 + wi) * WK + (lane & 3) * CODES < k_end ? row + (w0 + wi) * (WK * BITS / 32) : packed);
     }
     // The tables go to LDS, then x, split and laid out as fragments by the block itself: a thread
     // finds the (instruction, quarter) that holds its eight k - the exchange of registers is its
@@ -595,8 +462,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                 wd[rb][1] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[wi][rb].y)));
                 wd[rb][2] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[wi][rb].z)));
                 wd[rb][3] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[wi][rb].w)));
-                if (SW >= 1) wq_swap32(wd[rb][0], wd[rb][2]), wq_swap32(wd[rb][1], wd[rb][3]);
-                if (SW == 2) wq_swap16(wd[rb][0], wd[rb][1]), wq_swap16(wd[rb][2], wd[rb][3]);
+                wq_exchange<SW>(wd[rb]);
             }
 #pragma unroll
             for (int e = 0; e < GW; ++e) {
@@ -611,26 +477,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                     const int i = e * IPS + ii;
                     uint4 cf[RB];
 #pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) {
-                        if (BITS == 4) {
-                            const uint32_t c = wd[rb][i];
-                            cf[rb].x = (c & 0x000f000fu) | 0x43004300u;
-                            cf[rb].y = ((c >> 4) & 0x000f000fu) | 0x43004300u;
-                            cf[rb].z = ((c >> 8) & 0x000f000fu) | 0x43004300u;
-                            cf[rb].w = ((c >> 12) & 0x000f000fu) | 0x43004300u;
-                        } else {
-                            // a byte as a float has zeros below bit 16: its upper half is the bfloat16
-                            const uint32_t a = wd[rb][2 * i], b = wd[rb][2 * i + 1];
-                            const uint32_t a0 = __float_as_uint(float(a & 0xffu)), a1 = __float_as_uint(float((a >> 8) & 0xffu));
-                            const uint32_t a2 = __float_as_uint(float((a >> 16) & 0xffu)), a3 = __float_as_uint(float(a >> 24));
-                            const uint32_t b0 = __float_as_uint(float(b & 0xffu)), b1 = __float_as_uint(float((b >> 8) & 0xffu));
-                            const uint32_t b2 = __float_as_uint(float((b >> 16) & 0xffu)), b3 = __float_as_uint(float(b >> 24));
-                            cf[rb].x = __builtin_amdgcn_perm(a1, a0, 0x07060302u);
-                            cf[rb].y = __builtin_amdgcn_perm(a3, a2, 0x07060302u);
-                            cf[rb].z = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-                            cf[rb].w = __builtin_amdgcn_perm(b3, b2, 0x07060302u);
-                        }
-                    }
+                    for (int rb = 0; rb < RB; ++rb) cf[rb] = wq_codes<BITS, OFF>(wd[rb], i);
 #pragma unroll
                     for (int p = 0; p < 3; ++p) {
                         const v8bf xf = __builtin_bit_cast(v8bf, x_lds[((wi * NI + i) * 3 + p) * 64 + wq_x_slot(lane & 15, lane >> 4, wi * NI + i)]);
@@ -645,8 +492,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                 for (int rb = 0; rb < RB; ++rb) {
                     const float sc = s_lds[(row_in_tile + rb * 16) * gp + g];
                     const float bi = b_lds[(row_in_tile + rb * 16) * gp + g];
-                    // the 4-bit codes entered as 128 + c
-                    const float bz = BITS == 4 ? bi - 128.0f * sc : bi;
+                    // the 4-bit codes entered as OFF + c
+                    const float bz = BITS == 4 ? bi - float(OFF) * sc : bi;
                     y[rb] = y[rb] + (acc[rb] * sc + acc[RB] * bz);
                 }
             }
@@ -726,7 +573,7 @@ int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, 
     using G = WqGeom<BITS>;
     constexpr int WPS = kWqSliceK / G::WK;
     const int sw = wq_swap_mode(BITS, gs);
-    const int mblocks = (M + 15) / 16, windows = K / G::WK;
+    const int mblocks = (M + 15) / 16, windows = (K + G::WK - 1) / G::WK;
     const int tiles = (N + kWqRows - 1) / kWqRows, slices = (windows + WPS - 1) / WPS;
     SkScratch sk;
     if (slices > 1) {
@@ -737,13 +584,23 @@ int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, 
     const int gs_shift = 31 - __builtin_clz(unsigned(gs));
     const int gmax = kWqSliceK / gs;
     const size_t lds = size_t(WPS) * G::NI * 3 * 64 * 16 + size_t(2) * kWqRows * ((gmax < 1 ? 1 : gmax) + 1) * 4;
+    // 2 .. 64 rows of whole windows keep the offset, and so the bits, that they have always had
+    constexpr int kFirst = BITS == 4 ? 128 : 0, kOther = BITS == 4 ? 16 : 0;
+    const bool first = BITS == 8 || (M > 1 && M <= 64 && K % G::WK == 0);
 #define LQ_WQ_LAUNCH(SWM)                                                                                         \
     do {                                                                                                          \
+        if (first)                                                                                                \
+            LQ_WQ_LAUNCH_OFF(SWM, kFirst);                                                                        \
+        else                                                                                                      \
+            LQ_WQ_LAUNCH_OFF(SWM, kOther);                                                                        \
+    } while (0)
+#define LQ_WQ_LAUNCH_OFF(SWM, OFF)                                                                                \
+    do {                                                                                                          \
         static DeviceOnce attr_once;                                                                              \
-        const int arc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SWM>),    \
+        const int arc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SWM, OFF>), \
                                           kWqMaxLds);                                                             \
         if (arc) return arc;                                                                                      \
-        hipLaunchKernelGGL((wq_mfma_kernel<BITS, SWM>), grid, dim3(512), lds, st, x, packed, scales, biases, M,   \
+        hipLaunchKernelGGL((wq_mfma_kernel<BITS, SWM, OFF>), grid, dim3(512), lds, st, x, packed, scales, biases, M, \
                            N, K, gs_shift, out, reinterpret_cast<float*>(sk.slabs), sk.counters);                 \
     } while (0)
     if (sw == 0)
@@ -753,6 +610,7 @@ int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, 
     else if constexpr (BITS == 4)
         LQ_WQ_LAUNCH(2);
 #undef LQ_WQ_LAUNCH
+#undef LQ_WQ_LAUNCH_OFF
     LQ_CHECK_LAUNCH("wq_mfma");
     return LQ_OK;
 }
@@ -810,33 +668,18 @@ int lq_wq_matmul(const float* x, const uint32_t* packed, const float* scales, co
     if (M == 0 || N == 0) return LQ_OK;
     LQ_REQUIRE(x && packed && scales && biases && out, LQ_ERR_VALUE, "wq_matmul: NULL pointer");
     hipStream_t st = as_stream(stream);
-    const bool fused_ok = aligned16(x) && aligned16(packed) && K % 4 == 0 && (K * bits / 8) % 16 == 0 &&
-                          size_t(4) * K * sizeof(float) <= 64 * 1024;
-    // 16 activation rows per launch on the matrix cores; a step covers 512 / bits weights per row
-    const bool mfma_ok = aligned16(x) && aligned16(packed) && K % (512 / bits) == 0;
-    if (M > 1 && M <= 64 && mfma_ok)
+    if (aligned16(x) && aligned16(packed)) {
+        // one row is a stream of the weight; more rows go to the matrix cores: 16 rows x 512 k of 256 columns
+        // per block, or (wq_gemm.hip) tiles over all of K
+        if (M == 1 && wq_gemv1_lds(K, bits) <= size_t(kGemv1MaxLds))
+            return bits == 4 ? launch_gemv1<4>(x, packed, scales, biases, N, K, group_size, out, st)
+                             : launch_gemv1<8>(x, packed, scales, biases, N, K, group_size, out, st);
+        if (wq_gemm_beats_small_batch(M, N, K, group_size, bits))
+            return launch_wq_gemm(x, packed, scales, biases, M, N, K, group_size, bits, out, st);
         return bits == 4 ? launch_wq_mfma<4>(x, packed, scales, biases, M, N, K, group_size, out, st)
                          : launch_wq_mfma<8>(x, packed, scales, biases, M, N, K, group_size, out, st);
-    if (M == 1 && fused_ok && K % (8192 / bits) == 0)
-        return bits == 4 ? launch_gemv1<4>(x, packed, scales, biases, N, K, group_size, out, st)
-                         : launch_gemv1<8>(x, packed, scales, biases, N, K, group_size, out, st);
-    if (M <= 16 && fused_ok) {
-        // decode shapes: weights are read once per pass of up to four activation rows
-        for (int m0 = 0; m0 < M; m0 += 4) {
-            const int rows = M - m0;
-            if (bits == 4)
-                rc = rows == 1 ? launch_gemv<4, 1>(x, packed, scales, biases, M, N, K, group_size, m0, out, st)
-                     : rows == 2 ? launch_gemv<4, 2>(x, packed, scales, biases, M, N, K, group_size, m0, out, st)
-                                 : launch_gemv<4, 4>(x, packed, scales, biases, M, N, K, group_size, m0, out, st);
-            else
-                rc = rows == 1 ? launch_gemv<8, 1>(x, packed, scales, biases, M, N, K, group_size, m0, out, st)
-                     : rows == 2 ? launch_gemv<8, 2>(x, packed, scales, biases, M, N, K, group_size, m0, out, st)
-                                 : launch_gemv<8, 4>(x, packed, scales, biases, M, N, K, group_size, m0, out, st);
-            if (rc) return rc;
-        }
-        return LQ_OK;
     }
-    // compute-bound shapes: decode once into the workspace, then the float32 MFMA GEMM
+    // operands that are not 16-byte aligned: decode once into the workspace, then the float32 MFMA GEMM
     void* ws = nullptr;
     rc = workspace(size_t(N) * K * sizeof(float), st, &ws);
     if (rc) return rc;

@@ -76,6 +76,28 @@ def test_small_batch_matmul_is_reproducible_and_exact_on_exact_inputs(bits):
     assert np.array_equal(y1.astype(np.float64), x.astype(np.float64) @ w.T)
 
 
+@pytest.mark.parametrize("M,N,K,gs,bits", [
+    (1025, 3003, 288, 32, 4), (700, 2500, 416, 32, 8), (513, 4097, 256, 64, 4), (300, 6000, 256, 128, 8),
+    (130, 11008, 320, 64, 8), (600, 1000, 1024, 64, 4), (1100, 5370, 128, 128, 4), (1100, 5370, 96, 32, 8),
+    (333, 10999, 128, 128, 8), (330, 11008, 192, 64, 4), (333, 9000, 224, 32, 4),
+    # the small-batch kernel with a partial last window
+    (5, 300, 2016, 32, 8), (33, 258, 1056, 32, 4), (16, 77, 192, 64, 4),
+    # one row: K that does not fill the last step, several steps
+    (1, 300, 32, 32, 4), (1, 33, 2016, 32, 8), (1, 77, 2112, 64, 4), (1, 18, 8224, 32, 8)])
+def test_large_batch_matmul_is_exact_on_exact_inputs(M, N, K, gs, bits):
+    """Every tile of the large-batch kernel (rows, columns and K that do not fill tiles, stages or turns
+    of the main loop) on integers whose products and sums are all exact in float32."""
+    rng = np.random.default_rng(M + N + K)
+    packed = rng.integers(0, 2**32, (N, K * bits // 32), dtype=np.uint32).view(np.int32)
+    s = rng.integers(1, 3, (N, K // gs)).astype(np.float32)
+    b = rng.integers(-8, 9, (N, K // gs)).astype(np.float32)
+    x = rng.integers(-7, 8, (M, K)).astype(np.float32)  # |sums| <= K * 7 * (2 * 255 + 8), or the dot of one lane, < 2^24
+    if K > 4096:
+        x[:, ::3] = 0  # (keeps the long sum below 2^24)
+    y = _qgemm.quantized_matmul(hip(x), hip(packed), hip(s), hip(b), True, gs, bits).numpy()
+    assert np.array_equal(y, x @ W.dequantize(packed, s, b, gs, bits).T)
+
+
 def test_decoding_takes_foreign_scales_and_biases_as_given():
     # a weight packed elsewhere under the same contract may carry negative scales
     rng = np.random.default_rng(1)
