@@ -45,7 +45,8 @@ int hip_fail(hipError_t e, const char* what);
 // this request and holds no defined contents.
 int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, bool* fresh);
 // kind 0: the general workspace (at least 4 MiB); 1 / 2: stream-K counters / slabs;
-// 3: raw accumulators and operand sums of a layer with affine weights; 4: padded copies of ragged GEMM operands
+// 3: raw accumulators and operand sums of a layer with affine weights; 4: padded copies of ragged GEMM operands;
+// 5: the range slots of a dynamic quantization; 6: the codes and qparams of a dynamic Linear's activation
 int workspace(size_t nbytes, hipStream_t stream, void** ptr);
 // Split-K scratch of one stream: arrival counters (zero between launches: the finisher of a
 // tile resets its counter) and slabs for the partial results, whose layout the kernel defines.

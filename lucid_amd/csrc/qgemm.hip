@@ -850,10 +850,13 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
     const bool vec_ok = g.K % 16 == 0 && g.K > 0 && aligned16(g.a) && aligned16(g.w);
     int path = force_path;  // 0 = choose, 1 = tile, 2 = skinny, 3 = naive
     if (path == 0) {
-        // The small-batch kernels stream the weight once whatever its alignment.  More rows than they take,
-        // or a kept range, need the tile kernel: ragged or unaligned operands are copied to padded rows
-        // first (333 x 1001 x 1000: 1340 -> 11 us; 100 x 11008 x 5001: 26.4 ms -> 50 us).  Rows shorter than one chunk stay with the plain kernel.
-        path = g.K < 16 ? 3 : (g.M <= 64 && g.range == nullptr ? 2 : 1);
+        // The small-batch kernels stream the weight once whatever its alignment.  From 17 rows on 64 x 64 tiles
+        // are faster (us, small batch / tiles: 17 x 11008 x 4096 17.2 / 11.0, 64 rows 33.4 / 11.5; 17 x 4096 x
+        // 4096 11.8 / 9.8; 17 x 1024 x 4096 9.0 / 9.5, 64 rows 15.8 / 9.3), but ragged or unaligned operands
+        // have to be copied to padded rows for them, the whole weight too: that pays from 65 rows (333 x 1001
+        // x 1000: 1340 -> 11 us against the plain kernel; 100 x 11008 x 5001: 26.4 ms -> 50 us).  A kept range
+        // needs the tile kernel.  Rows shorter than one chunk stay with the plain kernel.
+        path = g.K < 16 ? 3 : (g.M <= (vec_ok ? 16 : 64) && g.range == nullptr ? 2 : 1);
         if (path == 1 && !vec_ok) {
             const int ld = (g.K + 63) / 64 * 64;
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;

@@ -6,6 +6,7 @@
 // round-half-even, add zero point, clamp, cast.  No reciprocal, no FMA.
 #include <mutex>
 #include "common.hpp"
+#include "qgemm.hpp"
 #include "range_slots.hpp"
 
 using namespace lq;
@@ -325,30 +326,7 @@ __device__ __forceinline__ void mm_update(MinMax& m, float v) {
 }
 
 __device__ __forceinline__ MinMax mm_block_reduce(MinMax m) {
-    // wavefront (64 lanes) butterfly, then across the block's waves via LDS
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        m.lo = fminf(m.lo, __shfl_xor(m.lo, d, 64));
-        m.hi = fmaxf(m.hi, __shfl_xor(m.hi, d, 64));
-        m.nan |= __shfl_xor(m.nan, d, 64);
-    }
-    __shared__ float s_lo[16], s_hi[16];  // up to 1024 threads
-    __shared__ int s_nan[16];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int nwaves = (blockDim.x + 63) >> 6;
-    if (lane == 0) {
-        s_lo[wave] = m.lo;
-        s_hi[wave] = m.hi;
-        s_nan[wave] = m.nan;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < nwaves; ++w) {
-            m.lo = fminf(m.lo, s_lo[w]);
-            m.hi = fmaxf(m.hi, s_hi[w]);
-            m.nan |= s_nan[w];
-        }
-    }
+    block_minmax(m.lo, m.hi, m.nan);
     return m;
 }
 
@@ -538,7 +516,6 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
     const float4* __restrict__ x, int quads, int symmetric, int qmin, int qmax, int is_signed, float eps,
     float half_range, int off, float* __restrict__ scale, float* __restrict__ zp, float* __restrict__ mn_out,
     float* __restrict__ mx_out, Code8x4* __restrict__ q) {
-    __shared__ float s_sz[2];
     const size_t row = blockIdx.x;
     const float4* xr = x + row * size_t(quads);
     float4 v[R];
@@ -552,18 +529,16 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
         }
     }
     m = mm_block_reduce(m);
+    const float qnan = __builtin_nanf("");
+    const float mn = m.nan ? qnan : m.lo, mx = m.nan ? qnan : m.hi;
+    float s, z;
+    qparams_of(mn, mx, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
     if (threadIdx.x == 0) {
-        const float qnan = __builtin_nanf("");
-        const float mn = m.nan ? qnan : m.lo, mx = m.nan ? qnan : m.hi;
-        float s, z;
-        qparams_of(mn, mx, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
         scale[row] = s, zp[row] = z;
         if (mn_out) mn_out[row] = mn;
         if (mx_out) mx_out[row] = mx;
-        s_sz[0] = s, s_sz[1] = z;
     }
-    __syncthreads();
-    const float s = s_sz[0], z = s_sz[1], r = 1.0f / s;
+    const float r = 1.0f / s;
     const QuantizeOp<int8_t> op{nullptr, nullptr, float(double(qmin)), float(double(qmax)), off};
     Code8x4* qr = q + row * size_t(quads);
 #pragma unroll
@@ -573,85 +548,275 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
     }
 }
 
-// Dynamic per-tensor quantization of a small tensor in one launch (one block): global
-// min / max (observer.py:363-375), qparams, codes.  Up to 16 float4 per lane (65536
-// elements) stay in registers between the two phases, all their loads in flight at once;
-// beyond that the block works in batches of 8 and re-reads x (from the L2) for the codes.
-__global__ __launch_bounds__(1024) void quantize_tensor_dynamic_kernel(
-    const float* __restrict__ x, size_t n, int symmetric, int qmin, int qmax, int is_signed, float eps,
-    float half_range, int off, float* __restrict__ scale, float* __restrict__ zp, float* __restrict__ mn_out,
-    float* __restrict__ mx_out, int8_t* __restrict__ q) {
-    __shared__ float s_sz[2];
-    constexpr int kKeep = 16, kBatch = 8;
-    const bool vec = aligned16(x) && (reinterpret_cast<uintptr_t>(q) & 3u) == 0;
-    const size_t quads = vec ? n / 4 : 0;
-    const bool keep = quads <= size_t(kKeep) * 1024;
-    const float4* x4 = reinterpret_cast<const float4*>(x);
-    MinMax m{__builtin_inff(), -__builtin_inff(), 0};
-    float4 v[kKeep];
-    if (keep) {
-#pragma unroll
-        for (int u = 0; u < kKeep; ++u) {
-            const size_t i = size_t(u) * 1024 + threadIdx.x;
-            if (i < quads) v[u] = x4[i];
-        }
-#pragma unroll
-        for (int u = 0; u < kKeep; ++u)
-            if (size_t(u) * 1024 + threadIdx.x < quads)
-                mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
+// Dynamic per-tensor quantization: global min / max (observer.py:363-375), qparams, codes.  A block holds 8192
+// elements in registers.
+//
+// Small tensors (up to kExchange blocks) in one launch, x read once: the blocks' ranges meet through a slot per
+// block in device memory - written through, and polled by every block until it is filled - and each block then
+// derives the qparams itself and writes its codes.  The last block to leave empties the slots for the next
+// launch.  All blocks have to be resident (see lstm.hip on what the launcher has to leave free: kExchange
+// blocks of 512 threads and 64 registers are far below it), and a wait is bounded.
+//
+// Beyond, two launches: slices' ranges (minmax_seg_kernel), then this kernel with PARTS - every block reduces
+// the slices' ranges itself, which saves the finalize and qparams launches between.
+//
+// Rows of `cols` elements go to rows of `ld` codes, zeros past `cols` (what a GEMM of ragged rows wants).
+//
+// 8192 elements 3.4 us, 65536 (8 blocks, the exchange) 5.9; with all 128 blocks of 1 M elements polling each other's
+// slots it was 17 us, in two launches 3.8 + 5.0.  Before: one block on one CU for up to 262144 elements (61 us), five
+// launches beyond (1 M elements: 12.3 us).
+constexpr int kDynThreads = 512, kDynQuads = 4, kDynPerBlock = kDynThreads * kDynQuads * 4;
+constexpr int kExchange = 16, kMaxParts = 512;
+constexpr unsigned long long kSlotEmpty = ~0ull;  // NaNs that no range contains: mm_write's NaN is the canonical one
+struct DynScratch {
+    unsigned long long slot[kExchange];    // low word: the block's minimum, high word: its maximum
+    unsigned left;                        // blocks that have read the slots
+};
+
+// Elements e .. e+3 of x[0 .. n), zeros past n.  One unconditional 16-byte load (any float address) from where all
+// four exist: a load under a condition would be waited for before the next one is issued.
+__device__ __forceinline__ float4 load_quad(const float* x, size_t e, size_t n) {
+    float4 v{0.f, 0.f, 0.f, 0.f};
+    if (n < 4) {  // uniform
+        if (e < n) v.x = x[e];
+        if (e + 1 < n) v.y = x[e + 1];
+        if (e + 2 < n) v.z = x[e + 2];
+        return v;
+    }
+    const size_t at = e < n - 4 ? e : n - 4;
+    __builtin_memcpy(&v, x + at, 16);
+    return v;
+}
+// ... and, once it has arrived, the elements in place
+__device__ __forceinline__ float4 place_quad(float4 v, size_t e, size_t n) {
+    if (n < 4 || e + 4 <= n) return v;
+    const size_t d = e - (n - 4);
+    return d == 1 ? float4{v.y, v.z, v.w, 0.f}
+                  : (d == 2 ? float4{v.z, v.w, 0.f, 0.f} : (d == 3 ? float4{v.w, 0.f, 0.f, 0.f} : float4{0.f, 0.f, 0.f, 0.f}));
+}
+__device__ __forceinline__ void mm_update_quad(MinMax& m, float4 v, size_t e, size_t n) {
+    if (e + 4 <= n) {
+        mm_update(m, v.x), mm_update(m, v.y), mm_update(m, v.z), mm_update(m, v.w);
     } else {
-        for (size_t i0 = 0; i0 < quads; i0 += size_t(kBatch) * 1024) {
-            float4 w[kBatch];
+        if (e < n) mm_update(m, v.x);
+        if (e + 1 < n) mm_update(m, v.y);
+        if (e + 2 < n) mm_update(m, v.z);
+    }
+}
+
+// RAGGED: rows of `cols` elements to rows of `ld` codes (a multiple of 4); the quads are those of the codes, so
+// that every store is one aligned word.  Otherwise one run of n elements.
+template <bool PARTS, bool RAGGED>
+__global__ __launch_bounds__(kDynThreads) __attribute__((amdgpu_waves_per_eu(8)))
+void quantize_tensor_dynamic_kernel(const float* __restrict__ x, size_t n, unsigned cols, unsigned ld, int symmetric,
+                                    int qmin, int qmax, int is_signed, float eps, float half_range, int off,
+                                    DynScratch* slots, const float* __restrict__ parts, int n_parts, float* scale,
+                                    float* zp, float* mn_out, float* mx_out, int8_t* __restrict__ q) {
+    __shared__ int s_last;
+    const int tid = threadIdx.x;
+    const size_t first = size_t(blockIdx.x) * kDynPerBlock;
+    const float qnan = __builtin_nanf("");
+    MinMax m{__builtin_inff(), -__builtin_inff(), 0};
+    if (PARTS && tid < n_parts) m.lo = parts[tid], m.hi = parts[n_parts + tid];
+    float4 v[kDynQuads];
+    int count[kDynQuads];  // elements of the quad that exist
+    auto at = [&](int u) { return first + size_t(u * kDynThreads + tid) * 4; };
+    auto element = [&](int u) {
+        if (!RAGGED) return at(u);
+        const unsigned row = unsigned(at(u)) / ld;  // (fewer than 2^32 codes: see the launcher)
+        return size_t(row) * cols + (unsigned(at(u)) - row * ld);
+    };
 #pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const size_t i = i0 + size_t(u) * 1024 + threadIdx.x;
-                if (i < quads) w[u] = x4[i];
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                if (i0 + size_t(u) * 1024 + threadIdx.x < quads)
-                    mm_update(m, w[u].x), mm_update(m, w[u].y), mm_update(m, w[u].z), mm_update(m, w[u].w);
+    for (int u = 0; u < kDynQuads; ++u) {
+        const size_t e = element(u);
+        v[u] = load_quad(x, e, n);
+        if (RAGGED) {
+            const int left = int(cols) - int(unsigned(at(u)) % ld);
+            count[u] = e >= n || left <= 0 ? 0 : (left < 4 ? left : 4);
+        } else {
+            count[u] = e + 4 <= n ? 4 : (e < n ? int(n - e) : 0);
         }
     }
-    for (size_t e = quads * 4 + threadIdx.x; e < n; e += 1024) mm_update(m, x[e]);
+    if (RAGGED || first + kDynPerBlock > n) {
+#pragma unroll
+        for (int u = 0; u < kDynQuads; ++u) v[u] = place_quad(v[u], element(u), n);
+    }
+    if (PARTS) {
+        m.nan = (m.lo != m.lo) | (m.hi != m.hi);
+    } else if (!RAGGED && first + kDynPerBlock <= n) {
+#pragma unroll
+        for (int u = 0; u < kDynQuads; ++u)
+            mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
+    } else {
+#pragma unroll
+        for (int u = 0; u < kDynQuads; ++u) mm_update_quad(m, v[u], 0, count[u]);
+    }
     m = mm_block_reduce(m);
-    if (threadIdx.x == 0) {
-        const float qnan = __builtin_nanf("");
-        const float mn = m.nan ? qnan : m.lo, mx = m.nan ? qnan : m.hi;
-        float s, z;
-        qparams_of(mn, mx, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
+    if (!PARTS && gridDim.x > 1) {
+        if (tid == 0) {
+            const unsigned lo = __float_as_uint(m.nan ? qnan : m.lo), hi = __float_as_uint(m.nan ? qnan : m.hi);
+            __hip_atomic_store(&slots->slot[blockIdx.x], (unsigned long long)hi << 32 | lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        m = MinMax{__builtin_inff(), -__builtin_inff(), 0};
+        if (tid < int(gridDim.x)) {
+            unsigned long long got = kSlotEmpty;
+            for (int spin = 0; got == kSlotEmpty && spin < (1 << 20); ++spin)
+                got = __hip_atomic_load(&slots->slot[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            m.lo = __uint_as_float(unsigned(got)), m.hi = __uint_as_float(unsigned(got >> 32));
+            m.nan = (m.lo != m.lo) | (m.hi != m.hi);
+        }
+        __syncthreads();  // every slot has been read (and the reduction may use its LDS again)
+        if (tid == 0) {
+            const unsigned before = __hip_atomic_fetch_add(&slots->left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_last = before == gridDim.x - 1;
+        }
+        m = mm_block_reduce(m);
+    }
+    const float mn = m.nan ? qnan : m.lo, mx = m.nan ? qnan : m.hi;
+    float s, z;
+    qparams_of(mn, mx, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
+    if (blockIdx.x == 0 && tid == 0) {
         *scale = s, *zp = z;
         if (mn_out) *mn_out = mn;
         if (mx_out) *mx_out = mx;
-        s_sz[0] = s, s_sz[1] = z;
     }
-    __syncthreads();
-    const float s = s_sz[0], z = s_sz[1], r = 1.0f / s;
-    const QuantizeOp<int8_t> op{x4, reinterpret_cast<Code8x4*>(q), float(double(qmin)), float(double(qmax)), off};
-    if (keep) {
+    if (!PARTS && gridDim.x > 1 && s_last) {  // nobody reads the slots any more
+        if (tid < kExchange) slots->slot[tid] = kSlotEmpty;
+        if (tid == 0) slots->left = 0;
+    }
+    const float r = 1.0f / s;
+    const QuantizeOp<int8_t> op{nullptr, nullptr, float(double(qmin)), float(double(qmax)), off};
 #pragma unroll
-        for (int u = 0; u < kKeep; ++u) {
-            const size_t i = size_t(u) * 1024 + threadIdx.x;
-            if (i < quads) op.q[i] = op.pack(v[u], s, z, r);
-        }
-    } else {
-        for (size_t i0 = 0; i0 < quads; i0 += size_t(kBatch) * 1024) {
-            float4 w[kBatch];
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const size_t i = i0 + size_t(u) * 1024 + threadIdx.x;
-                if (i < quads) w[u] = x4[i];
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const size_t i = i0 + size_t(u) * 1024 + threadIdx.x;
-                if (i < quads) op.q[i] = op.pack(w[u], s, z, r);
-            }
+    for (int u = 0; u < kDynQuads; ++u) {
+        Code8x4 c = op.pack(v[u], s, z, r);
+        if (RAGGED) {
+            unsigned w;
+            __builtin_memcpy(&w, &c, 4);
+            w = count[u] >= 4 ? w : (count[u] <= 0 ? 0u : w & ((1u << (8 * count[u])) - 1u));  // zeros past the row
+            if (at(u) < size_t(n / cols) * ld) __builtin_memcpy(q + at(u), &w, 4);
+        } else if (count[u] == 4) {
+            __builtin_memcpy(q + at(u), &c, 4);
+        } else {
+            for (int i = 0; i < count[u]; ++i) q[at(u) + i] = c.v[i];
         }
     }
-    for (size_t e = quads * 4 + threadIdx.x; e < n; e += 1024) op.scalar(e, s, z);
 }
 
+// One row: a whole dynamic-quantized Linear as a stream of the weight.  Every block needs the row's range and
+// codes: it takes them itself (the row is at most 64 KiB of L2 reads per block) while its first weights are on
+// the way - they are requested before the range is known -, so the layer costs what lq_qlinear_i8 of one row
+// does (qgemv1_kernel: four weight rows per wavefront, a KiB of a row per load, v_dot4) plus the two block
+// reductions.  4096 -> 11008: 24.2 us with the 16 x 16-tile kernel above (688 blocks of 1024 threads, each
+// waiting for its range before its one weight fragment per wavefront), now 10.2 us (4.4 TB/s of weight).
+// w rows are `ld` bytes apart, zeros past K; K <= 16384, ld % 16 == 0.
+__global__ __launch_bounds__(512) void dynamic_gemv1_kernel(
+    const float* __restrict__ x, int K, const int8_t* __restrict__ w, int ld, int N, const float* __restrict__ w_scale,
+    const int32_t* __restrict__ wsum, const float* __restrict__ bias, int relu, int symmetric, int qmin, int qmax,
+    int is_signed, float eps, float half_range, int off, float* __restrict__ out) {
+    extern __shared__ __attribute__((aligned(16))) int8_t dv_codes[];  // K bytes rounded up to a multiple of 4 KiB
+    typedef int dv_v4i __attribute__((ext_vector_type(4)));
+    constexpr int RW = 4, kKeep = 4;  // (with the weights' 64 registers: two blocks per CU)
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, threads = blockDim.x, waves = threads >> 6;
+    const int chunks = (K + 4095) / 4096;
+    // threads x kKeep quads in registers; smaller blocks walk the row in several rounds (the last stays)
+    const int quads = (K + 3) / 4, rounds = (quads + threads * kKeep - 1) / (threads * kKeep);
+    float4 v[kKeep];
+    MinMax m{__builtin_inff(), -__builtin_inff(), 0};
+    for (int rd = 0; rd < rounds; ++rd) {
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) v[u] = load_quad(x, size_t((rd * kKeep + u) * threads + tid) * 4, K);
+        if (rounds > 1) {
+#pragma unroll
+            for (int u = 0; u < kKeep; ++u) {
+                const int e = ((rd * kKeep + u) * threads + tid) * 4;
+                v[u] = place_quad(v[u], e, K);
+                mm_update_quad(m, v[u], e, K);
+            }
+        }
+    }
+    const int nb = (blockIdx.x * waves + wave) * RW;
+    dv_v4i wv[RW][4];
+    auto load_chunk = [&](int kc) {
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            const int n = nb + r < N ? nb + r : N - 1;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int k = kc * 4096 + i * 1024 + lane * 16;
+                wv[r][i] = k < ld ? *reinterpret_cast<const dv_v4i*>(w + size_t(n) * ld + k) : dv_v4i{0, 0, 0, 0};
+            }
+        }
+    };
+    load_chunk(0);
+    const int n_mine = nb + (lane < RW ? lane : 0);
+    const bool mine = lane < RW && n_mine < N;
+    const float c_ws = mine && w_scale ? w_scale[n_mine] : 1.0f;
+    const int c_wsum = mine && wsum ? wsum[n_mine] : 0;
+    const float c_bias = mine && bias ? bias[n_mine] : -0.0f;
+    __builtin_amdgcn_sched_barrier(0);
+    if (rounds == 1) {
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) {
+            const int e = (u * threads + tid) * 4;
+            v[u] = place_quad(v[u], e, K);
+            mm_update_quad(m, v[u], e, K);
+        }
+    }
+    m = mm_block_reduce(m);
+    // (every thread derives the qparams: cheaper than one thread, a barrier and a read)
+    const float qnan = __builtin_nanf("");
+    float s, z;
+    qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
+    const float rcp = 1.0f / s;
+    const QuantizeOp<int8_t> op{nullptr, nullptr, float(double(qmin)), float(double(qmax)), off};
+    for (int rd = rounds - 1; rd >= 0; --rd) {
+        if (rd != rounds - 1) {
+#pragma unroll
+            for (int u = 0; u < kKeep; ++u) v[u] = load_quad(x, size_t((rd * kKeep + u) * threads + tid) * 4, K);
+#pragma unroll
+            for (int u = 0; u < kKeep; ++u) v[u] = place_quad(v[u], ((rd * kKeep + u) * threads + tid) * 4, K);
+        }
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) {
+            // (whatever lies past K, stored or not, meets zeros of the weight)
+            const int i = (rd * kKeep + u) * threads + tid;
+            if (i < quads) *reinterpret_cast<Code8x4*>(dv_codes + i * 4) = op.pack(v[u], s, z, rcp);
+        }
+    }
+    __syncthreads();
+    int acc[RW] = {0, 0, 0, 0};
+    for (int kc = 0; kc < chunks; ++kc) {
+        if (kc) load_chunk(kc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const dv_v4i av = *reinterpret_cast<const dv_v4i*>(dv_codes + kc * 4096 + i * 1024 + lane * 16);
+#pragma unroll
+            for (int r = 0; r < RW; ++r)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[r] = __builtin_amdgcn_sdot4(wv[r][i][e], av[e], acc[r], false);
+        }
+    }
+    int sum = 0;
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        int t = acc[r];
+        t += __builtin_amdgcn_update_dpp(0, t, 0x128, 0xf, 0xf, false);
+        t += __builtin_amdgcn_update_dpp(0, t, 0x124, 0xf, 0xf, false);
+        t += __builtin_amdgcn_update_dpp(0, t, 0x122, 0xf, 0xf, false);
+        t += __builtin_amdgcn_update_dpp(0, t, 0x121, 0xf, 0xf, false);
+        t = __builtin_amdgcn_readlane(t, 0) + __builtin_amdgcn_readlane(t, 16) + __builtin_amdgcn_readlane(t, 32) +
+            __builtin_amdgcn_readlane(t, 48);
+        if (lane == r) sum = t;
+    }
+    if (mine) {
+        const int zi = int(z) + off;
+        const int corr = (wsum != nullptr && zi != 0) ? zi * c_wsum : 0;
+        float y = float(sum - corr) * (s * c_ws);
+        y = y + c_bias;
+        const float floor = relu ? 0.0f : -__builtin_inff();
+        out[n_mine] = (y < floor) ? floor : y;
+    }
+}
 
 // ---------------------------------------------------------------- static scratch (no-allocation entry point)
 // lq_minmax_noalloc keeps the partial results of its two-stage reduction here instead of in
@@ -772,7 +937,6 @@ __global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
     const int32_t* __restrict__ wsum, const float* __restrict__ bias, int relu, int symmetric, int qmin, int qmax,
     int is_signed, float eps, float half_range, int off, float* __restrict__ out) {
     extern __shared__ __attribute__((aligned(16))) int8_t dl_smem[];
-    __shared__ float s_sz[2];
     typedef int dl_v4i __attribute__((ext_vector_type(4)));
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int8_t* const codes = dl_smem;                                     // [16][K]: the block's rows
@@ -818,14 +982,11 @@ __global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
     for (int u = 0; u < kKeep; ++u)
         if (u * 1024 + tid < quads) mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
     m = mm_block_reduce(m);
-    if (tid == 0) {
-        const float qnan = __builtin_nanf("");
-        float s, z;
-        qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
-        s_sz[0] = s, s_sz[1] = z;
-    }
-    __syncthreads();
-    const float s = s_sz[0], z = s_sz[1], r = 1.0f / s;
+    // (every thread derives the qparams: cheaper than one thread, a barrier and a read)
+    const float qnan = __builtin_nanf("");
+    float s, z;
+    qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
+    const float r = 1.0f / s;
     const QuantizeOp<int8_t> op{x4, reinterpret_cast<Code8x4*>(codes), float(double(qmin)), float(double(qmax)), off};
 #pragma unroll
     for (int u = 0; u < kKeep; ++u) {
@@ -889,7 +1050,6 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     int symmetric, int qmin, int qmax, int is_signed, float eps, float half_range, int off, float* __restrict__ out,
     float* hid, int* counter) {
     extern __shared__ __attribute__((aligned(16))) int8_t mb_smem[];
-    __shared__ float s_sz[4];
     __shared__ int s_arrived;
     typedef int mb_v4i __attribute__((ext_vector_type(4)));
     typedef unsigned mb_v4u __attribute__((ext_vector_type(4)));
@@ -937,13 +1097,9 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     for (int u = 0; u < kKeep; ++u)
         if (u * 1024 + tid < quads) mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
     m = mm_block_reduce(m);
-    if (tid == 0) {
-        float s, z;
-        qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
-        s_sz[0] = s, s_sz[1] = z;
-    }
-    __syncthreads();
-    const float s = s_sz[0], z = s_sz[1], r = 1.0f / s;
+    float s, z;
+    qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
+    const float r = 1.0f / s;
     {
         const QuantizeOp<int8_t> op{x4, reinterpret_cast<Code8x4*>(codes), float(double(qmin)), float(double(qmax)), off};
 #pragma unroll
@@ -1031,14 +1187,9 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     MinMax tm{slot_lo, slot_hi, int((slot_lo != slot_lo) | (slot_hi != slot_hi))};
     if (tm.nan) tm.lo = __builtin_inff(), tm.hi = -__builtin_inff();
     tm = mm_block_reduce(tm);
-    if (tid == 0) {
-        float s2, z2;
-        qparams_of(tm.nan ? qnan : tm.lo, tm.nan ? qnan : tm.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s2, &z2);
-        s_sz[2] = s2, s_sz[3] = z2;
-        *counter = 0;  // ready for the next launch
-    }
-    __syncthreads();
-    const float s2 = s_sz[2], z2 = s_sz[3];
+    if (tid == 0) *counter = 0;  // ready for the next launch
+    float s2, z2;
+    qparams_of(tm.nan ? qnan : tm.lo, tm.nan ? qnan : tm.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s2, &z2);
     {
         const float r2 = 1.0f / s2;
         const QuantizeOp<int8_t> op{nullptr, reinterpret_cast<Code8x4*>(codes2), float(double(qmin)), float(double(qmax)), off};
@@ -1078,6 +1229,53 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     }
 }
 
+// Dynamic per-tensor quantization of n = rows * cols elements to rows of ld codes.
+int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int symmetric, int qmin, int qmax, int is_signed,
+                    float eps, int off, float* scale, float* zp, float* mn, float* mx, int8_t* q, hipStream_t st) {
+    const float half_range = float((double(qmax) - double(qmin)) / 2.0);
+    const bool ragged = ld != cols;
+    const size_t codes = ragged ? n / cols * ld : n;
+    const size_t blocks = codes ? (codes + kDynPerBlock - 1) / kDynPerBlock : 1;
+    LQ_REQUIRE((!ragged || blocks * kDynPerBlock < (size_t(1) << 32)) && blocks < 0x7fffffffull, LQ_ERR_SHAPE,
+               "dynamic quantization of %zu elements", n);
+    void* tmp = nullptr;
+    bool fresh = false;
+    if (blocks > 1) {
+        const int rc = stream_buffer(5, sizeof(DynScratch) + 2 * kMaxParts * sizeof(float), 0, st, &tmp, &fresh);
+        if (rc) return rc;
+    }
+    DynScratch* d = static_cast<DynScratch*>(tmp);
+    float* parts = reinterpret_cast<float*>(d + 1);
+    if (fresh) {
+        int rc = lq_fill_bytes(d, 0xff, sizeof(d->slot), reinterpret_cast<lq_stream>(st));
+        if (!rc) rc = lq_fill_bytes(&d->left, 0, sizeof(d->left), reinterpret_cast<lq_stream>(st));
+        if (rc) return rc;
+    }
+    auto launch = [&](auto kernel, const float* ranges, int n_ranges) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(kDynThreads), 0, st, x, n, cols, ld, symmetric, qmin, qmax,
+                           is_signed, eps, half_range, off, d, ranges, n_ranges, scale, zp, mn, mx, q);
+    };
+    if (blocks <= size_t(kExchange)) {
+        ragged ? launch(quantize_tensor_dynamic_kernel<false, true>, nullptr, 0)
+               : launch(quantize_tensor_dynamic_kernel<false, false>, nullptr, 0);
+        LQ_CHECK_LAUNCH("quantize_tensor_dynamic");
+        return LQ_OK;
+    }
+    // slices of at least 4096 elements
+    const unsigned splits = n < 4096 ? 1u : (n / 4096 < size_t(kMaxParts) ? unsigned(n / 4096) : unsigned(kMaxParts));
+    if (n % 4 == 0 && aligned16(x))
+        hipLaunchKernelGGL((minmax_seg_kernel<true>), dim3(splits), dim3(kThreads), 0, st, x, size_t(1), size_t(1), n, splits,
+                           parts, parts + splits);
+    else
+        hipLaunchKernelGGL((minmax_seg_kernel<false>), dim3(splits), dim3(kThreads), 0, st, x, size_t(1), size_t(1), n, splits,
+                           parts, parts + splits);
+    LQ_CHECK_LAUNCH("minmax_seg");
+    ragged ? launch(quantize_tensor_dynamic_kernel<true, true>, parts, int(splits))
+           : launch(quantize_tensor_dynamic_kernel<true, false>, parts, int(splits));
+    LQ_CHECK_LAUNCH("quantize_tensor_parts");
+    return LQ_OK;
+}
+
 }  // namespace
 
 namespace lq {
@@ -1098,11 +1296,48 @@ int lq_quantize_tensor_dynamic_i8(const float* x, size_t n, int symmetric, int q
     LQ_REQUIRE(n <= (size_t(1) << 18), LQ_ERR_NOT_IMPLEMENTED,
                "quantize_tensor_dynamic: the one-launch form is for tensors of up to 262144 elements (got %zu); "
                "use lq_minmax + lq_calc_qparams + lq_quantize", n);
+    return quantize_tensor(x, n, unsigned(n ? n : 1), unsigned(n ? n : 1), symmetric, qmin, qmax, is_signed, eps,
+                           code_offset, scale, zp, mn_out, mx_out, q, as_stream(stream));
+}
+
+int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw, int N, const float* w_scale,
+                          const int32_t* wsum, const float* bias, int relu, int symmetric, int qmin, int qmax,
+                          int is_signed, float eps, int code_offset, float* out, lq_stream stream) {
+    LQ_REQUIRE(M >= 0 && N >= 0 && K >= 0, LQ_ERR_SHAPE, "dynamic_linear: negative extent");
+    if (M == 0 || N == 0) return LQ_OK;
+    LQ_REQUIRE(out && w_scale && wsum && (K == 0 || (x && w)), LQ_ERR_VALUE, "dynamic_linear: NULL pointer");
+    LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
+               "dynamic_linear: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
+    LQ_REQUIRE(ldw >= K && ldw % 16 == 0 && (K == 0 || aligned16(w)), LQ_ERR_VALUE,
+               "dynamic_linear: weight rows of %d bytes for K = %d (a multiple of 16, zeros past K, 16-byte aligned)", ldw, K);
+    LQ_REQUIRE(ldw <= 131071, LQ_ERR_SHAPE, "dynamic_linear: K = %d overflows the int32 accumulator", K);
+    hipStream_t st = as_stream(stream);
     const float half_range = float((double(qmax) - double(qmin)) / 2.0);
-    hipLaunchKernelGGL(quantize_tensor_dynamic_kernel, dim3(1), dim3(1024), 0, as_stream(stream), x, n, symmetric,
-                       qmin, qmax, is_signed, eps, half_range, code_offset, scale, zp, mn_out, mx_out, q);
-    LQ_CHECK_LAUNCH("quantize_tensor_dynamic");
-    return LQ_OK;
+    const size_t n = size_t(M) * K;
+    if (M == 1 && K > 0 && K <= 16384) {
+        // every block quantizes the whole row: eight wavefronts, or four where that leaves CUs without a block
+        const int waves = (N + 31) / 32 < 256 ? 4 : 8;
+        hipLaunchKernelGGL(dynamic_gemv1_kernel, dim3(unsigned((N + 4 * waves - 1) / (4 * waves))), dim3(waves * 64),
+                           size_t((K + 4095) / 4096) * 4096, st, x, K, w, ldw, N, w_scale, wsum, bias, relu, symmetric, qmin,
+                           qmax, is_signed, eps, half_range, code_offset, out);
+        LQ_CHECK_LAUNCH("dynamic_gemv1");
+        return LQ_OK;
+    }
+    // codes (rows as long as the weight's), scale and zero point, then the GEMM
+    const size_t code_bytes = (size_t(M) * ldw + 255) / 256 * 256;
+    void* tmp = nullptr;
+    int rc = stream_buffer(6, code_bytes + 256, 0, st, &tmp, nullptr);
+    if (rc) return rc;
+    int8_t* codes = static_cast<int8_t*>(tmp);
+    float* qp = reinterpret_cast<float*>(codes + code_bytes);
+    rc = quantize_tensor(x, n, unsigned(K ? K : 1), unsigned(ldw ? ldw : 1), symmetric, qmin, qmax, is_signed, eps,
+                         code_offset, qp, qp + 1, qp + 2, qp + 3, codes, st);
+    if (rc) return rc;
+    GemmArgs g{};
+    g.a = codes, g.w = w, g.M = M, g.N = N, g.K = ldw;
+    g.wsum = wsum, g.a_zp = code_offset, g.a_zp_dev = qp + 1, g.a_scale = qp, g.w_scale = w_scale;
+    g.bias = bias, g.bias_dtype = LQ_F32, g.relu = relu, g.out_mode = OUT_F32, g.out = out, g.ldo = N, g.ldr = N;
+    return run_gemm(g, 0, 0, st);
 }
 
 int lq_dynamic_mlp2_small_f32(const float* x, int M, int K1, const int8_t* w1, int N1, const float* w1_scale,

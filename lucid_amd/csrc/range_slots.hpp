@@ -10,7 +10,7 @@
 // min and max are exact and order-independent, so the result is bit-identical
 // to a separate min / max pass.
 #pragma once
-#include "common.hpp"
+#include "wave_reduce.hpp"
 
 namespace lq {
 
@@ -21,23 +21,8 @@ constexpr int kRangeWords = 4 + 2 * kRangeSlots;
 // block's slot.  All threads of the block must call it; gridDim.x * gridDim.y
 // must not exceed kRangeSlots.
 __device__ __forceinline__ void range_block_store(float* range, float lo, float hi, int nan) {
-    __shared__ float s_lo[16], s_hi[16];
-    __shared__ int s_nan[16];
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        lo = fminf(lo, __shfl_xor(lo, d, 64));
-        hi = fmaxf(hi, __shfl_xor(hi, d, 64));
-        nan |= __shfl_xor(nan, d, 64);
-    }
-    const int wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-    if ((threadIdx.x & 63) == 0) s_lo[wave] = lo, s_hi[wave] = hi, s_nan[wave] = nan;
-    __syncthreads();
+    block_minmax(lo, hi, nan);
     if (threadIdx.x == 0) {
-        for (int w = 1; w < nw; ++w) {
-            lo = fminf(lo, s_lo[w]);
-            hi = fmaxf(hi, s_hi[w]);
-            nan |= s_nan[w];
-        }
         if (nan) lo = hi = __builtin_nanf("");
         const unsigned slot = blockIdx.y * gridDim.x + blockIdx.x;
         range[4 + slot] = lo;

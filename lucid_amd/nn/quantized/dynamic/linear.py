@@ -23,9 +23,18 @@ from ...module import Module
 from .._utils import forget_weight_zero_points, storage_offset, weight_zero_points
 
 
-# The one-launch kernel keeps 16 rows of activation codes (16 K bytes) plus 1 KiB of scratch in
-# the 96 KiB of LDS it may use: wider layers take the two-launch route, whatever the batch.
+# Rows of activation codes that fit the LDS of the one-launch kernel of small layers: wider layers
+# quantize in a launch of their own, whatever the batch.
 SMALL_LINEAR_MAX_K = 6080
+
+
+def _one_launch_pays(M: int, K: int, N: int) -> bool:
+    """Whether the one-launch kernel of a small layer beats quantizing (4 us) and multiplying (5 us and
+    up) in two.  Its blocks each take the range of all of x and quantize 16 rows: about 4 us + 0.043 us per
+    1000 activations + 2.4 us per 1000 of K, one round of 256 blocks.  Measured: 64 x 784 -> 256 8.0 us,
+    7 x 1024 -> 1024 7.2, 16 x 4096 -> 1024 16.5, 32 x 2048 -> 4096 (512 blocks) 22.7, 16 x 4096 -> 11008 48.5."""
+    return (1 < M <= 64 and K % 16 == 0 and 0 < K <= SMALL_LINEAR_MAX_K and M * K <= 65536
+            and ((M + 15) // 16) * ((N + 15) // 16) <= 256 and 43 * M * K + 2400 * K <= 6_000_000)
 
 
 def fused_pair(first, relu_between: bool, second, x):
@@ -79,12 +88,28 @@ class Linear(Module):
         self.register_buffer("bias", T.tensor(np.zeros(out_features, np.float32), device="hip")
                              if bias else None)
         self._wsum = None
+        self._wrows = None
 
     def _state_loaded(self, name: str) -> None:
         if name == "weight_int8":
-            self._wsum = None
+            self._wsum = self._wrows = None
         if name == "weight_zero_point":
             forget_weight_zero_points(self)
+
+    def _weight_rows(self) -> tuple[Tensor, int]:
+        """The weight codes in rows of a multiple of 16 bytes (``weight_int8`` itself where its rows are) and
+        that length; rows of a ragged layer are laid out once, with zeros behind them."""
+        if self._wrows is None:
+            N, K = self.out_features, self.in_features
+            if K % 16 == 0:
+                self._wrows = (self.weight_int8, K)
+            else:
+                ld = (K + 63) // 64 * 64
+                rows = Tensor.empty((N, ld), T.int8, "hip")
+                _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
+                _C.call("lq_d2d_rows", rows.data_ptr, ld, self.weight_int8.data_ptr, K, K, N, None)
+                self._wrows = (rows, ld)
+        return self._wrows
 
     def forward(self, x: Tensor, residual: Tensor | None = None, activation: str | None = None,
                 track_range: bool = False) -> Tensor:
@@ -104,17 +129,24 @@ class Linear(Module):
         M = x.numel // K
         qd = self.act_qdtype
         off = storage_offset(qd)
-        if (x._range is None and residual is None and activation is None and not track_range and 0 < M <= 64
-                and K % 16 == 0 and K <= SMALL_LINEAR_MAX_K and M * K <= 65536 and weight_zero_points(self) is None
-                and (self.bias is None or self.bias.dtype == T.float32)):
-            # a small activation: min / max, qparams, codes, GEMM and bias in one launch (same bits)
+        bias = self._buffers["bias"]
+        if (x._range is None and residual is None and activation is None and not track_range
+                and weight_zero_points(self) is None and (bias is None or bias.dtype == T.float32)):
+            # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
             if self._wsum is None:
                 self._wsum = _ops.rowsum_i8(self.weight_int8)
-            y = Tensor.empty((M, N), T.float32, "hip")
-            _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, self.weight_int8.data_ptr, N,
-                    self.weight_scale.data_ptr, self._wsum.data_ptr, None if self.bias is None else self.bias.data_ptr,
-                    0, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, off, y.data_ptr, None)
-            return y.reshape(*x.shape[:-1], N)
+            y = Tensor.empty((*x.shape[:-1], N), T.float32, "hip")
+            grid = (0, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, off)
+            scale, wsum = self._buffers["weight_scale"].data_ptr, self._wsum.data_ptr
+            b = None if bias is None else bias.data_ptr
+            if _one_launch_pays(M, K, N):
+                _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, self._buffers["weight_int8"].data_ptr, N, scale, wsum,
+                        b, *grid, y.data_ptr, None)
+            else:
+                w, ldw = self._weight_rows()
+                _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale, wsum, b, *grid,
+                        y.data_ptr if M else None, None)
+            return y
         xq = Tensor.empty((M, K), T.int8, "hip")
         small = x._range is None and x.numel <= (1 << 18)
         if small:

@@ -530,6 +530,39 @@ def test_dynamic_linear_wide_layer_at_small_batch(M, K):
                     -128, out.data_ptr, None)
 
 
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (1, 17, 1100), (1, 4095, 33), (1, 4097, 2100), (1, 16384, 7),  # a stream of the weight
+                                   (1, 16385, 40), (3, 5, 7), (2, 2731, 3), (2, 4097, 65),  # 1 and 2 blocks of 8192, ragged rows
+                                   (65, 126, 130), (100, 250, 257), (257, 8160, 65),  # all 256 blocks, and one too many
+                                   (520, 4096, 48), (419, 5011, 20)])
+@pytest.mark.parametrize("kind", ["normal", "constant", "nan"])
+def test_dynamic_linear_of_any_size(M, K, N, kind):
+    """One call for the layer, whatever its size, with the bits of the separate operators: min / max,
+    qparams, quantize and the GEMM.  Twice: the second launch finds the first one's scratch."""
+    import lucid_amd.nn.quantized.dynamic as nnqd
+    from lucid_amd import _ops
+    rng = np.random.default_rng(K + M + N)
+    lin = nnqd.Linear(K, N)
+    lin.weight_int8 = hip(rng.integers(-127, 128, (N, K)).astype(np.int8))
+    lin.weight_scale = hip(rng.uniform(0.001, 0.01, N).astype(np.float32))
+    lin.bias = hip(rng.standard_normal(N).astype(np.float32))
+    lin._state_loaded("weight_int8")
+    x = (rng.standard_normal((M, K)) * 2).astype(np.float32)
+    if kind == "constant":
+        x[:] = -0.25
+    elif kind == "nan":
+        x[M // 2, K // 3] = np.nan
+    for scale in (1.0, 0.5):
+        xd = hip(x * np.float32(scale))
+        got = lin(xd).numpy()
+        mn, mx = Q.minmax(xd)
+        s, z = Q.calculate_qparams(mn, mx, Q.per_tensor_affine, Q.quint8)
+        xq = L.tensor(np.ascontiguousarray(Q.quantize(xd, s, z, Q.quint8).numpy() - 128).astype(np.int8), device="hip")
+        want = _ops.qlinear_i8(xq, lin.weight_int8, a_zp=-128, a_zp_dev=z, a_scale=s, w_scale=lin.weight_scale,
+                               wsum=_ops.rowsum_i8(lin.weight_int8), bias=lin.bias, out_mode=_ops.OUT_F32).numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(got[~np.isnan(got)].view(np.uint32), want[~np.isnan(want)].view(np.uint32))
+
+
 class _recorded_calls:
     """The names of the compute entry points called through the binding while the block runs."""
 
