@@ -187,26 +187,33 @@ int lq_lstm_cell_f32(const float* gates_x, size_t gates_x_ld, const float* gates
                      const float* c_in, int batch, int hidden, float* h_out, float* c_out, float* y,
                      size_t y_ld, lq_stream stream);
 
-/* The recurrence of one LSTM layer with int8 recurrent weights over a whole sequence (one launch per
- * 16 batch rows that fit the device, all directions together; dynamic/rnn.py:66-84,
- * CpuBackend.h:13394-13519).  Gate order i, f, g, o:
- *   raw[t] = gates_x[t] + scale * (h[t-1] . codes) + (bias_ih + bias_hh)
+/* LSTM layers with int8 weights over a whole sequence (one launch per 16 batch rows that fit the device,
+ * all directions or stacked layers together; dynamic/rnn.py:66-84, CpuBackend.h:13394-13519).  Gate order
+ * i, f, g, o:
+ *   raw[t] = x[t] W_ih^T + scale * (h[t-1] . codes) + (bias_ih + bias_hh)
  *   c[t] = sigmoid(f)*c[t-1] + sigmoid(i)*tanh(g),  h[t] = sigmoid(o)*tanh(c[t])
  * Direction 1 walks the steps backwards.  Float32 arithmetic throughout: the codes enter exactly,
- * h as three bfloat16 parts. */
+ * h and x as three bfloat16 parts.  "Part": a direction of one layer, or one of the stacked layers
+ * (layers > 1: directions is 1 and x is given; layer k reads the output of layer k - 1). */
+#define LQ_LSTM_PARTS 4
 typedef struct lq_lstm_args {
-    const float* gates_x[2];    /* per direction: x W_ih^T of every step, [4*hidden] per (step, row) in the order of y */
-    const int8_t* w_hh[2];      /* [4*hidden, hidden] codes, symmetric */
-    const float* w_hh_scale[2]; /* [4*hidden] */
-    const float* bias_ih[2];    /* [4*hidden], or NULL together with bias_hh */
-    const float* bias_hh[2];
-    const float* h0;            /* [directions, batch, hidden], or NULL for zeros */
+    const float* gates_x[2];    /* x NULL: per direction, x W_ih^T of every step, [4*hidden] per (step, row) as in y */
+    const float* x;             /* [steps, batch, inputs], or [batch, steps, ...]: inputs, hidden at most 512 */
+    const int8_t* w_ih[LQ_LSTM_PARTS];    /* with x: [4*hidden, columns of the part's input] codes, symmetric */
+    const float* w_ih_scale[LQ_LSTM_PARTS];
+    const int8_t* w_hh[LQ_LSTM_PARTS];    /* [4*hidden, hidden] codes, symmetric */
+    const float* w_hh_scale[LQ_LSTM_PARTS]; /* [4*hidden] */
+    const float* bias_ih[LQ_LSTM_PARTS];  /* [4*hidden], or NULL together with bias_hh */
+    const float* bias_hh[LQ_LSTM_PARTS];
+    const float* h0;            /* [parts, batch, hidden], or NULL for zeros */
     const float* c0;
-    float* h_n;                 /* [directions, batch, hidden] */
+    float* h_n;                 /* [parts, batch, hidden] */
     float* c_n;
-    float* y;                   /* [steps, batch, directions*hidden], or [batch, steps, ...] when batch_first */
-    int steps, batch, hidden, directions, batch_first; /* hidden at most 1024 (LQ_ERR_NOT_IMPLEMENTED beyond) */
+    float* y[LQ_LSTM_PARTS];    /* per layer: [steps, batch, directions*hidden], or [batch, steps, ...] when batch_first */
+    int steps, batch, inputs, hidden, layers, directions, batch_first; /* hidden at most 1024 (LQ_ERR_NOT_IMPLEMENTED beyond) */
 } lq_lstm_args;
+/* How many of `layers` stacked layers the next call should take with x given (0: take gates_x). */
+int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layers, int directions, int* fused);
 int lq_lstm_sequence_f32(const lq_lstm_args* args, lq_stream stream);
 
 /* Self-test of the tile kernels' requantize arithmetic.  Their epilogue computes

@@ -238,12 +238,14 @@ class LstmArgs(C.Structure):
     """``lq_lstm_args`` of ``include/lucid_hip.h``."""
 
     _fields_ = [
-        ("gates_x", _vp * 2), ("w_hh", _vp * 2), ("w_hh_scale", _vp * 2), ("bias_ih", _vp * 2), ("bias_hh", _vp * 2),
-        ("h0", _vp), ("c0", _vp), ("h_n", _vp), ("c_n", _vp), ("y", _vp),
-        ("steps", _i), ("batch", _i), ("hidden", _i), ("directions", _i), ("batch_first", _i),
+        ("gates_x", _vp * 2), ("x", _vp), ("w_ih", _vp * 4), ("w_ih_scale", _vp * 4), ("w_hh", _vp * 4),
+        ("w_hh_scale", _vp * 4), ("bias_ih", _vp * 4), ("bias_hh", _vp * 4),
+        ("h0", _vp), ("c0", _vp), ("h_n", _vp), ("c_n", _vp), ("y", _vp * 4),
+        ("steps", _i), ("batch", _i), ("inputs", _i), ("hidden", _i), ("layers", _i), ("directions", _i), ("batch_first", _i),
     ]
 
 
+_SIGNATURES["lq_lstm_fused_layers"] = [_i] * 6 + [C.POINTER(_i)]
 _SIGNATURES["lq_lstm_sequence_f32"] = [C.POINTER(LstmArgs), _vp]
 _SIGNATURES["lq_qconv3d_i8"] = [C.POINTER(QConv3dArgs), _vp]
 _SIGNATURES["lq_quantize_nchw_to_nhwc"] = [_vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _vp]

@@ -1,11 +1,10 @@
-// The recurrence of a weight-only int8 LSTM layer over a whole sequence, in one launch.
+// Weight-only int8 LSTM layers over a whole sequence, in one launch.
 //
 //   raw[t] = x[t] W_ih^T + h[t-1] W_hh^T + (b_ih + b_hh)        gates i, f, g, o
 //   c[t] = sigmoid(f) c[t-1] + sigmoid(i) tanh(g),  h[t] = sigmoid(o) tanh(c[t])
 //
-// (lucid/nn/quantized/dynamic/rnn.py:66-84, CpuBackend.h:13394-13519).  The input products of all
-// steps are taken beforehand (`gx`); what is left is a chain of `steps` small dependent products,
-// so the time is the number of steps times the latency of one.
+// (lucid/nn/quantized/dynamic/rnn.py:66-84, CpuBackend.h:13394-13519).  A chain of `steps` small
+// dependent products: the time is the number of steps times the latency of one.
 //
 // Split.  A block keeps the recurrent weights of 16 hidden units (64 gate rows x hidden codes) in
 // registers for the whole sequence, as bfloat16 matrix operands: an int8 code is exact in bfloat16,
@@ -16,6 +15,13 @@
 // tiles, and the partial sums meet in LDS; wavefront w of the first four then finishes batch rows
 // 4 j + w of the 16 units, with c in registers.  ceil(hidden / 16) blocks serve 16 batch rows of one
 // direction; other rows and the other direction are independent groups in the same grid.
+//
+// Input.  Up to 512 columns a block also keeps the input weights of its units and takes the input product
+// of the next step while its h travels to the other blocks, where it costs nothing.  Stacked layers then
+// share the launch: layer k reads h[t] of layer k - 1 from that one's output as it appears, so L layers
+// take steps + L - 1 step times in place of L * steps.  The registers of the second weight halve the blocks
+// per CU; where that would mean more launches than it saves (lq_lstm_fused_layers), or beyond 512 columns,
+// the input products of all steps are taken beforehand (`gx`) and a layer is a launch of its own.
 //
 // Exchange.  h[t] is the layer's output, so the blocks of a group hand it to each other through y
 // itself: y is filled with a bit pattern no h can have (all ones, a NaN) before the launch, h is
@@ -28,8 +34,10 @@
 // larger batches run as several launches.  A wait is bounded besides: after kSpinLimit reads the
 // block stops waiting for the rest of the sequence and the output keeps its NaNs.
 //
-// hidden 512, 16 rows: 3.4 us per step on the MI355X, against 36 us for a float32 GEMM, a gate kernel and
-// the host's share of their launches per step.
+// hidden 512, 16 rows: 3.4 us per step with gx, 3.8 with the input product; two such layers of 64 steps
+// 272 us per call, against 580 us as two launches with a GEMM (43 us with the decoding of its weight) each
+// and 4.67 ms with a float32 GEMM, a gate kernel and the host's share of their launches per step.
+#include <type_traits>
 #include "common.hpp"
 
 using namespace lq;
@@ -47,20 +55,25 @@ constexpr unsigned kEmpty = 0xffffffffu;   // a word of y that has not been writ
 constexpr int kSpinLimit = 1 << 20;        // about a second of waiting for one step
 constexpr int kScopeDevice = 16;           // "sc1" cache-policy bit of buffer accesses
 
+constexpr int kParts = LQ_LSTM_PARTS;      // grid z: the directions of one layer, or stacked layers
+
 struct LstmArgs {
     const float* gx[2];
-    const int8_t* w[2];
-    const float* w_scale[2];
-    const float* b_ih[2];
-    const float* b_hh[2];
-    const float* h0;   // [dirs][B][H] or null (zeros), likewise c0
+    const float* x;              // input of part 0 (of every direction) where the kernel takes the input product
+    const int8_t* wx[kParts];
+    const float* wx_scale[kParts];
+    const int8_t* w[kParts];
+    const float* w_scale[kParts];
+    const float* b_ih[kParts];
+    const float* b_hh[kParts];
+    const float* h0;   // [parts][B][H] or null (zeros), likewise c0
     const float* c0;
-    float* h_n;        // [dirs][B][H]
+    float* h_n;        // [parts][B][H]
     float* c_n;
-    float* y;          // element (t, b, d * H + j) at t * y_step + b * y_row + d * H + j
-    long y_step, y_row, gx_step, gx_row;
-    long y_elems;
-    int T, B, H, row0, dir0;
+    float* y[kParts];  // element (t, b, col + j) at t * y_step + b * y_row + col + j; col = d * H in direction d
+    long y_step, y_row, gx_step, gx_row, x_step, x_row;
+    long y_elems, x_elems;
+    int T, B, H, I, row0, dir0, stacked;
 };
 
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
@@ -80,39 +93,104 @@ __device__ __forceinline__ uint32_t codes_bf16(int c0, int c1) {
 }
 __device__ __forceinline__ float sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-// W wavefronts, each with KPW steps of 32 hidden columns: hidden <= 32 W KPW.  The weights take 16 KPW
-// registers: KPW <= 2 fits four wavefronts per SIMD, KPW = 4 (hidden > 512) two.
-template <int W, int KPW>
-__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(KPW <= 2 ? 4 : 2, KPW <= 2 ? 4 : 2)))
+// the codes of one row of a weight at this lane's eight columns of an instruction, as bfloat16
+__device__ __forceinline__ v8bf load_codes(const int8_t* row, int k, int K) {
+    int c[8];
+    if (k + 8 <= K) {
+        uint64_t raw;
+        __builtin_memcpy(&raw, row + k, 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[e] = int(int8_t(raw >> (8 * e)));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[e] = k + e < K ? int(row[k + e]) : 0;
+    }
+    return __builtin_bit_cast(v8bf, v4u{codes_bf16(c[0], c[1]), codes_bf16(c[2], c[3]), codes_bf16(c[4], c[5]),
+                                        codes_bf16(c[6], c[7])});
+}
+// device-scope access to what follows element `at` of an array of `elems` floats
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t words_from(const float* base, long at, long elems) {
+    const long bytes = (elems - at) * 4;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + at, 0,
+                                             bytes < 0x7fffffffl ? int(bytes) : 0x7fffffff, 0x00020000);
+}
+template <int KP>
+__device__ __forceinline__ void load_columns(v4u (&raw)[KP][2], __amdgpu_buffer_rsrc_t src, unsigned off) {
+#pragma unroll
+    for (int i = 0; i < KP; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            raw[i][j] = __builtin_amdgcn_raw_buffer_load_b128(src, off + unsigned(i * 32 + j * 4) * 4, 0, kScopeDevice);
+}
+// columns from `left` on (of another direction, row or step) become zero; the largest word left
+template <int KP>
+__device__ __forceinline__ unsigned mask_columns(v4u (&raw)[KP][2], int left) {
+    unsigned worst = 0;
+#pragma unroll
+    for (int i = 0; i < KP; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (i * 32 + e >= left) raw[i][e >> 2][e & 3] = 0u;
+            worst = worst > raw[i][e >> 2][e & 3] ? worst : raw[i][e >> 2][e & 3];
+        }
+    return worst;
+}
+// acc[g] += columns . codes of gate g: three exact part products each
+template <int KP>
+__device__ __forceinline__ void multiply(v4f (&acc)[4], const v4u (&raw)[KP][2], const v8bf (&wf)[4][KP]) {
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+        v4u part3[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const v4u r = raw[i][e >> 1];
+            uint32_t hh, mm, ll;
+            split3(__uint_as_float(r[(2 * e) & 3]), __uint_as_float(r[(2 * e + 1) & 3]), hh, mm, ll);
+            part3[0][e] = hh, part3[1][e] = mm, part3[2][e] = ll;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, part3[q]), wf[g][i], acc[g], 0, 0, 0);
+    }
+}
+
+// W wavefronts, each with KPW instructions of 32 hidden columns (hidden <= 32 W KPW) and KX of 32 input
+// columns; KX = 0 reads the input products from gx.  The weights take 16 (KPW + KX) registers, which
+// decides how many wavefronts a SIMD holds.
+template <int W, int KPW, int KX>
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(KX == 0 && KPW <= 2 ? 4 : 2, KX == 0 && KPW <= 2 ? 4 : 2)))
 void lstm_sequence_kernel(LstmArgs p) {
     __shared__ float part[2][W][4][4][64];  // [step parity][wavefront][gate][row of the quad][lane]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ln = lane & 15, lq4 = lane >> 4;
-    const int d = p.dir0 + blockIdx.z, H = p.H;
+    const int z = p.dir0 + blockIdx.z, d = p.stacked ? 0 : z, H = p.H;
     const int u0 = blockIdx.x * kUnits, m0 = p.row0 + blockIdx.y * kRows;
+    float* const y = p.y[z];
 
-    // ---- the block's weights: tile g = gate g of units u0 .. u0+15, this wavefront's hidden columns
-    v8bf wf[4][KPW];
+    // ---- the block's weights: tile g = gate g of units u0 .. u0+15, this wavefront's columns
+    v8bf wf[4][KPW], wxf[4][KX > 0 ? KX : 1];
+    float scale_h[4], scale_x[4];  // of the unit whose products this lane accumulates
+    // ---- the input of this part: x, or the output of the layer below
+    const bool above = p.stacked && z > 0;
+    const float* const in = above ? p.y[above ? z - 1 : 0] : p.x;
+    const int I = above ? H : p.I;
+    const long in_step = above ? p.y_step : p.x_step, in_row = above ? p.y_row : p.x_row;
+    const long in_elems = above ? p.y_elems : p.x_elems;
+    const int kx_lane = wave * KX * 32 + lq4 * 8;
     {
         const int unit = u0 + ln < H ? u0 + ln : H - 1;  // units past H are computed and never stored
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int8_t* row = p.w[d] + (size_t(g) * H + unit) * H;
 #pragma unroll
-            for (int i = 0; i < KPW; ++i) {
-                const int k = (wave * KPW + i) * 32 + lq4 * 8;
-                int c[8];
-                if (k + 8 <= H) {
-                    uint64_t raw;
-                    __builtin_memcpy(&raw, row + k, 8);
+            for (int i = 0; i < KPW; ++i)
+                wf[g][i] = load_codes(p.w[z] + (size_t(g) * H + unit) * H, (wave * KPW + i) * 32 + lq4 * 8, H);
+            if constexpr (KX > 0) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) c[e] = int(int8_t(raw >> (8 * e)));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) c[e] = k + e < H ? int(row[k + e]) : 0;
-                }
-                wf[g][i] = __builtin_bit_cast(v8bf, v4u{codes_bf16(c[0], c[1]), codes_bf16(c[2], c[3]),
-                                                        codes_bf16(c[4], c[5]), codes_bf16(c[6], c[7])});
+                for (int i = 0; i < KX; ++i)
+                    wxf[g][i] = load_codes(p.wx[z] + (size_t(g) * H + unit) * I, kx_lane + i * 32, I);
+                scale_h[g] = p.w_scale[z][g * H + unit], scale_x[g] = p.wx_scale[z][g * H + unit];
             }
         }
     }
@@ -120,14 +198,14 @@ void lstm_sequence_kernel(LstmArgs p) {
     const int unit = u0 + ln, row = m0 + 4 * lq4 + wave;
     const bool mine = wave < 4 && unit < H && row < p.B;
     float ws[4], bias[4], c = 0.0f;
-    const size_t state = (size_t(d) * p.B + (row < p.B ? row : 0)) * H + unit;
+    const size_t state = (size_t(z) * p.B + (row < p.B ? row : 0)) * H + unit;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-        ws[g] = mine ? p.w_scale[d][g * H + unit] : 0.0f;
-        bias[g] = mine && p.b_ih[d] ? p.b_ih[d][g * H + unit] + p.b_hh[d][g * H + unit] : 0.0f;
+        ws[g] = KX > 0 ? 1.0f : mine ? p.w_scale[z][g * H + unit] : 0.0f;
+        bias[g] = mine && p.b_ih[z] ? p.b_ih[z][g * H + unit] + p.b_hh[z][g * H + unit] : 0.0f;
     }
     if (mine && p.c0) c = p.c0[state];
-    const float* gx_lane = p.gx[d] + size_t(mine ? row : 0) * p.gx_row + (mine ? unit : 0);
+    const float* gx_lane = KX > 0 ? nullptr : p.gx[d] + size_t(mine ? row : 0) * p.gx_row + (mine ? unit : 0);
     // ---- the row whose h this lane reads; rows past the batch repeat the last one
     const int hrow = m0 + ln < p.B ? m0 + ln : p.B - 1;
     const int k_lane = wave * KPW * 32 + lq4 * 8;
@@ -135,10 +213,39 @@ void lstm_sequence_kernel(LstmArgs p) {
     bool waiting = true;
     float hv = 0.0f;
 
+    // The input product of a step needs nothing of the step before it, so it is taken while the h of that
+    // step is on its way to the other blocks; its first read is issued before the gates are computed.
+    const unsigned x_off = unsigned(hrow * in_row + kx_lane) * 4;
+    v4u rx[KX > 0 ? KX : 1][2];
+    v4f accx[4];  // scaled
+    auto input_words = [&](int t) { return words_from(in, long(t) * in_step, in_elems); };
+    auto input_product = [&](int t) {
+        if constexpr (KX > 0) {
+            for (int spin = 0;; ++spin) {
+                const unsigned worst = mask_columns<KX>(rx, I - kx_lane);
+                if (!above || !waiting || __builtin_amdgcn_ballot_w64(worst == kEmpty) == 0) break;
+                if (spin >= kSpinLimit) waiting = false;
+                asm volatile("" ::: "memory");
+                load_columns<KX>(rx, input_words(t), x_off);
+            }
+#pragma unroll
+            for (int g = 0; g < 4; ++g) accx[g] = v4f{0.f, 0.f, 0.f, 0.f};
+            multiply<KX>(accx, rx, wxf);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) accx[g] *= scale_x[g];
+        }
+    };
+    if constexpr (KX > 0) {
+        const int t = d ? p.T - 1 : 0;
+        load_columns<KX>(rx, input_words(t), x_off);
+        input_product(t);
+    }
+
     for (int s = 0; s < p.T; ++s) {
         const int t = d ? p.T - 1 - s : s;
+        const int t_next = d ? t - 1 : t + 1;  // of the next step, if there is one
         float gx[4];
-        if (mine) {
+        if (KX == 0 && mine) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) gx[g] = gx_lane[size_t(t) * p.gx_step + size_t(g) * H];
         }
@@ -150,52 +257,30 @@ void lstm_sequence_kernel(LstmArgs p) {
                 for (int e = 0; e < 8; ++e) {
                     const int k = k_lane + i * 32 + e;
                     raw[i][e >> 2][e & 3] =
-                        p.h0 && k < H ? __float_as_uint(p.h0[(size_t(d) * p.B + hrow) * H + k]) : 0u;
+                        p.h0 && k < H ? __float_as_uint(p.h0[(size_t(z) * p.B + hrow) * H + k]) : 0u;
                 }
         } else {
-            const long at = long(d ? t + 1 : t - 1) * p.y_step + long(d) * H;
-            const long bytes = (p.y_elems - at) * 4;
-            const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
-                p.y + at, 0, bytes < 0x7fffffffl ? int(bytes) : 0x7fffffff, 0x00020000);
+            const __amdgpu_buffer_rsrc_t src =
+                words_from(y, long(d ? t + 1 : t - 1) * p.y_step + long(d) * H, p.y_elems);
             const unsigned off = unsigned(hrow * p.y_row + k_lane) * 4;
             for (int spin = 0;; ++spin) {
                 asm volatile("" ::: "memory");  // read again: the words change under the loop
-#pragma unroll
-                for (int i = 0; i < KPW; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        raw[i][j] = __builtin_amdgcn_raw_buffer_load_b128(src, off + unsigned(i * 32 + j * 4) * 4, 0, kScopeDevice);
-                unsigned worst = 0;
-#pragma unroll
-                for (int i = 0; i < KPW; ++i)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        // columns past H (of another direction, row or step) count as zero
-                        if (i * 32 + e >= left) raw[i][e >> 2][e & 3] = 0u;
-                        worst = worst > raw[i][e >> 2][e & 3] ? worst : raw[i][e >> 2][e & 3];
-                    }
+                load_columns<KPW>(raw, src, off);
+                const unsigned worst = mask_columns<KPW>(raw, left);
                 if (!waiting || __builtin_amdgcn_ballot_w64(worst == kEmpty) == 0) break;
                 if (spin >= kSpinLimit) waiting = false;
             }
         }
+        if constexpr (KX > 0) {
+            if (s + 1 < p.T) load_columns<KX>(rx, input_words(t_next), x_off);
+        }
         v4f acc[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) acc[g] = v4f{0.f, 0.f, 0.f, 0.f};
+        multiply<KPW>(acc, raw, wf);
+        if constexpr (KX > 0) {
 #pragma unroll
-        for (int i = 0; i < KPW; ++i) {
-            v4u part3[3];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const v4u r = raw[i][e >> 1];
-                uint32_t hh, mm, ll;
-                split3(__uint_as_float(r[(2 * e) & 3]), __uint_as_float(r[(2 * e + 1) & 3]), hh, mm, ll);
-                part3[0][e] = hh, part3[1][e] = mm, part3[2][e] = ll;
-            }
-#pragma unroll
-            for (int q = 0; q < 3; ++q)
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, part3[q]), wf[g][i], acc[g], 0, 0, 0);
+            for (int g = 0; g < 4; ++g) acc[g] = acc[g] * scale_h[g] + accx[g];
         }
         float(*const mine_part)[4][64] = part[s & 1][wave];
 #pragma unroll
@@ -211,7 +296,7 @@ void lstm_sequence_kernel(LstmArgs p) {
                 float sum = part[s & 1][0][g][wave][lane];
 #pragma unroll
                 for (int w = 1; w < W; ++w) sum += part[s & 1][w][g][wave][lane];
-                raw4[g] = mine ? (gx[g] + sum * ws[g]) + bias[g] : 0.0f;
+                raw4[g] = mine ? (KX > 0 ? sum : gx[g] + sum * ws[g]) + bias[g] : 0.0f;
             }
             const float ig = sigmoid(raw4[0]), fg = sigmoid(raw4[1]), gg = tanhf(raw4[2]), og = sigmoid(raw4[3]);
             c = fg * c + ig * gg;
@@ -219,13 +304,11 @@ void lstm_sequence_kernel(LstmArgs p) {
             if (mine) {
                 unsigned bits = __float_as_uint(hv);
                 bits = bits == kEmpty ? 0x7fc00000u : bits;  // a NaN, but not the one that means "not written"
-                const long at = long(t) * p.y_step + long(d) * H;
-                const long bytes = (p.y_elems - at) * 4;
-                const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(
-                    p.y + at, 0, bytes < 0x7fffffffl ? int(bytes) : 0x7fffffff, 0x00020000);
+                const __amdgpu_buffer_rsrc_t dst = words_from(y, long(t) * p.y_step + long(d) * H, p.y_elems);
                 __builtin_amdgcn_raw_buffer_store_b32(bits, dst, unsigned(row * p.y_row + unit) * 4, 0, kScopeDevice);
             }
         }
+        if (KX > 0 && s + 1 < p.T) input_product(t_next);
     }
     if (mine) {
         p.h_n[state] = hv;
@@ -233,8 +316,21 @@ void lstm_sequence_kernel(LstmArgs p) {
     }
 }
 
-template <int W, int KPW>
-int launch_lstm(LstmArgs p, int dirs, hipStream_t st) {
+// every word of the outputs "not written yet"
+__global__ __launch_bounds__(256) void lstm_empty_kernel(LstmArgs p) {
+    float* const y = p.y[blockIdx.y];
+    const long stride = long(gridDim.x) * 256;
+    for (long i = long(blockIdx.x) * 256 + threadIdx.x; i < p.y_elems; i += stride) y[i] = __uint_as_float(kEmpty);
+}
+
+// Launches of one kernel form: 16-row groups of one direction or of one stack, as many at once as may be.
+struct LstmSplit {
+    int per_group, groups, at_once, both;  // blocks of a group; groups; groups of a launch; its parts
+    int launches;
+};
+
+template <int W, int KPW, int KX>
+int split_lstm(int B, int H, int parts, bool stacked, LstmSplit* out) {
     static DeviceOnce once;
     static int capacity[32] = {0};  // blocks of this kernel the device holds at once
     int dev = 0;
@@ -242,67 +338,140 @@ int launch_lstm(LstmArgs p, int dirs, hipStream_t st) {
     const int rc = device_once(once, [&]() -> int {
         int per_cu = 0;
         hipDeviceProp_t prop;
-        LQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lstm_sequence_kernel<W, KPW>, W * 64, 0));
+        LQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lstm_sequence_kernel<W, KPW, KX>, W * 64, 0));
         LQ_HIP(hipGetDeviceProperties(&prop, dev));
         capacity[dev] = per_cu * prop.multiProcessorCount;
         return LQ_OK;
     });
     if (rc) return rc;
-    const int per_group = (p.H + kUnits - 1) / kUnits;
-    const int groups = (p.B + kRows - 1) / kRows;
-    int at_once = capacity[dev] / 4 / per_group;  // groups (16 rows of one direction) of a launch
-    LQ_REQUIRE(at_once >= 1, LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: hidden %d does not fit the device at once", p.H);
-    const int both = at_once >= dirs ? dirs : 1;
-    at_once = at_once / both < groups ? at_once / both : groups;
-    for (p.dir0 = 0; p.dir0 < dirs; p.dir0 += both)
-        for (int g = 0; g < groups; g += at_once) {
+    LstmSplit s;
+    s.per_group = (H + kUnits - 1) / kUnits;
+    s.groups = (B + kRows - 1) / kRows;
+    const int fit = capacity[dev] / 4 / s.per_group;
+    s.both = stacked || fit >= parts ? parts : 1;
+    s.at_once = fit / s.both < s.groups ? fit / s.both : s.groups;
+    s.launches = s.at_once < 1 ? 0 : (parts / s.both) * ((s.groups + s.at_once - 1) / s.at_once);
+    *out = s;
+    return LQ_OK;
+}
+
+template <int W, int KPW, int KX>
+int launch_lstm(LstmArgs p, int parts, hipStream_t st) {
+    LstmSplit s;
+    if (int rc = split_lstm<W, KPW, KX>(p.B, p.H, parts, p.stacked != 0, &s)) return rc;
+    LQ_REQUIRE(s.launches >= 1, LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: %d x hidden %d do not fit the device at once",
+               p.stacked ? parts : 1, p.H);
+    const int n_y = p.stacked ? parts : 1;
+    const long fill_blocks = (p.y_elems + 1023) / 1024;
+    hipLaunchKernelGGL(lstm_empty_kernel, dim3(unsigned(fill_blocks < 2048 ? fill_blocks : 2048), unsigned(n_y)), dim3(256),
+                       0, st, p);
+    LQ_CHECK_LAUNCH("lstm_empty");
+    for (p.dir0 = 0; p.dir0 < parts; p.dir0 += s.both)
+        for (int g = 0; g < s.groups; g += s.at_once) {
             p.row0 = g * kRows;
-            const int n = groups - g < at_once ? groups - g : at_once;
-            hipLaunchKernelGGL((lstm_sequence_kernel<W, KPW>), dim3(unsigned(per_group), unsigned(n), unsigned(both)),
+            const int n = s.groups - g < s.at_once ? s.groups - g : s.at_once;
+            hipLaunchKernelGGL((lstm_sequence_kernel<W, KPW, KX>), dim3(unsigned(s.per_group), unsigned(n), unsigned(s.both)),
                                dim3(W * 64), 0, st, p);
             LQ_CHECK_LAUNCH("lstm_sequence");
         }
     return LQ_OK;
 }
 
+// f(W, KPW, KX) for the form that serves `hidden` columns and `inputs` (0: gates_x).  More wavefronts
+// before more columns each: a wavefront's loads, splits and products are a serial chain.
+template <typename F>
+int with_form(int hidden, int inputs, F f) {
+    const int ks = (hidden + 31) / 32, kx = (inputs + 31) / 32;
+    using std::integral_constant;
+    if (kx == 0) {
+        if (ks <= 4) return f(integral_constant<int, 4>(), integral_constant<int, 1>(), integral_constant<int, 0>());
+        if (ks <= 8) return f(integral_constant<int, 8>(), integral_constant<int, 1>(), integral_constant<int, 0>());
+        if (ks <= 16) return f(integral_constant<int, 8>(), integral_constant<int, 2>(), integral_constant<int, 0>());
+        return f(integral_constant<int, 8>(), integral_constant<int, 4>(), integral_constant<int, 0>());
+    }
+    if (ks <= 4 && kx <= 4) return f(integral_constant<int, 4>(), integral_constant<int, 1>(), integral_constant<int, 1>());
+    if (ks <= 8)
+        return kx <= 8 ? f(integral_constant<int, 8>(), integral_constant<int, 1>(), integral_constant<int, 1>())
+                       : f(integral_constant<int, 8>(), integral_constant<int, 1>(), integral_constant<int, 2>());
+    return kx <= 8 ? f(integral_constant<int, 8>(), integral_constant<int, 2>(), integral_constant<int, 1>())
+                   : f(integral_constant<int, 8>(), integral_constant<int, 2>(), integral_constant<int, 2>());
+}
+constexpr int kMaxFused = 512;  // hidden and input columns of a form that takes the input product
+
 }  // namespace
 
 extern "C" {
+
+int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layers, int directions, int* fused) {
+    LQ_REQUIRE(fused, LQ_ERR_VALUE, "lstm_fused_layers: NULL pointer");
+    LQ_REQUIRE(steps >= 0 && batch >= 0 && inputs > 0 && hidden > 0 && layers > 0, LQ_ERR_SHAPE,
+               "lstm_fused_layers: bad extent (%d, %d, %d, %d, %d)", steps, batch, inputs, hidden, layers);
+    LQ_REQUIRE(directions == 1 || directions == 2, LQ_ERR_VALUE, "lstm_fused_layers: directions must be 1 or 2");
+    *fused = 0;
+    if (steps == 0 || batch == 0 || hidden > kMaxFused || inputs > kMaxFused) return LQ_OK;
+    // Costs per layer in steps of the recurrence.  An input product in a GEMM of its own, with the decoded
+    // weight it reads, is worth twelve (43 us at 1024 x 2048 x 512, a step 3.4).
+    constexpr long kGemm = 12;
+    LstmSplit s;
+    int rc = with_form(hidden, 0, [&](auto w, auto k, auto x) { return split_lstm<w(), k(), x()>(batch, hidden, directions, false, &s); });
+    if (rc) return rc;
+    double best = s.launches ? double(s.launches) * steps + kGemm * directions : 1e30;
+    for (int n = 1; n <= (directions == 1 ? (layers < kParts ? layers : kParts) : 1); ++n) {
+        const int columns = n > 1 && hidden > inputs ? hidden : inputs;
+        rc = with_form(hidden, columns, [&](auto w, auto k, auto x) {
+            return split_lstm<w(), k(), x()>(batch, hidden, directions == 2 ? 2 : n, n > 1, &s);
+        });
+        if (rc) return rc;
+        const double cost = double(s.launches) * (steps + n - 1) / n;
+        if (s.launches && cost < best) best = cost, *fused = n;
+    }
+    return LQ_OK;
+}
 
 int lq_lstm_sequence_f32(const lq_lstm_args* a, lq_stream stream) {
     LQ_REQUIRE(a, LQ_ERR_VALUE, "lstm_sequence: args is NULL");
     LQ_REQUIRE(a->steps >= 0 && a->batch >= 0 && a->hidden > 0, LQ_ERR_SHAPE, "lstm_sequence: bad extent (%d, %d, %d)",
                a->steps, a->batch, a->hidden);
     LQ_REQUIRE(a->directions == 1 || a->directions == 2, LQ_ERR_VALUE, "lstm_sequence: directions must be 1 or 2");
+    LQ_REQUIRE(a->layers >= 1 && a->layers <= kParts && (a->layers == 1 || (a->directions == 1 && a->x)), LQ_ERR_VALUE,
+               "lstm_sequence: %d layers, 1 or (one direction, input product taken here) at most %d", a->layers, kParts);
     LQ_REQUIRE(a->hidden <= 1024, LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: hidden %d, at most 1024", a->hidden);
+    LQ_REQUIRE(!a->x || (a->inputs > 0 && a->inputs <= kMaxFused && a->hidden <= kMaxFused), LQ_ERR_NOT_IMPLEMENTED,
+               "lstm_sequence: input product of %d columns for hidden %d, at most %d", a->inputs, a->hidden, kMaxFused);
     if (a->steps == 0 || a->batch == 0) return LQ_OK;
-    LQ_REQUIRE(a->y && a->h_n && a->c_n, LQ_ERR_VALUE, "lstm_sequence: NULL output pointer");
+    LQ_REQUIRE(a->h_n && a->c_n, LQ_ERR_VALUE, "lstm_sequence: NULL output pointer");
     LstmArgs p{};
-    for (int d = 0; d < a->directions; ++d) {
-        LQ_REQUIRE(a->gates_x[d] && a->w_hh[d] && a->w_hh_scale[d], LQ_ERR_VALUE, "lstm_sequence: NULL operand");
-        LQ_REQUIRE((a->bias_ih[d] == nullptr) == (a->bias_hh[d] == nullptr), LQ_ERR_VALUE,
+    p.stacked = a->layers > 1;
+    const int parts = p.stacked ? a->layers : a->directions;
+    for (int z = 0; z < parts; ++z) {
+        if (!a->x) {
+            LQ_REQUIRE(a->gates_x[z], LQ_ERR_VALUE, "lstm_sequence: NULL operand");
+            p.gx[z] = a->gates_x[z];
+        } else {
+            LQ_REQUIRE(a->w_ih[z] && a->w_ih_scale[z], LQ_ERR_VALUE, "lstm_sequence: NULL operand");
+        }
+        LQ_REQUIRE(a->w_hh[z] && a->w_hh_scale[z], LQ_ERR_VALUE, "lstm_sequence: NULL operand");
+        LQ_REQUIRE((a->bias_ih[z] == nullptr) == (a->bias_hh[z] == nullptr), LQ_ERR_VALUE,
                    "lstm_sequence: one of the two biases is NULL");
-        p.gx[d] = a->gates_x[d], p.w[d] = a->w_hh[d], p.w_scale[d] = a->w_hh_scale[d];
-        p.b_ih[d] = a->bias_ih[d], p.b_hh[d] = a->bias_hh[d];
+        p.y[z] = a->y[p.stacked ? z : 0];
+        LQ_REQUIRE(p.y[z], LQ_ERR_VALUE, "lstm_sequence: NULL output pointer");
+        p.wx[z] = a->w_ih[z], p.wx_scale[z] = a->w_ih_scale[z];
+        p.w[z] = a->w_hh[z], p.w_scale[z] = a->w_hh_scale[z];
+        p.b_ih[z] = a->bias_ih[z], p.b_hh[z] = a->bias_hh[z];
     }
-    p.h0 = a->h0, p.c0 = a->c0, p.h_n = a->h_n, p.c_n = a->c_n, p.y = a->y;
+    p.x = a->x, p.I = a->inputs;
+    p.h0 = a->h0, p.c0 = a->c0, p.h_n = a->h_n, p.c_n = a->c_n;
     p.T = a->steps, p.B = a->batch, p.H = a->hidden;
     const long width = long(a->directions) * p.H, gates = 4L * p.H;
     p.y_step = a->batch_first ? width : p.B * width, p.y_row = a->batch_first ? p.T * width : width;
     p.gx_step = a->batch_first ? gates : p.B * gates, p.gx_row = a->batch_first ? p.T * gates : gates;
-    p.y_elems = long(p.T) * p.B * width;
+    p.x_step = a->batch_first ? p.I : long(p.B) * p.I, p.x_row = a->batch_first ? long(p.T) * p.I : p.I;
+    p.y_elems = long(p.T) * p.B * width, p.x_elems = long(p.T) * p.B * p.I;
     // an element is addressed as a 32-bit byte offset from its step's first
-    LQ_REQUIRE((p.B - 1) * p.y_row + width < 0x7fffffffL / 4, LQ_ERR_NOT_IMPLEMENTED,
-               "lstm_sequence: output of %ld elements is too large", p.y_elems);
-    hipStream_t st = as_stream(stream);
-    const int rc = lq_fill_bytes(a->y, 0xff, size_t(p.y_elems) * 4, stream);
-    if (rc) return rc;
-    const int ksteps = (p.H + 31) / 32;
-    // more wavefronts before more columns each: a wavefront's loads, splits and products are a serial chain
-    if (ksteps <= 4) return launch_lstm<4, 1>(p, a->directions, st);
-    if (ksteps <= 8) return launch_lstm<8, 1>(p, a->directions, st);
-    if (ksteps <= 16) return launch_lstm<8, 2>(p, a->directions, st);
-    return launch_lstm<8, 4>(p, a->directions, st);
+    LQ_REQUIRE((p.B - 1) * p.y_row + width < 0x7fffffffL / 4 && (p.B - 1) * p.x_row + p.I < 0x7fffffffL / 4,
+               LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: %ld outputs or %ld inputs are too many", p.y_elems, p.x_elems);
+    const int columns = !a->x ? 0 : p.stacked && p.H > p.I ? p.H : p.I;
+    return with_form(p.H, columns, [&](auto w, auto k, auto x) { return launch_lstm<w(), k(), x()>(p, parts, as_stream(stream)); });
 }
 
 }  // extern "C"

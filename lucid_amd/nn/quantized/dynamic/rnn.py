@@ -5,9 +5,10 @@ stored as ``<name>_int8`` codes with a per-row ``<name>_scale`` (symmetric, zero
 (``CpuBackend.h:13394-13519``: gates i, f, g, o; ``raw = x W_ih^T + h W_hh^T + (b_ih +
 b_hh)``).
 
-On the device the input product of a layer is taken once over all time steps
-(float32 MFMA GEMM), then the recurrence of all steps and directions is one launch
-(``lq_lstm_sequence_f32``).  Packed sequences, projections and hidden sizes beyond 1024
+On the device the recurrence of all steps and directions is one launch
+(``lq_lstm_sequence_f32``), which takes the input products and the layers stacked on top of the
+first as well where they fit; else the input product of a layer is taken over all time steps
+beforehand (float32 MFMA GEMM).  Packed sequences, projections and hidden sizes beyond 1024
 take a recurrent GEMM and a gate kernel per step instead.
 """
 
@@ -181,26 +182,38 @@ class LSTM(Module):
         return PackedSequence(out, packed.batch_sizes, packed.sorted_indices, packed.unsorted_indices), (h_n, c_n)
 
     def _forward_sequences(self, x, h0, c0, h_n, c_n, Tn, Bn):
-        """Whole sequences, one launch per layer for the recurrence; fills ``h_n`` / ``c_n``."""
+        """Whole sequences, one launch for the recurrence of a layer or of several stacked ones; fills
+        ``h_n`` / ``c_n``."""
         H, dirs = self.hidden_size, 2 if self.bidirectional else 1
         bufs, state = self._buffers, Bn * H * 4
-        for k in range(self.num_layers):
-            y = Tensor.empty((Bn, Tn, dirs * H) if self.batch_first else (Tn, Bn, dirs * H), T.float32, "hip")
+        shape = (Bn, Tn, dirs * H) if self.batch_first else (Tn, Bn, dirs * H)
+        fused, k = C.c_int(), 0
+        while k < self.num_layers:
+            _C.call("lq_lstm_fused_layers", Tn, Bn, x.shape[2], H, self.num_layers - k, dirs, C.byref(fused))
+            layers = max(1, fused.value)
             a = _C.LstmArgs()
+            a.inputs, a.x = x.shape[2], x.data_ptr if fused.value else None
+            ys = [Tensor.empty(shape, T.float32, "hip") for _ in range(layers)]
             gates = []
-            for d, suffix in enumerate(("", "_reverse")[:dirs]):
-                name = f"l{k}{suffix}"
-                gates.append(linear_f32(x, self._weight("weight_ih_" + name)))
-                a.gates_x[d] = gates[-1].data_ptr
-                a.w_hh[d], a.w_hh_scale[d] = bufs[f"weight_hh_{name}_int8"].data_ptr, bufs[f"weight_hh_{name}_scale"].data_ptr
+            for z in range(layers * dirs):  # one of the two is 1
+                name = f"l{k + z}" if dirs == 1 else f"l{k}" + ("", "_reverse")[z]
+                if fused.value:
+                    a.w_ih[z], a.w_ih_scale[z] = (bufs[f"weight_ih_{name}_{v}"].data_ptr for v in ("int8", "scale"))
+                else:
+                    gates.append(linear_f32(x, self._weight("weight_ih_" + name)))
+                    a.gates_x[z] = gates[-1].data_ptr
+                a.w_hh[z], a.w_hh_scale[z] = (bufs[f"weight_hh_{name}_{v}"].data_ptr for v in ("int8", "scale"))
                 if self.bias:
-                    a.bias_ih[d], a.bias_hh[d] = bufs["bias_ih_" + name].data_ptr, bufs["bias_hh_" + name].data_ptr
+                    a.bias_ih[z], a.bias_hh[z] = bufs["bias_ih_" + name].data_ptr, bufs["bias_hh_" + name].data_ptr
+            for z, y in enumerate(ys):
+                a.y[z] = y.data_ptr
             at = k * dirs * state
             a.h0, a.c0 = (None, None) if h0 is None else (h0.data_ptr + at, c0.data_ptr + at)
-            a.h_n, a.c_n, a.y = h_n.data_ptr + at, c_n.data_ptr + at, y.data_ptr
+            a.h_n, a.c_n = h_n.data_ptr + at, c_n.data_ptr + at
             a.steps, a.batch, a.hidden, a.directions, a.batch_first = Tn, Bn, H, dirs, int(self.batch_first)
+            a.layers = layers
             _C.call("lq_lstm_sequence_f32", C.byref(a), None)
-            x = y
+            x, k = ys[-1], k + layers
         return x
 
     @classmethod

@@ -312,6 +312,27 @@ def test_dynamic_lstm_sequence_sizes(I, H, Bn, Tn, bidir, batch_first):
         del y, hn, cn
 
 
+@pytest.mark.parametrize("I,H,layers,Bn,Tn,bidir,batch_first",
+                         [(3, 1, 2, 1, 3, False, False), (130, 17, 3, 5, 4, False, True), (500, 129, 5, 33, 2, False, False),
+                          (100, 300, 2, 16, 5, False, True), (512, 512, 2, 17, 4, False, False), (257, 250, 2, 18, 3, True, True),
+                          (513, 64, 2, 3, 3, False, False), (64, 500, 2, 64, 3, False, False)])
+def test_dynamic_lstm_stack_sizes(I, H, layers, Bn, Tn, bidir, batch_first):
+    """The input product taken inside the recurrence and layers handing h to each other, at the edges of
+    both column splits (the input's and the hidden one), past the layers and rows of one launch and on
+    either side of the widest input it takes.  Bound as above, a layer's error passing through the next."""
+    rng = np.random.default_rng(I + H)
+    qm = Q.quantize_dynamic(nn.LSTM(I, H, num_layers=layers, batch_first=batch_first, bidirectional=bidir))
+    x = rng.standard_normal((Bn, Tn, I) if batch_first else (Tn, Bn, I)).astype(np.float32)
+    hx = tuple(rng.standard_normal((layers * (2 if bidir else 1), Bn, H)).astype(np.float32) for _ in range(2))
+    xd, hd = hip(x), tuple(hip(v) for v in hx)
+    want = _oracle_lstm_stack(qm, x, hx, batch_first)
+    for _ in range(2):
+        y, (hn, cn) = qm(xd, hd)
+        for got, ref in zip((y, hn, cn), want):
+            assert np.abs(got.numpy() - ref).max() < layers * 7 * (H + max(I, 2 * H)) ** 0.5 * 2.0 ** -24 * 8
+        del y, hn, cn
+
+
 def _deq(q, name):
     return (getattr(q, name + "_int8").numpy().astype(np.float32) *
             getattr(q, name + "_scale").numpy()[:, None]).astype(np.float32)
