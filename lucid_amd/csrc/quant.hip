@@ -63,21 +63,23 @@ __device__ __forceinline__ float clamp_code(float r, float z, float lo, float hi
     return (u < lo) ? lo : ((u > hi) ? hi : u);
 }
 
-// four quotients at once; `r` is fl(1/s), uniform over the block
-__device__ __forceinline__ float4 rint_div4(float4 v, float s, float r) {
-    float4 t = {v.x * r, v.y * r, v.z * r, v.w * r};
+// four quotients at once; `r` is fl(1/s)
+__device__ __forceinline__ float4 rint_div4(float4 v, float4 s, float4 r) {
+    float4 t = {v.x * r.x, v.y * r.y, v.z * r.z, v.w * r.w};
     float4 n = {__builtin_rintf(t.x), __builtin_rintf(t.y), __builtin_rintf(t.z), __builtin_rintf(t.w)};
     // branch-free conjunction: the four tests are evaluated unconditionally
     const bool ok = (int(rint_quotient_safe(t.x, n.x)) & int(rint_quotient_safe(t.y, n.y)) &
                      int(rint_quotient_safe(t.z, n.z)) & int(rint_quotient_safe(t.w, n.w))) != 0;
     if (__builtin_expect(!ok, 0)) {
-        n.x = __builtin_rintf(v.x / s);
-        n.y = __builtin_rintf(v.y / s);
-        n.z = __builtin_rintf(v.z / s);
-        n.w = __builtin_rintf(v.w / s);
+        n.x = __builtin_rintf(v.x / s.x);
+        n.y = __builtin_rintf(v.y / s.y);
+        n.z = __builtin_rintf(v.z / s.z);
+        n.w = __builtin_rintf(v.w / s.w);
     }
     return n;
 }
+
+__device__ __forceinline__ float4 splat(float v) { return float4{v, v, v, v}; }
 
 struct alignas(4) Code8x4 {
     int8_t v[4];
@@ -133,16 +135,19 @@ struct QuantizeOp {
     int off;
     __device__ __forceinline__ In load(size_t i) const { return nt_load(&x[i]); }
     static constexpr int kMaxU = 2;  // loads in flight per lane; measured best for 4 B in / 1 B out
-    __device__ __forceinline__ Vec pack(In v, float s, float z, float r) const {
+    __device__ __forceinline__ Vec pack(In v, float4 s, float4 z, float4 r) const {
         const float4 n = rint_div4(v, s, r);
         Vec o;
-        o.v[0] = CodeT(to_code(clamp_code(n.x, z, lo, hi)) + off);
-        o.v[1] = CodeT(to_code(clamp_code(n.y, z, lo, hi)) + off);
-        o.v[2] = CodeT(to_code(clamp_code(n.z, z, lo, hi)) + off);
-        o.v[3] = CodeT(to_code(clamp_code(n.w, z, lo, hi)) + off);
+        o.v[0] = CodeT(to_code(clamp_code(n.x, z.x, lo, hi)) + off);
+        o.v[1] = CodeT(to_code(clamp_code(n.y, z.y, lo, hi)) + off);
+        o.v[2] = CodeT(to_code(clamp_code(n.z, z.z, lo, hi)) + off);
+        o.v[3] = CodeT(to_code(clamp_code(n.w, z.w, lo, hi)) + off);
         return o;
     }
-    __device__ __forceinline__ void store(size_t i, In v, float s, float z, float r) const {
+    __device__ __forceinline__ Vec pack(In v, float s, float z, float r) const {
+        return pack(v, splat(s), splat(z), splat(r));
+    }
+    __device__ __forceinline__ void store(size_t i, In v, float4 s, float4 z, float4 r) const {
         nt_store(&q[i], pack(v, s, z, r));
     }
     // scalar tail / generic path
@@ -162,12 +167,12 @@ struct DequantizeOp {
     float4* __restrict__ out;
     int off;
     __device__ __forceinline__ In load(size_t i) const { return nt_load(&q[i]); }
-    __device__ __forceinline__ void store(size_t i, In v, float s, float z, float) const {
+    __device__ __forceinline__ void store(size_t i, In v, float4 s, float4 z, float4) const {
         float4 o;
-        o.x = (float(int(v.v[0]) - off) - z) * s;
-        o.y = (float(int(v.v[1]) - off) - z) * s;
-        o.z = (float(int(v.v[2]) - off) - z) * s;
-        o.w = (float(int(v.v[3]) - off) - z) * s;
+        o.x = (float(int(v.v[0]) - off) - z.x) * s.x;
+        o.y = (float(int(v.v[1]) - off) - z.y) * s.y;
+        o.z = (float(int(v.v[2]) - off) - z.z) * s.z;
+        o.w = (float(int(v.v[3]) - off) - z.w) * s.w;
         nt_store(&out[i], o);
     }
     __device__ __forceinline__ void scalar(size_t e, float s, float z) const {
@@ -184,13 +189,13 @@ struct FakeQuantizeOp {
     float4* __restrict__ out;
     float lo, hi;
     __device__ __forceinline__ In load(size_t i) const { return nt_load(&x[i]); }
-    __device__ __forceinline__ void store(size_t i, In v, float s, float z, float r) const {
+    __device__ __forceinline__ void store(size_t i, In v, float4 s, float4 z, float4 r) const {
         const float4 n = rint_div4(v, s, r);
         float4 o;
-        o.x = (clamp_code(n.x, z, lo, hi) - z) * s;
-        o.y = (clamp_code(n.y, z, lo, hi) - z) * s;
-        o.z = (clamp_code(n.z, z, lo, hi) - z) * s;
-        o.w = (clamp_code(n.w, z, lo, hi) - z) * s;
+        o.x = (clamp_code(n.x, z.x, lo, hi) - z.x) * s.x;
+        o.y = (clamp_code(n.y, z.y, lo, hi) - z.y) * s.y;
+        o.z = (clamp_code(n.z, z.z, lo, hi) - z.z) * s.z;
+        o.w = (clamp_code(n.w, z.w, lo, hi) - z.w) * s.w;
         nt_store(&out[i], o);
     }
     __device__ __forceinline__ void scalar(size_t e, float s, float z) const {
@@ -209,8 +214,9 @@ struct QParams {
 // One block = one chunk of U*256 quads inside one [outer][C] segment, so the
 // (scale, zero_point) pair is uniform across the block.  All U loads are
 // issued before the first store.
+// `tail` elements (a single segment only) behind its last quad are left to the first block.
 template <typename Op, int U>
-__global__ __launch_bounds__(kThreads) void seg_kernel(Op op, size_t inner4,
+__global__ __launch_bounds__(kThreads) void seg_kernel(Op op, size_t inner4, unsigned tail,
                                                        unsigned chunks_per_seg, size_t C,
                                                        QParams qp) {
     const size_t seg = blockIdx.x / chunks_per_seg;
@@ -225,6 +231,7 @@ __global__ __launch_bounds__(kThreads) void seg_kernel(Op op, size_t inner4,
         z = qp.z_host;
     }
     const float r = 1.0f / s;  // once per lane; the per-element quotients use it under a guard
+    if (blockIdx.x == 0 && threadIdx.x < tail) op.scalar(inner4 * 4 + threadIdx.x, s, z);
     const size_t base = seg * inner4;
     const size_t i0 = size_t(chunk) * (U * kThreads) + threadIdx.x;
     typename Op::In v[U];
@@ -232,7 +239,7 @@ __global__ __launch_bounds__(kThreads) void seg_kernel(Op op, size_t inner4,
 #pragma unroll
         for (int j = 0; j < U; ++j) v[j] = op.load(base + i0 + size_t(j) * kThreads);
 #pragma unroll
-        for (int j = 0; j < U; ++j) op.store(base + i0 + size_t(j) * kThreads, v[j], s, z, r);
+        for (int j = 0; j < U; ++j) op.store(base + i0 + size_t(j) * kThreads, v[j], splat(s), splat(z), splat(r));
         return;
     }
 #pragma unroll
@@ -243,12 +250,70 @@ __global__ __launch_bounds__(kThreads) void seg_kernel(Op op, size_t inner4,
 #pragma unroll
     for (int j = 0; j < U; ++j) {
         size_t i = i0 + size_t(j) * kThreads;
-        if (i < inner4) op.store(base + i, v[j], s, z, r);
+        if (i < inner4) op.store(base + i, v[j], splat(s), splat(z), splat(r));
     }
 }
 
-// Any shape, any alignment: one element per thread, channel looked up per
-// element.  Used for small or oddly shaped tensors (e.g. a 7x7x3 kernel).
+// floor(n / d) for n < 2^31: one multiplication by ceil(2^(31 + l) / d), 2^(l-1) < d <= 2^l
+struct FastDiv {
+    unsigned d, m;
+    int shift;
+    explicit FastDiv(unsigned div) : d(div), m(0), shift(31) {
+        int l = 0;
+        while ((1ull << l) < div) ++l;
+        shift = 31 + l;
+        m = unsigned(((1ull << shift) + div - 1) / div);
+    }
+    __device__ __forceinline__ unsigned operator()(unsigned n) const { return unsigned((uint64_t(n) * m) >> shift); }
+};
+
+// Segments that no block can have to itself (short, or not whole quads; the channel-last layouts among them): quads
+// of consecutive elements whatever segment they are of, with the channel found per quad and carried from element to
+// element.  CHANNELS: most channels a quad can be of - 2 where a segment is at least 4 elements, 4 below.  As
+// elements on generic_kernel, a lane did a 64-bit division and an IEEE division for each 4 bytes it moved.
+// (The address arithmetic still is what bounds it with 4 channels, memory with 2.)
+template <typename Op, int U, int CHANNELS>
+__global__ __launch_bounds__(kThreads) void flat_kernel(Op op, unsigned n, FastDiv inner, FastDiv C, QParams qp) {
+    const unsigned n4 = n / 4, i0 = blockIdx.x * unsigned(U * kThreads) + threadIdx.x;
+    typename Op::In v[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const unsigned i = i0 + j * kThreads;
+        v[j] = op.load(i < n4 ? i : n4 - 1);
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const unsigned i = i0 + j * kThreads;
+        if (i >= n4) break;
+        unsigned seg = inner(i * 4), at = i * 4 - seg * inner.d, c = seg - C(seg) * C.d;
+        float s[4], z[4], r[4];
+        if constexpr (CHANNELS == 2) {
+            const unsigned next = c + 1 == C.d ? 0 : c + 1, left = inner.d - at;
+            const float s0 = qp.scale[c], z0 = qp.zp[c], s1 = qp.scale[next], z1 = qp.zp[next];
+            const float r0 = 1.0f / s0, r1 = 1.0f / s1;
+#pragma unroll
+            for (unsigned e = 0; e < 4; ++e) s[e] = e < left ? s0 : s1, z[e] = e < left ? z0 : z1, r[e] = e < left ? r0 : r1;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s[e] = qp.scale[c], z[e] = qp.zp[c];
+                const bool wrap = ++at == inner.d;
+                at = wrap ? 0 : at;
+                c = wrap ? (c + 1 == C.d ? 0 : c + 1) : c;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = 1.0f / s[e];
+        }
+        op.store(i, v[j], float4{s[0], s[1], s[2], s[3]}, float4{z[0], z[1], z[2], z[3]}, float4{r[0], r[1], r[2], r[3]});
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n % 4) {
+        const unsigned e = n4 * 4 + threadIdx.x, seg = inner(e), c = seg - C(seg) * C.d;
+        op.scalar(e, qp.scale[c], qp.zp[c]);
+    }
+}
+
+// Any shape, any alignment: one element per thread, channel looked up per element.  For tensors
+// whose first element is not aligned, and 2^31 elements and more of short segments.
 template <typename Op>
 __global__ __launch_bounds__(kThreads) void generic_kernel(Op op, size_t n, size_t C, size_t inner,
                                                            QParams qp) {
@@ -273,8 +338,10 @@ int launch_elementwise(Op op, size_t outer, size_t C, size_t inner, QParams qp, 
                        hipStream_t st, const char* name) {
     const size_t n = outer * C * inner;
     if (n == 0) return LQ_OK;
-    const size_t segs = outer * C;
-    if (vec_ok && inner % 4 == 0 && inner >= 256) {
+    size_t segs = outer * C;
+    if (C == 1) segs = 1, inner = n;  // one (scale, zero_point): one run, whatever its shape
+    const size_t tail = C == 1 ? n % 4 : 0;
+    if (vec_ok && inner >= 256 && inner % 4 == tail) {
         const size_t inner4 = inner / 4;
         int U = inner4 >= 8 * kThreads ? 8 : (inner4 >= 4 * kThreads ? 4 : (inner4 >= 2 * kThreads ? 2 : 1));
         if (U > Op::kMaxU) U = Op::kMaxU;
@@ -285,11 +352,19 @@ int launch_elementwise(Op op, size_t outer, size_t C, size_t inner, QParams qp, 
                    "%s: tensor too large for one launch (%zu blocks)", name, blocks);
         dim3 grid{unsigned(blocks)}, block{kThreads};
         switch (U) {
-        case 8: hipLaunchKernelGGL((seg_kernel<Op, 8>), grid, block, 0, st, op, inner4, unsigned(chunks), C, qp); break;
-        case 4: hipLaunchKernelGGL((seg_kernel<Op, 4>), grid, block, 0, st, op, inner4, unsigned(chunks), C, qp); break;
-        case 2: hipLaunchKernelGGL((seg_kernel<Op, 2>), grid, block, 0, st, op, inner4, unsigned(chunks), C, qp); break;
-        default: hipLaunchKernelGGL((seg_kernel<Op, 1>), grid, block, 0, st, op, inner4, unsigned(chunks), C, qp); break;
+        case 8: hipLaunchKernelGGL((seg_kernel<Op, 8>), grid, block, 0, st, op, inner4, unsigned(tail), unsigned(chunks), C, qp); break;
+        case 4: hipLaunchKernelGGL((seg_kernel<Op, 4>), grid, block, 0, st, op, inner4, unsigned(tail), unsigned(chunks), C, qp); break;
+        case 2: hipLaunchKernelGGL((seg_kernel<Op, 2>), grid, block, 0, st, op, inner4, unsigned(tail), unsigned(chunks), C, qp); break;
+        default: hipLaunchKernelGGL((seg_kernel<Op, 1>), grid, block, 0, st, op, inner4, unsigned(tail), unsigned(chunks), C, qp); break;
         }
+    } else if (vec_ok && n >= 4 && n < (size_t(1) << 31) && qp.scale) {
+        constexpr int U = Op::kMaxU < 4 ? Op::kMaxU : 4;
+        const unsigned blocks = unsigned((n / 4 + U * kThreads - 1) / (U * kThreads));
+        const FastDiv by_inner{unsigned(inner)}, by_c{unsigned(C)};
+        if (inner >= 4)
+            hipLaunchKernelGGL((flat_kernel<Op, U, 2>), dim3(blocks), dim3(kThreads), 0, st, op, unsigned(n), by_inner, by_c, qp);
+        else
+            hipLaunchKernelGGL((flat_kernel<Op, U, 4>), dim3(blocks), dim3(kThreads), 0, st, op, unsigned(n), by_inner, by_c, qp);
     } else {
         size_t blocks = (n + kThreads - 1) / kThreads;
         if (blocks > 262144) blocks = 262144;
@@ -336,10 +411,21 @@ __device__ __forceinline__ void mm_write(MinMax m, float* mn, float* mx, size_t 
     mx[idx] = m.nan ? qnan : m.hi;
 }
 
+// Elements e .. e+3 at any float address
+__device__ __forceinline__ float4 nt_load_any(const float* p) {
+    typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    const f32x4u v = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(p));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void mm_update(MinMax& m, float4 v) {
+    mm_update(m, v.x), mm_update(m, v.y), mm_update(m, v.z), mm_update(m, v.w);
+}
+
 // Channel elements lie in `outer` contiguous runs of `inner`.  Block
 // (c, split) scans its slice of every run.  Partials are laid out
-// [split][c]; with splits == 1 they are the final answer.
-template <bool VEC>
+// [split][c]; with splits == 1 they are the final answer.  The last quad of a run
+// that is not whole quads begins at its fourth element from the end: the elements it
+// takes twice change nothing.
 __global__ __launch_bounds__(kThreads) void minmax_seg_kernel(const float* __restrict__ x,
                                                               size_t outer, size_t C, size_t inner,
                                                               unsigned splits, float* pmin,
@@ -347,36 +433,40 @@ __global__ __launch_bounds__(kThreads) void minmax_seg_kernel(const float* __res
     const size_t c = blockIdx.x / splits;
     const unsigned sp = blockIdx.x - unsigned(c * splits);
     MinMax m{__builtin_inff(), -__builtin_inff(), 0};
-    if (VEC) {
-        const size_t inner4 = inner / 4;
+    if (inner >= 4 && inner <= 2 * kThreads && outer > 1 && splits == 1) {
+        // runs shorter than the block: a power of two of lanes per run, several runs at once
+        const unsigned last = unsigned(inner) - 4, quads = unsigned(inner + 3) / 4;
+        const unsigned shift = quads > 1 ? 32 - __builtin_clz(quads - 1) : 0, runs = kThreads >> shift;
+        const unsigned i = threadIdx.x & ((1u << shift) - 1);
+        const float* p = x + c * inner + (i * 4 < last ? i * 4 : last);  // lanes past the run read its end again
+        const size_t run = C * inner;
+        size_t o = threadIdx.x >> shift;
+        for (; o + 3 * runs < outer; o += 4 * runs) {
+            const float4 a = nt_load_any(p + o * run), b = nt_load_any(p + (o + runs) * run),
+                         d = nt_load_any(p + (o + 2 * runs) * run), e = nt_load_any(p + (o + 3 * runs) * run);
+            mm_update(m, a), mm_update(m, b), mm_update(m, d), mm_update(m, e);
+        }
+        for (; o < outer; o += runs) mm_update(m, nt_load_any(p + o * run));
+    } else if (inner >= 4) {
+        const size_t inner4 = (inner + 3) / 4;
         const size_t per = (inner4 + splits - 1) / splits;
         const size_t lo4 = size_t(sp) * per;
         const size_t hi4 = lo4 + per < inner4 ? lo4 + per : inner4;
-        for (size_t o = 0; o < outer; ++o) {
-            const float4* p = reinterpret_cast<const float4*>(x + (o * C + c) * inner);
-            size_t i = lo4 + threadIdx.x;
-            // four independent loads in flight per lane
-            for (; i + 3 * kThreads < hi4; i += 4 * kThreads) {
-                float4 a = nt_load(&p[i]), b = nt_load(&p[i + kThreads]), d = nt_load(&p[i + 2 * kThreads]),
-                       e = nt_load(&p[i + 3 * kThreads]);
-                mm_update(m, a.x); mm_update(m, a.y); mm_update(m, a.z); mm_update(m, a.w);
-                mm_update(m, b.x); mm_update(m, b.y); mm_update(m, b.z); mm_update(m, b.w);
-                mm_update(m, d.x); mm_update(m, d.y); mm_update(m, d.z); mm_update(m, d.w);
-                mm_update(m, e.x); mm_update(m, e.y); mm_update(m, e.z); mm_update(m, e.w);
-            }
-            for (; i < hi4; i += kThreads) {
-                float4 a = nt_load(&p[i]);
-                mm_update(m, a.x); mm_update(m, a.y); mm_update(m, a.z); mm_update(m, a.w);
-            }
-        }
-    } else {
-        const size_t per = (inner + splits - 1) / splits;
-        const size_t lo = size_t(sp) * per;
-        const size_t hi = lo + per < inner ? lo + per : inner;
+        const size_t whole = hi4 < inner / 4 ? hi4 : inner / 4;
         for (size_t o = 0; o < outer; ++o) {
             const float* p = x + (o * C + c) * inner;
-            for (size_t i = lo + threadIdx.x; i < hi; i += kThreads) mm_update(m, p[i]);
+            size_t i = lo4 + threadIdx.x;
+            // four independent loads in flight per lane
+            for (; i + 3 * kThreads < whole; i += 4 * kThreads) {
+                const float4 a = nt_load_any(p + i * 4), b = nt_load_any(p + (i + kThreads) * 4),
+                             d = nt_load_any(p + (i + 2 * kThreads) * 4), e = nt_load_any(p + (i + 3 * kThreads) * 4);
+                mm_update(m, a), mm_update(m, b), mm_update(m, d), mm_update(m, e);
+            }
+            for (; i < hi4; i += kThreads) mm_update(m, nt_load_any(p + (i * 4 < inner - 4 ? i * 4 : inner - 4)));
         }
+    } else {
+        for (size_t o = threadIdx.x; o < outer; o += kThreads)
+            for (size_t i = 0; i < inner; ++i) mm_update(m, x[(o * C + c) * inner + i]);
     }
     m = mm_block_reduce(m);
     if (threadIdx.x == 0) mm_write(m, pmin, pmax, size_t(sp) * C + c);
@@ -396,8 +486,65 @@ __global__ __launch_bounds__(kThreads) void minmax_col_kernel(const float* __res
     const size_t lo = size_t(sp) * per;
     const size_t hi = lo + per < outer ? lo + per : outer;
     MinMax m{__builtin_inff(), -__builtin_inff(), 0};
-    for (size_t r = lo; r < hi; ++r) mm_update(m, x[r * cols + col]);
+    size_t r = lo;
+    for (; r + 8 <= hi; r += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = __builtin_nontemporal_load(&x[(r + u) * cols + col]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) mm_update(m, v[u]);
+    }
+    for (; r < hi; ++r) mm_update(m, x[r * cols + col]);
     mm_write(m, pmin, pmax, size_t(sp) * cols + col);
+}
+
+// The same for few columns, where a thread per column would leave most of a block's lanes idle: `lanes` threads,
+// 4 * lanes a multiple of cols, read consecutive quads of x, so that each of a thread's four elements stays in
+// one column; the rows a block has read at once are folded in LDS.  Block b takes steps b, b + blocks, ... of
+// 4 * lanes elements.  Partials [block][cols].
+__global__ __launch_bounds__(kThreads) void minmax_period_kernel(const float* __restrict__ x, size_t n, unsigned cols,
+                                                                 unsigned lanes, float* pmin, float* pmax) {
+    __shared__ float s_lo[4 * kThreads], s_hi[4 * kThreads];
+    const unsigned tid = threadIdx.x, step = 4 * lanes;
+    MinMax m[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m[e] = MinMax{__builtin_inff(), -__builtin_inff(), 0};
+    auto take = [&](float4 v) {
+        mm_update(m[0], v.x), mm_update(m[1], v.y), mm_update(m[2], v.z), mm_update(m[3], v.w);
+    };
+    if (tid < lanes) {
+        const size_t stride = size_t(gridDim.x) * step;
+        size_t i = size_t(blockIdx.x) * step + tid * 4;
+        for (; i + 3 * stride + 4 <= n; i += 4 * stride) {
+            const float4 a = nt_load_any(x + i), b = nt_load_any(x + i + stride), c = nt_load_any(x + i + 2 * stride),
+                         d = nt_load_any(x + i + 3 * stride);
+            take(a), take(b), take(c), take(d);
+        }
+        for (; i + 4 <= n; i += stride) take(nt_load_any(x + i));
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            if (i + e < n) mm_update(m[e], x[i + e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s_lo[tid * 4 + e] = m[e].nan ? __builtin_nanf("") : m[e].lo;
+            s_hi[tid * 4 + e] = m[e].nan ? __builtin_nanf("") : m[e].hi;
+        }
+    }
+    __syncthreads();
+    for (unsigned rows = step / cols; rows > 1;) {  // entry row * cols + col; the upper rows into the lower ones
+        const unsigned keep = (rows + 1) / 2;
+        for (unsigned k = tid; k < (rows - keep) * cols; k += kThreads) {
+            const float a = s_lo[k], b = s_lo[k + keep * cols], c = s_hi[k], d = s_hi[k + keep * cols];
+            s_lo[k] = a != a || b < a ? a != a ? a : b : b != b ? b : a;
+            s_hi[k] = c != c || d > c ? c != c ? c : d : d != d ? d : c;
+        }
+        __syncthreads();
+        rows = keep;
+    }
+    for (unsigned k = tid; k < cols; k += kThreads) {
+        pmin[size_t(blockIdx.x) * cols + k] = s_lo[k];
+        pmax[size_t(blockIdx.x) * cols + k] = s_hi[k];
+    }
 }
 
 // Folds partials [groups][C][inner_cols] into mn[C], mx[C]; one block per
@@ -879,9 +1026,18 @@ int minmax_launch(const float* x, size_t outer, size_t C, size_t inner, float* m
         if (rc) return rc;
         float* pmin = static_cast<float*>(ws);
         float* pmax = pmin + splits * cols;
-        hipLaunchKernelGGL(minmax_col_kernel, dim3(unsigned(col_blocks), unsigned(splits)),
-                           dim3(kThreads), 0, st, x, outer, cols, unsigned(splits), pmin, pmax);
-        LQ_CHECK_LAUNCH("minmax_col");
+        // quads of one row of lanes keep their columns when 4 * lanes is a multiple of cols
+        const size_t period = cols % 4 == 0 ? cols / 4 : (cols % 2 == 0 ? cols / 2 : cols);
+        if (period <= kThreads) {
+            const size_t lanes = kThreads / period * period;
+            hipLaunchKernelGGL(minmax_period_kernel, dim3(unsigned(splits)), dim3(kThreads), 0, st, x, outer * cols,
+                               unsigned(cols), unsigned(lanes), pmin, pmax);
+            LQ_CHECK_LAUNCH("minmax_period");
+        } else {
+            hipLaunchKernelGGL(minmax_col_kernel, dim3(unsigned(col_blocks), unsigned(splits)),
+                               dim3(kThreads), 0, st, x, outer, cols, unsigned(splits), pmin, pmax);
+            LQ_CHECK_LAUNCH("minmax_col");
+        }
         hipLaunchKernelGGL(minmax_finalize_kernel, dim3(unsigned(C)), dim3(256), 0, st, pmin, pmax, C,
                            unsigned(splits), unsigned(inner), mn, mx);
         LQ_CHECK_LAUNCH("minmax_finalize");
@@ -896,7 +1052,6 @@ int minmax_launch(const float* x, size_t outer, size_t C, size_t inner, float* m
         if (splits > max_splits) splits = max_splits;
         if (splits < 1) splits = 1;
     }
-    const bool vec = (inner % 4 == 0) && aligned16(x);
     float *pmin = mn, *pmax = mx;
     if (splits > ws_limit / (2 * C * sizeof(float))) splits = ws_limit / (2 * C * sizeof(float));
     if (splits < 1) splits = 1;  // one block per channel writes mn / mx directly: no partials at all
@@ -908,12 +1063,7 @@ int minmax_launch(const float* x, size_t outer, size_t C, size_t inner, float* m
         pmax = pmin + splits * C;
     }
     dim3 grid{unsigned(C * splits)}, block{kThreads};
-    if (vec)
-        hipLaunchKernelGGL((minmax_seg_kernel<true>), grid, block, 0, st, x, outer, C, inner,
-                           unsigned(splits), pmin, pmax);
-    else
-        hipLaunchKernelGGL((minmax_seg_kernel<false>), grid, block, 0, st, x, outer, C, inner,
-                           unsigned(splits), pmin, pmax);
+    hipLaunchKernelGGL(minmax_seg_kernel, grid, block, 0, st, x, outer, C, inner, unsigned(splits), pmin, pmax);
     LQ_CHECK_LAUNCH("minmax_seg");
     if (splits > 1) {
         hipLaunchKernelGGL(minmax_finalize_kernel, dim3(unsigned(C)), dim3(256), 0, st, pmin, pmax, C,
@@ -1263,12 +1413,8 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
     }
     // slices of at least 4096 elements
     const unsigned splits = n < 4096 ? 1u : (n / 4096 < size_t(kMaxParts) ? unsigned(n / 4096) : unsigned(kMaxParts));
-    if (n % 4 == 0 && aligned16(x))
-        hipLaunchKernelGGL((minmax_seg_kernel<true>), dim3(splits), dim3(kThreads), 0, st, x, size_t(1), size_t(1), n, splits,
-                           parts, parts + splits);
-    else
-        hipLaunchKernelGGL((minmax_seg_kernel<false>), dim3(splits), dim3(kThreads), 0, st, x, size_t(1), size_t(1), n, splits,
-                           parts, parts + splits);
+    hipLaunchKernelGGL(minmax_seg_kernel, dim3(splits), dim3(kThreads), 0, st, x, size_t(1), size_t(1), n, splits, parts,
+                       parts + splits);
     LQ_CHECK_LAUNCH("minmax_seg");
     ragged ? launch(quantize_tensor_dynamic_kernel<true, true>, parts, int(splits))
            : launch(quantize_tensor_dynamic_kernel<true, false>, parts, int(splits));

@@ -263,6 +263,37 @@ def test_minmax_propagates_nan():
     assert np.isnan(mx.numpy()[1]) and mn.numpy()[0] == 0.0 and mx.numpy()[2] == 14999.0
 
 
+# Segments that are short or not whole quads: 1 - 5 elements per channel (one to four channels in a quad), runs of
+# columns on both sides of what a row of 256 lanes covers, more rows than a block folds, totals that end inside a quad.
+@pytest.mark.parametrize("shape,ch_axis", [
+    ((1031, 17), 1), ((3, 1), 1), ((70, 54, 12), 1), ((9001, 2), 1), ((37, 5, 3), 1), ((129, 255), 1), ((130, 257), 1),
+    ((131, 1024), 1), ((132, 1026), 1), ((67, 26, 6), 1), ((41, 3, 5), 1), ((5, 4, 67), 1), ((6, 1029), 0), ((3, 4099), 0),
+    ((100003,), None), ((1026,), None), ((257,), None), ((50000, 3), 1),
+    ((301, 3, 64), 1), ((77, 2, 67), 1), ((9, 3, 511), 1), ((9, 3, 513), 1),
+])
+def test_ragged_segments_bit_exact(shape, ch_axis):
+    rng = np.random.default_rng(sum(shape))
+    qd = Q.quint8
+    s, z = _params(rng, shape, ch_axis, True)
+    x = _adversarial(rng, shape, s[0])
+    mn, mx = Q.minmax(hip(x), ch_axis=ch_axis)
+    emn, emx = O.minmax(x, ch_axis=ch_axis)
+    assert np.array_equal(mn.numpy().reshape(-1), emn) and np.array_equal(mx.numpy().reshape(-1), emx)
+    y = x.copy()
+    y.reshape(-1)[-1] = np.nan
+    mn, mx = Q.minmax(hip(y), ch_axis=ch_axis)
+    emn, emx = O.minmax(y, ch_axis=ch_axis)
+    assert same_f32(mn.numpy().reshape(-1), emn) and same_f32(mx.numpy().reshape(-1), emx)
+    st, zt = (hip(s[0]), hip(z[0])) if ch_axis is None else (hip(s), hip(z))
+    q = Q.quantize(hip(x), st, zt, qd, ch_axis=ch_axis)
+    eq = O.quantize(x, s, z, qd.quant_min, qd.quant_max, ch_axis=ch_axis, q_dtype=O.I16)
+    assert np.array_equal(q.numpy(), eq)
+    assert np.array_equal(bits(Q.dequantize(q, st, zt, ch_axis=ch_axis).numpy()),
+                          bits(O.dequantize(eq, s, z, ch_axis=ch_axis)))
+    assert np.array_equal(bits(Q.fake_quantize(hip(x), st, zt, qd.quant_min, qd.quant_max, ch_axis=ch_axis).numpy()),
+                          bits(O.fake_quantize(x, s, z, qd.quant_min, qd.quant_max, ch_axis=ch_axis)))
+
+
 # ------------------------------------------------------------------ full-size properties
 def test_round_trip_properties_at_benchmark_size():
     """4096 x 4096 x 16 float32, per-channel symmetric along dim 0, then
