@@ -126,8 +126,8 @@ __host__ __device__ constexpr int wq_stages(int K, int gs) {
     return ((K + 63) / 64 + wq_unroll(gs) - 1) / wq_unroll(gs) * wq_unroll(gs);
 }
 
-// s_waitcnt immediate for vmcnt <= n only
-constexpr int wq_vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
+// s_waitcnt immediate for vmcnt <= n and every LDS read done
+constexpr int wq_vmcnt_lds(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4); }
 
 template <int BITS, int GS, int MT, int NT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -219,7 +219,9 @@ void wq_gemm_kernel(const char* __restrict__ parts, const char* __restrict__ xsu
     for (int s0 = 0; s0 < stages; s0 += UNROLL) {
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
-            __builtin_amdgcn_s_waitcnt(wq_vmcnt(S::PER_WAVE * (S::RING - 2)));
+            // (the sums and scales read in the stage before may not be needed until after the barrier, which opens
+            // their slot to the next loads: they are waited for here)
+            __builtin_amdgcn_s_waitcnt(wq_vmcnt_lds(S::PER_WAVE * (S::RING - 2)));
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             // (the slot that everybody has just left)
@@ -288,7 +290,7 @@ void wq_gemm_kernel(const char* __restrict__ parts, const char* __restrict__ xsu
         }
     }
     apply(1);
-    __builtin_amdgcn_s_waitcnt(wq_vmcnt(0));  // the loads past the end have landed before the LDS is given up
+    __builtin_amdgcn_s_waitcnt(wq_vmcnt_lds(0));  // the loads past the end have landed before the LDS is given up
     // accumulator element r of a lane: row 4 * quarter + r, column lane % 16
     const int m_base = (tm * 2 + wm) * MT * 16 + q * 4, n_base = (tn * 4 + wn) * (NT * 16) + ln;
 #pragma unroll
