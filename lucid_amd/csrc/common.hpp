@@ -46,8 +46,12 @@ int hip_fail(hipError_t e, const char* what);
 int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, bool* fresh);
 // kind 0: the general workspace (at least 4 MiB); 1 / 2: stream-K counters / slabs;
 // 3: raw accumulators and operand sums of a layer with affine weights; 4: padded copies of ragged GEMM operands;
-// 5: the range slots of a dynamic quantization; 6: the codes and qparams of a dynamic Linear's activation
+// 5: the range slots of a dynamic quantization; 6: the codes and qparams of a dynamic Linear's activation;
+// 7: the slots of a dynamic quantization in one launch
 int workspace(size_t nbytes, hipStream_t stream, void** ptr);
+// Held while launches that hand data to each other through a stream's scratch are issued: two threads
+// that use one stream would otherwise interleave them.
+std::unique_lock<std::recursive_mutex> scratch_lock();
 // Split-K scratch of one stream: arrival counters (zero between launches: the finisher of a
 // tile resets its counter) and slabs for the partial results, whose layout the kernel defines.
 struct SkScratch {

@@ -861,6 +861,7 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
             const int ld = (g.K + 63) / 64 * 64;
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;
             void* tmp = nullptr;
+            const auto lock = scratch_lock();
             int rc = stream_buffer(4, a_bytes + w_bytes, 0, st, &tmp, nullptr);
             if (rc) return rc;
             int8_t* pa = static_cast<int8_t*>(tmp);

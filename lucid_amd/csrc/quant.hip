@@ -1390,7 +1390,9 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
                "dynamic quantization of %zu elements", n);
     void* tmp = nullptr;
     bool fresh = false;
+    std::unique_lock<std::recursive_mutex> lock;
     if (blocks > 1) {
+        lock = scratch_lock();
         const int rc = stream_buffer(5, sizeof(DynScratch) + 2 * kMaxParts * sizeof(float), 0, st, &tmp, &fresh);
         if (rc) return rc;
     }
@@ -1472,6 +1474,7 @@ int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw
     // codes (rows as long as the weight's), scale and zero point, then the GEMM
     const size_t code_bytes = (size_t(M) * ldw + 255) / 256 * 256;
     void* tmp = nullptr;
+    const auto lock = scratch_lock();
     int rc = stream_buffer(6, code_bytes + 256, 0, st, &tmp, nullptr);
     if (rc) return rc;
     int8_t* codes = static_cast<int8_t*>(tmp);

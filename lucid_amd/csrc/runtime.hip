@@ -113,6 +113,11 @@ int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream,
     return LQ_OK;
 }
 
+std::unique_lock<std::recursive_mutex> scratch_lock() {
+    static std::recursive_mutex mu;
+    return std::unique_lock<std::recursive_mutex>(mu);
+}
+
 int workspace(size_t nbytes, hipStream_t stream, void** ptr) {
     return stream_buffer(0, nbytes, size_t(4) << 20, stream, ptr, nullptr);
 }

@@ -670,3 +670,30 @@ def test_two_dynamic_linears_are_captured_as_separate_launches_with_the_same_bit
         # the one launch again, smaller: its arrival counter and scratch are the previous call's
         assert np.array_equal(model(other).numpy().view(np.uint32), other_eager.view(np.uint32))
     g.destroy()
+
+
+def test_two_threads_on_one_stream_share_scratch_safely():
+    """Calls of several launches that pass data through the stream's scratch (codes of a dynamic Linear,
+    padded rows) keep them together: two threads on the default stream get the bits of one thread."""
+    import threading
+    rng = np.random.default_rng(5)
+    work = []
+    for K, scale in ((1000, 1.0), (1000, 3.0)):
+        lin = nnqd.Linear(K, 130)
+        lin.weight_int8 = hip(rng.integers(-127, 128, (130, K)).astype(np.int8))
+        lin.weight_scale = hip(rng.uniform(0.001, 0.01, 130).astype(np.float32))
+        lin._state_loaded("weight_int8")
+        x = hip((rng.standard_normal((70, K)) * scale).astype(np.float32))
+        work.append((lin, x, lin(x).numpy()))
+    go, bad = threading.Barrier(2), []
+
+    def run(lin, x, want):
+        go.wait()
+        for _ in range(50):
+            ys = [lin(x) for _ in range(4)]
+            bad.extend(1 for y in ys if not np.array_equal(y.numpy(), want))
+
+    ts = [threading.Thread(target=run, args=w) for w in work]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad
