@@ -1389,15 +1389,23 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
     LQ_REQUIRE((!ragged || blocks * kDynPerBlock < (size_t(1) << 32)) && blocks < 0x7fffffffull, LQ_ERR_SHAPE,
                "dynamic quantization of %zu elements", n);
     void* tmp = nullptr;
-    bool fresh = false;
+    bool exchange = blocks <= size_t(kExchange), fresh = false;
     std::unique_lock<std::recursive_mutex> lock;
     if (blocks > 1) {
         lock = scratch_lock();
-        const int rc = stream_buffer(5, sizeof(DynScratch) + 2 * kMaxParts * sizeof(float), 0, st, &tmp, &fresh);
+        if (exchange) {
+            // not in a graph: slots first cleared there would be unset until its replay, and replays on
+            // another stream would share them with this one
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            LQ_HIP(hipStreamIsCapturing(st, &capturing));
+            exchange = capturing == hipStreamCaptureStatusNone;
+        }
+        const int rc = exchange ? stream_buffer(7, sizeof(DynScratch), 0, st, &tmp, &fresh)
+                                : stream_buffer(5, 2 * kMaxParts * sizeof(float), 0, st, &tmp, nullptr);
         if (rc) return rc;
     }
-    DynScratch* d = static_cast<DynScratch*>(tmp);
-    float* parts = reinterpret_cast<float*>(d + 1);
+    DynScratch* d = exchange ? static_cast<DynScratch*>(tmp) : nullptr;
+    float* parts = static_cast<float*>(tmp);
     if (fresh) {
         int rc = lq_fill_bytes(d, 0xff, sizeof(d->slot), reinterpret_cast<lq_stream>(st));
         if (!rc) rc = lq_fill_bytes(&d->left, 0, sizeof(d->left), reinterpret_cast<lq_stream>(st));
@@ -1407,7 +1415,7 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
         hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(kDynThreads), 0, st, x, n, cols, ld, symmetric, qmin, qmax,
                            is_signed, eps, half_range, off, d, ranges, n_ranges, scale, zp, mn, mx, q);
     };
-    if (blocks <= size_t(kExchange)) {
+    if (exchange) {
         ragged ? launch(quantize_tensor_dynamic_kernel<false, true>, nullptr, 0)
                : launch(quantize_tensor_dynamic_kernel<false, false>, nullptr, 0);
         LQ_CHECK_LAUNCH("quantize_tensor_dynamic");

@@ -697,3 +697,41 @@ def test_two_threads_on_one_stream_share_scratch_safely():
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+@pytest.mark.parametrize("n", [8193, 40001])
+def test_dynamic_quantization_first_issued_in_a_capture(n):
+    """A stream whose first dynamic quantization is recorded into a graph: an eager call before the first
+    replay, and every replay, have the bits of a plain call."""
+    import ctypes as C
+    from lucid_amd import _C
+    rng = np.random.default_rng(n)
+    xs = [rng.standard_normal(n).astype(np.float32) * s for s in (1.0, 4.0, 0.5)]
+    x, q, s, z = hip(xs[0]), L.Tensor.empty((n,), L.int8, "hip"), L.Tensor.empty((), L.float32, "hip"), L.Tensor.empty((), L.float32, "hip")
+    xds = [hip(v) for v in xs]
+
+    def call(src, stream):
+        _C.call("lq_quantize_tensor_dynamic_i8", src.data_ptr, n, 0, 0, 255, 0, 1e-8, -128, s.data_ptr, z.data_ptr, None,
+                None, q.data_ptr, stream)
+
+    want = []
+    for v in xds:
+        call(v, None)
+        L.synchronize()
+        want.append((q.numpy().copy(), s.numpy().copy()))
+    stream, gid = C.c_void_p(), C.c_int()
+    _C.call("lq_stream_create", C.byref(stream))
+    try:
+        _C.call("lq_graph_begin", stream, C.byref(gid))
+        call(x, stream)
+        _C.call("lq_graph_end", stream, gid)
+        for i in range(3):
+            call(xds[i], stream)
+            _C.call("lq_sync", stream)
+            assert np.array_equal(q.numpy(), want[i][0]) and s.numpy() == want[i][1]
+            _C.call("lq_graph_launch", gid, stream)
+            _C.call("lq_sync", stream)
+            assert np.array_equal(q.numpy(), want[0][0]) and s.numpy() == want[0][1]
+        _C.call("lq_graph_destroy", gid)
+    finally:
+        _C.call("lq_stream_destroy", stream)
