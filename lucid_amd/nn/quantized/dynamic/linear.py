@@ -99,16 +99,15 @@ class Linear(Module):
     def _weight_rows(self) -> tuple[Tensor, int]:
         """The weight codes in rows of a multiple of 16 bytes (``weight_int8`` itself where its rows are) and
         that length; rows of a ragged layer are laid out once, with zeros behind them."""
+        N, K = self.out_features, self.in_features
+        if K % 16 == 0:
+            return self._buffers["weight_int8"], K
         if self._wrows is None:
-            N, K = self.out_features, self.in_features
-            if K % 16 == 0:
-                self._wrows = (self.weight_int8, K)
-            else:
-                ld = (K + 63) // 64 * 64
-                rows = Tensor.empty((N, ld), T.int8, "hip")
-                _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
-                _C.call("lq_d2d_rows", rows.data_ptr, ld, self.weight_int8.data_ptr, K, K, N, None)
-                self._wrows = (rows, ld)
+            ld = (K + 63) // 64 * 64
+            rows = Tensor.empty((N, ld), T.int8, "hip")
+            _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
+            _C.call("lq_d2d_rows", rows.data_ptr, ld, self.weight_int8.data_ptr, K, K, N, None)
+            self._wrows = (rows, ld)
         return self._wrows
 
     def forward(self, x: Tensor, residual: Tensor | None = None, activation: str | None = None,
@@ -131,7 +130,8 @@ class Linear(Module):
         off = storage_offset(qd)
         bias = self._buffers["bias"]
         if (x._range is None and residual is None and activation is None and not track_range
-                and weight_zero_points(self) is None and (bias is None or bias.dtype == T.float32)):
+                and weight_zero_points(self) is None and (bias is None or bias.dtype == T.float32)
+                and K < 131008 and x.numel < 1 << 31):  # (padded rows past either are more than the call takes)
             # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
             if self._wsum is None:
                 self._wsum = _ops.rowsum_i8(self.weight_int8)

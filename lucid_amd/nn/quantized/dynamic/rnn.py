@@ -190,6 +190,9 @@ class LSTM(Module):
         fused, k = C.c_int(), 0
         while k < self.num_layers:
             _C.call("lq_lstm_fused_layers", Tn, Bn, x.shape[2], H, self.num_layers - k, dirs, C.byref(fused))
+            # (an input whose rows are 2 GiB apart is beyond the recurrence's own input product)
+            if Bn * (Tn if self.batch_first else 1) * x.shape[2] >= 1 << 29:
+                fused.value = 0
             layers = max(1, fused.value)
             a = _C.LstmArgs()
             a.inputs, a.x = x.shape[2], x.data_ptr if fused.value else None
