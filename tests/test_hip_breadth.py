@@ -312,6 +312,20 @@ def test_dynamic_lstm_sequence_sizes(I, H, Bn, Tn, bidir, batch_first):
         del y, hn, cn
 
 
+def test_dynamic_lstm_input_of_two_gib():
+    """batch_first rows that span 2 GiB of input: beyond what the recurrence addresses itself, still taken.
+    A zero input gives every row the bits of a batch of one."""
+    from lucid_amd import _C
+    I, H, Bn = 512, 16, 1 << 20
+    qm = Q.quantize_dynamic(nn.LSTM(I, H, batch_first=True))
+    x = L.Tensor.empty((Bn, 1, I), L.float32, "hip")
+    _C.call("lq_fill_bytes", x.data_ptr, 0, x.nbytes, None)
+    y, _ = qm(x)
+    one, _ = qm(hip(np.zeros((1, 1, I), np.float32)))
+    y = y.numpy()
+    assert np.array_equal(y, np.broadcast_to(one.numpy(), y.shape))
+
+
 @pytest.mark.parametrize("I,H,layers,Bn,Tn,bidir,batch_first",
                          [(3, 1, 2, 1, 3, False, False), (130, 17, 3, 5, 4, False, True), (500, 129, 5, 33, 2, False, False),
                           (100, 300, 2, 16, 5, False, True), (512, 512, 2, 17, 4, False, False), (257, 250, 2, 18, 3, True, True),
