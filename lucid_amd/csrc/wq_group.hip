@@ -676,10 +676,12 @@ int lq_wq_matmul(const float* x, const uint32_t* packed, const float* scales, co
                              : launch_gemv1<8>(x, packed, scales, biases, N, K, group_size, out, st);
         if (wq_gemm_beats_small_batch(M, N, K, group_size, bits))
             return launch_wq_gemm(x, packed, scales, biases, M, N, K, group_size, bits, out, st);
-        return bits == 4 ? launch_wq_mfma<4>(x, packed, scales, biases, M, N, K, group_size, out, st)
-                         : launch_wq_mfma<8>(x, packed, scales, biases, M, N, K, group_size, out, st);
+        // (its slabs grow with M x N x K: not for the weights of 2 GiB that the large-batch kernel leaves)
+        if (M <= 64 || size_t(N) * K * bits / 8 < 0x7fffffffull)
+            return bits == 4 ? launch_wq_mfma<4>(x, packed, scales, biases, M, N, K, group_size, out, st)
+                             : launch_wq_mfma<8>(x, packed, scales, biases, M, N, K, group_size, out, st);
     }
-    // operands that are not 16-byte aligned: decode once into the workspace, then the float32 MFMA GEMM
+    // operands that are not 16-byte aligned, large batches on such a weight: decode once into the workspace, then the float32 MFMA GEMM
     void* ws = nullptr;
     rc = workspace(size_t(N) * K * sizeof(float), st, &ws);
     if (rc) return rc;
