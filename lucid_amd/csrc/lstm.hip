@@ -468,7 +468,8 @@ int lq_lstm_sequence_f32(const lq_lstm_args* a, lq_stream stream) {
     p.x_step = a->batch_first ? p.I : long(p.B) * p.I, p.x_row = a->batch_first ? long(p.T) * p.I : p.I;
     p.y_elems = long(p.T) * p.B * width, p.x_elems = long(p.T) * p.B * p.I;
     // an element is addressed as a 32-bit byte offset from its step's first
-    LQ_REQUIRE((p.B - 1) * p.y_row + width < 0x7fffffffL / 4 && (p.B - 1) * p.x_row + p.I < 0x7fffffffL / 4,
+    LQ_REQUIRE((p.B - 1) * p.y_row + width < 0x7fffffffL / 4 &&
+                   (!a->x || (p.B - 1) * p.x_row + p.I < 0x7fffffffL / 4),
                LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: %ld outputs or %ld inputs are too many", p.y_elems, p.x_elems);
     const int columns = !a->x ? 0 : p.stacked && p.H > p.I ? p.H : p.I;
     return with_form(p.H, columns, [&](auto w, auto k, auto x) { return launch_lstm<w(), k(), x()>(p, parts, as_stream(stream)); });
