@@ -704,7 +704,8 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 // launch.  All blocks have to be resident (see lstm.hip on what the launcher has to leave free: kExchange
 // blocks of 512 threads and 64 registers are far below it), and a wait is bounded.
 //
-// Beyond, two launches: slices' ranges (minmax_seg_kernel), then this kernel with PARTS - every block reduces
+// Beyond, and under capture (slots cleared inside a graph are unset until its replay), two launches: slices'
+// ranges (minmax_seg_kernel), then this kernel with PARTS - every block reduces
 // the slices' ranges itself, which saves the finalize and qparams launches between.
 //
 // Rows of `cols` elements go to rows of `ld` codes, zeros past `cols` (what a GEMM of ragged rows wants).

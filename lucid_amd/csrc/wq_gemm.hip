@@ -25,7 +25,7 @@
 // all, which with two wavefronts per SIMD (one hides the other's scaling and LDS reads) caps MT NT at 12.
 //
 // The sums of a group are scaled while the next group is multiplied (two sets of accumulators take turns).
-// 333 x 11008 x 4096, int4, groups of 128: 123 us, 0.73 POP/s in bfloat16 terms (a library product of plain
+// 333 x 11008 x 4096, int4, groups of 128: 100 us, 0.90 PFLOP/s in bfloat16 terms (a library product of plain
 // bfloat16 operands reaches 1.18 on the card); decoding to float32 (109 us) and a float32 GEMM (286 us) before.
 //
 // The codes' 16-byte chunks are placed in LDS at chunk ^ (row / 4) (int8) or chunk ^ (row / 8) (int4), which
