@@ -325,8 +325,9 @@ Tile wq_gemm_tile(int M, int N, int stages) {
     return best;
 }
 
+// One chunk of rows: prepare, product.
 template <int BITS, int GS, int MT, int NT>
-int launch_tile(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N, int K,
+int launch_rows(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N, int K,
                 float* out, hipStream_t st) {
     constexpr int SEGS = wq_segs(GS);
     using S = WqStage<BITS, SEGS, MT, NT>;
@@ -359,6 +360,25 @@ int launch_tile(const float* x, const uint32_t* packed, const float* scales, con
     hipLaunchKernelGGL((wq_gemm_kernel<BITS, GS, MT, NT>), dim3(unsigned(tiles_m) * unsigned(tiles_n)), dim3(512), smem,
                        st, parts, xsum, reinterpret_cast<const char*>(packed), sb, M, N, K, mtiles, n_pad, out);
     LQ_CHECK_LAUNCH("wq_gemm");
+    return LQ_OK;
+}
+
+// The kernel's strides from stage to stage are 32-bit, and the prepared rows take half as much again as x: rows are
+// taken in chunks of at most kMaxParts of them (43 thousand rows at K = 4096, far more than fill the chip).  Chunks
+// are whole row tiles, so the bits do not depend on the split.
+constexpr size_t kMaxParts = size_t(1) << 30;
+template <int BITS, int GS, int MT, int NT>
+int launch_tile(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N, int K,
+                float* out, hipStream_t st) {
+    constexpr int bm = 32 * MT;
+    const size_t tile_bytes = size_t(wq_stages(K, GS)) * (2 * MT) * (6 * kPiece);
+    const size_t tiles = tile_bytes < kMaxParts ? kMaxParts / tile_bytes : 1;
+    const int rows = tiles * bm < size_t(M) ? int(tiles * bm) : M;
+    for (int m0 = 0; m0 < M; m0 += rows) {
+        const int rc = launch_rows<BITS, GS, MT, NT>(x + size_t(m0) * K, packed, scales, biases, M - m0 < rows ? M - m0 : rows,
+                                                     N, K, out + size_t(m0) * N, st);
+        if (rc || M - m0 <= rows) return rc;
+    }
     return LQ_OK;
 }
 

@@ -98,6 +98,32 @@ def test_large_batch_matmul_is_exact_on_exact_inputs(M, N, K, gs, bits):
     assert np.array_equal(y, x @ W.dequantize(packed, s, b, gs, bits).T)
 
 
+@pytest.mark.parametrize("M,N,K,gs", [(1_500_003, 3, 128, 64),   # two chunks of rows, the second one ragged
+                                      (11_200_000, 2, 128, 64)])  # operands of more than 2^32 bytes between stages
+def test_matmul_of_very_many_rows(M, N, K, gs):
+    """Rows beyond what one launch's 32-bit strides reach: every row of a repeated block of 4000 has the
+    block's exact result."""
+    from lucid_amd import _C
+    rng = np.random.default_rng(M)
+    block = 4000
+    packed = rng.integers(0, 2**32, (N, K * 4 // 32), dtype=np.uint32).view(np.int32)
+    s = rng.integers(1, 3, (N, K // gs)).astype(np.float32)
+    b = rng.integers(-8, 9, (N, K // gs)).astype(np.float32)
+    xb = rng.integers(-7, 8, (block, K)).astype(np.float32)
+    x = L.Tensor.empty((M, K), L.float32, "hip")
+    _C.call("lq_h2d", x.data_ptr, xb.ctypes.data, xb.nbytes, None)
+    have = block
+    while have < M:
+        n = min(have, M - have)
+        _C.call("lq_d2d", x.data_ptr + have * K * 4, x.data_ptr, n * K * 4, None)
+        have += n
+    y = _qgemm.quantized_matmul(x, hip(packed), hip(s), hip(b), True, gs, 4).numpy()
+    want = xb @ W.dequantize(packed, s, b, gs, 4).T
+    whole = M // block
+    assert np.array_equal(y[:whole * block].reshape(whole, block, N), np.broadcast_to(want, (whole, block, N)))
+    assert np.array_equal(y[whole * block:], want[:M - whole * block])
+
+
 def test_decoding_takes_foreign_scales_and_biases_as_given():
     # a weight packed elsewhere under the same contract may carry negative scales
     rng = np.random.default_rng(1)
