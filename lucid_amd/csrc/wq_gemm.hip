@@ -184,9 +184,12 @@ void wq_gemm_kernel(const char* __restrict__ parts, const char* __restrict__ xsu
             const char* base = src[u] + size_t(sc) * step[u];
             unsigned o = off[u];
             if (u * 8 + 7 >= S::X + S::SUMS + S::SB) {  // (a round that may hold codes)
-                // a last stage of 32 k runs past its row: into the next one, or here, onto any bytes (its x is zero)
-                const unsigned over = unsigned(sc) * ROW + o;
-                if (at >= S::X + S::SUMS + S::SB && over > w_last) o -= over - w_last;
+                // a stage past K runs past its row: into the next ones, or at the end of the weight onto its last
+                // bytes (its x is zero).  Taken from the start of the weight: the last row may be the first one.
+                if (at >= S::X + S::SUMS + S::SB) {
+                    const unsigned from = unsigned(sc) * ROW + o;
+                    base = packed, o = from < w_last ? from : w_last;
+                }
             }
             __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(base + o),
                                              (__attribute__((address_space(3))) void*)(wq_smem + (slot * S::PIECES + at) * kPiece),

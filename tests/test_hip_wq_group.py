@@ -80,6 +80,8 @@ def test_small_batch_matmul_is_reproducible_and_exact_on_exact_inputs(bits):
     (1025, 3003, 288, 32, 4), (700, 2500, 416, 32, 8), (513, 4097, 256, 64, 4), (300, 6000, 256, 128, 8),
     (130, 11008, 320, 64, 8), (600, 1000, 1024, 64, 4), (1100, 5370, 128, 128, 4), (1100, 5370, 96, 32, 8),
     (333, 10999, 128, 128, 8), (330, 11008, 192, 64, 4), (333, 9000, 224, 32, 4),
+    # a weight of one row, K that leaves the last stages of the main loop past it
+    (100_003, 1, 384, 128, 4), (100_003, 1, 384, 128, 8), (100_003, 1, 192, 64, 4), (100_003, 2, 192, 64, 8), (100_003, 1, 96, 32, 8),
     # the small-batch kernel with a partial last window
     (5, 300, 2016, 32, 8), (33, 258, 1056, 32, 4), (16, 77, 192, 64, 4),
     # one row: K that does not fill the last step, several steps
