@@ -464,10 +464,9 @@ __device__ __forceinline__ v4i act16(const int8_t* row, int k, int K) {
 // memory: at 333 x 1001 x 1000 it is 3.9 us and the product 7 us, where the one-output-per-lane kernel took
 // 1340 us (2000 x 4000 x 4090: 147 ms -> 0.06 ms for the two).
 __global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t* __restrict__ a, int M,
-                                                       const int8_t* __restrict__ w, int N, int K, int ld,
+                                                       const int8_t* __restrict__ w, size_t total, int K, int ld,
                                                        int8_t* __restrict__ pa, int8_t* __restrict__ pw) {
-    const unsigned per_row = unsigned(ld) >> 4;
-    const size_t total = size_t(M + N) * per_row;
+    const unsigned per_row = unsigned(ld) >> 4;  // total: chunks of 16 bytes of all rows (M + N may not fit an int)
     for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < total; i += size_t(gridDim.x) * 256) {
         const unsigned row = unsigned(i / per_row), c = unsigned(i - size_t(row) * per_row);
         const bool is_a = row < unsigned(M);
@@ -863,11 +862,15 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
             void* tmp = nullptr;
             const auto lock = scratch_lock();
             int rc = stream_buffer(4, a_bytes + w_bytes, 0, st, &tmp, nullptr);
+            if (rc == LQ_ERR_OOM && g.range == nullptr) {  // no room for the copies: the plain kernel needs none
+                (void)hipGetLastError();
+                return run_gemm(g_in, 3, tile_config, st);
+            }
             if (rc) return rc;
             int8_t* pa = static_cast<int8_t*>(tmp);
             const size_t chunks = (a_bytes + w_bytes) / 16;
             const size_t blocks = (chunks + 255) / 256 < 16384 ? (chunks + 255) / 256 : 16384;
-            hipLaunchKernelGGL(pad_rows_kernel, dim3(unsigned(blocks)), dim3(256), 0, st, g.a, g.M, g.w, g.N, g.K, ld,
+            hipLaunchKernelGGL(pad_rows_kernel, dim3(unsigned(blocks)), dim3(256), 0, st, g.a, g.M, g.w, chunks, g.K, ld,
                                pa, pa + a_bytes);
             LQ_CHECK_LAUNCH("pad_rows");
             g.a = pa, g.w = pa + a_bytes, g.K = ld;
