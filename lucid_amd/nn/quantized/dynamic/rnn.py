@@ -8,8 +8,9 @@ b_hh)``).
 On the device the recurrence of all steps and directions is one launch
 (``lq_lstm_sequence_f32``), which takes the input products and the layers stacked on top of the
 first as well where they fit; else the input product of a layer is taken over all time steps
-beforehand (float32 MFMA GEMM).  Packed sequences, projections and hidden sizes beyond 1024
-take a recurrent GEMM and a gate kernel per step instead.
+beforehand (float32 MFMA GEMM).  Packed sequences, projections, hidden sizes beyond 1024 and
+states of other types than ``from_float`` leaves take a recurrent GEMM and a gate kernel per step
+instead.
 """
 
 from __future__ import annotations
@@ -36,6 +37,8 @@ class LSTM(Module):
         self.proj_size = proj_size
         self._weight_names: list[str] = []
         self._bias_names: list[str] = []
+        # per layer, what lq_lstm_sequence_f32 reads: name, shape and type of each buffer
+        self._kernel_buffers: list[list[tuple]] = [[] for _ in range(num_layers)]
         dirs = 2 if bidirectional else 1
         rec = proj_size if proj_size > 0 else hidden_size  # width of the state that re-enters the recurrence
         for k in range(num_layers):
@@ -48,10 +51,21 @@ class LSTM(Module):
                     self._weight_names.append(name)
                     self.register_buffer(name + "_int8", T.tensor(np.zeros((rows, cols), np.int8), device="hip"))
                     self.register_buffer(name + "_scale", T.tensor(np.ones(rows, np.float32), device="hip"))
+                    self._kernel_buffers[k] += [(name + "_int8", (rows, cols), T.int8), (name + "_scale", (rows,), T.float32)]
                 if bias:
                     for name in (f"bias_ih_l{k}{suffix}", f"bias_hh_l{k}{suffix}"):
                         self._bias_names.append(name)
                         self.register_buffer(name, T.tensor(np.zeros(4 * hidden_size, np.float32), device="hip"))
+                        self._kernel_buffers[k].append((name, (4 * hidden_size,), T.float32))
+
+    def _kernel_takes(self, k: int) -> bool:
+        """Whether layer ``k`` holds what the one-launch recurrence reads.  A loaded state may hold other types
+        (int16 codes, float16 biases) or sizes: the steps one by one convert those, or refuse them."""
+        for name, shape, dt in self._kernel_buffers[k]:
+            b = self._buffers[name]
+            if b is None or b.shape != shape or b.dtype is not dt or b.device != "hip":
+                return False
+        return True
 
     def _weight(self, name: str) -> Tensor:
         codes, scale = getattr(self, name + "_int8"), getattr(self, name + "_scale")
@@ -111,7 +125,8 @@ class LSTM(Module):
         h_n = Tensor.empty((n_state, Bn, R), T.float32, "hip")
         c_n = Tensor.empty((n_state, Bn, H), T.float32, "hip")
         # (the one-launch recurrence addresses a step's rows with 32-bit byte offsets)
-        if packed is None and P == 0 and H <= 1024 and Tn > 0 and Bn > 0 and Tn * Bn * dirs * H < 1 << 29:
+        if (packed is None and P == 0 and H <= 1024 and Tn > 0 and Bn > 0 and Tn * Bn * dirs * H < 1 << 29
+                and all(self._kernel_takes(k) for k in range(self.num_layers))):
             return self._forward_sequences(x, h0, c0, h_n, c_n, Tn, Bn), (h_n, c_n)
         ragged = any(bs != Bn for bs in batch_sizes)
         layer_in = x
@@ -127,6 +142,10 @@ class LSTM(Module):
                 if self.bias:
                     b = getattr(self, f"bias_ih_l{k}{suffix}").numpy() + getattr(self, f"bias_hh_l{k}{suffix}").numpy()
                     bias = T.tensor(b.astype(np.float32), device="hip")
+                # (the gate kernel takes 4 H of each by address)
+                if w_ih.shape[0] != 4 * H or w_hh.shape != (4 * H, R) or (bias is not None and bias.numel != 4 * H):
+                    raise _C.ShapeMismatch(f"dynamic LSTM: layer {k}{suffix} holds weights {w_ih.shape} and {w_hh.shape} and "
+                                           f"{0 if bias is None else bias.numel} biases for hidden size {H}")
                 gx = linear_f32(layer_in, w_ih)  # (.., .., 4H), same row order as layer_in
                 idx = k * dirs + d
                 h = Tensor.empty((Bn, R), T.float32, "hip")

@@ -352,6 +352,42 @@ def _deq(q, name):
             getattr(q, name + "_scale").numpy()[:, None]).astype(np.float32)
 
 
+def test_dynamic_lstm_states_of_other_types_and_sizes():
+    """The one-launch recurrence reads int8 codes and float32 scales and biases of the layer's sizes.  Any other
+    state does what it does step by step: int16 codes (what a quint8 weight quantizes to) and float16 biases
+    give their values, float16 scales and other shapes are refused."""
+    import lucid_amd.nn.quantized.dynamic as nnqd
+    from lucid_amd import _C
+    I, H, Tn, Bn = 24, 40, 3, 5
+    rng = np.random.default_rng(3)
+    x = hip(rng.standard_normal((Tn, Bn, I)).astype(np.float32))
+    base = Q.quantize_dynamic(nn.LSTM(I, H, num_layers=2))
+    state = {n: t.numpy() for n, t in base.state_dict().items()}
+
+    def loaded(**other):
+        q = nnqd.LSTM(I, H, 2)
+        q.load_state_dict({n: hip(other.get(n, v)) for n, v in state.items()})
+        return q
+
+    half = {n: v.astype(np.float16) for n, v in state.items() if n.startswith("bias")}
+    # (the two are added as they are)
+    rounded = {n: (v + half[n.replace("_ih_", "_hh_")] if "_ih_" in n else 0 * v).astype(np.float32) for n, v in half.items()}
+    short = {"weight_hh_l1_int8": state["weight_hh_l1_int8"].astype(np.int16)}
+    for other, same in ((half, rounded), (short, {})):
+        y, (h, c) = loaded(**other)(x)
+        wy, (wh, wc) = loaded(**same)(x)
+        for a, b in ((y, wy), (h, wh), (c, wc)):
+            assert np.abs(a.numpy() - b.numpy()).max() < 2e-6  # the sums of the steps are in another order
+    with pytest.raises(_C.DtypeMismatch):
+        loaded(weight_ih_l0_scale=state["weight_ih_l0_scale"].astype(np.float16))(x)
+    wrong = [{"weight_hh_l0_int8": state["weight_hh_l0_int8"][:, :H - 8]}, {"weight_ih_l1_scale": state["weight_ih_l1_scale"][:H]},
+             {n: state[n][:H] for n in ("weight_hh_l0_int8", "weight_hh_l0_scale")},
+             {n: state[n][:H] for n in ("bias_ih_l1", "bias_hh_l1")}]
+    for other in wrong:
+        with pytest.raises(_C.ShapeMismatch):
+            loaded(**other)(x)
+
+
 @pytest.mark.parametrize("layers,bidir,proj,sorted_input", [(1, False, 0, True), (2, True, 0, False), (1, False, 6, True),
                                                             (2, True, 5, False)])
 def test_dynamic_lstm_packed_sequences_and_projection(layers, bidir, proj, sorted_input):
