@@ -37,6 +37,16 @@ def _one_launch_pays(M: int, K: int, N: int) -> bool:
             and ((M + 15) // 16) * ((N + 15) // 16) <= 256 and 43 * M * K + 2400 * K <= 6_000_000)
 
 
+def _kernel_takes(lin) -> bool:
+    """Whether ``lin`` holds what the one-call kernels read by address.  A loaded state may hold other types or
+    sizes, or a weight that is an unaligned view: the separate operators take those, or refuse them."""
+    b, N = lin._buffers, lin.out_features
+    w, scale, bias = b["weight_int8"], b["weight_scale"], b["bias"]
+    return (w.shape == (N, lin.in_features) and w.dtype is T.int8 and w._offset % 16 == 0
+            and scale.shape == (N,) and scale.dtype is T.float32
+            and (bias is None or (bias.shape == (N,) and bias.dtype is T.float32)))
+
+
 def fused_pair(first, relu_between: bool, second, x):
     """``second(relu(first(x)))`` (or without the ReLU) for two dynamic ``Linear`` layers on a small
     activation as ONE launch (``lq_dynamic_mlp2_small_f32``: the last block of layer 1 to finish
@@ -58,8 +68,8 @@ def fused_pair(first, relu_between: bool, second, x):
     # (the buffers straight from the registries: this path is bound by what a forward costs the host)
     b1, b2 = first._buffers, second._buffers
     bias1, bias2 = b1.get("bias"), b2.get("bias")
-    for lin, bias in ((first, bias1), (second, bias2)):
-        if weight_zero_points(lin) is not None or (bias is not None and bias.dtype != T.float32):
+    for lin in (first, second):
+        if weight_zero_points(lin) is not None or not _kernel_takes(lin):
             return None
         if lin._wsum is None:
             lin._wsum = _ops.rowsum_i8(lin.weight_int8)
@@ -130,7 +140,7 @@ class Linear(Module):
         off = storage_offset(qd)
         bias = self._buffers["bias"]
         if (x._range is None and residual is None and activation is None and not track_range
-                and weight_zero_points(self) is None and (bias is None or bias.dtype == T.float32)
+                and weight_zero_points(self) is None and _kernel_takes(self)
                 and K < 131008 and x.numel < 1 << 31):  # (padded rows past either are more than the call takes)
             # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
             if self._wsum is None:

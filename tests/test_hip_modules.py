@@ -564,6 +564,41 @@ def test_dynamic_linear_of_any_size(M, K, N, kind):
         assert np.array_equal(got[~np.isnan(got)].view(np.uint32), want[~np.isnan(want)].view(np.uint32))
 
 
+@pytest.mark.parametrize("M", [1, 4, 70])
+@pytest.mark.parametrize("K", [64, 50])
+def test_dynamic_linear_states_of_other_types_and_sizes(M, K):
+    """A float16 bias and an unaligned weight give their values; codes, scales and biases of other types or
+    sizes are refused, whatever the batch: no kernel reads them as what they are not."""
+    from lucid_amd import _C
+    N = 24
+    rng = np.random.default_rng(M + K)
+    x = hip(rng.standard_normal((M, K)).astype(np.float32))
+    state = {"weight_int8": rng.integers(-127, 128, (N, K)).astype(np.int8),
+             "weight_scale": rng.uniform(0.001, 0.01, N).astype(np.float32),
+             "weight_zero_point": np.zeros(N, np.float32), "bias": rng.standard_normal(N).astype(np.float32)}
+
+    def loaded(**other):
+        lin = nnqd.Linear(K, N)
+        lin.load_state_dict({n: v if isinstance(v, L.Tensor) else hip(v) for n, v in {**state, **other}.items()})
+        return lin
+
+    half = state["bias"].astype(np.float16)
+    want = loaded(bias=half.astype(np.float32))(x).numpy()
+    assert np.array_equal(loaded(bias=half)(x).numpy(), want)
+    shifted = np.zeros(N * K + 4, np.int8)
+    shifted[4:] = state["weight_int8"].reshape(-1)
+    view = L.Tensor((N, K), L.int8, "hip", buf=hip(shifted)._buf, offset=4)
+    assert np.array_equal(loaded(weight_int8=view)(x).numpy(), loaded()(x).numpy())
+    for bad in ({"weight_int8": state["weight_int8"].astype(np.int16)}, {"weight_scale": state["weight_scale"].astype(np.float16)},
+                {"bias": state["bias"].astype(np.int32)}):
+        with pytest.raises(_C.DtypeMismatch):
+            loaded(**bad)(x)
+    for bad in ({"weight_int8": state["weight_int8"][:, :K - 2].copy()}, {"weight_int8": state["weight_int8"][:N - 1].copy()},
+                {"weight_scale": state["weight_scale"][:N - 1].copy()}, {"bias": state["bias"][:N - 1].copy()}):
+        with pytest.raises(_C.ShapeMismatch):
+            loaded(**bad)(x)
+
+
 class _recorded_calls:
     """The names of the compute entry points called through the binding while the block runs."""
 

@@ -1,0 +1,36 @@
+"""Which kernels a dynamically quantized layer may take: the host's decisions, without a GPU."""
+
+import numpy as np
+import pytest
+
+import lucid_amd as L
+import lucid_amd.nn.quantized.dynamic as nnqd
+from lucid_amd.nn.module import Module
+from lucid_amd.nn.quantized.dynamic import linear as dl
+
+
+def _layer(N, K, **other):
+    """A layer whose buffers are host tensors."""
+    lin = object.__new__(nnqd.Linear)
+    Module.__init__(lin)
+    lin.in_features, lin.out_features = K, N
+    lin._wsum = lin._wrows = None
+    bufs = dict(weight_int8=np.zeros((N, K), np.int8), weight_scale=np.ones(N, np.float32),
+                weight_zero_point=np.zeros(N, np.float32), bias=np.zeros(N, np.float32))
+    for name, v in {**bufs, **other}.items():
+        lin.register_buffer(name, v if v is None or isinstance(v, L.Tensor) else L.Tensor.from_numpy(v, "cpu"))
+    return lin
+
+
+@pytest.mark.parametrize("other,takes", [
+    ({}, True), ({"bias": None}, True),
+    ({"weight_int8": np.zeros((8, 31), np.int8)}, False), ({"weight_int8": np.zeros((7, 32), np.int8)}, False),
+    ({"weight_int8": np.zeros(8 * 32, np.int8)}, False), ({"weight_int8": np.zeros((8, 32), np.int16)}, False),
+    ({"weight_scale": np.ones(7, np.float32)}, False), ({"weight_scale": np.ones(8, np.float16)}, False),
+    ({"bias": np.zeros(7, np.float32)}, False), ({"bias": np.zeros(8, np.float16)}, False),
+    ({"bias": np.zeros(8, np.float64)}, False),
+    ({"weight_int8": L.Tensor((8, 32), L.int8, "cpu", host=np.zeros((8, 32), np.int8), offset=4)}, False),
+])
+def test_kernels_read_by_address_only_what_they_expect(other, takes):
+    """Sizes, types and the weight's alignment: all else is left to the operators that check."""
+    assert dl._kernel_takes(_layer(8, 32, **other)) is takes
