@@ -37,6 +37,23 @@ def _one_launch_pays(M: int, K: int, N: int) -> bool:
             and ((M + 15) // 16) * ((N + 15) // 16) <= 256 and 43 * M * K + 2400 * K <= 6_000_000)
 
 
+# Bytes of activation codes that the one-call route keeps in the stream's scratch at most (from there on the
+# launches it saves are about 1 % of a layer's time).
+MAX_CODE_BYTES = 1 << 28
+
+
+def _code_row_bytes(K: int) -> int:
+    """Length of a row of codes, of the weight or the activation, as the one-call route lays it out."""
+    return K if K % 16 == 0 else (K + 63) // 64 * 64
+
+
+def _one_call_takes(M: int, K: int) -> bool:
+    """Whether ``lq_dynamic_linear_f32`` takes M rows of K: the padded row within the int32 accumulator, the padded
+    codes within the scratch they may have (a short ragged row grows to 64 bytes)."""
+    ld = _code_row_bytes(K)
+    return ld <= 131071 and M * ld <= MAX_CODE_BYTES
+
+
 def _kernel_takes(lin) -> bool:
     """Whether ``lin`` holds what the one-call kernels read by address.  A loaded state may hold other types or
     sizes, or a weight that is an unaligned view: the separate operators take those, or refuse them."""
@@ -110,10 +127,10 @@ class Linear(Module):
         """The weight codes in rows of a multiple of 16 bytes (``weight_int8`` itself where its rows are) and
         that length; rows of a ragged layer are laid out once, with zeros behind them."""
         N, K = self.out_features, self.in_features
-        if K % 16 == 0:
+        ld = _code_row_bytes(K)
+        if ld == K:
             return self._buffers["weight_int8"], K
         if self._wrows is None:
-            ld = (K + 63) // 64 * 64
             rows = Tensor.empty((N, ld), T.int8, "hip")
             _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
             _C.call("lq_d2d_rows", rows.data_ptr, ld, self.weight_int8.data_ptr, K, K, N, None)
@@ -141,7 +158,7 @@ class Linear(Module):
         bias = self._buffers["bias"]
         if (x._range is None and residual is None and activation is None and not track_range
                 and weight_zero_points(self) is None and _kernel_takes(self)
-                and K < 131008 and x.numel < 1 << 31):  # (padded rows past either are more than the call takes)
+                and _one_call_takes(M, K)):
             # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
             if self._wsum is None:
                 self._wsum = _ops.rowsum_i8(self.weight_int8)

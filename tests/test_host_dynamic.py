@@ -34,3 +34,16 @@ def _layer(N, K, **other):
 def test_kernels_read_by_address_only_what_they_expect(other, takes):
     """Sizes, types and the weight's alignment: all else is left to the operators that check."""
     assert dl._kernel_takes(_layer(8, 32, **other)) is takes
+
+
+@pytest.mark.parametrize("M,K,takes", [
+    (1, 1, True), (1, 131071, False), (1, 131007, True), (1, 131056, True), (1, 131072, False),
+    # 64-byte rows of a short K: far fewer of them than M * K suggests
+    (1 << 22, 3, True), ((1 << 22) + 1, 3, False), (1 << 26, 3, False), (1 << 26, 17, False), (1 << 22, 64, True),
+    ((1 << 22) + 1, 64, False), ((1 << 21), 127, True), ((1 << 21) + 1, 127, False), (1 << 24, 16, True), (1 << 27, 16, False),
+])
+def test_one_call_is_for_codes_that_fit_its_rows_and_scratch(M, K, takes):
+    assert dl._one_call_takes(M, K) is takes
+    if takes:  # what the call itself refuses: padded codes in whole blocks of 8192 from 2^32 on, rows beyond 131071
+        ld = dl._code_row_bytes(K)
+        assert ld % 16 == 0 and K <= ld <= 131071 and (M * ld + 8191) // 8192 * 8192 < 1 << 32
