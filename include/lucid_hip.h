@@ -117,6 +117,9 @@ int lq_event_elapsed_ms(lq_event start, lq_event stop, float* ms);
 int lq_graph_begin(lq_stream stream, int* graph_id);
 int lq_graph_end(lq_stream stream, int graph_id);
 int lq_graph_launch(int graph_id, lq_stream stream);
+/* Whether what is launched on `stream` now is recorded instead of run (whoever began the capture): what a
+ * caller derives once and keeps has to be derived outside. */
+int lq_stream_is_capturing(int* capturing, lq_stream stream);
 int lq_graph_destroy(int graph_id);
 
 /* Op registry: OpSchema{name, version, deterministic}

@@ -80,6 +80,7 @@ _SIGNATURES = {
     "lq_memory_stats": [C.POINTER(_sz), C.POINTER(_sz)],
     "lq_graph_begin": [_vp, C.POINTER(_i)],
     "lq_graph_end": [_vp, _i],
+    "lq_stream_is_capturing": [C.POINTER(_i), _vp],
     "lq_graph_launch": [_i, _vp],
     "lq_graph_destroy": [_i],
     "lq_h2d": [_vp, _vp, _sz, _vp],

@@ -375,6 +375,14 @@ extern "C" int lq_graph_end(lq_stream stream, int graph_id) {
     return LQ_OK;
 }
 
+extern "C" int lq_stream_is_capturing(int* capturing, lq_stream stream) {
+    LQ_REQUIRE(capturing, LQ_ERR_VALUE, "stream_is_capturing: NULL pointer");
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    LQ_HIP(hipStreamIsCapturing(as_stream(stream), &status));
+    *capturing = status != hipStreamCaptureStatusNone;
+    return LQ_OK;
+}
+
 extern "C" int lq_graph_launch(int graph_id, lq_stream stream) {
     hipGraphExec_t exec = nullptr;
     {

@@ -11,10 +11,13 @@ the forward never waits for the host.
 
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 
 from .... import _C, _ops
 from .... import _tensor as T
+from .... import graph as _graph
 from ...._tensor import Tensor
 from ....quantization._functional import minmax, quantize
 from ....quantization._qparams import calculate_qparams
@@ -88,13 +91,12 @@ def fused_pair(first, relu_between: bool, second, x):
     for lin in (first, second):
         if weight_zero_points(lin) is not None or not _kernel_takes(lin):
             return None
-        if lin._wsum is None:
-            lin._wsum = _ops.rowsum_i8(lin.weight_int8)
+    wsum1, wsum2 = first._weight_sums(), second._weight_sums()
     qd = first.act_qdtype
     y = Tensor.empty((*x.shape[:-1], N2), T.float32, "hip")
     _C.call("lq_dynamic_mlp2_small_f32", x.data_ptr, M, K1, b1["weight_int8"].data_ptr, N1, b1["weight_scale"].data_ptr,
-            first._wsum.data_ptr, None if bias1 is None else bias1.data_ptr, int(relu_between),
-            b2["weight_int8"].data_ptr, N2, b2["weight_scale"].data_ptr, second._wsum.data_ptr,
+            wsum1.data_ptr, None if bias1 is None else bias1.data_ptr, int(relu_between),
+            b2["weight_int8"].data_ptr, N2, b2["weight_scale"].data_ptr, wsum2.data_ptr,
             None if bias2 is None else bias2.data_ptr, 0, 0, qd.quant_min, qd.quant_max, int(qd.signed),
             1e-8, storage_offset(qd), y.data_ptr, None)
     return y
@@ -117,11 +119,38 @@ class Linear(Module):
         self._wsum = None
         self._wrows = None
 
+    # (a buffer that is assigned is another weight as much as one that is loaded)
+    def register_buffer(self, name: str, tensor: Tensor | None) -> None:
+        super().register_buffer(name, tensor)
+        self._state_loaded(name)
+
+    def __setattr__(self, name, value) -> None:
+        super().__setattr__(name, value)
+        self._state_loaded(name)
+
     def _state_loaded(self, name: str) -> None:
         if name == "weight_int8":
             self._wsum = self._wrows = None
         if name == "weight_zero_point":
             forget_weight_zero_points(self)
+
+    def _keep(self, name: str, made):
+        """``made``, derived from the weight by work just issued, for the calls to come: once that work is done, since
+        those may run on other streams.  A capture only records the work: it is then part of every replay, and
+        nothing is kept."""
+        capturing = C.c_int()
+        _C.check(_C.load().lq_stream_is_capturing(C.byref(capturing), _C.current_stream()))
+        if not capturing.value and not _graph.is_capturing():
+            _C.call("lq_sync", None)
+            setattr(self, name, made)
+        return made
+
+    def _weight_sums(self) -> Tensor:
+        """The sums of the weight's rows."""
+        kept = self._wsum
+        if kept is not None:
+            return kept
+        return self._keep("_wsum", _ops.rowsum_i8(self._buffers["weight_int8"]))
 
     def _weight_rows(self) -> tuple[Tensor, int]:
         """The weight codes in rows of a multiple of 16 bytes (``weight_int8`` itself where its rows are) and
@@ -130,12 +159,13 @@ class Linear(Module):
         ld = _code_row_bytes(K)
         if ld == K:
             return self._buffers["weight_int8"], K
-        if self._wrows is None:
-            rows = Tensor.empty((N, ld), T.int8, "hip")
-            _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
-            _C.call("lq_d2d_rows", rows.data_ptr, ld, self.weight_int8.data_ptr, K, K, N, None)
-            self._wrows = (rows, ld)
-        return self._wrows
+        kept = self._wrows
+        if kept is not None:
+            return kept
+        rows = Tensor.empty((N, ld), T.int8, "hip")
+        _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
+        _C.call("lq_d2d_rows", rows.data_ptr, ld, self._buffers["weight_int8"].data_ptr, K, K, N, None)
+        return self._keep("_wrows", (rows, ld))
 
     def forward(self, x: Tensor, residual: Tensor | None = None, activation: str | None = None,
                 track_range: bool = False) -> Tensor:
@@ -160,19 +190,18 @@ class Linear(Module):
                 and weight_zero_points(self) is None and _kernel_takes(self)
                 and _one_call_takes(M, K)):
             # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
-            if self._wsum is None:
-                self._wsum = _ops.rowsum_i8(self.weight_int8)
+            wsum = self._weight_sums()
             y = Tensor.empty((*x.shape[:-1], N), T.float32, "hip")
             grid = (0, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, off)
-            scale, wsum = self._buffers["weight_scale"].data_ptr, self._wsum.data_ptr
+            scale = self._buffers["weight_scale"].data_ptr
             b = None if bias is None else bias.data_ptr
             if _one_launch_pays(M, K, N):
-                _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, self._buffers["weight_int8"].data_ptr, N, scale, wsum,
-                        b, *grid, y.data_ptr, None)
+                _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, self._buffers["weight_int8"].data_ptr, N, scale,
+                        wsum.data_ptr, b, *grid, y.data_ptr, None)
             else:
                 w, ldw = self._weight_rows()
-                _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale, wsum, b, *grid,
-                        y.data_ptr if M else None, None)
+                _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale,
+                        wsum.data_ptr, b, *grid, y.data_ptr if M else None, None)
             return y
         xq = Tensor.empty((M, K), T.int8, "hip")
         small = x._range is None and x.numel <= (1 << 18)
@@ -205,8 +234,7 @@ class Linear(Module):
         (``functional.layer_norm_dynamic_quantize``)."""
         N = self.out_features
         off = storage_offset(self.act_qdtype)
-        if self._wsum is None:
-            self._wsum = _ops.rowsum_i8(self.weight_int8)
+        wsum = self._weight_sums()
         rng = None
         w_zp = weight_zero_points(self)
         if track_range and w_zp is not None:
@@ -216,7 +244,7 @@ class Linear(Module):
             from ...functional import _new_range
             rng = _new_range()
         y = _ops.qlinear_i8(xq, self.weight_int8, a_zp=off, a_zp_dev=x_zp, a_scale=x_scale,
-                            w_scale=self.weight_scale, wsum=self._wsum, bias=self.bias,
+                            w_scale=self.weight_scale, wsum=wsum, bias=self.bias,
                             out_mode=_ops.OUT_F32, residual=residual, gelu=activation == "gelu",
                             range_buf=rng, w_zp=w_zp)
         y = y.reshape(*lead_shape, N)

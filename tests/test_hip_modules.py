@@ -599,6 +599,32 @@ def test_dynamic_linear_states_of_other_types_and_sizes(M, K):
             loaded(**bad)(x)
 
 
+@pytest.mark.parametrize("M,K,N", [(4, 50, 24), (70, 50, 24), (1, 1000, 33), (70, 64, 24)])
+def test_dynamic_linear_weight_rows_first_needed_in_a_capture(M, K, N):
+    """Row sums and padded weight rows that a capture needs first are made by its replays only: an eager call before
+    the first replay, and every replay, have the bits of a layer that never was captured."""
+    rng = np.random.default_rng(M + K)
+    state = {"weight_int8": rng.integers(-127, 128, (N, K)).astype(np.int8),
+             "weight_scale": rng.uniform(0.001, 0.01, N).astype(np.float32),
+             "weight_zero_point": np.zeros(N, np.float32), "bias": rng.standard_normal(N).astype(np.float32)}
+    lin, plain = nnqd.Linear(K, N), nnqd.Linear(K, N)
+    for q in (lin, plain):
+        q.load_state_dict({n: hip(v) for n, v in state.items()})
+    x, other = (hip((rng.standard_normal((M, K)) * f).astype(np.float32)) for f in (1, 3))
+    want, want_other = plain(x).numpy(), plain(other).numpy()
+    lin(x, residual=hip(np.zeros((M, N), np.float32)))  # (the zero points are read, by the separate operators)
+    lin._wsum = None
+    with L.graph.capture() as g:
+        y = lin(x)
+    for _ in range(3):
+        assert np.array_equal(lin(other).numpy(), want_other)
+        g.replay()
+        L.synchronize()
+        assert np.array_equal(y.numpy(), want)
+    g.destroy()
+    assert np.array_equal(lin(other).numpy(), want_other)
+
+
 class _recorded_calls:
     """The names of the compute entry points called through the binding while the block runs."""
 

@@ -14,7 +14,6 @@ def _layer(N, K, **other):
     lin = object.__new__(nnqd.Linear)
     Module.__init__(lin)
     lin.in_features, lin.out_features = K, N
-    lin._wsum = lin._wrows = None
     bufs = dict(weight_int8=np.zeros((N, K), np.int8), weight_scale=np.ones(N, np.float32),
                 weight_zero_point=np.zeros(N, np.float32), bias=np.zeros(N, np.float32))
     for name, v in {**bufs, **other}.items():
@@ -47,3 +46,17 @@ def test_one_call_is_for_codes_that_fit_its_rows_and_scratch(M, K, takes):
     if takes:  # what the call itself refuses: padded codes in whole blocks of 8192 from 2^32 on, rows beyond 131071
         ld = dl._code_row_bytes(K)
         assert ld % 16 == 0 and K <= ld <= 131071 and (M * ld + 8191) // 8192 * 8192 < 1 << 32
+
+
+def test_another_weight_forgets_what_was_derived_from_the_last():
+    """Assigned, registered or loaded: the row sums and padded rows are those of the weight that is there."""
+    lin = _layer(8, 30)
+    new = L.Tensor.from_numpy(np.ones((8, 30), np.int8), "cpu")
+    for replace in (lambda: setattr(lin, "weight_int8", new), lambda: lin.register_buffer("weight_int8", new),
+                    lambda: lin.load_state_dict({"weight_int8": new}, strict=False)):
+        lin._wsum = lin._wrows = "of the last weight"
+        replace()
+        assert lin._wsum is None and lin._wrows is None
+    lin._wsum = "of this weight"
+    lin.bias = None
+    assert lin._wsum == "of this weight"
