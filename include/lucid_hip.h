@@ -112,7 +112,9 @@ int lq_event_elapsed_ms(lq_event start, lq_event stop, float* ms);
  * (a created stream, not the default one), then replay it with one launch -
  * for launch-bound inference loops (a quantized ResNet-50 forward is ~75 short
  * kernels).  Memory allocated during capture stays reserved for the graph until
- * lq_graph_destroy.  No counterpart in Lucid (its Metal backend batches lazily
+ * lq_graph_destroy.  The library's scratch of `stream` is part of what is recorded (split-K slabs, partial
+ * min / max, convolution patches, decoded or prepared weight-only operands): do not replay a graph beside another that was
+ * captured on the same stream, or beside eager calls on that stream.  No counterpart in Lucid (its Metal backend batches lazily
  * through MLX instead). */
 int lq_graph_begin(lq_stream stream, int* graph_id);
 int lq_graph_end(lq_stream stream, int graph_id);

@@ -49,6 +49,9 @@ int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream,
 // 5: the range slots of a dynamic quantization; 6: the codes and qparams of a dynamic Linear's activation;
 // 7: the slots of a dynamic quantization in one launch
 int workspace(size_t nbytes, hipStream_t stream, void** ptr);
+// Scratch (kinds 4 to 6) of one call's launches.  While this thread records a graph it is memory of that graph's own:
+// replays may run on any stream, beside each other and beside the stream's eager calls.
+int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr);
 // Held while launches that hand data to each other through a stream's scratch are issued: two threads
 // that use one stream would otherwise interleave them.
 std::unique_lock<std::recursive_mutex> scratch_lock();

@@ -861,7 +861,7 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;
             void* tmp = nullptr;
             const auto lock = scratch_lock();
-            int rc = stream_buffer(4, a_bytes + w_bytes, 0, st, &tmp, nullptr);
+            int rc = call_buffer(4, a_bytes + w_bytes, st, &tmp);
             if (rc == LQ_ERR_OOM && g.range == nullptr) {  // no room for the copies: the plain kernel needs none
                 (void)hipGetLastError();
                 return run_gemm(g_in, 3, tile_config, st);

@@ -1402,7 +1402,7 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
             exchange = capturing == hipStreamCaptureStatusNone;
         }
         const int rc = exchange ? stream_buffer(7, sizeof(DynScratch), 0, st, &tmp, &fresh)
-                                : stream_buffer(5, 2 * kMaxParts * sizeof(float), 0, st, &tmp, nullptr);
+                                : call_buffer(5, 2 * kMaxParts * sizeof(float), st, &tmp);
         if (rc) return rc;
     }
     DynScratch* d = exchange ? static_cast<DynScratch*>(tmp) : nullptr;
@@ -1484,7 +1484,7 @@ int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw
     const size_t code_bytes = (size_t(M) * ldw + 255) / 256 * 256;
     void* tmp = nullptr;
     const auto lock = scratch_lock();
-    int rc = stream_buffer(6, code_bytes + 256, 0, st, &tmp, nullptr);
+    int rc = call_buffer(6, code_bytes + 256, st, &tmp);
     if (rc) return rc;
     int8_t* codes = static_cast<int8_t*>(tmp);
     float* qp = reinterpret_cast<float*>(codes + code_bytes);

@@ -118,6 +118,13 @@ std::unique_lock<std::recursive_mutex> scratch_lock() {
     return std::unique_lock<std::recursive_mutex>(mu);
 }
 
+int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr) {
+    if (!t_capturing_graph) return stream_buffer(kind, nbytes, 0, stream, ptr, nullptr);
+    // pinned to the graph by the allocator, and given back with it
+    const int rc = lq_alloc(ptr, nbytes);
+    return rc ? rc : lq_free(*ptr);
+}
+
 int workspace(size_t nbytes, hipStream_t stream, void** ptr) {
     return stream_buffer(0, nbytes, size_t(4) << 20, stream, ptr, nullptr);
 }

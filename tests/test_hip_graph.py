@@ -263,3 +263,59 @@ def test_vit_b16_batch64_graph_replay_matches_eager():
     g.destroy()
     x.copy_from(batches[2])
     assert np.array_equal(model(x).numpy().view(np.uint32), eager[2].view(np.uint32))
+
+
+def _linear_of(rng, K, N):
+    import lucid_amd.nn.quantized.dynamic as nnqd
+    lin = nnqd.Linear(K, N)
+    lin.load_state_dict({n: L.tensor(v, device="hip") for n, v in {
+        "weight_int8": rng.integers(-127, 128, (N, K)).astype(np.int8),
+        "weight_scale": rng.uniform(0.001, 0.01, N).astype(np.float32),
+        "weight_zero_point": np.zeros(N, np.float32), "bias": rng.standard_normal(N).astype(np.float32)}.items()})
+    return lin
+
+
+@pytest.mark.parametrize("M,K,N", [(70, 512, 48), (600, 500, 130)])
+def test_captured_dynamic_linears_have_codes_of_their_own(M, K, N):
+    """Two layers captured on one stream: their codes, ranges and qparams belong to the graphs, so that replays beside
+    each other on two streams and eager calls on the third one have the bits of calls one after the other."""
+    _C.init()
+    rng = np.random.default_rng(M)
+    lins = [_linear_of(rng, K, N) for _ in range(3)]
+    xs = [L.tensor((rng.standard_normal((M, K)) * f).astype(np.float32), device="hip") for f in (1, 5, 25)]
+    want = [lin(x).numpy() for lin, x in zip(lins, xs)]
+    streams = [C.c_void_p() for _ in range(3)]
+    for s in streams:
+        _C.call("lq_stream_create_nonblocking", C.byref(s))
+    prev, graphs, ys = _C.current_stream(), [], []
+    try:
+        _C.set_current_stream(streams[0])
+        lins[2](xs[2])
+        _C.call("lq_sync", streams[0])
+        for i in (0, 1):
+            used0, used1, res = C.c_size_t(), C.c_size_t(), C.c_size_t()
+            _C.call("lq_memory_stats", C.byref(used0), C.byref(res))
+            gid = C.c_int()
+            _C.call("lq_graph_begin", streams[0], C.byref(gid))
+            ys.append(lins[i](xs[i]))
+            _C.call("lq_graph_end", streams[0], gid)
+            graphs.append(gid)
+            _C.call("lq_memory_stats", C.byref(used1), C.byref(res))
+            assert used1.value - used0.value >= M * N * 4 + M * K  # the output and the codes
+        for _ in range(20):
+            eager = []
+            for _ in range(10):
+                for i in (0, 1):
+                    _C.call("lq_graph_launch", graphs[i], streams[i + 1])
+                eager.append(lins[2](xs[2]))
+            for s in streams:
+                _C.call("lq_sync", s)
+            for i in (0, 1):
+                assert np.array_equal(ys[i].numpy(), want[i])
+            assert all(np.array_equal(y.numpy(), want[2]) for y in eager)
+    finally:
+        _C.set_current_stream(prev)
+        for g in graphs:
+            _C.call("lq_graph_destroy", g)
+        for s in streams:
+            _C.call("lq_stream_destroy", s)
