@@ -52,10 +52,11 @@ int workspace(size_t nbytes, hipStream_t stream, void** ptr);
 // Scratch (kinds 4 to 6) of one call's launches.  While this thread records a graph it is memory of that graph's own:
 // replays may run on any stream, beside each other and beside the stream's eager calls.
 int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr);
-// Held while launches that hand data to each other through a stream's scratch are issued: two threads
-// that use one stream would otherwise interleave them.
-std::unique_lock<std::recursive_mutex> scratch_lock();
-// Split-K scratch of one stream: arrival counters (zero between launches: the finisher of a
+// Held by every user of a stream's scratch from before it asks for the buffer until its last launch on it is issued:
+// two threads that use one stream would otherwise interleave launches that hand data to each other, or free
+// a buffer that the other one has outgrown before it is launched on.  One per (device, stream).
+std::unique_lock<std::recursive_mutex> scratch_lock(hipStream_t stream);
+// Split-K scratch of one stream (the caller holds its scratch_lock): arrival counters (zero between launches: the finisher of a
 // tile resets its counter) and slabs for the partial results, whose layout the kernel defines.
 struct SkScratch {
     int* counters = nullptr;

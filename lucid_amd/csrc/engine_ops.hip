@@ -331,6 +331,7 @@ int lq_batchnorm_eval_f32(const float* x, float* out, size_t B, int C, size_t sp
     LQ_REQUIRE(x && out && mean && var, LQ_ERR_VALUE, "batchnorm_eval_f32: NULL pointer");
     hipStream_t st = as_stream(stream);
     void* ws = nullptr;
+    const auto lock = scratch_lock(st);
     int rc = workspace(size_t(C) * 4, st, &ws);
     if (rc) return rc;
     float* rstd = static_cast<float*>(ws);

@@ -621,6 +621,7 @@ int lq_qconv2d_i8(const lq_qconv2d_args* p, lq_stream stream) {
         const size_t ones_bytes = size_t(p->groups) * K;
         void* tmp = nullptr;
         bool fresh = false;
+        const auto lock = scratch_lock(st);
         int rc = stream_buffer(3, acc_bytes + sum_bytes + ones_bytes, 0, st, &tmp, &fresh);
         if (rc) return rc;
         int32_t* acc = static_cast<int32_t*>(tmp);
@@ -666,6 +667,7 @@ int lq_qconv2d_i8(const lq_qconv2d_args* p, lq_stream stream) {
         LQ_REQUIRE(size_t(p->B) * Hp * Wp * 4 < 0xffffffffull, LQ_ERR_SHAPE, "qconv2d_i8: padded image too large");
         const int8_t* img = p->x;
         const int8_t* flt = p->w;
+        const auto lock = scratch_lock(st);
         if (path == 5) {
             const size_t img_bytes = (size_t(p->B) * Hp * Wp * 4 + 255) / 256 * 256;
             const size_t flt_bytes = (size_t(p->Cout) * p->KH * KWp * 4 + 255) / 256 * 256;
@@ -717,6 +719,7 @@ int lq_qconv2d_i8(const lq_qconv2d_args* p, lq_stream stream) {
     const size_t cols_bytes = (M * Kp + 255) / 256 * 256;
     const size_t w_bytes = (size_t(Og) * Kp + 255) / 256 * 256;
     void* ws = nullptr;
+    const auto lock = scratch_lock(st);
     int rc = workspace(cols_bytes + w_bytes, st, &ws);
     if (rc) return rc;
     int8_t* cols = static_cast<int8_t*>(ws);
@@ -822,6 +825,7 @@ int lq_qconv3d_i8(const lq_qconv3d_args* p, lq_stream stream) {
         const size_t ones_bytes = size_t(p->groups) * K;
         void* tmp = nullptr;
         bool fresh = false;
+        const auto lock = scratch_lock(st);
         int rc = stream_buffer(3, acc_bytes + sum_bytes + ones_bytes, 0, st, &tmp, &fresh);
         if (rc) return rc;
         int32_t* acc = static_cast<int32_t*>(tmp);

@@ -860,7 +860,7 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
             const int ld = (g.K + 63) / 64 * 64;
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;
             void* tmp = nullptr;
-            const auto lock = scratch_lock();
+            const auto lock = scratch_lock(st);
             int rc = call_buffer(4, a_bytes + w_bytes, st, &tmp);
             if (rc == LQ_ERR_OOM && g.range == nullptr) {  // no room for the copies: the plain kernel needs none
                 (void)hipGetLastError();
@@ -1114,6 +1114,7 @@ int lq_qlinear_i8(const lq_qlinear_args* p, lq_stream stream) {
         hipStream_t st = as_stream(stream);
         void* tmp = nullptr;
         bool fresh = false;
+        const auto lock = scratch_lock(st);
         const size_t acc_bytes = (size_t(p->M) * p->N * 4 + 255) / 256 * 256;
         int rc = stream_buffer(3, acc_bytes + size_t(p->M) * 4, 0, st, &tmp, &fresh);
         if (rc) return rc;

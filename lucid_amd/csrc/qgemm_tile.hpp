@@ -924,6 +924,7 @@ int launch_tile_mode(const GemmArgs& g, int groups, int schedule, hipStream_t st
         workers = long(tiles) * (split < 1 ? 1 : split);
     }
     SkScratch s;
+    const auto lock = scratch_lock(st);
     const size_t slab_words = size_t(Cfg::TM) * Cfg::TN * 16 * Cfg::THREADS;
     int rc = sk_scratch(size_t(sk_tiles) * groups, size_t(groups) * workers * 2 * slab_words * 4, st, &s);
     if (rc) return rc;

@@ -1393,7 +1393,7 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
     bool exchange = blocks <= size_t(kExchange), fresh = false;
     std::unique_lock<std::recursive_mutex> lock;
     if (blocks > 1) {
-        lock = scratch_lock();
+        lock = scratch_lock(st);
         if (exchange) {
             // not in a graph: slots first cleared there would be unset until its replay, and replays on
             // another stream would share them with this one
@@ -1483,7 +1483,7 @@ int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw
     // codes (rows as long as the weight's), scale and zero point, then the GEMM
     const size_t code_bytes = (size_t(M) * ldw + 255) / 256 * 256;
     void* tmp = nullptr;
-    const auto lock = scratch_lock();
+    const auto lock = scratch_lock(st);
     int rc = call_buffer(6, code_bytes + 256, st, &tmp);
     if (rc) return rc;
     int8_t* codes = static_cast<int8_t*>(tmp);
@@ -1517,6 +1517,7 @@ int lq_dynamic_mlp2_small_f32(const float* x, int M, int K1, const int8_t* w1, i
     const float half_range = float((double(qmax) - double(qmin)) / 2.0);
     // the hidden activation and the tiles' ranges pass through the stream's split-K scratch
     SkScratch sk;
+    const auto lock = scratch_lock(as_stream(stream));
     const size_t hid_bytes = size_t(M) * N1 * 4;
     if (int rc = sk_scratch(1, hid_bytes + 512, as_stream(stream), &sk)) return rc;
     const size_t lds = size_t(16) * K1 + 1024 + size_t(64) * N1;
@@ -1592,6 +1593,7 @@ int lq_quantize_rows_dynamic_i8(const float* x, size_t rows, size_t cols, int sy
 int lq_minmax(const float* x, size_t outer, size_t C, size_t inner, float* mn, float* mx,
               lq_stream stream) {
     hipStream_t st = as_stream(stream);
+    const auto lock = scratch_lock(st);
     return minmax_launch(x, outer, C, inner, mn, mx, st, ~size_t(0),
                          [st](size_t nbytes, void** ws) { return workspace(nbytes, st, ws); });
 }

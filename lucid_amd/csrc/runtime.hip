@@ -113,9 +113,13 @@ int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream,
     return LQ_OK;
 }
 
-std::unique_lock<std::recursive_mutex> scratch_lock() {
-    static std::recursive_mutex mu;
-    return std::unique_lock<std::recursive_mutex>(mu);
+std::unique_lock<std::recursive_mutex> scratch_lock(hipStream_t stream) {
+    // (two streams that share an entry only wait for each other's launches)
+    static std::recursive_mutex mu[64];
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    const uint64_t h = (reinterpret_cast<uintptr_t>(stream) + uint64_t(dev)) * 0x9e3779b97f4a7c15ull;
+    return std::unique_lock<std::recursive_mutex>(mu[h >> 58]);
 }
 
 int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr) {

@@ -342,7 +342,7 @@ int launch_rows(const float* x, const uint32_t* packed, const float* scales, con
     const size_t sum_bytes = size_t(stages) * SEGS * mtiles * 16 * 4 + kPiece;
     const size_t sb_bytes = size_t(stages) * SEGS * n_pad * 8 + kPiece;
     void* ws = nullptr;
-    const auto lock = scratch_lock();
+    const auto lock = scratch_lock(st);
     const int rc = workspace(part_bytes + sum_bytes + sb_bytes, st, &ws);
     if (rc) return rc;
     char* parts = static_cast<char*>(ws);

@@ -576,6 +576,7 @@ int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, 
     const int mblocks = (M + 15) / 16, windows = (K + G::WK - 1) / G::WK;
     const int tiles = (N + kWqRows - 1) / kWqRows, slices = (windows + WPS - 1) / WPS;
     SkScratch sk;
+    const auto lock = scratch_lock(st);
     if (slices > 1) {
         const int rc = sk_scratch(size_t(mblocks) * tiles, size_t(mblocks) * tiles * slices * (8 * 2 * 64 * 16), st, &sk);
         if (rc) return rc;
@@ -683,6 +684,7 @@ int lq_wq_matmul(const float* x, const uint32_t* packed, const float* scales, co
     }
     // operands that are not 16-byte aligned, large batches on such a weight: decode once into the workspace, then the float32 MFMA GEMM
     void* ws = nullptr;
+    const auto lock = scratch_lock(st);
     rc = workspace(size_t(N) * K * sizeof(float), st, &ws);
     if (rc) return rc;
     rc = lq_wq_dequantize(packed, scales, biases, N, K, group_size, bits, static_cast<float*>(ws), stream);

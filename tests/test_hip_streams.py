@@ -102,3 +102,40 @@ def test_fork_and_join_with_events_on_non_blocking_streams():
             _C.call("lq_event_destroy", e)
     with pytest.raises(ValueError, match="event is NULL"):
         _C.call("lq_stream_wait_event", None, None)
+
+
+def test_threads_in_different_calls_share_one_streams_scratch():
+    """Threads on one stream whose calls use the same scratch for other things: prepared weight-only operands,
+    two-stage min / max, histograms, split-K slabs, codes.  Sizes grow while they run, so buffers are outgrown."""
+    import threading
+    import lucid_amd.quantization as Q
+    from lucid_amd.quantization import _qgemm
+    _C.init()
+    rng = np.random.default_rng(4)
+    w = _qgemm.quantize(L.tensor((rng.standard_normal((1100, 512)) * 0.02).astype(np.float32), device="hip"), 64, 4)
+    xs = [L.tensor(rng.standard_normal((m, 512)).astype(np.float32), device="hip") for m in (300, 900, 2500)]
+    big = [L.tensor(rng.standard_normal(n).astype(np.float32), device="hip") for n in (300_000, 1 << 21, 5_000_000)]
+    cols = [L.tensor(rng.standard_normal((r, 300)).astype(np.float32), device="hip") for r in (2000, 9000, 30_000)]
+    a8, w8 = (L.tensor(rng.integers(-128, 128, s, dtype=np.int8), device="hip") for s in ((256, 8192), (256, 8192)))
+    hist = L.Tensor.empty((1000,), L.float32, "hip")
+
+    def histogram(i):
+        _C.call("lq_histc_f32", big[i].data_ptr, big[i].numel, -3.0, 3.0, 1000, hist.data_ptr, None)
+        return (hist,)
+
+    work = [lambda i: (_qgemm.quantized_matmul(xs[i], *w, True, 64, 4),), lambda i: Q.minmax(big[i]),
+            lambda i: Q.minmax(cols[i], ch_axis=1), histogram, lambda i: (_linear(a8, w8, 5 | (2 << 8)),)]
+    want = [[tuple(t.numpy().copy() for t in f(i)) for i in range(3)] for f in work]
+    go, bad = threading.Barrier(len(work)), []
+
+    def run(f, expected):
+        go.wait()
+        for rep in range(30):
+            i = rep % 3
+            if not all(np.array_equal(t.numpy(), e) for t, e in zip(f(i), expected[i])):
+                bad.append(f)
+
+    threads = [threading.Thread(target=run, args=a) for a in zip(work, want)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad
