@@ -38,9 +38,6 @@ namespace {
 
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 
-template <int BITS>
-constexpr int kOffset = BITS == 4 ? 16 : 0;  // how codes enter the products, see wq_codes
-
 constexpr int kPiece = 1024;  // bytes one wavefront moves into LDS with one instruction
 
 // One launch, two kinds of blocks.  The first `split_blocks`: one thread = eight consecutive k of one
@@ -67,7 +64,7 @@ __global__ __launch_bounds__(256) void wq_prepare_kernel(const float* __restrict
         for (int e = 0; e < 4; ++e)
             for (int r = 0; r < per; ++r)
                 if ((g0 + e) * per + r < stages * segs)
-                    sb[size_t((g0 + e) * per + r) * n_pad + n] = float2{s[e], b[e] - float(kOffset<BITS>) * s[e]};
+                    sb[size_t((g0 + e) * per + r) * n_pad + n] = float2{kWqUnit<BITS, kWqCentre<BITS>> * s[e], b[e] - float(kWqCentre<BITS>) * s[e]};
         return;
     }
     const unsigned pairs = unsigned(stages + 1) / 2;
@@ -278,7 +275,7 @@ void wq_gemm_kernel(const char* __restrict__ parts, const char* __restrict__ xsu
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
                     const uint32_t w4[4] = {wd[ii][j][0], wd[ii][j][1], 0u, 0u};
-                    cf[j] = __builtin_bit_cast(v8bf, wq_codes<BITS, kOffset<BITS>>(w4, 0));
+                    cf[j] = __builtin_bit_cast(v8bf, wq_codes<BITS, kWqCentre<BITS>>(w4, 0));
                 }
 #pragma unroll
                 for (int i = 0; i < MT; ++i)

@@ -257,8 +257,7 @@ int launch_gemv1(const float* x, const uint32_t* packed, const float* scales, co
 //
 // y[m, n] = sum over groups g of  s[n, g] * (sum_{k in g} c[n, k] x[m, k])  +  b[n, g] * (sum_{k in g} x[m, k]):
 // the inner sums run on v_mfma_f32_16x16x32_bf16 with the codes themselves as one operand -
-// an 8-bit code is exact in bfloat16, a 4-bit code c is formed as the bit pattern of OFF + c
-// (wq_codes) and the OFF goes into the bias term - and x as the
+// a code c enters exactly as c + OFF (wq_codes) and the OFF goes into the bias term - and x as the
 // other, split into three bfloat16 parts x = hi + mid + lo (exact: 8 + 8 + 8 significant
 // bits, wq_split3x2), one MFMA each.  Products are exact and accumulate in float32, so nothing of x or
 // of the weight is rounded before the sums.
@@ -492,9 +491,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                 for (int rb = 0; rb < RB; ++rb) {
                     const float sc = s_lds[(row_in_tile + rb * 16) * gp + g];
                     const float bi = b_lds[(row_in_tile + rb * 16) * gp + g];
-                    // the 4-bit codes entered as OFF + c
-                    const float bz = BITS == 4 ? bi - float(OFF) * sc : bi;
-                    y[rb] = y[rb] + (acc[rb] * sc + acc[RB] * bz);
+                    // the codes entered as (c + OFF) / unit
+                    const float bz = OFF != 0 ? bi - float(OFF) * sc : bi;
+                    y[rb] = y[rb] + (acc[rb] * (kWqUnit<BITS, OFF> * sc) + acc[RB] * bz);
                 }
             }
         }
@@ -585,9 +584,9 @@ int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, 
     const int gs_shift = 31 - __builtin_clz(unsigned(gs));
     const int gmax = kWqSliceK / gs;
     const size_t lds = size_t(WPS) * G::NI * 3 * 64 * 16 + size_t(2) * kWqRows * ((gmax < 1 ? 1 : gmax) + 1) * 4;
-    // 2 .. 64 rows of whole windows keep the offset, and so the bits, that they have always had
-    constexpr int kFirst = BITS == 4 ? 128 : 0, kOther = BITS == 4 ? 16 : 0;
-    const bool first = BITS == 8 || (M > 1 && M <= 64 && K % G::WK == 0);
+    // 2 .. 64 rows of whole windows keep the offset, and so the bits, that they have always had here
+    constexpr int kFirst = BITS == 4 ? 128 : 0, kOther = kWqCentre<BITS>;
+    const bool first = M > 1 && M <= 64 && K % G::WK == 0;
 #define LQ_WQ_LAUNCH(SWM)                                                                                         \
     do {                                                                                                          \
         if (first)                                                                                                \

@@ -100,6 +100,34 @@ def test_large_batch_matmul_is_exact_on_exact_inputs(M, N, K, gs, bits):
     assert np.array_equal(y, x @ W.dequantize(packed, s, b, gs, bits).T)
 
 
+@pytest.mark.parametrize("bits,gs", [(4, 32), (4, 64), (4, 128), (8, 32), (8, 128)])
+@pytest.mark.parametrize("M,K", [(333, 2048), (80, 4096), (20, 2048 + 32)])  # large batch, small batch, its partial window
+@pytest.mark.parametrize("kind", ["normal", "relu", "mean1"])
+def test_matmul_is_no_further_from_float64_than_decoding_first(M, K, bits, gs, kind):
+    """Whatever the mean of the activations: the relative error against float64 is at most that of decoding the
+    weight and a float32 product (which an x that is not 16-byte aligned takes)."""
+    if K % gs:
+        K += gs - K % gs
+    if M <= 64 and K % (512 // bits) == 0:
+        pytest.skip("2 to 64 rows of whole windows keep uncentred codes")
+    rng = np.random.default_rng(M + gs)
+    N = 1024
+    packed, s, b = _qgemm.quantize(hip((rng.standard_normal((N, K)) * 0.02).astype(np.float32)), gs, bits)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x = {"normal": x, "relu": np.maximum(x, 0), "mean1": x + np.float32(1)}[kind]
+    per = 32 // bits
+    codes = (packed.numpy().view(np.uint32)[:, :, None] >> (np.arange(per, dtype=np.uint32) * bits)) & ((1 << bits) - 1)
+    w = (codes.reshape(N, K // gs, gs).astype(np.float64) * s.numpy().astype(np.float64)[:, :, None]
+         + b.numpy().astype(np.float64)[:, :, None]).reshape(N, K)
+    want = x.astype(np.float64) @ w.T
+    shifted = np.zeros(M * K + 1, np.float32)
+    shifted[1:] = x.reshape(-1)
+    view = L.Tensor((M, K), L.float32, "hip", buf=hip(shifted)._buf, offset=4)
+    err, bound = (np.linalg.norm(_qgemm.quantized_matmul(v, packed, s, b, True, gs, bits).numpy() - want) / np.linalg.norm(want)
+                  for v in (hip(x), view))
+    assert err <= bound
+
+
 @pytest.mark.parametrize("M,N,K,gs", [(1_500_003, 3, 128, 64),   # two chunks of rows, the second one ragged
                                       (11_200_000, 2, 128, 64)])  # operands of more than 2^32 bytes between stages
 def test_matmul_of_very_many_rows(M, N, K, gs):
