@@ -25,8 +25,10 @@
 // all, which with two wavefronts per SIMD (one hides the other's scaling and LDS reads) caps MT NT at 12.
 //
 // The sums of a group are scaled while the next group is multiplied (two sets of accumulators take turns).
-// 333 x 11008 x 4096, int4, groups of 128: 100 us, 0.90 PFLOP/s in bfloat16 terms (a library product of plain
+// 333 x 11008 x 4096, int4, groups of 128: 112 us, 0.80 PFLOP/s in bfloat16 terms (a library product of plain
 // bfloat16 operands reaches 1.18 on the card); decoding to float32 (109 us) and a float32 GEMM (286 us) before.
+// Of the 112, 11 are for centred codes (wq_codes): their decode is vector work that the matrix instructions do not
+// hide.  (Interleaving the two by scheduling groups, two or three vector instructions per matrix one: 114.)
 //
 // The codes' 16-byte chunks are placed in LDS at chunk ^ (row / 4) (int8) or chunk ^ (row / 8) (int4), which
 // spreads the 16 rows of an operand read over all banks; the permutation is applied on the global side.
@@ -312,7 +314,8 @@ struct Tile {
 };
 // The block tile whose blocks take the least time: rounds of 256 blocks times a stage of 64 k, which is
 // 0.38 us (barrier, LDS reads, loads) + 0.125 us per 16 x 16 x 8 tiles of a block.  Measured at K = 4096:
-// 32 x 128 tiles 0.63 us per stage, 64 x 128 and 32 x 256 0.95, 64 x 256 1.45, 96 x 192 1.5, 96 x 256 1.95.
+// 32 x 128 tiles 0.63 us per stage, 64 x 128 and 32 x 256 0.95, 64 x 256 1.45, 96 x 192 1.5, 96 x 256 1.95
+// (8-bit codes; centred 4-bit ones take about a tenth more in every shape, which changes no choice).
 Tile wq_gemm_tile(int M, int N, int stages) {
     static const int tiles[][2] = {{3, 4}, {3, 3}, {2, 4}, {2, 2}, {1, 4}, {1, 2}};
     Tile best{0, 0, 0.0f};
@@ -404,13 +407,16 @@ namespace lq {
 
 // The small-batch kernel splits K between its blocks (512 k each), so it fills the chip where M x N alone
 // does not, but reads and decodes the weight once per 16 rows: 8 us + 31 ns (int4) or 38 ns (int8) per block.
-// This one prepares its operands first (7 us).  Measured either side (us, small batch / this): 65 x 11008 x
-// 4096 int4 59 / 66, 96 rows 71 / 68, 128 rows 93 / 70; 400 x 1000 x 4096 30 / 47, 1024 rows 59 / 55;
-// 1024 x 300 x 8192 64 / 88.
+// This one prepares its operands first (7 us).  Both timed over 17 .. 512 rows, N 300 .. 32000, K 1024 .. 11008 and
+// every group size: what this picks is 0.7 % slower than the better one on average; from 65 rows 1.6 x at worst (512 x
+// 1000 x 1024: 12.7 / 20.1 us), 3 % of the problems by more than 5 %.  Up to 64 rows the estimates are closer together,
+// so it has to be a tenth the faster one (0.4 % on average, 1.2 x at worst; with the small-batch kernel for all of them
+// 11 % and 2.6 x).  us, small batch / this: 64 x 32000 x 4096 int4 groups of 128 131 / 74, int8 of 64 156 / 98;
+// 64 x 11008 x 4096 int4 of 64 46 / 56.
 bool wq_gemm_beats_small_batch(int M, int N, int K, int gs, int bits) {
     if (size_t(N) * K * bits / 8 >= 0x7fffffffull) return false;  // its weight offsets are 32-bit
     const double blocks = double((M + 15) / 16) * ((N + 255) / 256) * ((K + 511) / 512);
-    return 7.0 + wq_gemm_tile(M, N, wq_stages(K, gs)).us < 8.0 + blocks * (bits == 4 ? 0.031 : 0.038);
+    return 7.0 + wq_gemm_tile(M, N, wq_stages(K, gs)).us < (M <= 64 ? 0.9 : 1.0) * (8.0 + blocks * (bits == 4 ? 0.031 : 0.038));
 }
 
 int launch_wq_gemm(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
