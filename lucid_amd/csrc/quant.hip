@@ -663,6 +663,7 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
     const float4* __restrict__ x, int quads, int symmetric, int qmin, int qmax, int is_signed, float eps,
     float half_range, int off, float* __restrict__ scale, float* __restrict__ zp, float* __restrict__ mn_out,
     float* __restrict__ mx_out, Code8x4* __restrict__ q) {
+    __shared__ float s_sz[2];
     const size_t row = blockIdx.x;
     const float4* xr = x + row * size_t(quads);
     float4 v[R];
@@ -676,16 +677,19 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
         }
     }
     m = mm_block_reduce(m);
-    const float qnan = __builtin_nanf("");
-    const float mn = m.nan ? qnan : m.lo, mx = m.nan ? qnan : m.hi;
-    float s, z;
-    qparams_of(mn, mx, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
+    // (one thread's division: other blocks have the SIMDs meanwhile, and would wait for everybody's)
     if (threadIdx.x == 0) {
+        const float qnan = __builtin_nanf("");
+        const float mn = m.nan ? qnan : m.lo, mx = m.nan ? qnan : m.hi;
+        float s, z;
+        qparams_of(mn, mx, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
         scale[row] = s, zp[row] = z;
         if (mn_out) mn_out[row] = mn;
         if (mx_out) mx_out[row] = mx;
+        s_sz[0] = s, s_sz[1] = z;
     }
-    const float r = 1.0f / s;
+    __syncthreads();
+    const float s = s_sz[0], z = s_sz[1], r = 1.0f / s;
     const QuantizeOp<int8_t> op{nullptr, nullptr, float(double(qmin)), float(double(qmax)), off};
     Code8x4* qr = q + row * size_t(quads);
 #pragma unroll
