@@ -57,14 +57,16 @@ def _one_call_takes(M: int, K: int) -> bool:
     return ld <= 131071 and M * ld <= MAX_CODE_BYTES
 
 
-def _kernel_takes(lin) -> bool:
-    """Whether ``lin`` holds what the one-call kernels read by address.  A loaded state may hold other types or
-    sizes, or a weight that is an unaligned view: the separate operators take those, or refuse them."""
-    b, N = lin._buffers, lin.out_features
-    w, scale, bias = b["weight_int8"], b["weight_scale"], b["bias"]
-    return (w.shape == (N, lin.in_features) and w.dtype is T.int8 and w._offset % 16 == 0
-            and scale.shape == (N,) and scale.dtype is T.float32
-            and (bias is None or (bias.shape == (N,) and bias.dtype is T.float32)))
+def _kernel_operands(lin, N: int, K: int):
+    """Weight, scales and bias of ``lin`` if they are what the one-call kernels read by address, else ``None``.  A
+    loaded state may hold other types or sizes, or a weight that is an unaligned view: the separate operators take
+    those, or refuse them.  (Straight from the registry, and once: these calls are bound by what they cost the host.)"""
+    b, f32, n = lin._buffers, T.float32, (N,)
+    w, scale, bias = taken = b["weight_int8"], b["weight_scale"], b["bias"]
+    if (w.dtype is T.int8 and w.shape == (N, K) and not w._offset & 15 and scale.dtype is f32 and scale.shape == n
+            and (bias is None or bias.dtype is f32 and bias.shape == n)):
+        return taken
+    return None
 
 
 def fused_pair(first, relu_between: bool, second, x):
@@ -85,20 +87,19 @@ def fused_pair(first, relu_between: bool, second, x):
         return None
     if first.act_qdtype is not second.act_qdtype:
         return None
-    # (the buffers straight from the registries: this path is bound by what a forward costs the host)
-    b1, b2 = first._buffers, second._buffers
-    bias1, bias2 = b1.get("bias"), b2.get("bias")
-    for lin in (first, second):
-        if weight_zero_points(lin) is not None or not _kernel_takes(lin):
-            return None
+    if weight_zero_points(first) is not None or weight_zero_points(second) is not None:
+        return None
+    taken1, taken2 = _kernel_operands(first, N1, K1), _kernel_operands(second, N2, N1)
+    if taken1 is None or taken2 is None:
+        return None
+    (w1, scale1, bias1), (w2, scale2, bias2) = taken1, taken2
     wsum1, wsum2 = first._weight_sums(), second._weight_sums()
     qd = first.act_qdtype
     y = Tensor.empty((*x.shape[:-1], N2), T.float32, "hip")
-    _C.call("lq_dynamic_mlp2_small_f32", x.data_ptr, M, K1, b1["weight_int8"].data_ptr, N1, b1["weight_scale"].data_ptr,
-            wsum1.data_ptr, None if bias1 is None else bias1.data_ptr, int(relu_between),
-            b2["weight_int8"].data_ptr, N2, b2["weight_scale"].data_ptr, wsum2.data_ptr,
-            None if bias2 is None else bias2.data_ptr, 0, 0, qd.quant_min, qd.quant_max, int(qd.signed),
-            1e-8, storage_offset(qd), y.data_ptr, None)
+    _C.call("lq_dynamic_mlp2_small_f32", x.data_ptr, M, K1, w1.data_ptr, N1, scale1.data_ptr, wsum1.data_ptr,
+            None if bias1 is None else bias1.data_ptr, int(relu_between),
+            w2.data_ptr, N2, scale2.data_ptr, wsum2.data_ptr, None if bias2 is None else bias2.data_ptr, 0, 0,
+            qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, storage_offset(qd), y.data_ptr, None)
     return y
 
 
@@ -185,22 +186,21 @@ class Linear(Module):
         M = x.numel // K
         qd = self.act_qdtype
         off = storage_offset(qd)
-        bias = self._buffers["bias"]
         if (x._range is None and residual is None and activation is None and not track_range
-                and weight_zero_points(self) is None and _kernel_takes(self)
-                and _one_call_takes(M, K)):
+                and weight_zero_points(self) is None and _one_call_takes(M, K)
+                and (taken := _kernel_operands(self, N, K)) is not None):
             # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
+            w, scale, bias = taken
             wsum = self._weight_sums()
             y = Tensor.empty((*x.shape[:-1], N), T.float32, "hip")
             grid = (0, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, off)
-            scale = self._buffers["weight_scale"].data_ptr
             b = None if bias is None else bias.data_ptr
             if _one_launch_pays(M, K, N):
-                _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, self._buffers["weight_int8"].data_ptr, N, scale,
+                _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, w.data_ptr, N, scale.data_ptr,
                         wsum.data_ptr, b, *grid, y.data_ptr, None)
             else:
                 w, ldw = self._weight_rows()
-                _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale,
+                _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale.data_ptr,
                         wsum.data_ptr, b, *grid, y.data_ptr if M else None, None)
             return y
         xq = Tensor.empty((M, K), T.int8, "hip")

@@ -32,7 +32,7 @@ def _layer(N, K, **other):
 ])
 def test_kernels_read_by_address_only_what_they_expect(other, takes):
     """Sizes, types and the weight's alignment: all else is left to the operators that check."""
-    assert dl._kernel_takes(_layer(8, 32, **other)) is takes
+    assert (dl._kernel_operands(_layer(8, 32, **other), 8, 32) is not None) is takes
 
 
 @pytest.mark.parametrize("M,K,takes", [
