@@ -217,6 +217,11 @@ typedef struct lq_lstm_args {
     float* y[LQ_LSTM_PARTS];    /* per layer: [steps, batch, directions*hidden], or [batch, steps, ...] when batch_first */
     int steps, batch, inputs, hidden, layers, directions, batch_first; /* hidden at most 1024 (LQ_ERR_NOT_IMPLEMENTED beyond) */
 } lq_lstm_args;
+/* Whether lq_lstm_sequence_f32 fits the device and is faster than a GEMM and lq_lstm_cell_f32 per step (large batches
+ * go through it in many launches).  What fits depends on the hardware queues of the process (GPU_MAX_HW_QUEUES, read at
+ * the first call); streams of another priority than the default have queues of their own beside those: run no recurrences
+ * on both at once. */
+int lq_lstm_sequence_pays(int batch, int hidden, int directions, int* pays);
 /* How many of `layers` stacked layers the next call should take with x given (0: take gates_x). */
 int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layers, int directions, int* fused);
 int lq_lstm_sequence_f32(const lq_lstm_args* args, lq_stream stream);

@@ -29,14 +29,16 @@
 // there - no flags, no barrier, one memory trip each way per step.
 //
 // Progress.  A block waits only for blocks of its own launch, so all of them have to be resident: the
-// launcher bounds the grid by a quarter of what the device holds of this kernel (streams share four
-// hardware queues, and a queue starts a launch only after the one before it is fully placed), and
-// larger batches run as several launches.  A wait is bounded besides: after kSpinLimit reads the
-// block stops waiting for the rest of the sequence and the output keeps its NaNs.
+// launcher bounds the grid by what the device holds of this kernel over the number of hardware queues
+// that streams share (four unless GPU_MAX_HW_QUEUES says more; a queue starts a launch only after the one
+// before it is fully placed), and larger batches run as several launches.  A wait is bounded besides:
+// after kSpinLimit reads the block stops waiting for the rest of the sequence and the output keeps its NaNs.
 //
 // hidden 512, 16 rows: 3.4 us per step with gx, 3.8 with the input product; two such layers of 64 steps
 // 272 us per call, against 580 us as two launches with a GEMM (43 us with the decoding of its weight) each
 // and 4.67 ms with a float32 GEMM, a gate kernel and the host's share of their launches per step.
+#include <cmath>
+#include <cstdlib>
 #include <type_traits>
 #include "common.hpp"
 
@@ -323,6 +325,16 @@ __global__ __launch_bounds__(256) void lstm_empty_kernel(LstmArgs p) {
     for (long i = long(blockIdx.x) * 256 + threadIdx.x; i < p.y_elems; i += stride) y[i] = __uint_as_float(kEmpty);
 }
 
+// Launches that may be placed at once: the hardware queues of the process, which HIP takes from the environment.
+int hardware_queues() {
+    static const int n = [] {
+        const char* v = std::getenv("GPU_MAX_HW_QUEUES");
+        const long q = v ? std::strtol(v, nullptr, 10) : 0;
+        return q > 4 ? int(q < 1024 ? q : 1024) : 4;
+    }();
+    return n;
+}
+
 // Launches of one kernel form: 16-row groups of one direction or of one stack, as many at once as may be.
 struct LstmSplit {
     int per_group, groups, at_once, both;  // blocks of a group; groups; groups of a launch; its parts
@@ -347,7 +359,7 @@ int split_lstm(int B, int H, int parts, bool stacked, LstmSplit* out) {
     LstmSplit s;
     s.per_group = (H + kUnits - 1) / kUnits;
     s.groups = (B + kRows - 1) / kRows;
-    const int fit = capacity[dev] / 4 / s.per_group;
+    const int fit = capacity[dev] / hardware_queues() / s.per_group;
     s.both = stacked || fit >= parts ? parts : 1;
     s.at_once = fit / s.both < s.groups ? fit / s.both : s.groups;
     s.launches = s.at_once < 1 ? 0 : (parts / s.both) * ((s.groups + s.at_once - 1) / s.at_once);
@@ -397,10 +409,37 @@ int with_form(int hidden, int inputs, F f) {
                    : f(integral_constant<int, 8>(), integral_constant<int, 2>(), integral_constant<int, 2>());
 }
 constexpr int kMaxFused = 512;  // hidden and input columns of a form that takes the input product
+constexpr int kMaxHidden = 1024;
+
+// A step of all rows: one launch of the recurrence per rows that fit the device, or a float32 GEMM and a gate kernel
+// (lq_lstm_cell_f32) on decoded weights, issued from Python.  Measured, us per step of both: hidden 64, 8192 rows 25.7 /
+// 32.9; 128, 4096 rows 25.6 / 35.4, 8192 rows 46.9 / 47.2; 256, 1024 rows 29.6 / 37.4, 2048 rows 57.9 / 43.1; 512, 512
+// rows 37 / 49, 1024 rows 73 / 56; 768, 128 rows 41 / 58, 256 rows 80 / 60; 1024, 128 rows 46 / 71, 256 rows 89 / 73,
+// 4096 rows 1399 / 289; 1024 in two directions, 16 rows 15 / 130, 256 rows 180 / 146.  The estimates are within 20 %.
+double sequence_step_us(int hidden) { return 2.9 + 0.0026 * hidden; }
+double gemm_step_us(int batch, int hidden) {
+    const double least = 17.0 + 0.05 * hidden, rows = batch * (2.8e-5 * hidden + 3.8e-8 * hidden * hidden);
+    return std::sqrt(least * least + rows * rows);
+}
 
 }  // namespace
 
 extern "C" {
+
+int lq_lstm_sequence_pays(int batch, int hidden, int directions, int* pays) {
+    LQ_REQUIRE(pays, LQ_ERR_VALUE, "lstm_sequence_pays: NULL pointer");
+    LQ_REQUIRE(batch >= 0 && hidden > 0, LQ_ERR_SHAPE, "lstm_sequence_pays: bad extent (%d, %d)", batch, hidden);
+    LQ_REQUIRE(directions == 1 || directions == 2, LQ_ERR_VALUE, "lstm_sequence_pays: directions must be 1 or 2");
+    *pays = 0;
+    if (batch == 0 || hidden > kMaxHidden) return LQ_OK;
+    LstmSplit s;
+    const int rc = with_form(hidden, 0, [&](auto w, auto k, auto x) {
+        return split_lstm<w(), k(), x()>(batch, hidden, directions, false, &s);
+    });
+    if (rc) return rc;
+    *pays = s.launches > 0 && s.launches * sequence_step_us(hidden) <= directions * gemm_step_us(batch, hidden);
+    return LQ_OK;
+}
 
 int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layers, int directions, int* fused) {
     LQ_REQUIRE(fused, LQ_ERR_VALUE, "lstm_fused_layers: NULL pointer");
@@ -435,7 +474,7 @@ int lq_lstm_sequence_f32(const lq_lstm_args* a, lq_stream stream) {
     LQ_REQUIRE(a->directions == 1 || a->directions == 2, LQ_ERR_VALUE, "lstm_sequence: directions must be 1 or 2");
     LQ_REQUIRE(a->layers >= 1 && a->layers <= kParts && (a->layers == 1 || (a->directions == 1 && a->x)), LQ_ERR_VALUE,
                "lstm_sequence: %d layers, 1 or (one direction, input product taken here) at most %d", a->layers, kParts);
-    LQ_REQUIRE(a->hidden <= 1024, LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: hidden %d, at most 1024", a->hidden);
+    LQ_REQUIRE(a->hidden <= kMaxHidden, LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: hidden %d, at most %d", a->hidden, kMaxHidden);
     LQ_REQUIRE(!a->x || (a->inputs > 0 && a->inputs <= kMaxFused && a->hidden <= kMaxFused), LQ_ERR_NOT_IMPLEMENTED,
                "lstm_sequence: input product of %d columns for hidden %d, at most %d", a->inputs, a->hidden, kMaxFused);
     if (a->steps == 0 || a->batch == 0) return LQ_OK;

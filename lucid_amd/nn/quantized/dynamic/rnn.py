@@ -8,9 +8,9 @@ b_hh)``).
 On the device the recurrence of all steps and directions is one launch
 (``lq_lstm_sequence_f32``), which takes the input products and the layers stacked on top of the
 first as well where they fit; else the input product of a layer is taken over all time steps
-beforehand (float32 MFMA GEMM).  Packed sequences, projections, hidden sizes beyond 1024 and
-states of other types than ``from_float`` leaves take a recurrent GEMM and a gate kernel per step
-instead.
+beforehand (float32 MFMA GEMM).  Packed sequences, projections, hidden sizes beyond 1024, batches
+whose rows would go through that launch in too many turns and states of other types than
+``from_float`` leaves take a recurrent GEMM and a gate kernel per step instead.
 """
 
 from __future__ import annotations
@@ -66,6 +66,15 @@ class LSTM(Module):
             if b is None or b.shape != shape or b.dtype is not dt or b.device != "hip":
                 return False
         return True
+
+    def _sequence_pays(self, Bn: int) -> bool:
+        """Whether the one-launch recurrence takes the steps of ``Bn`` rows.  While a graph is recorded it takes any it
+        can: the steps one by one add the biases on the host."""
+        flag = C.c_int()
+        _C.call("lq_lstm_sequence_pays", Bn, self.hidden_size, 2 if self.bidirectional else 1, C.byref(flag))
+        if not flag.value:
+            _C.check(_C.load().lq_stream_is_capturing(C.byref(flag), _C.current_stream()))
+        return flag.value != 0
 
     def _weight(self, name: str) -> Tensor:
         codes, scale = getattr(self, name + "_int8"), getattr(self, name + "_scale")
@@ -126,7 +135,7 @@ class LSTM(Module):
         c_n = Tensor.empty((n_state, Bn, H), T.float32, "hip")
         # (the one-launch recurrence addresses a step's rows with 32-bit byte offsets)
         if (packed is None and P == 0 and H <= 1024 and Tn > 0 and Bn > 0 and Tn * Bn * dirs * H < 1 << 29
-                and all(self._kernel_takes(k) for k in range(self.num_layers))):
+                and all(self._kernel_takes(k) for k in range(self.num_layers)) and self._sequence_pays(Bn)):
             return self._forward_sequences(x, h0, c0, h_n, c_n, Tn, Bn), (h_n, c_n)
         ragged = any(bs != Bn for bs in batch_sizes)
         layer_in = x

@@ -326,6 +326,25 @@ def test_dynamic_lstm_input_of_two_gib():
     assert np.array_equal(y, np.broadcast_to(one.numpy(), y.shape))
 
 
+def test_dynamic_lstm_long_sequences_of_two_gib():
+    """The same with few rows of many steps, where the recurrence stays the faster one: it gets its input products from
+    a GEMM.  A zero input gives every row the values of a batch of one, which takes them itself."""
+    from lucid_amd import _C
+    I, H, Bn, Tn = 512, 16, 16, 1 << 16
+    assert _sequence_pays(Bn, H, 1) == 1
+    qm = Q.quantize_dynamic(nn.LSTM(I, H, batch_first=True))
+    x = L.Tensor.empty((Bn, Tn, I), L.float32, "hip")
+    _C.call("lq_fill_bytes", x.data_ptr, 0, x.nbytes, None)
+    y, _ = qm(x)
+    del x
+    one = L.Tensor.empty((1, Tn, I), L.float32, "hip")
+    _C.call("lq_fill_bytes", one.data_ptr, 0, one.nbytes, None)
+    want, _ = qm(one)
+    y = y.numpy()
+    assert np.array_equal(y, np.broadcast_to(y[:1], y.shape))
+    assert np.abs(y[0] - want.numpy()[0]).max() < 7 * H ** 0.5 * 2.0 ** -24 * 8
+
+
 @pytest.mark.parametrize("I,H,layers,Bn,Tn,bidir,batch_first",
                          [(3, 1, 2, 1, 3, False, False), (130, 17, 3, 5, 4, False, True), (500, 129, 5, 33, 2, False, False),
                           (100, 300, 2, 16, 5, False, True), (512, 512, 2, 17, 4, False, False), (257, 250, 2, 18, 3, True, True),
@@ -386,6 +405,75 @@ def test_dynamic_lstm_states_of_other_types_and_sizes():
     for other in wrong:
         with pytest.raises(_C.ShapeMismatch):
             loaded(**other)(x)
+
+
+def _sequence_pays(Bn, H, dirs):
+    import ctypes as C
+    from lucid_amd import _C
+    n = C.c_int(7)
+    _C.call("lq_lstm_sequence_pays", Bn, H, dirs, C.byref(n))
+    return n.value
+
+
+@pytest.mark.parametrize("I,H,Bn,layers,bidir", [(40, 1024, 300, 1, False), (72, 768, 401, 2, False), (24, 520, 1600, 1, True)])
+def test_dynamic_lstm_batches_beyond_the_recurrence(I, H, Bn, layers, bidir):
+    """Batches whose rows would go through the recurrence in too many turns take the steps one by one, and have the
+    values that their rows have in a batch that does not."""
+    Tn, dirs, rows = 3, 2 if bidir else 1, 16
+    assert _sequence_pays(Bn, H, dirs) == 0 and _sequence_pays(rows, H, dirs) == 1
+    rng = np.random.default_rng(H)
+    q = Q.quantize_dynamic(nn.LSTM(I, H, num_layers=layers, bidirectional=bidir))
+    x = rng.standard_normal((Tn, Bn, I)).astype(np.float32)
+    hx = [rng.standard_normal((layers * dirs, Bn, H)).astype(np.float32) for _ in range(2)]
+    y, (h, c) = q(hip(x), (hip(hx[0]), hip(hx[1])))
+    for at in (0, 112, Bn - rows):
+        few = [hip(np.ascontiguousarray(v[:, at:at + rows])) for v in (x, *hx)]
+        wy, (wh, wc) = q(few[0], (few[1], few[2]))
+        for want, got in ((wy, y), (wh, h), (wc, c)):
+            # the sums of the steps are in another order
+            assert np.abs(got.numpy()[:, at:at + rows] - want.numpy()).max() < 7 * (H + I) ** 0.5 * 2.0 ** -24 * 8
+
+
+def test_captured_dynamic_lstm_of_a_large_batch_is_the_recurrence():
+    """Recorded calls go through the recurrence in as many launches as it takes: the steps one by one would read the
+    biases back.  (One step of these sizes: the recurrence takes the input product as well, which needs no upload.)"""
+    I, H, Bn = 16, 256, 1300
+    assert _sequence_pays(Bn, H, 1) == 0
+    rng = np.random.default_rng(1)
+    q = Q.quantize_dynamic(nn.LSTM(I, H))
+    x = hip(rng.standard_normal((1, Bn, I)).astype(np.float32))
+    want, _ = q(x)
+    with L.graph.capture() as g:
+        y, _ = q(x)
+    for _ in range(3):
+        g.replay()
+        L.synchronize()
+        assert np.abs(y.numpy() - want.numpy()).max() < 7 * (H + I) ** 0.5 * 2.0 ** -24 * 8
+    g.destroy()
+
+
+def test_dynamic_lstm_where_streams_have_more_hardware_queues():
+    """The recurrence takes the share of the device that one of the process's hardware queues may have; a layer that
+    does not fit there goes through the steps one by one."""
+    import os, subprocess, sys, textwrap
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    script = textwrap.dedent("""
+        import sys
+        sys.path.insert(0, %r); sys.path.insert(0, %r)
+        import numpy as np
+        import lucid_amd as L, lucid_amd.nn as nn, lucid_amd.quantization as Q
+        from test_hip_breadth import _sequence_pays, _oracle_lstm_stack
+        L._C.init(0)
+        assert _sequence_pays(16, 1024, 1) == 0 and _sequence_pays(16, 64, 1) == 1
+        q = Q.quantize_dynamic(nn.LSTM(64, 1024))
+        x = np.random.default_rng(0).standard_normal((4, 5, 64)).astype(np.float32)
+        y, _ = q(L.tensor(x, device="hip"))
+        want = _oracle_lstm_stack(q, x, None, False)[0]
+        print("OK" if np.abs(y.numpy() - want).max() < 1e-5 else "BAD", flush=True)
+    """ % (root, os.path.join(root, "tests")))
+    r = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=110,
+                       env={**os.environ, "GPU_MAX_HW_QUEUES": "16"})
+    assert r.returncode == 0 and r.stdout.strip().endswith("OK"), r.stdout + r.stderr
 
 
 @pytest.mark.parametrize("layers,bidir,proj,sorted_input", [(1, False, 0, True), (2, True, 0, False), (1, False, 6, True),
