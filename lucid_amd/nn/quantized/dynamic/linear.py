@@ -93,7 +93,9 @@ def fused_pair(first, relu_between: bool, second, x):
     if taken1 is None or taken2 is None:
         return None
     (w1, scale1, bias1), (w2, scale2, bias2) = taken1, taken2
-    wsum1, wsum2 = first._weight_sums(), second._weight_sums()
+    wsum1, wsum2 = first._wsum, second._wsum
+    if wsum1 is None or wsum2 is None:
+        wsum1, wsum2 = first._weight_sums(), second._weight_sums()
     qd = first.act_qdtype
     y = Tensor.empty((*x.shape[:-1], N2), T.float32, "hip")
     _C.call("lq_dynamic_mlp2_small_f32", x.data_ptr, M, K1, w1.data_ptr, N1, scale1.data_ptr, wsum1.data_ptr,
@@ -154,15 +156,13 @@ class Linear(Module):
         return self._keep("_wsum", _ops.rowsum_i8(self._buffers["weight_int8"]))
 
     def _weight_rows(self) -> tuple[Tensor, int]:
-        """The weight codes in rows of a multiple of 16 bytes (``weight_int8`` itself where its rows are) and
-        that length; rows of a ragged layer are laid out once, with zeros behind them."""
-        N, K = self.out_features, self.in_features
-        ld = _code_row_bytes(K)
-        if ld == K:
-            return self._buffers["weight_int8"], K
+        """The weight codes of a ragged layer in rows of a multiple of 64 bytes, laid out once with zeros behind them,
+        and that length."""
         kept = self._wrows
         if kept is not None:
             return kept
+        N, K = self.out_features, self.in_features
+        ld = _code_row_bytes(K)
         rows = Tensor.empty((N, ld), T.int8, "hip")
         _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
         _C.call("lq_d2d_rows", rows.data_ptr, ld, self._buffers["weight_int8"].data_ptr, K, K, N, None)
@@ -191,7 +191,9 @@ class Linear(Module):
                 and (taken := _kernel_operands(self, N, K)) is not None):
             # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
             w, scale, bias = taken
-            wsum = self._weight_sums()
+            wsum = self._wsum
+            if wsum is None:
+                wsum = self._weight_sums()
             y = Tensor.empty((*x.shape[:-1], N), T.float32, "hip")
             grid = (0, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, off)
             b = None if bias is None else bias.data_ptr
@@ -199,7 +201,7 @@ class Linear(Module):
                 _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, w.data_ptr, N, scale.data_ptr,
                         wsum.data_ptr, b, *grid, y.data_ptr, None)
             else:
-                w, ldw = self._weight_rows()
+                w, ldw = self._weight_rows() if K % 16 else (w, K)
                 _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale.data_ptr,
                         wsum.data_ptr, b, *grid, y.data_ptr if M else None, None)
             return y
