@@ -378,7 +378,8 @@ def test_quantize_rows_dynamic_equals_the_three_calls_and_the_oracle(rows, cols,
     assert np.array_equal(q.numpy()[ok], oq[ok])
 
 
-@pytest.mark.parametrize("n", [0, 1, 3, 4, 1000, 64 * 784, 262144, 50177])
+@pytest.mark.parametrize("n", [0, 1, 3, 4, 1000, 64 * 784, 262144, 50177,
+                               122881, 131071, 131072, 131073])  # 16 blocks of 8192 in one launch, 17 in two
 @pytest.mark.parametrize("qd", ["quint8", "qint8"])
 def test_quantize_tensor_dynamic_equals_the_three_calls(n, qd):
     """Global min / max, qparams and codes of a small tensor in one launch: the bits of
