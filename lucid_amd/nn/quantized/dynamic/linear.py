@@ -69,6 +69,20 @@ def _kernel_operands(lin, N: int, K: int):
     return None
 
 
+def _keep(*derived) -> None:
+    """Keeps ``(layer, name, value)``, derived from the weights by work that this call has issued, for the calls to come:
+    once that work is done, since those may run on other streams.  (Waited for behind the call's own launches: before
+    them it made a first call 25 to 45 us longer.)  A capture only records the work: it is then part of every
+    replay, and nothing is kept."""
+    capturing = C.c_int()
+    _C.check(_C.load().lq_stream_is_capturing(C.byref(capturing), _C.current_stream()))
+    if capturing.value or _graph.is_capturing():
+        return
+    _C.call("lq_sync", None)
+    for lin, name, value in derived:
+        setattr(lin, name, value)
+
+
 def fused_pair(first, relu_between: bool, second, x):
     """``second(relu(first(x)))`` (or without the ReLU) for two dynamic ``Linear`` layers on a small
     activation as ONE launch (``lq_dynamic_mlp2_small_f32``: the last block of layer 1 to finish
@@ -94,7 +108,8 @@ def fused_pair(first, relu_between: bool, second, x):
         return None
     (w1, scale1, bias1), (w2, scale2, bias2) = taken1, taken2
     wsum1, wsum2 = first._wsum, second._wsum
-    if wsum1 is None or wsum2 is None:
+    fresh = wsum1 is None or wsum2 is None
+    if fresh:
         wsum1, wsum2 = first._weight_sums(), second._weight_sums()
     qd = first.act_qdtype
     y = Tensor.empty((*x.shape[:-1], N2), T.float32, "hip")
@@ -102,6 +117,8 @@ def fused_pair(first, relu_between: bool, second, x):
             None if bias1 is None else bias1.data_ptr, int(relu_between),
             w2.data_ptr, N2, scale2.data_ptr, wsum2.data_ptr, None if bias2 is None else bias2.data_ptr, 0, 0,
             qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, storage_offset(qd), y.data_ptr, None)
+    if fresh:
+        _keep((first, "_wsum", wsum1), (second, "_wsum", wsum2))
     return y
 
 
@@ -137,36 +154,18 @@ class Linear(Module):
         if name == "weight_zero_point":
             forget_weight_zero_points(self)
 
-    def _keep(self, name: str, made):
-        """``made``, derived from the weight by work just issued, for the calls to come: once that work is done, since
-        those may run on other streams.  A capture only records the work: it is then part of every replay, and
-        nothing is kept."""
-        capturing = C.c_int()
-        _C.check(_C.load().lq_stream_is_capturing(C.byref(capturing), _C.current_stream()))
-        if not capturing.value and not _graph.is_capturing():
-            _C.call("lq_sync", None)
-            setattr(self, name, made)
-        return made
-
     def _weight_sums(self) -> Tensor:
         """The sums of the weight's rows."""
-        kept = self._wsum
-        if kept is not None:
-            return kept
-        return self._keep("_wsum", _ops.rowsum_i8(self._buffers["weight_int8"]))
+        return _ops.rowsum_i8(self._buffers["weight_int8"])
 
     def _weight_rows(self) -> tuple[Tensor, int]:
-        """The weight codes of a ragged layer in rows of a multiple of 64 bytes, laid out once with zeros behind them,
-        and that length."""
-        kept = self._wrows
-        if kept is not None:
-            return kept
+        """The weight codes of a ragged layer in rows of a multiple of 64 bytes with zeros behind them, and that length."""
         N, K = self.out_features, self.in_features
         ld = _code_row_bytes(K)
         rows = Tensor.empty((N, ld), T.int8, "hip")
         _C.call("lq_fill_bytes", rows.data_ptr, 0, rows.nbytes, None)
         _C.call("lq_d2d_rows", rows.data_ptr, ld, self._buffers["weight_int8"].data_ptr, K, K, N, None)
-        return self._keep("_wrows", (rows, ld))
+        return rows, ld
 
     def forward(self, x: Tensor, residual: Tensor | None = None, activation: str | None = None,
                 track_range: bool = False) -> Tensor:
@@ -191,9 +190,10 @@ class Linear(Module):
                 and (taken := _kernel_operands(self, N, K)) is not None):
             # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
             w, scale, bias = taken
-            wsum = self._wsum
+            wsum, fresh = self._wsum, ()
             if wsum is None:
                 wsum = self._weight_sums()
+                fresh = ((self, "_wsum", wsum),)
             y = Tensor.empty((*x.shape[:-1], N), T.float32, "hip")
             grid = (0, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, off)
             b = None if bias is None else bias.data_ptr
@@ -201,9 +201,17 @@ class Linear(Module):
                 _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, w.data_ptr, N, scale.data_ptr,
                         wsum.data_ptr, b, *grid, y.data_ptr, None)
             else:
-                w, ldw = self._weight_rows() if K % 16 else (w, K)
+                ldw = K
+                if K % 16:
+                    rows = self._wrows
+                    if rows is None:
+                        rows = self._weight_rows()
+                        fresh += ((self, "_wrows", rows),)
+                    w, ldw = rows
                 _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale.data_ptr,
                         wsum.data_ptr, b, *grid, y.data_ptr if M else None, None)
+            if fresh:
+                _keep(*fresh)
             return y
         xq = Tensor.empty((M, K), T.int8, "hip")
         small = x._range is None and x.numel <= (1 << 18)
@@ -236,7 +244,8 @@ class Linear(Module):
         (``functional.layer_norm_dynamic_quantize``)."""
         N = self.out_features
         off = storage_offset(self.act_qdtype)
-        wsum = self._weight_sums()
+        kept = self._wsum
+        wsum = self._weight_sums() if kept is None else kept
         rng = None
         w_zp = weight_zero_points(self)
         if track_range and w_zp is not None:
@@ -251,6 +260,8 @@ class Linear(Module):
                             range_buf=rng, w_zp=w_zp)
         y = y.reshape(*lead_shape, N)
         y._range = rng
+        if kept is None:
+            _keep((self, "_wsum", wsum))
         return y
 
     @classmethod
