@@ -1402,7 +1402,7 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
             // not in a graph: slots first cleared there would be unset until its replay, and replays on
             // another stream would share them with this one
             hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-            LQ_HIP(hipStreamIsCapturing(st, &capturing));
+            if (st) LQ_HIP(hipStreamIsCapturing(st, &capturing));  // (see lq_stream_is_capturing)
             exchange = capturing == hipStreamCaptureStatusNone;
         }
         const int rc = exchange ? stream_buffer(7, sizeof(DynScratch), 0, st, &tmp, &fresh)

@@ -389,7 +389,8 @@ extern "C" int lq_graph_end(lq_stream stream, int graph_id) {
 extern "C" int lq_stream_is_capturing(int* capturing, lq_stream stream) {
     LQ_REQUIRE(capturing, LQ_ERR_VALUE, "stream_is_capturing: NULL pointer");
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    LQ_HIP(hipStreamIsCapturing(as_stream(stream), &status));
+    // (the default stream is never recorded, and asking about it is an error while a stream is that synchronises with it)
+    if (stream) LQ_HIP(hipStreamIsCapturing(as_stream(stream), &status));
     *capturing = status != hipStreamCaptureStatusNone;
     return LQ_OK;
 }

@@ -319,3 +319,20 @@ def test_captured_dynamic_linears_have_codes_of_their_own(M, K, N):
             _C.call("lq_graph_destroy", g)
         for s in streams:
             _C.call("lq_stream_destroy", s)
+
+
+def test_the_default_stream_is_not_recorded_while_another_is():
+    """What a thread on the default stream is told, whoever records a graph on a stream of their own."""
+    _C.init()
+    lib, stream, gid, flag = _C.load(), C.c_void_p(), C.c_int(), C.c_int(7)
+    _C.call("lq_stream_create", C.byref(stream))
+    _C.call("lq_graph_begin", stream, C.byref(gid))
+    try:
+        _C.check(lib.lq_stream_is_capturing(C.byref(flag), None))
+        assert flag.value == 0
+        _C.check(lib.lq_stream_is_capturing(C.byref(flag), stream))
+        assert flag.value == 1
+    finally:
+        _C.call("lq_graph_end", stream, gid)
+        _C.call("lq_graph_destroy", gid)
+        _C.call("lq_stream_destroy", stream)
