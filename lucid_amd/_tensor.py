@@ -35,6 +35,13 @@ class dtype:
     def __repr__(self) -> str:
         return f"lucid.{self.name}"
 
+    # (one object per type: what tells types apart by identity does so in a copied module too)
+    def __copy__(self) -> "dtype":
+        return self
+
+    def __deepcopy__(self, memo) -> "dtype":
+        return self
+
 
 bool_ = dtype("bool", _C.BOOL, 1, np.bool_)
 int8 = dtype("int8", _C.I8, 1, np.int8)

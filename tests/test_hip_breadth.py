@@ -407,6 +407,22 @@ def test_dynamic_lstm_states_of_other_types_and_sizes():
             loaded(**other)(x)
 
 
+def test_copied_dynamic_lstm_is_the_recurrence_too():
+    """A deep copy (what prepare and convert make of a model) takes the one launch, and has the original's bits."""
+    import copy
+    from lucid_amd import _C
+    q = Q.quantize_dynamic(nn.LSTM(24, 40, num_layers=2))
+    x = hip(np.random.default_rng(0).standard_normal((4, 3, 24)).astype(np.float32))
+    twin, names, call = copy.deepcopy(q), [], _C.call
+    _C.call = lambda name, *args: (names.append(name), call(name, *args))[1]
+    try:
+        y, _ = twin(x)
+    finally:
+        _C.call = call
+    assert "lq_lstm_sequence_f32" in names and "lq_lstm_cell_f32" not in names
+    assert np.array_equal(y.numpy(), q(x)[0].numpy())
+
+
 def _sequence_pays(Bn, H, dirs):
     import ctypes as C
     from lucid_amd import _C

@@ -48,6 +48,13 @@ def test_one_call_is_for_codes_that_fit_its_rows_and_scratch(M, K, takes):
         assert ld % 16 == 0 and K <= ld <= 131071 and (M * ld + 8191) // 8192 * 8192 < 1 << 32
 
 
+def test_a_copied_type_is_the_type():
+    import copy
+    from lucid_amd import _tensor as T
+    for dt in T._ALL:
+        assert copy.deepcopy([dt])[0] is dt and copy.copy(dt) is dt
+
+
 def test_another_weight_forgets_what_was_derived_from_the_last():
     """Assigned, registered or loaded: the row sums and padded rows are those of the weight that is there."""
     lin = _layer(8, 30)
