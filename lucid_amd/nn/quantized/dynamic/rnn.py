@@ -37,7 +37,8 @@ class LSTM(Module):
         self.proj_size = proj_size
         self._weight_names: list[str] = []
         self._bias_names: list[str] = []
-        # per layer, what lq_lstm_sequence_f32 reads: name, shape and type of each buffer
+        # per layer, what lq_lstm_sequence_f32 reads: name, shape and type of each buffer (per direction w_ih, w_hh, each
+        # codes and scales, then b_ih, b_hh)
         self._kernel_buffers: list[list[tuple]] = [[] for _ in range(num_layers)]
         dirs = 2 if bidirectional else 1
         rec = proj_size if proj_size > 0 else hidden_size  # width of the state that re-enters the recurrence
@@ -58,14 +59,20 @@ class LSTM(Module):
                         self.register_buffer(name, T.tensor(np.zeros(4 * hidden_size, np.float32), device="hip"))
                         self._kernel_buffers[k].append((name, (4 * hidden_size,), T.float32))
 
-    def _kernel_takes(self, k: int) -> bool:
-        """Whether layer ``k`` holds what the one-launch recurrence reads.  A loaded state may hold other types
-        (int16 codes, float16 biases) or sizes: the steps one by one convert those, or refuse them."""
-        for name, shape, dt in self._kernel_buffers[k]:
-            b = self._buffers[name]
-            if b is None or b.shape != shape or b.dtype is not dt or b.device != "hip":
-                return False
-        return True
+    def _kernel_operands(self) -> list[list[Tensor]] | None:
+        """Per layer, what the one-launch recurrence reads (``_kernel_buffers``), or ``None`` if the layers hold something
+        else.  A loaded state may have other types (int16 codes, float16 biases) or sizes: the steps one by one convert
+        those, or refuse them.  (Looked up once per call: short sequences are bound by what they cost the host.)"""
+        bufs, taken = self._buffers, []
+        for layer in self._kernel_buffers:
+            held = []
+            for name, shape, dt in layer:
+                b = bufs[name]
+                if b is None or b.dtype is not dt or b.shape != shape or b.device != "hip":
+                    return None
+                held.append(b)
+            taken.append(held)
+        return taken
 
     def _sequence_pays(self, Bn: int) -> bool:
         """Whether the one-launch recurrence takes the steps of ``Bn`` rows.  While a graph is recorded it takes any it
@@ -135,8 +142,8 @@ class LSTM(Module):
         c_n = Tensor.empty((n_state, Bn, H), T.float32, "hip")
         # (the one-launch recurrence addresses a step's rows with 32-bit byte offsets)
         if (packed is None and P == 0 and H <= 1024 and Tn > 0 and Bn > 0 and Tn * Bn * dirs * H < 1 << 29
-                and all(self._kernel_takes(k) for k in range(self.num_layers)) and self._sequence_pays(Bn)):
-            return self._forward_sequences(x, h0, c0, h_n, c_n, Tn, Bn), (h_n, c_n)
+                and (operands := self._kernel_operands()) is not None and self._sequence_pays(Bn)):
+            return self._forward_sequences(x, h0, c0, h_n, c_n, Tn, Bn, operands), (h_n, c_n)
         ragged = any(bs != Bn for bs in batch_sizes)
         layer_in = x
         for k in range(self.num_layers):
@@ -209,11 +216,11 @@ class LSTM(Module):
                 h_n, c_n = restore(h_n, R), restore(c_n, H)
         return PackedSequence(out, packed.batch_sizes, packed.sorted_indices, packed.unsorted_indices), (h_n, c_n)
 
-    def _forward_sequences(self, x, h0, c0, h_n, c_n, Tn, Bn):
+    def _forward_sequences(self, x, h0, c0, h_n, c_n, Tn, Bn, operands):
         """Whole sequences, one launch for the recurrence of a layer or of several stacked ones; fills
-        ``h_n`` / ``c_n``."""
+        ``h_n`` / ``c_n``.  ``operands``: of ``_kernel_operands``."""
         H, dirs = self.hidden_size, 2 if self.bidirectional else 1
-        bufs, state = self._buffers, Bn * H * 4
+        state, per = Bn * H * 4, 6 if self.bias else 4
         shape = (Bn, Tn, dirs * H) if self.batch_first else (Tn, Bn, dirs * H)
         fused, k = C.c_int(), 0
         while k < self.num_layers:
@@ -227,15 +234,16 @@ class LSTM(Module):
             ys = [Tensor.empty(shape, T.float32, "hip") for _ in range(layers)]
             gates = []
             for z in range(layers * dirs):  # one of the two is 1
-                name = f"l{k + z}" if dirs == 1 else f"l{k}" + ("", "_reverse")[z]
+                w_ih, s_ih, w_hh, s_hh, *biases = operands[k + z] if dirs == 1 else operands[k][z * per:(z + 1) * per]
                 if fused.value:
-                    a.w_ih[z], a.w_ih_scale[z] = (bufs[f"weight_ih_{name}_{v}"].data_ptr for v in ("int8", "scale"))
+                    a.w_ih[z], a.w_ih_scale[z] = w_ih.data_ptr, s_ih.data_ptr
                 else:
-                    gates.append(linear_f32(x, self._weight("weight_ih_" + name)))
+                    gates.append(linear_f32(x, self._weight(f"weight_ih_l{k + z}" if dirs == 1 else
+                                                            f"weight_ih_l{k}" + ("", "_reverse")[z])))
                     a.gates_x[z] = gates[-1].data_ptr
-                a.w_hh[z], a.w_hh_scale[z] = (bufs[f"weight_hh_{name}_{v}"].data_ptr for v in ("int8", "scale"))
-                if self.bias:
-                    a.bias_ih[z], a.bias_hh[z] = bufs["bias_ih_" + name].data_ptr, bufs["bias_hh_" + name].data_ptr
+                a.w_hh[z], a.w_hh_scale[z] = w_hh.data_ptr, s_hh.data_ptr
+                if biases:
+                    a.bias_ih[z], a.bias_hh[z] = biases[0].data_ptr, biases[1].data_ptr
             for z, y in enumerate(ys):
                 a.y[z] = y.data_ptr
             at = k * dirs * state
