@@ -11,32 +11,39 @@
 // and h is split into three bfloat16 parts (exact: 8 + 8 + 8 significant bits), so every product is
 // exact and accumulates in float32; the row's scale is applied to the sum.  The wavefronts of a
 // block divide the hidden axis between them: each loads its own columns of h[t-1] straight into
-// operand layout (16 batch rows x 32 columns per instruction), multiplies them with all four gate
-// tiles, and the partial sums meet in LDS; wavefront w of the first four then finishes batch rows
-// 4 j + w of the 16 units, with c in registers.  ceil(hidden / 16) blocks serve 16 batch rows of one
+// operand layout (16 batch rows x 16 columns per load), multiplies them with all four gate
+// tiles, and the partial sums meet in LDS; wavefront w of the first four then finishes units 4 w .. 4 w + 3
+// of the 16 rows, with c in registers.  ceil(hidden / 16) blocks serve 16 batch rows of one
 // direction; other rows and the other direction are independent groups in the same grid.
 //
-// Input.  Up to 512 columns a block also keeps the input weights of its units and takes the input product
-// of the next step while its h travels to the other blocks, where it costs nothing.  Stacked layers then
+// Input.  Up to 512 columns a block also keeps the input weights of its units, in wavefronts of their own: they
+// take the input product of the next step while h travels to the other blocks.  Stacked layers then
 // share the launch: layer k reads h[t] of layer k - 1 from that one's output as it appears, so L layers
-// take steps + L - 1 step times in place of L * steps.  The registers of the second weight halve the blocks
+// take little more than the steps of one.  The second weight halves the blocks
 // per CU; where that would mean more launches than it saves (lq_lstm_fused_layers), or beyond 512 columns,
 // the input products of all steps are taken beforehand (`gx`) and a layer is a launch of its own.
 //
-// Exchange.  h[t] is the layer's output, so the blocks of a group hand it to each other through y
-// itself: y is filled with a bit pattern no h can have (all ones, a NaN) before the launch, h is
-// written through to device scope, and a wavefront re-reads its columns of h[t-1] until every word is
-// there - no flags, no barrier, one memory trip each way per step.
+// Exchange.  The blocks of a group hand h[t] to each other through a ring of four steps in device memory, laid out as
+// the loads read it: a block writes eight whole 128-byte lines, a load is 1 KiB in a row.  Empty words hold a bit pattern no h
+// can have (all ones, a NaN); h is written through to device scope, and a wavefront re-reads what is missing of h[t-1]
+// until every word is there - no flags, no barrier, one memory trip each way per step.  A block empties its slot again two
+// steps before it is written.  Layers above read their input from the output y of the layer below, emptied before the launch.
+//
+// Order of the loads.  A CU returns loads in the order they were issued, so an input load that misses the L2 ahead of the
+// loads of h holds those up: input loads are issued when h has arrived (a barrier tells), for the step after
+// the next one.
 //
 // Progress.  A block waits only for blocks of its own launch, so all of them have to be resident: the
 // launcher bounds the grid by what the device holds of this kernel over the number of hardware queues
 // that streams share (four unless GPU_MAX_HW_QUEUES says more; a queue starts a launch only after the one
 // before it is fully placed), and larger batches run as several launches.  A wait is bounded besides:
-// after kSpinLimit reads the block stops waiting for the rest of the sequence and the output keeps its NaNs.
+// after kSpinLimit reads the block stops waiting for the rest of the sequence and what it computes is NaN.
 //
-// hidden 512, 16 rows: 3.4 us per step with gx, 3.8 with the input product; two such layers of 64 steps
-// 272 us per call, against 580 us as two launches with a GEMM (43 us with the decoding of its weight) each
-// and 4.67 ms with a float32 GEMM, a gate kernel and the host's share of their launches per step.
+// hidden 512, 16 rows, a step of 2.2 us (5100 cycles, timestamps): 450 before the first read, 1850 for the 32 KiB of h a
+// CU reads past its L2 (1000 at hidden 128), 1390 splits and products, 70 barrier, 1000 sums and gates.  Two such layers of
+// 64 steps take 168 us; 272 when h was read from y's rows (every line twice), the input loads stood between h and its
+// products, and one set of wavefronts took both products.  Placing a group's blocks on one XCD and exchanging through its L2 instead
+// measured 150 against 153 us for one layer: not worth the placement.
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -56,6 +63,10 @@ constexpr int kUnits = 16, kRows = 16;     // hidden units of a block, batch row
 constexpr unsigned kEmpty = 0xffffffffu;   // a word of y that has not been written
 constexpr int kSpinLimit = 1 << 20;        // about a second of waiting for one step
 constexpr int kScopeDevice = 16;           // "sc1" cache-policy bit of buffer accesses
+constexpr int kSlots = 4;                  // steps of h that a ring holds
+constexpr int kSlotWords = kUnits * kRows; // of one block's h of one step
+// partial sums of a gate tile in LDS: four rows of 64 lanes, the rows 4 banks apart (read four units x 16 rows at a time)
+constexpr int kGateRow = 68, kGateFloats = 4 * kGateRow;
 
 constexpr int kParts = LQ_LSTM_PARTS;      // grid z: the directions of one layer, or stacked layers
 
@@ -75,6 +86,8 @@ struct LstmArgs {
     float* y[kParts];  // element (t, b, col + j) at t * y_step + b * y_row + col + j; col = d * H in direction d
     long y_step, y_row, gx_step, gx_row, x_step, x_row;
     long y_elems, x_elems;
+    unsigned* rings;             // [part][group][slot][block of units][kSlotWords]
+    long ring_words;             // of all of them
     int T, B, H, I, row0, dir0, stacked;
 };
 
@@ -93,22 +106,87 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
 __device__ __forceinline__ uint32_t codes_bf16(int c0, int c1) {
     return __builtin_amdgcn_perm(__float_as_uint(float(c1)), __float_as_uint(float(c0)), 0x07060302u);
 }
-__device__ __forceinline__ float sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
+// The gates are on the chain of a step, so both functions are straight-line code, within 2 units in the last place of
+// the exact values (the library's expf and tanhf branch, and both sides run in a wavefront).
+// exp(x) for x <= 60: 2^(x log2 e) with the rounding error of the product put back
+__device__ __forceinline__ float exp_gate(float x) {
+    constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596299e-8f, kLn2 = 0.693147182f;
+    const float t = x * kLog2e;
+    const float low = __builtin_fmaf(x, kLog2eLow, __builtin_fmaf(x, kLog2e, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    return __builtin_fmaf(e, low * kLn2, e);
+}
+// 1 / x for 1 <= x < 2^100
+__device__ __forceinline__ float reciprocal(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float sigmoid(float x) {  // (a NaN fails the comparison and stays one)
+    return reciprocal(1.0f + exp_gate(x < -60.0f ? 60.0f : x > 60.0f ? -60.0f : -x));
+}
+__device__ __forceinline__ float tanh_gate(float x) {
+    const float a = __builtin_fabsf(x), u = x * x;
+    // below 0.6 x + x^3 P(x^2): P fitted for the least relative error, 2.8e-9
+    float q = __builtin_fmaf(u, -0x1.8257d2p-8f, 0x1.54b882p-6f);
+    q = __builtin_fmaf(q, u, -0x1.b898dap-5f);
+    q = __builtin_fmaf(q, u, 0x1.1109aep-3f);
+    q = __builtin_fmaf(q, u, -0x1.55553ep-2f);
+    const float small = __builtin_fmaf(x * u, q, x);
+    const float large = __builtin_fmaf(-2.0f, reciprocal(1.0f + exp_gate(a > 20.0f ? 40.0f : 2.0f * a)), 1.0f);
+    return a < 0.6f ? small : __builtin_copysignf(large, x);
+}
 
-// the codes of one row of a weight at this lane's eight columns of an instruction, as bfloat16
-__device__ __forceinline__ v8bf load_codes(const int8_t* row, int k, int K) {
-    int c[8];
-    if (k + 8 <= K) {
-        uint64_t raw;
-        __builtin_memcpy(&raw, row + k, 8);
+// Columns of a wavefront.  An instruction's 32 columns are two runs of 16, of which the lane's quarter has four each
+// (`kRun` apart): a lane's 16-byte loads then lie beside those of the other quarters, 64 bytes of a row per load.  Which
+// column is which k of the instruction does not matter as long as the weight is held in the same order.
+constexpr int kRun = 16;
+
+// Gate tiles of a weight [4 H][K] as bfloat16 operands: rows `unit` + g H, this lane's eight columns per instruction, all
+// of them requested before the first is used (columns past K are zero: four codes that end with the row are shifted).
+template <int KP>
+__device__ __forceinline__ void load_weights(v8bf (&wf)[4][KP], const int8_t* w, int H, int unit, int k_lane, int K) {
+    uint32_t raw[4][KP][2];
+    if (K >= 4) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) c[e] = int(int8_t(raw >> (8 * e)));
+        for (int g = 0; g < 4; ++g) {
+            const int8_t* const row = w + (size_t(g) * H + unit) * K;
+#pragma unroll
+            for (int i = 0; i < 2 * KP; ++i) {
+                const int k = k_lane + i * kRun;
+                __builtin_memcpy(&raw[g][i >> 1][i & 1], row + (k < K - 4 ? k : K - 4), 4);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * KP; ++i) {
+            const int past = k_lane + i * kRun - (K - 4);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const uint32_t four = raw[g][i >> 1][i & 1];
+                raw[g][i >> 1][i & 1] = past <= 0 ? four : past < 4 ? four >> (8 * past) : 0u;
+            }
+        }
     } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) c[e] = k + e < K ? int(row[k + e]) : 0;
+        for (int g = 0; g < 4; ++g)
+            for (int i = 0; i < 2 * KP; ++i) {
+                uint32_t four = 0;
+                for (int e = 0; e < 4; ++e)
+                    if (k_lane + i * kRun + e < K)
+                        four |= uint32_t(uint8_t(w[(size_t(g) * H + unit) * K + k_lane + i * kRun + e])) << (8 * e);
+                raw[g][i >> 1][i & 1] = four;
+            }
     }
-    return __builtin_bit_cast(v8bf, v4u{codes_bf16(c[0], c[1]), codes_bf16(c[2], c[3]), codes_bf16(c[4], c[5]),
-                                        codes_bf16(c[6], c[7])});
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int i = 0; i < KP; ++i) {
+            v4u pairs;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t two = raw[g][i][e >> 1] >> (16 * (e & 1));
+                pairs[e] = codes_bf16(int(int8_t(two)), int(int8_t(two >> 8)));
+            }
+            wf[g][i] = __builtin_bit_cast(v8bf, pairs);
+        }
 }
 // device-scope access to what follows element `at` of an array of `elems` floats
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t words_from(const float* base, long at, long elems) {
@@ -116,201 +194,287 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t words_from(const float* base, 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + at, 0,
                                              bytes < 0x7fffffffl ? int(bytes) : 0x7fffffff, 0x00020000);
 }
-template <int KP>
-__device__ __forceinline__ void load_columns(v4u (&raw)[KP][2], __amdgpu_buffer_rsrc_t src, unsigned off) {
+template <int KP, int SCOPE>
+__device__ __forceinline__ void load_columns(v4u (&raw)[KP][2], __amdgpu_buffer_rsrc_t src, unsigned off, unsigned missing = ~0u) {
 #pragma unroll
-    for (int i = 0; i < KP; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            raw[i][j] = __builtin_amdgcn_raw_buffer_load_b128(src, off + unsigned(i * 32 + j * 4) * 4, 0, kScopeDevice);
+    for (int i = 0; i < 2 * KP; ++i)
+        if (missing >> i & 1)
+            raw[i >> 1][i & 1] = __builtin_amdgcn_raw_buffer_load_b128(src, off + unsigned(i * kRun) * 4, 0, SCOPE);
 }
-// columns from `left` on (of another direction, row or step) become zero; the largest word left
+// columns from `left` on (of another direction, row or step) become zero
 template <int KP>
-__device__ __forceinline__ unsigned mask_columns(v4u (&raw)[KP][2], int left) {
-    unsigned worst = 0;
+__device__ __forceinline__ void mask_columns(v4u (&raw)[KP][2], int left) {
 #pragma unroll
-    for (int i = 0; i < KP; ++i)
+    for (int i = 0; i < 2 * KP; ++i)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            if (i * 32 + e >= left) raw[i][e >> 2][e & 3] = 0u;
-            worst = worst > raw[i][e >> 2][e & 3] ? worst : raw[i][e >> 2][e & 3];
-        }
-    return worst;
+        for (int e = 0; e < 4; ++e)
+            if (i * kRun + e >= left) raw[i >> 1][i & 1][e] = 0u;
 }
-// acc[g] += columns . codes of gate g: three exact part products each
+// the loads of which some lane has words that have not been written
+template <int KP>
+__device__ __forceinline__ unsigned missing_words(const v4u (&raw)[KP][2]) {
+    unsigned missing = 0;
+#pragma unroll
+    for (int i = 0; i < 2 * KP; ++i) {
+        const v4u r = raw[i >> 1][i & 1];
+        const unsigned a = r[0] > r[1] ? r[0] : r[1], b = r[2] > r[3] ? r[2] : r[3];
+        if (__builtin_amdgcn_ballot_w64((a > b ? a : b) == kEmpty)) missing |= 1u << i;
+    }
+    return missing;
+}
+// the barrier of the block for what is in LDS: loads and stores of memory stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+// eight columns as three operands, whose sum they are
+__device__ __forceinline__ void split_columns(v4u (&parts)[3], const v4u (&raw)[2]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const v4u r = raw[e >> 1];
+        uint32_t hh, mm, ll;
+        split3(__uint_as_float(r[(2 * e) & 3]), __uint_as_float(r[(2 * e + 1) & 3]), hh, mm, ll);
+        parts[0][e] = hh, parts[1][e] = mm, parts[2][e] = ll;
+    }
+}
+// acc[g] += columns . codes of gate g: three exact part products each.  The splits of an instruction's columns come
+// before the products of the one before, which they do not wait for.
 template <int KP>
 __device__ __forceinline__ void multiply(v4f (&acc)[4], const v4u (&raw)[KP][2], const v8bf (&wf)[4][KP]) {
+    v4u parts[2][3];
+    split_columns(parts[0], raw[0]);
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
-        v4u part3[3];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const v4u r = raw[i][e >> 1];
-            uint32_t hh, mm, ll;
-            split3(__uint_as_float(r[(2 * e) & 3]), __uint_as_float(r[(2 * e + 1) & 3]), hh, mm, ll);
-            part3[0][e] = hh, part3[1][e] = mm, part3[2][e] = ll;
-        }
+        if (i + 1 < KP) split_columns(parts[(i + 1) & 1], raw[i + 1]);
 #pragma unroll
         for (int q = 0; q < 3; ++q)
 #pragma unroll
             for (int g = 0; g < 4; ++g)
-                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, part3[q]), wf[g][i], acc[g], 0, 0, 0);
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, parts[i & 1][q]), wf[g][i], acc[g], 0, 0, 0);
     }
 }
 
-// W wavefronts, each with KPW instructions of 32 hidden columns (hidden <= 32 W KPW) and KX of 32 input
-// columns; KX = 0 reads the input products from gx.  The weights take 16 (KPW + KX) registers, which
-// decides how many wavefronts a SIMD holds.
-template <int W, int KPW, int KX>
-__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(KX == 0 && KPW <= 2 ? 4 : 2, KX == 0 && KPW <= 2 ? 4 : 2)))
+// W wavefronts for h, each with KPW instructions of 32 hidden columns (hidden <= 32 W KPW), and XW for the
+// input, each with KX of 32 input columns; XW = 0 reads the input products from gx.
+//
+// The two roles meet at one barrier a step.  An h wavefront waits for its columns of h[t-1], multiplies them, adds the
+// input product its partner left in LDS and puts its partial sums there; behind the barrier the first four finish the
+// gates.  An input wavefront is a step ahead and off the chain: x[t+1] arrives while it multiplies x[t].
+template <int W, int KPW, int XW, int KX>
+struct LstmForm {
+    static constexpr int kThreads = (W + XW) * 64;
+    static constexpr int kPartFloats = W * 4 * kGateFloats, kInputFloats = XW * 4 * 4 * 64;
+    static constexpr int kLdsBytes = 2 * (kPartFloats + kInputFloats) * 4;
+    // wavefronts of a SIMD: the weights take 16 registers per instruction, the rest about 100
+    static constexpr int kPerSimd = XW == 0 && KPW <= 2 ? 4 : 2;
+};
+
+template <int W, int KPW, int XW, int KX>
+__global__ __launch_bounds__((W + XW) * 64)
+    __attribute__((amdgpu_waves_per_eu(LstmForm<W, KPW, XW, KX>::kPerSimd, LstmForm<W, KPW, XW, KX>::kPerSimd)))
 void lstm_sequence_kernel(LstmArgs p) {
-    __shared__ float part[2][W][4][4][64];  // [step parity][wavefront][gate][row of the quad][lane]
+    using Form = LstmForm<W, KPW, XW, KX>;
+    extern __shared__ __align__(16) float lds[];
+    // partial sums [step parity][wavefront][gate][kGateFloats]; scaled input products [parity][wavefront][gate][lane][row]
+    float* const part = lds;
+    float* const inputs = lds + 2 * Form::kPartFloats;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ln = lane & 15, lq4 = lane >> 4;
     const int z = p.dir0 + blockIdx.z, d = p.stacked ? 0 : z, H = p.H;
     const int u0 = blockIdx.x * kUnits, m0 = p.row0 + blockIdx.y * kRows;
     float* const y = p.y[z];
+    // the row whose h and x this lane reads; rows past the batch repeat the last one
+    const int in_batch = m0 + ln < p.B ? m0 + ln : p.B - 1;
+    const int tile_unit = u0 + ln < H ? u0 + ln : H - 1;  // units past H are computed and never stored
+
+    if constexpr (XW > 0) {
+        if (wave >= W) {
+            // ---- the input of this part: x, or the output of the layer below
+            const int w = wave - W;
+            const bool above = p.stacked && z > 0;
+            const float* const in = above ? p.y[above ? z - 1 : 0] : p.x;
+            const int I = above ? H : p.I;
+            const long in_step = above ? p.y_step : p.x_step, in_row = above ? p.y_row : p.x_row;
+            const long in_elems = above ? p.y_elems : p.x_elems;
+            const int k_lane = w * KX * 32 + lq4 * 4;
+            const bool whole = (w + 1) * KX * 32 <= I;
+            v8bf wf[4][KX];
+            float scale[4];
+            load_weights<KX>(wf, p.wx[z], H, tile_unit, k_lane, I);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) scale[g] = p.wx_scale[z][g * H + tile_unit];
+            const unsigned off = unsigned(in_batch * in_row + k_lane) * 4;
+            bool waiting = above;
+            v4u raw[KX][2], next[KX][2];  // of the step to multiply and of the one after
+            auto request = [&](v4u (&raw)[KX][2], int s, unsigned missing) {
+                const __amdgpu_buffer_rsrc_t src = words_from(in, long(d ? p.T - 1 - s : s) * in_step, in_elems);
+                if (above) load_columns<KX, kScopeDevice>(raw, src, off, missing);
+                else load_columns<KX, 0>(raw, src, off);
+            };
+            auto product = [&](v4u (&raw)[KX][2], int s) {
+                for (int spin = 0;; ++spin) {
+                    if (!whole) mask_columns<KX>(raw, I - k_lane);
+                    const unsigned missing = waiting ? missing_words<KX>(raw) : 0;
+                    if (!missing) break;
+                    if (spin >= kSpinLimit) waiting = false;
+                    asm volatile("" ::: "memory");  // read again: the words change under the loop
+                    request(raw, s, missing);
+                }
+                v4f acc[4];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) acc[g] = v4f{0.f, 0.f, 0.f, 0.f};
+                multiply<KX>(acc, raw, wf);
+                v4f* const out = reinterpret_cast<v4f*>(inputs + (s & 1) * Form::kInputFloats) + w * 4 * 64 + lane;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) out[g * 64] = acc[g] * scale[g];
+            };
+            auto step = [&](v4u (&raw)[KX][2], v4u (&next)[KX][2], int s) {
+                lds_barrier();  // h[s - 1] is there: until the next wait for h the loads are the input's
+                request(next, s + 2 < p.T ? s + 2 : p.T - 1, ~0u);
+                lds_barrier();  // the products of step s are done: the matrix unit is the input's
+                if (s + 1 < p.T) product(raw, s + 1);  // (this half of `inputs` was read at step s - 1)
+            };
+            request(raw, 0, ~0u);
+            product(raw, 0);
+            request(raw, 1 < p.T ? 1 : 0, ~0u);
+            for (int s = 0; s < p.T; s += 2) {
+                step(raw, next, s);
+                if (s + 1 < p.T) step(next, raw, s + 1);
+            }
+            return;
+        }
+    }
 
     // ---- the block's weights: tile g = gate g of units u0 .. u0+15, this wavefront's columns
-    v8bf wf[4][KPW], wxf[4][KX > 0 ? KX : 1];
-    float scale_h[4], scale_x[4];  // of the unit whose products this lane accumulates
-    // ---- the input of this part: x, or the output of the layer below
-    const bool above = p.stacked && z > 0;
-    const float* const in = above ? p.y[above ? z - 1 : 0] : p.x;
-    const int I = above ? H : p.I;
-    const long in_step = above ? p.y_step : p.x_step, in_row = above ? p.y_row : p.x_row;
-    const long in_elems = above ? p.y_elems : p.x_elems;
-    const int kx_lane = wave * KX * 32 + lq4 * 8;
-    {
-        const int unit = u0 + ln < H ? u0 + ln : H - 1;  // units past H are computed and never stored
+    const int k_lane = wave * KPW * 32 + lq4 * 4;
+    v8bf wf[4][KPW];
+    float scale_h[4];  // of the unit whose products this lane accumulates
+    load_weights<KPW>(wf, p.w[z], H, tile_unit, k_lane, H);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-#pragma unroll
-            for (int i = 0; i < KPW; ++i)
-                wf[g][i] = load_codes(p.w[z] + (size_t(g) * H + unit) * H, (wave * KPW + i) * 32 + lq4 * 8, H);
-            if constexpr (KX > 0) {
-#pragma unroll
-                for (int i = 0; i < KX; ++i)
-                    wxf[g][i] = load_codes(p.wx[z] + (size_t(g) * H + unit) * I, kx_lane + i * 32, I);
-                scale_h[g] = p.w_scale[z][g * H + unit], scale_x[g] = p.wx_scale[z][g * H + unit];
-            }
-        }
-    }
+    for (int g = 0; g < 4; ++g) scale_h[g] = p.w_scale[z][g * H + tile_unit];
     // ---- the element this lane finishes (wavefronts 0..3)
-    const int unit = u0 + ln, row = m0 + 4 * lq4 + wave;
+    const int tile_row = lane >> 2, unit = u0 + 4 * wave + (lane & 3), row = m0 + tile_row;
     const bool mine = wave < 4 && unit < H && row < p.B;
-    float ws[4], bias[4], c = 0.0f;
+    float bias[4], c = 0.0f, hv = 0.0f;
     const size_t state = (size_t(z) * p.B + (row < p.B ? row : 0)) * H + unit;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        ws[g] = KX > 0 ? 1.0f : mine ? p.w_scale[z][g * H + unit] : 0.0f;
-        bias[g] = mine && p.b_ih[z] ? p.b_ih[z][g * H + unit] + p.b_hh[z][g * H + unit] : 0.0f;
-    }
+    for (int g = 0; g < 4; ++g) bias[g] = mine && p.b_ih[z] ? p.b_ih[z][g * H + unit] + p.b_hh[z][g * H + unit] : 0.0f;
     if (mine && p.c0) c = p.c0[state];
-    const float* gx_lane = KX > 0 ? nullptr : p.gx[d] + size_t(mine ? row : 0) * p.gx_row + (mine ? unit : 0);
-    // ---- the row whose h this lane reads; rows past the batch repeat the last one
-    const int hrow = m0 + ln < p.B ? m0 + ln : p.B - 1;
-    const int k_lane = wave * KPW * 32 + lq4 * 8;
-    const int left = H - k_lane;  // columns of this wavefront's first step from k_lane on that exist
-    bool waiting = true;
-    float hv = 0.0f;
-
-    // The input product of a step needs nothing of the step before it, so it is taken while the h of that
-    // step is on its way to the other blocks; its first read is issued before the gates are computed.
-    const unsigned x_off = unsigned(hrow * in_row + kx_lane) * 4;
-    v4u rx[KX > 0 ? KX : 1][2];
-    v4f accx[4];  // scaled
-    auto input_words = [&](int t) { return words_from(in, long(t) * in_step, in_elems); };
-    auto input_product = [&](int t) {
-        if constexpr (KX > 0) {
-            for (int spin = 0;; ++spin) {
-                const unsigned worst = mask_columns<KX>(rx, I - kx_lane);
-                if (!above || !waiting || __builtin_amdgcn_ballot_w64(worst == kEmpty) == 0) break;
-                if (spin >= kSpinLimit) waiting = false;
-                asm volatile("" ::: "memory");
-                load_columns<KX>(rx, input_words(t), x_off);
-            }
+    const float* const gx_lane = XW > 0 ? nullptr : p.gx[d] + size_t(mine ? row : 0) * p.gx_row + (mine ? unit : 0);
+    float gx[4], gx_next[4];
+    auto request_gx = [&](int s) {
+        const float* const at = gx_lane + size_t(d ? p.T - 1 - s : s) * p.gx_step;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) accx[g] = v4f{0.f, 0.f, 0.f, 0.f};
-            multiply<KX>(accx, rx, wxf);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) accx[g] *= scale_x[g];
-        }
+        for (int g = 0; g < 4; ++g) gx_next[g] = at[size_t(g) * H];
     };
-    if constexpr (KX > 0) {
-        const int t = d ? p.T - 1 : 0;
-        load_columns<KX>(rx, input_words(t), x_off);
-        input_product(t);
-    }
-
-    for (int s = 0; s < p.T; ++s) {
+    if (XW == 0 && wave < 4) request_gx(0);
+    // ---- the ring of this group
+    const unsigned slot_bytes = unsigned(gridDim.x) * kSlotWords * 4;
+    const long group = long(z) * ((p.B + kRows - 1) / kRows) + m0 / kRows;
+    const __amdgpu_buffer_rsrc_t ring = __builtin_amdgcn_make_buffer_rsrc(
+        p.rings + group * kSlots * gridDim.x * kSlotWords, 0, int(slot_bytes * kSlots), 0x00020000);
+    const unsigned h_off = unsigned(wave * 2 * KPW * kSlotWords + lane * 4) * 4;
+    // the loads behind which there is a block; the columns of the others stay zero
+    const int blocks_left = int(gridDim.x) - wave * 2 * KPW;
+    const unsigned present = blocks_left <= 0 ? 0u : blocks_left >= 2 * KPW ? ~0u : (1u << blocks_left) - 1u;
+    const unsigned own_off = (blockIdx.x * kSlotWords + wave * 64 + lane) * 4;  // four units of a row side by side
+    const int own_sum = (tile_row & 3) * kGateRow + (tile_row >> 2) * 16 + 4 * wave + (lane & 3);
+    bool waiting = true;
+    unsigned bits = 0;
+    auto store_y = [&](int s) {
         const int t = d ? p.T - 1 - s : s;
-        const int t_next = d ? t - 1 : t + 1;  // of the next step, if there is one
-        float gx[4];
-        if (KX == 0 && mine) {
+        const __amdgpu_buffer_rsrc_t dst = words_from(y, long(t) * p.y_step + long(d) * H, p.y_elems);
+        __builtin_amdgcn_raw_buffer_store_b32(bits, dst, unsigned(row * p.y_row + unit) * 4, 0, kScopeDevice);
+    };
+    v4u raw[KPW][2];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) gx[g] = gx_lane[size_t(t) * p.gx_step + size_t(g) * H];
-        }
-        v4u raw[KPW][2];
-        if (s == 0) {
+    for (int i = 0; i < KPW; ++i) raw[i][0] = raw[i][1] = v4u{0u, 0u, 0u, 0u};
+    if (p.h0) {
 #pragma unroll
-            for (int i = 0; i < KPW; ++i)
+        for (int i = 0; i < KPW; ++i)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int k = k_lane + i * 32 + e;
-                    raw[i][e >> 2][e & 3] =
-                        p.h0 && k < H ? __float_as_uint(p.h0[(size_t(z) * p.B + hrow) * H + k]) : 0u;
-                }
-        } else {
-            const __amdgpu_buffer_rsrc_t src =
-                words_from(y, long(d ? t + 1 : t - 1) * p.y_step + long(d) * H, p.y_elems);
-            const unsigned off = unsigned(hrow * p.y_row + k_lane) * 4;
+            for (int e = 0; e < 8; ++e) {
+                const int k = k_lane + (i * 2 + (e >> 2)) * kRun + (e & 3);
+                const float v = p.h0[(size_t(z) * p.B + in_batch) * H + (k < H ? k : 0)];
+                raw[i][e >> 2][e & 3] = k < H ? __float_as_uint(v) : 0u;
+            }
+    }
+    for (int s = 0; s < p.T; ++s) {
+        v4f in_acc[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) in_acc[g] = v4f{0.f, 0.f, 0.f, 0.f};
+        if (s > 0) {
+            const unsigned slot = unsigned((s - 1) % kSlots) * slot_bytes;
+            // A read that meets the writes of the same line delays both, and one that comes too early costs a whole trip
+            // more: the first is issued when most of h has arrived.  Steps of hidden 512 / 256 / 128, 16 rows, in us: at
+            // once 2.75 / 2.05 / 1.6, after 448 cycles 2.25 / 1.7 / 1.5, after 576 2.2 / 1.7 / 1.45, after 896 2.3 / 1.8 / 1.55.
+            if (gridDim.x > 16) __builtin_amdgcn_s_sleep(8);
+            else __builtin_amdgcn_s_sleep(5);
+            unsigned missing = present;
             for (int spin = 0;; ++spin) {
                 asm volatile("" ::: "memory");  // read again: the words change under the loop
-                load_columns<KPW>(raw, src, off);
-                const unsigned worst = mask_columns<KPW>(raw, left);
-                if (!waiting || __builtin_amdgcn_ballot_w64(worst == kEmpty) == 0) break;
+#pragma unroll
+                for (int i = 0; i < 2 * KPW; ++i)
+                    if (missing >> i & 1)
+                        raw[i >> 1][i & 1] =
+                            __builtin_amdgcn_raw_buffer_load_b128(ring, h_off + unsigned(i * kSlotWords) * 4, slot, kScopeDevice);
+                missing = waiting ? missing_words<KPW>(raw) : 0;
+                if (!missing) break;
                 if (spin >= kSpinLimit) waiting = false;
             }
         }
-        if constexpr (KX > 0) {
-            if (s + 1 < p.T) load_columns<KX>(rx, input_words(t_next), x_off);
+        if constexpr (XW > 0) {
+            lds_barrier();
+            if (wave < XW) {
+                const v4f* const left = reinterpret_cast<const v4f*>(inputs + (s & 1) * Form::kInputFloats) + wave * 4 * 64 + lane;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) in_acc[g] = left[g * 64];
+            }
+        }
+        if (XW == 0 && wave < 4) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) gx[g] = gx_next[g];
+            request_gx(s + 1 < p.T ? s + 1 : s);
         }
         v4f acc[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) acc[g] = v4f{0.f, 0.f, 0.f, 0.f};
         multiply<KPW>(acc, raw, wf);
-        if constexpr (KX > 0) {
+        float* const parts = part + (s & 1) * Form::kPartFloats;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) acc[g] = acc[g] * scale_h[g] + accx[g];
+        for (int g = 0; g < 4; ++g) {
+            acc[g] = acc[g] * scale_h[g] + in_acc[g];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) parts[(wave * 4 + g) * kGateFloats + r * kGateRow + lane] = acc[g][r];
         }
-        float(*const mine_part)[4][64] = part[s & 1][wave];
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mine_part[g][r][lane] = acc[g][r];
         // (a buffer is written again two steps later, after the next step's barrier: by then it has been read)
-        __syncthreads();
+        lds_barrier();
         if (wave < 4) {
             float raw4[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                float sum = part[s & 1][0][g][wave][lane];
+                float sum = parts[g * kGateFloats + own_sum];
 #pragma unroll
-                for (int w = 1; w < W; ++w) sum += part[s & 1][w][g][wave][lane];
-                raw4[g] = mine ? (KX > 0 ? sum : gx[g] + sum * ws[g]) + bias[g] : 0.0f;
+                for (int w = 1; w < W; ++w) sum += parts[(w * 4 + g) * kGateFloats + own_sum];
+                raw4[g] = (XW > 0 ? sum : gx[g] + sum) + bias[g];
             }
-            const float ig = sigmoid(raw4[0]), fg = sigmoid(raw4[1]), gg = tanhf(raw4[2]), og = sigmoid(raw4[3]);
+            const float ig = sigmoid(raw4[0]), fg = sigmoid(raw4[1]), gg = tanh_gate(raw4[2]), og = sigmoid(raw4[3]);
             c = fg * c + ig * gg;
-            hv = og * tanhf(c);
-            if (mine) {
-                unsigned bits = __float_as_uint(hv);
-                bits = bits == kEmpty ? 0x7fc00000u : bits;  // a NaN, but not the one that means "not written"
-                const __amdgpu_buffer_rsrc_t dst = words_from(y, long(t) * p.y_step + long(d) * H, p.y_elems);
-                __builtin_amdgcn_raw_buffer_store_b32(bits, dst, unsigned(row * p.y_row + unit) * 4, 0, kScopeDevice);
+            hv = og * tanh_gate(c);
+            bits = __float_as_uint(hv);
+            bits = bits == kEmpty ? 0x7fc00000u : bits;  // a NaN, but not the one that means "not written"
+            if (s + 1 < p.T) {
+                __builtin_amdgcn_raw_buffer_store_b32(unit < H ? bits : 0u, ring, own_off, unsigned(s % kSlots) * slot_bytes,
+                                                      kScopeDevice);
+                // Every block has taken h[s - 2], or it would not have handed out h[s - 1]: its slot is for h[s + 2].  The
+                // next wait for h[s] is also for this store, so nobody who has h[s + 1] still finds h[s - 2] there.
+                if (s >= 2)
+                    __builtin_amdgcn_raw_buffer_store_b32(kEmpty, ring, own_off, unsigned((s + 2) % kSlots) * slot_bytes,
+                                                          kScopeDevice);
             }
+            if (mine) store_y(s);
         }
-        if (KX > 0 && s + 1 < p.T) input_product(t_next);
     }
     if (mine) {
         p.h_n[state] = hv;
@@ -318,11 +482,11 @@ void lstm_sequence_kernel(LstmArgs p) {
     }
 }
 
-// every word of the outputs "not written yet"
+// every word that is handed from block to block "not written yet": the rings, and the outputs of the layers below others
 __global__ __launch_bounds__(256) void lstm_empty_kernel(LstmArgs p) {
-    float* const y = p.y[blockIdx.y];
-    const long stride = long(gridDim.x) * 256;
-    for (long i = long(blockIdx.x) * 256 + threadIdx.x; i < p.y_elems; i += stride) y[i] = __uint_as_float(kEmpty);
+    unsigned* const words = blockIdx.y ? reinterpret_cast<unsigned*>(p.y[blockIdx.y - 1]) : p.rings;
+    const long n = blockIdx.y ? p.y_elems : p.ring_words, stride = long(gridDim.x) * 256;
+    for (long i = long(blockIdx.x) * 256 + threadIdx.x; i < n; i += stride) words[i] = kEmpty;
 }
 
 // Launches that may be placed at once: the hardware queues of the process, which HIP takes from the environment.
@@ -341,16 +505,20 @@ struct LstmSplit {
     int launches;
 };
 
-template <int W, int KPW, int KX>
+template <int W, int KPW, int XW, int KX>
 int split_lstm(int B, int H, int parts, bool stacked, LstmSplit* out) {
     static DeviceOnce once;
     static int capacity[32] = {0};  // blocks of this kernel the device holds at once
     int dev = 0;
     LQ_HIP(hipGetDevice(&dev));
     const int rc = device_once(once, [&]() -> int {
+        using Form = LstmForm<W, KPW, XW, KX>;
         int per_cu = 0;
         hipDeviceProp_t prop;
-        LQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lstm_sequence_kernel<W, KPW, KX>, W * 64, 0));
+        const auto kernel = lstm_sequence_kernel<W, KPW, XW, KX>;
+        LQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   Form::kLdsBytes));
+        LQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, Form::kThreads, Form::kLdsBytes));
         LQ_HIP(hipGetDeviceProperties(&prop, dev));
         capacity[dev] = per_cu * prop.multiProcessorCount;
         return LQ_OK;
@@ -367,46 +535,51 @@ int split_lstm(int B, int H, int parts, bool stacked, LstmSplit* out) {
     return LQ_OK;
 }
 
-template <int W, int KPW, int KX>
+template <int W, int KPW, int XW, int KX>
 int launch_lstm(LstmArgs p, int parts, hipStream_t st) {
     LstmSplit s;
-    if (int rc = split_lstm<W, KPW, KX>(p.B, p.H, parts, p.stacked != 0, &s)) return rc;
+    if (int rc = split_lstm<W, KPW, XW, KX>(p.B, p.H, parts, p.stacked != 0, &s)) return rc;
     LQ_REQUIRE(s.launches >= 1, LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: %d x hidden %d do not fit the device at once",
                p.stacked ? parts : 1, p.H);
-    const int n_y = p.stacked ? parts : 1;
-    const long fill_blocks = (p.y_elems + 1023) / 1024;
-    hipLaunchKernelGGL(lstm_empty_kernel, dim3(unsigned(fill_blocks < 2048 ? fill_blocks : 2048), unsigned(n_y)), dim3(256),
-                       0, st, p);
+    p.ring_words = long(parts) * s.groups * kSlots * s.per_group * kSlotWords;
+    const auto lock = scratch_lock(st);
+    void* tmp = nullptr;
+    if (int rc = call_buffer(8, size_t(p.ring_words) * 4, st, &tmp)) return rc;
+    p.rings = static_cast<unsigned*>(tmp);
+    const int below = p.stacked ? parts - 1 : 0;
+    const long most = below && p.y_elems > p.ring_words ? p.y_elems : p.ring_words, fill_blocks = (most + 1023) / 1024;
+    hipLaunchKernelGGL(lstm_empty_kernel, dim3(unsigned(fill_blocks < 2048 ? fill_blocks : 2048), unsigned(below + 1)),
+                       dim3(256), 0, st, p);
     LQ_CHECK_LAUNCH("lstm_empty");
     for (p.dir0 = 0; p.dir0 < parts; p.dir0 += s.both)
         for (int g = 0; g < s.groups; g += s.at_once) {
             p.row0 = g * kRows;
             const int n = s.groups - g < s.at_once ? s.groups - g : s.at_once;
-            hipLaunchKernelGGL((lstm_sequence_kernel<W, KPW, KX>), dim3(unsigned(s.per_group), unsigned(n), unsigned(s.both)),
-                               dim3(W * 64), 0, st, p);
+            hipLaunchKernelGGL((lstm_sequence_kernel<W, KPW, XW, KX>),
+                               dim3(unsigned(s.per_group), unsigned(n), unsigned(s.both)),
+                               dim3(unsigned(LstmForm<W, KPW, XW, KX>::kThreads)), unsigned(LstmForm<W, KPW, XW, KX>::kLdsBytes),
+                               st, p);
             LQ_CHECK_LAUNCH("lstm_sequence");
         }
     return LQ_OK;
 }
 
-// f(W, KPW, KX) for the form that serves `hidden` columns and `inputs` (0: gates_x).  More wavefronts
-// before more columns each: a wavefront's loads, splits and products are a serial chain.
+template <int N>
+using Int = std::integral_constant<int, N>;
+
+// f(W, KPW, XW, KX) for the form that serves `hidden` columns and `inputs` (0: gates_x).
 template <typename F>
 int with_form(int hidden, int inputs, F f) {
     const int ks = (hidden + 31) / 32, kx = (inputs + 31) / 32;
-    using std::integral_constant;
     if (kx == 0) {
-        if (ks <= 4) return f(integral_constant<int, 4>(), integral_constant<int, 1>(), integral_constant<int, 0>());
-        if (ks <= 8) return f(integral_constant<int, 8>(), integral_constant<int, 1>(), integral_constant<int, 0>());
-        if (ks <= 16) return f(integral_constant<int, 8>(), integral_constant<int, 2>(), integral_constant<int, 0>());
-        return f(integral_constant<int, 8>(), integral_constant<int, 4>(), integral_constant<int, 0>());
+        if (ks <= 4) return f(Int<4>(), Int<1>(), Int<0>(), Int<0>());
+        if (ks <= 8) return f(Int<8>(), Int<1>(), Int<0>(), Int<0>());
+        if (ks <= 16) return f(Int<8>(), Int<2>(), Int<0>(), Int<0>());
+        return f(Int<8>(), Int<4>(), Int<0>(), Int<0>());
     }
-    if (ks <= 4 && kx <= 4) return f(integral_constant<int, 4>(), integral_constant<int, 1>(), integral_constant<int, 1>());
-    if (ks <= 8)
-        return kx <= 8 ? f(integral_constant<int, 8>(), integral_constant<int, 1>(), integral_constant<int, 1>())
-                       : f(integral_constant<int, 8>(), integral_constant<int, 1>(), integral_constant<int, 2>());
-    return kx <= 8 ? f(integral_constant<int, 8>(), integral_constant<int, 2>(), integral_constant<int, 1>())
-                   : f(integral_constant<int, 8>(), integral_constant<int, 2>(), integral_constant<int, 2>());
+    if (ks <= 4 && kx <= 4) return f(Int<4>(), Int<1>(), Int<4>(), Int<1>());
+    if (ks <= 8) return kx <= 8 ? f(Int<4>(), Int<2>(), Int<4>(), Int<2>()) : f(Int<4>(), Int<2>(), Int<4>(), Int<4>());
+    return kx <= 8 ? f(Int<4>(), Int<4>(), Int<4>(), Int<2>()) : f(Int<4>(), Int<4>(), Int<4>(), Int<4>());
 }
 constexpr int kMaxFused = 512;  // hidden and input columns of a form that takes the input product
 constexpr int kMaxHidden = 1024;
@@ -433,8 +606,8 @@ int lq_lstm_sequence_pays(int batch, int hidden, int directions, int* pays) {
     *pays = 0;
     if (batch == 0 || hidden > kMaxHidden) return LQ_OK;
     LstmSplit s;
-    const int rc = with_form(hidden, 0, [&](auto w, auto k, auto x) {
-        return split_lstm<w(), k(), x()>(batch, hidden, directions, false, &s);
+    const int rc = with_form(hidden, 0, [&](auto w, auto k, auto xw, auto x) {
+        return split_lstm<w(), k(), xw(), x()>(batch, hidden, directions, false, &s);
     });
     if (rc) return rc;
     *pays = s.launches > 0 && s.launches * sequence_step_us(hidden) <= directions * gemm_step_us(batch, hidden);
@@ -452,13 +625,13 @@ int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layer
     // weight it reads, is worth twelve (43 us at 1024 x 2048 x 512, a step 3.4).
     constexpr long kGemm = 12;
     LstmSplit s;
-    int rc = with_form(hidden, 0, [&](auto w, auto k, auto x) { return split_lstm<w(), k(), x()>(batch, hidden, directions, false, &s); });
+    int rc = with_form(hidden, 0, [&](auto w, auto k, auto xw, auto x) { return split_lstm<w(), k(), xw(), x()>(batch, hidden, directions, false, &s); });
     if (rc) return rc;
     double best = s.launches ? double(s.launches) * steps + kGemm * directions : 1e30;
     for (int n = 1; n <= (directions == 1 ? (layers < kParts ? layers : kParts) : 1); ++n) {
         const int columns = n > 1 && hidden > inputs ? hidden : inputs;
-        rc = with_form(hidden, columns, [&](auto w, auto k, auto x) {
-            return split_lstm<w(), k(), x()>(batch, hidden, directions == 2 ? 2 : n, n > 1, &s);
+        rc = with_form(hidden, columns, [&](auto w, auto k, auto xw, auto x) {
+            return split_lstm<w(), k(), xw(), x()>(batch, hidden, directions == 2 ? 2 : n, n > 1, &s);
         });
         if (rc) return rc;
         const double cost = double(s.launches) * (steps + n - 1) / n;
@@ -511,7 +684,7 @@ int lq_lstm_sequence_f32(const lq_lstm_args* a, lq_stream stream) {
                    (!a->x || (p.B - 1) * p.x_row + p.I < 0x7fffffffL / 4),
                LQ_ERR_NOT_IMPLEMENTED, "lstm_sequence: %ld outputs or %ld inputs are too many", p.y_elems, p.x_elems);
     const int columns = !a->x ? 0 : p.stacked && p.H > p.I ? p.H : p.I;
-    return with_form(p.H, columns, [&](auto w, auto k, auto x) { return launch_lstm<w(), k(), x()>(p, parts, as_stream(stream)); });
+    return with_form(p.H, columns, [&](auto w, auto k, auto xw, auto x) { return launch_lstm<w(), k(), xw(), x()>(p, parts, as_stream(stream)); });
 }
 
 }  // extern "C"

@@ -290,6 +290,31 @@ def test_dynamic_lstm(layers, bidir, batch_first, bias, with_state):
     assert np.abs(yf - y.numpy()).mean() / (np.abs(yf).mean() + 1e-9) < 0.03
 
 
+@pytest.mark.parametrize("I,H,layers,Bn,Tn,bidir", [(5, 16, 1, 1, 11, False), (31, 40, 3, 17, 9, False), (2, 2, 1, 16, 6, True),
+                                                    (300, 257, 1, 33, 13, False), (600, 512, 1, 16, 10, True)])
+def test_dynamic_lstm_steps_reuse_what_blocks_hand_over(I, H, layers, Bn, Tn, bidir):
+    # more steps than the ring between the blocks holds, sizes that end inside a load; values across the gates' branches
+    # (tanh changes form at 0.6, the exponentials are clamped at 60 and 20) and one sequence with a NaN and one with large
+    # inputs, which must stay theirs.  2e-5 as in the tests above; a float32 sum of the large inputs may be off by
+    # 2^-23 sum |x w| (both sides round; no gate is steeper than 1), which a cell adds up over the steps.
+    rng = np.random.default_rng(H)
+    lstm = nn.LSTM(I, H, num_layers=layers, bidirectional=bidir)
+    qm = Q.quantize_dynamic(lstm)
+    x = rng.standard_normal((Tn, Bn, I)).astype(np.float32) * np.float32(3)
+    if Bn > 1:
+        x[Tn // 2, 1, 0] = np.nan
+        x[:, 0] *= np.float32(30)
+    slack = Tn * 2.0 ** -23 * np.abs(x[:, 0]).sum(axis=1).max() / np.sqrt(H)
+    y, (hn, cn) = qm(hip(x))
+    with np.errstate(over="ignore", invalid="ignore"):
+        wy, wh, wc = _oracle_lstm_stack(qm, x, None, False)
+    for got, want in ((y.numpy(), wy), (hn.numpy(), wh), (cn.numpy(), wc)):
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        off = np.where(ok, np.abs(got - want), 0.0)  # (rows are axis 1)
+        assert off[:, 1:].max(initial=0.0) < 2e-5 and off[:, 0].max() < 2e-5 + slack
+
+
 @pytest.mark.parametrize("I,H,Bn,Tn,bidir,batch_first",
                          [(3, 1, 1, 3, False, False), (8, 17, 5, 4, True, True), (16, 33, 16, 2, False, True),
                           (8, 128, 17, 3, True, False), (7, 129, 33, 2, False, False), (16, 300, 3, 1, True, True),
