@@ -332,7 +332,7 @@ def call(name: str, *args):
     if _current_stream is not None and args and args[-1] is None and name in _stream_last():
         args = args[:-1] + (_current_stream,)
     rc = fn(*args)
-    if name not in _NO_STATUS:
+    if rc and name not in _NO_STATUS:
         check(rc)
     return rc
 

@@ -57,37 +57,53 @@ def qlinear_i8(a: Tensor, w: Tensor, *, a_zp: int = 0, a_zp_dev: Tensor | None =
     N = w.shape[0]
     if out is None:
         out = Tensor.empty((M, N), _OUT_DTYPE[out_mode], "hip")
-    args = _C.QLinearArgs()
+    args = _C.QLinearArgs()  # (zeros: what is absent is not set)
     args.a, args.w = _ptr(a, "a", T.int8), _ptr(w, "w", T.int8)
     args.M, args.N, args.K = M, N, K
-    args.wsum = _ptr(wsum, "wsum", T.int32)
-    args.a_zp = int(a_zp)
-    args.a_zp_dev = _ptr(a_zp_dev, "a_zp_dev", T.float32)
-    args.a_scale = _ptr(a_scale, "a_scale", T.float32)
-    args.a_scale_per_row = int(a_scale is not None and a_scale.numel != 1)
-    if a_scale is not None and a_scale.numel not in (1, M):
-        raise _C.ShapeMismatch(f"a_scale has {a_scale.numel} entries for M = {M}")
-    if w_scale is not None and w_scale.numel != N:
-        raise _C.ShapeMismatch(f"w_scale has {w_scale.numel} entries for N = {N}")
-    args.w_scale = _ptr(w_scale, "w_scale", T.float32)
-    args.bias = _ptr(bias, "bias", (T.float32, T.float16))
-    args.bias_dtype = bias.dtype.code if bias is not None else 0
-    if bias is not None and bias.numel != N:
-        raise _C.ShapeMismatch(f"bias has {bias.numel} entries for N = {N}")
+    if wsum is not None:
+        args.wsum = _ptr(wsum, "wsum", T.int32)
+    if a_zp:
+        args.a_zp = int(a_zp)
+    if a_zp_dev is not None:
+        args.a_zp_dev = _ptr(a_zp_dev, "a_zp_dev", T.float32)
+    if a_scale is not None:
+        args.a_scale = _ptr(a_scale, "a_scale", T.float32)
+        entries = a_scale.numel
+        args.a_scale_per_row = int(entries != 1)
+        if entries not in (1, M):
+            raise _C.ShapeMismatch(f"a_scale has {entries} entries for M = {M}")
+    if w_scale is not None:
+        if w_scale.numel != N:
+            raise _C.ShapeMismatch(f"w_scale has {w_scale.numel} entries for N = {N}")
+        args.w_scale = _ptr(w_scale, "w_scale", T.float32)
+    if bias is not None:
+        args.bias = _ptr(bias, "bias", (T.float32, T.float16))
+        args.bias_dtype = bias.dtype.code
+        if bias.numel != N:
+            raise _C.ShapeMismatch(f"bias has {bias.numel} entries for N = {N}")
     args.relu, args.out_mode = int(relu), int(out_mode)
-    args.out_scale = _ptr(out_scale, "out_scale", T.float32)
-    args.out_zp = _ptr(out_zp, "out_zp", T.float32)
+    if out_scale is not None:
+        args.out_scale = _ptr(out_scale, "out_scale", T.float32)
+    if out_zp is not None:
+        args.out_zp = _ptr(out_zp, "out_zp", T.float32)
     args.out_qmin, args.out_qmax, args.out_offset = int(out_qmin), int(out_qmax), int(out_offset)
-    args.out, args.ldo, args.force_path = out.data_ptr, 0, int(path)
-    args.tile_config = int(tile_config)
-    if residual is not None and residual.numel != M * N:
-        raise _C.ShapeMismatch(f"residual has {residual.numel} elements for an output of {M}x{N}")
-    args.residual, args.ldr = _ptr(residual, "residual", T.float32), 0
-    _fill_join(args.join, join, (M, N))
-    args.gelu, args.range = int(gelu), _ptr(range_buf, "range", T.float32)
-    if w_zp is not None and w_zp.numel != N:
-        raise _C.ShapeMismatch(f"w_zp has {w_zp.numel} entries for N = {N}")
-    args.w_zp = _ptr(w_zp, "w_zp", T.int32)
+    args.out = out.data_ptr
+    if path or tile_config:
+        args.force_path, args.tile_config = int(path), int(tile_config)
+    if residual is not None:
+        if residual.numel != M * N:
+            raise _C.ShapeMismatch(f"residual has {residual.numel} elements for an output of {M}x{N}")
+        args.residual = _ptr(residual, "residual", T.float32)
+    if join is not None:
+        _fill_join(args.join, join, (M, N))
+    if gelu:
+        args.gelu = int(gelu)
+    if range_buf is not None:
+        args.range = _ptr(range_buf, "range", T.float32)
+    if w_zp is not None:
+        if w_zp.numel != N:
+            raise _C.ShapeMismatch(f"w_zp has {w_zp.numel} entries for N = {N}")
+        args.w_zp = _ptr(w_zp, "w_zp", T.int32)
     if repeat == 1:
         _C.call("lq_qlinear_i8", C.byref(args), None)
     else:

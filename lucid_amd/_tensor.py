@@ -14,7 +14,6 @@ from __future__ import annotations
 
 import ctypes as C
 import math
-import weakref
 from dataclasses import dataclass
 
 import numpy as np
@@ -23,7 +22,7 @@ from . import _C
 
 
 # ---------------------------------------------------------------- dtypes
-@dataclass(frozen=True)
+@dataclass(frozen=True, eq=False)
 class dtype:
     """Element type; ``code`` is Lucid's ``Dtype`` enum value (``core/Dtype.h``)."""
 
@@ -34,6 +33,17 @@ class dtype:
 
     def __repr__(self) -> str:
         return f"lucid.{self.name}"
+
+    # (one object per type, so nearly always the identity decides: the generated comparison builds two tuples first)
+    def __eq__(self, other) -> bool:
+        if self is other:
+            return True
+        if other.__class__ is not self.__class__:
+            return NotImplemented
+        return (self.name, self.code, self.itemsize, self.np) == (other.name, other.code, other.itemsize, other.np)
+
+    def __hash__(self) -> int:
+        return hash((self.name, self.code, self.itemsize, self.np))
 
     # (one object per type: what tells types apart by identity does so in a copied module too)
     def __copy__(self) -> "dtype":
@@ -98,24 +108,28 @@ class Grid:
 
 
 class DeviceBuffer:
-    """Owns one ``lq_alloc`` allocation; freed when the last reference dies."""
+    """Owns one ``lq_alloc`` allocation; freed when the last reference dies.
 
-    __slots__ = ("ptr", "nbytes", "_fin", "__weakref__")
+    (Every operator makes at least one: a ``weakref.finalize`` in place of ``__del__`` took 3 of the
+    5 us that an empty tensor costs the host.)"""
+
+    __slots__ = ("ptr", "nbytes", "__weakref__")
 
     def __init__(self, nbytes: int) -> None:
-        _C.init()
+        self.ptr = None
+        if _C._initialised_device != 0:
+            _C.init()
         p = C.c_void_p()
         _C.call("lq_alloc", C.byref(p), int(nbytes))
         self.ptr = p.value
         self.nbytes = int(nbytes)
-        self._fin = weakref.finalize(self, _free, self.ptr)
 
-
-def _free(ptr) -> None:
-    try:
-        _C.load().lq_free(ptr)
-    except Exception:  # interpreter shutdown
-        pass
+    def __del__(self) -> None:
+        try:
+            if self.ptr is not None:
+                _C.load().lq_free(self.ptr)
+        except Exception:  # interpreter shutdown
+            pass
 
 
 class Tensor:
@@ -139,6 +153,12 @@ class Tensor:
     # -- construction
     @staticmethod
     def empty(shape, dt=float32, device="hip") -> "Tensor":
+        if device == "hip" and type(dt) is dtype and type(shape) is tuple and all([type(s) is int for s in shape]):
+            # (nothing to normalise: the operators' own outputs)
+            t = _new_tensor(Tensor)
+            t.shape, t.dtype, t.device = shape, dt, "hip"
+            t._buf, t._host, t._offset, t._grid, t._range = DeviceBuffer(math.prod(shape) * dt.itemsize), None, 0, None, None
+            return t
         dt = as_dtype(dt)
         shape = tuple(int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,)))
         n = math.prod(shape)
@@ -372,6 +392,9 @@ class Tensor:
     def __deepcopy__(self, memo) -> "Tensor":
         # a device allocation has exactly one owner: copy the bytes, not the handle
         return self.clone()
+
+
+_new_tensor = object.__new__
 
 
 def tensor(data, dtype=None, device="cpu") -> Tensor:

@@ -9,12 +9,14 @@ here; the per-element arithmetic and its order are unchanged.
 from __future__ import annotations
 
 import ctypes as C
+import math
 
 import numpy as np
 
 from .. import _C
 from .. import _tensor as T
 from .._tensor import Tensor
+from ._qparams import calculate_qparams
 from ._qscheme import QDtype
 
 
@@ -22,14 +24,12 @@ def _extents(shape, ch_axis):
     """Split ``shape`` around ``ch_axis`` into (outer, C, inner) - the
     broadcast of ``_reshape_for_channel`` (``_functional.py:45-54``)."""
     if ch_axis is None:
-        return 1, 1, int(np.prod(shape, dtype=np.int64))
+        return 1, 1, math.prod(shape)
     nd = len(shape)
     if not -nd <= ch_axis < nd:
         raise IndexError(f"ch_axis {ch_axis} out of range for rank {nd}")
     ch_axis %= nd
-    outer = int(np.prod(shape[:ch_axis], dtype=np.int64))
-    inner = int(np.prod(shape[ch_axis + 1:], dtype=np.int64))
-    return outer, int(shape[ch_axis]), inner
+    return math.prod(shape[:ch_axis]), int(shape[ch_axis]), math.prod(shape[ch_axis + 1:])
 
 
 class _QP:
@@ -72,7 +72,8 @@ class _QP:
             v = T.tensor(np.float32(float(v)))
         if v.dtype != T.float32:
             raise _C.DtypeMismatch(f"scale / zero_point must be float32, got {v.dtype}")
-        v = v.to("hip")
+        if v.device != "hip":
+            v = v.to("hip")
         self.keep.append(v)
         return v
 
@@ -140,7 +141,6 @@ def quantize_rows_dynamic(x: Tensor, qscheme, qdtype: QDtype, eps: float = 1e-8
     (``observer.py:634-653``, ``_qparams.py:198-215``, ``_functional.py:164-182``) with ``x``
     read once.  Rows the one-pass kernel does not take (longer than 16384, not a multiple
     of 4, int16 storage) go through those three calls."""
-    from ._qparams import calculate_qparams
     _require_hip(x, "quantize_rows_dynamic")
     if x.dtype != T.float32 or x.ndim != 2:
         raise _C.DtypeMismatch(f"quantize_rows_dynamic expects a 2-d float32 tensor, got {x.dtype} {x.shape}")

@@ -32,7 +32,7 @@ def _as_hip_f32(v) -> Tensor:
     if isinstance(v, Tensor):
         if v.dtype != float32:
             raise _C.DtypeMismatch(f"calculate_qparams expects float32 ranges, got {v.dtype}")
-        return v.to("hip")
+        return v if v.device == "hip" else v.to("hip")
     return tensor(np.float32(float(v)), device="hip")
 
 
