@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256) void wq_prepare_kernel(const float* __restrict
         for (int e = 0; e < 4; ++e)
             for (int r = 0; r < per; ++r)
                 if ((g0 + e) * per + r < stages * segs)
-                    sb[size_t((g0 + e) * per + r) * n_pad + n] = float2{kWqUnit<BITS, kWqCentre<BITS>> * s[e], b[e] - float(kWqCentre<BITS>) * s[e]};
+                    sb[size_t((g0 + e) * per + r) * n_pad + n] = float2{kWqUnit<BITS> * s[e], b[e] - float(kWqCentre<BITS>) * s[e]};
         return;
     }
     const unsigned pairs = unsigned(stages + 1) / 2;
@@ -277,7 +277,7 @@ void wq_gemm_kernel(const char* __restrict__ parts, const char* __restrict__ xsu
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
                     const uint32_t w4[4] = {wd[ii][j][0], wd[ii][j][1], 0u, 0u};
-                    cf[j] = __builtin_bit_cast(v8bf, wq_codes<BITS, kWqCentre<BITS>>(w4, 0));
+                    cf[j] = __builtin_bit_cast(v8bf, wq_codes<BITS>(w4, 0));
                 }
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
@@ -406,17 +406,18 @@ int launch(const float* x, const uint32_t* packed, const float* scales, const fl
 namespace lq {
 
 // The small-batch kernel splits K between its blocks (512 k each), so it fills the chip where M x N alone
-// does not, but reads and decodes the weight once per 16 rows: 8 us + 31 ns (int4) or 38 ns (int8) per block.
+// does not, but reads and decodes the weight once per 16 rows: 6.5 us + 30 ns (int4) or 35 ns (int8) per 256 rows x 512 k.
 // This one prepares its operands first (7 us).  Both timed over 17 .. 512 rows, N 300 .. 32000, K 1024 .. 11008 and
 // every group size: what this picks is 0.7 % slower than the better one on average; from 65 rows 1.6 x at worst (512 x
 // 1000 x 1024: 12.7 / 20.1 us), 3 % of the problems by more than 5 %.  Up to 64 rows the estimates are closer together,
 // so it has to be a tenth the faster one (0.4 % on average, 1.2 x at worst; with the small-batch kernel for all of them
-// 11 % and 2.6 x).  us, small batch / this: 64 x 32000 x 4096 int4 groups of 128 131 / 74, int8 of 64 156 / 98;
+// 11 % and 2.6 x; all of this with 8 us + 31 or 38 ns per block, before the small-batch kernel was a fifth faster).  us, small
+// batch / this: 64 x 32000 x 4096 int4 groups of 128 131 / 74, int8 of 64 156 / 98;
 // 64 x 11008 x 4096 int4 of 64 46 / 56.
 bool wq_gemm_beats_small_batch(int M, int N, int K, int gs, int bits) {
     if (size_t(N) * K * bits / 8 >= 0x7fffffffull) return false;  // its weight offsets are 32-bit
     const double blocks = double((M + 15) / 16) * ((N + 255) / 256) * ((K + 511) / 512);
-    return 7.0 + wq_gemm_tile(M, N, wq_stages(K, gs)).us < (M <= 64 ? 0.9 : 1.0) * (8.0 + blocks * (bits == 4 ? 0.031 : 0.038));
+    return 7.0 + wq_gemm_tile(M, N, wq_stages(K, gs)).us < (M <= 64 ? 0.9 : 1.0) * (6.5 + blocks * (bits == 4 ? 0.030 : 0.035));
 }
 
 int launch_wq_gemm(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,

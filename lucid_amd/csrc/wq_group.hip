@@ -257,7 +257,7 @@ int launch_gemv1(const float* x, const uint32_t* packed, const float* scales, co
 //
 // y[m, n] = sum over groups g of  s[n, g] * (sum_{k in g} c[n, k] x[m, k])  +  b[n, g] * (sum_{k in g} x[m, k]):
 // the inner sums run on v_mfma_f32_16x16x32_bf16 with the codes themselves as one operand -
-// a code c enters exactly as c + OFF (wq_codes) and the OFF goes into the bias term - and x as the
+// a code c enters exactly as c - 2^(bits-1) (wq_codes), which goes into the bias term - and x as the
 // other, split into three bfloat16 parts x = hi + mid + lo (exact: 8 + 8 + 8 significant
 // bits, wq_split3x2), one MFMA each.  Products are exact and accumulate in float32, so nothing of x or
 // of the weight is rounded before the sums.
@@ -277,23 +277,26 @@ int launch_gemv1(const float* x, const uint32_t* packed, const float* scales, co
 // quarter) matrix is transposed (v_permlane32_swap + v_permlane16_swap), so instruction i
 // holds the k of quarter i.  Which k a slot of an instruction ends up with does not matter
 // as long as x follows: the block writes the three parts of its x range into LDS in exactly
-// that order.  The sum of x over a group segment comes from the same fragments against a
-// row of ones (one more accumulator tile per wavefront), already in the layout the lanes
-// need it in.
+// that order.  The threads that split x also add it up per group segment, in float32
+// pair by pair, and leave the sums in LDS (as one more accumulator tile against a row of ones they took a third of the
+// matrix instructions).
 //
 // Every block needs the x of its k range next to its weights (64 bytes of x per k against
 // rows / 2 or rows bytes of codes), and every block converts it again.  So a block takes
-// many rows (256: eight wavefronts with two 16-row tiles each) and a short k range (512),
-// keeps that range's fragments in LDS for all its wavefronts, and requests all its weights
-// at once when it starts.  The k ranges of a row tile are blocks of their own (grid.y); each
+// many rows (eight wavefronts with one to three 16-row tiles each, wq_tiles_per_wave) and a short k range (512),
+// keeps that range's fragments in LDS for all its wavefronts, and requests its first weights
+// when it starts.  The k ranges of a row tile are blocks of their own (grid.y); each
 // writes its partial sums to a slab, and the last one to arrive (an arrival counter per row
 // tile, reset by that block) adds the slabs in index order - the result does not depend on
 // the order of arrival - and stores.  One launch, no workspace besides the slabs.
-// LDS a block may ask for: 48 KiB of x fragments and the tables of 256 rows x 16 groups
-constexpr int kWqMaxLds = 512 / 32 * 3 * 64 * 16 + 2 * 256 * 17 * 4;
-
-constexpr int kWqRows = 256;    // weight rows per block
 constexpr int kWqSliceK = 512;  // k per block
+constexpr int kWqWaves = 8;
+// weight rows of a block whose wavefronts take `rb` tiles of 16 each
+constexpr int wq_rows(int rb) { return kWqWaves * rb * 16; }
+// its LDS: 48 KiB of x fragments, the sums of x per group segment, the tables of its rows
+constexpr size_t wq_lds_bytes(int rb, int gs) {
+    return size_t(kWqSliceK / 32) * 3 * 64 * 16 + (kWqSliceK / 32) * 16 * 4 + size_t(2) * wq_rows(rb) * (kWqSliceK / gs + 1) * 4;
+}
 
 // Where the A fragment of row m, lane quarter qd of instruction block `blk` sits among the block's
 // 64 16-byte slots.  The threads of a wavefront that write the fragments share one m and differ in
@@ -303,18 +306,31 @@ constexpr int kWqSliceK = 512;  // k per block
 // stay conflict-free.
 __device__ __forceinline__ int wq_x_slot(int m, int qd, int blk) { return ((m + 4 * qd + blk) & 15) + 16 * qd; }
 
-template <int BITS, int SW, int OFF>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void wq_mfma_kernel(
+// lanes of a group of N neighbours (4, 8 or 16): everyone gets the sum
+template <int N>
+__device__ __forceinline__ float wq_neighbour_sum(float v) {
+    auto moved = [&](auto ctrl) { return __uint_as_float(unsigned(__builtin_amdgcn_mov_dpp(int(__float_as_uint(v)), ctrl(), 0xf, 0xf, true))); };
+    v += moved(std::integral_constant<int, 0xb1>());  // the other of the pair
+    v += moved(std::integral_constant<int, 0x4e>());  // the other pair of the quad
+    if (N >= 8) v += moved(std::integral_constant<int, 0x141>());   // the other quad (lanes 0..7 mirrored)
+    if (N >= 16) v += moved(std::integral_constant<int, 0x140>());  // the other eight (lanes 0..15 mirrored)
+    return v;
+}
+
+template <int BITS, int SW, int RB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4 : 2, RB <= 2 ? 4 : 2))) void wq_mfma_kernel(
     const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N, int K,
     int gs_shift, float* out, float* slabs, int* counters) {
     using G = WqGeom<BITS>;
     constexpr int CODES = G::CODES, WK = G::WK, NI = G::NI;
     constexpr int GW = 1 << SW, SEG = WK / GW;  // group segments per window and their length
     constexpr int IPS = NI / GW;                // instructions per segment
-    constexpr int RB = 2, WAVES = 8, WPS = kWqSliceK / WK;  // windows per block: 4 or 8
+    constexpr int WAVES = kWqWaves, WPS = kWqSliceK / WK;  // windows per block: 4 or 8
+    constexpr int kWqRows = wq_rows(RB);
     constexpr int UNITS = WPS * NI * 64;                    // (window, instruction, lane) triples of the block's x
+    constexpr int AHEAD = RB == 1 ? WPS : 2;                // windows of weights a wavefront has requested and not used
     static_assert(IPS >= 1, "a segment is at least one instruction");
-    static_assert(WAVES * RB * 16 == kWqRows && UNITS % 512 == 0, "");
+    static_assert(UNITS % 512 == 0, "");
     // Dynamic LDS: the x fragments of the block's windows ([window][instruction][part][lane],
     // 16 bytes each), then the block's rows of scales and of biases for the groups of those
     // windows - each row padded by one float: lanes of a quarter read 16 different rows at the
@@ -385,28 +401,34 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             raw[u][1] = *reinterpret_cast<const float4*>(src + 4);
         }
     }
-    // All the weights of this wavefront are requested now and used window by window.  For the
-    // request a lane takes quarter lane % 4 of row lane / 4 - four neighbouring lanes read 64
+    // The weights of the first windows are requested now (of all of them where a wavefront has one tile; more tiles keep
+    // enough bytes in flight with two, in a loop of a third of the code).  For the request a lane takes quarter lane % 4 of row lane / 4 - four neighbouring lanes read 64
     // contiguous bytes, where the operand layout (row lane % 16, quarter lane / 16) would make
     // every lane a cache access of its own -; a lane permutation below puts each 16 bytes
     // where the instruction wants them.
-    uint4 wv[WPS][RB];
+    const uint32_t* row[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         int n = n_base + rb * 16 + (lane >> 2);
         n = n < N ? n : N - 1;  // clamped rows are computed and dropped at the store
-        const uint32_t* row = packed + size_t(n) * words_per_row + (lane & 3) * (CODES * BITS / 32);
-#pragma unroll
-        for (int wi = 0; wi < WPS; ++wi)
-            // past K every lane reads the same 16 bytes: one cache line, dropped later or multiplied by zeros of x
-            wv[wi][rb] = *reinterpret_cast<const uint4*>(
-                (w0 + wi) * WK + (lane & 3) * CODES < k_end ? row + (w0 + wi) * (WK * BITS / 32) : packed);
+        row[rb] = packed + size_t(n) * words_per_row + (lane & 3) * (CODES * BITS / 32);
     }
+    auto fetch = [&](uint4 (&w)[RB], int wi) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+            // past K every lane reads the same 16 bytes: one cache line, dropped later or multiplied by zeros of x
+            w[rb] = *reinterpret_cast<const uint4*>(
+                (w0 + wi) * WK + (lane & 3) * CODES < k_end ? row[rb] + (w0 + wi) * (WK * BITS / 32) : packed);
+    };
+    uint4 ahead[AHEAD][RB];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) fetch(ahead[j], j);
     // The tables go to LDS, then x, split and laid out as fragments by the block itself: a thread
     // finds the (instruction, quarter) that holds its eight k - the exchange of registers is its
     // own inverse.
     uint4* x_lds = wq_lds;
-    float* s_lds = reinterpret_cast<float*>(wq_lds + WPS * NI * 3 * 64);
+    float* sum_lds = reinterpret_cast<float*>(wq_lds + WPS * NI * 3 * 64);  // of x: [segment][row]
+    float* s_lds = sum_lds + kWqSliceK / 32 * 16;
     float* b_lds = s_lds + kWqRows * gp;
 #pragma unroll
     for (int u = 0; u < kTabVec; ++u) {
@@ -428,6 +450,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             const int i = BITS == 4 ? rho : rho / 2;
             const float v[8] = {raw[u][0].x, raw[u][0].y, raw[u][0].z, raw[u][0].w,
                                 raw[u][1].x, raw[u][1].y, raw[u][1].z, raw[u][1].w};
+            // a wavefront has one row of x: the segments' sums, in float32, pair by pair
+            const float sum = wq_neighbour_sum<SEG / 8>(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+            if (lane % (SEG / 8) == 0) sum_lds[kl / SEG * 16 + ml] = sum;
             uint32_t d3[3][4];
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
@@ -448,56 +473,59 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) y[rb] = v4f{0.f, 0.f, 0.f, 0.f};
     const int row_in_tile = wave * (RB * 16) + r;
-    const uint4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // eight times 1.0
+    auto window = [&](int wi, const uint4 (&wv)[RB]) {
+        uint32_t wd[RB][4];
 #pragma unroll
-    for (int wi = 0; wi < WPS; ++wi) {
-        if (wi < nw) {
-            uint32_t wd[RB][4];
+        for (int rb = 0; rb < RB; ++rb) {
+            // lane (row r, quarter q) takes what lane 4 r + q loaded
+            const int from = (4 * r + q) * 4;
+            wd[rb][0] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[rb].x)));
+            wd[rb][1] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[rb].y)));
+            wd[rb][2] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[rb].z)));
+            wd[rb][3] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[rb].w)));
+            wq_exchange<SW>(wd[rb]);
+        }
+#pragma unroll
+        for (int e = 0; e < GW; ++e) {
+            const int g = (((w0 + wi) * WK + e * SEG) >> gs_shift) - g0;
+            v4f acc[RB];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) acc[rb] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ii = 0; ii < IPS; ++ii) {
+                const int i = e * IPS + ii;
+                uint4 cf[RB];
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) cf[rb] = wq_codes<BITS>(wd[rb], i);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) {
+                    const v8bf xf = __builtin_bit_cast(v8bf, x_lds[((wi * NI + i) * 3 + p) * 64 + wq_x_slot(lane & 15, lane >> 4, wi * NI + i)]);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+                        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, __builtin_bit_cast(v8bf, cf[rb]),
+                                                                          acc[rb], 0, 0, 0);
+                }
+            }
+            const v4f sums = *reinterpret_cast<const v4f*>(sum_lds + (wi * GW + e) * 16 + 4 * q);  // of the lane's rows m
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                // lane (row r, quarter q) takes what lane 4 r + q loaded
-                const int from = (4 * r + q) * 4;
-                wd[rb][0] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[wi][rb].x)));
-                wd[rb][1] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[wi][rb].y)));
-                wd[rb][2] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[wi][rb].z)));
-                wd[rb][3] = uint32_t(__builtin_amdgcn_ds_bpermute(from, int(wv[wi][rb].w)));
-                wq_exchange<SW>(wd[rb]);
-            }
+                const float sc = s_lds[(row_in_tile + rb * 16) * gp + g];
+                const float bi = b_lds[(row_in_tile + rb * 16) * gp + g];
+                // the codes entered as (c + centre) / unit
+                const float bz = bi - float(kWqCentre<BITS>) * sc;
 #pragma unroll
-            for (int e = 0; e < GW; ++e) {
-                const int g = (((w0 + wi) * WK + e * SEG) >> gs_shift) - g0;
-                // acc[RB]: the segment's sum of x, from the same fragments against a row of ones (every
-                // column of that tile holds it: exactly the value each lane needs for its rows m)
-                v4f acc[RB + 1];
-#pragma unroll
-                for (int rb = 0; rb <= RB; ++rb) acc[rb] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int ii = 0; ii < IPS; ++ii) {
-                    const int i = e * IPS + ii;
-                    uint4 cf[RB];
-#pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) cf[rb] = wq_codes<BITS, OFF>(wd[rb], i);
-#pragma unroll
-                    for (int p = 0; p < 3; ++p) {
-                        const v8bf xf = __builtin_bit_cast(v8bf, x_lds[((wi * NI + i) * 3 + p) * 64 + wq_x_slot(lane & 15, lane >> 4, wi * NI + i)]);
-#pragma unroll
-                        for (int rb = 0; rb < RB; ++rb)
-                            acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, __builtin_bit_cast(v8bf, cf[rb]),
-                                                                              acc[rb], 0, 0, 0);
-                        acc[RB] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, __builtin_bit_cast(v8bf, ones), acc[RB], 0, 0, 0);
-                    }
-                }
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    const float sc = s_lds[(row_in_tile + rb * 16) * gp + g];
-                    const float bi = b_lds[(row_in_tile + rb * 16) * gp + g];
-                    // the codes entered as (c + OFF) / unit
-                    const float bz = OFF != 0 ? bi - float(OFF) * sc : bi;
-                    y[rb] = y[rb] + (acc[rb] * (kWqUnit<BITS, OFF> * sc) + acc[RB] * bz);
-                }
+                for (int t = 0; t < 4; ++t)
+                    y[rb][t] = __builtin_fmaf(acc[rb][t], kWqUnit<BITS> * sc, __builtin_fmaf(sums[t], bz, y[rb][t]));
             }
         }
-    }
+    };
+#pragma unroll 1
+    for (int w = 0; w < nw; w += AHEAD)
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+            if (w + j < nw) window(w + j, ahead[j]);
+            if (AHEAD < WPS) fetch(ahead[j], w + j + AHEAD);
+        }
 
     // accumulator element t of a lane: row m = 4 * quarter + t, column n = lane % 16
     auto store_out = [&](const v4f (&v)[RB]) {
@@ -566,53 +594,65 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 }
 
 
-template <int BITS>
-int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
-                   int K, int gs, float* out, hipStream_t st) {
+// Tiles of 16 weight rows per wavefront.  One tile spreads a small weight over the most CUs and leaves room for two blocks on
+// one; three need a CU each, and fetch and split x for the fewest blocks.  us of 1 / 2 / 3 tiles, and of two tiles with all
+// weights requested at once and the sums of x on the matrix unit: 16 x 4096 x 4096 int8 groups of 32 (256 / 128 / 88 blocks)
+// 10.0 / 13.1 / 16.1, 13.9; 16 x 11008 x 4096 int8 of 64 (688 / 344 / 232) 20.6 / 20.1 / 18.8, 22.4; the same int4
+// 19.0 / 19.3 / 19.0, 18.8; 64 x 4096 x 4096 int4 of 64 (1024 / 512 / 352) 21.6 / 18.0 / 27.3, 18.7; 16 x 32000 x 4096 int4
+// of 128 (2000 / 1000 / 672) 38.0 / 37.0 / 46.0, 37.6; 5 x 4096 x 11008 int4 of 32 (704 / 352 / 242) 22.9 / 27.2 / 25.1, 26.9;
+// 3 x 300 x 512 int4 of 64 5.1 / 7.7 / 9.6, 6.8.  The costs below follow those, in us behind the first 3.
+int wq_tiles_per_wave(int M, int N, int slices, int sw) {
+    constexpr double kBlock[4] = {0.0, 4.8, 7.7, 14.5};
+    int best = 1;
+    double least = 1e30;
+    for (int rb = 1; rb <= 3; ++rb) {
+        const long blocks = long((M + 15) / 16) * ((N + wq_rows(rb) - 1) / wq_rows(rb)) * slices;
+        // (four groups per window: three tiles of them are more than a block has registers and LDS for)
+        const double cost = double((blocks + 255) / 256) * (kBlock[rb] + (rb == 3 && sw == 2 ? 4.0 : 0.0)) + (rb < 3 ? 2.0 : 0.5);
+        if (cost < least) least = cost, best = rb;
+    }
+    return best;
+}
+
+template <int BITS, int SW, int RB>
+int launch_wq_mfma_form(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
+                        int K, int gs, float* out, hipStream_t st) {
     using G = WqGeom<BITS>;
     constexpr int WPS = kWqSliceK / G::WK;
-    const int sw = wq_swap_mode(BITS, gs);
     const int mblocks = (M + 15) / 16, windows = (K + G::WK - 1) / G::WK;
-    const int tiles = (N + kWqRows - 1) / kWqRows, slices = (windows + WPS - 1) / WPS;
+    const int tiles = (N + wq_rows(RB) - 1) / wq_rows(RB), slices = (windows + WPS - 1) / WPS;
+    static DeviceOnce attr_once;
+    if (const int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SW, RB>),
+                                         int(wq_lds_bytes(RB, 32))))
+        return rc;
     SkScratch sk;
     const auto lock = scratch_lock(st);
     if (slices > 1) {
-        const int rc = sk_scratch(size_t(mblocks) * tiles, size_t(mblocks) * tiles * slices * (8 * 2 * 64 * 16), st, &sk);
+        const int rc = sk_scratch(size_t(mblocks) * tiles, size_t(mblocks) * tiles * slices * (kWqWaves * RB * 64 * 16), st, &sk);
         if (rc) return rc;
     }
-    const dim3 grid{unsigned(slices), unsigned(tiles), unsigned(mblocks)};
-    const int gs_shift = 31 - __builtin_clz(unsigned(gs));
-    const int gmax = kWqSliceK / gs;
-    const size_t lds = size_t(WPS) * G::NI * 3 * 64 * 16 + size_t(2) * kWqRows * ((gmax < 1 ? 1 : gmax) + 1) * 4;
-    // 2 .. 64 rows of whole windows keep the offset, and so the bits, that they have always had here
-    constexpr int kFirst = BITS == 4 ? 128 : 0, kOther = kWqCentre<BITS>;
-    const bool first = M > 1 && M <= 64 && K % G::WK == 0;
-#define LQ_WQ_LAUNCH(SWM)                                                                                         \
-    do {                                                                                                          \
-        if (first)                                                                                                \
-            LQ_WQ_LAUNCH_OFF(SWM, kFirst);                                                                        \
-        else                                                                                                      \
-            LQ_WQ_LAUNCH_OFF(SWM, kOther);                                                                        \
-    } while (0)
-#define LQ_WQ_LAUNCH_OFF(SWM, OFF)                                                                                \
-    do {                                                                                                          \
-        static DeviceOnce attr_once;                                                                              \
-        const int arc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SWM, OFF>), \
-                                          kWqMaxLds);                                                             \
-        if (arc) return arc;                                                                                      \
-        hipLaunchKernelGGL((wq_mfma_kernel<BITS, SWM, OFF>), grid, dim3(512), lds, st, x, packed, scales, biases, M, \
-                           N, K, gs_shift, out, reinterpret_cast<float*>(sk.slabs), sk.counters);                 \
-    } while (0)
-    if (sw == 0)
-        LQ_WQ_LAUNCH(0);
-    else if (sw == 1)
-        LQ_WQ_LAUNCH(1);
-    else if constexpr (BITS == 4)
-        LQ_WQ_LAUNCH(2);
-#undef LQ_WQ_LAUNCH
-#undef LQ_WQ_LAUNCH_OFF
+    hipLaunchKernelGGL((wq_mfma_kernel<BITS, SW, RB>), dim3(unsigned(slices), unsigned(tiles), unsigned(mblocks)), dim3(512),
+                       wq_lds_bytes(RB, gs), st, x, packed, scales, biases, M, N, K, 31 - __builtin_clz(unsigned(gs)), out,
+                       reinterpret_cast<float*>(sk.slabs), sk.counters);
     LQ_CHECK_LAUNCH("wq_mfma");
     return LQ_OK;
+}
+
+template <int BITS>
+int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
+                   int K, int gs, float* out, hipStream_t st) {
+    const int sw = wq_swap_mode(BITS, gs), rb = wq_tiles_per_wave(M, N, (K + kWqSliceK - 1) / kWqSliceK, sw);
+#define LQ_WQ_FORM(SWM, RBS) \
+    if (sw == SWM && rb == RBS) return launch_wq_mfma_form<BITS, SWM, RBS>(x, packed, scales, biases, M, N, K, gs, out, st)
+#define LQ_WQ_FORMS(SWM) LQ_WQ_FORM(SWM, 1); LQ_WQ_FORM(SWM, 2); LQ_WQ_FORM(SWM, 3)
+    LQ_WQ_FORMS(0);
+    LQ_WQ_FORMS(1);
+    if constexpr (BITS == 4) {
+        LQ_WQ_FORMS(2);
+    }
+#undef LQ_WQ_FORMS
+#undef LQ_WQ_FORM
+    return fail(LQ_ERR_VALUE, "wq_matmul: group_size %d, bits %d", gs, BITS);
 }
 
 int check_group(const char* who, int K, int gs, int bits) {

@@ -76,6 +76,24 @@ def test_small_batch_matmul_is_reproducible_and_exact_on_exact_inputs(bits):
     assert np.array_equal(y1.astype(np.float64), x.astype(np.float64) @ w.T)
 
 
+# the small-batch kernel with one, two and three tiles per wavefront (how many blocks each would have decides): rows that
+# end inside a tile and inside a block, batches that end inside sixteen, a last window and a last k range that are partial
+@pytest.mark.parametrize("M,N,K,gs,bits", [(2, 127, 544, 32, 4), (17, 129, 1088, 64, 8), (16, 4097, 4096, 128, 4),
+                                           (31, 8191, 2112, 64, 8), (7, 11007, 4096, 64, 8), (16, 10999, 4224, 128, 4),
+                                           (13, 7000, 6176, 32, 4), (64, 4100, 4096, 32, 8)])
+def test_small_batch_forms_against_float64(M, N, K, gs, bits):
+    rng = np.random.default_rng(N)
+    w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
+    x = np.abs(rng.standard_normal((M, K))).astype(np.float32)  # a mean, which the groups' biases cancel
+    packed, s, b = _qgemm.quantize(hip(w), gs, bits)
+    y = _qgemm.quantized_matmul(hip(x), packed, s, b, True, gs, bits).numpy()
+    ref = x.astype(np.float64) @ W.dequantize(packed.numpy(), s.numpy(), b.numpy(), gs, bits).astype(np.float64).T
+    # products are exact; a float32 sum of K / 32 of them per lane chain, then K / gs groups and K / 512 slabs: a few 2^-24
+    # of the root mean square for each, and the decoded weight of the reference is itself rounded (2^-24 each)
+    assert np.linalg.norm(y - ref) <= 1e-6 * np.linalg.norm(ref)
+    assert np.abs(y - ref).max() <= 2e-5 * np.sqrt(np.mean(ref ** 2))
+
+
 @pytest.mark.parametrize("M,N,K,gs,bits", [
     (1025, 3003, 288, 32, 4), (700, 2500, 416, 32, 8), (513, 4097, 256, 64, 4), (300, 6000, 256, 128, 8),
     (130, 11008, 320, 64, 8), (600, 1000, 1024, 64, 4), (1100, 5370, 128, 128, 4), (1100, 5370, 96, 32, 8),
