@@ -513,6 +513,12 @@ size_t lq_range_buffer_bytes(void);
 int lq_calc_qparams_from_range(const float* range, int symmetric, int qmin, int qmax, int is_signed,
                                float eps, float* scale, float* zp, float* mn_out, float* mx_out,
                                lq_stream stream);
+/* The same and the int8 codes of the tensor whose range it is (n floats at x; code_offset as
+ * in lq_quantize): lq_calc_qparams_from_range + lq_quantize, bit for bit, in one launch for
+ * up to 4 Mi elements. */
+int lq_quantize_from_range_i8(const float* x, size_t n, const float* range, int symmetric, int qmin, int qmax,
+                              int is_signed, float eps, int code_offset, float* scale, float* zp, int8_t* q,
+                              lq_stream stream);
 
 /* ------------------------------------------------- float32 steps of a ViT block */
 /* What Lucid's dynamic-quantized ViT keeps in float32 between its int8 Linears
@@ -539,6 +545,11 @@ int lq_layernorm_stats_f32(const float* x, const float* gamma, const float* beta
 int lq_layernorm_quantize_i8(const float* x, const float* gamma, const float* beta, const float* stats, long rows,
                              int cols, const float* scale, const float* zp, int qmin, int qmax, int code_offset,
                              int8_t* q, lq_stream stream);
+/* lq_calc_qparams_from_range + lq_layernorm_quantize_i8, in one launch for up to 2048 rows; scale, zp: out. */
+int lq_layernorm_quantize_from_range_i8(const float* x, const float* gamma, const float* beta, const float* stats,
+                                        long rows, int cols, const float* range, int symmetric, int qmin, int qmax,
+                                        int is_signed, float eps, int code_offset, float* scale, float* zp, int8_t* q,
+                                        lq_stream stream);
 
 /* GELU, exact erf form (lucid/nn/functional/activations.py:219, approximate="none"). */
 int lq_gelu_f32(const float* x, float* out, size_t n, float* range, lq_stream stream);

@@ -31,4 +31,49 @@ __device__ __forceinline__ void range_block_store(float* range, float lo, float 
     }
 }
 
+// The range itself, for every thread of a block (up to 1024; all must call it): the reduction of the slots.
+__device__ __forceinline__ void range_block_load(const float* __restrict__ range, float& mn, float& mx) {
+    const unsigned n = reinterpret_cast<const unsigned*>(range)[0];
+    mn = __builtin_inff(), mx = -__builtin_inff();
+    int nan = 0;
+    for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
+        const float a = range[4 + i], b = range[4 + kRangeSlots + i];
+        nan |= (a != a) | (b != b);
+        mn = fminf(mn, a);
+        mx = fmaxf(mx, b);
+    }
+    block_minmax(mn, mx, nan);
+    if (nan) mn = mx = __builtin_nanf("");
+}
+
+// vDSP_vmax / vDSP_vmin single precision propagate NaN (Vdsp.cpp:140-151).
+__device__ __forceinline__ float vmaxf(float a, float b) {
+    if (a != a || b != b) return __builtin_nanf("");
+    return a > b ? a : b;
+}
+__device__ __forceinline__ float vminf(float a, float b) {
+    if (a != a || b != b) return __builtin_nanf("");
+    return a < b ? a : b;
+}
+
+// lucid/quantization/_qparams.py:198-215, float32 throughout.
+__device__ __forceinline__ void qparams_of(float mn, float mx, int symmetric, int qmin, int qmax,
+                                           int is_signed, float eps, float half_range, float* scale,
+                                           float* zp) {
+    float lo = vminf(mn, 0.0f);
+    float hi = vmaxf(mx, 0.0f);
+    if (symmetric) {
+        float max_abs = vmaxf(fabsf(lo), fabsf(hi));
+        *scale = vmaxf(max_abs / half_range, eps);
+        *zp = is_signed ? 0.0f : float((qmax + qmin + 1) >> 1);
+    } else {
+        float s = vmaxf((hi - lo) / float(qmax - qmin), eps);
+        float z = float(qmin) - __builtin_rintf(lo / s);
+        float qlo = float(qmin), qhi = float(qmax);
+        z = (z < qlo) ? qlo : ((z > qhi) ? qhi : z);
+        *scale = s;
+        *zp = z;
+    }
+}
+
 }  // namespace lq

@@ -216,34 +216,61 @@ __global__ __launch_bounds__(256) void layernorm_stats_kernel(const float* __res
     range_block_store(range, lo, hi, nan);
 }
 
+// four codes of normalized values
+__device__ __forceinline__ uint32_t layernorm_codes(float4 v, float4 g, float4 b, float mean, float rstd, const QGrid& G, int off) {
+    const int c0 = int(quant_fast<false>(((v.x - mean) * rstd) * g.x + b.x, G)) + off;
+    const int c1 = int(quant_fast<false>(((v.y - mean) * rstd) * g.y + b.y, G)) + off;
+    const int c2 = int(quant_fast<false>(((v.z - mean) * rstd) * g.z + b.z, G)) + off;
+    const int c3 = int(quant_fast<false>(((v.w - mean) * rstd) * g.w + b.w, G)) + off;
+    return uint32_t(c0 & 0xff) | (uint32_t(c1 & 0xff) << 8) | (uint32_t(c2 & 0xff) << 16) | (uint32_t(c3) << 24);
+}
+
+constexpr long kRangeRows = 2048;  // rows whose blocks reduce the kept range themselves
+// One wavefront per row.  RANGE: the grid is that of the kept range, which every block reduces while its rows are on
+// their way; the first block hands it out.
+struct LnGrid {
+    const float* range;
+    int symmetric, qmin, qmax, is_signed;
+    float eps, half_range;
+};
+template <int KEEP, bool RANGE>
 __global__ __launch_bounds__(256) void layernorm_quantize_kernel(const float* __restrict__ x,
                                                                  const float* __restrict__ gamma,
                                                                  const float* __restrict__ beta,
                                                                  const float* __restrict__ stats, long rows, int cols,
-                                                                 const float* __restrict__ scale,
-                                                                 const float* __restrict__ zp, float qlo, float qhi,
-                                                                 int off, int8_t* __restrict__ q) {
+                                                                 float* scale, float* zp, LnGrid grid, int off,
+                                                                 int8_t* __restrict__ q) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long row = long(blockIdx.x) * 4 + wave;
-    if (row >= rows) return;
-    const QGrid G = make_qgrid(scale[0], zp[0], qlo, qhi, true);
-    const float mean = stats[2 * row], rstd = stats[2 * row + 1];
-    const float* xr = x + row * cols;
-    int8_t* qr = q + row * cols;
+    const long at = row < rows ? row : 0;
+    const float* xr = x + at * cols;
+    float4 v[KEEP], g[KEEP], b[KEEP];
 #pragma unroll
-    for (int u = 0; u < LN_KEEP; ++u) {
+    for (int u = 0; u < KEEP; ++u) {
         const int c = lane * 4 + u * 256;
         if (c < cols) {
-            const float4 v = *reinterpret_cast<const float4*>(xr + c);
-            const float4 g = *reinterpret_cast<const float4*>(gamma + c);
-            const float4 b = *reinterpret_cast<const float4*>(beta + c);
-            const int c0 = int(quant_fast<false>(((v.x - mean) * rstd) * g.x + b.x, G)) + off;
-            const int c1 = int(quant_fast<false>(((v.y - mean) * rstd) * g.y + b.y, G)) + off;
-            const int c2 = int(quant_fast<false>(((v.z - mean) * rstd) * g.z + b.z, G)) + off;
-            const int c3 = int(quant_fast<false>(((v.w - mean) * rstd) * g.w + b.w, G)) + off;
-            *reinterpret_cast<uint32_t*>(qr + c) = uint32_t(c0 & 0xff) | (uint32_t(c1 & 0xff) << 8) |
-                                                   (uint32_t(c2 & 0xff) << 16) | (uint32_t(c3) << 24);
+            v[u] = *reinterpret_cast<const float4*>(xr + c);
+            g[u] = *reinterpret_cast<const float4*>(gamma + c);
+            b[u] = *reinterpret_cast<const float4*>(beta + c);
         }
+    }
+    const float mean = stats[2 * at], rstd = stats[2 * at + 1];
+    float s, z;
+    if constexpr (RANGE) {
+        float mn, mx;
+        range_block_load(grid.range, mn, mx);
+        qparams_of(mn, mx, grid.symmetric, grid.qmin, grid.qmax, grid.is_signed, grid.eps, grid.half_range, &s, &z);
+        if (blockIdx.x == 0 && threadIdx.x == 0) *scale = s, *zp = z;
+    } else {
+        s = *scale, z = *zp;
+    }
+    if (row >= rows) return;
+    const QGrid G = make_qgrid(s, z, float(grid.qmin), float(grid.qmax), true);
+    int8_t* qr = q + row * cols;
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u) {
+        const int c = lane * 4 + u * 256;
+        if (c < cols) *reinterpret_cast<uint32_t*>(qr + c) = layernorm_codes(v[u], g[u], b[u], mean, rstd, G, off);
     }
 }
 
@@ -959,21 +986,56 @@ int lq_layernorm_stats_f32(const float* x, const float* gamma, const float* beta
     return LQ_OK;
 }
 
-int lq_layernorm_quantize_i8(const float* x, const float* gamma, const float* beta, const float* stats, long rows,
-                             int cols, const float* scale, const float* zp, int qmin, int qmax, int code_offset,
-                             int8_t* q, void* stream) {
+namespace {
+int launch_layernorm_quantize(const float* x, const float* gamma, const float* beta, const float* stats, long rows, int cols,
+                              float* scale, float* zp, const LnGrid& grid, int code_offset, int8_t* q, void* stream) {
     LQ_REQUIRE(x && gamma && beta && stats && scale && zp && q, LQ_ERR_VALUE, "layernorm_quantize: null pointer");
     LQ_REQUIRE(rows >= 0 && cols > 0, LQ_ERR_SHAPE, "layernorm_quantize: bad shape (%ld, %d)", rows, cols);
     LQ_REQUIRE(cols % 4 == 0 && cols <= LN_KEEP * 256 && aligned16(x) && aligned16(gamma) && aligned16(beta) &&
                    (reinterpret_cast<uintptr_t>(q) & 3u) == 0,
                LQ_ERR_NOT_IMPLEMENTED, "layernorm_quantize: rows of %d floats are not what the fused form takes", cols);
-    LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
-               "layernorm_quantize: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
+    LQ_REQUIRE(grid.qmax > grid.qmin && grid.qmin + code_offset >= -128 && grid.qmax + code_offset <= 127, LQ_ERR_VALUE,
+               "layernorm_quantize: grid [%d,%d] + offset %d does not fit int8", grid.qmin, grid.qmax, code_offset);
     if (rows == 0) return LQ_OK;
-    layernorm_quantize_kernel<<<unsigned((rows + 3) / 4), 256, 0, as_stream(stream)>>>(
-        x, gamma, beta, stats, rows, cols, scale, zp, float(qmin), float(qmax), code_offset, q);
+    const long blocks = (rows + 3) / 4;
+    LQ_REQUIRE(blocks < 0x7fffffffL, LQ_ERR_SHAPE, "layernorm_quantize: too many rows");
+#define LQ_LN_QUANTIZE(KEEP, RANGE) \
+    layernorm_quantize_kernel<KEEP, RANGE><<<unsigned(blocks), 256, 0, as_stream(stream)>>>(x, gamma, beta, stats, rows, \
+                                                                                                  cols, scale, zp, grid, code_offset, q)
+    if (cols <= 4 * 256 && grid.range)
+        LQ_LN_QUANTIZE(4, true);
+    else if (cols <= 4 * 256)
+        LQ_LN_QUANTIZE(4, false);
+    else if (grid.range)
+        LQ_LN_QUANTIZE(LN_KEEP, true);
+    else
+        LQ_LN_QUANTIZE(LN_KEEP, false);
+#undef LQ_LN_QUANTIZE
     LQ_CHECK_LAUNCH();
     return LQ_OK;
+}
+}  // namespace
+
+int lq_layernorm_quantize_i8(const float* x, const float* gamma, const float* beta, const float* stats, long rows,
+                             int cols, const float* scale, const float* zp, int qmin, int qmax, int code_offset,
+                             int8_t* q, void* stream) {
+    const LnGrid grid{nullptr, 0, qmin, qmax, 0, 0.0f, 0.0f};
+    return launch_layernorm_quantize(x, gamma, beta, stats, rows, cols, const_cast<float*>(scale), const_cast<float*>(zp), grid,
+                                     code_offset, q, stream);
+}
+
+int lq_layernorm_quantize_from_range_i8(const float* x, const float* gamma, const float* beta, const float* stats, long rows,
+                                        int cols, const float* range, int symmetric, int qmin, int qmax, int is_signed,
+                                        float eps, int code_offset, float* scale, float* zp, int8_t* q, void* stream) {
+    LQ_REQUIRE(range && scale && zp, LQ_ERR_VALUE, "layernorm_quantize: null pointer");
+    // Every block of the one launch reads a slot per block of the statistics: up to 2048 rows that is less than the launch it
+    // saves (12 608 rows of 768: 16.6 us against 8.3 + 4.6).
+    if (rows > kRangeRows) {
+        const int rc = lq_calc_qparams_from_range(range, symmetric, qmin, qmax, is_signed, eps, scale, zp, nullptr, nullptr, stream);
+        return rc ? rc : lq_layernorm_quantize_i8(x, gamma, beta, stats, rows, cols, scale, zp, qmin, qmax, code_offset, q, stream);
+    }
+    const LnGrid grid{range, symmetric, qmin, qmax, is_signed, eps, float((double(qmax) - double(qmin)) / 2.0)};
+    return launch_layernorm_quantize(x, gamma, beta, stats, rows, cols, scale, zp, grid, code_offset, q, stream);
 }
 
 int lq_gelu_f32(const float* x, float* out, size_t n, float* range, void* stream) {

@@ -64,11 +64,10 @@ def layer_norm_dynamic_quantize(x: Tensor, normalized_shape, weight: Tensor, bia
     _C.call("lq_layernorm_stats_f32", x.data_ptr, weight.data_ptr, bias.data_ptr, rows, cols, float(eps),
             stats.data_ptr, rng.data_ptr, None)
     scale, zp = Tensor.empty((), T.float32, "hip"), Tensor.empty((), T.float32, "hip")
-    _C.call("lq_calc_qparams_from_range", rng.data_ptr, 0, qdtype.quant_min, qdtype.quant_max, int(qdtype.signed),
-            1e-8, scale.data_ptr, zp.data_ptr, None, None, None)
     q = Tensor.empty((rows, cols), T.int8, "hip")
-    _C.call("lq_layernorm_quantize_i8", x.data_ptr, weight.data_ptr, bias.data_ptr, stats.data_ptr, rows, cols,
-            scale.data_ptr, zp.data_ptr, qdtype.quant_min, qdtype.quant_max, storage_offset(qdtype), q.data_ptr, None)
+    _C.call("lq_layernorm_quantize_from_range_i8", x.data_ptr, weight.data_ptr, bias.data_ptr, stats.data_ptr, rows, cols,
+            rng.data_ptr, 0, qdtype.quant_min, qdtype.quant_max, int(qdtype.signed), 1e-8, storage_offset(qdtype),
+            scale.data_ptr, zp.data_ptr, q.data_ptr, None)
     return q, scale, zp
 
 

@@ -223,15 +223,15 @@ class Linear(Module):
                     qd.quant_max, int(qd.signed), 1e-8, off, x_scale.data_ptr, x_zp.data_ptr, None, None,
                     xq.data_ptr if x.numel else None, None)
         elif x._range is not None:
-            # the kernel that wrote x kept its min / max: qparams straight from them
+            # the kernel that wrote x kept its min / max: qparams and codes straight from them
             x_scale = Tensor.empty((), T.float32, "hip")
             x_zp = Tensor.empty((), T.float32, "hip")
-            _C.call("lq_calc_qparams_from_range", x._range.data_ptr, 0, qd.quant_min, qd.quant_max,
-                    int(qd.signed), 1e-8, x_scale.data_ptr, x_zp.data_ptr, None, None, None)
+            _C.call("lq_quantize_from_range_i8", x.data_ptr if x.numel else None, x.numel, x._range.data_ptr, 0, qd.quant_min,
+                    qd.quant_max, int(qd.signed), 1e-8, off, x_scale.data_ptr, x_zp.data_ptr,
+                    xq.data_ptr if x.numel else None, None)
         else:
             mn, mx = minmax(x)
             x_scale, x_zp = calculate_qparams(mn, mx, per_tensor_affine, qd)
-        if not small:
             _C.call("lq_quantize", x.data_ptr, xq.data_ptr, _C.I8, off, 1, 1, x.numel,
                     x_scale.data_ptr, x_zp.data_ptr, 0, qd.quant_min, qd.quant_max, None)
         return self.forward_quantized(xq, x_scale, x_zp, x.shape[:-1], residual, activation, track_range)

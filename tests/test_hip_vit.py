@@ -294,7 +294,8 @@ def test_vit_block_fused_and_unfused_gelu_agree(monkeypatch):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-@pytest.mark.parametrize("rows,cols", [(394, 768), (12608, 768), (5, 192), (7, 2048), (64, 4)])
+@pytest.mark.parametrize("rows,cols", [(394, 768), (12608, 768), (5, 192), (7, 2048), (64, 4), (1, 4),
+                                       (2048, 64), (2049, 64), (2050, 1028)])
 def test_layernorm_dynamic_quantize_equals_layernorm_then_quantize(rows, cols):
     """LayerNorm that writes the next dynamic Linear's codes directly: codes, scale and zero
     point are the bits of layer_norm(track_range) + calc_qparams_from_range + quantize."""
@@ -325,6 +326,34 @@ def test_layernorm_dynamic_quantize_declines_other_rows():
     x = hip(np.zeros((4, 2052), np.float32))
     w = hip(np.ones(2052, np.float32))
     assert F.layer_norm_dynamic_quantize(x, 2052, w, w, 1e-6, Q.quint8) is None
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 8191, 8192, 8195, 1 << 22, (1 << 22) + 2])  # tails, one block and one more, one launch and two
+@pytest.mark.parametrize("nan", [False, True])
+def test_codes_straight_from_a_kept_range(n, nan):
+    """``lq_quantize_from_range_i8`` writes the scale, zero point and codes of the two calls it stands for."""
+    from lucid_amd.nn.functional import _new_range
+    rng = np.random.default_rng(n)
+    a = (rng.standard_normal(n) * 3 + 1).astype(np.float32)
+    if nan:
+        a[n // 2] = np.nan
+    x = L.tensor(a, device="hip")
+    y, kept = L.Tensor.empty((n,), L.float32, "hip"), _new_range()
+    _C.call("lq_gelu_f32", x.data_ptr, y.data_ptr, n, kept.data_ptr, None)
+    one, two = [[L.Tensor.empty((), L.float32, "hip"), L.Tensor.empty((), L.float32, "hip"), L.Tensor.empty((n,), L.int8, "hip")]
+                for _ in range(2)]
+    _C.call("lq_calc_qparams_from_range", kept.data_ptr, 0, 0, 255, 0, 1e-8, one[0].data_ptr, one[1].data_ptr, None, None, None)
+    _C.call("lq_quantize", y.data_ptr, one[2].data_ptr, _C.I8, -128, 1, 1, n, one[0].data_ptr, one[1].data_ptr, 0, 0, 255, None)
+    _C.call("lq_quantize_from_range_i8", y.data_ptr, n, kept.data_ptr, 0, 0, 255, 0, 1e-8, -128, two[0].data_ptr,
+            two[1].data_ptr, two[2].data_ptr, None)
+    for a1, a2 in zip(one, two):
+        assert a1.numpy().tobytes() == a2.numpy().tobytes()
+    if n > 8:  # an address that vectors cannot take
+        _C.call("lq_quantize", y.data_ptr + 4, one[2].data_ptr, _C.I8, -128, 1, 1, n - 1, one[0].data_ptr, one[1].data_ptr, 0, 0,
+                255, None)
+        _C.call("lq_quantize_from_range_i8", y.data_ptr + 4, n - 1, kept.data_ptr, 0, 0, 255, 0, 1e-8, -128, two[0].data_ptr,
+                two[1].data_ptr, two[2].data_ptr, None)
+        assert np.array_equal(one[2].numpy()[:n - 1], two[2].numpy()[:n - 1])
 
 
 def test_vit_block_with_and_without_fused_layernorm_quantize_agree(monkeypatch):
