@@ -63,6 +63,9 @@ struct SkScratch {
     int32_t* slabs = nullptr;
 };
 int sk_scratch(size_t counters, size_t slab_bytes, hipStream_t st, SkScratch* out);
+// Launches that may be placed at once: the hardware queues of the process, which HIP takes from the environment (four unless
+// GPU_MAX_HW_QUEUES says more).  What a kernel whose blocks wait for each other leaves free for launches like it.
+int hardware_queues();
 // Resolves, for the current device, the address of the static scratch array that
 // lq_minmax_noalloc uses (called by lq_init; the entry point does it on first use otherwise).
 int minmax_noalloc_init();

@@ -489,16 +489,6 @@ __global__ __launch_bounds__(256) void lstm_empty_kernel(LstmArgs p) {
     for (long i = long(blockIdx.x) * 256 + threadIdx.x; i < n; i += stride) words[i] = kEmpty;
 }
 
-// Launches that may be placed at once: the hardware queues of the process, which HIP takes from the environment.
-int hardware_queues() {
-    static const int n = [] {
-        const char* v = std::getenv("GPU_MAX_HW_QUEUES");
-        const long q = v ? std::strtol(v, nullptr, 10) : 0;
-        return q > 4 ? int(q < 1024 ? q : 1024) : 4;
-    }();
-    return n;
-}
-
 // Launches of one kernel form: 16-row groups of one direction or of one stack, as many at once as may be.
 struct LstmSplit {
     int per_group, groups, at_once, both;  // blocks of a group; groups; groups of a launch; its parts

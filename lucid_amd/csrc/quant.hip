@@ -695,7 +695,8 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 // block in device memory - written through, and polled by every block until it is filled - and each block then
 // derives the qparams itself and writes its codes.  The last block to leave empties the slots for the next
 // launch.  All blocks have to be resident (see lstm.hip on what the launcher has to leave free: kExchange
-// blocks of 512 threads and 64 registers are far below it), and a wait is bounded.
+// blocks of 512 threads and 64 registers are the quarter of the device that one of four hardware queues may have; with more
+// queues it is fewer blocks, exchange_blocks), and a wait is bounded.
 //
 // Beyond, and under capture (slots cleared inside a graph are unset until its replay), two launches: slices'
 // ranges (minmax_seg_kernel), then this kernel with PARTS - every block reduces
@@ -703,11 +704,13 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 //
 // Rows of `cols` elements go to rows of `ld` codes, zeros past `cols` (what a GEMM of ragged rows wants).
 //
-// 8192 elements 3.4 us, 65536 (8 blocks, the exchange) 5.9; with all 128 blocks of 1 M elements polling each other's
-// slots it was 17 us, in two launches 3.8 + 5.0.  Before: one block on one CU for up to 262144 elements (61 us), five
-// launches beyond (1 M elements: 12.3 us).
+// 8192 elements 3.4 us, 65536 (8 blocks, the exchange) 5.9.  A slot is read first when most of them have been written, and
+// not at once again: 128 blocks of 1 M elements that polled without a pause took 17 us, in two launches 3.8 + 5.0.  A dynamic
+// Linear behind it, in two launches / in one, us: 333 x 1000 -> 1001 16.6 / 13.6, 256 x 4096 -> 1024 (128 blocks) 25.7 / 24.9,
+// 512 x 4096 -> 1024 (256) 32.7 / 30.7.  Before either: one block on one CU for up to 262144 elements (61 us), five launches
+// beyond (1 M elements: 12.3 us).
 constexpr int kDynThreads = 512, kDynQuads = 4, kDynPerBlock = kDynThreads * kDynQuads * 4;
-constexpr int kExchange = 16, kMaxParts = 512;
+constexpr int kExchange = 256, kMaxParts = 512;
 constexpr unsigned long long kSlotEmpty = ~0ull;  // NaNs that no range contains: mm_write's NaN is the canonical one
 struct DynScratch {
     unsigned long long slot[kExchange];    // low word: the block's minimum, high word: its maximum
@@ -801,8 +804,11 @@ void quantize_tensor_dynamic_kernel(const float* __restrict__ x, size_t n, unsig
         m = MinMax{__builtin_inff(), -__builtin_inff(), 0};
         if (tid < int(gridDim.x)) {
             unsigned long long got = kSlotEmpty;
-            for (int spin = 0; got == kSlotEmpty && spin < (1 << 20); ++spin)
+            __builtin_amdgcn_s_sleep(12);
+            for (int spin = 0; got == kSlotEmpty && spin < (1 << 20); ++spin) {
+                if (spin) __builtin_amdgcn_s_sleep(4);
                 got = __hip_atomic_load(&slots->slot[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
             m.lo = __uint_as_float(unsigned(got)), m.hi = __uint_as_float(unsigned(got >> 32));
             m.nan = (m.lo != m.lo) | (m.hi != m.hi);
         }
@@ -1373,6 +1379,27 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     }
 }
 
+// Blocks that may meet through the slots: the share of the device that one hardware queue may have (16, the least, are far
+// below any).
+int exchange_blocks(int* most) {
+    static DeviceOnce once;
+    static int capacity[32] = {0};
+    int dev = 0;
+    LQ_HIP(hipGetDevice(&dev));
+    const int rc = device_once(once, [&]() -> int {
+        int flat = 0, ragged = 0, cus = 0;
+        LQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&flat, quantize_tensor_dynamic_kernel<false, false>, kDynThreads, 0));
+        LQ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&ragged, quantize_tensor_dynamic_kernel<false, true>, kDynThreads, 0));
+        LQ_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        capacity[dev] = (flat < ragged ? flat : ragged) * cus;
+        return LQ_OK;
+    });
+    if (rc) return rc;
+    const int share = capacity[dev] / hardware_queues();
+    *most = share < 16 ? 16 : share < kExchange ? share : kExchange;
+    return LQ_OK;
+}
+
 // Dynamic per-tensor quantization of n = rows * cols elements to rows of ld codes.
 int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int symmetric, int qmin, int qmax, int is_signed,
                     float eps, int off, float* scale, float* zp, float* mn, float* mx, int8_t* q, hipStream_t st) {
@@ -1383,7 +1410,11 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
     LQ_REQUIRE((!ragged || blocks * kDynPerBlock < (size_t(1) << 32)) && blocks < 0x7fffffffull, LQ_ERR_SHAPE,
                "dynamic quantization of %zu elements", n);
     void* tmp = nullptr;
-    bool exchange = blocks <= size_t(kExchange), fresh = false;
+    int most = 1;
+    if (blocks > 1 && blocks <= size_t(kExchange)) {
+        if (const int rc = exchange_blocks(&most)) return rc;
+    }
+    bool exchange = blocks <= size_t(most), fresh = false;
     std::unique_lock<std::recursive_mutex> lock;
     if (blocks > 1) {
         lock = scratch_lock(st);

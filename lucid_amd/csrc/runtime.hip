@@ -1,5 +1,6 @@
 // Runtime entry points of the C ABI: device selection, storage, transfers,
 // events, the op registry and synthetic-data fills.
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -120,6 +121,15 @@ std::unique_lock<std::recursive_mutex> scratch_lock(hipStream_t stream) {
     (void)hipGetDevice(&dev);
     const uint64_t h = (reinterpret_cast<uintptr_t>(stream) + uint64_t(dev)) * 0x9e3779b97f4a7c15ull;
     return std::unique_lock<std::recursive_mutex>(mu[h >> 58]);
+}
+
+int hardware_queues() {
+    static const int n = [] {
+        const char* v = std::getenv("GPU_MAX_HW_QUEUES");
+        const long q = v ? std::strtol(v, nullptr, 10) : 0;
+        return q > 4 ? int(q < 1024 ? q : 1024) : 4;
+    }();
+    return n;
 }
 
 int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr) {

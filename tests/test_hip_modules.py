@@ -533,10 +533,11 @@ def test_dynamic_linear_wide_layer_at_small_batch(M, K):
 @pytest.mark.parametrize("M,K,N", [(1, 1, 1), (1, 17, 1100), (1, 4095, 33), (1, 4097, 2100), (1, 16384, 7),  # a stream of the weight
                                    (1, 16385, 40), (3, 5, 7), (2, 2731, 3), (2, 4097, 65),  # 1 and 2 blocks of 8192, ragged rows
                                    (65, 126, 130), (100, 250, 257), (257, 8160, 65),
-                                   # 16 blocks of 8192 codes, which exchange their ranges, whole and partial, and 17, which
-                                   # get them from slices
+                                   # 16 and 17 blocks of 8192 codes, which exchange their ranges, whole and partial
                                    (16, 8192, 33), (7, 18720, 20), (17, 8192, 33), (2, 65535, 9), (17, 7710, 20), (16, 8193, 20),
                                    (520, 4096, 48), (419, 5011, 20),
+                                   # 256 blocks, the most that exchange them, and 257, which get them from slices
+                                   (256, 8192, 20), (255, 8225, 20), (257, 8192, 20), (256, 8193, 20),
                                    (2, 131007, 3), (2, 131008, 3), (2, 131071, 3)])  # the longest rows
 @pytest.mark.parametrize("kind", ["normal", "constant", "nan"])
 def test_dynamic_linear_of_any_size(M, K, N, kind):

@@ -379,7 +379,7 @@ def test_quantize_rows_dynamic_equals_the_three_calls_and_the_oracle(rows, cols,
 
 
 @pytest.mark.parametrize("n", [0, 1, 3, 4, 1000, 64 * 784, 262144, 50177,
-                               122881, 131071, 131072, 131073])  # 16 blocks of 8192 in one launch, 17 in two
+                               122881, 131071, 131072, 131073])  # 16 blocks of 8192, and 17
 @pytest.mark.parametrize("qd", ["quint8", "qint8"])
 def test_quantize_tensor_dynamic_equals_the_three_calls(n, qd):
     """Global min / max, qparams and codes of a small tensor in one launch: the bits of
