@@ -257,7 +257,7 @@ int launch_gemv1(const float* x, const uint32_t* packed, const float* scales, co
 //
 // y[m, n] = sum over groups g of  s[n, g] * (sum_{k in g} c[n, k] x[m, k])  +  b[n, g] * (sum_{k in g} x[m, k]):
 // the inner sums run on v_mfma_f32_16x16x32_bf16 with the codes themselves as one operand -
-// a code c enters exactly as c - 2^(bits-1) (wq_codes), which goes into the bias term - and x as the
+// a code c enters exactly as c - 2^(bits-1), or 128 + c (wq_codes), which goes into the bias term - and x as the
 // other, split into three bfloat16 parts x = hi + mid + lo (exact: 8 + 8 + 8 significant
 // bits, wq_split3x2), one MFMA each.  Products are exact and accumulate in float32, so nothing of x or
 // of the weight is rounded before the sums.
@@ -278,8 +278,8 @@ int launch_gemv1(const float* x, const uint32_t* packed, const float* scales, co
 // holds the k of quarter i.  Which k a slot of an instruction ends up with does not matter
 // as long as x follows: the block writes the three parts of its x range into LDS in exactly
 // that order.  The threads that split x also add it up per group segment, in float32
-// pair by pair, and leave the sums in LDS (as one more accumulator tile against a row of ones they took a third of the
-// matrix instructions).
+// pair by pair, and leave the sums in LDS (as one more accumulator tile against a row of ones, which the calls with 128 + c
+// keep, they take a third of the matrix instructions).
 //
 // Every block needs the x of its k range next to its weights (64 bytes of x per k against
 // rows / 2 or rows bytes of codes), and every block converts it again.  So a block takes
@@ -317,7 +317,7 @@ __device__ __forceinline__ float wq_neighbour_sum(float v) {
     return v;
 }
 
-template <int BITS, int SW, int RB>
+template <int BITS, int SW, int RB, bool PATTERN>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4 : 2, RB <= 2 ? 4 : 2))) void wq_mfma_kernel(
     const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N, int K,
     int gs_shift, float* out, float* slabs, int* counters) {
@@ -451,8 +451,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
             const float v[8] = {raw[u][0].x, raw[u][0].y, raw[u][0].z, raw[u][0].w,
                                 raw[u][1].x, raw[u][1].y, raw[u][1].z, raw[u][1].w};
             // a wavefront has one row of x: the segments' sums, in float32, pair by pair
-            const float sum = wq_neighbour_sum<SEG / 8>(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
-            if (lane % (SEG / 8) == 0) sum_lds[kl / SEG * 16 + ml] = sum;
+            if constexpr (!PATTERN) {
+                const float sum = wq_neighbour_sum<SEG / 8>(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+                if (lane % (SEG / 8) == 0) sum_lds[kl / SEG * 16 + ml] = sum;
+            }
             uint32_t d3[3][4];
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
@@ -488,15 +490,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
 #pragma unroll
         for (int e = 0; e < GW; ++e) {
             const int g = (((w0 + wi) * WK + e * SEG) >> gs_shift) - g0;
-            v4f acc[RB];
+            // (PATTERN: acc[RB] is the segment's sum of x, from the same fragments against ones: what of its rounding the
+            // codes' sums share, the bias takes out again)
+            constexpr int ACC = PATTERN ? RB + 1 : RB;
+            const uint4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // eight times 1.0
+            v4f acc[ACC];
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb) acc[rb] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int rb = 0; rb < ACC; ++rb) acc[rb] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ii = 0; ii < IPS; ++ii) {
                 const int i = e * IPS + ii;
                 uint4 cf[RB];
 #pragma unroll
-                for (int rb = 0; rb < RB; ++rb) cf[rb] = wq_codes<BITS>(wd[rb], i);
+                for (int rb = 0; rb < RB; ++rb) cf[rb] = wq_codes<BITS, PATTERN>(wd[rb], i);
 #pragma unroll
                 for (int p = 0; p < 3; ++p) {
                     const v8bf xf = __builtin_bit_cast(v8bf, x_lds[((wi * NI + i) * 3 + p) * 64 + wq_x_slot(lane & 15, lane >> 4, wi * NI + i)]);
@@ -504,18 +510,25 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
                     for (int rb = 0; rb < RB; ++rb)
                         acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, __builtin_bit_cast(v8bf, cf[rb]),
                                                                           acc[rb], 0, 0, 0);
+                    if constexpr (PATTERN)
+                        acc[RB] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, __builtin_bit_cast(v8bf, ones), acc[RB], 0, 0, 0);
                 }
             }
-            const v4f sums = *reinterpret_cast<const v4f*>(sum_lds + (wi * GW + e) * 16 + 4 * q);  // of the lane's rows m
+            // the sums of the lane's rows m
+            const v4f sums = PATTERN ? acc[ACC - 1] : *reinterpret_cast<const v4f*>(sum_lds + (wi * GW + e) * 16 + 4 * q);
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
                 const float sc = s_lds[(row_in_tile + rb * 16) * gp + g];
                 const float bi = b_lds[(row_in_tile + rb * 16) * gp + g];
-                // the codes entered as (c + centre) / unit
-                const float bz = bi - float(kWqCentre<BITS>) * sc;
+                if constexpr (PATTERN) {
+                    y[rb] = y[rb] + (acc[rb] * sc + sums * (bi - 128.0f * sc));
+                } else {
+                    // the codes entered as (c + centre) / unit
+                    const float bz = bi - float(kWqCentre<BITS>) * sc;
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    y[rb][t] = __builtin_fmaf(acc[rb][t], kWqUnit<BITS> * sc, __builtin_fmaf(sums[t], bz, y[rb][t]));
+                    for (int t = 0; t < 4; ++t)
+                        y[rb][t] = __builtin_fmaf(acc[rb][t], kWqUnit<BITS> * sc, __builtin_fmaf(sums[t], bz, y[rb][t]));
+                }
             }
         }
     };
@@ -614,7 +627,7 @@ int wq_tiles_per_wave(int M, int N, int slices, int sw) {
     return best;
 }
 
-template <int BITS, int SW, int RB>
+template <int BITS, int SW, int RB, bool PATTERN>
 int launch_wq_mfma_form(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
                         int K, int gs, float* out, hipStream_t st) {
     using G = WqGeom<BITS>;
@@ -622,7 +635,7 @@ int launch_wq_mfma_form(const float* x, const uint32_t* packed, const float* sca
     const int mblocks = (M + 15) / 16, windows = (K + G::WK - 1) / G::WK;
     const int tiles = (N + wq_rows(RB) - 1) / wq_rows(RB), slices = (windows + WPS - 1) / WPS;
     static DeviceOnce attr_once;
-    if (const int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SW, RB>),
+    if (const int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SW, RB, PATTERN>),
                                          int(wq_lds_bytes(RB, 32))))
         return rc;
     SkScratch sk;
@@ -631,7 +644,7 @@ int launch_wq_mfma_form(const float* x, const uint32_t* packed, const float* sca
         const int rc = sk_scratch(size_t(mblocks) * tiles, size_t(mblocks) * tiles * slices * (kWqWaves * RB * 64 * 16), st, &sk);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL((wq_mfma_kernel<BITS, SW, RB>), dim3(unsigned(slices), unsigned(tiles), unsigned(mblocks)), dim3(512),
+    hipLaunchKernelGGL((wq_mfma_kernel<BITS, SW, RB, PATTERN>), dim3(unsigned(slices), unsigned(tiles), unsigned(mblocks)), dim3(512),
                        wq_lds_bytes(RB, gs), st, x, packed, scales, biases, M, N, K, 31 - __builtin_clz(unsigned(gs)), out,
                        reinterpret_cast<float*>(sk.slabs), sk.counters);
     LQ_CHECK_LAUNCH("wq_mfma");
@@ -642,8 +655,11 @@ template <int BITS>
 int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
                    int K, int gs, float* out, hipStream_t st) {
     const int sw = wq_swap_mode(BITS, gs), rb = wq_tiles_per_wave(M, N, (K + kWqSliceK - 1) / kWqSliceK, sw);
-#define LQ_WQ_FORM(SWM, RBS) \
-    if (sw == SWM && rb == RBS) return launch_wq_mfma_form<BITS, SWM, RBS>(x, packed, scales, biases, M, N, K, gs, out, st)
+    const bool pattern = BITS == 4 && M > 1 && M <= 64 && K % WqGeom<BITS>::WK == 0;
+#define LQ_WQ_FORM(SWM, RBS)                                                                                       \
+    if (sw == SWM && rb == RBS)                                                                                    \
+        return pattern ? launch_wq_mfma_form<BITS, SWM, RBS, BITS == 4>(x, packed, scales, biases, M, N, K, gs, out, st) \
+                       : launch_wq_mfma_form<BITS, SWM, RBS, false>(x, packed, scales, biases, M, N, K, gs, out, st)
 #define LQ_WQ_FORMS(SWM) LQ_WQ_FORM(SWM, 1); LQ_WQ_FORM(SWM, 2); LQ_WQ_FORM(SWM, 3)
     LQ_WQ_FORMS(0);
     LQ_WQ_FORMS(1);

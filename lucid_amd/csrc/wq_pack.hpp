@@ -54,20 +54,31 @@ __device__ __forceinline__ void wq_exchange(uint32_t (&wd)[4]) {
 // are codes 2d and 2d + 1.  A code c enters as (c + centre) / unit, and the centre is taken out again with the bias: with
 // centre = -2^(bits-1) the sums stay as small as the products are.  4 bits: with the top bit flipped a nibble is
 // the signed code, and v_cvt_off_f32_i4 gives a sixteenth of that as a float whose upper half is the bfloat16.  8 bits: the
-// signed byte as a float, likewise.  (4 bits as the pattern 0x4300 | c = 128 + c take 8 instructions in place of 14, but the
-// sums then grow with the mean of x and are cancelled by the bias afterwards: against float64, K = 4096, groups of 128,
-// relative, x normal / after a ReLU: 8e-6 / 4e-5, 8 bits uncentred 4e-7 / 1.4e-6; centred 1.5e-7 / 3e-7, and 1e-6 when the
-// weight is decoded first.)
+// signed byte as a float, likewise.
+// PATTERN (4 bits): c as the bit pattern 0x4300 | c = 128 + c, which needs no conversion (8 instructions in place of 14): the
+// calls that have always had it, 2 .. 64 rows of whole windows, keep their bits.  Its sums grow with the mean of x and are
+// cancelled by the bias afterwards: against float64, K = 4096, groups of 128, relative, x normal / after a ReLU: 8e-6 / 4e-5,
+// 8 bits uncentred 4e-7 / 1.4e-6; centred 1.5e-7 / 3e-7, and 1e-6 when the weight is decoded first.
 template <int BITS>
 constexpr int kWqCentre = -(1 << (BITS - 1));
-template <int BITS>
-constexpr float kWqUnit = BITS == 4 ? 16.0f : 1.0f;
+template <int BITS, bool PATTERN = false>
+constexpr float kWqUnit = BITS == 4 && !PATTERN ? 16.0f : 1.0f;
 
-template <int BITS>
+template <int BITS, bool PATTERN = false>
 __device__ __forceinline__ uint4 wq_codes(const uint32_t (&wd)[4], int i) {
+    static_assert(!PATTERN || BITS == 4, "");
     auto upper = [](float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); };
     uint4 f;
-    if constexpr (BITS == 4) {
+    if constexpr (PATTERN) {
+        const uint32_t c = wd[i];
+        uint32_t mask = 0x000f000fu, one = 0x43004300u;
+        asm("" : "+s"(mask));  // in registers: an AND-OR takes one literal at most
+        asm("" : "+v"(one));
+        f.x = (c & mask) | one;
+        f.y = ((c >> 4) & mask) | one;
+        f.z = ((c >> 8) & mask) | one;
+        f.w = ((c >> 12) & mask) | one;
+    } else if constexpr (BITS == 4) {
         const uint32_t even = wd[i] ^ 0x88888888u, odd = even >> 4;
         auto at = [](uint32_t w, int byte) { return __builtin_amdgcn_cvt_off_f32_i4(int((w >> (8 * byte)) & 0xffu)); };
         f.x = upper(at(even, 0), at(even, 2));
