@@ -100,6 +100,14 @@ inline int allow_dynamic_lds(DeviceOnce& o, const void* fn, int bytes) {
 
 inline hipStream_t as_stream(lq_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
+// The barrier of a block for what is in LDS.  __syncthreads waits for every memory operation of the wavefront first: loads that
+// were requested early, to arrive under the work on both sides of the barrier, would have to arrive before it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 __host__ __device__ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // erf for the GELU kernels: Abramowitz & Stegun 7.1.26, |error| <= 1.5e-7 (the rational

@@ -222,12 +222,6 @@ __device__ __forceinline__ unsigned missing_words(const v4u (&raw)[KP][2]) {
     }
     return missing;
 }
-// the barrier of the block for what is in LDS: loads and stores of memory stay in flight
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 // eight columns as three operands, whose sum they are
 __device__ __forceinline__ void split_columns(v4u (&parts)[3], const v4u (&raw)[2]) {
 #pragma unroll

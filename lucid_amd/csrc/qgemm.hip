@@ -634,7 +634,7 @@ __global__ __launch_bounds__(512) void qgemv1_kernel(GemmArgs g) {
                 wv[r][i] = (n < g.N && k < g.K) ? load16(row + chunk_at(k, g.K)) : v4i{0, 0, 0, 0};
             }
         }
-        if (kc == 0) __syncthreads();  // the activation row is in LDS (uniform: every wave runs chunk 0)
+        if (kc == 0) lds_barrier();  // the activation row is in LDS (uniform: every wave runs chunk 0)
         v4i av[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) av[i] = *reinterpret_cast<const v4i*>(a_lds + kc * 4096 + i * 1024 + lane * 16);
@@ -693,7 +693,7 @@ __global__ __launch_bounds__(1024) void qgemm_skinny16_kernel(GemmArgs g, int ro
         cp = load_col(g, n_mine);
         as_uniform = g.a_scale ? g.a_scale[0] : 1.0f;
     }
-    __syncthreads();  // the accumulators are zero before anyone adds to them
+    lds_barrier();  // the accumulators are zero before anyone adds to them (what was requested is still on its way)
 
     const int kblocks = (g.K + 255) / 256;
     const bool m_ok = ln < g.M;

@@ -930,7 +930,7 @@ __global__ __launch_bounds__(512) void dynamic_gemv1_kernel(
             if (i < quads) *reinterpret_cast<Code8x4*>(dv_codes + i * 4) = op.pack(v[u], s, z, rcp);
         }
     }
-    __syncthreads();
+    lds_barrier();  // (the weights are still on their way)
     int acc[RW] = {0, 0, 0, 0};
     for (int kc = 0; kc < chunks; ++kc) {
         if (kc) load_chunk(kc);
@@ -1143,7 +1143,7 @@ __global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
         const int i = u * 1024 + tid;
         if (i >= q_lo && i < q_hi) op.q[i - q_lo] = op.pack(v[u], s, z, r);
     }
-    __syncthreads();
+    lds_barrier();  // (the weights are still on their way)
 
     dl_v4i acc = dl_v4i{0, 0, 0, 0};
     for (int ks = wave; ks < ksteps; ks += 16) {
@@ -1258,7 +1258,7 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
             if (i >= q_lo && i < q_hi) op.q[i - q_lo] = op.pack(v[u], s, z, r);
         }
     }
-    __syncthreads();
+    lds_barrier();  // (the weights are still on their way)
     mb_v4i acc = mb_v4i{0, 0, 0, 0};
     for (int ks = wave; ks < ksteps; ks += 16) {
         const int k = ks * 64 + lg * 16;

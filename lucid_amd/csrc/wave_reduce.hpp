@@ -44,7 +44,7 @@ __device__ __forceinline__ void block_minmax(float& lo, float& hi, int& nan) {
     lo = wave_min(lo), hi = wave_max(hi), nan = wave_any(nan);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, waves = (blockDim.x + 63) >> 6;
     if (lane == 0) s_lo[wave] = lo, s_hi[wave] = hi, s_nan[wave] = nan;
-    __syncthreads();
+    lds_barrier();
     const int w = (lane & 15) < waves ? lane & 15 : 0;
     lo = wave_reduce_detail::row<false>(s_lo[w]), hi = wave_reduce_detail::row<true>(s_hi[w]);
     lo = __uint_as_float(unsigned(__builtin_amdgcn_readlane(int(__float_as_uint(lo)), 15)));

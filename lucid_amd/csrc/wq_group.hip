@@ -87,7 +87,7 @@ constexpr int WQ_ROWS = 16;  // output columns per block, four per wavefront
 // contiguous weight per load.  The weight stream is software-pipelined:
 // a wavefront owns four weight rows and walks K in steps of 64 * CODES; the 16-byte code
 // loads (and scale / bias) of all four rows for the next step are in flight while the current
-// step is multiplied, and the first step's loads are issued before x is staged, so the only
+// step is multiplied, and the first step's loads are issued before x is staged (behind the requests of x itself), so the only
 // exposed memory latency is the first one.  K need not fill the last step: its lanes past K read
 // the row's last 16 bytes against zeros of x.
 template <int BITS>
@@ -139,7 +139,16 @@ __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uin
         __builtin_amdgcn_sched_barrier(0);
     };
     Operands o0, o1;
-    fetch(0, o0);
+    // Loads return in the order they were requested: the first 4096 of x, which every block finds in its L2, before the scales
+    // and the weights, so that x is in LDS by the time the first codes arrive.
+    constexpr int kAhead = 4;
+    float4 xv[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+        const int i = (u * 256 + tid) * 4;
+        xv[u] = *reinterpret_cast<const float4*>(x + (i < K ? i : 0));
+    }
+    pin();
     if (sb_lds) {
         const int r = lane >> 4;
         int part = (lane & 15) * 4;
@@ -150,17 +159,25 @@ __global__ __launch_bounds__(256) void wq_gemv1_kernel(const float* x, const uin
         __builtin_amdgcn_global_load_lds((gptr)(brow[r % RW] + part), (lptr)(sb + 256), 16, 0, 0);
     }
     pin();
+    fetch(0, o0);
+    pin();
     // (in LDS the lanes of a wavefront read consecutive 16-byte slots: lane L of a step, quad j of its chunk)
-    for (int i = tid * 4; i < chunks * CODES; i += 256 * 4) {
-        float4 v{0.f, 0.f, 0.f, 0.f};
-        if (i < K) v = *reinterpret_cast<const float4*>(x + i);
+    auto stage = [&](int i, float4 v) {
         const int L = i / CODES, j = (i % CODES) / 4;
         *reinterpret_cast<float4*>(sx + (j * chunks + L) * 4) = v;
+    };
+    const float4 zero{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+        const int i = (u * 256 + tid) * 4;
+        if (i < chunks * CODES) stage(i, i < K ? xv[u] : zero);
     }
-    // the activation loads above are younger than the direct loads: once they have been consumed (they
-    // were, by the LDS stores), the scales and biases have landed as well
-    __builtin_amdgcn_s_waitcnt(0x0070 | (0xF << 8));  // vmcnt(0)
-    __syncthreads();
+    for (int i = (kAhead * 256 + tid) * 4; i < chunks * CODES; i += 256 * 4)
+        stage(i, i < K ? *reinterpret_cast<const float4*>(x + i) : zero);
+    // the direct loads are older than the RW weight loads, which may still be on their way
+    static_assert(RW == 4, "the count below");
+    __builtin_amdgcn_s_waitcnt(0x0074 | (0xF << 8));  // vmcnt(4)
+    lds_barrier();
     float acc[RW];
 #pragma unroll
     for (int r = 0; r < RW; ++r) acc[r] = 0.0f;
@@ -469,7 +486,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
             }
         }
     }
-    __syncthreads();
+    lds_barrier();  // (the weights are still on their way)
 
     v4f y[RB];
 #pragma unroll
