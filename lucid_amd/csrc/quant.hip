@@ -854,8 +854,14 @@ void quantize_tensor_dynamic_kernel(const float* __restrict__ x, size_t n, unsig
 // the way - they are requested before the range is known -, so the layer costs what lq_qlinear_i8 of one row
 // does (qgemv1_kernel: four weight rows per wavefront, a KiB of a row per load, v_dot4) plus the two block
 // reductions.  4096 -> 11008: 24.2 us with the 16 x 16-tile kernel above (688 blocks of 1024 threads, each
-// waiting for its range before its one weight fragment per wavefront), now 10.2 us (4.4 TB/s of weight).
+// waiting for its range before its one weight fragment per wavefront), 11.5 when the weights had to arrive before the row's
+// reductions could end (a barrier that waits for all loads, branches behind which the compiler does), now 10.4 with its
+// launch (4.3 TB/s of weight).
 // w rows are `ld` bytes apart, zeros past K; K <= 16384, ld % 16 == 0.
+// ONE_ROUND: the block's registers hold the row (4 <= K <= 16 per thread).  Then nothing between the requests of the weights and
+// their use branches or loops, so that what waits for the row waits for the row alone: loads past the row and the weight
+// repeat their last ones (a range does not mind, and codes past K are zeros in LDS).
+template <bool ONE_ROUND>
 __global__ __launch_bounds__(512) void dynamic_gemv1_kernel(
     const float* __restrict__ x, int K, const int8_t* __restrict__ w, int ld, int N, const float* __restrict__ w_scale,
     const int32_t* __restrict__ wsum, const float* __restrict__ bias, int relu, int symmetric, int qmin, int qmax,
@@ -869,6 +875,13 @@ __global__ __launch_bounds__(512) void dynamic_gemv1_kernel(
     const int quads = (K + 3) / 4, rounds = (quads + threads * kKeep - 1) / (threads * kKeep);
     float4 v[kKeep];
     MinMax m{__builtin_inff(), -__builtin_inff(), 0};
+    if constexpr (ONE_ROUND) {
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) {
+            const int e = (u * threads + tid) * 4;
+            __builtin_memcpy(&v[u], x + (e < K - 4 ? e : K - 4), 16);
+        }
+    } else
     for (int rd = 0; rd < rounds; ++rd) {
 #pragma unroll
         for (int u = 0; u < kKeep; ++u) v[u] = load_quad(x, size_t((rd * kKeep + u) * threads + tid) * 4, K);
@@ -890,18 +903,25 @@ __global__ __launch_bounds__(512) void dynamic_gemv1_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int k = kc * 4096 + i * 1024 + lane * 16;
-                wv[r][i] = k < ld ? *reinterpret_cast<const dv_v4i*>(w + size_t(n) * ld + k) : dv_v4i{0, 0, 0, 0};
+                if constexpr (ONE_ROUND)
+                    wv[r][i] = *reinterpret_cast<const dv_v4i*>(w + size_t(n) * ld + (k < ld ? k : 0));
+                else
+                    wv[r][i] = k < ld ? *reinterpret_cast<const dv_v4i*>(w + size_t(n) * ld + k) : dv_v4i{0, 0, 0, 0};
             }
         }
     };
-    load_chunk(0);
     const int n_mine = nb + (lane < RW ? lane : 0);
     const bool mine = lane < RW && n_mine < N;
     const float c_ws = mine && w_scale ? w_scale[n_mine] : 1.0f;
     const int c_wsum = mine && wsum ? wsum[n_mine] : 0;
     const float c_bias = mine && bias ? bias[n_mine] : -0.0f;
     __builtin_amdgcn_sched_barrier(0);
-    if (rounds == 1) {
+    load_chunk(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ONE_ROUND) {
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) mm_update(m, v[u]);
+    } else if (rounds == 1) {
 #pragma unroll
         for (int u = 0; u < kKeep; ++u) {
             const int e = (u * threads + tid) * 4;
@@ -916,6 +936,18 @@ __global__ __launch_bounds__(512) void dynamic_gemv1_kernel(
     qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
     const float rcp = 1.0f / s;
     const QuantizeOp<int8_t> op{nullptr, nullptr, float(double(qmin)), float(double(qmax)), off};
+    if constexpr (ONE_ROUND) {
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) {
+            const int i = u * threads + tid, past = i * 4 - (K - 4);  // elements of the quad that lie in the one before
+            const Code8x4 c = op.pack(v[u], s, z, rcp);
+            unsigned word;
+            __builtin_memcpy(&word, &c, 4);
+            word = past <= 0 ? word : past < 4 ? word >> (8 * past) : 0u;
+            if (i < chunks * 1024) *reinterpret_cast<unsigned*>(dv_codes + i * 4) = word;
+        }
+        for (int i = kKeep * threads + tid; i < chunks * 1024; i += threads) *reinterpret_cast<unsigned*>(dv_codes + i * 4) = 0u;
+    } else
     for (int rd = rounds - 1; rd >= 0; --rd) {
         if (rd != rounds - 1) {
 #pragma unroll
@@ -1498,7 +1530,8 @@ int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw
     if (M == 1 && K > 0 && K <= 16384) {
         // every block quantizes the whole row: eight wavefronts, or four where that leaves CUs without a block
         const int waves = (N + 31) / 32 < 256 ? 4 : 8;
-        hipLaunchKernelGGL(dynamic_gemv1_kernel, dim3(unsigned((N + 4 * waves - 1) / (4 * waves))), dim3(waves * 64),
+        const auto kernel = K >= 4 && K <= waves * 64 * 16 ? dynamic_gemv1_kernel<true> : dynamic_gemv1_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3(unsigned((N + 4 * waves - 1) / (4 * waves))), dim3(waves * 64),
                            size_t((K + 4095) / 4096) * 4096, st, x, K, w, ldw, N, w_scale, wsum, bias, relu, symmetric, qmin,
                            qmax, is_signed, eps, half_range, code_offset, out);
         LQ_CHECK_LAUNCH("dynamic_gemv1");

@@ -536,6 +536,8 @@ def test_dynamic_linear_wide_layer_at_small_batch(M, K):
                                    # 16 and 17 blocks of 8192 codes, which exchange their ranges, whole and partial
                                    (16, 8192, 33), (7, 18720, 20), (17, 8192, 33), (2, 65535, 9), (17, 7710, 20), (16, 8193, 20),
                                    (520, 4096, 48), (419, 5011, 20),
+                                   (1, 3, 9), (1, 4, 9), (1, 5, 40), (1, 1030, 8200), (1, 4096, 50), (1, 4099, 50), (1, 8191, 8193),
+                                   (1, 8192, 8200), (1, 8193, 8200),  # one row, in a block's registers or not
                                    # 256 blocks, the most that exchange them, and 257, which get them from slices
                                    (256, 8192, 20), (255, 8225, 20), (257, 8192, 20), (256, 8193, 20),
                                    (2, 131007, 3), (2, 131008, 3), (2, 131071, 3)])  # the longest rows
