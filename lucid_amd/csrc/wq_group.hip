@@ -380,27 +380,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     constexpr int kTabVec = kWqRows * 16 / 4 / 512;  // 16-byte loads per thread and table, at 16 groups per k range
     const int gcap = gp - 1, gsh = 31 - __builtin_clz(unsigned(gcap));  // a power of two: shifts, no division
     const bool tab_vec = ng == gcap && (groups_per_row & 3) == 0 && aligned16(scales) && aligned16(biases);
+    // (No branch between these requests and none that gives a register another value: the compiler would wait for each load
+    // where the two meet - a memory trip per table and row of x before the first weight was asked for.)
     float4 tab_s[kTabVec], tab_b[kTabVec];
-    {
-        const int row_first = tile * kWqRows;
+    const int row_first = tile * kWqRows;
+    auto table_at = [&](int i) {
+        const int n = row_first + (i >> gsh) < N ? row_first + (i >> gsh) : N - 1;
+        return size_t(n) * groups_per_row + g0 + (i & (gcap - 1));
+    };
+    if (tab_vec) {
 #pragma unroll
         for (int u = 0; u < kTabVec; ++u) {
-            const int i = (threadIdx.x + u * 512) * 4, row = i >> gsh, g = i & (gcap - 1);
-            tab_s[u] = tab_b[u] = float4{0.f, 0.f, 0.f, 0.f};
-            if (i < kWqRows * gcap) {
-                const int n = row_first + row < N ? row_first + row : N - 1;
-                const size_t at = size_t(n) * groups_per_row + g0 + g;
-                if (tab_vec) {
-                    tab_s[u] = *reinterpret_cast<const float4*>(scales + at);
-                    tab_b[u] = *reinterpret_cast<const float4*>(biases + at);
-                } else {
-                    // ragged: the last k range of a K that is not a multiple of 512, or unaligned rows
-                    if (g < ng) tab_s[u].x = scales[at], tab_b[u].x = biases[at];
-                    if (g + 1 < ng) tab_s[u].y = scales[at + 1], tab_b[u].y = biases[at + 1];
-                    if (g + 2 < ng) tab_s[u].z = scales[at + 2], tab_b[u].z = biases[at + 2];
-                    if (g + 3 < ng) tab_s[u].w = scales[at + 3], tab_b[u].w = biases[at + 3];
-                }
-            }
+            const int i = (threadIdx.x + u * 512) * 4;
+            const size_t at = table_at(i < kWqRows * gcap ? i : 0);
+            tab_s[u] = *reinterpret_cast<const float4*>(scales + at);
+            tab_b[u] = *reinterpret_cast<const float4*>(biases + at);
         }
     }
     // x of the block's windows: a thread takes eight consecutive k of one row (a wavefront reads
@@ -411,12 +405,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
 #pragma unroll
     for (int u = 0; u < UNITS / 512; ++u) {
         const int unit = u * 512 + threadIdx.x, m = m0 + unit / OCTS, kl = (unit % OCTS) * 8;
-        raw[u][0] = raw[u][1] = float4{0.f, 0.f, 0.f, 0.f};
-        if (m < M && w0 * WK + kl < k_end) {
-            const float* src = x + size_t(m) * K + w0 * WK + kl;
-            raw[u][0] = *reinterpret_cast<const float4*>(src);
-            raw[u][1] = *reinterpret_cast<const float4*>(src + 4);
-        }
+        // (K is a multiple of 32; what lies past M and K becomes zero below)
+        const float* src = x + size_t(m < M ? m : M - 1) * K + (w0 * WK + kl < k_end ? w0 * WK + kl : 0);
+        raw[u][0] = *reinterpret_cast<const float4*>(src);
+        raw[u][1] = *reinterpret_cast<const float4*>(src + 4);
     }
     // The weights of the first windows are requested now (of all of them where a wavefront has one tile; more tiles keep
     // enough bytes in flight with two, in a loop of a third of the code).  For the request a lane takes quarter lane % 4 of row lane / 4 - four neighbouring lanes read 64
@@ -447,14 +439,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     float* sum_lds = reinterpret_cast<float*>(wq_lds + WPS * NI * 3 * 64);  // of x: [segment][row]
     float* s_lds = sum_lds + kWqSliceK / 32 * 16;
     float* b_lds = s_lds + kWqRows * gp;
+    if (tab_vec) {
 #pragma unroll
-    for (int u = 0; u < kTabVec; ++u) {
-        const int i = (threadIdx.x + u * 512) * 4, row = i >> gsh, g = i & (gcap - 1);
-        if (i < kWqRows * gcap) {  // (slots past ng hold zeros and are never read)
-            float* sd = s_lds + row * gp + g;
-            float* bd = b_lds + row * gp + g;
-            sd[0] = tab_s[u].x, sd[1] = tab_s[u].y, sd[2] = tab_s[u].z, sd[3] = tab_s[u].w;
-            bd[0] = tab_b[u].x, bd[1] = tab_b[u].y, bd[2] = tab_b[u].z, bd[3] = tab_b[u].w;
+        for (int u = 0; u < kTabVec; ++u) {
+            const int i = (threadIdx.x + u * 512) * 4, row = i >> gsh, g = i & (gcap - 1);
+            if (i < kWqRows * gcap) {
+                float* sd = s_lds + row * gp + g;
+                float* bd = b_lds + row * gp + g;
+                sd[0] = tab_s[u].x, sd[1] = tab_s[u].y, sd[2] = tab_s[u].z, sd[3] = tab_s[u].w;
+                bd[0] = tab_b[u].x, bd[1] = tab_b[u].y, bd[2] = tab_b[u].z, bd[3] = tab_b[u].w;
+            }
+        }
+    } else {  // the last k range of a K that is not a multiple of 512, or rows that vectors cannot take
+        for (int i = threadIdx.x; i < kWqRows * gcap; i += 512) {
+            const int row = i >> gsh, g = i & (gcap - 1);
+            // (zeros past the row's groups: a partial window's segments past K read them)
+            s_lds[row * gp + g] = g < ng ? scales[table_at(i)] : 0.0f;
+            b_lds[row * gp + g] = g < ng ? biases[table_at(i)] : 0.0f;
         }
     }
     {
@@ -465,8 +466,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
             int qd, rho;
             wq_source(SW, js, qs, qd, rho);
             const int i = BITS == 4 ? rho : rho / 2;
-            const float v[8] = {raw[u][0].x, raw[u][0].y, raw[u][0].z, raw[u][0].w,
-                                raw[u][1].x, raw[u][1].y, raw[u][1].z, raw[u][1].w};
+            float v[8] = {raw[u][0].x, raw[u][0].y, raw[u][0].z, raw[u][0].w,
+                          raw[u][1].x, raw[u][1].y, raw[u][1].z, raw[u][1].w};
+            const bool there = m0 + ml < M && w0 * WK + kl < k_end;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = there ? v[e] : 0.0f;
             // a wavefront has one row of x: the segments' sums, in float32, pair by pair
             if constexpr (!PATTERN) {
                 const float sum = wq_neighbour_sum<SEG / 8>(((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));

@@ -80,7 +80,7 @@ def test_small_batch_matmul_is_reproducible_and_exact_on_exact_inputs(bits):
 # end inside a tile and inside a block, batches that end inside sixteen, a last window and a last k range that are partial
 @pytest.mark.parametrize("M,N,K,gs,bits", [(2, 127, 544, 32, 4), (17, 129, 1088, 64, 8), (16, 4097, 4096, 128, 4),
                                            (31, 8191, 2112, 64, 8), (7, 11007, 4096, 64, 8), (16, 10999, 4224, 128, 4),
-                                           (13, 7000, 6176, 32, 4), (64, 4100, 4096, 32, 8)])
+                                           (13, 7000, 6176, 32, 4), (64, 4100, 4096, 32, 8), (24, 8000, 992, 32, 4)])
 def test_small_batch_forms_against_float64(M, N, K, gs, bits):
     rng = np.random.default_rng(N)
     w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
