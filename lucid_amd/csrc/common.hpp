@@ -47,9 +47,9 @@ int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream,
 // kind 0: the general workspace (at least 4 MiB); 1 / 2: stream-K counters / slabs;
 // 3: raw accumulators and operand sums of a layer with affine weights; 4: padded copies of ragged GEMM operands;
 // 5: the range slots of a dynamic quantization; 6: the codes and qparams of a dynamic Linear's activation;
-// 7: the slots of a dynamic quantization in one launch
+// 7: the slots of a dynamic quantization in one launch; 8: the rings of an LSTM recurrence
 int workspace(size_t nbytes, hipStream_t stream, void** ptr);
-// Scratch (kinds 4 to 6) of one call's launches.  While this thread records a graph it is memory of that graph's own:
+// Scratch (kinds 4 to 6 and 8) of one call's launches.  While this thread records a graph it is memory of that graph's own:
 // replays may run on any stream, beside each other and beside the stream's eager calls.
 int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr);
 // Held by every user of a stream's scratch from before it asks for the buffer until its last launch on it is issued:

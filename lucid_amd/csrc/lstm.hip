@@ -572,7 +572,8 @@ constexpr int kMaxHidden = 1024;
 // (lq_lstm_cell_f32) on decoded weights, issued from Python.  Measured, us per step of both: hidden 64, 8192 rows 25.7 /
 // 32.9; 128, 4096 rows 25.6 / 35.4, 8192 rows 46.9 / 47.2; 256, 1024 rows 29.6 / 37.4, 2048 rows 57.9 / 43.1; 512, 512
 // rows 37 / 49, 1024 rows 73 / 56; 768, 128 rows 41 / 58, 256 rows 80 / 60; 1024, 128 rows 46 / 71, 256 rows 89 / 73,
-// 4096 rows 1399 / 289; 1024 in two directions, 16 rows 15 / 130, 256 rows 180 / 146.  The estimates are within 20 %.
+// 4096 rows 1399 / 289; 1024 in two directions, 16 rows 15 / 130, 256 rows 180 / 146.  The estimates are within 20 % of those; steps have become
+// 1.1 to 1.6 times as fast since, so that what is left to the GEMM on the line is within as much of the better one.
 double sequence_step_us(int hidden) { return 2.9 + 0.0026 * hidden; }
 double gemm_step_us(int batch, int hidden) {
     const double least = 17.0 + 0.05 * hidden, rows = batch * (2.8e-5 * hidden + 3.8e-8 * hidden * hidden);
@@ -606,7 +607,8 @@ int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layer
     *fused = 0;
     if (steps == 0 || batch == 0 || hidden > kMaxFused || inputs > kMaxFused) return LQ_OK;
     // Costs per layer in steps of the recurrence.  An input product in a GEMM of its own, with the decoded
-    // weight it reads, is worth twelve (43 us at 1024 x 2048 x 512, a step 3.4).
+    // weight it reads, is worth twelve (43 us at 1024 x 2048 x 512, a step 3.4 then; 20 x 33 rows of 200 -> 300 in two
+    // directions, where a step is 2: 61 us with the GEMMs, about 120 as three launches without).
     constexpr long kGemm = 12;
     LstmSplit s;
     int rc = with_form(hidden, 0, [&](auto w, auto k, auto xw, auto x) { return split_lstm<w(), k(), xw(), x()>(batch, hidden, directions, false, &s); });
