@@ -41,7 +41,7 @@
 //
 // hidden 512, 16 rows, a step of 2.2 us (5100 cycles, timestamps): 450 before the first read, 1850 for the 32 KiB of h a
 // CU reads past its L2 (1000 at hidden 128), 1390 splits and products, 70 barrier, 1000 sums and gates.  Two such layers of
-// 64 steps take 168 us; 272 when h was read from y's rows (every line twice), the input loads stood between h and its
+// 64 steps take 170 us; 272 when h was read from y's rows (every line twice), the input loads stood between h and its
 // products, and one set of wavefronts took both products.  Placing a group's blocks on one XCD and exchanging through its L2 instead
 // measured 150 against 153 us for one layer: not worth the placement.
 #include <cmath>
@@ -232,21 +232,29 @@ __device__ __forceinline__ void split_columns(v4u (&parts)[3], const v4u (&raw)[
         parts[0][e] = hh, parts[1][e] = mm, parts[2][e] = ll;
     }
 }
-// acc[g] += columns . codes of gate g: three exact part products each.  The splits of an instruction's columns come
+// acc[g] += columns . codes of gate g: three exact part products each, the smaller ones added up among themselves first
+// (against float64, outputs of eight sizes: 0.9 to 1.3e-7, 1.1 to 1.7e-7 as one chain in two halves; 2 % of a step).  The splits of an instruction's columns come
 // before the products of the one before, which they do not wait for.
 template <int KP>
 __device__ __forceinline__ void multiply(v4f (&acc)[4], const v4u (&raw)[KP][2], const v8bf (&wf)[4][KP]) {
     v4u parts[2][3];
+    v4f low[4];  // of the two smaller parts: their sums are rounded at their own size
+#pragma unroll
+    for (int g = 0; g < 4; ++g) low[g] = v4f{0.f, 0.f, 0.f, 0.f};
     split_columns(parts[0], raw[0]);
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
         if (i + 1 < KP) split_columns(parts[(i + 1) & 1], raw[i + 1]);
 #pragma unroll
-        for (int q = 0; q < 3; ++q)
+        for (int q = 2; q >= 0; --q)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, parts[i & 1][q]), wf[g][i], acc[g], 0, 0, 0);
+            for (int g = 0; g < 4; ++g) {
+                v4f& to = q == 0 ? acc[g] : low[g];
+                to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, parts[i & 1][q]), wf[g][i], to, 0, 0, 0);
+            }
     }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g] += low[g];
 }
 
 // W wavefronts for h, each with KPW instructions of 32 hidden columns (hidden <= 32 W KPW), and XW for the
