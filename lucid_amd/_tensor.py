@@ -108,7 +108,8 @@ class Grid:
 
 
 class DeviceBuffer:
-    """Owns one ``lq_alloc`` allocation; freed when the last reference dies.
+    """Owns one ``lq_alloc`` allocation; freed when the last reference dies.  A copied or pickled buffer
+    holds the bytes in an allocation of its own: an address that two objects own is freed twice.
 
     (Every operator makes at least one: a ``weakref.finalize`` in place of ``__del__`` took 3 of the
     5 us that an empty tensor costs the host.)"""
@@ -130,6 +131,19 @@ class DeviceBuffer:
                 _C.load().lq_free(self.ptr)
         except Exception:  # interpreter shutdown
             pass
+
+    def __reduce__(self):
+        host = (C.c_char * self.nbytes)()
+        if self.nbytes:
+            _C.call("lq_d2h", C.addressof(host), self.ptr, self.nbytes, None)
+        return _buffer_of, (host.raw,)
+
+
+def _buffer_of(data: bytes) -> DeviceBuffer:
+    buf = DeviceBuffer(len(data))
+    if data:
+        _C.call("lq_h2d", buf.ptr, data, len(data), None)
+    return buf
 
 
 class Tensor:
