@@ -451,6 +451,12 @@ int lq_bias_act_f32(float* y, const float* bias, size_t M, int N, int relu, lq_s
 int lq_quantize_tensor_dynamic_i8(const float* x, size_t n, int symmetric, int qmin, int qmax, int is_signed,
                                   float eps, int code_offset, float* scale, float* zp, float* mn_out,
                                   float* mx_out, int8_t* q, lq_stream stream);
+/* The same for rows of `cols` elements that become rows of `ld` codes, zeros past `cols` (ld = cols, or a larger multiple
+ * of 4), of any size, with the bound on a block's wait for the ranges of the others: after `polls` reads (at most 4096,
+ * the bound of the call above) it takes the range of x itself.  The results do not depend on it. */
+int lq_quantize_tensor_dynamic_polls_i8(const float* x, size_t rows, unsigned cols, unsigned ld, int symmetric, int qmin,
+                                        int qmax, int is_signed, float eps, int code_offset, float* scale, float* zp,
+                                        float* mn_out, float* mx_out, int8_t* q, int polls, lq_stream stream);
 
 /* A dynamic-quantized Linear on a small activation in ONE launch: nnqd.Linear.forward
  * (lucid/nn/quantized/dynamic/linear.py:87-99) for x [M, K] float32 with M <= 64,

@@ -694,9 +694,10 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 // Small tensors (up to kExchange blocks) in one launch, x read once: the blocks' ranges meet through a slot per
 // block in device memory - written through, and polled by every block until it is filled - and each block then
 // derives the qparams itself and writes its codes.  The last block to leave empties the slots for the next
-// launch.  All blocks have to be resident (see lstm.hip on what the launcher has to leave free: kExchange
-// blocks of 512 threads and 64 registers are the quarter of the device that one of four hardware queues may have; with more
-// queues it is fewer blocks, exchange_blocks), and a wait is bounded.
+// launch.  That is quick where all blocks are resident, and kExchange of them are the quarter of the device that one of four
+// hardware queues may have (fewer blocks with more queues, exchange_blocks).  Nothing depends on it: kernels of other processes,
+// or a stream that may not use every CU, can keep a block out for any time, so a block that has read a slot kExchangePolls
+// times without finding a range (about 3 ms) takes the range of x itself - the same minimum and maximum -, ends, and makes room.
 //
 // Beyond, and under capture (slots cleared inside a graph are unset until its replay), two launches: slices'
 // ranges (minmax_seg_kernel), then this kernel with PARTS - every block reduces
@@ -710,7 +711,7 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 // 512 x 4096 -> 1024 (256) 32.7 / 30.7.  Before either: one block on one CU for up to 262144 elements (61 us), five launches
 // beyond (1 M elements: 12.3 us).
 constexpr int kDynThreads = 512, kDynQuads = 4, kDynPerBlock = kDynThreads * kDynQuads * 4;
-constexpr int kExchange = 256, kMaxParts = 512;
+constexpr int kExchange = 256, kExchangePolls = 4096, kMaxParts = 512;
 constexpr unsigned long long kSlotEmpty = ~0ull;  // NaNs that no range contains: mm_write's NaN is the canonical one
 struct DynScratch {
     unsigned long long slot[kExchange];    // low word: the block's minimum, high word: its maximum
@@ -754,10 +755,11 @@ template <bool PARTS, bool RAGGED>
 __global__ __launch_bounds__(kDynThreads) __attribute__((amdgpu_waves_per_eu(8)))
 void quantize_tensor_dynamic_kernel(const float* __restrict__ x, size_t n, unsigned cols, unsigned ld, int symmetric,
                                     int qmin, int qmax, int is_signed, float eps, float half_range, int off,
-                                    DynScratch* slots, const float* __restrict__ parts, int n_parts, float* scale,
+                                    DynScratch* slots, int polls, const float* __restrict__ parts, int n_parts, float* scale,
                                     float* zp, float* mn_out, float* mx_out, int8_t* __restrict__ q) {
-    __shared__ int s_last;
+    __shared__ int s_last, s_missing;
     const int tid = threadIdx.x;
+    if (tid == 0) s_missing = 0;  // (the first reduction's barrier is between this and the slots)
     const size_t first = size_t(blockIdx.x) * kDynPerBlock;
     const float qnan = __builtin_nanf("");
     MinMax m{__builtin_inff(), -__builtin_inff(), 0};
@@ -805,14 +807,20 @@ void quantize_tensor_dynamic_kernel(const float* __restrict__ x, size_t n, unsig
         if (tid < int(gridDim.x)) {
             unsigned long long got = kSlotEmpty;
             __builtin_amdgcn_s_sleep(12);
-            for (int spin = 0; got == kSlotEmpty && spin < (1 << 20); ++spin) {
+            for (int spin = 0; got == kSlotEmpty && spin < polls; ++spin) {
                 if (spin) __builtin_amdgcn_s_sleep(4);
                 got = __hip_atomic_load(&slots->slot[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             m.lo = __uint_as_float(unsigned(got)), m.hi = __uint_as_float(unsigned(got >> 32));
             m.nan = (m.lo != m.lo) | (m.hi != m.hi);
+            if (got == kSlotEmpty) s_missing = 1;
         }
         __syncthreads();  // every slot has been read (and the reduction may use its LDS again)
+        if (s_missing) {  // a block that has not started: its elements and all others, read here
+            m = MinMax{__builtin_inff(), -__builtin_inff(), 0};
+            for (size_t e = size_t(tid) * 4; e < n; e += kDynThreads * 4)
+                mm_update_quad(m, place_quad(load_quad(x, e, n), e, n), e, n);
+        }
         if (tid == 0) {
             const unsigned before = __hip_atomic_fetch_add(&slots->left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             s_last = before == gridDim.x - 1;
@@ -1411,8 +1419,8 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     }
 }
 
-// Blocks that may meet through the slots: the share of the device that one hardware queue may have (16, the least, are far
-// below any).
+// Blocks that may meet through the slots: no more than the share of the device that one hardware queue may have (with 32
+// queues that is 32; 16 are far below any).
 int exchange_blocks(int* most) {
     static DeviceOnce once;
     static int capacity[32] = {0};
@@ -1434,7 +1442,8 @@ int exchange_blocks(int* most) {
 
 // Dynamic per-tensor quantization of n = rows * cols elements to rows of ld codes.
 int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int symmetric, int qmin, int qmax, int is_signed,
-                    float eps, int off, float* scale, float* zp, float* mn, float* mx, int8_t* q, hipStream_t st) {
+                    float eps, int off, float* scale, float* zp, float* mn, float* mx, int8_t* q, hipStream_t st,
+                    int polls = kExchangePolls) {
     const float half_range = float((double(qmax) - double(qmin)) / 2.0);
     const bool ragged = ld != cols;
     const size_t codes = ragged ? n / cols * ld : n;
@@ -1470,7 +1479,7 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
     }
     auto launch = [&](auto kernel, const float* ranges, int n_ranges) {
         hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(kDynThreads), 0, st, x, n, cols, ld, symmetric, qmin, qmax,
-                           is_signed, eps, half_range, off, d, ranges, n_ranges, scale, zp, mn, mx, q);
+                           is_signed, eps, half_range, off, d, polls, ranges, n_ranges, scale, zp, mn, mx, q);
     };
     if (exchange) {
         ragged ? launch(quantize_tensor_dynamic_kernel<false, true>, nullptr, 0)
@@ -1511,6 +1520,19 @@ int lq_quantize_tensor_dynamic_i8(const float* x, size_t n, int symmetric, int q
                "use lq_minmax + lq_calc_qparams + lq_quantize", n);
     return quantize_tensor(x, n, unsigned(n ? n : 1), unsigned(n ? n : 1), symmetric, qmin, qmax, is_signed, eps,
                            code_offset, scale, zp, mn_out, mx_out, q, as_stream(stream));
+}
+
+int lq_quantize_tensor_dynamic_polls_i8(const float* x, size_t rows, unsigned cols, unsigned ld, int symmetric, int qmin,
+                                        int qmax, int is_signed, float eps, int code_offset, float* scale, float* zp,
+                                        float* mn_out, float* mx_out, int8_t* q, int polls, lq_stream stream) {
+    LQ_REQUIRE(scale && zp && x && q, LQ_ERR_VALUE, "quantize_tensor_dynamic: NULL pointer");
+    LQ_REQUIRE(rows > 0 && cols > 0 && ld >= cols && (ld == cols || ld % 4 == 0) && rows <= (size_t(1) << 32) / ld,
+               LQ_ERR_SHAPE, "quantize_tensor_dynamic: %zu rows of %u elements and %u codes", rows, cols, ld);
+    LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
+               "quantize_tensor_dynamic: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
+    LQ_REQUIRE(polls >= 0, LQ_ERR_VALUE, "quantize_tensor_dynamic: %d polls", polls);
+    return quantize_tensor(x, rows * cols, cols, ld, symmetric, qmin, qmax, is_signed, eps, code_offset, scale, zp, mn_out,
+                           mx_out, q, as_stream(stream), polls < kExchangePolls ? polls : kExchangePolls);
 }
 
 int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw, int N, const float* w_scale,

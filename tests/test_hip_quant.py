@@ -409,6 +409,34 @@ def test_quantize_tensor_dynamic_equals_the_three_calls(n, qd):
         assert np.array_equal(q.numpy(), exp)
 
 
+@pytest.mark.parametrize("rows,cols,ld", [(1, 8193, 8193), (2, 131072, 131072), (17, 7710, 7712), (409, 1000, 1024),
+                                          (43690, 5, 12), (64, 8192, 8192)])  # 2 .. 64 blocks, whole, partial and ragged
+@pytest.mark.parametrize("polls", [0, 1, 4096])
+@pytest.mark.parametrize("nan", [False, True])
+def test_a_block_that_does_not_wait_for_the_others_ranges_takes_them_itself(rows, cols, ld, polls, nan):
+    """Blocks that meet through slots have no claim on being resident together: what one does that gives up waiting
+    (here at once, or after one read) is the same scale, zero point, range and codes."""
+    from lucid_amd import _C
+    rng = np.random.default_rng(cols)
+    x = (rng.standard_normal((rows, cols)) * 3 + 0.5).astype(np.float32)
+    if nan:
+        x[rows // 2, cols // 3] = np.nan
+    xt = L.tensor(x, device="hip")
+    s, z, mn, mx = [L.Tensor.empty((), L.float32, "hip") for _ in range(4)]
+    for _ in range(3):  # the slots are empty again after each
+        q = L.tensor(np.full((rows, ld), 77, np.int8), device="hip")
+        _C.call("lq_quantize_tensor_dynamic_polls_i8", xt.data_ptr, rows, cols, ld, 0, 0, 255, 0, 1e-8, -128, s.data_ptr,
+                z.data_ptr, mn.data_ptr, mx.data_ptr, q.data_ptr, polls, None)
+        wmn, wmx = Q.minmax(xt)
+        ws, wz = Q.calculate_qparams(wmn, wmx, Q.per_tensor_affine, Q.quint8)
+        wq = L.Tensor.empty((rows, cols), L.int8, "hip")
+        _C.call("lq_quantize", xt.data_ptr, wq.data_ptr, _C.I8, -128, 1, 1, rows * cols, ws.data_ptr, wz.data_ptr, 0, 0, 255,
+                None)
+        for got, want in ((s, ws), (z, wz), (mn, wmn), (mx, wmx)):
+            assert np.array_equal(bits(got.numpy()), bits(want.numpy()))
+        assert np.array_equal(q.numpy()[:, :cols], wq.numpy()) and not q.numpy()[:, cols:].any()
+
+
 def test_quantize_tensor_dynamic_refuses_large_tensors():
     from lucid_amd import _C
     x = L.Tensor.empty((262145,), L.float32, "hip")
