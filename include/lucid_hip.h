@@ -473,7 +473,7 @@ int lq_dynamic_linear_small_f32(const float* x, int M, int K, const int8_t* w, i
 /* nnqd.Linear.forward for any activation: x [M, K] float32, per-tensor qparams from its runtime min / max, w [N]
  * rows of `ldw` bytes (K codes, then zeros: a multiple of 16, 16-byte aligned), wsum [N] their sums.  One row is
  * one launch (a stream of the weight; K at most 16384); otherwise the activation is quantized to rows of `ldw` codes (up to
- * 131072 of them in one launch, beyond and under capture in two) and multiplied, with codes and qparams in the stream's scratch or,
+ * 524288 of them in one launch, beyond and under capture in two) and multiplied, with codes and qparams in the stream's scratch or,
  * while a graph is recorded, in the graph's memory.  (For a few hundred rows and columns lq_dynamic_linear_small_f32 is faster still.)  Same bits whichever runs: lq_minmax, lq_calc_qparams, lq_quantize,
  * lq_qlinear_i8 (mode F32).  Symmetric weights only. */
 int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw, int N, const float* w_scale,

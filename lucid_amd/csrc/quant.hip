@@ -694,8 +694,8 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 // Small tensors (up to kExchange blocks) in one launch, x read once: the blocks' ranges meet through a slot per
 // block in device memory - written through, and polled by every block until it is filled - and each block then
 // derives the qparams itself and writes its codes.  The last block to leave empties the slots for the next
-// launch.  That is quick where all blocks are resident, and kExchange of them are the quarter of the device that one of four
-// hardware queues may have (fewer blocks with more queues, exchange_blocks).  Nothing depends on it: kernels of other processes,
+// launch.  That is quick where all blocks are resident, and kExchange of them are a sixteenth of the device, less than the
+// share of one of the hardware queues that streams have (exchange_blocks).  Nothing depends on it: kernels of other processes,
 // or a stream that may not use every CU, can keep a block out for any time, so a block that has read a slot kExchangePolls
 // times without finding a range (about 3 ms) takes the range of x itself - the same minimum and maximum -, ends, and makes room.
 //
@@ -707,11 +707,11 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 //
 // 8192 elements 3.4 us, 65536 (8 blocks, the exchange) 5.9.  A slot is read first when most of them have been written, and
 // not at once again: 128 blocks of 1 M elements that polled without a pause took 17 us, in two launches 3.8 + 5.0.  A dynamic
-// Linear behind it, in two launches / in one, us: 333 x 1000 -> 1001 16.6 / 13.6, 256 x 4096 -> 1024 (128 blocks) 25.7 / 24.9,
-// 512 x 4096 -> 1024 (256) 32.7 / 30.7.  Before either: one block on one CU for up to 262144 elements (61 us), five launches
-// beyond (1 M elements: 12.3 us).
+// Linear behind it, in two launches / in one, us: 333 x 1000 -> 1001 (42 blocks) 16.6 / 13.6; with 128 blocks it is 25.7 / 24.9,
+// with 256 32.7 / 30.7, too little for that much of the device.  Before either: one block on one CU for up to 262144
+// elements (61 us), five launches beyond (1 M elements: 12.3 us).
 constexpr int kDynThreads = 512, kDynQuads = 4, kDynPerBlock = kDynThreads * kDynQuads * 4;
-constexpr int kExchange = 256, kExchangePolls = 4096, kMaxParts = 512;
+constexpr int kExchange = 64, kExchangePolls = 4096, kMaxParts = 512;
 constexpr unsigned long long kSlotEmpty = ~0ull;  // NaNs that no range contains: mm_write's NaN is the canonical one
 struct DynScratch {
     unsigned long long slot[kExchange];    // low word: the block's minimum, high word: its maximum

@@ -538,8 +538,8 @@ def test_dynamic_linear_wide_layer_at_small_batch(M, K):
                                    (520, 4096, 48), (419, 5011, 20),
                                    (1, 3, 9), (1, 4, 9), (1, 5, 40), (1, 1030, 8200), (1, 4096, 50), (1, 4099, 50), (1, 8191, 8193),
                                    (1, 8192, 8200), (1, 8193, 8200),  # one row, in a block's registers or not
-                                   # 256 blocks, the most that exchange them, and 257, which get them from slices
-                                   (256, 8192, 20), (255, 8225, 20), (257, 8192, 20), (256, 8193, 20),
+                                   # 64 blocks, the most that exchange them, and 65 and more, which get them from slices
+                                   (64, 8192, 20), (63, 8322, 20), (65, 8192, 20), (64, 8193, 20), (256, 8192, 20), (255, 8225, 20), (257, 8192, 20), (256, 8193, 20),
                                    (2, 131007, 3), (2, 131008, 3), (2, 131071, 3)])  # the longest rows
 @pytest.mark.parametrize("kind", ["normal", "constant", "nan"])
 def test_dynamic_linear_of_any_size(M, K, N, kind):

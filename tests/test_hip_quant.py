@@ -437,6 +437,28 @@ def test_a_block_that_does_not_wait_for_the_others_ranges_takes_them_itself(rows
         assert np.array_equal(q.numpy()[:, :cols], wq.numpy()) and not q.numpy()[:, cols:].any()
 
 
+def test_quantize_tensor_dynamic_where_streams_have_more_hardware_queues():
+    """Fewer blocks exchange their ranges there (32 with 32 queues): 33 of them take two launches, with the same bits."""
+    import os, subprocess, sys, textwrap
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    script = textwrap.dedent("""
+        import sys
+        sys.path.insert(0, %r); sys.path.insert(0, %r)
+        from test_hip_quant import test_quantize_tensor_dynamic_equals_the_three_calls as check
+        import lucid_amd as L
+        L._C.init(0)
+        for n in (16 * 8192, 17 * 8192, 262144):
+            check(n, "quint8")
+        from test_hip_quant import test_a_block_that_does_not_wait_for_the_others_ranges_takes_them_itself as exchange
+        for rows in (32, 33):
+            exchange(rows, 8192, 8192, 0, False)
+        print("OK", flush=True)
+    """ % (root, os.path.join(root, "tests")))
+    r = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=110,
+                       env={**os.environ, "GPU_MAX_HW_QUEUES": "32"})
+    assert r.returncode == 0 and r.stdout.strip().endswith("OK"), r.stdout + r.stderr
+
+
 def test_quantize_tensor_dynamic_refuses_large_tensors():
     from lucid_amd import _C
     x = L.Tensor.empty((262145,), L.float32, "hip")
