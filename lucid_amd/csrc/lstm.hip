@@ -253,6 +253,8 @@ __device__ __forceinline__ void multiply(v4f (&acc)[4], const v4u (&raw)[KP][2],
                 to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, parts[i & 1][q]), wf[g][i], to, 0, 0, 0);
             }
     }
+    // (every product is issued before the first sum waits: for a few registers less the compiler would go gate by gate)
+    if (KP == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int g = 0; g < 4; ++g) acc[g] += low[g];
 }
@@ -268,13 +270,16 @@ struct LstmForm {
     static constexpr int kThreads = (W + XW) * 64;
     static constexpr int kPartFloats = W * 4 * kGateFloats, kInputFloats = XW * 4 * 4 * 64;
     static constexpr int kLdsBytes = 2 * (kPartFloats + kInputFloats) * 4;
-    // wavefronts of a SIMD: the weights take 16 registers per instruction, the rest about 100
+    // wavefronts of a SIMD: the weights take 16 registers per instruction, the rest about 100.  At most as many as the
+    // registers used leave room for: the compiler keeps further ones out by allotting more registers, which the occupancy query of
+    // split_lstm does not see (two per SIMD at hidden 128, 114 registers: it counted on two blocks per CU where one fitted).
     static constexpr int kPerSimd = XW == 0 && KPW <= 2 ? 4 : 2;
+    static constexpr int kMostPerSimd = KPW == 1 && KX == 1 ? 4 : kPerSimd;
 };
 
 template <int W, int KPW, int XW, int KX>
 __global__ __launch_bounds__((W + XW) * 64)
-    __attribute__((amdgpu_waves_per_eu(LstmForm<W, KPW, XW, KX>::kPerSimd, LstmForm<W, KPW, XW, KX>::kPerSimd)))
+    __attribute__((amdgpu_waves_per_eu(LstmForm<W, KPW, XW, KX>::kPerSimd, LstmForm<W, KPW, XW, KX>::kMostPerSimd)))
 void lstm_sequence_kernel(LstmArgs p) {
     using Form = LstmForm<W, KPW, XW, KX>;
     extern __shared__ __align__(16) float lds[];

@@ -31,6 +31,24 @@ def test_inline_assembly_mfma_loop_is_clean():
     assert r.stdout.count("clean") >= 2 and "NOT CLEAN" not in r.stdout
 
 
+def test_lstm_recurrence_reports_the_registers_it_is_given():
+    """The launcher keeps all blocks of a launch resident by the runtime's occupancy query, which goes by the register
+    count that the code object reports.  An upper bound on the wavefronts of a SIMD makes the compiler allot more than
+    that: the query would promise blocks that do not fit.  512 registers per lane and SIMD, handed out by eights."""
+    import os
+    import re
+    import subprocess
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lucid_amd", "csrc")
+    subprocess.run(["make", "-C", csrc, "build/lstm.s"], check=True, capture_output=True, timeout=600)
+    text = open(os.path.join(csrc, "build", "lstm.s")).read()
+    given = dict(re.findall(r"\.amdhsa_kernel (\S+).*?\.amdhsa_next_free_vgpr (\d+)", text, re.S))
+    kernels = re.findall(r"\.max_flat_workgroup_size: (\d+)\s+\.name: +(\S*lstm_sequence\S*).*?\.vgpr_count: +(\d+)", text, re.S)
+    assert len(kernels) >= 9
+    for threads, name, reported in kernels:
+        blocks = [512 // -(-int(n) // 8 * 8) * 4 // (int(threads) // 64) for n in (given[name], reported)]
+        assert blocks[0] == blocks[1], (name, given[name], reported)
+
+
 def test_version_and_registry():
     assert _C.load().lq_version() == _C.ABI_VERSION == 3
     ops = dict((n, (v, d)) for n, v, d in _C.op_registry())
