@@ -430,6 +430,9 @@ void lstm_sequence_kernel(LstmArgs p) {
                 if (!missing) break;
                 if (spin >= kSpinLimit) waiting = false;
             }
+            // What this wavefront stored in the last step is there before it hands out more (see where a slot is emptied).
+            // The loads above have waited for it; a wavefront whose columns no block has made none.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         if constexpr (XW > 0) {
             lds_barrier();
@@ -475,7 +478,7 @@ void lstm_sequence_kernel(LstmArgs p) {
                 __builtin_amdgcn_raw_buffer_store_b32(unit < H ? bits : 0u, ring, own_off, unsigned(s % kSlots) * slot_bytes,
                                                       kScopeDevice);
                 // Every block has taken h[s - 2], or it would not have handed out h[s - 1]: its slot is for h[s + 2].  The
-                // next wait for h[s] is also for this store, so nobody who has h[s + 1] still finds h[s - 2] there.
+                // next step waits for this store before it hands out h[s + 1], so nobody who has that still finds h[s - 2] here.
                 if (s >= 2)
                     __builtin_amdgcn_raw_buffer_store_b32(kEmpty, ring, own_off, unsigned((s + 2) % kSlots) * slot_bytes,
                                                           kScopeDevice);

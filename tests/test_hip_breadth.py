@@ -291,6 +291,8 @@ def test_dynamic_lstm(layers, bidir, batch_first, bias, with_state):
 
 
 @pytest.mark.parametrize("I,H,layers,Bn,Tn,bidir", [(5, 16, 1, 1, 11, False), (31, 40, 3, 17, 9, False), (2, 2, 1, 16, 6, True),
+                                                    # wavefronts of the first four without columns of h to read
+                                                    (130, 90, 1, 16, 12, False), (64, 150, 2, 20, 12, False), (280, 300, 1, 16, 12, True),
                                                     (300, 257, 1, 33, 13, False), (600, 512, 1, 16, 10, True)])
 def test_dynamic_lstm_steps_reuse_what_blocks_hand_over(I, H, layers, Bn, Tn, bidir):
     # more steps than the ring between the blocks holds, sizes that end inside a load; values across the gates' branches
