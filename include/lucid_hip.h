@@ -225,6 +225,9 @@ int lq_lstm_sequence_pays(int batch, int hidden, int directions, int* pays);
 /* How many of `layers` stacked layers the next call should take with x given (0: take gates_x). */
 int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layers, int directions, int* fused);
 int lq_lstm_sequence_f32(const lq_lstm_args* args, lq_stream stream);
+/* The same with the bound on a wait between its blocks (about 2^20 reads above, the most): after `spins` reads without
+ * finding h a block gives up, and its outputs from that step on, and what other blocks compute of them, are NaN. */
+int lq_lstm_sequence_spins_f32(const lq_lstm_args* args, int spins, lq_stream stream);
 
 /* Self-test of the tile kernels' requantize arithmetic.  Their epilogue computes
  * clamp(rint(x / scale) + zp, qmin, qmax) mostly without dividing (x * (1/scale),

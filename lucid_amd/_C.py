@@ -254,6 +254,7 @@ class LstmArgs(C.Structure):
 _SIGNATURES["lq_lstm_sequence_pays"] = [_i] * 3 + [C.POINTER(_i)]
 _SIGNATURES["lq_lstm_fused_layers"] = [_i] * 6 + [C.POINTER(_i)]
 _SIGNATURES["lq_lstm_sequence_f32"] = [C.POINTER(LstmArgs), _vp]
+_SIGNATURES["lq_lstm_sequence_spins_f32"] = [C.POINTER(LstmArgs), _i, _vp]
 _SIGNATURES["lq_qconv3d_i8"] = [C.POINTER(QConv3dArgs), _vp]
 _SIGNATURES["lq_quantize_nchw_to_nhwc"] = [_vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _vp]
 _SIGNATURES["lq_qconv2d_packed4_geometry"] = [C.POINTER(QConv2dArgs), C.POINTER(_i), C.POINTER(_i), C.POINTER(_i)]

@@ -37,7 +37,8 @@
 // launcher bounds the grid by what the device holds of this kernel over the number of hardware queues
 // that streams share (four unless GPU_MAX_HW_QUEUES says more; a queue starts a launch only after the one
 // before it is fully placed), and larger batches run as several launches.  A wait is bounded besides:
-// after kSpinLimit reads the block stops waiting for the rest of the sequence and what it computes is NaN.
+// after kSpinLimit reads a wavefront gives up.  It is out of step with the others then, and the ring may hold any step of theirs,
+// so its products are NaN from there on, and with them all that the block computes and hands out.
 //
 // hidden 512, 16 rows, a step of 2.2 us (5100 cycles, timestamps): 450 before the first read, 1850 for the 32 KiB of h a
 // CU reads past its L2 (1000 at hidden 128), 1390 splits and products, 70 barrier, 1000 sums and gates.  Two such layers of
@@ -60,7 +61,8 @@ typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 
 constexpr int kUnits = 16, kRows = 16;     // hidden units of a block, batch rows of a group
-constexpr unsigned kEmpty = 0xffffffffu;   // a word of y that has not been written
+constexpr unsigned kEmpty = 0xffffffffu;   // a word of h that has not been written
+constexpr unsigned kNan = 0x7fc00000u;
 constexpr int kSpinLimit = 1 << 20;        // about a second of waiting for one step
 constexpr int kScopeDevice = 16;           // "sc1" cache-policy bit of buffer accesses
 constexpr int kSlots = 4;                  // steps of h that a ring holds
@@ -88,7 +90,7 @@ struct LstmArgs {
     long y_elems, x_elems;
     unsigned* rings;             // [part][group][slot][block of units][kSlotWords]
     long ring_words;             // of all of them
-    int T, B, H, I, row0, dir0, stacked;
+    int T, B, H, I, row0, dir0, stacked, spins;
 };
 
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
@@ -324,7 +326,7 @@ void lstm_sequence_kernel(LstmArgs p) {
                     if (!whole) mask_columns<KX>(raw, I - k_lane);
                     const unsigned missing = waiting ? missing_words<KX>(raw) : 0;
                     if (!missing) break;
-                    if (spin >= kSpinLimit) waiting = false;
+                    if (spin >= p.spins) waiting = false;  // (what is not written is NaN, what is written is right)
                     asm volatile("" ::: "memory");  // read again: the words change under the loop
                     request(raw, s, missing);
                 }
@@ -387,7 +389,6 @@ void lstm_sequence_kernel(LstmArgs p) {
     const unsigned present = blocks_left <= 0 ? 0u : blocks_left >= 2 * KPW ? ~0u : (1u << blocks_left) - 1u;
     const unsigned own_off = (blockIdx.x * kSlotWords + wave * 64 + lane) * 4;  // four units of a row side by side
     const int own_sum = (tile_row & 3) * kGateRow + (tile_row >> 2) * 16 + 4 * wave + (lane & 3);
-    bool waiting = true;
     unsigned bits = 0;
     auto store_y = [&](int s) {
         const int t = d ? p.T - 1 - s : s;
@@ -407,7 +408,8 @@ void lstm_sequence_kernel(LstmArgs p) {
                 raw[i][e >> 2][e & 3] = k < H ? __float_as_uint(v) : 0u;
             }
     }
-    for (int s = 0; s < p.T; ++s) {
+    int s = 0;
+    for (; s < p.T; ++s) {
         v4f in_acc[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) in_acc[g] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -419,6 +421,7 @@ void lstm_sequence_kernel(LstmArgs p) {
             if (gridDim.x > 16) __builtin_amdgcn_s_sleep(8);
             else __builtin_amdgcn_s_sleep(5);
             unsigned missing = present;
+            bool gave_up = false;
             for (int spin = 0;; ++spin) {
                 asm volatile("" ::: "memory");  // read again: the words change under the loop
 #pragma unroll
@@ -426,10 +429,14 @@ void lstm_sequence_kernel(LstmArgs p) {
                     if (missing >> i & 1)
                         raw[i >> 1][i & 1] =
                             __builtin_amdgcn_raw_buffer_load_b128(ring, h_off + unsigned(i * kSlotWords) * 4, slot, kScopeDevice);
-                missing = waiting ? missing_words<KPW>(raw) : 0;
+                missing = missing_words<KPW>(raw);
                 if (!missing) break;
-                if (spin >= kSpinLimit) waiting = false;
+                if (spin >= p.spins) {
+                    gave_up = true;
+                    break;
+                }
             }
+            if (gave_up) break;
             // What this wavefront stored in the last step is there before it hands out more (see where a slot is emptied).
             // The loads above have waited for it; a wavefront whose columns no block has made none.
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -473,7 +480,7 @@ void lstm_sequence_kernel(LstmArgs p) {
             c = fg * c + ig * gg;
             hv = og * tanh_gate(c);
             bits = __float_as_uint(hv);
-            bits = bits == kEmpty ? 0x7fc00000u : bits;  // a NaN, but not the one that means "not written"
+            bits = bits == kEmpty ? kNan : bits;  // a NaN, but not the one that means "not written"
             if (s + 1 < p.T) {
                 __builtin_amdgcn_raw_buffer_store_b32(unit < H ? bits : 0u, ring, own_off, unsigned(s % kSlots) * slot_bytes,
                                                       kScopeDevice);
@@ -483,6 +490,18 @@ void lstm_sequence_kernel(LstmArgs p) {
                     __builtin_amdgcn_raw_buffer_store_b32(kEmpty, ring, own_off, unsigned((s + 2) % kSlots) * slot_bytes,
                                                           kScopeDevice);
             }
+            if (mine) store_y(s);
+        }
+    }
+    if (s < p.T) {  // gave up at step s: what is left of the sequence, with its barriers
+        bits = kNan, hv = c = __uint_as_float(kNan);
+        if (wave < 4)
+            for (int slot = 0; slot < kSlots; ++slot)
+                __builtin_amdgcn_raw_buffer_store_b32(bits, ring, own_off, unsigned(slot) * slot_bytes, kScopeDevice);
+        for (; s < p.T; ++s) {
+            if constexpr (XW > 0) lds_barrier();
+            for (int i = lane; i < 4 * kGateFloats; i += 64) part[(s & 1) * Form::kPartFloats + wave * 4 * kGateFloats + i] = hv;
+            lds_barrier();
             if (mine) store_y(s);
         }
     }
@@ -642,7 +661,10 @@ int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layer
     return LQ_OK;
 }
 
-int lq_lstm_sequence_f32(const lq_lstm_args* a, lq_stream stream) {
+int lq_lstm_sequence_f32(const lq_lstm_args* a, lq_stream stream) { return lq_lstm_sequence_spins_f32(a, kSpinLimit, stream); }
+
+int lq_lstm_sequence_spins_f32(const lq_lstm_args* a, int spins, lq_stream stream) {
+    LQ_REQUIRE(spins >= 0, LQ_ERR_VALUE, "lstm_sequence: %d spins", spins);
     LQ_REQUIRE(a, LQ_ERR_VALUE, "lstm_sequence: args is NULL");
     LQ_REQUIRE(a->steps >= 0 && a->batch >= 0 && a->hidden > 0, LQ_ERR_SHAPE, "lstm_sequence: bad extent (%d, %d, %d)",
                a->steps, a->batch, a->hidden);
@@ -675,7 +697,7 @@ int lq_lstm_sequence_f32(const lq_lstm_args* a, lq_stream stream) {
     }
     p.x = a->x, p.I = a->inputs;
     p.h0 = a->h0, p.c0 = a->c0, p.h_n = a->h_n, p.c_n = a->c_n;
-    p.T = a->steps, p.B = a->batch, p.H = a->hidden;
+    p.T = a->steps, p.B = a->batch, p.H = a->hidden, p.spins = spins < kSpinLimit ? spins : kSpinLimit;
     const long width = long(a->directions) * p.H, gates = 4L * p.H;
     p.y_step = a->batch_first ? width : p.B * width, p.y_row = a->batch_first ? p.T * width : width;
     p.gx_step = a->batch_first ? gates : p.B * gates, p.gx_row = a->batch_first ? p.T * gates : gates;

@@ -317,6 +317,32 @@ def test_dynamic_lstm_steps_reuse_what_blocks_hand_over(I, H, layers, Bn, Tn, bi
         assert off[:, 1:].max(initial=0.0) < 2e-5 and off[:, 0].max() < 2e-5 + slack
 
 
+@pytest.mark.parametrize("I,H,layers,Bn,Tn,bidir", [(64, 512, 1, 40, 14, False), (40, 120, 3, 100, 14, False),
+                                                    (512, 512, 1, 16, 14, True), (600, 1024, 1, 16, 14, False)])
+@pytest.mark.parametrize("spins", [0, 1, 2, 4])
+def test_a_wait_of_the_recurrence_that_is_given_up_gives_nan(monkeypatch, I, H, layers, Bn, Tn, bidir, spins):
+    """A block that gave up no longer runs in step with the others, and the ring between them holds other steps' h: its
+    outputs are NaN from there on, or right."""
+    from lucid_amd import _C
+    rng = np.random.default_rng(H + spins)
+    qm = Q.quantize_dynamic(nn.LSTM(I, H, num_layers=layers, bidirectional=bidir))
+    x = rng.standard_normal((Tn, Bn, I)).astype(np.float32)
+    wy, wh, wc = _oracle_lstm_stack(qm, x, None, False)
+    call, bounded = _C.call, []
+
+    def call_with_bound(name, *args):
+        if name == "lq_lstm_sequence_f32":
+            bounded.append(name)
+            return call("lq_lstm_sequence_spins_f32", args[0], spins, *args[1:])
+        return call(name, *args)
+    monkeypatch.setattr(_C, "call", call_with_bound)
+    for _ in range(3):
+        y, (hn, cn) = qm(hip(x))
+        for got, want in ((y.numpy(), wy), (hn.numpy(), wh), (cn.numpy(), wc)):
+            assert np.abs(np.where(np.isnan(got), want, got) - want).max() < 2e-5
+    assert bounded
+
+
 @pytest.mark.parametrize("I,H,Bn,Tn,bidir,batch_first",
                          [(3, 1, 1, 3, False, False), (8, 17, 5, 4, True, True), (16, 33, 16, 2, False, True),
                           (8, 128, 17, 3, True, False), (7, 129, 33, 2, False, False), (16, 300, 3, 1, True, True),
