@@ -8,6 +8,7 @@
 // that are asked for are read, and decoded on the way out - the values are the same
 // (float(code) - z) * s per element.
 #include "common.hpp"
+#include "lstm_gates.hpp"
 #include "qepilogue.hpp"
 
 using namespace lq;
@@ -230,8 +231,6 @@ __global__ __launch_bounds__(256) void dilate_nhwc_i8_kernel(const int8_t* __res
 // One time step of the gates (CpuBackend.h:13456-13506; i, f, g, o in this order
 // along the 4H axis): raw = x W_ih^T + h W_hh^T + (b_ih + b_hh),
 // c' = sigmoid(f) * c + sigmoid(i) * tanh(g), h' = sigmoid(o) * tanh(c').
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
-
 __global__ __launch_bounds__(256) void lstm_cell_kernel(const float* __restrict__ gx, const float* __restrict__ gh,
                                                         const float* __restrict__ bias,
                                                         const float* __restrict__ c_in, int B, int H, size_t gx_ld,
@@ -245,12 +244,12 @@ __global__ __launch_bounds__(256) void lstm_cell_kernel(const float* __restrict_
         const size_t H2 = 2 * size_t(H), H3 = 3 * size_t(H);
         const float bi = bias ? bias[j] : 0.0f, bf = bias ? bias[H + j] : 0.0f;
         const float bg = bias ? bias[H2 + j] : 0.0f, bo = bias ? bias[H3 + j] : 0.0f;
-        const float ig = sigmoidf_((px[j] + ph[j]) + bi);
-        const float fg = sigmoidf_((px[H + j] + ph[H + j]) + bf);
-        const float gg = tanhf((px[H2 + j] + ph[H2 + j]) + bg);
-        const float og = sigmoidf_((px[H3 + j] + ph[H3 + j]) + bo);
+        const float ig = sigmoid((px[j] + ph[j]) + bi);
+        const float fg = sigmoid((px[H + j] + ph[H + j]) + bf);
+        const float gg = tanh_gate((px[H2 + j] + ph[H2 + j]) + bg);
+        const float og = sigmoid((px[H3 + j] + ph[H3 + j]) + bo);
         const float c = fg * c_in[e] + ig * gg;
-        const float h = og * tanhf(c);
+        const float h = og * tanh_gate(c);
         c_out[e] = c;
         h_out[e] = h;
         if (y) y[b * y_ld + j] = h;

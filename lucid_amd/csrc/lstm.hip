@@ -49,6 +49,7 @@
 #include <cstdlib>
 #include <type_traits>
 #include "common.hpp"
+#include "lstm_gates.hpp"
 
 using namespace lq;
 
@@ -108,36 +109,6 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
 __device__ __forceinline__ uint32_t codes_bf16(int c0, int c1) {
     return __builtin_amdgcn_perm(__float_as_uint(float(c1)), __float_as_uint(float(c0)), 0x07060302u);
 }
-// The gates are on the chain of a step, so both functions are straight-line code, within 2 units in the last place of
-// the exact values (the library's expf and tanhf branch, and both sides run in a wavefront).
-// exp(x) for x <= 60: 2^(x log2 e) with the rounding error of the product put back
-__device__ __forceinline__ float exp_gate(float x) {
-    constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596299e-8f, kLn2 = 0.693147182f;
-    const float t = x * kLog2e;
-    const float low = __builtin_fmaf(x, kLog2eLow, __builtin_fmaf(x, kLog2e, -t));
-    const float e = __builtin_amdgcn_exp2f(t);
-    return __builtin_fmaf(e, low * kLn2, e);
-}
-// 1 / x for 1 <= x < 2^100
-__device__ __forceinline__ float reciprocal(float x) {
-    const float r = __builtin_amdgcn_rcpf(x);
-    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
-}
-__device__ __forceinline__ float sigmoid(float x) {  // (a NaN fails the comparison and stays one)
-    return reciprocal(1.0f + exp_gate(x < -60.0f ? 60.0f : x > 60.0f ? -60.0f : -x));
-}
-__device__ __forceinline__ float tanh_gate(float x) {
-    const float a = __builtin_fabsf(x), u = x * x;
-    // below 0.6 x + x^3 P(x^2): P fitted for the least relative error, 2.8e-9
-    float q = __builtin_fmaf(u, -0x1.8257d2p-8f, 0x1.54b882p-6f);
-    q = __builtin_fmaf(q, u, -0x1.b898dap-5f);
-    q = __builtin_fmaf(q, u, 0x1.1109aep-3f);
-    q = __builtin_fmaf(q, u, -0x1.55553ep-2f);
-    const float small = __builtin_fmaf(x * u, q, x);
-    const float large = __builtin_fmaf(-2.0f, reciprocal(1.0f + exp_gate(a > 20.0f ? 40.0f : 2.0f * a)), 1.0f);
-    return a < 0.6f ? small : __builtin_copysignf(large, x);
-}
-
 // Columns of a wavefront.  An instruction's 32 columns are two runs of 16, of which the lane's quarter has four each
 // (`kRun` apart): a lane's 16-byte loads then lie beside those of the other quarters, 64 bytes of a row per load.  Which
 // column is which k of the instruction does not matter as long as the weight is held in the same order.

@@ -296,7 +296,7 @@ def test_dynamic_lstm(layers, bidir, batch_first, bias, with_state):
                                                     (300, 257, 1, 33, 13, False), (600, 512, 1, 16, 10, True)])
 def test_dynamic_lstm_steps_reuse_what_blocks_hand_over(I, H, layers, Bn, Tn, bidir):
     # more steps than the ring between the blocks holds, sizes that end inside a load; values across the gates' branches
-    # (tanh changes form at 0.6, the exponentials are clamped at 60 and 20) and one sequence with a NaN and one with large
+    # (tanh changes form at 0.6, the exponentials end at 110 and 20) and one sequence with a NaN and one with large
     # inputs, which must stay theirs.  2e-5 as in the tests above; a float32 sum of the large inputs may be off by
     # 2^-23 sum |x w| (both sides round; no gate is steeper than 1), which a cell adds up over the steps.
     rng = np.random.default_rng(H)
@@ -315,6 +315,49 @@ def test_dynamic_lstm_steps_reuse_what_blocks_hand_over(I, H, layers, Bn, Tn, bi
         ok = ~np.isnan(want)
         off = np.where(ok, np.abs(got - want), 0.0)  # (rows are axis 1)
         assert off[:, 1:].max(initial=0.0) < 2e-5 and off[:, 0].max() < 2e-5 + slack
+
+
+def _units_off(got, want):
+    """Distance in units of the last place of ``want`` (float64), which below 2^-126 is 2^-149."""
+    return np.abs(got.astype(np.float64) - want) / np.exp2(np.maximum(np.floor(np.log2(np.maximum(np.abs(want), 2.0 ** -126))), -126) - 23)
+
+
+@pytest.mark.parametrize("H", [512, 768])  # with the input product and without
+def test_gates_against_float64(H):
+    """One step on zero inputs: the gates are the biases.  With the input gate shut and c = 1 the new c is sigmoid(f), with
+    the forget gate shut and the input gate open it is tanh(g).  Units of the last place: the exponential's two (the
+    instruction has one) and half of one each for the product and the result, for tanh less than half of that again."""
+    from lucid_amd import _C
+    qm = Q.quantize_dynamic(nn.LSTM(4, H))
+    special = np.array([np.inf, -np.inf, np.nan, -0.0, 0.0, 3e38, -3e38, 1e-40, -1e-40, -60.5, -87.5, -100.0, -103.9], np.float32)
+    values = np.concatenate([special, np.linspace(-104, -10, H), np.linspace(-12, 12, 3 * H), np.linspace(-0.8, 0.8, 2 * H)])
+    values = np.resize(values.astype(np.float32), (7, H))
+    x = hip(np.zeros((1, 1, 4), np.float32))
+    wide = values.astype(np.float64)
+    with np.errstate(over="ignore"):
+        sig = np.where(wide < 0, np.exp(np.minimum(wide, 0)) / (1 + np.exp(np.minimum(wide, 0))), 1 / (1 + np.exp(-np.maximum(wide, 0))))
+    for shut, c0, want, most in ((True, 1.0, sig, 2.5), (False, -0.0, np.tanh(wide), 1.5)):
+        for v, w in zip(values, want):
+            bias = np.full((4, H), 200.0, np.float32)
+            bias[0] = -200.0 if shut else 200.0
+            bias[1] = v if shut else -200.0
+            bias[2] = 0.0 if shut else v
+            qm.bias_ih_l0, qm.bias_hh_l0 = hip(bias.reshape(-1)), hip(np.zeros(4 * H, np.float32))
+            c = hip(np.full((1, 1, H), c0, np.float32))
+            _, (hn, cn) = qm(x, (hip(np.zeros((1, 1, H), np.float32)), c))
+            got, ok = cn.numpy().reshape(-1), ~np.isnan(v)
+            assert np.isnan(got[~ok]).all() and _units_off(got[ok], w[ok]).max() <= most
+            assert bool((np.signbit(got) == np.signbit(w))[ok & (v != 0)].all())  # (a bias of -0 is added to a product of +0)
+            # the kernel of a single step gives the same bits
+            zero, h1, c1 = hip(np.zeros(4 * H, np.float32)), hip(np.zeros(H, np.float32)), hip(np.zeros(H, np.float32))
+            _C.call("lq_lstm_cell_f32", qm.bias_ih_l0.data_ptr, 4 * H, zero.data_ptr, None, c.data_ptr, 1, H, h1.data_ptr,
+                    c1.data_ptr, None, 0, None)
+            assert np.array_equal(got, c1.numpy(), equal_nan=True)
+            assert np.array_equal(hn.numpy().reshape(-1), h1.numpy(), equal_nan=True)
+    bias = np.stack([np.full(H, v, np.float32) for v in (-200, 200, -1, 0)])  # c stays -0, and h is a half of its tanh
+    qm.bias_ih_l0 = hip(bias.reshape(-1))
+    _, (hn, cn) = qm(x, (hip(np.zeros((1, 1, H), np.float32)), hip(np.full((1, 1, H), -0.0, np.float32))))
+    assert bool(np.signbit(cn.numpy()).all()) and bool(np.signbit(hn.numpy()).all()) and not hn.numpy().any()
 
 
 @pytest.mark.parametrize("I,H,layers,Bn,Tn,bidir", [(64, 512, 1, 40, 14, False), (40, 120, 3, 100, 14, False),
