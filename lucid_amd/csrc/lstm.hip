@@ -37,8 +37,8 @@
 // launcher bounds the grid by what the device holds of this kernel over the number of hardware queues
 // that streams share (four unless GPU_MAX_HW_QUEUES says more; a queue starts a launch only after the one
 // before it is fully placed), and larger batches run as several launches.  A wait is bounded besides:
-// after kSpinLimit reads a wavefront gives up.  It is out of step with the others then, and the ring may hold any step of theirs,
-// so its products are NaN from there on, and with them all that the block computes and hands out.
+// after kSpinLimit reads a wavefront gives up for the rest of the sequence.  It is out of step with the others then, and the ring may
+// hold any step of theirs, so its sums are NaN from there on, and with them all that the block computes and hands out.
 //
 // hidden 512, 16 rows, a step of 2.2 us (5100 cycles, timestamps): 450 before the first read, 1850 for the 32 KiB of h a
 // CU reads past its L2 (1000 at hidden 128), 1390 splits and products, 70 barrier, 1000 sums and gates.  Two such layers of
@@ -360,6 +360,7 @@ void lstm_sequence_kernel(LstmArgs p) {
     const unsigned present = blocks_left <= 0 ? 0u : blocks_left >= 2 * KPW ? ~0u : (1u << blocks_left) - 1u;
     const unsigned own_off = (blockIdx.x * kSlotWords + wave * 64 + lane) * 4;  // four units of a row side by side
     const int own_sum = (tile_row & 3) * kGateRow + (tile_row >> 2) * 16 + 4 * wave + (lane & 3);
+    bool waiting = true;
     unsigned bits = 0;
     auto store_y = [&](int s) {
         const int t = d ? p.T - 1 - s : s;
@@ -379,8 +380,7 @@ void lstm_sequence_kernel(LstmArgs p) {
                 raw[i][e >> 2][e & 3] = k < H ? __float_as_uint(v) : 0u;
             }
     }
-    int s = 0;
-    for (; s < p.T; ++s) {
+    for (int s = 0; s < p.T; ++s) {
         v4f in_acc[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) in_acc[g] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -392,7 +392,6 @@ void lstm_sequence_kernel(LstmArgs p) {
             if (gridDim.x > 16) __builtin_amdgcn_s_sleep(8);
             else __builtin_amdgcn_s_sleep(5);
             unsigned missing = present;
-            bool gave_up = false;
             for (int spin = 0;; ++spin) {
                 asm volatile("" ::: "memory");  // read again: the words change under the loop
 #pragma unroll
@@ -400,14 +399,10 @@ void lstm_sequence_kernel(LstmArgs p) {
                     if (missing >> i & 1)
                         raw[i >> 1][i & 1] =
                             __builtin_amdgcn_raw_buffer_load_b128(ring, h_off + unsigned(i * kSlotWords) * 4, slot, kScopeDevice);
-                missing = missing_words<KPW>(raw);
+                missing = waiting ? missing_words<KPW>(raw) : 0;
                 if (!missing) break;
-                if (spin >= p.spins) {
-                    gave_up = true;
-                    break;
-                }
+                if (spin >= p.spins) waiting = false;
             }
-            if (gave_up) break;
             // What this wavefront stored in the last step is there before it hands out more (see where a slot is emptied).
             // The loads above have waited for it; a wavefront whose columns no block has made none.
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -436,6 +431,8 @@ void lstm_sequence_kernel(LstmArgs p) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) parts[(wave * 4 + g) * kGateFloats + r * kGateRow + lane] = acc[g][r];
         }
+        if (!waiting)  // (once more, and not in place of the sums: what gives them another value here costs a step 3 %)
+            for (int i = lane; i < 4 * kGateFloats; i += 64) parts[wave * 4 * kGateFloats + i] = __uint_as_float(kNan);
         // (a buffer is written again two steps later, after the next step's barrier: by then it has been read)
         lds_barrier();
         if (wave < 4) {
@@ -461,18 +458,6 @@ void lstm_sequence_kernel(LstmArgs p) {
                     __builtin_amdgcn_raw_buffer_store_b32(kEmpty, ring, own_off, unsigned((s + 2) % kSlots) * slot_bytes,
                                                           kScopeDevice);
             }
-            if (mine) store_y(s);
-        }
-    }
-    if (s < p.T) {  // gave up at step s: what is left of the sequence, with its barriers
-        bits = kNan, hv = c = __uint_as_float(kNan);
-        if (wave < 4)
-            for (int slot = 0; slot < kSlots; ++slot)
-                __builtin_amdgcn_raw_buffer_store_b32(bits, ring, own_off, unsigned(slot) * slot_bytes, kScopeDevice);
-        for (; s < p.T; ++s) {
-            if constexpr (XW > 0) lds_barrier();
-            for (int i = lane; i < 4 * kGateFloats; i += 64) part[(s & 1) * Form::kPartFloats + wave * 4 * kGateFloats + i] = hv;
-            lds_barrier();
             if (mine) store_y(s);
         }
     }
