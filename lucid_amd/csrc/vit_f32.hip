@@ -1030,7 +1030,8 @@ int lq_layernorm_quantize_from_range_i8(const float* x, const float* gamma, cons
     LQ_REQUIRE(range && scale && zp, LQ_ERR_VALUE, "layernorm_quantize: null pointer");
     // Every block of the one launch reads a slot per block of the statistics: up to 2048 rows that is less than the launch it
     // saves (12 608 rows of 768: 16.6 us against 8.3 + 4.6).
-    if (rows > kRangeRows) {
+    // No rows have no block that hands out the qparams.
+    if (rows > kRangeRows || rows == 0) {
         const int rc = lq_calc_qparams_from_range(range, symmetric, qmin, qmax, is_signed, eps, scale, zp, nullptr, nullptr, stream);
         return rc ? rc : lq_layernorm_quantize_i8(x, gamma, beta, stats, rows, cols, scale, zp, qmin, qmax, code_offset, q, stream);
     }

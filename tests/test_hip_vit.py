@@ -356,6 +356,20 @@ def test_codes_straight_from_a_kept_range(n, nan):
         assert np.array_equal(one[2].numpy()[:n - 1], two[2].numpy()[:n - 1])
 
 
+def test_layernorm_codes_of_no_rows_still_give_the_qparams():
+    """``lq_layernorm_quantize_from_range_i8`` stands for two calls, of which the first does not look at the rows."""
+    from lucid_amd.nn.functional import _new_range
+    rng = np.random.default_rng(3)
+    x, w = (L.tensor(rng.standard_normal(n).astype(np.float32), device="hip") for n in (64, 64))
+    kept, stats, q = _new_range(), L.Tensor.empty((2,), L.float32, "hip"), L.Tensor.empty((64,), L.int8, "hip")
+    _C.call("lq_gelu_f32", x.data_ptr, x.data_ptr, 64, kept.data_ptr, None)
+    want, got = ([L.tensor(np.float32(-7), device="hip") for _ in range(2)] for _ in range(2))
+    _C.call("lq_calc_qparams_from_range", kept.data_ptr, 0, 0, 255, 0, 1e-8, *(t.data_ptr for t in want), None, None, None)
+    _C.call("lq_layernorm_quantize_from_range_i8", x.data_ptr, w.data_ptr, w.data_ptr, stats.data_ptr, 0, 64, kept.data_ptr, 0, 0,
+            255, 0, 1e-8, -128, *(t.data_ptr for t in got), q.data_ptr, None)
+    assert [t.numpy().tobytes() for t in got] == [t.numpy().tobytes() for t in want]
+
+
 def test_vit_block_with_and_without_fused_layernorm_quantize_agree(monkeypatch):
     import workloads as W
     cfg = dict(W.VIT_B16, depth=2, dim=192, heads=3, mlp=768)
