@@ -57,12 +57,13 @@ def qlinear_i8(a: Tensor, w: Tensor, *, a_zp: int = 0, a_zp_dev: Tensor | None =
     N = w.shape[0]
     if out is None:
         out = Tensor.empty((M, N), _OUT_DTYPE[out_mode], "hip")
-    args = _C.QLinearArgs()  # (zeros: what is absent is not set)
+    # (zeros: what is absent is not set.  Numbers are compared with 0 and not tested, so that None is still refused)
+    args = _C.QLinearArgs()
     args.a, args.w = _ptr(a, "a", T.int8), _ptr(w, "w", T.int8)
     args.M, args.N, args.K = M, N, K
     if wsum is not None:
         args.wsum = _ptr(wsum, "wsum", T.int32)
-    if a_zp:
+    if a_zp != 0:
         args.a_zp = int(a_zp)
     if a_zp_dev is not None:
         args.a_zp_dev = _ptr(a_zp_dev, "a_zp_dev", T.float32)
@@ -88,7 +89,7 @@ def qlinear_i8(a: Tensor, w: Tensor, *, a_zp: int = 0, a_zp_dev: Tensor | None =
         args.out_zp = _ptr(out_zp, "out_zp", T.float32)
     args.out_qmin, args.out_qmax, args.out_offset = int(out_qmin), int(out_qmax), int(out_offset)
     args.out = out.data_ptr
-    if path or tile_config:
+    if path != 0 or tile_config != 0:
         args.force_path, args.tile_config = int(path), int(tile_config)
     if residual is not None:
         if residual.numel != M * N:
@@ -96,7 +97,7 @@ def qlinear_i8(a: Tensor, w: Tensor, *, a_zp: int = 0, a_zp_dev: Tensor | None =
         args.residual = _ptr(residual, "residual", T.float32)
     if join is not None:
         _fill_join(args.join, join, (M, N))
-    if gelu:
+    if gelu != 0:
         args.gelu = int(gelu)
     if range_buf is not None:
         args.range = _ptr(range_buf, "range", T.float32)

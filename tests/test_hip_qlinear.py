@@ -23,6 +23,13 @@ def codes(rng, shape, lo=-128, hi=127):
     return rng.integers(lo, hi + 1, shape).astype(np.int8)
 
 
+@pytest.mark.parametrize("absent", [dict(a_zp=None), dict(path=None), dict(tile_config=None), dict(gelu=None)])
+def test_numbers_that_are_none_are_refused(absent):
+    a, w = hip(np.ones((2, 16), np.int8)), hip(np.ones((4, 16), np.int8))
+    with pytest.raises(TypeError):
+        _ops.qlinear_i8(a, w, **absent)
+
+
 ACC_CASES = [
     # M, N, K, path
     (256, 256, 128, TILE), (256, 256, 256, TILE), (512, 512, 4096, TILE), (300, 260, 144, TILE),
