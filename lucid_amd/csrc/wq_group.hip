@@ -374,7 +374,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     // Every global load of the block is requested before anything is consumed, in the order of
     // consumption (the wait counter retires loads in order): the scale / bias tables (short, from
     // the L2), x, the weights.
-    // Tables: 256 rows x gcap slots (gcap = the groups of a full k range, 4, 8 or 16), four slots per
+    // Tables: wq_rows(RB) rows x gcap slots (gcap = the groups of a full k range, 4, 8 or 16), four slots per
     // 16-byte load where the rows allow it (a dword per lane costs the vector cache as many cycles
     // as 16 bytes per lane do).
     constexpr int kTabVec = kWqRows * 16 / 4 / 512;  // 16-byte loads per thread and table, at 16 groups per k range
@@ -746,8 +746,8 @@ int lq_wq_matmul(const float* x, const uint32_t* packed, const float* scales, co
     LQ_REQUIRE(x && packed && scales && biases && out, LQ_ERR_VALUE, "wq_matmul: NULL pointer");
     hipStream_t st = as_stream(stream);
     if (aligned16(x) && aligned16(packed)) {
-        // one row is a stream of the weight; more rows go to the matrix cores: 16 rows x 512 k of 256 columns
-        // per block, or (wq_gemm.hip) tiles over all of K
+        // one row is a stream of the weight; more rows go to the matrix cores: 16 rows x 512 k of
+        // wq_rows(1 .. 3) columns per block, or (wq_gemm.hip) tiles over all of K
         if (M == 1 && wq_gemv1_lds(K, bits) <= size_t(kGemv1MaxLds))
             return bits == 4 ? launch_gemv1<4>(x, packed, scales, biases, N, K, group_size, out, st)
                              : launch_gemv1<8>(x, packed, scales, biases, N, K, group_size, out, st);

@@ -61,8 +61,8 @@ __device__ __forceinline__ void wq_exchange(uint32_t (&wd)[4]) {
 // 8 bits uncentred 4e-7 / 1.4e-6; centred 1.5e-7 / 3e-7, and 1e-6 when the weight is decoded first.
 template <int BITS>
 constexpr int kWqCentre = -(1 << (BITS - 1));
-template <int BITS, bool PATTERN = false>
-constexpr float kWqUnit = BITS == 4 && !PATTERN ? 16.0f : 1.0f;
+template <int BITS>
+constexpr float kWqUnit = BITS == 4 ? 16.0f : 1.0f;  // (not of PATTERN)
 
 template <int BITS, bool PATTERN = false>
 __device__ __forceinline__ uint4 wq_codes(const uint32_t (&wd)[4], int i) {

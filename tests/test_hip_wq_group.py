@@ -78,9 +78,25 @@ def test_small_batch_matmul_is_reproducible_and_exact_on_exact_inputs(bits):
 
 # the small-batch kernel with one, two and three tiles per wavefront (how many blocks each would have decides): rows that
 # end inside a tile and inside a block, batches that end inside sixteen, a last window and a last k range that are partial
-@pytest.mark.parametrize("M,N,K,gs,bits", [(2, 127, 544, 32, 4), (17, 129, 1088, 64, 8), (16, 4097, 4096, 128, 4),
-                                           (31, 8191, 2112, 64, 8), (7, 11007, 4096, 64, 8), (16, 10999, 4224, 128, 4),
-                                           (13, 7000, 6176, 32, 4), (64, 4100, 4096, 32, 8), (24, 8000, 992, 32, 4)])
+SMALL_BATCH_FORMS = [(2, 127, 544, 32, 4), (17, 129, 1088, 64, 8), (16, 4097, 4096, 128, 4),
+                     (31, 8191, 2112, 64, 8), (7, 11007, 4096, 64, 8), (16, 10999, 4224, 128, 4),
+                     (13, 7000, 6176, 32, 4), (64, 4100, 4096, 32, 8), (24, 8000, 992, 32, 4)]
+
+
+@pytest.mark.parametrize("M,N,K,gs,bits", SMALL_BATCH_FORMS + [(5, 385, 640, 64, 4), (33, 6000, 1024, 32, 4)])
+def test_small_batch_forms_are_exact_on_exact_inputs(M, N, K, gs, bits):
+    # small integers and scales of 1 and 2 keep every product and sum exact in float32 (below 2^24, 128 + c included): one
+    # code, row or group out of place shows
+    rng = np.random.default_rng(N + 1)
+    packed = rng.integers(0, 2**32, (N, K * bits // 32), dtype=np.uint32).view(np.int32)
+    s = rng.integers(1, 3, (N, K // gs)).astype(np.float32)
+    b = rng.integers(-8, 9, (N, K // gs)).astype(np.float32)
+    x = rng.integers(-7, 8, (M, K)).astype(np.float32)
+    y = _qgemm.quantized_matmul(hip(x), hip(packed), hip(s), hip(b), True, gs, bits).numpy()
+    assert np.array_equal(y.astype(np.float64), x.astype(np.float64) @ W.dequantize(packed, s, b, gs, bits).astype(np.float64).T)
+
+
+@pytest.mark.parametrize("M,N,K,gs,bits", SMALL_BATCH_FORMS)
 def test_small_batch_forms_against_float64(M, N, K, gs, bits):
     rng = np.random.default_rng(N)
     w = (rng.standard_normal((N, K)) * 0.05).astype(np.float32)
@@ -91,10 +107,11 @@ def test_small_batch_forms_against_float64(M, N, K, gs, bits):
     # products are exact; a float32 sum of K / 32 of them per lane chain, then K / gs groups and K / 512 slabs: a few 2^-24
     # of the root mean square for each, and the decoded weight of the reference is itself rounded (2^-24 each).  4-bit codes
     # of whole windows enter as 128 + c: a group's sum is then up to 136 / 7.5 = 18 times as large as what is left of it, and
-    # with x > 0 it grows with gs where the rest grows with its root (11 at 128): 200 times the error.
-    loose = 200 if bits == 4 and K % 128 == 0 else 1
+    # with x > 0 it grows with gs where the rest grows with its root (11 at 128): up to 200 times the error.  Rounding errors of
+    # that size do not all point the same way: half of that (5.6e-5 measured, 2.4e-4 at most; 2.3e-7 and 1.1e-6 for the others).
+    loose = 100 if bits == 4 and K % 128 == 0 else 1
     assert np.linalg.norm(y - ref) <= loose * 1e-6 * np.linalg.norm(ref)
-    assert np.abs(y - ref).max() <= loose * 2e-5 * np.sqrt(np.mean(ref ** 2))
+    assert np.abs(y - ref).max() <= loose * 1e-5 * np.sqrt(np.mean(ref ** 2))
 
 
 @pytest.mark.parametrize("M,N,K,gs,bits", [
