@@ -40,11 +40,13 @@
 // after kSpinLimit reads a wavefront gives up for the rest of the sequence.  It is out of step with the others then, and the ring may
 // hold any step of theirs, so its sums are NaN from there on, and with them all that the block computes and hands out.
 //
-// hidden 512, 16 rows, a step of 2.2 us (5100 cycles, timestamps): 450 before the first read, 1850 for the 32 KiB of h a
-// CU reads past its L2 (1000 at hidden 128), 1390 splits and products, 70 barrier, 1000 sums and gates.  Two such layers of
-// 64 steps take 170 us; 272 when h was read from y's rows (every line twice), the input loads stood between h and its
-// products, and one set of wavefronts took both products.  Placing a group's blocks on one XCD and exchanging through its L2 instead
-// measured 150 against 153 us for one layer: not worth the placement.
+// hidden 512, 512 inputs, 16 rows, 64 steps: the kernel takes 157 us, 2.45 per step (1.9 at hidden 256, 1.56 at 128).  Of a step's
+// 5700 cycles (timestamps) 780 pass before the first read, 1650 with the 32 KiB of h that a CU reads past its L2 (940 at hidden
+// 128), 2040 in splits and products, 80 at the barrier, 1130 with sums and gates.  A second such layer adds 11 us (168): two steps,
+// and what its input wavefronts wait for on each of the others, y of the layer below, which they read row by row.  It was 272 when h
+// was read from y's rows too (every line twice), the input loads stood between h and its products, and one set of wavefronts took
+// both products.  Placing a group's blocks on one XCD and exchanging through its L2 instead measured 150 against 153 us for one
+// layer (sums in one chain then): not worth the placement.
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -388,7 +390,8 @@ void lstm_sequence_kernel(LstmArgs p) {
             const unsigned slot = unsigned((s - 1) % kSlots) * slot_bytes;
             // A read that meets the writes of the same line delays both, and one that comes too early costs a whole trip
             // more: the first is issued when most of h has arrived.  Steps of hidden 512 / 256 / 128, 16 rows, in us: at
-            // once 2.75 / 2.05 / 1.6, after 448 cycles 2.25 / 1.7 / 1.5, after 576 2.2 / 1.7 / 1.45, after 896 2.3 / 1.8 / 1.55.
+            // once 2.75 / 2.05 / 1.6, after 448 cycles 2.25 / 1.7 / 1.5, after 576 2.2 / 1.7 / 1.45, after 896 2.3 / 1.8 / 1.55
+            // (sums and gates of then; now 64 cycles either way are within 2 %, and 128 late costs 1 to 2 %).
             if (gridDim.x > 16) __builtin_amdgcn_s_sleep(8);
             else __builtin_amdgcn_s_sleep(5);
             unsigned missing = present;
@@ -560,11 +563,13 @@ constexpr int kMaxFused = 512;  // hidden and input columns of a form that takes
 constexpr int kMaxHidden = 1024;
 
 // A step of all rows: one launch of the recurrence per rows that fit the device, or a float32 GEMM and a gate kernel
-// (lq_lstm_cell_f32) on decoded weights, issued from Python.  Measured, us per step of both: hidden 64, 8192 rows 25.7 /
-// 32.9; 128, 4096 rows 25.6 / 35.4, 8192 rows 46.9 / 47.2; 256, 1024 rows 29.6 / 37.4, 2048 rows 57.9 / 43.1; 512, 512
-// rows 37 / 49, 1024 rows 73 / 56; 768, 128 rows 41 / 58, 256 rows 80 / 60; 1024, 128 rows 46 / 71, 256 rows 89 / 73,
-// 4096 rows 1399 / 289; 1024 in two directions, 16 rows 15 / 130, 256 rows 180 / 146.  The estimates are within 20 % of those; steps have become
-// 1.1 to 1.6 times as fast since, so that what is left to the GEMM on the line is within as much of the better one.
+// (lq_lstm_cell_f32) on decoded weights, issued from Python.  Measured, us per step of both: hidden 64, 8192 rows 19.0 /
+// 23.6; 128, 4096 rows 19.7 / 25.8, 8192 rows 45.6 / 35.4; 256, 1024 rows 19.0 / 28.7, 1500 rows 28.0 / 31.0, 2048 rows 39.5 /
+// 34.0; 512, 512 rows 27.2 / 41.3, 768 rows 40.3 / 43.4, 1024 rows 54.8 / 45.2; 768, 128 rows 25.4 / 51.8, 256 rows 50.5 / 53.6,
+// 384 rows 76.0 / 54.6; 1024, 128 rows 26.6 / 64.8, 256 rows 54.2 / 66.6, 384 rows 80.9 / 67.7; 1024 in two directions, 256 rows
+// 111 / 131.  The estimates below are those of an earlier recurrence, a fifth to two thirds above these (a launch's step is 2.4 up
+// to hidden 256, 3.3 beyond), and 3 to 17 % above for the GEMM.  So the line lies low: of the sizes here hidden 256 with 1500 rows,
+// 512 with 768, 768 and 1024 with 256 go to the GEMM for 6 to 23 % more.
 double sequence_step_us(int hidden) { return 2.9 + 0.0026 * hidden; }
 double gemm_step_us(int batch, int hidden) {
     const double least = 17.0 + 0.05 * hidden, rows = batch * (2.8e-5 * hidden + 3.8e-8 * hidden * hidden);
@@ -597,9 +602,11 @@ int lq_lstm_fused_layers(int steps, int batch, int inputs, int hidden, int layer
     LQ_REQUIRE(directions == 1 || directions == 2, LQ_ERR_VALUE, "lstm_fused_layers: directions must be 1 or 2");
     *fused = 0;
     if (steps == 0 || batch == 0 || hidden > kMaxFused || inputs > kMaxFused) return LQ_OK;
-    // Costs per layer in steps of the recurrence.  An input product in a GEMM of its own, with the decoded
-    // weight it reads, is worth twelve (43 us at 1024 x 2048 x 512, a step 3.4 then; 20 x 33 rows of 200 -> 300 in two
-    // directions, where a step is 2: 61 us with the GEMMs, about 120 as three launches without).
+    // Costs per layer in steps of the recurrence.  An input product in a GEMM of its own, with the decoded weight it reads, is worth
+    // twelve and, where inputs and hidden are 512, up to 24.  us of the device with the GEMM / with more launches: 512 -> 512, 64
+    // rows, 16 steps 111 / 101, 24 139 / 139, 32 167 / 174; 256 -> 256, 128 rows, 16 steps 78 / 76, 24 97 / 106; 128 -> 512, 64
+    // rows, 12 steps 76 / 76; 128 -> 128, 400 rows, 12 steps 58 / 51, 24 86 / 89; 200 -> 300 in two directions, 33 rows, 10 steps
+    // 98 / 88, 20 135 / 154.
     constexpr long kGemm = 12;
     LstmSplit s;
     int rc = with_form(hidden, 0, [&](auto w, auto k, auto xw, auto x) { return split_lstm<w(), k(), xw(), x()>(batch, hidden, directions, false, &s); });

@@ -697,7 +697,7 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 // launch.  That is quick where all blocks are resident, and kExchange of them are a sixteenth of the device, less than the
 // share of one of the hardware queues that streams have (exchange_blocks).  Nothing depends on it: kernels of other processes,
 // or a stream that may not use every CU, can keep a block out for any time, so a block that has read a slot kExchangePolls
-// times without finding a range (about 3 ms) takes the range of x itself - the same minimum and maximum -, ends, and makes room.
+// times without finding a range (a few milliseconds) takes the range of x itself - the same minimum and maximum -, ends, and makes room.
 //
 // Beyond, and under capture (slots cleared inside a graph are unset until its replay), two launches: slices'
 // ranges (minmax_seg_kernel), then this kernel with PARTS - every block reduces
