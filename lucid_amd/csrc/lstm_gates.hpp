@@ -7,9 +7,10 @@ namespace lq {
 // They are on the chain of a step of the recurrence, so both are straight-line code (the library's expf and tanhf branch, and both
 // sides run in a wavefront).  Against float64, 4 M points of each range, largest error in units of the last place and relative root
 // mean square, in brackets 1 / (1 + expf(-x)) and tanhf:
-//   sigmoid  -10 .. 10    @A       tanh  -0.7 .. 0.7  1.25 (1.37)  2.8e-8 (2.9e-8)
-//            -60 .. -10   @B             -10 .. 10    1.19 (1.37)  1.88e-8 (1.93e-8)
-//            -110 .. -60  @C (beyond -88.7 the library's is 0)
+//   sigmoid  -10 .. 10    2.02 (2.18)  3.1e-8 (3.8e-8)       tanh  -0.7 .. 0.7  1.25 (1.37)  2.8e-8 (2.9e-8)
+//            -60 .. -10   1.64 (2.61)  2.9e-8 (3.7e-8)             -10 .. 10    1.19 (1.37)  1.88e-8 (1.93e-8)
+//            -110 .. -60  0.89 (1.78 to -87; beyond -88.7 the library's is 0)
+// Without the reduction to a whole and a fraction the exponential alone takes sigmoid to 2.77.
 
 constexpr float kLog2e = 1.44269502f, kLog2eLow = 1.92596299e-8f, kLn2 = 0.693147182f;
 

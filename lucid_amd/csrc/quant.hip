@@ -1526,7 +1526,8 @@ int lq_quantize_tensor_dynamic_polls_i8(const float* x, size_t rows, unsigned co
                                         int qmax, int is_signed, float eps, int code_offset, float* scale, float* zp,
                                         float* mn_out, float* mx_out, int8_t* q, int polls, lq_stream stream) {
     LQ_REQUIRE(scale && zp && x && q, LQ_ERR_VALUE, "quantize_tensor_dynamic: NULL pointer");
-    LQ_REQUIRE(rows > 0 && cols > 0 && ld >= cols && (ld == cols || ld % 4 == 0) && rows <= (size_t(1) << 32) / ld,
+    LQ_REQUIRE(rows > 0 && cols > 0 && ld >= cols && (ld == cols || ld % 4 == 0) && ld <= 0x7fffffffu &&
+                   rows <= (size_t(1) << 32) / ld,
                LQ_ERR_SHAPE, "quantize_tensor_dynamic: %zu rows of %u elements and %u codes", rows, cols, ld);
     LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
                "quantize_tensor_dynamic: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
