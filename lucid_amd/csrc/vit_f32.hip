@@ -638,8 +638,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restric
 }
 
 // ---------------------------------------------------------------- attention
-// One block per (batch, head); one wavefront per 16 queries; head dim 64, at
-// most 208 tokens.  qkv is the packed activation [B, T, 3, H, 64] of the qkv
+// Head dim 64, at most 208 tokens.  qkv is the packed activation [B, T, 3, H, 64] of the qkv
 // Linear; out is [B, T, H*64].
 //
 // float32 operands on the bfloat16 matrix instruction.  A float32 is the exact sum of three
@@ -650,10 +649,20 @@ __global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restric
 // v_mfma_f32_16x16x32_bf16 runs sixteen times the rate of v_mfma_f32_16x16x4_f32: six
 // instructions of the one replace eight of the other at a sixth of the time each.
 //
-// The three parts of K (row-major) and of V^T ([column][key]) are both in LDS from the start -
-// 79 872 + 81 408 bytes of the CU's 160 KiB - so after the one barrier that follows the splits
-// a wavefront runs scores, softmax and P . V on its own, and the 13 wavefronts (four on one
-// SIMD, three on the others) drift apart instead of waiting for each other between phases.
+// A head's queries are dealt to `parts` blocks of four wavefronts; a wavefront takes up to QT
+// tiles of 16 queries and reads each fragment of K and V once for all of them.  The three parts
+// of K, and after the scores those of V^T in their place, are the block's 80 KB of LDS, so that
+// two blocks share a CU.  What is read from memory is requested a phase ahead (V under the scores,
+// the next head's K and queries under the products with V), fragments a step ahead, and the
+// exponentials and splits of the probabilities are issued between the products with V.
+//
+// Bound by the matrix pipe and the vector unit together: of the about 36 000 cycles that two blocks of
+// a CU take for a head of 197 tokens, the products are 16 800 of every SIMD, splits, exponentials and
+// LDS writes about as much, and at 64 x 12 heads the power limit holds the clock near 1.7 GHz.
+// 12 heads of 197 tokens 18.3 -> 10.5 us, 96 heads 20.1 -> 16.3, 384 46.4 -> 34.5, 768 77.4 -> 67.6
+// against one block of 16 wavefronts per head with K and V side by side (all K and V fragments read
+// once per 16 queries, the softmax a phase of its own).  The same eight wavefronts on a whole head with
+// K and V side by side (one split for all queries): 65.1 at 768 heads, but 41.5 against 32.5 at 288.
 //
 // Per wavefront: S^T = K . Q^T as 13 tiles of 16 keys x 16 queries (accumulators stay in
 // registers), softmax over the keys of each query (a lane holds 52 of a query's keys, the other
@@ -662,286 +671,366 @@ __global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restric
 // a lane the eight k slots of an instruction, which is a valid k-slice assignment as long as V
 // is read with the same one ([column][key] keeps a lane's four keys of a tile in 8 contiguous
 // bytes); the thirteenth tile goes through the 16-key form of the instruction alone.
-constexpr int AT_D = 64, AT_TMAX = 208;
-// K: rows of 64 bfloat16 = 128 bytes = all 32 banks; the 16-byte chunk k of row r sits at chunk
-// k ^ (r % 8), so the 16 rows of a fragment (same logical chunk) cover every bank exactly twice
-constexpr int AT_PART_K = AT_TMAX * AT_D;
+constexpr int AT_D = 64, AT_TMAX = 208, AT_NT = AT_TMAX / 16, AT_WAVES = 4;
+// K: rows of 64 bfloat16 = 128 bytes = half of the 64 banks; the 16-byte chunk k of row r sits at chunk
+// k ^ (r / 2 % 8), so the 16 rows of a fragment (same logical chunk) cover every bank once.
 // V^T: 106 dwords per row = 10 mod 32: the 16 rows a fragment reads (8 bytes each) fall on 16
 // different bank pairs
 constexpr int AT_VLD = AT_TMAX + 4;
-constexpr int AT_PART_V = AT_D * AT_VLD;  // elements of one part
-constexpr size_t AT_K_BYTES = size_t(3) * AT_PART_K * 2;
-constexpr size_t AT_SMEM = AT_K_BYTES + size_t(3) * AT_PART_V * 2;
-static_assert(AT_SMEM + 1024 <= 160 * 1024, "LDS of a CU, with the range reduction's few words");
+constexpr int AT_PART_K = AT_TMAX * AT_D, AT_PART_V = AT_D * AT_VLD;  // elements of one part
+constexpr size_t AT_SMEM = size_t(3) * (AT_PART_V > AT_PART_K ? AT_PART_V : AT_PART_K) * 2;
+static_assert(2 * (AT_SMEM + 192) <= 160 * 1024, "two blocks per CU, with the range reduction's few words");
 
 typedef __bf16 at_v8bf __attribute__((ext_vector_type(8)));
 typedef short at_v4s __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int at_k_index(int row, int col) {  // col a multiple of 4
-    return row * AT_D + ((((col >> 3) ^ (row & 7)) << 3) | (col & 7));
+    return row * AT_D + ((((col >> 3) ^ (row >> 1 & 7)) << 3) | (col & 7));
+}
+// V^T's row of a column: tile j of the output is columns 4 i + j, i = 0..15, so that a lane has four consecutive floats of a
+// query at the end
+__device__ __forceinline__ int at_v_index(int j, int i, int key) { return (16 * j + i) * AT_VLD + key; }
+// f over the four lanes of one number in the four rows of 16 lanes; every lane gets it
+template <class F>
+__device__ __forceinline__ float at_rows4(float v, F f) {
+    auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = f(__uint_as_float(x[0]), __uint_as_float(x[1]));
+    x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return f(__uint_as_float(x[0]), __uint_as_float(x[1]));
 }
 
-// acc += a * b from the parts, smallest terms first
-__device__ __forceinline__ v4f at_mma6(const uint4 (&a)[3], const uint4 (&b)[3], v4f acc) {
-    auto mm = [&](const uint4& x, const uint4& y) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_v8bf, x), __builtin_bit_cast(at_v8bf, y), acc,
-                                                      0, 0, 0);
-    };
-    mm(a[1], b[1]);
-    mm(a[0], b[2]);
-    mm(a[2], b[0]);
-    mm(a[0], b[1]);
-    mm(a[1], b[0]);
-    mm(a[0], b[0]);
-    return acc;
+// acc[q] += a[q] . b from the parts, smallest terms first.  16 bytes a lane: 32 k slots; 8 bytes: 16.
+constexpr int kAtPa[6] = {1, 0, 2, 0, 1, 0}, kAtPb[6] = {1, 2, 0, 1, 0, 0};
+__device__ __forceinline__ v4f at_mm(const uint4& x, const uint4& y, v4f acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(at_v8bf, x), __builtin_bit_cast(at_v8bf, y), acc, 0,
+                                                   0, 0);
 }
-// the same over 16 k slots (four per lane)
-__device__ __forceinline__ v4f at_mma6_k16(const uint2 (&a)[3], const uint2 (&b)[3], v4f acc) {
-    auto mm = [&](const uint2& x, const uint2& y) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(at_v4s, x), __builtin_bit_cast(at_v4s, y), acc,
-                                                        0, 0, 0);
-    };
-    mm(a[1], b[1]);
-    mm(a[0], b[2]);
-    mm(a[2], b[0]);
-    mm(a[0], b[1]);
-    mm(a[1], b[0]);
-    mm(a[0], b[0]);
-    return acc;
+__device__ __forceinline__ v4f at_mm(const uint2& x, const uint2& y, v4f acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(at_v4s, x), __builtin_bit_cast(at_v4s, y), acc, 0,
+                                                     0, 0);
 }
 
-__global__ __launch_bounds__(1024) void attention_kernel(const float* __restrict__ qkv, float* __restrict__ out,
-                                                        int B, int T, int H, float scale, float* range) {
-    extern __shared__ __attribute__((aligned(16))) uint16_t at_smem[];
-    uint16_t* const k_lds = at_smem;
-    uint16_t* const v_lds = at_smem + 3 * AT_PART_K;
-    const int b = blockIdx.x / H, h = blockIdx.x % H;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// WIDE: offsets within 32 token rows take more than 32 bits
+template <int QT, bool WIDE>
+__global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float* __restrict__ qkv,
+                                                                     float* __restrict__ out, int T, int H, int heads,
+                                                                     int parts, int out_vec, float scale,
+                                                                     float* range) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t at_smem[];  // K's parts, then V^T's
+    constexpr int THREADS = 64 * AT_WAVES, ROW4 = AT_D / 4;
+    constexpr int KP = AT_TMAX * ROW4 / THREADS;  // 16-byte pieces of K per thread: one of every 16 rows
+    constexpr int VP = (AT_TMAX + 31) / 32;       // pairs of such pieces of V: one of every 32 rows
+    static_assert(AT_TMAX * ROW4 % THREADS == 0 && THREADS / ROW4 == 16 && AT_D == 64, "");
     const size_t tok_stride = size_t(3) * H * AT_D;
-    const float* base = qkv + size_t(b) * T * tok_stride + size_t(h) * AT_D;
-    // K and V are requested before anything is used (a block of 13 wavefronts holds all of both: four
-    // 16-byte pieces of each per thread).  A thread's V pieces are two pairs of consecutive keys at the
-    // same four columns: V^T keeps a column's keys contiguous, so a pair of keys is one dword of each part
-    constexpr int kPieces = AT_TMAX * (AT_D / 4), kHeld = 4;
-    constexpr int kPairs = (AT_TMAX / 2) * (AT_D / 4);
-    float4 kheld[kHeld], vheld[kHeld];
-#pragma unroll
-    for (int u = 0; u < kHeld; ++u) {
-        const int i = tid + u * int(blockDim.x), row = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
-        kheld[u] = float4{0.f, 0.f, 0.f, 0.f};
-        if (i < kPieces && row < T) kheld[u] = *reinterpret_cast<const float4*>(base + size_t(row) * tok_stride + size_t(H) * AT_D + c4);
-    }
-#pragma unroll
-    for (int u = 0; u < kHeld; ++u) {
-        const int i = tid + (u >> 1) * int(blockDim.x), row = 2 * (i / (AT_D / 4)) + (u & 1), c4 = (i % (AT_D / 4)) * 4;
-        vheld[u] = float4{0.f, 0.f, 0.f, 0.f};
-        if (i < kPairs && row < T) vheld[u] = *reinterpret_cast<const float4*>(base + size_t(row) * tok_stride + size_t(2) * H * AT_D + c4);
-    }
-    // One wavefront per tile of 16 queries.  With 4 n + 1 tiles one SIMD would hold a wavefront more
-    // than the others and everybody would wait for it: the launch then has three more wavefronts,
-    // and the last tile's four each compute its scores but only one 16-column tile of its output.
+    using Offset = std::conditional_t<WIDE, size_t, unsigned>;
+    const Offset row_bytes = Offset(tok_stride) * 4u;
     const int tiles = (T + 15) / 16;
-    const bool shared_last = int(blockDim.x) > tiles * 64;
-    const int q0 = (wave < tiles ? wave : tiles - 1) * 16;
-    const int only_j = (shared_last && wave >= tiles - 1) ? wave - (tiles - 1) : -1;  // wavefront-uniform
-    const int g = lane >> 4, c = lane & 15;
-    // the lane's slice of its query row: Q[q0 + c][32 u + 8 g + 0..7]
-    float4 qheld[2 * (AT_D / 32)];
-    {
-        const int q = q0 + c;
-        const float* qp = base + size_t(q < T ? q : T - 1) * tok_stride;
-#pragma unroll
-        for (int u = 0; u < AT_D / 32; ++u) {
-            qheld[2 * u] = *reinterpret_cast<const float4*>(qp + 32 * u + 8 * g);
-            qheld[2 * u + 1] = *reinterpret_cast<const float4*>(qp + 32 * u + 8 * g + 4);
-        }
-    }
-    // K rows into LDS as three bfloat16 parts (rows past T are zero)
-    auto place_k = [&](int i, float4 kv) {
-        const int row = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
-        uint32_t lo[3], hi[3];
-        at_split3x2(kv.x, kv.y, lo[0], lo[1], lo[2]);
-        at_split3x2(kv.z, kv.w, hi[0], hi[1], hi[2]);
-        const int at = at_k_index(row, c4);
-#pragma unroll
-        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(k_lds + p * AT_PART_K + at) = uint2{lo[p], hi[p]};
+    // Blocks are dealt to the 8 XCDs in turn: the parts of a head follow each other on one of them, where
+    // the second finds the first one's K and V in the L2.
+    const int items = (heads + 7) / 8 * 8 * parts;
+    float4 kheld[KP], qheld[QT][2 * (AT_D / 32)];
+    // Four floats of token row row0 + r (row0 the same in the whole wavefront; past the last token: a row of the
+    // tokens there are - such a key's probability is 0, such a query is not stored), as a scalar base and
+    // an offset per lane.
+    auto fetch = [&](const float* head_base, int which, int row0, int r, int col) {
+        const int rb = row0 < T ? row0 : 0;
+        const float* p = head_base + size_t(rb) * tok_stride + size_t(which) * H * AT_D;
+        const Offset off = (rb + r < T ? Offset(r) * row_bytes : Offset(0)) + Offset(col) * 4u;
+        return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(p) + off);
     };
+    struct Item {
+        const float* base;
+        int head, t0, nq;  // this wavefront's queries are tiles t0 .. t0 + nq - 1
+    };
+    auto item_of = [&](int item, int wave_id) {
+        Item it;
+        const int part = item / 8 % parts;
+        it.head = item / (8 * parts) * 8 + item % 8;
+        const int b = it.head / H;
+        it.base = qkv + size_t(b) * T * tok_stride + size_t(it.head - b * H) * AT_D;
+        // Tiles [first, end) are the part's.  Which wavefronts get fewer than QT changes from block to block: those of
+        // one number mostly share a SIMD.
+        const int first = tiles * part / parts, n = tiles * (part + 1) / parts - first;
+        const int wave = (wave_id + item / 8) % AT_WAVES;
+        it.t0 = first + n * wave / AT_WAVES;
+        it.nq = first + n * (wave + 1) / AT_WAVES - it.t0;
+        return it;
+    };
+    // piece x of what a wavefront has of an item before its scores: K, then the lane's slice of its query rows
+    // (Q[16 tile + c][32 u + 8 g + 0..7])
+    constexpr int PIECES = KP + QT * 2 * (AT_D / 32);
+    auto request = [&](const Item& it, int x, int tid) {
+        if (x < KP) {
+            kheld[x] = fetch(it.base, 1, x * (THREADS / ROW4), tid / ROW4, tid % ROW4 * 4);
+        } else {
+            const int q = (x - KP) / 4, e = (x - KP) % 4, lane = tid & 63;
+            qheld[q][e] = fetch(it.base, 0, (it.t0 + q) * 16, lane & 15, 32 * (e / 2) + 8 * (lane >> 4) + 4 * (e % 2));
+        }
+    };
+    const int wave_id = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+    int next = blockIdx.x;
+    while (next < items && item_of(next, 0).head >= heads) next += gridDim.x;
+    if (next < items) {
+        const Item it = item_of(next, wave_id);
 #pragma unroll
-    for (int u = 0; u < kHeld; ++u) {
-        const int i = tid + u * int(blockDim.x);
-        if (i < kPieces) place_k(i, kheld[u]);
+        for (int x = 0; x < PIECES; ++x) request(it, x, threadIdx.x);
     }
-    for (int i = tid + kHeld * int(blockDim.x); i < kPieces; i += blockDim.x) {  // fewer than 13 wavefronts
-        const int row = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
-        float4 kv = {0.f, 0.f, 0.f, 0.f};
-        if (row < T) kv = *reinterpret_cast<const float4*>(base + size_t(row) * tok_stride + size_t(H) * AT_D + c4);
-        place_k(i, kv);
-    }
-    // V^T's parts: keys 2 pair and 2 pair + 1 at columns c4 .. c4 + 3 (keys past T are zero)
-    auto place_v = [&](int i, float4 v0, float4 v1) {
-        const int pair = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
-        const float a[4] = {v0.x, v0.y, v0.z, v0.w}, bb[4] = {v1.x, v1.y, v1.z, v1.w};
+    while (next < items) {
+        const Item it = item_of(next, wave_id);
+        do next += gridDim.x;
+        while (next < items && item_of(next, 0).head >= heads);
+        // behind the last item it is requested again, rather than leaving the registers' old values alive through the loop
+        const Item after = next < items ? item_of(next, wave_id) : it;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // what follows from the lane is computed per item: kept across items, it would be spilled
+        const int lane = tid & 63, g = lane >> 4, c = lane & 15;
+        // K rows into LDS as three bfloat16 parts
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            uint32_t d[3];
-            at_split3x2(a[e], bb[e], d[0], d[1], d[2]);
+        for (int u = 0; u < KP; ++u) {
+            const int i = tid + u * THREADS, row = i / ROW4, c4 = (i % ROW4) * 4;
+            uint32_t d0[3], d1[3];
+            at_split3x2(kheld[u].x, kheld[u].y, d0[0], d0[1], d0[2]);
+            at_split3x2(kheld[u].z, kheld[u].w, d1[0], d1[1], d1[2]);
 #pragma unroll
             for (int p = 0; p < 3; ++p)
-                *reinterpret_cast<uint32_t*>(v_lds + p * AT_PART_V + (c4 + e) * AT_VLD + 2 * pair) = d[p];
+                *reinterpret_cast<uint2*>(at_smem + p * AT_PART_K + at_k_index(row, c4)) = uint2{d0[p], d1[p]};
         }
-    };
-#pragma unroll
-    for (int u = 0; u < kHeld / 2; ++u) {
-        const int i = tid + u * int(blockDim.x);
-        if (i < kPairs) place_v(i, vheld[2 * u], vheld[2 * u + 1]);
-    }
-    for (int i = tid + (kHeld / 2) * int(blockDim.x); i < kPairs; i += blockDim.x) {  // fewer than 13 wavefronts
-        const int pair = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
-        float4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = {0.f, 0.f, 0.f, 0.f};
-        const float* vp = base + size_t(2) * H * AT_D + c4;
-        if (2 * pair < T) v0 = *reinterpret_cast<const float4*>(vp + size_t(2 * pair) * tok_stride);
-        if (2 * pair + 1 < T) v1 = *reinterpret_cast<const float4*>(vp + size_t(2 * pair + 1) * tok_stride);
-        place_v(i, v0, v1);
-    }
-    // B operand of S^T, pre-scaled so that S = scale * log2(e) * Q.K^T (the scores are kept in the
-    // base-2 domain, so that the softmax numerators are one v_exp_f32 each)
-    uint4 qf[AT_D / 32][3];
-    {
+        // B operand of S^T, pre-scaled so that S = scale * log2(e) * Q.K^T (the scores are kept in the
+        // base-2 domain, so that the softmax numerators are one v_exp_f32 each)
+        uint4 qf[QT][AT_D / 32][3];
         const float qs = scale * 1.4426950408889634f;
 #pragma unroll
-        for (int u = 0; u < AT_D / 32; ++u) {
-            const float4 a = qheld[2 * u], bq = qheld[2 * u + 1];
-            const float v[8] = {a.x * qs, a.y * qs, a.z * qs, a.w * qs, bq.x * qs, bq.y * qs, bq.z * qs, bq.w * qs};
-            uint32_t d[3][4];
+        for (int q = 0; q < QT; ++q)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) at_split3x2(v[2 * e], v[2 * e + 1], d[0][e], d[1][e], d[2][e]);
+            for (int u = 0; u < AT_D / 32; ++u) {
+                const float4 a = qheld[q][2 * u], bq = qheld[q][2 * u + 1];
+                const float v[8] = {a.x * qs, a.y * qs, a.z * qs, a.w * qs, bq.x * qs, bq.y * qs, bq.z * qs, bq.w * qs};
+                uint32_t d[3][4];
 #pragma unroll
-            for (int p = 0; p < 3; ++p) qf[u][p] = uint4{d[p][0], d[p][1], d[p][2], d[p][3]};
-        }
-    }
-    __syncthreads();  // the only one before the range reduction: from here on a wavefront is on its own
-    constexpr int NT = AT_TMAX / 16;
-    v4f st[NT];
+                for (int e = 0; e < 4; ++e) at_split3x2(v[2 * e], v[2 * e + 1], d[0][e], d[1][e], d[2][e]);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) st[t] = v4f{0.f, 0.f, 0.f, 0.f};
-    // k slice outermost: the 13 tiles' accumulators are independent chains
-#pragma unroll
-    for (int u = 0; u < AT_D / 32; ++u)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            uint4 kf[3];
-            const int at = at_k_index(16 * t + c, 32 * u + 8 * g);
-#pragma unroll
-            for (int p = 0; p < 3; ++p) kf[p] = *reinterpret_cast<const uint4*>(k_lds + p * AT_PART_K + at);
-            st[t] = at_mma6(kf, qf[u], st[t]);
-        }
-    // st[t][r] = S[query q0 + c][key 16t + 4g + r]
-    float mx = -__builtin_inff();
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int key = 16 * t + 4 * g + r;
-            if (key >= T) st[t][r] = -__builtin_inff();
-            mx = fmaxf(mx, st[t][r]);
-        }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    float sum = 0.0f;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float e = __builtin_amdgcn_exp2f(st[t][r] - mx);  // 2^(-inf) = 0 for the padded keys
-            st[t][r] = e;
-            sum += e;
-        }
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
-    const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
-
-    // O[q][n] = sum_key P[q][key] V[key][n], four 16-wide column tiles; tile j of the output holds
-    // head-dim columns 16 j + c: the 16 lanes of a fragment read consecutive V^T rows (rows 4 c + j,
-    // which would let a lane store four consecutive floats, fall on four bank pairs only)
-    static_assert(NT % 2 == 1, "tile pairs and one single tile");
-    v4f o[AT_D / 16];
-#pragma unroll
-    for (int j = 0; j < AT_D / 16; ++j) o[j] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int tp = 0; tp < NT / 2; ++tp) {
-        // the eight k slots of this lane: keys 32 tp + 4 g + 0..3 and 32 tp + 16 + 4 g + 0..3
-        float pv[8];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            pv[r] = st[2 * tp][r] * inv;
-            pv[4 + r] = st[2 * tp + 1][r] * inv;
-        }
-        uint32_t d[3][4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) at_split3x2(pv[2 * e], pv[2 * e + 1], d[0][e], d[1][e], d[2][e]);
-        uint4 pf[3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p) pf[p] = uint4{d[p][0], d[p][1], d[p][2], d[p][3]};
-#pragma unroll
-        for (int j = 0; j < AT_D / 16; ++j) {
-            if (only_j >= 0 && only_j != j) continue;
-            uint4 vf[3];
-#pragma unroll
-            for (int p = 0; p < 3; ++p) {
-                const uint16_t* vrow = v_lds + p * AT_PART_V + (16 * j + c) * AT_VLD + 32 * tp + 4 * g;
-                const uint2 lo = *reinterpret_cast<const uint2*>(vrow), hi = *reinterpret_cast<const uint2*>(vrow + 16);
-                vf[p] = uint4{lo.x, lo.y, hi.x, hi.y};
+                for (int p = 0; p < 3; ++p) qf[q][u][p] = uint4{d[p][0], d[p][1], d[p][2], d[p][3]};
             }
-            o[j] = at_mma6(pf, vf, o[j]);
+        __syncthreads();  // K is in LDS
+        // Pairs of consecutive keys of V at the same four columns (V^T keeps a column's keys contiguous, so a pair of
+        // keys is one dword of each part).  Four lanes cover 64 bytes of a row and 16 pairs follow each other, so that
+        // the dwords of a write fall on all banks evenly.
+        const int vpair = tid / 4 % 16, vcol = (tid / 64 * 4 + tid % 4) * 4;
+        float4 vheld[VP][2];
+        auto request_v = [&](int u, int e) { vheld[u][e] = fetch(it.base, 2, 32 * u, 2 * vpair + e, vcol); };
+        // st[q][t][r] = S[query 16 (t0 + q) + c][key 16t + 4g + r]
+        v4f st[QT][AT_NT];
+#pragma unroll
+        for (int q = 0; q < QT; ++q)
+#pragma unroll
+            for (int t = 0; t < AT_NT; ++t) st[q][t] = v4f{0.f, 0.f, 0.f, 0.f};
+        // A step is a tile of keys and half of the head's columns; the next step's fragments are read ahead of its
+        // products.  V is requested a piece per step when half of the queries' fragments are done with.
+        auto scores = [&](auto n) {
+            constexpr int NQ = decltype(n)::value, STEPS = AT_NT * (AT_D / 32);
+            uint4 kf[2][3];
+            auto read = [&](int s) {
+                const int at = at_k_index(16 * (s % AT_NT) + c, 32 * (s / AT_NT) + 8 * g);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) kf[s & 1][p] = *reinterpret_cast<const uint4*>(at_smem + p * AT_PART_K + at);
+            };
+            read(0);
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                const int u = s / AT_NT, t = s % AT_NT;
+                if (s + 1 < STEPS) read(s + 1);
+                if (s >= AT_NT) request_v((s - AT_NT) / 2, (s - AT_NT) % 2);
+                if (s == STEPS - 1) request_v(VP - 1, 1);
+#pragma unroll
+                for (int x = 0; x < 6; ++x)
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) st[q][t] = at_mm(kf[s & 1][kAtPa[x]], qf[q][u][kAtPb[x]], st[q][t]);
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);  // the reads first
+                __builtin_amdgcn_sched_group_barrier(0x008, 6 * NQ, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        if (QT == 2 && it.nq == 2)
+            scores(std::integral_constant<int, QT>{});
+        else if (it.nq > 0)
+            scores(std::integral_constant<int, 1>{});
+        else
+#pragma unroll
+            for (int u = 0; u < 2 * VP; ++u) request_v(u / 2, u % 2);
+        static_assert(AT_NT == 2 * VP - 1, "a piece of V per step, two in the last");
+        __syncthreads();  // nobody reads K any more
+#pragma unroll
+        for (int u = 0; u < VP; ++u) {
+            if (32 * u + 32 > AT_TMAX && 32 * u + 2 * vpair >= AT_TMAX) continue;
+            const float4 v0 = vheld[u][0], v1 = vheld[u][1];
+            const float a[4] = {v0.x, v0.y, v0.z, v0.w}, bb[4] = {v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t d[3];
+                at_split3x2(a[e], bb[e], d[0], d[1], d[2]);
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    *reinterpret_cast<uint32_t*>(at_smem + p * AT_PART_V + at_v_index(e, vcol / 4, 32 * u + 2 * vpair)) = d[p];
+            }
         }
-    }
-    {
-        // the last tile: keys 16 (NT - 1) + 4 g + 0..3, four k slots per lane
-        float pv[4];
+        float mx[QT], sum[QT][4];  // four sums of every fourth key each: shorter chains round less
+        auto mask = [&](int t) {  // keys past the last token
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pv[r] = st[NT - 1][r] * inv;
-        uint32_t d[3][2];
+            for (int q = 0; q < QT; ++q)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) at_split3x2(pv[2 * e], pv[2 * e + 1], d[0][e], d[1][e], d[2][e]);
-        uint2 pf[3];
+                for (int r = 0; r < 4; ++r)
+                    if (16 * t + 4 * g + r >= T) st[q][t][r] = -__builtin_inff();
+        };
+        mask(AT_NT - 1);
+        if (T <= 16 * (AT_NT - 1)) {
 #pragma unroll
-        for (int p = 0; p < 3; ++p) pf[p] = uint2{d[p][0], d[p][1]};
-#pragma unroll
-        for (int j = 0; j < AT_D / 16; ++j) {
-            if (only_j >= 0 && only_j != j) continue;
-            uint2 vf[3];
-#pragma unroll
-            for (int p = 0; p < 3; ++p)
-                vf[p] = *reinterpret_cast<const uint2*>(v_lds + p * AT_PART_V + (16 * j + c) * AT_VLD + 16 * (NT - 1) + 4 * g);
-            o[j] = at_mma6_k16(pf, vf, o[j]);
+            for (int t = 0; t < AT_NT - 1; ++t) mask(t);
         }
-    }
-    // result layout of the 16x16 MFMA: column slot = lane % 16, row = 4*(lane/16) + r; the 16 lanes
-    // of a row store 64 consecutive bytes
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int q = q0 + 4 * g + r;
-        if (q < T) {
-            float* orow = out + (size_t(b) * T + q) * (size_t(H) * AT_D) + size_t(h) * AT_D + c;
+        for (int q = 0; q < QT; ++q) {
+            mx[q] = -__builtin_inff(), sum[q][0] = sum[q][1] = sum[q][2] = sum[q][3] = 0.0f;
 #pragma unroll
-            for (int j = 0; j < AT_D / 16; ++j)
-                if (only_j < 0 || only_j == j) orow[16 * j] = o[j][r];
+            for (int t = 0; t < AT_NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mx[q] = __builtin_elementwise_maximum(mx[q], st[q][t][r]);
+            mx[q] = at_rows4(mx[q], [](float a, float b) { return __builtin_elementwise_maximum(a, b); });
         }
-    }
-    if (range) {
-        float lo = __builtin_inff(), hi = -__builtin_inff();
-        int nan = 0;
+        __syncthreads();  // V^T is in LDS
+
+        // O[q][n] = sum_key P[q][key] V[key][n] with P = 2^(S - max), divided by P's sum at the end, in four tiles of 16
+        // columns
+        static_assert(AT_NT % 2 == 1, "tile pairs and one single tile");
+        constexpr int NJ = AT_D / 16;
+        v4f o[QT][NJ];
 #pragma unroll
-        for (int j = 0; j < AT_D / 16; ++j)
+        for (int q = 0; q < QT; ++q)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (q0 + 4 * g + r < T && (only_j < 0 || only_j == j)) {
-                    nan |= (o[j][r] != o[j][r]);
-                    lo = fminf(lo, o[j][r]);
-                    hi = fmaxf(hi, o[j][r]);
+            for (int j = 0; j < NJ; ++j) o[q][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        auto values = [&](auto n) {
+            constexpr int NQ = decltype(n)::value, PAIRS = AT_NT / 2;
+            // Parts of the probabilities of tiles 2 tp and 2 tp + 1: the eight k slots of this lane are keys
+            // 32 tp + 4 g + 0..3 and 32 tp + 16 + 4 g + 0..3.  Pair e is slots 2 e and 2 e + 1.
+            uint32_t pd[2][NQ][3][4];
+            auto probs = [&](int tp, int q, int e) {
+                const int t = 2 * tp + e / 2, r = e % 2 * 2;
+                const float a = __builtin_amdgcn_exp2f(st[q][t][r] - mx[q]);  // 2^(-inf) = 0 for the padded keys
+                const float b = __builtin_amdgcn_exp2f(st[q][t][r + 1] - mx[q]);
+                sum[q][r] += a;
+                sum[q][r + 1] += b;
+                auto& d = pd[tp & 1][q];
+                at_split3x2(a, b, d[0][e], d[1][e], d[2][e]);
+            };
+            uint4 vf[2][3];
+            auto read = [&](int s) {
+#pragma unroll
+                for (int p = 0; p < 3; ++p) {
+                    const uint16_t* vpart = at_smem + p * AT_PART_V;
+                    const int key = 32 * (s / NJ) + 4 * g;
+                    const uint2 x = *reinterpret_cast<const uint2*>(vpart + at_v_index(s % NJ, c, key));
+                    uint2 y = {0, 0};
+                    if (s / NJ < PAIRS) y = *reinterpret_cast<const uint2*>(vpart + at_v_index(s % NJ, c, key + 16));
+                    vf[s & 1][p] = uint4{x.x, x.y, y.x, y.y};
                 }
-        range_block_store(range, lo, hi, nan);
+            };
+            read(0);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) probs(0, q, e);
+            // a step is a pair of key tiles and 16 columns; under its products the vector unit makes a fourth of the
+            // next pair's probabilities, and the last steps request the next item
+#pragma unroll
+            for (int s = 0; s < PAIRS * NJ; ++s) {
+                const int tp = s / NJ, j = s % NJ;
+                read(s + 1);
+                constexpr int FROM = PAIRS * NJ * 3 / 4, N = PAIRS * NJ - FROM;
+                if (QT == 2 && s >= FROM) {
+#pragma unroll
+                    for (int x = (s - FROM) * PIECES / N; x < (s - FROM + 1) * PIECES / N; ++x) request(after, x, tid);
+                }
+#pragma unroll
+                for (int q = 0; q < NQ; ++q)
+                    if (tp + 1 < PAIRS || j < 2) probs(tp + 1, q, j);
+#pragma unroll
+                for (int x = 0; x < 6; ++x)
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) {
+                        const auto& d = pd[tp & 1][q][kAtPa[x]];
+                        o[q][j] = at_mm(uint4{d[0], d[1], d[2], d[3]}, vf[s & 1][kAtPb[x]], o[q][j]);
+                    }
+                __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+                for (int x = 0; x < 6 * NQ; ++x) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x402, 3, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the last tile: keys 16 (AT_NT - 1) + 4 g + 0..3, four k slots per lane
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int s = PAIRS * NJ + j;
+                if (j + 1 < NJ) read(s + 1);
+#pragma unroll
+                for (int x = 0; x < 6; ++x)
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) {
+                        const auto& d = pd[PAIRS & 1][q][kAtPa[x]];
+                        const uint4& v = vf[s & 1][kAtPb[x]];
+                        o[q][j] = at_mm(uint2{d[0], d[1]}, uint2{v.x, v.y}, o[q][j]);
+                    }
+            }
+        };
+        if (QT == 2 && it.nq == 2)
+            values(std::integral_constant<int, QT>{});
+        else if (it.nq > 0)
+            values(std::integral_constant<int, 1>{});
+        else if (QT == 2)
+#pragma unroll
+            for (int x = 0; x < PIECES; ++x) request(after, x, tid);
+        if (QT == 1) {  // mostly one item per block: nothing to request
+#pragma unroll
+            for (int x = 0; x < KP; ++x) kheld[x] = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int x = 0; x < 2 * (AT_D / 32); ++x) qheld[0][x] = float4{0.f, 0.f, 0.f, 0.f};
+            if (next < items) {
+#pragma unroll
+                for (int x = 0; x < PIECES; ++x) request(after, x, tid);
+            }
+        }
+        // result layout of the 16x16 MFMA: column slot = lane % 16, row = 4*(lane/16) + r; the 16 lanes
+        // of a row store 256 consecutive bytes
+        const int b = it.head / H, h = it.head - b * H;
+#pragma unroll
+        for (int q = 0; q < QT; ++q) {
+            if (q >= it.nq) continue;
+            const float total = at_rows4((sum[q][0] + sum[q][1]) + (sum[q][2] + sum[q][3]), [](float a, float b) { return a + b; });
+            const float inv = total > 0.0f ? 1.0f / total : 0.0f;
+            const int row0 = (it.t0 + q) * 16;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float by = __shfl(inv, 4 * g + r, 64);  // of query row0 + 4 g + r
+                const int row = row0 + 4 * g + r;
+                if (row < T) {
+                    float v[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) {
+                        v[j] = o[q][j][r] * by;
+                        lo = __builtin_elementwise_minimum(lo, v[j]);  // a NaN stays
+                        hi = __builtin_elementwise_maximum(hi, v[j]);
+                    }
+                    float* at = out + (size_t(b) * T + row) * (size_t(H) * AT_D) + size_t(h) * AT_D + 4 * c;
+                    if (out_vec)
+                        *reinterpret_cast<float4*>(at) = float4{v[0], v[1], v[2], v[3]};
+                    else
+                        at[0] = v[0], at[1] = v[1], at[2] = v[2], at[3] = v[3];
+                }
+            }
+        }
+        __syncthreads();  // V^T has been read: the next item's K may be written
     }
+    if (range) range_block_store(range, lo, hi, lo != lo);
 }
 
 unsigned blocks_for(size_t n) { return unsigned((n + 255) / 256); }
@@ -1141,13 +1230,30 @@ int lq_attention_f32(const float* qkv, float* out, int B, int T, int H, int D, f
     if (B == 0) return LQ_OK;
     LQ_REQUIRE(range == nullptr || long(B) * H <= kRangeSlots, LQ_ERR_SHAPE,
                "attention: too many (batch, head) pairs for a kept range");
-    const int tiles = (T + 15) / 16;
-    const int waves = tiles + ((tiles > 1 && tiles % 4 == 1) ? 3 : 0);  // see the kernel: the last tile shared by four
-    constexpr size_t kSmem = AT_SMEM;
-    static DeviceOnce attr_once;
-    if (int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(attention_kernel), int(kSmem))) return rc;
-    attention_kernel<<<unsigned(B) * H, waves * 64, kSmem, as_stream(stream)>>>(qkv, out, B, T, H, scale,
-                                                                                 range);
+    const int heads = B * H, tiles = (T + 15) / 16;
+    const auto launch = [&](auto qt, auto wide) -> int {
+        constexpr int QT = decltype(qt)::value;
+        const auto kernel = attention_kernel<QT, decltype(wide)::value>;
+        static DeviceOnce attr_once;
+        if (int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(kernel), int(AT_SMEM))) return rc;
+        const int parts = (tiles + QT * AT_WAVES - 1) / (QT * AT_WAVES);
+        const long items = (long(heads) + 7) / 8 * 8 * parts;
+        constexpr long kSlots = 512;  // two blocks on each of 256 CUs, which take further items in turn
+        kernel<<<unsigned(items < kSlots ? items : kSlots), 64 * AT_WAVES, AT_SMEM, as_stream(stream)>>>(
+            qkv, out, T, H, heads, parts, aligned16(out), scale, range);
+        return LQ_OK;
+    };
+    // One tile of queries per wavefront while the blocks do not outnumber the CUs (12 heads of 197 tokens 10.5 us against
+    // 14.7 with two); beyond that they would only share them (96 heads: 16.3 either way, 288: 34.7 against 32.2).
+    using One = std::integral_constant<int, 1>;
+    int rc;
+    if (size_t(H) * 3 * AT_D * 4 * 32 > UINT32_MAX)
+        rc = launch(One{}, std::true_type{});
+    else if (heads <= 64)
+        rc = launch(One{}, std::false_type{});
+    else
+        rc = launch(std::integral_constant<int, 2>{}, std::false_type{});
+    if (rc) return rc;
     LQ_CHECK_LAUNCH();
     return LQ_OK;
 }
