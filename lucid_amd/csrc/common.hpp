@@ -110,22 +110,21 @@ __device__ __forceinline__ void lds_barrier() {
 
 __host__ __device__ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// erf for the GELU kernels: Abramowitz & Stegun 7.1.26, |error| <= 1.5e-7 (the rational
-// term through v_rcp_f32, the Gaussian through v_exp_f32), 13 instructions where the
-// library erff takes about 45 with both of its branches live in a wavefront.  The GELU
-// it feeds, 0.5 x (1 + erf(x / sqrt 2)), is within 1e-6 of the exactly rounded one for
-// every x (the error peaks for |x| < 4.2; beyond |x| = 5.6 the result is x or 0 exactly
-// as with erff).  Not for erf on its own near 0: 1 - p e cancels there.
-__device__ __forceinline__ float erf_as(float v) {
-    const float z = __builtin_fabsf(v);
-    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3275911f, z, 1.0f));
-    float p = __builtin_fmaf(1.061405429f, t, -1.453152027f);
-    p = __builtin_fmaf(p, t, 1.421413741f);
-    p = __builtin_fmaf(p, t, -0.284496736f);
-    p = __builtin_fmaf(p, t, 0.254829592f);
+// GELU in its erf form, 0.5 x (1 + erf(x / sqrt 2)) (lucid/nn/functional/activations.py:219), erf by Abramowitz & Stegun
+// 7.1.26, |error| <= 1.5e-7: with t = 1 / (1 + 0.3275911 |x| / sqrt 2), 1 - erf(|x| / sqrt 2) is P(t) e^(-x^2 / 2), so that
+// the value is 0.5 x + |x| (0.5 - 0.5 P(t) e^(-x^2 / 2)).  The constants carry the halves and the 1 / sqrt 2: 13 instructions,
+// two of them v_rcp_f32 and v_exp_f32, where erf on its own and the product around it take 16.  Within 1e-6 of the exactly
+// rounded value for every x; x or 0 (from -0.5 |x| + 0.5 |x|) beyond |x| = 5.6; +inf gives +inf, -inf and a NaN give NaN.
+__device__ __forceinline__ float gelu_erf(float x) {
+    const float z = __builtin_fabsf(x);
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3275911f * 0.70710678118654752440f, z, 1.0f));
+    float p = __builtin_fmaf(0.5f * 1.061405429f, t, 0.5f * -1.453152027f);
+    p = __builtin_fmaf(p, t, 0.5f * 1.421413741f);
+    p = __builtin_fmaf(p, t, 0.5f * -0.284496736f);
+    p = __builtin_fmaf(p, t, 0.5f * 0.254829592f);
     p = p * t;
-    const float e = __builtin_amdgcn_exp2f((z * z) * -1.4426950408889634f);
-    return __builtin_copysignf(__builtin_fmaf(-p, e, 1.0f), v);
+    const float e = __builtin_amdgcn_exp2f((x * x) * (0.5f * -1.4426950408889634f));
+    return __builtin_fmaf(z, __builtin_fmaf(-p, e, 0.5f), 0.5f * x);
 }
 
 }  // namespace lq

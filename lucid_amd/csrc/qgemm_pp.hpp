@@ -141,16 +141,11 @@ __device__ __forceinline__ int pp_rotation(const GemmArgs& g, int wn0) {
 template <int TM, int TN, int MODE>
 __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM][TN], const float (&as_row)[TM],
                                             const float* s_ws, const float* s_bias, const int32_t* s_corr, int n0,
-                                            int wm0, int wn0, int lane, int rot, float& r_lo, float& r_hi, int& r_nan) {
+                                            int wm0, int wn0, int lane, int rot, RangeKeep& kept) {
     if (wm0 >= g.M || wn0 >= g.N) return;
     // running range of what this lane stores (float32 output with a kept range only)
     const bool keep = MODE == OUT_F32X && g.range != nullptr;
-    auto track = [&](uint32_t bits) {
-        const float y = __uint_as_float(bits);
-        r_nan |= (y != y);
-        r_lo = fminf(r_lo, y);
-        r_hi = fmaxf(r_hi, y);
-    };
+    auto track = [&](uint32_t bits) { kept.add(__uint_as_float(bits)); };
     float S = 1.0f, Z = 0.0f;
     constexpr bool kRequant = MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN || MODE == OUT_FAKEQUANT_F32;
     if (kRequant) {
@@ -163,7 +158,8 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
     const CodePack cpk = make_code_pack<MODE>(g, MODE == OUT_REQUANT_JOIN ? jp.out : G);
     constexpr int esize = MODE == OUT_F16 ? 2 : ((MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) ? 1 : 4);
     constexpr bool kFloatOut = MODE == OUT_F32 || MODE == OUT_F16 || MODE == OUT_F32X;
-    const bool prescaled = (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) && !g.a_scale_per_row;
+    const EpilogueForm form = kFloatOut ? epilogue_form(g) : kFormAny;
+    const bool prescaled = (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN || form != kFormAny) && !g.a_scale_per_row;
     const bool cols_in = wn0 + TN * 16 <= g.N, rows_in = wm0 + TM * 16 <= g.M;
     // uniform: every access of this wavefront may be a whole aligned vector
     const bool vec_out = cols_in && g.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(g.out) % (4 * esize) == 0 &&
@@ -306,11 +302,18 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
     // values of one tile in the lane's own layout, residual / join applied; (ri, rj): the tile's
     // place among the wavefront's accumulators
     auto tile_values = [&](int m, const pp_v4i& a, const ColParams (&c4)[4], float as, int nq, uint4& v, int ri, int rj) {
-        if (prescaled) {
-            v.x = epilogue_value<MODE, true>(g, a[0], 1.0f, c4[0], G);
-            v.y = epilogue_value<MODE, true>(g, a[1], 1.0f, c4[1], G);
-            v.z = epilogue_value<MODE, true>(g, a[2], 1.0f, c4[2], G);
-            v.w = epilogue_value<MODE, true>(g, a[3], 1.0f, c4[3], G);
+        auto one_scale = [&](auto f) {
+            v.x = epilogue_value<MODE, true, decltype(f)::value>(g, a[0], 1.0f, c4[0], G);
+            v.y = epilogue_value<MODE, true, decltype(f)::value>(g, a[1], 1.0f, c4[1], G);
+            v.z = epilogue_value<MODE, true, decltype(f)::value>(g, a[2], 1.0f, c4[2], G);
+            v.w = epilogue_value<MODE, true, decltype(f)::value>(g, a[3], 1.0f, c4[3], G);
+        };
+        if (prescaled && kFloatOut && form == kFormPlain) {
+            one_scale(std::integral_constant<EpilogueForm, kFormPlain>{});
+        } else if (prescaled && MODE == OUT_F32X) {
+            one_scale(std::integral_constant<EpilogueForm, kFormGelu>{});
+        } else if (prescaled && !kFloatOut) {
+            one_scale(std::integral_constant<EpilogueForm, kFormAny>{});
         } else {
             v.x = epilogue_value<MODE, false>(g, a[0], as, c4[0], G);
             v.y = epilogue_value<MODE, false>(g, a[1], as, c4[1], G);
@@ -601,12 +604,11 @@ __global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(2,
     // ---- epilogue: no staging through LDS and no barrier; group 0 runs it while group 1 still
     // issues its last MFMAs.
     __builtin_amdgcn_s_waitcnt(pp_vmcnt_imm(0));  // no direct load may land in LDS after this wavefront has ended
-    float r_lo = __builtin_inff(), r_hi = -__builtin_inff();
-    int r_nan = 0;
-    pp_epilogue<TM, TN, MODE>(g, acc, as_row, s_ws, s_bias, s_corr, n0, wm0, wn0, lane, rot, r_lo, r_hi, r_nan);
+    RangeKeep kept;
+    pp_epilogue<TM, TN, MODE>(g, acc, as_row, s_ws, s_bias, s_corr, n0, wm0, wn0, lane, rot, kept);
     // one block per tile: the block's slot is the tile's (every wavefront has passed the same
     // number of barriers by now)
-    if (MODE == OUT_F32X && g.range != nullptr) range_block_store(g.range, r_lo, r_hi, r_nan);
+    if (MODE == OUT_F32X && g.range != nullptr) kept.store(g.range);
 }
 
 template <class Cfg, int MODE>

@@ -97,7 +97,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                                               const ColParams (&cp)[Cfg::TN], const float* s_as,
                                               uint32_t* stage, int m0, int n0, int n_limit, int wm,
                                               int wn, int lane, float S, float Z, bool interior,
-                                              bool prescaled, float& r_lo, float& r_hi, int& r_nan) {
+                                              bool prescaled, RangeKeep& kept) {
     constexpr int TM = Cfg::TM, TN = Cfg::TN, STRIDE = Cfg::STAGE_STRIDE;
     constexpr int QUADS_PER_ROW = TN * 8;            // four-column groups per staged row
     constexpr int EPI_ROWS = Cfg::EPI_ROWS;          // rows staged at a time (32 or 16)
@@ -119,12 +119,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
     const CodePack cpk = make_code_pack<MODE>(g, MODE == OUT_REQUANT_JOIN ? jp.out : G);
     // running range of what this lane stores (float32 output with a kept range only)
     const bool keep = MODE == OUT_F32X && g.range != nullptr;
-    auto track = [&](uint32_t bits) {
-        const float y = __uint_as_float(bits);
-        r_nan |= (y != y);
-        r_lo = fminf(r_lo, y);
-        r_hi = fmaxf(r_hi, y);
-    };
+    auto track = [&](uint32_t bits) { kept.add(__uint_as_float(bits)); };
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -153,6 +148,8 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
             }
             // this lane's rows of the part: groups of four consecutive rows
             if (prescaled) {
+                // a float form comes here without a ReLU and with a GELU exactly in OUT_F32X (run_epilogue)
+                constexpr EpilogueForm kForm = MODE == OUT_F32X ? kFormGelu : (kFloatOut ? kFormPlain : kFormAny);
 #pragma unroll
                 for (int rr = 0; rr < RPP; ++rr) {
                     const int r = part * RPP + rr;
@@ -160,7 +157,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
                         stage[row * STRIDE + j * 32 + (lane & 31)] =
-                            epilogue_value<MODE, true>(g, acc[i][j][r], 1.0f, cp[j], G);
+                            epilogue_value<MODE, true, kForm>(g, acc[i][j][r], 1.0f, cp[j], G);
                 }
             } else {
                 float as[RPP];
@@ -636,21 +633,22 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
                               (g.join_q == nullptr ||
                                (g.join_ld % 4 == 0 && reinterpret_cast<uintptr_t>(g.join_q) % 4 == 0));
         __syncthreads();
-        float r_lo = __builtin_inff(), r_hi = -__builtin_inff();
-        int r_nan = 0;
+        RangeKeep kept;
         // one activation scale for all rows (always so for a convolution): the kernels that
-        // write codes fold it into the column scales (as * ws, the product every element would
-        // form) and save each element that multiplication
-        const bool prescaled = (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) && (CONV || !g.a_scale_per_row);
+        // write codes, and the float forms without a ReLU, fold it into the column scales (as * ws, the product
+        // every element would form) and save each element that multiplication
+        constexpr EpilogueForm kLean = MODE == OUT_F32X ? kFormGelu : kFormPlain;
+        const bool lean = (MODE == OUT_F32 || MODE == OUT_F16 || MODE == OUT_F32X) && epilogue_form(g) == kLean;
+        const bool prescaled = (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN || lean) && (CONV || !g.a_scale_per_row);
         if (prescaled) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) cp[j].ws = as_mine * cp[j].ws;
         }
         tile_epilogue<Cfg, MODE>(g, acc, cp, s_as, stage, m0, n0, n_limit, wm, wn, lane, S, Z, interior, prescaled,
-                                 r_lo, r_hi, r_nan);
+                                 kept);
         __syncthreads();  // the staging area is the next tile's first LDS stage
         // one block per tile here (the launcher sees to it), so the block's slot is the tile's
-        if (MODE == OUT_F32X && !SK && g.range != nullptr) range_block_store(g.range, r_lo, r_hi, r_nan);
+        if (MODE == OUT_F32X && !SK && g.range != nullptr) kept.store(g.range);
     };
 
     if (!SK) {

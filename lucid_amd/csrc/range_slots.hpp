@@ -31,6 +31,17 @@ __device__ __forceinline__ void range_block_store(float* range, float lo, float 
     }
 }
 
+// The range a lane keeps of what it writes: IEEE 754-2019 minimum / maximum, which a NaN passes through (one
+// v_minimum3_f32 / v_maximum3_f32 per two values; fminf / fmaxf beside a NaN flag take five instructions per value).
+struct RangeKeep {
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+    __device__ __forceinline__ void add(float y) {
+        lo = __builtin_elementwise_minimum(lo, y);
+        hi = __builtin_elementwise_maximum(hi, y);
+    }
+    __device__ __forceinline__ void store(float* range) const { range_block_store(range, lo, hi, lo != lo); }
+};
+
 // The range itself, for every thread of a block (up to 1024; all must call it): the reduction of the slots.
 __device__ __forceinline__ void range_block_load(const float* __restrict__ range, float& mn, float& mx) {
     const unsigned n = reinterpret_cast<const unsigned*>(range)[0];

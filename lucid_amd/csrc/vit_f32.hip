@@ -47,13 +47,8 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const bool vec = (cols % 4 == 0) && aligned16(x) && aligned16(out) && aligned16(gamma) && aligned16(beta);
     const float inv_n = 1.0f / float(cols);
-    float lo = __builtin_inff(), hi = -__builtin_inff();
-    int nan = 0;
-    auto track = [&](float y) {
-        nan |= (y != y);
-        lo = fminf(lo, y);
-        hi = fmaxf(hi, y);
-    };
+    RangeKeep kept;
+    auto track = [&](float y) { kept.add(y); };
     for (int rr = 0; rr < LN_ROWS_PER_WAVE; ++rr) {
         const long row = (long(blockIdx.x) * 4 + wave) * LN_ROWS_PER_WAVE + rr;
         if (row >= rows) break;
@@ -145,7 +140,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
             }
         }
     }
-    if (range) range_block_store(range, lo, hi, nan);
+    if (range) kept.store(range);
 }
 
 // LayerNorm feeding a dynamic quantizer without ever storing its float32 output: the first
@@ -161,13 +156,8 @@ __global__ __launch_bounds__(256) void layernorm_stats_kernel(const float* __res
                                                               float eps, float* __restrict__ stats, float* range) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const float inv_n = 1.0f / float(cols);
-    float lo = __builtin_inff(), hi = -__builtin_inff();
-    int nan = 0;
-    auto track = [&](float y) {
-        nan |= (y != y);
-        lo = fminf(lo, y);
-        hi = fmaxf(hi, y);
-    };
+    RangeKeep kept;
+    auto track = [&](float y) { kept.add(y); };
     const long row = long(blockIdx.x) * 4 + wave;
     if (row < rows) {
         const float* xr = x + row * cols;
@@ -213,7 +203,7 @@ __global__ __launch_bounds__(256) void layernorm_stats_kernel(const float* __res
             }
         }
     }
-    range_block_store(range, lo, hi, nan);
+    kept.store(range);
 }
 
 // four codes of normalized values
@@ -275,23 +265,14 @@ __global__ __launch_bounds__(256) void layernorm_quantize_kernel(const float* __
 }
 
 // ---------------------------------------------------------------- elementwise
-__device__ __forceinline__ float gelu_erf(float x) {
-    return (0.5f * x) * (1.0f + lq::erf_as(x * 0.70710678118654752440f));
-}
-
 // Four float4 per thread (block-strided, so each access of a wavefront is
 // contiguous); the optional range costs one partial slot per block.
 constexpr int GELU_PER_THREAD = 4;
 
 __global__ __launch_bounds__(256) void gelu_kernel(const float* __restrict__ x, float* __restrict__ out,
                                                    size_t n, int vec, float* range) {
-    float lo = __builtin_inff(), hi = -__builtin_inff();
-    int nan = 0;
-    auto track = [&](float y) {
-        nan |= (y != y);
-        lo = fminf(lo, y);
-        hi = fmaxf(hi, y);
-    };
+    RangeKeep kept;
+    auto track = [&](float y) { kept.add(y); };
     const size_t base = size_t(blockIdx.x) * (256 * GELU_PER_THREAD) + threadIdx.x;
     if (vec) {
         float4 v[GELU_PER_THREAD];
@@ -320,7 +301,7 @@ __global__ __launch_bounds__(256) void gelu_kernel(const float* __restrict__ x, 
             }
         }
     }
-    if (range) range_block_store(range, lo, hi, nan);
+    if (range) kept.store(range);
 }
 
 // dst[r, :] = src[r * src_row_stride : r * src_row_stride + cols]
@@ -768,7 +749,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
         }
     };
     const int wave_id = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
-    float lo = __builtin_inff(), hi = -__builtin_inff();
+    RangeKeep kept;
     int next = blockIdx.x;
     while (next < items && item_of(next, 0).head >= heads) next += gridDim.x;
     if (next < items) {
@@ -1017,8 +998,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
                         v[j] = o[q][j][r] * by;
-                        lo = __builtin_elementwise_minimum(lo, v[j]);  // a NaN stays
-                        hi = __builtin_elementwise_maximum(hi, v[j]);
+                        kept.add(v[j]);
                     }
                     float* at = out + (size_t(b) * T + row) * (size_t(H) * AT_D) + size_t(h) * AT_D + 4 * c;
                     if (out_vec)
@@ -1030,7 +1010,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
         }
         __syncthreads();  // V^T has been read: the next item's K may be written
     }
-    if (range) range_block_store(range, lo, hi, lo != lo);
+    if (range) kept.store(range);
 }
 
 unsigned blocks_for(size_t n) { return unsigned((n + 255) / 256); }

@@ -604,6 +604,47 @@ def test_ping_pong_kernel_gelu_and_kept_range(cfg, M, N, K):
     assert np.isnan(mn) and np.isnan(mx)
 
 
+@pytest.mark.parametrize("cfg", [1, 2, 3, 4, 5, 7, 9, 10, 11, 14, 22])
+@pytest.mark.parametrize("per_row", [False, True])
+def test_float_epilogues_with_and_without_relu_and_gelu(cfg, per_row):
+    """Every combination of ReLU, GELU, kept range and residual in the float output forms, which the kernels sort into forms
+    of their own loops: the bits of the plain product (checked against the oracle), then ReLU, the stand-alone GELU and the
+    sum.  Ragged sizes and sizes of whole tiles."""
+    import lucid_amd.nn.functional as F
+    for M, N, K in ((512, 512, 256), (300, 277, 128)):
+        rng = np.random.default_rng(cfg + M)
+        a, w = codes(rng, (M, K), -100, 100), codes(rng, (N, K), -100, 100)
+        ad, wd = hip(a), hip(w)
+        a_scale = rng.uniform(0.002, 0.01, M if per_row else 1).astype(np.float32)
+        w_scale = rng.uniform(0.0005, 0.004, N).astype(np.float32)
+        bias, res = (rng.standard_normal(s).astype(np.float32) for s in (N, (M, N)))
+        kw = dict(a_zp=5, a_scale=hip(a_scale), w_scale=hip(w_scale), wsum=_ops.rowsum_i8(wd), bias=hip(bias),
+                  out_mode=_ops.OUT_F32, path=TILE, tile_config=cfg)
+        plain = O.qlinear(a, w, 5, a_scale, w_scale, bias=bias, out_mode=O.OUT_F32)
+        for relu in (False, True):
+            for gelu in (False, True):
+                for keep in (False, True):
+                    for residual in (None, res):
+                        y = np.maximum(plain, 0) if relu else plain
+                        y = F.gelu(hip(y)).numpy() if gelu else y
+                        y = y + residual if residual is not None else y
+                        rb = hip(np.zeros(_range_words(), np.float32)) if keep else None
+                        got = _ops.qlinear_i8(ad, wd, relu=relu, gelu=gelu, range_buf=rb,
+                                              residual=hip(residual) if residual is not None else None, **kw).numpy()
+                        assert np.array_equal(got, y), (M, relu, gelu, keep, residual is not None)
+                        if keep:
+                            n, r = int(rb.numpy()[:1].view(np.uint32)[0]), rb.numpy()
+                            slots = (len(r) - 4) // 2
+                            assert r[4:4 + n].min() == y.min() and r[4 + slots:4 + slots + n].max() == y.max()
+        half = _ops.qlinear_i8(ad, wd, **{**kw, "out_mode": _ops.OUT_F16}).numpy()
+        assert np.array_equal(half, O.qlinear(a, w, 5, a_scale, w_scale, bias=bias, out_mode=O.OUT_F16))
+
+
+def _range_words():
+    from lucid_amd import _C
+    return _C.range_buffer_words()
+
+
 # ------------------------------------------------------------------ affine weight codes
 AFFINE_CASES = [
     # M, N, K, path

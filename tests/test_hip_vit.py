@@ -50,6 +50,17 @@ def test_gelu_and_add(n):
     assert np.array_equal(F.add(hip(x), hip(y)).numpy(), x + y)
 
 
+def test_gelu_against_float64():
+    """erf by a formula good to 1.5e-7, in float32: 4e-7 absolute at most (measured 3.8e-7), 1.5e-7 relative overall."""
+    from scipy.special import erf
+    x = np.concatenate([np.linspace(-12, 12, 1 << 20), np.random.default_rng(0).standard_normal(1 << 20)]).astype(np.float32)
+    d = x.astype(np.float64)
+    exp, got = 0.5 * d * (1 + erf(d / np.sqrt(2))), F.gelu(hip(x)).numpy()
+    assert np.max(np.abs(got - exp)) <= 4e-7 and rel(got, exp) <= 1.5e-7
+    edge = F.gelu(hip(np.array([np.inf, -np.inf, np.nan, 0, 3e38, -3e38], np.float32))).numpy()
+    assert edge[0] == np.inf and np.isnan(edge[1:3]).all() and (edge[3:] == np.array([0, 3e38, 0], np.float32)).all()
+
+
 @pytest.mark.parametrize("B,T,H", [(2, 197, 12), (1, 1, 1), (3, 16, 2), (2, 17, 3), (1, 208, 2), (4, 50, 12),
                                    (2, 70, 3), (1, 130, 2), (1, 193, 1), (2, 144, 2)])   # 5, 9, 13 tiles: the last one shared
 def test_attention_on_packed_qkv(B, T, H):
