@@ -166,11 +166,7 @@ __global__ __launch_bounds__(256) void qconv_few_kernel(GemmArgs g, FewGeom q) {
                     for (int r = 0; r < 4; ++r) c4[r].ws = as * c4[r].ws;
                 }
                 const fv4i a = acc[j];
-                uint4 v;
-                v.x = epilogue_value<MODE, prescaled>(g, a[0], prescaled ? 1.0f : as, c4[0], G);
-                v.y = epilogue_value<MODE, prescaled>(g, a[1], prescaled ? 1.0f : as, c4[1], G);
-                v.z = epilogue_value<MODE, prescaled>(g, a[2], prescaled ? 1.0f : as, c4[2], G);
-                v.w = epilogue_value<MODE, prescaled>(g, a[3], prescaled ? 1.0f : as, c4[3], G);
+                const uint4 v = epilogue_quad<MODE, prescaled>(g, a, prescaled ? 1.0f : as, c4, G);
                 if (vec_out) {
                     if (MODE == OUT_REQUANT_I8)
                         codes[j] = few_pack_codes(v, cpk);

@@ -228,18 +228,7 @@ __global__ __launch_bounds__(256, 2) void qconv_halo_kernel(GemmArgs g, HaloGeom
         for (int i = 0; i < TI; ++i) {
             if (m_row[i] < 0) continue;
             const hv4i a = acc[i][j];
-            uint4 v;
-            if (prescaled) {
-                v.x = epilogue_value<MODE, true>(g, a[0], 1.0f, c4[0], G);
-                v.y = epilogue_value<MODE, true>(g, a[1], 1.0f, c4[1], G);
-                v.z = epilogue_value<MODE, true>(g, a[2], 1.0f, c4[2], G);
-                v.w = epilogue_value<MODE, true>(g, a[3], 1.0f, c4[3], G);
-            } else {
-                v.x = epilogue_value<MODE, false>(g, a[0], as, c4[0], G);
-                v.y = epilogue_value<MODE, false>(g, a[1], as, c4[1], G);
-                v.z = epilogue_value<MODE, false>(g, a[2], as, c4[2], G);
-                v.w = epilogue_value<MODE, false>(g, a[3], as, c4[3], G);
-            }
+            const uint4 v = prescaled ? epilogue_quad<MODE, true>(g, a, 1.0f, c4, G) : epilogue_quad<MODE, false>(g, a, as, c4, G);
             const size_t idx = size_t(m_row[i]) * size_t(g.ldo) + size_t(nq);
             if (vec_out) {
                 store_vec4<MODE>(g, idx, v, cpk);

@@ -85,6 +85,7 @@ struct QGrid {
     float s, inv, z, lo, hi;  // z, lo, hi include `bias`
     float lof;       // lower bound of the multiplying route: max(lo, z) under a ReLU, else lo
     float loc, hic;  // lof - z and hi - z: the bounds of a code taken relative to z
+    float guard;     // what the multiplying route vouches for: distances of x * inv to its integer below this
     float bias;      // 0, or 128 for a signed range: codes come out as code + bias, in 0..255
     bool in_byte;    // ... so that four of them pack with v_cvt_pk_u8_f32 (see CodePack)
     bool relu;
@@ -118,6 +119,7 @@ __device__ __forceinline__ QGrid make_qgrid(float s, float z, float lo, float hi
     G.inv = ok ? 1.0f / s : __builtin_nanf("");
     G.lof = (relu && z > lo) ? z : lo;
     G.loc = G.lof - z, G.hic = hi - z;
+    G.guard = (lo <= z && z <= hi && hi - lo <= 255.0f) ? 0.5f - 0x1p-14f : 0.5f - 0x1p-12f;
     return G;
 }
 
@@ -130,31 +132,50 @@ __device__ __forceinline__ QGrid make_qgrid(float s, float z, float lo, float hi
 // 2^-24.  rint only changes value at the half-integers.
 //  * |tp| < 512: tp is within 6.2e-5 of e and fl(x / s) within 3.1e-5; when tp is farther
 //    than 2^-12 = 2.4e-4 from every half-integer, both lie strictly between the same two of
-//    them and round to the same integer.
-//  * 512 <= |tp| < inf, with d passing the test: both rint(tp) and rint(fl(x / s)) are
-//    beyond +-511 with the same sign, and with |z|, |lo|, |hi| <= 255 both clamp to the
+//    them and round to the same integer.  Where z lies within the bounds and these at most 255 apart (any
+//    grid of 8-bit codes), what |tp| >= 256.5 rounds to is clamped, and up to there the two are within 3.3e-5 and 1.6e-5:
+//    2^-14 = 6.1e-5 suffices.
+//  * 512 (256.5) <= |tp| < inf, with d passing the test: both rint(tp) and rint(fl(x / s)) are
+//    beyond +-511 (255) with the same sign, and with |z|, |lo|, |hi| <= 255 (z within the bounds) both clamp to the
 //    same bound.
-// Otherwise (a few elements in ten thousand, and whatever is infinite or NaN: d = NaN
+// Otherwise (one element in ten thousand, and whatever is infinite or NaN: d = NaN
 // fails the test) the lane divides.
+// N elements share the test, so that their chains of a dozen dependent instructions overlap: with a branch per
+// element a wavefront runs them one after the other.  (Four: any more divide too often - 3 % of the groups of a
+// wavefront have an element near a half - and with the wider guard, 12 %, four were slower than one.)
+template <bool KEEP_NAN, bool CENTERED = false, int N>
+__device__ __forceinline__ void quant_fast(const float (&x)[N], const QGrid& G, float (&c)[N]) {
+    float far = 0.0f;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const float tp = x[k] * G.inv;
+        const float r = __builtin_rintf(tp);
+        const float d = tp - r;  // exact where it matters
+        far = k == 0 ? __builtin_fabsf(d) : __builtin_elementwise_maximum(far, __builtin_fabsf(d));  // a NaN stays
+        c[k] = CENTERED ? __builtin_amdgcn_fmed3f(r, G.loc, G.hic) : __builtin_amdgcn_fmed3f(r + G.z, G.lof, G.hi);
+    }
+    if (__builtin_expect(!(far < G.guard), 0)) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const float xr = (G.relu && x[k] < 0.0f) ? 0.0f : x[k];
+            const float u = __builtin_rintf(xr / G.s) + G.z;
+            c[k] = (u != u) ? (KEEP_NAN ? u : G.bias) : __builtin_amdgcn_fmed3f(u, G.lo, G.hi);
+            if (CENTERED) c[k] = c[k] - G.z;
+        }
+    }
+}
 template <bool KEEP_NAN, bool CENTERED = false>
 __device__ __forceinline__ float quant_fast(float x, const QGrid& G) {
-    const float tp = x * G.inv;
-    const float r = __builtin_rintf(tp);
-    const float d = tp - r;  // exact where it matters
-    float c = CENTERED ? __builtin_amdgcn_fmed3f(r, G.loc, G.hic) : __builtin_amdgcn_fmed3f(r + G.z, G.lof, G.hi);
-    if (__builtin_expect(!(__builtin_fabsf(d) < 0.5f - 0x1p-12f), 0)) {
-        const float xr = (G.relu && x < 0.0f) ? 0.0f : x;
-        const float u = __builtin_rintf(xr / G.s) + G.z;
-        c = (u != u) ? (KEEP_NAN ? u : G.bias) : __builtin_amdgcn_fmed3f(u, G.lo, G.hi);
-        if (CENTERED) c = c - G.z;
-    }
-    return c;
+    const float v[1] = {x};
+    float c[1];
+    quant_fast<KEEP_NAN, CENTERED>(v, G, c);
+    return c[0];
 }
 
-// One output element.  Float steps are separate (no FMA) and in the order the
+// N output elements.  Float steps are separate (no FMA) and in the order the
 // CPU restatement uses, so results are bit-identical to it.  MODE is a
 // compile-time constant so that each output form gets a tight loop.
-// epilogue_value returns the element as 32 bits: float bits, the integer accumulator,
+// Each comes back as 32 bits: float bits, the integer accumulator,
 // the requantized code as a float (plus G.bias) or - ahead of a fused join - that code
 // minus its zero point (finish_value / join_code take it from there); store_* narrows
 // and writes.  G was made with relu = g.relu: the requantizing forms
@@ -166,28 +187,63 @@ enum EpilogueForm { kFormAny, kFormPlain /* neither ReLU nor GELU */, kFormGelu 
 __device__ __forceinline__ EpilogueForm epilogue_form(const GemmArgs& g) {
     return g.relu ? kFormAny : (g.gelu ? kFormGelu : kFormPlain);
 }
-template <int MODE, bool PRESCALED = false, EpilogueForm FORM = kFormAny>
-__device__ __forceinline__ uint32_t epilogue_value(const GemmArgs& g, int32_t acc, float as,
-                                                   const ColParams& c, const QGrid& G) {
-    if (MODE == OUT_ACC_I32) return uint32_t(acc);
-    float f = float(acc - c.corr);
-    float sc = PRESCALED ? c.ws : as * c.ws;
-    float y = f * sc;
-    y = y + c.bias;
-    if (MODE == OUT_REQUANT_JOIN) return __float_as_uint(quant_fast<false, true>(y, G));
-    // still a float (plus G.bias): store_* narrows it and adds out_offset
-    if (MODE == OUT_REQUANT_I8) return __float_as_uint(quant_fast<false>(y, G));
-    // not the centered form: its -0 (from rint(x / s) = -0) would survive the multiplication
-    if (MODE == OUT_FAKEQUANT_F32) return __float_as_uint((quant_fast<true>(y, G) - G.z) * G.s);
-    // ReLU as a floor of 0, no ReLU as a floor of -inf: one compare and select either
-    // way (a NaN fails the compare and passes through, as in the CPU formulation)
-    if (FORM == kFormAny) {
-        const float floor = g.relu ? 0.0f : -__builtin_inff();
-        y = (y < floor) ? floor : y;
+template <int MODE, bool PRESCALED = false, EpilogueForm FORM = kFormAny, int N>
+__device__ __forceinline__ void epilogue_values(const GemmArgs& g, const int32_t (&acc)[N], const float (&as)[N],
+                                                const ColParams (&c)[N], const QGrid& G, uint32_t (&out)[N]) {
+    float y[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        if (MODE == OUT_ACC_I32) {
+            out[k] = uint32_t(acc[k]);
+            continue;
+        }
+        const float f = float(acc[k] - c[k].corr);
+        const float sc = PRESCALED ? c[k].ws : as[k] * c[k].ws;
+        y[k] = f * sc;
+        y[k] = y[k] + c[k].bias;
     }
-    // the expression of the stand-alone kernel, so fusing it changes no bit
-    if (MODE == OUT_F32X && (FORM == kFormGelu || (FORM == kFormAny && g.gelu))) y = gelu_erf(y);
-    return __float_as_uint(y);
+    if (MODE == OUT_ACC_I32) return;
+    if (MODE == OUT_REQUANT_JOIN || MODE == OUT_REQUANT_I8 || MODE == OUT_FAKEQUANT_F32) {
+        // still a float (plus G.bias): store_* narrows it and adds out_offset
+        float q[N];
+        quant_fast<MODE == OUT_FAKEQUANT_F32, MODE == OUT_REQUANT_JOIN>(y, G, q);
+        // (fake-quantize: not the centered form: its -0, from rint(x / s) = -0, would survive the multiplication)
+#pragma unroll
+        for (int k = 0; k < N; ++k) out[k] = __float_as_uint(MODE == OUT_FAKEQUANT_F32 ? (q[k] - G.z) * G.s : q[k]);
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        // ReLU as a floor of 0, no ReLU as a floor of -inf: one compare and select either
+        // way (a NaN fails the compare and passes through, as in the CPU formulation)
+        if (FORM == kFormAny) {
+            const float floor = g.relu ? 0.0f : -__builtin_inff();
+            y[k] = (y[k] < floor) ? floor : y[k];
+        }
+        // the expression of the stand-alone kernel, so fusing it changes no bit
+        if (MODE == OUT_F32X && (FORM == kFormGelu || (FORM == kFormAny && g.gelu))) y[k] = gelu_erf(y[k]);
+        out[k] = __float_as_uint(y[k]);
+    }
+}
+template <int MODE>
+__device__ __forceinline__ uint32_t epilogue_value(const GemmArgs& g, int32_t acc, float as, const ColParams& c,
+                                                   const QGrid& G) {
+    const int32_t a1[1] = {acc};
+    const float s1[1] = {as};
+    const ColParams c1[1] = {c};
+    uint32_t o1[1];
+    epilogue_values<MODE>(g, a1, s1, c1, G, o1);
+    return o1[0];
+}
+// four columns of one row
+template <int MODE, bool PRESCALED = false, EpilogueForm FORM = kFormAny, class Acc>
+__device__ __forceinline__ uint4 epilogue_quad(const GemmArgs& g, const Acc& acc, float as, const ColParams (&c)[4],
+                                               const QGrid& G) {
+    const int32_t a4[4] = {acc[0], acc[1], acc[2], acc[3]};
+    const float s4[4] = {as, as, as, as};
+    uint32_t o[4];
+    epilogue_values<MODE, PRESCALED, FORM>(g, a4, s4, c, G, o);
+    return uint4{o[0], o[1], o[2], o[3]};
 }
 
 // y + residual[m, n] for the float output forms (x + linear(...), the residual
@@ -223,18 +279,24 @@ __device__ __forceinline__ JoinParams load_join(const GemmArgs& g, const QGrid& 
 }
 
 // bits: this layer's requantized code minus its zero point, as a float (what
-// epilogue_value<OUT_REQUANT_JOIN> returned); other: the partner's stored code
+// epilogue_values<OUT_REQUANT_JOIN> returned); other: the partner's stored code
 __device__ __forceinline__ uint32_t join_code(const GemmArgs& g, const JoinParams& jp, uint32_t bits, int other) {
     const float x1 = __uint_as_float(bits) * jp.S1;
     const float x2 = (float(other - g.join_off) - jp.z2) * jp.s2;
     return __float_as_uint(quant_fast<false>(x1 + x2, jp.out));  // store_* narrows, adds join_out_offset
 }
 
-// The same with the partner's stored byte + 128 (0..255) already a float; needs jp.k2_exact.
-__device__ __forceinline__ uint32_t join_code_biased(const JoinParams& jp, uint32_t bits, float other_biased) {
-    const float x1 = __uint_as_float(bits) * jp.S1;
-    const float x2 = (other_biased - jp.k2) * jp.s2;
-    return __float_as_uint(quant_fast<false>(x1 + x2, jp.out));
+// The same for four elements, `other` the partner's four stored bytes; needs jp.k2_exact.
+__device__ __forceinline__ uint4 join_codes(const JoinParams& jp, uint4 bits, uint32_t other) {
+    const uint32_t b = other ^ 0x80808080u;  // stored bytes + 128: 0..255
+    const float x1[4] = {__uint_as_float(bits.x) * jp.S1, __uint_as_float(bits.y) * jp.S1, __uint_as_float(bits.z) * jp.S1,
+                         __uint_as_float(bits.w) * jp.S1};
+    const float x2[4] = {(float(b & 0xffu) - jp.k2) * jp.s2, (float((b >> 8) & 0xffu) - jp.k2) * jp.s2,
+                         (float((b >> 16) & 0xffu) - jp.k2) * jp.s2, (float(b >> 24) - jp.k2) * jp.s2};
+    const float x[4] = {x1[0] + x2[0], x1[1] + x2[1], x1[2] + x2[2], x1[3] + x2[3]};
+    float c[4];
+    quant_fast<false>(x, jp.out, c);
+    return uint4{__float_as_uint(c[0]), __float_as_uint(c[1]), __float_as_uint(c[2]), __float_as_uint(c[3])};
 }
 
 // one element's residual step, whichever form the output mode has (jp: read by the join only)
@@ -245,7 +307,7 @@ __device__ __forceinline__ uint32_t finish_value(const GemmArgs& g, uint32_t bit
     return add_residual<MODE>(g, bits, m, n);
 }
 
-// Codes leave epilogue_value / join_code as floats, plus the grid's bias and without their
+// Codes leave epilogue_values / join_codes as floats, plus the grid's bias and without their
 // storage offset (-128 for the quint8 form, else 0).  stored byte = (value - bias + offset)
 // mod 256: when the values lie in 0..255 and offset - bias is 0 or +-128 modulo 256, four of
 // them are converted and packed by v_cvt_pk_u8_f32 and the offset is an XOR on the dword.

@@ -934,7 +934,8 @@ namespace {
 
 // x = every float32 bit pattern of [first, first + count): the tile epilogue's requantize
 // (quant_fast: reciprocal multiply with a guard band, division for the rest), in its three
-// forms (the code, the code minus the zero point, the code shifted into 0..255), against the
+// forms (the code, the code minus the zero point, the code shifted into 0..255), alone and as one of four that
+// share the test - all the others clear of the halves, and one of them on a half -, against the
 // plain [floor at zero,] divide-round-add-clamp, compared as the codes the two would store.
 __global__ __launch_bounds__(256) void quant_route_check_kernel(float s, float z, float lo, float hi, int relu,
                                                                 unsigned long long first,
@@ -953,11 +954,16 @@ __global__ __launch_bounds__(256) void quant_route_check_kernel(float s, float z
         const float plain = (u != u) ? 0.0f : u;
         const float plain_c = plain - z;
         const float biased = lq::quant_fast<false>(x, Gb);
+        const float clear[4] = {1.25f * s, x, -2.0f * s, 3.25f * s}, half[4] = {0.5f * s, x, 1.25f * s, x};
+        float c[4], h[4];
+        lq::quant_fast<false>(clear, G, c);
+        lq::quant_fast<false, true>(half, G, h);
+        bad += __float_as_uint(c[1]) != __float_as_uint(fast) || !(h[1] == centered) || !(h[3] == centered);
         bad += (__float_as_uint(fast) != __float_as_uint(plain) && !(fast == 0.0f && plain == 0.0f)) ||
                (__float_as_uint(centered) != __float_as_uint(plain_c) && !(centered == 0.0f && plain_c == 0.0f)) ||
                !(biased == plain + Gb.bias) || (Gb.in_byte && !(biased >= 0.0f && biased <= 255.0f));
         const float tp = x * G.inv;
-        slow += !(__builtin_fabsf(tp - __builtin_rintf(tp)) < 0.5f - 0x1p-12f);
+        slow += !(__builtin_fabsf(tp - __builtin_rintf(tp)) < G.guard);
     }
     if (bad) atomicAdd(mismatches, bad);
     if (slow) atomicAdd(divided, slow);

@@ -302,12 +302,7 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
     // values of one tile in the lane's own layout, residual / join applied; (ri, rj): the tile's
     // place among the wavefront's accumulators
     auto tile_values = [&](int m, const pp_v4i& a, const ColParams (&c4)[4], float as, int nq, uint4& v, int ri, int rj) {
-        auto one_scale = [&](auto f) {
-            v.x = epilogue_value<MODE, true, decltype(f)::value>(g, a[0], 1.0f, c4[0], G);
-            v.y = epilogue_value<MODE, true, decltype(f)::value>(g, a[1], 1.0f, c4[1], G);
-            v.z = epilogue_value<MODE, true, decltype(f)::value>(g, a[2], 1.0f, c4[2], G);
-            v.w = epilogue_value<MODE, true, decltype(f)::value>(g, a[3], 1.0f, c4[3], G);
-        };
+        auto one_scale = [&](auto f) { v = epilogue_quad<MODE, true, decltype(f)::value>(g, a, 1.0f, c4, G); };
         if (prescaled && kFloatOut && form == kFormPlain) {
             one_scale(std::integral_constant<EpilogueForm, kFormPlain>{});
         } else if (prescaled && MODE == OUT_F32X) {
@@ -315,10 +310,7 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
         } else if (prescaled && !kFloatOut) {
             one_scale(std::integral_constant<EpilogueForm, kFormAny>{});
         } else {
-            v.x = epilogue_value<MODE, false>(g, a[0], as, c4[0], G);
-            v.y = epilogue_value<MODE, false>(g, a[1], as, c4[1], G);
-            v.z = epilogue_value<MODE, false>(g, a[2], as, c4[2], G);
-            v.w = epilogue_value<MODE, false>(g, a[3], as, c4[3], G);
+            v = epilogue_quad<MODE, false>(g, a, as, c4, G);
         }
         if (vec_out && (rows_in || m < g.M)) {
             if (kFloatOut && g.residual != nullptr) {
@@ -331,12 +323,7 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
                 v.w = __float_as_uint(__uint_as_float(v.w) + rv.w);
             }
             if (MODE == OUT_REQUANT_JOIN) {
-                const uint32_t jb = *reinterpret_cast<const uint32_t*>(g.join_q + size_t(m) * size_t(g.join_ld) + size_t(nq)) ^
-                                    0x80808080u;  // stored bytes + 128, all four
-                v.x = join_code_biased(jp, v.x, float(jb & 0xffu));
-                v.y = join_code_biased(jp, v.y, float((jb >> 8) & 0xffu));
-                v.z = join_code_biased(jp, v.z, float((jb >> 16) & 0xffu));
-                v.w = join_code_biased(jp, v.w, float(jb >> 24));
+                v = join_codes(jp, v, *reinterpret_cast<const uint32_t*>(g.join_q + size_t(m) * size_t(g.join_ld) + size_t(nq)));
             }
         }
     };

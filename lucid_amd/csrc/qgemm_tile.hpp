@@ -147,34 +147,36 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                     jv[p] = *reinterpret_cast<const uint32_t*>(jq + size_t(p) * ROWS_PER_PASS * size_t(g.join_ld));
             }
             // this lane's rows of the part: groups of four consecutive rows
+            auto four_rows = [&](int q, auto pre, auto f, const float (&as)[4]) {
+                const int row = 8 * q + 4 * (lane >> 5);  // the first one's within the staged part
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const v16i& a = acc[i][j];
+                    const int r = part * RPP + 4 * q;
+                    const int32_t a4[4] = {a[r], a[r + 1], a[r + 2], a[r + 3]};
+                    const ColParams c4[4] = {cp[j], cp[j], cp[j], cp[j]};
+                    uint32_t v[4];
+                    epilogue_values<MODE, decltype(pre)::value, decltype(f)::value>(g, a4, as, c4, G, v);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) stage[(row + k) * STRIDE + j * 32 + (lane & 31)] = v[k];
+                }
+            };
             if (prescaled) {
                 // a float form comes here without a ReLU and with a GELU exactly in OUT_F32X (run_epilogue)
                 constexpr EpilogueForm kForm = MODE == OUT_F32X ? kFormGelu : (kFloatOut ? kFormPlain : kFormAny);
+                const float one[4] = {1.0f, 1.0f, 1.0f, 1.0f};
 #pragma unroll
-                for (int rr = 0; rr < RPP; ++rr) {
-                    const int r = part * RPP + rr;
-                    const int row = 8 * (rr >> 2) + 4 * (lane >> 5) + (rr & 3);  // row within the staged part
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        stage[row * STRIDE + j * 32 + (lane & 31)] =
-                            epilogue_value<MODE, true, kForm>(g, acc[i][j][r], 1.0f, cp[j], G);
-                }
+                for (int q = 0; q < RPP / 4; ++q) four_rows(q, std::integral_constant<bool, true>{}, std::integral_constant<EpilogueForm, kForm>{}, one);
             } else {
-                float as[RPP];
+                float as[RPP / 4][4];
 #pragma unroll
                 for (int q = 0; q < RPP / 4; ++q) {
                     const float4 v = *reinterpret_cast<const float4*>(s_as + band + 8 * q + 4 * (lane >> 5));
-                    as[4 * q] = v.x, as[4 * q + 1] = v.y, as[4 * q + 2] = v.z, as[4 * q + 3] = v.w;
+                    as[q][0] = v.x, as[q][1] = v.y, as[q][2] = v.z, as[q][3] = v.w;
                 }
 #pragma unroll
-                for (int rr = 0; rr < RPP; ++rr) {
-                    const int r = part * RPP + rr;
-                    const int row = 8 * (rr >> 2) + 4 * (lane >> 5) + (rr & 3);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        stage[row * STRIDE + j * 32 + (lane & 31)] =
-                            epilogue_value<MODE, false>(g, acc[i][j][r], as[rr], cp[j], G);
-                }
+                for (int q = 0; q < RPP / 4; ++q)
+                    four_rows(q, std::integral_constant<bool, false>{}, std::integral_constant<EpilogueForm, kFormAny>{}, as[q]);
             }
             wave_lds_sync();
             const uint32_t* src = stage + row0 * STRIDE + cq;
@@ -196,13 +198,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                 }
                 if (MODE == OUT_REQUANT_JOIN && join_fast) {
 #pragma unroll
-                    for (int p = 0; p < PASSES; ++p) {
-                        const uint32_t b = jv[p] ^ 0x80808080u;  // stored bytes + 128, all four
-                        v[p].x = join_code_biased(jp, v[p].x, float(b & 0xffu));
-                        v[p].y = join_code_biased(jp, v[p].y, float((b >> 8) & 0xffu));
-                        v[p].z = join_code_biased(jp, v[p].z, float((b >> 16) & 0xffu));
-                        v[p].w = join_code_biased(jp, v[p].w, float(b >> 24));
-                    }
+                    for (int p = 0; p < PASSES; ++p) v[p] = join_codes(jp, v[p], jv[p]);
                 }
                 if (MODE == OUT_F32X && keep) {
 #pragma unroll

@@ -208,10 +208,11 @@ __global__ __launch_bounds__(256) void layernorm_stats_kernel(const float* __res
 
 // four codes of normalized values
 __device__ __forceinline__ uint32_t layernorm_codes(float4 v, float4 g, float4 b, float mean, float rstd, const QGrid& G, int off) {
-    const int c0 = int(quant_fast<false>(((v.x - mean) * rstd) * g.x + b.x, G)) + off;
-    const int c1 = int(quant_fast<false>(((v.y - mean) * rstd) * g.y + b.y, G)) + off;
-    const int c2 = int(quant_fast<false>(((v.z - mean) * rstd) * g.z + b.z, G)) + off;
-    const int c3 = int(quant_fast<false>(((v.w - mean) * rstd) * g.w + b.w, G)) + off;
+    const float y[4] = {((v.x - mean) * rstd) * g.x + b.x, ((v.y - mean) * rstd) * g.y + b.y,
+                        ((v.z - mean) * rstd) * g.z + b.z, ((v.w - mean) * rstd) * g.w + b.w};
+    float c[4];
+    quant_fast<false>(y, G, c);
+    const int c0 = int(c[0]) + off, c1 = int(c[1]) + off, c2 = int(c[2]) + off, c3 = int(c[3]) + off;
     return uint32_t(c0 & 0xff) | (uint32_t(c1 & 0xff) << 8) | (uint32_t(c2 & 0xff) << 16) | (uint32_t(c3) << 24);
 }
 
