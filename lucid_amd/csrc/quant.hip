@@ -607,7 +607,7 @@ __global__ __launch_bounds__(1024) void calc_qparams_from_range_kernel(const flo
                                                                         float* zp, float* mn_out,
                                                                         float* mx_out) {
     float mn, mx;
-    range_block_load(range, mn, mx);
+    range_block_load<4>(range, mn, mx);
     if (threadIdx.x == 0) {
         if (mn_out) *mn_out = mn;
         if (mx_out) *mx_out = mx;
@@ -631,7 +631,7 @@ __global__ __launch_bounds__(1024) void quantize_range_kernel(QuantizeOp<int8_t>
     for (int u = 0; u < kRangeChunk; ++u)
         if (at + u * 1024 < quads) v[u] = op.load(at + u * 1024);
     float mn, mx, s, z;
-    range_block_load(range, mn, mx);
+    range_block_load<1>(range, mn, mx);
     qparams_of(mn, mx, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
     if (blockIdx.x == 0) {
         if (threadIdx.x == 0) *scale = s, *zp = z;

@@ -42,19 +42,31 @@ struct RangeKeep {
     __device__ __forceinline__ void store(float* range) const { range_block_store(range, lo, hi, lo != lo); }
 };
 
-// The range itself, for every thread of a block (up to 1024; all must call it): the reduction of the slots.
+// The range itself, for every thread of a block (up to 1024; all must call it): the reduction of the slots.  The first
+// AHEAD slots of each thread are requested together with their number, which would otherwise be a memory round trip
+// before them (they are words of the buffer in any case; what lies past the number is not looked at).
+template <int AHEAD>
 __device__ __forceinline__ void range_block_load(const float* __restrict__ range, float& mn, float& mx) {
-    const unsigned n = reinterpret_cast<const unsigned*>(range)[0];
-    mn = __builtin_inff(), mx = -__builtin_inff();
-    int nan = 0;
-    for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
-        const float a = range[4 + i], b = range[4 + kRangeSlots + i];
-        nan |= (a != a) | (b != b);
-        mn = fminf(mn, a);
-        mx = fmaxf(mx, b);
+    static_assert(AHEAD * 1024 <= kRangeSlots, "within the buffer for blocks of up to 1024 threads");
+    float a[AHEAD], b[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+        const unsigned i = threadIdx.x + u * blockDim.x;
+        a[u] = range[4 + i], b[u] = range[4 + kRangeSlots + i];
     }
-    block_minmax(mn, mx, nan);
-    if (nan) mn = mx = __builtin_nanf("");
+    const unsigned n = reinterpret_cast<const unsigned*>(range)[0];
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+    auto add = [&](float x, float y) {
+        lo = __builtin_elementwise_minimum(lo, x);
+        hi = __builtin_elementwise_maximum(hi, y);
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (threadIdx.x + u * blockDim.x < n) add(a[u], b[u]);
+    for (unsigned i = threadIdx.x + AHEAD * blockDim.x; i < n; i += blockDim.x) add(range[4 + i], range[4 + kRangeSlots + i]);
+    int nan = (lo != lo) | (hi != hi);
+    block_minmax(lo, hi, nan);
+    mn = nan ? __builtin_nanf("") : lo, mx = nan ? __builtin_nanf("") : hi;
 }
 
 // vDSP_vmax / vDSP_vmin single precision propagate NaN (Vdsp.cpp:140-151).

@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256) void layernorm_quantize_kernel(const float* __
     float s, z;
     if constexpr (RANGE) {
         float mn, mx;
-        range_block_load(grid.range, mn, mx);
+        range_block_load<2>(grid.range, mn, mx);
         qparams_of(mn, mx, grid.symmetric, grid.qmin, grid.qmax, grid.is_signed, grid.eps, grid.half_range, &s, &z);
         if (blockIdx.x == 0 && threadIdx.x == 0) *scale = s, *zp = z;
     } else {

@@ -390,6 +390,41 @@ def test_codes_straight_from_a_kept_range(n, nan):
         assert np.array_equal(one[2].numpy()[:n - 1], two[2].numpy()[:n - 1])
 
 
+@pytest.mark.parametrize("n", [1, 63, 511, 512, 513, 1024, 1025, 4096, 4097, 16384])
+@pytest.mark.parametrize("nan", [False, True])
+def test_range_of_any_number_of_slots(n, nan):
+    """The first slots of a range are read before their number is known: what lies past it (here NaNs, beyond any other value)
+    does not count, the last slot does, whether it is among the first ones or not - for all three readers of a range."""
+    import lucid_amd.quantization as Q
+    rng = np.random.default_rng(n)
+    words = _C.range_buffer_words()
+    slots = (words - 4) // 2
+    buf = np.full(words, np.nan, np.float32)
+    buf[:1].view(np.uint32)[0] = n
+    lo, hi = -rng.random(n).astype(np.float32), rng.random(n).astype(np.float32)
+    lo[-1], hi[n // 2] = -2, 3
+    if nan:
+        lo[-1] = hi[-1] = np.nan
+    buf[4:4 + n], buf[4 + slots:4 + slots + n] = lo, hi
+    r, f32 = L.tensor(buf, device="hip"), lambda: L.Tensor.empty((), L.float32, "hip")
+    x, w = (L.tensor(rng.standard_normal(m).astype(np.float32), device="hip") for m in (4096, 64))
+    q = L.Tensor.empty((4096,), L.int8, "hip")
+    mn, mx, sz = f32(), f32(), [(f32(), f32()) for _ in range(3)]
+    args = (0, 0, 255, 0, 1e-8)
+    _C.call("lq_calc_qparams_from_range", r.data_ptr, *args, *(v.data_ptr for v in sz[0]), mn.data_ptr, mx.data_ptr, None)
+    _C.call("lq_quantize_from_range_i8", x.data_ptr, 4096, r.data_ptr, *args, -128, *(v.data_ptr for v in sz[1]), q.data_ptr, None)
+    stats = L.tensor(np.tile(np.float32([0, 1]), 64), device="hip")
+    _C.call("lq_layernorm_quantize_from_range_i8", x.data_ptr, w.data_ptr, w.data_ptr, stats.data_ptr, 64, 64, r.data_ptr, *args,
+            -128, *(v.data_ptr for v in sz[2]), q.data_ptr, None)
+    if nan:
+        assert np.isnan(mn.numpy()) and np.isnan(mx.numpy()) and all(np.isnan(s.numpy()) for s, _ in sz)
+    else:
+        assert mn.numpy() == -2 and mx.numpy() == hi.max()
+        want = Q.calculate_qparams(mn, mx, Q.per_tensor_affine, Q.quint8)
+        for s, z in sz:
+            assert s.numpy().tobytes() == want[0].numpy().tobytes() and z.numpy().tobytes() == want[1].numpy().tobytes()
+
+
 def test_layernorm_codes_of_no_rows_still_give_the_qparams():
     """``lq_layernorm_quantize_from_range_i8`` stands for two calls, of which the first does not look at the rows."""
     from lucid_amd.nn.functional import _new_range
