@@ -388,6 +388,40 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
             c_kh = tap / g.cKW;
             c_kw = tap - c_kh * g.cKW;
         }
+        // CONV, channels of a group in whole stages (Cg % BK == 0): a stage lies inside one tap, so the
+        // position is the same for all lanes (scalar registers), and inside a tap a lane's sources only
+        // advance.  The position kept per lane, below, cost a k-iteration of a 64 x 64 tile about 500
+        // cycles beside the 350 of its LDS traffic: 784 x 512 x 4608 (3x3, 7x7 images) 18.0 -> 11.8 us,
+        // 1568 x 256 x 2304 11.5 -> 8.9, the plain GEMMs of these sizes 10.3 and 7.4.
+        const bool one_tap = CONV && g.cCg % BK == 0;
+        int u_ci = 0, u_kh = 0, u_kw = 0, u_kd = 0;
+        const int8_t* a_src[CONV ? PA : 1];
+        int a_step[CONV ? PA : 1];  // 0 where the tap falls outside the image: the pad bytes are read again
+        auto enter_tap = [&] {
+            const int dh = u_kh * g.cdh, dw = u_kw * g.cdw, dd = CONV == 2 ? u_kd * g.cdd : 0;
+            const unsigned delta = unsigned((dd * g.cH + dh) * g.cW + dw) * unsigned(g.cCin) + unsigned(u_ci);
+#pragma unroll
+            for (int it = 0; it < PA; ++it) {
+                const int ih = (a_hw[it] >> 16) + dh;
+                const int iw = int(short(a_hw[it] & 0xffff)) + dw;
+                bool ok = unsigned(ih) < unsigned(g.cH) && unsigned(iw) < unsigned(g.cW);
+                if constexpr (CONV == 2) ok = ok && unsigned(a_d[it] + dd) < unsigned(g.cD);
+                a_src[it] = ok ? a_tile + (a_off[it] + delta + unsigned(kc * 16)) : g.pad_src;
+                a_step[it] = ok ? BK : 0;
+            }
+        };
+        if (one_tap) {
+            int tap = kb * BK / g.cCg;
+            u_ci = kb * BK - tap * g.cCg;
+            if (CONV == 2) {
+                const int taps_hw = g.cKH * g.cKW;
+                u_kd = tap / taps_hw;
+                tap -= u_kd * taps_hw;
+            }
+            u_kh = tap / g.cKW;
+            u_kw = tap - u_kh * g.cKW;
+            enter_tap();
+        }
 
         // `full` (compile time): the whole stage lies inside K, so no lane needs the
         // zero source and the address is a uniform base plus a per-lane offset
@@ -402,6 +436,28 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
 #pragma unroll
                 for (int it = 0; it < PA; ++it)
                     __builtin_amdgcn_global_load_lds(LQ_GPTR(ab + a_off[it]), LQ_LPTR(sa + it * (THREADS * 16)), 16, 0, 0);
+#pragma unroll
+                for (int it = 0; it < PB; ++it)
+                    __builtin_amdgcn_global_load_lds(LQ_GPTR(bb + b_off[it]), LQ_LPTR(sb + it * (THREADS * 16)), 16, 0, 0);
+                return;
+            }
+            if (CONV && decltype(full)::value) {
+                // reached with one_tap only
+                if (u_ci == g.cCg) {
+                    u_ci = 0;
+                    if (++u_kw == g.cKW) {
+                        u_kw = 0, ++u_kh;
+                        if (CONV == 2 && u_kh == g.cKH) u_kh = 0, ++u_kd;
+                    }
+                    enter_tap();
+                }
+                u_ci += BK;
+                const int8_t* bb = b_tile + k0;
+#pragma unroll
+                for (int it = 0; it < PA; ++it) {
+                    __builtin_amdgcn_global_load_lds(LQ_GPTR(a_src[it]), LQ_LPTR(sa + it * (THREADS * 16)), 16, 0, 0);
+                    a_src[it] += a_step[it];
+                }
 #pragma unroll
                 for (int it = 0; it < PB; ++it)
                     __builtin_amdgcn_global_load_lds(LQ_GPTR(bb + b_off[it]), LQ_LPTR(sb + it * (THREADS * 16)), 16, 0, 0);
@@ -467,9 +523,19 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
         // current stage, so its latency is covered by that step's MFMAs.  Stages
         // past the end are loaded from the block of zeros, which keeps the number
         // of outstanding loads - and so the vmcnt to wait for - constant.
+        if (one_tap) {
+            // (K is whole stages too, so that stages are either inside the segment or past its end)
+            for (int s = 0; s < STAGES; ++s) {
+                if (kb + s < ke)
+                    load_stage((kb + s) * BK, smem + s * Cfg::STAGE_BYTES, std::true_type{});
+                else
+                    load_stage((kb + s) * BK, smem + s * Cfg::STAGE_BYTES, std::false_type{});
+            }
+        } else {
 #pragma unroll
-        for (int s = 0; s < STAGES; ++s)
-            load_stage((kb + s) * BK, smem + s * Cfg::STAGE_BYTES, std::false_type{});
+            for (int s = 0; s < STAGES; ++s)
+                load_stage((kb + s) * BK, smem + s * Cfg::STAGE_BYTES, std::false_type{});
+        }
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((STAGES - 1) * (PA + PB)));
         __syncthreads();
 
@@ -514,7 +580,7 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
             };
             const int n_it = ke - kb;
             int n_full = (k_end / BK) - kb - STAGES;
-            n_full = n_full < 0 ? 0 : (n_full > n_it - 1 ? n_it - 1 : n_full);
+            n_full = n_full < 0 || (CONV && !one_tap) ? 0 : (n_full > n_it - 1 ? n_it - 1 : n_full);
             int t = 0;
             for (; t < n_full; ++t) stage_steps(t, false, std::true_type{});
             for (; t + 1 < n_it; ++t) stage_steps(t, false, std::false_type{});
@@ -598,7 +664,7 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
         const int n_it = ke - kb;
         // iterations whose refill stage (t + STAGES) lies wholly inside K come first
         int n_full = (k_end / BK) - kb - STAGES;
-        n_full = n_full < 0 ? 0 : (n_full > n_it - 1 ? n_it - 1 : n_full);
+        n_full = n_full < 0 || (CONV && !one_tap) ? 0 : (n_full > n_it - 1 ? n_it - 1 : n_full);
         int t = 0;
         for (; t < n_full; ++t) k_steps(t, false, std::true_type{});
         for (; t + 1 < n_it; ++t) k_steps(t, false, std::false_type{});

@@ -59,6 +59,33 @@ def test_accumulators_exact_on_every_route(case):
     assert np.array_equal(auto, exp)
 
 
+# B, H, W, Cin, Cout, KH, KW, stride, pad, dil, groups: channels of a group in whole k-iterations of 64 and of
+# 128 (the gather steps its sources inside a tap), in 64 but not 128, and in neither
+TAP_CASES = [
+    (2, 7, 7, 128, 70, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),
+    (1, 9, 6, 256, 64, 3, 2, (2, 1), (0, 2, 1, 0), (1, 2), 2),
+    (3, 5, 5, 64, 40, 2, 3, (1, 2), (1, 0, 2, 2), (2, 1), 1),
+    (1, 8, 7, 192, 33, 5, 1, (1, 1), (2, 2, 0, 0), (1, 1), 1),
+    (2, 6, 6, 80, 24, 3, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1),
+    (5, 9, 9, 128, 130, 1, 1, (2, 2), (0, 0, 0, 0), (1, 1), 1),
+    (1, 2, 2, 64, 8, 3, 3, (1, 1), (2, 2, 2, 2), (2, 2), 1),
+]
+
+
+@pytest.mark.parametrize("cfg", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12])
+@pytest.mark.parametrize("case", TAP_CASES)
+def test_gather_exact_at_every_tile_shape(case, cfg):
+    B, H, W, Cin, Cout, KH, KW, st, pad, dil, groups = case
+    rng = np.random.default_rng(sum(case[:7]))
+    x, w = codes(rng, (B, H, W, Cin)), codes(rng, (Cout, KH, KW, Cin // groups))
+    geo = dict(stride=st, pad=pad, dilation=dil, groups=groups)
+    exp = O.qconv2d(x, w, 91, 1.0, np.ones(Cout, np.float32), out_mode=O.OUT_ACC_I32, **geo)
+    for schedule in (1, 2):  # one block per tile; segments that begin inside a tap
+        got = _ops.qconv2d_i8(hip(x), hip(w), a_zp=91, out_mode=_ops.OUT_ACC_I32, path=IMPLICIT,
+                              tile_config=cfg | schedule << 8, **geo).numpy()
+        assert np.array_equal(got, exp), schedule
+
+
 @pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[3], CASES[4], CASES[7]])
 @pytest.mark.parametrize("relu,bias_kind", [(True, "f32"), (False, "f32"), (True, None)])
 def test_epilogue_bit_exact(case, relu, bias_kind):
