@@ -336,7 +336,7 @@ __device__ __forceinline__ void store_scalar(const GemmArgs& g, size_t idx, uint
         static_cast<uint32_t*>(g.out)[idx] = v;  // f32 / i32 bit patterns
 }
 
-// four consecutive elements; idx is a multiple of 4 and the row is 4-aligned
+// four consecutive elements, of 8 and 16 bits at a vector's alignment, of 32 bits at any element
 template <int MODE>
 __device__ __forceinline__ void store_vec4(const GemmArgs& g, size_t idx, uint4 v, const CodePack& cpk) {
     if (MODE == OUT_F16) {
@@ -360,7 +360,8 @@ __device__ __forceinline__ void store_vec4(const GemmArgs& g, size_t idx, uint4 
         }
         *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(g.out) + idx) = packed;
     } else {
-        *reinterpret_cast<uint4*>(static_cast<uint32_t*>(g.out) + idx) = v;
+        typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
+        *reinterpret_cast<u4*>(static_cast<uint32_t*>(g.out) + idx) = u4{v.x, v.y, v.z, v.w};
     }
 }
 

@@ -15,6 +15,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));  // at any element
 
 #define LQ_GPTR(p) ((__attribute__((address_space(1))) void*)(p))
 #define LQ_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
@@ -89,15 +90,19 @@ __device__ __forceinline__ void wave_lds_sync() {
 // MFMA result layout gives a lane one column and sixteen scattered rows; the
 // band is turned through a wavefront-private LDS area so that a lane ends up
 // with four consecutive columns of one row and the wavefront writes contiguous
-// row segments.  `interior` (uniform): the whole tile lies inside the output
-// and rows are vector-aligned, so the stores need no per-lane tests.  `prescaled`
-// (uniform): cp[].ws already carries the (single) activation scale, s_as is not read.
+// row segments.  `vec` (uniform): four consecutive columns may be accessed as one vector; `interior`
+// (uniform): and the whole tile lies inside the output, so the stores need no per-lane tests.  A tile
+// that leaves the output tests per group of four columns, and goes element by element only where
+// such a group straddles the last column.  (With the whole tile element by element, the tiles on
+// the edge were the last to finish: 3136 x 1024 x 256 with a join in 128-row tiles 15.1 -> 10.6 us, 50000 x 256 x 64
+// 19.8 -> 14.9, 333 x 1001 x 1008 to float32 6.2 -> 5.9.)
+// `prescaled` (uniform): cp[].ws already carries the (single) activation scale, s_as is not read.
 template <class Cfg, int MODE>
 __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg::TM][Cfg::TN],
                                               const ColParams (&cp)[Cfg::TN], const float* s_as,
                                               uint32_t* stage, int m0, int n0, int n_limit, int wm,
                                               int wn, int lane, float S, float Z, bool interior,
-                                              bool prescaled, RangeKeep& kept) {
+                                              bool vec, bool prescaled, RangeKeep& kept) {
     constexpr int TM = Cfg::TM, TN = Cfg::TN, STRIDE = Cfg::STAGE_STRIDE;
     constexpr int QUADS_PER_ROW = TN * 8;            // four-column groups per staged row
     constexpr int EPI_ROWS = Cfg::EPI_ROWS;          // rows staged at a time (32 or 16)
@@ -105,8 +110,6 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
     constexpr int PASSES = EPI_ROWS * QUADS_PER_ROW / 64;
     constexpr int ROWS_PER_PASS = 64 / QUADS_PER_ROW;
     static_assert(64 % QUADS_PER_ROW == 0 && RPP % 4 == 0, "");
-    const int esize = MODE == OUT_F16 ? 2 : ((MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) ? 1 : 4);
-    const bool vec_ok = (g.ldo % 4 == 0) && (reinterpret_cast<uintptr_t>(g.out) % (4 * esize) == 0);
     const int row0 = lane / QUADS_PER_ROW, cq = (lane % QUADS_PER_ROW) * 4;
     constexpr bool kRequant = MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN || MODE == OUT_FAKEQUANT_F32;
     const QGrid G = make_qgrid(S, Z, float(g.out_qmin), float(g.out_qmax), kRequant, g.relu != 0,
@@ -114,7 +117,8 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
     JoinParams jp;
     if (MODE == OUT_REQUANT_JOIN) {
         jp = load_join(g, G, true);
-        interior = interior && jp.k2_exact;  // the vector path subtracts the partner's offsets in one step
+        interior = interior && jp.k2_exact;  // the vector paths subtract the partner's offsets in one step
+        vec = vec && jp.k2_exact;
     }
     const CodePack cpk = make_code_pack<MODE>(g, MODE == OUT_REQUANT_JOIN ? jp.out : G);
     // running range of what this lane stores (float32 output with a kept range only)
@@ -130,12 +134,12 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
             // their latency is paid under it (`interior` vouches for alignment)
             constexpr bool kFloatOut = MODE == OUT_F32 || MODE == OUT_F16 || MODE == OUT_F32X;
             const bool res_fast = kFloatOut && interior && g.residual != nullptr;
-            float4 rv[kFloatOut ? PASSES : 1];
+            float4u rv[kFloatOut ? PASSES : 1];
             if (kFloatOut && res_fast) {
                 const float* rp = g.residual + size_t(m_first) * size_t(g.ldr) + size_t(n);
 #pragma unroll
                 for (int p = 0; p < PASSES; ++p)
-                    rv[p] = *reinterpret_cast<const float4*>(rp + size_t(p) * ROWS_PER_PASS * size_t(g.ldr));
+                    rv[p] = *reinterpret_cast<const float4u*>(rp + size_t(p) * ROWS_PER_PASS * size_t(g.ldr));
             }
             // the other operand of a fused join on codes: four codes per row, requested early too
             const bool join_fast = MODE == OUT_REQUANT_JOIN && interior;
@@ -210,11 +214,46 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                     idx += step;
                 }
             } else {
-#pragma unroll 4
-                for (int p = 0; p < PASSES; ++p) {
-                    uint4 v = *reinterpret_cast<const uint4*>(src + p * ROWS_PER_PASS * STRIDE);
-                    const int m = m_first + p * ROWS_PER_PASS;
-                    if (m < g.M && n < n_limit) {
+                int first = 0;  // the lane's first pass that goes element by element
+                if (vec && n + 4 <= n_limit) {
+                    // the passes of the lane whose rows lie inside the output
+                    const int passes = (g.M - m_first + ROWS_PER_PASS - 1) / ROWS_PER_PASS;
+                    float4u ev[kFloatOut ? PASSES : 1];
+                    uint32_t ej[MODE == OUT_REQUANT_JOIN ? PASSES : 1];
+                    if (kFloatOut && g.residual != nullptr) {
+                        const float* rp = g.residual + size_t(m_first) * size_t(g.ldr) + size_t(n);
+#pragma unroll
+                        for (int p = 0; p < PASSES; ++p)
+                            if (p < passes) ev[p] = *reinterpret_cast<const float4u*>(rp + size_t(p) * ROWS_PER_PASS * size_t(g.ldr));
+                    }
+                    if (MODE == OUT_REQUANT_JOIN) {
+                        const int8_t* jq = g.join_q + size_t(m_first) * size_t(g.join_ld) + size_t(n);
+#pragma unroll
+                        for (int p = 0; p < PASSES; ++p)
+                            if (p < passes) ej[p] = *reinterpret_cast<const uint32_t*>(jq + size_t(p) * ROWS_PER_PASS * size_t(g.join_ld));
+                    }
+#pragma unroll
+                    for (int p = 0; p < PASSES; ++p) {
+                        if (p >= passes) break;
+                        uint4 v = *reinterpret_cast<const uint4*>(src + p * ROWS_PER_PASS * STRIDE);
+                        if (kFloatOut && g.residual != nullptr) {
+                            v.x = __float_as_uint(__uint_as_float(v.x) + ev[p].x);
+                            v.y = __float_as_uint(__uint_as_float(v.y) + ev[p].y);
+                            v.z = __float_as_uint(__uint_as_float(v.z) + ev[p].z);
+                            v.w = __float_as_uint(__uint_as_float(v.w) + ev[p].w);
+                        }
+                        if (MODE == OUT_REQUANT_JOIN) v = join_codes(jp, v, ej[p]);
+                        if (MODE == OUT_F32X && keep) track(v.x), track(v.y), track(v.z), track(v.w);
+                        store_vec4<MODE>(g, size_t(m_first + p * ROWS_PER_PASS) * size_t(g.ldo) + size_t(n), v, cpk);
+                    }
+                    first = PASSES;
+                }
+                if (n < n_limit) {
+#pragma unroll 1
+                    for (int p = first; p < PASSES; ++p) {
+                        uint4 v = *reinterpret_cast<const uint4*>(src + p * ROWS_PER_PASS * STRIDE);
+                        const int m = m_first + p * ROWS_PER_PASS;
+                        if (m >= g.M) break;
                         v.x = finish_value<MODE>(g, v.x, m, n, jp);
                         if (n + 1 < n_limit) v.y = finish_value<MODE>(g, v.y, m, n + 1, jp);
                         if (n + 2 < n_limit) v.z = finish_value<MODE>(g, v.z, m, n + 2, jp);
@@ -226,14 +265,10 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                             if (n + 3 < n_limit) track(v.w);
                         }
                         const size_t idx = size_t(m) * size_t(g.ldo) + size_t(n);
-                        if (vec_ok && n + 4 <= n_limit) {
-                            store_vec4<MODE>(g, idx, v, cpk);
-                        } else {
-                            store_scalar<MODE>(g, idx, v.x, cpk);
-                            if (n + 1 < n_limit) store_scalar<MODE>(g, idx + 1, v.y, cpk);
-                            if (n + 2 < n_limit) store_scalar<MODE>(g, idx + 2, v.z, cpk);
-                            if (n + 3 < n_limit) store_scalar<MODE>(g, idx + 3, v.w, cpk);
-                        }
+                        store_scalar<MODE>(g, idx, v.x, cpk);
+                        if (n + 1 < n_limit) store_scalar<MODE>(g, idx + 1, v.y, cpk);
+                        if (n + 2 < n_limit) store_scalar<MODE>(g, idx + 2, v.z, cpk);
+                        if (n + 3 < n_limit) store_scalar<MODE>(g, idx + 3, v.w, cpk);
                     }
                 }
             }
@@ -688,12 +723,12 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
             Z = g.out_zp[0];
         }
         const int esize = MODE == OUT_F16 ? 2 : ((MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) ? 1 : 4);
-        const bool interior = m0 + BM <= g.M && n0 + BN <= n_limit && g.ldo % 4 == 0 &&
-                              reinterpret_cast<uintptr_t>(g.out) % (4 * esize) == 0 &&
-                              (g.residual == nullptr ||
-                               (g.ldr % 4 == 0 && reinterpret_cast<uintptr_t>(g.residual) % 16 == 0)) &&
-                              (g.join_q == nullptr ||
-                               (g.join_ld % 4 == 0 && reinterpret_cast<uintptr_t>(g.join_q) % 4 == 0));
+        const bool inside = m0 + BM <= g.M && n0 + BN <= n_limit;
+        // accesses to four elements of 32 bits need no alignment beyond an element's
+        const bool vec = esize == 4 || (g.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(g.out) % (4 * esize) == 0 &&
+                                        (inside || n0 % 4 == 0) &&
+                                        (g.join_q == nullptr ||
+                                         (g.join_ld % 4 == 0 && reinterpret_cast<uintptr_t>(g.join_q) % 4 == 0)));
         __syncthreads();
         RangeKeep kept;
         // one activation scale for all rows (always so for a convolution): the kernels that
@@ -706,7 +741,7 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
 #pragma unroll
             for (int j = 0; j < TN; ++j) cp[j].ws = as_mine * cp[j].ws;
         }
-        tile_epilogue<Cfg, MODE>(g, acc, cp, s_as, stage, m0, n0, n_limit, wm, wn, lane, S, Z, interior, prescaled,
+        tile_epilogue<Cfg, MODE>(g, acc, cp, s_as, stage, m0, n0, n_limit, wm, wn, lane, S, Z, inside && vec, vec, prescaled,
                                  kept);
         __syncthreads();  // the staging area is the next tile's first LDS stage
         // one block per tile here (the launcher sees to it), so the block's slot is the tile's

@@ -645,6 +645,44 @@ def _range_words():
     return _C.range_buffer_words()
 
 
+@pytest.mark.parametrize("M,N", [(1, 64), (65, 131), (131, 68), (70, 2), (63, 260), (258, 129)])
+@pytest.mark.parametrize("cfg", [1, 3, 5, 6, 8, 9, 10, 12])
+def test_edge_tiles_every_output_form(cfg, M, N):
+    """Tiles that leave the matrix store groups of four columns, and single columns where a group straddles the
+    last one: the bits of the naive kernel in every output form, with a residual, a join, a GELU and a kept range
+    (whose minimum and maximum are those of the result), and nothing written past the last element."""
+    from lucid_amd import _C
+    rng = np.random.default_rng(cfg * 1000 + M + N)
+    K = 80
+    a, w = hip(codes(rng, (M, K), -100, 100)), hip(codes(rng, (N, K), -100, 100))
+    for per_row in (False, True):
+        common = dict(a_zp=5, a_scale=hip(rng.uniform(0.01, 0.05, M if per_row else 1).astype(np.float32)),
+                      w_scale=hip(rng.uniform(0.0005, 0.004, N).astype(np.float32)), wsum=_ops.rowsum_i8(w),
+                      bias=hip(rng.standard_normal(N).astype(np.float32)), out_scale=hip(np.float32(0.07)),
+                      out_zp=hip(np.float32(3.0)), out_qmin=-128, out_qmax=127)
+        res = hip(rng.standard_normal((M, N)).astype(np.float32))
+        join = dict(q=hip(codes(rng, (M, N))), scale=hip(np.float32(0.03)), zp=hip(np.float32(-7.0)), offset=0, relu=True,
+                    out_scale=hip(np.float32(0.08)), out_zp=hip(np.float32(1.0)), out_qmin=-128, out_qmax=127, out_offset=0)
+        forms = [dict(out_mode=m) for m in range(5)] + [dict(out_mode=_ops.OUT_F32, residual=res),
+                                                        dict(out_mode=_ops.OUT_F16, residual=res, relu=True),
+                                                        dict(out_mode=_ops.OUT_REQUANT_I8, join=join),
+                                                        dict(out_mode=_ops.OUT_F32, gelu=True)]
+        for form in forms:
+            want = _ops.qlinear_i8(a, w, **common, **form, path=NAIVE).numpy()
+            # an output that is followed by bytes of its own
+            buf = np.full((M + 1, N), 77, want.dtype)
+            full = hip(buf)
+            got = _ops.qlinear_i8(a, w, **common, **form, path=TILE, tile_config=cfg | 0x100, out=full.row_range(0, M))
+            assert np.array_equal(got.numpy().view(np.uint8), want.view(np.uint8)), form
+            assert np.array_equal(full.numpy()[M], buf[M]), form
+        rb = L.Tensor.empty((_C.range_buffer_words(),), L.float32, "hip")
+        y = _ops.qlinear_i8(a, w, **common, out_mode=_ops.OUT_F32, gelu=True, range_buf=rb, path=TILE, tile_config=cfg | 0x100).numpy()
+        mn, mx, s, z = (L.Tensor.empty((), L.float32, "hip") for _ in range(4))
+        _C.call("lq_calc_qparams_from_range", rb.data_ptr, 0, 0, 255, 0, 1e-8, s.data_ptr, z.data_ptr, mn.data_ptr,
+                mx.data_ptr, None)
+        assert float(mn.numpy()) == y.min() and float(mx.numpy()) == y.max()
+
+
 # ------------------------------------------------------------------ affine weight codes
 AFFINE_CASES = [
     # M, N, K, path
