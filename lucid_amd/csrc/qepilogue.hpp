@@ -326,6 +326,15 @@ __device__ __forceinline__ CodePack make_code_pack(const GemmArgs& g, const QGri
     return c;
 }
 
+// four values as one dword of codes, where cpk.pk
+__device__ __forceinline__ uint32_t pack_codes_pk(uint4 v, const CodePack& cpk) {
+    uint32_t packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.x), 0, 0u);
+    packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.y), 1, packed);
+    packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.z), 2, packed);
+    packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.w), 3, packed);
+    return packed ^ cpk.flip;
+}
+
 template <int MODE>
 __device__ __forceinline__ void store_scalar(const GemmArgs& g, size_t idx, uint32_t v, const CodePack& cpk) {
     if (MODE == OUT_F16)
@@ -337,7 +346,8 @@ __device__ __forceinline__ void store_scalar(const GemmArgs& g, size_t idx, uint
 }
 
 // four consecutive elements, of 8 and 16 bits at a vector's alignment, of 32 bits at any element
-template <int MODE>
+// PK: the caller knows that cpk.pk (a kernel asks before its loops: no element group then branches on it)
+template <int MODE, bool PK = false>
 __device__ __forceinline__ void store_vec4(const GemmArgs& g, size_t idx, uint4 v, const CodePack& cpk) {
     if (MODE == OUT_F16) {
         typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -346,12 +356,8 @@ __device__ __forceinline__ void store_vec4(const GemmArgs& g, size_t idx, uint4 
         *reinterpret_cast<h4*>(static_cast<_Float16*>(g.out) + idx) = h;
     } else if (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) {
         uint32_t packed;
-        if (cpk.pk) {
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.x), 0, 0u);
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.y), 1, packed);
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.z), 2, packed);
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.w), 3, packed);
-            packed ^= cpk.flip;
+        if (PK || cpk.pk) {
+            packed = pack_codes_pk(v, cpk);
         } else {
             const uint32_t o = uint32_t(cpk.add);
             const uint32_t x = uint32_t(int(__uint_as_float(v.x))), y = uint32_t(int(__uint_as_float(v.y)));

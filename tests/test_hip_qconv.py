@@ -358,6 +358,8 @@ def test_float_image_quantized_into_the_packed_form(B, H, W, Cin, Cout, KH, KW, 
     (2, 11, 11, 4, 40, 3, 5, (1, 3), (0, 0, 2, 2), 1),      # stride 3 along the row
     (1, 40, 37, 3, 160, 5, 5, (1, 2), (2, 2, 2, 2), 1),     # three column tiles, the last one partial
     (5, 33, 70, 2, 128, 8, 8, (3, 1), (1, 2, 3, 4), 1),     # K = 256, boxes past the right edge
+    (7, 75, 64, 3, 600, 7, 7, (2, 2), (3, 3, 3, 3), 1),     # blocks of one and of two boxes, a partial column tile
+    (6, 130, 132, 3, 720, 3, 3, (4, 4), (1, 1, 1, 1), 1),   # ... whose halo is not requested ahead
 ])
 def test_few_channel_kernel_with_the_filter_in_registers(B, H, W, Cin, Cout, KH, KW, stride, pad, dil_h):
     """tile_config 20 on the packed route: accumulators and every output form equal the oracle's."""
