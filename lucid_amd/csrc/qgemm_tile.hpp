@@ -91,7 +91,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // band is turned through a wavefront-private LDS area so that a lane ends up
 // with four consecutive columns of one row and the wavefront writes contiguous
 // row segments.  `vec` (uniform): four consecutive columns may be accessed as one vector; `interior`
-// (uniform): and the whole tile lies inside the output, so the stores need no per-lane tests.  A tile
+// (uniform): and the whole tile lies inside the output, so the stores need no per-lane tests (codes: nor one of how they pack).  A tile
 // that leaves the output tests per group of four columns, and goes element by element only where
 // such a group straddles the last column.  (With the whole tile element by element, the tiles on
 // the edge were the last to finish: 3136 x 1024 x 256 with a join in 128-row tiles 15.1 -> 10.6 us, 50000 x 256 x 64
@@ -121,6 +121,8 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
         vec = vec && jp.k2_exact;
     }
     const CodePack cpk = make_code_pack<MODE>(g, MODE == OUT_REQUANT_JOIN ? jp.out : G);
+    constexpr bool kCodes = MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN;
+    if (kCodes) interior = interior && cpk.pk;
     // running range of what this lane stores (float32 output with a kept range only)
     const bool keep = MODE == OUT_F32X && g.range != nullptr;
     auto track = [&](uint32_t bits) { kept.add(__uint_as_float(bits)); };
@@ -210,7 +212,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                 }
 #pragma unroll
                 for (int p = 0; p < PASSES; ++p) {
-                    store_vec4<MODE>(g, idx, v[p], cpk);
+                    store_vec4<MODE, kCodes>(g, idx, v[p], cpk);
                     idx += step;
                 }
             } else {
