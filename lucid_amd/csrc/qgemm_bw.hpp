@@ -212,7 +212,7 @@ __global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(1,
     __builtin_amdgcn_s_waitcnt(pp_vmcnt_imm(0));  // no direct load may land in LDS after this wavefront has ended
     __builtin_amdgcn_sched_barrier(0);
     RangeKeep kept;  // (no kept range in this kernel's output forms)
-    pp_epilogue<TM, TN, MODE>(g, acc, as_row, s_ws, s_bias, s_corr, n0, wm0, wn0, lane, rot, kept);
+    pp_epilogue<TM, TN, MODE, false>(g, acc, as_row, s_ws, s_bias, s_corr, n0, wm0, wn0, lane, rot, kept);
 }
 
 template <class Cfg, int MODE>

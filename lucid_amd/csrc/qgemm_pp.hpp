@@ -137,8 +137,9 @@ __device__ __forceinline__ int pp_rotation(const GemmArgs& g, int wn0) {
 // wn0 + 16 t + 4 (lane / 16) + r with t = the column tile of j (pp_rotation): four consecutive
 // columns per lane and tile, so scale, bias, ReLU / requantize / join run on registers and the
 // packed values are stored directly.  s_ws / s_bias / s_corr: the block's column parameters in
-// LDS (column n0 first); as_row: this lane's row scales.
-template <int TM, int TN, int MODE>
+// LDS (column n0 first); as_row: this lane's row scales.  CORRECTED: the accumulators started from the zero point's
+// correction, and s_corr is not read.
+template <int TM, int TN, int MODE, bool CORRECTED>
 __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM][TN], const float (&as_row)[TM],
                                             const float* s_ws, const float* s_bias, const int32_t* s_corr, int n0,
                                             int wm0, int wn0, int lane, int rot, RangeKeep& kept) {
@@ -186,7 +187,7 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
     typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
     typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
 
-    // ---- the plain float forms (aligned output, no residual, no ReLU, no zero-point correction)
+    // ---- the plain float forms (aligned output, no residual, no ReLU, no zero-point correction left)
     // when the matrix ends on a 16 x 16 tile boundary inside this sub-tile or beyond it: the same
     // float steps - convert, as * ws, multiply, add the bias - and nothing else.  Row pointers are
     // formed once and every store takes a constant offset from one of them; row blocks and column
@@ -197,7 +198,7 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
         const int zp = g.a_zp_dev ? int(g.a_zp_dev[0]) + g.a_zp : g.a_zp;
         const int ncols = g.N - wn0, nrows = g.M - wm0;
         const bool lean = g.ldo % 8 == 0 && reinterpret_cast<uintptr_t>(g.out) % 16 == 0 && g.residual == nullptr &&
-                          !g.relu && (g.wsum == nullptr || zp == 0) && (ncols >= TN * 16 || ncols % 16 == 0) &&
+                          !g.relu && (CORRECTED || g.wsum == nullptr || zp == 0) && (ncols >= TN * 16 || ncols % 16 == 0) &&
                           (nrows >= TM * 16 || nrows % 16 == 0);
         if (lean) {
             const int vt = ncols >= TN * 16 ? TN : ncols / 16;  // column tiles and row blocks inside the matrix
@@ -331,7 +332,7 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
         const int cl = nq - n0;  // column within the block tile, a multiple of 4
         const float4 ws = *reinterpret_cast<const float4*>(s_ws + cl);
         const float4 b = *reinterpret_cast<const float4*>(s_bias + cl);
-        const int4 cr = *reinterpret_cast<const int4*>(s_corr + cl);
+        const int4 cr = CORRECTED ? int4{0, 0, 0, 0} : *reinterpret_cast<const int4*>(s_corr + cl);
         c4[0] = ColParams{ws.x, b.x, cr.x}, c4[1] = ColParams{ws.y, b.y, cr.y};
         c4[2] = ColParams{ws.z, b.z, cr.z}, c4[3] = ColParams{ws.w, b.w, cr.w};
         if (prescaled) {
@@ -505,10 +506,6 @@ __global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(2,
     };
 
     pp_v4i acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = pp_v4i{0, 0, 0, 0};
 
     // The MFMAs of one k step, column by column; within a column the row order alternates, so
     // that only one operand changes from one instruction to the next (fewer operand bits
@@ -539,9 +536,21 @@ __global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(2,
     pair_load_all(1, std::true_type{});
     __builtin_amdgcn_sched_barrier(0);
     if (tid < BN) s_ws[tid] = c_mine.ws, s_bias[tid] = c_mine.bias, s_corr[tid] = c_mine.corr;
-    __builtin_amdgcn_s_waitcnt(pp_vmcnt_imm(2 * LB));  // stage 0 has landed: only B(1,2) may be outstanding
+    // stage 0 has landed: only B(1,2) may be outstanding (and the column parameters are in LDS: lgkmcnt(0))
+    __builtin_amdgcn_s_waitcnt(pp_vmcnt_imm(2 * LB) & ~(0xF << 8));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
+    // The sums start from the zero point's correction (exact): an instruction less per element in the epilogue, and
+    // the plain float forms serve asymmetric activations too (4096 x 4096 x 4096 to float32 in 256 x 352 tiles 75.6 -> 66.9
+    // us, 2048 x 11008 x 4096 89.2 -> 82.2, in 256 x 256 tiles 62.9 -> 61.9 and 105.1 -> 104.7).
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int t = (TN % 2 == 1 && j == TN - 1) ? (rot ? 0 : TN - 1) : j + rot;
+        int4 cr{0, 0, 0, 0};
+        if (MODE != OUT_ACC_I32) cr = *reinterpret_cast<const int4*>(s_corr + (wn0 - n0) + 16 * t + 4 * (lane >> 4));
+#pragma unroll
+        for (int i = 0; i < TM; ++i) acc[i][j] = pp_v4i{-cr.x, -cr.y, -cr.z, -cr.w};
+    }
 
     // Row scales of this lane's TM rows, fetched during the wavefront's last read phase.
     float as_row[TM];
@@ -592,7 +601,7 @@ __global__ __launch_bounds__(Cfg::THREADS) __attribute__((amdgpu_waves_per_eu(2,
     // issues its last MFMAs.
     __builtin_amdgcn_s_waitcnt(pp_vmcnt_imm(0));  // no direct load may land in LDS after this wavefront has ended
     RangeKeep kept;
-    pp_epilogue<TM, TN, MODE>(g, acc, as_row, s_ws, s_bias, s_corr, n0, wm0, wn0, lane, rot, kept);
+    pp_epilogue<TM, TN, MODE, true>(g, acc, as_row, s_ws, s_bias, s_corr, n0, wm0, wn0, lane, rot, kept);
     // one block per tile: the block's slot is the tile's (every wavefront has passed the same
     // number of barriers by now)
     if (MODE == OUT_F32X && g.range != nullptr) kept.store(g.range);

@@ -505,6 +505,27 @@ def test_ping_pong_kernel_exact(cfg, M, N, K):
 
 
 @pytest.mark.parametrize("cfg", [13, 14, 16, 21, 22])
+@pytest.mark.parametrize("M,N", [(256, 352), (272, 368), (512, 256), (257, 400), (300, 362)])
+def test_ping_pong_kernel_plain_float_forms_with_a_zero_point(cfg, M, N):
+    """The zero point's correction goes into what the accumulators start from; with it the plain float forms, which
+    skip tiles past the matrix whole, serve asymmetric activations: a zero point on either side, none of it in the
+    raw accumulators."""
+    rng = np.random.default_rng(cfg + M + N)
+    K = 192
+    a, w = codes(rng, (M, K)), codes(rng, (N, K))
+    wd = hip(w)
+    a_scale, w_scale = rng.uniform(0.005, 0.05, M).astype(np.float32), rng.uniform(0.0005, 0.004, N).astype(np.float32)
+    bias = (rng.standard_normal(N) * 0.3).astype(np.float32)
+    common = dict(a_zp=-128, a_zp_dev=hip(np.float32(203.0)), wsum=_ops.rowsum_i8(wd), path=TILE, tile_config=cfg)
+    acc = _ops.qlinear_i8(hip(a), wd, **common, out_mode=_ops.OUT_ACC_I32).numpy()
+    assert np.array_equal(acc, O.igemm(a, w))
+    for mode, omode, bits in ((_ops.OUT_F32, O.OUT_F32, np.uint32), (_ops.OUT_F16, O.OUT_F16, np.uint16)):
+        got = _ops.qlinear_i8(hip(a), wd, **common, a_scale=hip(a_scale), w_scale=hip(w_scale), bias=hip(bias), out_mode=mode).numpy()
+        want = O.qlinear(a, w, 75, a_scale, w_scale, bias=bias, out_mode=omode)
+        assert np.array_equal(got.view(bits), want.view(bits))
+
+
+@pytest.mark.parametrize("cfg", [13, 14, 16, 21, 22])
 @pytest.mark.parametrize("M,N,K", [(512, 704, 256), (300, 260, 128), (129, 1001, 64), (512, 768, 192)])
 def test_ping_pong_kernel_every_output_form(cfg, M, N, K):
     """Every epilogue form of the eight-wavefront kernel equals the oracle: an activation zero
