@@ -326,7 +326,9 @@ __global__ __launch_bounds__(256) void qlinear_w8a32_patch_kernel(
 
 // Long K: the block's four wavefronts share one 4-column x 8-row patch and take every fourth
 // 256-wide k step each (four times the loads in flight per output); partial sums meet in
-// LDS, then each wavefront folds and stores eight of the 32 outputs.
+// LDS, then each wavefront folds and stores eight of the 32 outputs.  Bound by the chain of latencies: two steps'
+// loads go together, the eight folds run side by side, and a lane finishes one output with a bias that came with the
+// first loads (32 x 1000 x 2048 11.0 us, folded, finished and stored one after the other, -> 9.0; 8 rows 8.6 -> 5.3).
 __global__ __launch_bounds__(256) void qlinear_w8a32_patch_k4_kernel(
     const float* __restrict__ x, const int8_t* __restrict__ w, const float* __restrict__ w_scale,
     const float* __restrict__ w_zp, const float* __restrict__ bias, int M, int N, int K, int relu,
@@ -350,47 +352,74 @@ __global__ __launch_bounds__(256) void qlinear_w8a32_patch_k4_kernel(
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = 0.0f;
-    for (int k = wave * 256 + lane * 4; k < K; k += 1024) {
+    // the output that the lane finishes (lanes from 8 on: none)
+    const int mine = wave * 8 + (lane & 7), mi = m0 + mine / NT, nj = n0 + mine % NT;
+    const bool finishes = lane < 8 && mi < M && nj < N;
+    const float b = (bias && finishes) ? bias[nj] : 0.0f;
+    const float S = do_fq ? S_[0] : 1.0f, Z = do_fq ? Z_[0] : 0.0f;
+    auto request = [&](int k, uint32_t (&c)[NT], float4 (&xv)[MT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) c[j] = *reinterpret_cast<const uint32_t*>(wr[j] + k);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) xv[i] = *reinterpret_cast<const float4*>(xr[i] + k);
+    };
+    auto add_step = [&](const uint32_t (&c)[NT], const float4 (&xv)[MT]) {
         float wv[NT][4];
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const uint32_t c = *reinterpret_cast<const uint32_t*>(wr[j] + k);
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                wv[j][e] = (float(int(int8_t((c >> (8 * e)) & 0xff))) - wz[j]) * ws[j];  // dequantize, _functional.py:281
-        }
+                wv[j][e] = (float(int(int8_t((c[j] >> (8 * e)) & 0xff))) - wz[j]) * ws[j];  // dequantize, _functional.py:281
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            const float4 xv = *reinterpret_cast<const float4*>(xr[i] + k);
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 float a = acc[i][j];
-                a = a + xv.x * wv[j][0];
-                a = a + xv.y * wv[j][1];
-                a = a + xv.z * wv[j][2];
-                a = a + xv.w * wv[j][3];
+                a = a + xv[i].x * wv[j][0];
+                a = a + xv[i].y * wv[j][1];
+                a = a + xv[i].z * wv[j][2];
+                a = a + xv[i].w * wv[j][3];
                 acc[i][j] = a;
             }
-        }
+    };
+    int k = wave * 256 + lane * 4;
+    for (; k + 1024 < K; k += 2048) {
+        uint32_t c0[NT], c1[NT];
+        float4 x0[MT], x1[MT];
+        request(k, c0, x0);
+        request(k + 1024, c1, x1);
+        add_step(c0, x0);
+        add_step(c1, x1);
+    }
+    if (k < K) {
+        uint32_t c0[NT];
+        float4 x0[MT];
+        request(k, c0, x0);
+        add_step(c0, x0);
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) red[wave][i * NT + j][lane] = acc[i][j];
     __syncthreads();
-    const float S = do_fq ? S_[0] : 1.0f, Z = do_fq ? Z_[0] : 0.0f;
+    float y[8];
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
-        const int idx = wave * 8 + o, i = idx / NT, j = idx % NT;
-        float y = ((red[0][idx][lane] + red[1][idx][lane]) + red[2][idx][lane]) + red[3][idx][lane];
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) y = y + __shfl_xor(y, d, 64);
-        if (lane != 0 || m0 + i >= M || n0 + j >= N) continue;
-        if (bias) y = y + bias[n0 + j];
-        if (relu) y = (y < 0.0f) ? 0.0f : y;
-        if (do_fq) y = (q_core(y, S, Z, lo, hi) - Z) * S;
-        out[size_t(m0 + i) * N + n0 + j] = y;
+        const int idx = wave * 8 + o;
+        y[o] = ((red[0][idx][lane] + red[1][idx][lane]) + red[2][idx][lane]) + red[3][idx][lane];
     }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1)
+#pragma unroll
+        for (int o = 0; o < 8; ++o) y[o] = y[o] + __shfl_xor(y[o], d, 64);
+    float v = y[0];
+#pragma unroll
+    for (int o = 1; o < 8; ++o) v = lane == o ? y[o] : v;
+    if (!finishes) return;
+    if (bias) v = v + b;
+    if (relu) v = (v < 0.0f) ? 0.0f : v;
+    if (do_fq) v = (q_core(v, S, Z, lo, hi) - Z) * S;
+    out[size_t(mi) * N + nj] = v;
 }
 
 inline unsigned grid_for(size_t n, size_t per_block) {

@@ -704,6 +704,33 @@ def test_edge_tiles_every_output_form(cfg, M, N):
         assert float(mn.numpy()) == y.min() and float(mx.numpy()) == y.max()
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 3, 1024), (9, 33, 1028), (8, 4, 2048), (33, 7, 2052), (5, 10, 3076), (12, 5, 5120)])
+@pytest.mark.parametrize("with_bias", [True, False])
+def test_float_input_long_k_patches(M, N, K, with_bias):
+    """lq_qlinear_w8a32 with K split between a block's wavefronts, steps taken in pairs: K at, just past and far past a
+    pair, output patches past the matrix.  A sum of K rounded products is off by at most (K + 2) 2^-24 of the sum of their
+    magnitudes; the fake-quantized form is the grid point of the float one."""
+    from lucid_amd import _C
+    rng = np.random.default_rng(M + N + K)
+    x, w = rng.standard_normal((M, K)).astype(np.float32), codes(rng, (N, K))
+    s, z = rng.uniform(0.001, 0.01, N).astype(np.float32), rng.integers(-3, 4, N).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    S, Z = np.float32(0.05), np.float32(3.0)
+    dx, dw, ds, dz, db, dS, dZ = (hip(v) for v in (x, w, s, z, b, S, Z))
+    wf = (w.astype(np.float32) - z[:, None]) * s[:, None]
+    want = x.astype(np.float64) @ wf.T.astype(np.float64) + (b if with_bias else 0.0)
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(wf).T.astype(np.float64) + np.abs(b))
+    got = []
+    for fake in (0, 1):
+        full = hip(np.full((M + 1, N), 77.0, np.float32))
+        _C.call("lq_qlinear_w8a32", dx.data_ptr, dw.data_ptr, ds.data_ptr, dz.data_ptr, db.data_ptr if with_bias else None, M, N,
+                K, fake, fake, dS.data_ptr, dZ.data_ptr, -128, 127, full.data_ptr, None)
+        got.append(full.numpy())
+        assert np.all(got[-1][M] == 77.0)
+    assert np.all(np.abs(got[0][:M] - want) <= bound)
+    assert np.array_equal(got[1][:M], O.fake_quantize(np.maximum(got[0][:M], np.float32(0)), S, Z, -128, 127))
+
+
 # ------------------------------------------------------------------ affine weight codes
 AFFINE_CASES = [
     # M, N, K, path
