@@ -661,7 +661,7 @@ constexpr int AT_D = 64, AT_TMAX = 208, AT_NT = AT_TMAX / 16, AT_WAVES = 4;
 constexpr int AT_VLD = AT_TMAX + 4;
 constexpr int AT_PART_K = AT_TMAX * AT_D, AT_PART_V = AT_D * AT_VLD;  // elements of one part
 constexpr size_t AT_SMEM = size_t(3) * (AT_PART_V > AT_PART_K ? AT_PART_V : AT_PART_K) * 2;
-static_assert(2 * (AT_SMEM + 192) <= 160 * 1024, "two blocks per CU, with the range reduction's few words");
+static_assert(2 * (AT_SMEM + 208) <= 160 * 1024, "two blocks per CU, with a flag and the range reduction's few words");
 
 typedef __bf16 at_v8bf __attribute__((ext_vector_type(8)));
 typedef short at_v4s __attribute__((ext_vector_type(4)));
@@ -672,6 +672,13 @@ __device__ __forceinline__ int at_k_index(int row, int col) {  // col a multiple
 // V^T's row of a column: tile j of the output is columns 4 i + j, i = 0..15, so that a lane has four consecutive floats of a
 // query at the end
 __device__ __forceinline__ int at_v_index(int j, int i, int key) { return (16 * j + i) * AT_VLD + key; }
+// P is up to 1 for every key until the division by its sum, so that 208 keys of one score add up to 208 max |V| on the way to a
+// result of max |V| at most.  For a head with values of V beyond AT_VMAX, whose sums could be infinite, P is 2^-8 of that: the
+// subtraction S - (max + 8) then rounds what S - max has exactly near the maximum, and scores close to each other give results
+// 2.9e-7 from float64 instead of 2.2e-7, which is why other heads do without.  (V times 2^-8 instead: the matrix instruction
+// takes the subnormal parts of |V| < 1e-31 for zero, and 768 heads take 68.0 us where they take 67.3 with V's maximum, 66.2 without.)
+constexpr float AT_VMAX = 0x1p119f;
+static_assert(AT_TMAX < 256, "AT_TMAX * AT_VMAX and 2^-8 * AT_TMAX * FLT_MAX are finite");
 // f over the four lanes of one number in the four rows of 16 lanes; every lane gets it
 template <class F>
 __device__ __forceinline__ float at_rows4(float v, F f) {
@@ -699,6 +706,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
                                                                      int parts, int out_vec, float scale,
                                                                      float* range) {
     extern __shared__ __attribute__((aligned(16))) uint16_t at_smem[];  // K's parts, then V^T's
+    __shared__ int s_large;  // V has values beyond AT_VMAX
     constexpr int THREADS = 64 * AT_WAVES, ROW4 = AT_D / 4;
     constexpr int KP = AT_TMAX * ROW4 / THREADS;  // 16-byte pieces of K per thread: one of every 16 rows
     constexpr int VP = (AT_TMAX + 31) / 32;       // pairs of such pieces of V: one of every 32 rows
@@ -767,6 +775,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));  // what follows from the lane is computed per item: kept across items, it would be spilled
         const int lane = tid & 63, g = lane >> 4, c = lane & 15;
+        if (tid == 0) s_large = 0;  // between the barrier at the end of the item before, past which nobody reads it, and the next
         // K rows into LDS as three bfloat16 parts
 #pragma unroll
         for (int u = 0; u < KP; ++u) {
@@ -842,6 +851,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
             for (int u = 0; u < 2 * VP; ++u) request_v(u / 2, u % 2);
         static_assert(AT_NT == 2 * VP - 1, "a piece of V per step, two in the last");
         __syncthreads();  // nobody reads K any more
+        float vmax = 0.0f;  // a NaN stays
 #pragma unroll
         for (int u = 0; u < VP; ++u) {
             if (32 * u + 32 > AT_TMAX && 32 * u + 2 * vpair >= AT_TMAX) continue;
@@ -849,6 +859,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
             const float a[4] = {v0.x, v0.y, v0.z, v0.w}, bb[4] = {v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                vmax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(vmax, __builtin_fabsf(a[e])), __builtin_fabsf(bb[e]));
                 uint32_t d[3];
                 at_split3x2(a[e], bb[e], d[0], d[1], d[2]);
 #pragma unroll
@@ -856,6 +867,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
                     *reinterpret_cast<uint32_t*>(at_smem + p * AT_PART_V + at_v_index(e, vcol / 4, 32 * u + 2 * vpair)) = d[p];
             }
         }
+        if (!(vmax <= AT_VMAX)) s_large = 1;
         float mx[QT], sum[QT][4];  // four sums of every fourth key each: shorter chains round less
         auto mask = [&](int t) {  // keys past the last token
 #pragma unroll
@@ -879,9 +891,13 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
             mx[q] = at_rows4(mx[q], [](float a, float b) { return __builtin_elementwise_maximum(a, b); });
         }
         __syncthreads();  // V^T is in LDS
+        if (s_large) {
+#pragma unroll
+            for (int q = 0; q < QT; ++q) mx[q] += 8.0f;
+        }
 
-        // O[q][n] = sum_key P[q][key] V[key][n] with P = 2^(S - max), divided by P's sum at the end, in four tiles of 16
-        // columns
+        // O[q][n] = sum_key P[q][key] V[key][n] with P = 2^(S - max), or 2^(S - max - 8) (AT_VMAX), divided by P's sum at the
+        // end, in four tiles of 16 columns
         static_assert(AT_NT % 2 == 1, "tile pairs and one single tile");
         constexpr int NJ = AT_D / 16;
         v4f o[QT][NJ];

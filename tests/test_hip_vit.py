@@ -94,6 +94,28 @@ def test_attention_against_float64(B, T, H, std):
     assert np.isnan(_range_of(bad)[0])
 
 
+@pytest.mark.parametrize("B,T,H", [(1, 208, 2), (1, 17, 3), (6, 197, 12)])
+@pytest.mark.parametrize("mag", [1e38, -1e38, 1e-30])
+def test_attention_of_values_near_the_ends_of_the_range(B, T, H, mag):
+    """A result is a mean of V's rows and no larger than the largest of them: sums on the way there stay finite for every
+    finite V that the mean keeps finite, and small ones lose nothing.  The bound of the test above."""
+    rng = np.random.default_rng(B + T)
+    qkv = rng.uniform(0.5, 2.0, (B, T, 3, H, 64)).astype(np.float32)
+    qkv[:, :, :2] = 0.03125 * rng.standard_normal((B, T, 2, H, 64))  # scores close to each other
+    v = qkv[:, :, 2].astype(np.float64) * np.where(np.arange(64) % 2, mag, abs(mag))  # one sign per column
+    qkv[:, :, 2] = v
+    out = F.scaled_dot_product_attention_qkv(hip(qkv.reshape(B, T, -1)), H, track_range=True)
+    got = out.numpy()
+    q, k, v = (qkv[:, :, i].astype(np.float64).transpose(0, 2, 1, 3) for i in range(3))
+    s = q @ k.transpose(0, 1, 3, 2) * 0.125
+    p = np.exp(s - s.max(-1, keepdims=True))
+    exp = ((p / p.sum(-1, keepdims=True)) @ v).transpose(0, 2, 1, 3).reshape(B, T, H * 64)
+    assert np.isfinite(got).all()
+    assert np.linalg.norm((got - exp) / mag) <= 2e-6 * np.linalg.norm(exp / mag)
+    kmn, kmx, _, _ = _range_of(out)
+    assert kmn == got.min() and kmx == got.max()
+
+
 def test_attention_rejects_what_the_kernel_does_not_cover():
     with pytest.raises(NotImplementedError):
         F.scaled_dot_product_attention_qkv(hip(np.zeros((1, 4, 3 * 2 * 32), np.float32)), 2)  # head dim 32
