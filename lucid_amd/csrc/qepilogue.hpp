@@ -345,15 +345,19 @@ __device__ __forceinline__ void store_scalar(const GemmArgs& g, size_t idx, uint
         static_cast<uint32_t*>(g.out)[idx] = v;  // f32 / i32 bit patterns
 }
 
-// four consecutive elements, of 8 and 16 bits at a vector's alignment, of 32 bits at any element
+// Four consecutive elements, or four codes of a join's other operand, at any element: a group of a convolution may begin at a
+// column that is no multiple of four.  (One instruction each, as with the types' own alignment.)
+typedef _Float16 unaligned_h4 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t unaligned_u4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t unaligned_codes4 __attribute__((aligned(1)));
+
 // PK: the caller knows that cpk.pk (a kernel asks before its loops: no element group then branches on it)
 template <int MODE, bool PK = false>
 __device__ __forceinline__ void store_vec4(const GemmArgs& g, size_t idx, uint4 v, const CodePack& cpk) {
     if (MODE == OUT_F16) {
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        h4 h = {_Float16(__uint_as_float(v.x)), _Float16(__uint_as_float(v.y)),
-                _Float16(__uint_as_float(v.z)), _Float16(__uint_as_float(v.w))};
-        *reinterpret_cast<h4*>(static_cast<_Float16*>(g.out) + idx) = h;
+        unaligned_h4 h = {_Float16(__uint_as_float(v.x)), _Float16(__uint_as_float(v.y)),
+                          _Float16(__uint_as_float(v.z)), _Float16(__uint_as_float(v.w))};
+        *reinterpret_cast<unaligned_h4*>(static_cast<_Float16*>(g.out) + idx) = h;
     } else if (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) {
         uint32_t packed;
         if (PK || cpk.pk) {
@@ -364,10 +368,9 @@ __device__ __forceinline__ void store_vec4(const GemmArgs& g, size_t idx, uint4 
             const uint32_t z = uint32_t(int(__uint_as_float(v.z))), w = uint32_t(int(__uint_as_float(v.w)));
             packed = ((x + o) & 0xffu) | (((y + o) & 0xffu) << 8) | (((z + o) & 0xffu) << 16) | ((w + o) << 24);
         }
-        *reinterpret_cast<uint32_t*>(static_cast<int8_t*>(g.out) + idx) = packed;
+        *reinterpret_cast<unaligned_codes4*>(static_cast<int8_t*>(g.out) + idx) = packed;
     } else {
-        typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
-        *reinterpret_cast<u4*>(static_cast<uint32_t*>(g.out) + idx) = u4{v.x, v.y, v.z, v.w};
+        *reinterpret_cast<unaligned_u4*>(static_cast<uint32_t*>(g.out) + idx) = unaligned_u4{v.x, v.y, v.z, v.w};
     }
 }
 

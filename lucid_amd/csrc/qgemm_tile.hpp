@@ -150,7 +150,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                 const int8_t* jq = g.join_q + size_t(m_first) * size_t(g.join_ld) + size_t(n);
 #pragma unroll
                 for (int p = 0; p < PASSES; ++p)
-                    jv[p] = *reinterpret_cast<const uint32_t*>(jq + size_t(p) * ROWS_PER_PASS * size_t(g.join_ld));
+                    jv[p] = *reinterpret_cast<const unaligned_codes4*>(jq + size_t(p) * ROWS_PER_PASS * size_t(g.join_ld));
             }
             // this lane's rows of the part: groups of four consecutive rows
             auto four_rows = [&](int q, auto pre, auto f, const float (&as)[4]) {
@@ -232,7 +232,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v16i (&acc)[Cfg
                         const int8_t* jq = g.join_q + size_t(m_first) * size_t(g.join_ld) + size_t(n);
 #pragma unroll
                         for (int p = 0; p < PASSES; ++p)
-                            if (p < passes) ej[p] = *reinterpret_cast<const uint32_t*>(jq + size_t(p) * ROWS_PER_PASS * size_t(g.join_ld));
+                            if (p < passes) ej[p] = *reinterpret_cast<const unaligned_codes4*>(jq + size_t(p) * ROWS_PER_PASS * size_t(g.join_ld));
                     }
 #pragma unroll
                     for (int p = 0; p < PASSES; ++p) {
@@ -726,9 +726,8 @@ __global__ __launch_bounds__(Cfg::THREADS, Cfg::MINWAVES) void qgemm_tile_kernel
         }
         const int esize = MODE == OUT_F16 ? 2 : ((MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) ? 1 : 4);
         const bool inside = m0 + BM <= g.M && n0 + BN <= n_limit;
-        // accesses to four elements of 32 bits need no alignment beyond an element's
+        // (groups of a convolution may still begin between two vectors: store_vec4 takes any element)
         const bool vec = esize == 4 || (g.ldo % 4 == 0 && reinterpret_cast<uintptr_t>(g.out) % (4 * esize) == 0 &&
-                                        (inside || n0 % 4 == 0) &&
                                         (g.join_q == nullptr ||
                                          (g.join_ld % 4 == 0 && reinterpret_cast<uintptr_t>(g.join_q) % 4 == 0)));
         __syncthreads();

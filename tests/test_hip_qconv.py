@@ -86,6 +86,34 @@ def test_gather_exact_at_every_tile_shape(case, cfg):
         assert np.array_equal(got, exp), schedule
 
 
+@pytest.mark.parametrize("cfg", [0, 1, 3, 5, 8, 10, 12])
+@pytest.mark.parametrize("groups,og", [(2, 66), (2, 130), (4, 33), (3, 260), (4, 65)])
+def test_groups_that_begin_between_two_vectors(groups, og, cfg):
+    """Rows of whole vectors, groups that begin 1 to 3 columns into one: tiles inside the output, on the edge of a group
+    and across its last vector, at every width of an element, and a join's operand read the same way."""
+    rng = np.random.default_rng(groups * og)
+    B, H, W, N = 2, 9, 8, groups * og
+    x, w = codes(rng, (B, H, W, 32 * groups)), codes(rng, (N, 1, 1, 32))
+    ws, bias = rng.uniform(5e-4, 4e-3, N).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    q = dict(out_qmin=0, out_qmax=255, out_offset=-128)
+    kw = dict(a_zp=-9, groups=groups, a_scale=hip(np.float32(0.02)), w_scale=hip(ws), wsum=_ops.rowsum_i8(hip(w)),
+              bias=hip(bias), out_scale=hip(np.float32(0.03)), out_zp=hip(np.float32(117)), path=IMPLICIT,
+              tile_config=cfg, **q)
+    exp = {m: O.qconv2d(x, w, -9, 0.02, ws, groups=groups, bias=bias, out_mode=m, out_scale=0.03, out_zp=117.0, **q)
+           for m in (O.OUT_ACC_I32, O.OUT_F32, O.OUT_F16, O.OUT_REQUANT_I8, O.OUT_FAKEQUANT_F32)}
+    for mode, e in exp.items():
+        got = _ops.qconv2d_i8(hip(x), hip(w), out_mode=mode, **kw).numpy()
+        assert got.tobytes() == e.tobytes(), mode
+    if N % 4:
+        return
+    other = codes(rng, exp[0].shape)
+    join = dict(q=hip(other), offset=-128, scale=hip(np.float32(0.025)), zp=hip(np.float32(131)), relu=True,
+                out_scale=hip(np.float32(0.04)), out_zp=hip(np.float32(7)), **q)
+    got = _ops.qconv2d_i8(hip(x), hip(w), out_mode=_ops.OUT_REQUANT_I8, join=join, **kw).numpy()
+    e = O.add_requant(exp[O.OUT_REQUANT_I8], -128, 0.03, 117.0, other, -128, 0.025, 131.0, True, 0.04, 7.0, 0, 255, -128)
+    assert np.array_equal(got, e)
+
+
 @pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[3], CASES[4], CASES[7]])
 @pytest.mark.parametrize("relu,bias_kind", [(True, "f32"), (False, "f32"), (True, None)])
 def test_epilogue_bit_exact(case, relu, bias_kind):
