@@ -641,10 +641,9 @@ __global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restric
 // Bound by the matrix pipe and the vector unit together: of the about 36 000 cycles that two blocks of
 // a CU take for a head of 197 tokens, the products are 16 800 of every SIMD, splits, exponentials and
 // LDS writes about as much, and at 64 x 12 heads the power limit holds the clock near 1.7 GHz.
-// 12 heads of 197 tokens 18.3 -> 10.5 us, 96 heads 20.1 -> 16.3, 384 46.4 -> 34.5, 768 77.4 -> 67.6
-// against one block of 16 wavefronts per head with K and V side by side (all K and V fragments read
-// once per 16 queries, the softmax a phase of its own).  The same eight wavefronts on a whole head with
-// K and V side by side (one split for all queries): 65.1 at 768 heads, but 41.5 against 32.5 at 288.
+// 12 heads of 197 tokens 18.3 -> 10.5 us, 96 heads 20.1 -> 14.9, 384 46.4 -> 34.5, 768 77.4 -> 67.6
+// against attention_head_kernel below, a block of 16 wavefronts per head with K and V side by side (all K and V fragments
+// read once per 16 queries, the softmax a phase of its own), which is kept for the counts of heads that give every CU one.
 //
 // Per wavefront: S^T = K . Q^T as 13 tiles of 16 keys x 16 queries (accumulators stay in
 // registers), softmax over the keys of each query (a lane holds 52 of a query's keys, the other
@@ -1030,6 +1029,249 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attention_kernel(const float
     if (range) kept.store(range);
 }
 
+// One block per head, one wavefront per tile of 16 queries, K's parts and V^T's side by side in LDS: after the one barrier
+// that follows the splits a wavefront runs scores, softmax and P . V on its own.  K and V are split once per head where the
+// kernel above splits them once per part, which is what counts while every CU has one head (see lq_attention_f32 for the line
+// and both sides' times); each fragment serves 16 queries.  The probabilities are normalized before P . V.
+constexpr size_t AT_HEAD_SMEM = size_t(3) * (AT_PART_K + AT_PART_V) * 2;
+static_assert(AT_HEAD_SMEM + 1024 <= 160 * 1024, "LDS of a CU, with the range reduction's few words");
+
+// acc += a . b from the parts, smallest terms first
+template <class V>
+__device__ __forceinline__ v4f at_mma6(const V (&a)[3], const V (&b)[3], v4f acc) {
+#pragma unroll
+    for (int x = 0; x < 6; ++x) acc = at_mm(a[kAtPa[x]], b[kAtPb[x]], acc);
+    return acc;
+}
+
+__global__ __launch_bounds__(1024) void attention_head_kernel(const float* __restrict__ qkv, float* __restrict__ out, int T,
+                                                             int H, float scale, float* range) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t at_smem[];
+    uint16_t* const k_lds = at_smem;
+    uint16_t* const v_lds = at_smem + 3 * AT_PART_K;
+    const int b = blockIdx.x / H, h = blockIdx.x % H;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const size_t tok_stride = size_t(3) * H * AT_D;
+    const float* base = qkv + size_t(b) * T * tok_stride + size_t(h) * AT_D;
+    // K and V are requested before anything is used (a block of 13 wavefronts holds all of both: four
+    // 16-byte pieces of each per thread).  A thread's V pieces are two pairs of consecutive keys at the
+    // same four columns: V^T keeps a column's keys contiguous, so a pair of keys is one dword of each part
+    constexpr int kPieces = AT_TMAX * (AT_D / 4), kHeld = 4;
+    constexpr int kPairs = (AT_TMAX / 2) * (AT_D / 4);
+    float4 kheld[kHeld], vheld[kHeld];
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        const int i = tid + u * int(blockDim.x), row = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
+        kheld[u] = float4{0.f, 0.f, 0.f, 0.f};
+        if (i < kPieces && row < T) kheld[u] = *reinterpret_cast<const float4*>(base + size_t(row) * tok_stride + size_t(H) * AT_D + c4);
+    }
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        const int i = tid + (u >> 1) * int(blockDim.x), row = 2 * (i / (AT_D / 4)) + (u & 1), c4 = (i % (AT_D / 4)) * 4;
+        vheld[u] = float4{0.f, 0.f, 0.f, 0.f};
+        if (i < kPairs && row < T) vheld[u] = *reinterpret_cast<const float4*>(base + size_t(row) * tok_stride + size_t(2) * H * AT_D + c4);
+    }
+    // One wavefront per tile of 16 queries.  With 4 n + 1 tiles one SIMD would hold a wavefront more
+    // than the others and everybody would wait for it: the launch then has three more wavefronts,
+    // and the last tile's four each compute its scores but only one 16-column tile of its output.
+    const int tiles = (T + 15) / 16;
+    const bool shared_last = int(blockDim.x) > tiles * 64;
+    const int q0 = (wave < tiles ? wave : tiles - 1) * 16;
+    const int only_j = (shared_last && wave >= tiles - 1) ? wave - (tiles - 1) : -1;  // wavefront-uniform
+    const int g = lane >> 4, c = lane & 15;
+    // the lane's slice of its query row: Q[q0 + c][32 u + 8 g + 0..7]
+    float4 qheld[2 * (AT_D / 32)];
+    {
+        const int q = q0 + c;
+        const float* qp = base + size_t(q < T ? q : T - 1) * tok_stride;
+#pragma unroll
+        for (int u = 0; u < AT_D / 32; ++u) {
+            qheld[2 * u] = *reinterpret_cast<const float4*>(qp + 32 * u + 8 * g);
+            qheld[2 * u + 1] = *reinterpret_cast<const float4*>(qp + 32 * u + 8 * g + 4);
+        }
+    }
+    // K rows into LDS as three bfloat16 parts (rows past T are zero)
+    auto place_k = [&](int i, float4 kv) {
+        const int row = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
+        uint32_t lo[3], hi[3];
+        at_split3x2(kv.x, kv.y, lo[0], lo[1], lo[2]);
+        at_split3x2(kv.z, kv.w, hi[0], hi[1], hi[2]);
+        const int at = at_k_index(row, c4);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(k_lds + p * AT_PART_K + at) = uint2{lo[p], hi[p]};
+    };
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        const int i = tid + u * int(blockDim.x);
+        if (i < kPieces) place_k(i, kheld[u]);
+    }
+    for (int i = tid + kHeld * int(blockDim.x); i < kPieces; i += blockDim.x) {  // fewer than 13 wavefronts
+        const int row = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
+        float4 kv = {0.f, 0.f, 0.f, 0.f};
+        if (row < T) kv = *reinterpret_cast<const float4*>(base + size_t(row) * tok_stride + size_t(H) * AT_D + c4);
+        place_k(i, kv);
+    }
+    // V^T's parts: keys 2 pair and 2 pair + 1 at columns c4 .. c4 + 3 (keys past T are zero)
+    auto place_v = [&](int i, float4 v0, float4 v1) {
+        const int pair = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
+        const float a[4] = {v0.x, v0.y, v0.z, v0.w}, bb[4] = {v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t d[3];
+            at_split3x2(a[e], bb[e], d[0], d[1], d[2]);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                *reinterpret_cast<uint32_t*>(v_lds + p * AT_PART_V + (c4 + e) * AT_VLD + 2 * pair) = d[p];
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < kHeld / 2; ++u) {
+        const int i = tid + u * int(blockDim.x);
+        if (i < kPairs) place_v(i, vheld[2 * u], vheld[2 * u + 1]);
+    }
+    for (int i = tid + (kHeld / 2) * int(blockDim.x); i < kPairs; i += blockDim.x) {  // fewer than 13 wavefronts
+        const int pair = i / (AT_D / 4), c4 = (i % (AT_D / 4)) * 4;
+        float4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = {0.f, 0.f, 0.f, 0.f};
+        const float* vp = base + size_t(2) * H * AT_D + c4;
+        if (2 * pair < T) v0 = *reinterpret_cast<const float4*>(vp + size_t(2 * pair) * tok_stride);
+        if (2 * pair + 1 < T) v1 = *reinterpret_cast<const float4*>(vp + size_t(2 * pair + 1) * tok_stride);
+        place_v(i, v0, v1);
+    }
+    // B operand of S^T, pre-scaled so that S = scale * log2(e) * Q.K^T (the scores are kept in the
+    // base-2 domain, so that the softmax numerators are one v_exp_f32 each)
+    uint4 qf[AT_D / 32][3];
+    {
+        const float qs = scale * 1.4426950408889634f;
+#pragma unroll
+        for (int u = 0; u < AT_D / 32; ++u) {
+            const float4 a = qheld[2 * u], bq = qheld[2 * u + 1];
+            const float v[8] = {a.x * qs, a.y * qs, a.z * qs, a.w * qs, bq.x * qs, bq.y * qs, bq.z * qs, bq.w * qs};
+            uint32_t d[3][4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) at_split3x2(v[2 * e], v[2 * e + 1], d[0][e], d[1][e], d[2][e]);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) qf[u][p] = uint4{d[p][0], d[p][1], d[p][2], d[p][3]};
+        }
+    }
+    __syncthreads();  // the only one before the range reduction: from here on a wavefront is on its own
+    v4f st[AT_NT];
+#pragma unroll
+    for (int t = 0; t < AT_NT; ++t) st[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    // k slice outermost: the 13 tiles' accumulators are independent chains
+#pragma unroll
+    for (int u = 0; u < AT_D / 32; ++u)
+#pragma unroll
+        for (int t = 0; t < AT_NT; ++t) {
+            uint4 kf[3];
+            const int at = at_k_index(16 * t + c, 32 * u + 8 * g);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) kf[p] = *reinterpret_cast<const uint4*>(k_lds + p * AT_PART_K + at);
+            st[t] = at_mma6(kf, qf[u], st[t]);
+        }
+    // st[t][r] = S[query q0 + c][key 16t + 4g + r]
+    float mx = -__builtin_inff();
+#pragma unroll
+    for (int t = 0; t < AT_NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int key = 16 * t + 4 * g + r;
+            if (key >= T) st[t][r] = -__builtin_inff();
+            mx = fmaxf(mx, st[t][r]);
+        }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    float sum = 0.0f;
+#pragma unroll
+    for (int t = 0; t < AT_NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float e = __builtin_amdgcn_exp2f(st[t][r] - mx);  // 2^(-inf) = 0 for the padded keys
+            st[t][r] = e;
+            sum += e;
+        }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+
+    // O[q][n] = sum_key P[q][key] V[key][n], four 16-wide column tiles; tile j of the output holds
+    // head-dim columns 16 j + c: the 16 lanes of a fragment read consecutive V^T rows (rows 4 c + j,
+    // which would let a lane store four consecutive floats, fall on four bank pairs only)
+    static_assert(AT_NT % 2 == 1, "tile pairs and one single tile");
+    v4f o[AT_D / 16];
+#pragma unroll
+    for (int j = 0; j < AT_D / 16; ++j) o[j] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int tp = 0; tp < AT_NT / 2; ++tp) {
+        // the eight k slots of this lane: keys 32 tp + 4 g + 0..3 and 32 tp + 16 + 4 g + 0..3
+        float pv[8];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            pv[r] = st[2 * tp][r] * inv;
+            pv[4 + r] = st[2 * tp + 1][r] * inv;
+        }
+        uint32_t d[3][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) at_split3x2(pv[2 * e], pv[2 * e + 1], d[0][e], d[1][e], d[2][e]);
+        uint4 pf[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) pf[p] = uint4{d[p][0], d[p][1], d[p][2], d[p][3]};
+#pragma unroll
+        for (int j = 0; j < AT_D / 16; ++j) {
+            if (only_j >= 0 && only_j != j) continue;
+            uint4 vf[3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                const uint16_t* vrow = v_lds + p * AT_PART_V + (16 * j + c) * AT_VLD + 32 * tp + 4 * g;
+                const uint2 lo = *reinterpret_cast<const uint2*>(vrow), hi = *reinterpret_cast<const uint2*>(vrow + 16);
+                vf[p] = uint4{lo.x, lo.y, hi.x, hi.y};
+            }
+            o[j] = at_mma6(pf, vf, o[j]);
+        }
+    }
+    {
+        // the last tile: keys 16 (AT_NT - 1) + 4 g + 0..3, four k slots per lane
+        float pv[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pv[r] = st[AT_NT - 1][r] * inv;
+        uint32_t d[3][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) at_split3x2(pv[2 * e], pv[2 * e + 1], d[0][e], d[1][e], d[2][e]);
+        uint2 pf[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) pf[p] = uint2{d[p][0], d[p][1]};
+#pragma unroll
+        for (int j = 0; j < AT_D / 16; ++j) {
+            if (only_j >= 0 && only_j != j) continue;
+            uint2 vf[3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                vf[p] = *reinterpret_cast<const uint2*>(v_lds + p * AT_PART_V + (16 * j + c) * AT_VLD + 16 * (AT_NT - 1) + 4 * g);
+            o[j] = at_mma6(pf, vf, o[j]);
+        }
+    }
+    // result layout of the 16x16 MFMA: column slot = lane % 16, row = 4*(lane/16) + r; the 16 lanes
+    // of a row store 64 consecutive bytes
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int q = q0 + 4 * g + r;
+        if (q < T) {
+            float* orow = out + (size_t(b) * T + q) * (size_t(H) * AT_D) + size_t(h) * AT_D + c;
+#pragma unroll
+            for (int j = 0; j < AT_D / 16; ++j)
+                if (only_j < 0 || only_j == j) orow[16 * j] = o[j][r];
+        }
+    }
+    if (range) {
+        RangeKeep kept;
+#pragma unroll
+        for (int j = 0; j < AT_D / 16; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (q0 + 4 * g + r < T && (only_j < 0 || only_j == j)) kept.add(o[j][r]);
+        kept.store(range);
+    }
+}
+
 unsigned blocks_for(size_t n) { return unsigned((n + 255) / 256); }
 
 }  // namespace
@@ -1228,28 +1470,40 @@ int lq_attention_f32(const float* qkv, float* out, int B, int T, int H, int D, f
     LQ_REQUIRE(range == nullptr || long(B) * H <= kRangeSlots, LQ_ERR_SHAPE,
                "attention: too many (batch, head) pairs for a kept range");
     const int heads = B * H, tiles = (T + 15) / 16;
+    constexpr long kSlots = 512;  // two blocks of attention_kernel on each of 256 CUs, which take further items in turn
+    const auto blocks = [&](int qt) { return (long(heads) + 7) / 8 * 8 * ((tiles + qt * AT_WAVES - 1) / (qt * AT_WAVES)); };
     const auto launch = [&](auto qt, auto wide) -> int {
         constexpr int QT = decltype(qt)::value;
         const auto kernel = attention_kernel<QT, decltype(wide)::value>;
         static DeviceOnce attr_once;
         if (int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(kernel), int(AT_SMEM))) return rc;
-        const int parts = (tiles + QT * AT_WAVES - 1) / (QT * AT_WAVES);
-        const long items = (long(heads) + 7) / 8 * 8 * parts;
-        constexpr long kSlots = 512;  // two blocks on each of 256 CUs, which take further items in turn
+        const long items = blocks(QT);
         kernel<<<unsigned(items < kSlots ? items : kSlots), 64 * AT_WAVES, AT_SMEM, as_stream(stream)>>>(
-            qkv, out, T, H, heads, parts, aligned16(out), scale, range);
+            qkv, out, T, H, heads, int(items / ((long(heads) + 7) / 8 * 8)), aligned16(out), scale, range);
         return LQ_OK;
     };
-    // One tile of queries per wavefront while the blocks do not outnumber the CUs (12 heads of 197 tokens 10.5 us against
-    // 14.7 with two); beyond that they would only share them (96 heads: 16.3 either way, 288: 34.7 against 32.2).
+    // One tile of queries per wavefront while that makes no more blocks than have a place at once, or no more than two tiles
+    // would (up to 64 tokens: 1100 heads of 64 tokens 32.2 us against 34.6 with two): 64 heads of 197 tokens 10.5 (15.0 with
+    // two, 17.7 in one block per head), 160 heads of 160 tokens 15.6 (20.5, 17.5), 768 heads of 193 tokens 73.6 (59.1, 66.4).
+    // One block per head while every CU has one head and either of the others would give it two blocks: 192 heads of 130
+    // tokens 15.4 (20.4 with one tile per wavefront, 20.2 with two), 192 of 65 tokens 12.3 (14.7, 15.0), 192 of 193 tokens 19.2
+    // (20.9, 21.0).  With two blocks the CU does two thirds more for them than one block does, which longer heads
+    // earn back from about 2912 tiles on: 224 heads of 208 tokens 21.1 (26.8, 21.9), 256 of them 24.1 (27.0, 22.6).
     using One = std::integral_constant<int, 1>;
     int rc;
-    if (size_t(H) * 3 * AT_D * 4 * 32 > UINT32_MAX)
+    if (size_t(H) * 3 * AT_D * 4 * 32 > UINT32_MAX) {
         rc = launch(One{}, std::true_type{});
-    else if (heads <= 64)
+    } else if (tiles <= AT_WAVES || blocks(1) <= (tiles <= 2 * AT_WAVES ? kSlots / 2 : kSlots)) {
         rc = launch(One{}, std::false_type{});
-    else
+    } else if (heads <= 256 && heads * tiles <= 2912) {
+        static DeviceOnce attr_once;
+        rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(attention_head_kernel), int(AT_HEAD_SMEM));
+        const int waves = tiles + (tiles % 4 == 1 ? 3 : 0);  // see the kernel: the last tile shared by four
+        if (rc == LQ_OK)
+            attention_head_kernel<<<unsigned(heads), waves * 64, AT_HEAD_SMEM, as_stream(stream)>>>(qkv, out, T, H, scale, range);
+    } else {
         rc = launch(std::integral_constant<int, 2>{}, std::false_type{});
+    }
     if (rc) return rc;
     LQ_CHECK_LAUNCH();
     return LQ_OK;

@@ -71,9 +71,14 @@ def test_attention_on_packed_qkv(B, T, H):
     assert rel(got, exp) < 1e-4
 
 
-@pytest.mark.parametrize("B,T,H,std", [(1, 197, 64, 1.0), (5, 65, 13, 1.0),     # the last count with one tile per wavefront, the first with two
+@pytest.mark.parametrize("B,T,H,std", [(1, 197, 64, 1.0), (5, 65, 13, 1.0),
                                        (4, 129, 67, 1.0), (43, 17, 12, 3.0),     # blocks that take a second item, heads not in eights
-                                       (22, 197, 12, 2.0), (1, 208, 65, 0.1)])
+                                       (22, 197, 12, 2.0), (1, 208, 65, 0.1),
+                                       (3, 64, 171, 1.0),                          # four tiles: one per wavefront for any count
+                                       (8, 65, 16, 1.0), (3, 65, 43, 1.0), (2, 128, 128, 1.0), (1, 65, 257, 1.0),   # the last
+                                       # count with one tile per wavefront, the first and last with a block per head, the first with two
+                                       (4, 144, 42, 1.0), (1, 129, 169, 1.0), (8, 130, 32, 2.0), (2, 192, 121, 1.0),
+                                       (16, 197, 8, 1.0), (1, 193, 129, 1.0), (8, 208, 28, 0.1), (1, 193, 225, 1.0)])
 def test_attention_against_float64(B, T, H, std):
     """Scores and results are sums of 64 and T products, each exact to 2^-24 and accumulated in float32, behind
     exponentials good to an ulp: relative errors of a few 2^-24 per output (measured 1.4e-7 to 6e-7, growing with the scores)."""
@@ -94,7 +99,7 @@ def test_attention_against_float64(B, T, H, std):
     assert np.isnan(_range_of(bad)[0])
 
 
-@pytest.mark.parametrize("B,T,H", [(1, 208, 2), (1, 17, 3), (6, 197, 12)])
+@pytest.mark.parametrize("B,T,H", [(1, 208, 2), (1, 17, 3), (6, 197, 12), (16, 193, 12), (21, 197, 12)])
 @pytest.mark.parametrize("mag", [1e38, -1e38, 1e-30])
 def test_attention_of_values_near_the_ends_of_the_range(B, T, H, mag):
     """A result is a mean of V's rows and no larger than the largest of them: sums on the way there stay finite for every
