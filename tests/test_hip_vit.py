@@ -121,6 +121,25 @@ def test_attention_of_values_near_the_ends_of_the_range(B, T, H, mag):
     assert kmn == got.min() and kmx == got.max()
 
 
+def test_attention_of_a_row_beyond_32_bits():
+    """The first count of heads whose 32 token rows of the packed activation span more than 2^32 bytes: offsets of 64 bits,
+    blocks that take many items with one tile of queries per wavefront.  The bound of the tests above, on every head."""
+    T, H = 2, (1 << 32) // (3 * 64 * 4 * 32) + 1
+    rng = np.random.default_rng(H)
+    qkv = rng.standard_normal((T, 3, H, 64), dtype=np.float32)
+    x = hip(qkv.reshape(1, T, -1))
+    got = F.scaled_dot_product_attention_qkv(x, H).numpy().reshape(T, H, 64)
+    q, k, v = (qkv[:, i].transpose(1, 0, 2).astype(np.float64) for i in range(3))
+    s = q @ k.transpose(0, 2, 1) * 0.125
+    p = np.exp(s - s.max(-1, keepdims=True))
+    exp = ((p / p.sum(-1, keepdims=True)) @ v).transpose(1, 0, 2)
+    err = np.linalg.norm((got - exp).transpose(1, 0, 2).reshape(H, -1), axis=1)
+    assert (err <= 4e-6 * np.linalg.norm(exp.transpose(1, 0, 2).reshape(H, -1), axis=1)).all()  # per head: twice the bound overall
+    assert np.linalg.norm(got - exp) <= 2e-6 * np.linalg.norm(exp)
+    with pytest.raises(L.ShapeMismatch):  # a kept range stays limited to 16384 heads
+        F.scaled_dot_product_attention_qkv(x, H, track_range=True)
+
+
 def test_attention_rejects_what_the_kernel_does_not_cover():
     with pytest.raises(NotImplementedError):
         F.scaled_dot_product_attention_qkv(hip(np.zeros((1, 4, 3 * 2 * 32), np.float32)), 2)  # head dim 32
