@@ -334,6 +334,14 @@ __device__ __forceinline__ uint32_t pack_codes_pk(uint4 v, const CodePack& cpk) 
     packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.w), 3, packed);
     return packed ^ cpk.flip;
 }
+// the same for any grid
+__device__ __forceinline__ uint32_t pack_codes(uint4 v, const CodePack& cpk) {
+    if (cpk.pk) return pack_codes_pk(v, cpk);
+    const uint32_t o = uint32_t(cpk.add);
+    const uint32_t x = uint32_t(int(__uint_as_float(v.x))), y = uint32_t(int(__uint_as_float(v.y)));
+    const uint32_t z = uint32_t(int(__uint_as_float(v.z))), w = uint32_t(int(__uint_as_float(v.w)));
+    return ((x + o) & 0xffu) | (((y + o) & 0xffu) << 8) | (((z + o) & 0xffu) << 16) | ((w + o) << 24);
+}
 
 template <int MODE>
 __device__ __forceinline__ void store_scalar(const GemmArgs& g, size_t idx, uint32_t v, const CodePack& cpk) {
@@ -359,15 +367,7 @@ __device__ __forceinline__ void store_vec4(const GemmArgs& g, size_t idx, uint4 
                           _Float16(__uint_as_float(v.z)), _Float16(__uint_as_float(v.w))};
         *reinterpret_cast<unaligned_h4*>(static_cast<_Float16*>(g.out) + idx) = h;
     } else if (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) {
-        uint32_t packed;
-        if (PK || cpk.pk) {
-            packed = pack_codes_pk(v, cpk);
-        } else {
-            const uint32_t o = uint32_t(cpk.add);
-            const uint32_t x = uint32_t(int(__uint_as_float(v.x))), y = uint32_t(int(__uint_as_float(v.y)));
-            const uint32_t z = uint32_t(int(__uint_as_float(v.z))), w = uint32_t(int(__uint_as_float(v.w)));
-            packed = ((x + o) & 0xffu) | (((y + o) & 0xffu) << 8) | (((z + o) & 0xffu) << 16) | ((w + o) << 24);
-        }
+        const uint32_t packed = PK ? pack_codes_pk(v, cpk) : pack_codes(v, cpk);
         *reinterpret_cast<unaligned_codes4*>(static_cast<int8_t*>(g.out) + idx) = packed;
     } else {
         *reinterpret_cast<unaligned_u4*>(static_cast<uint32_t*>(g.out) + idx) = unaligned_u4{v.x, v.y, v.z, v.w};

@@ -98,20 +98,7 @@ __device__ __forceinline__ void pp_pack(uint4 v, const CodePack& cpk, uint32_t* 
         dw[0] = __builtin_bit_cast(uint32_t, a);
         dw[1] = __builtin_bit_cast(uint32_t, b);
     } else if (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) {
-        uint32_t packed;
-        if (cpk.pk) {
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.x), 0, 0u);
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.y), 1, packed);
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.z), 2, packed);
-            packed = __builtin_amdgcn_cvt_pk_u8_f32(__uint_as_float(v.w), 3, packed);
-            packed ^= cpk.flip;
-        } else {
-            const uint32_t o = uint32_t(cpk.add);
-            const uint32_t x = uint32_t(int(__uint_as_float(v.x))), y = uint32_t(int(__uint_as_float(v.y)));
-            const uint32_t z = uint32_t(int(__uint_as_float(v.z))), w = uint32_t(int(__uint_as_float(v.w)));
-            packed = ((x + o) & 0xffu) | (((y + o) & 0xffu) << 8) | (((z + o) & 0xffu) << 16) | ((w + o) << 24);
-        }
-        dw[0] = packed;
+        dw[0] = pack_codes(v, cpk);
     } else {
         dw[0] = v.x, dw[1] = v.y, dw[2] = v.z, dw[3] = v.w;
     }
