@@ -146,7 +146,12 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
     const CodePack cpk = make_code_pack<MODE>(g, MODE == OUT_REQUANT_JOIN ? jp.out : G);
     constexpr int esize = MODE == OUT_F16 ? 2 : ((MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN) ? 1 : 4);
     constexpr bool kFloatOut = MODE == OUT_F32 || MODE == OUT_F16 || MODE == OUT_F32X;
-    const EpilogueForm form = kFloatOut ? epilogue_form(g) : kFormAny;
+    // Float16 comes past the plain form below for the edges of a ragged M, mostly, and with row scales, which the forms
+    // without them do not serve: their code made those edges 2-3 % slower (3000 x 8192 x 2048 57.0 -> 58.3 us, 1000 x
+    // 8192 x 2048 22.3 -> 22.9).  The 352-column tiles, whose registers the compiler deals out otherwise, are 2-3 % faster with it
+    // (2048 x 11008 x 4096 77.2 -> 75.5, 2049 x 8192 x 2048 41.2 -> 39.9).
+    constexpr bool kForms = MODE == OUT_F32 || MODE == OUT_F32X || (MODE == OUT_F16 && TN % 2 == 1);
+    const EpilogueForm form = kForms ? epilogue_form(g) : kFormAny;
     const bool prescaled = (MODE == OUT_REQUANT_I8 || MODE == OUT_REQUANT_JOIN || form != kFormAny) && !g.a_scale_per_row;
     const bool cols_in = wn0 + TN * 16 <= g.N, rows_in = wm0 + TM * 16 <= g.M;
     // uniform: every access of this wavefront may be a whole aligned vector
@@ -291,7 +296,7 @@ __device__ __forceinline__ void pp_epilogue(const GemmArgs& g, pp_v4i (&acc)[TM]
     // place among the wavefront's accumulators
     auto tile_values = [&](int m, const pp_v4i& a, const ColParams (&c4)[4], float as, int nq, uint4& v, int ri, int rj) {
         auto one_scale = [&](auto f) { v = epilogue_quad<MODE, true, decltype(f)::value>(g, a, 1.0f, c4, G); };
-        if (prescaled && kFloatOut && form == kFormPlain) {
+        if (kForms && prescaled && form == kFormPlain) {
             one_scale(std::integral_constant<EpilogueForm, kFormPlain>{});
         } else if (prescaled && MODE == OUT_F32X) {
             one_scale(std::integral_constant<EpilogueForm, kFormGelu>{});
