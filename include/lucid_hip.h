@@ -570,7 +570,7 @@ int lq_add_f32(const float* a, const float* b, float* out, size_t n, lq_stream s
  * softmax(scale * Q K^T) V, no mask, no dropout) read straight from the packed
  * activation of the qkv Linear, [B, T, 3, H, D] (vit/_model.py:137-141), writing
  * [B, T, H*D] (vit/_model.py:158).  D must be 64 and T <= 208 (ViT-B/16: T = 197);
- * anything else returns LQ_ERR_NOT_IMPLEMENTED. */
+ * anything else returns LQ_ERR_NOT_IMPLEMENTED.  With a kept range B * H is at most 16384. */
 int lq_attention_f32(const float* qkv, float* out, int B, int T, int H, int D, float scale,
                      float* range, lq_stream stream);
 

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         return Box{t / q.tiles_h, thi * 16, twi * 16};
     };
     auto halo_chunk = [&](const Box& o, int i) {
-        // i < 2560 and HWq <= 160 (15 rows at least): the 20-bit reciprocal gives the exact quotient
+        // i < 2560 and HWq <= 160 (16 rows at least): the 20-bit reciprocal gives the exact quotient
         const int r = int((unsigned(i) * q.inv_hwq) >> 20), cq = i - r * q.HWq;
         const int ih = o.oh0 * q.sh + r, pix = o.ow0 * q.sw + cq * 4;  // ow0 * sw * 4 bytes is a multiple of 16
         // rows and pixel quads past the image belong to positions past the output: never stored

@@ -1467,8 +1467,9 @@ int lq_attention_f32(const float* qkv, float* out, int B, int T, int H, int D, f
                "attention: head dim %d / %d tokens; this kernel handles head dim 64 and up to 208 tokens", D, T);
     LQ_REQUIRE(aligned16(qkv), LQ_ERR_VALUE, "attention: qkv must be 16-byte aligned");
     if (B == 0) return LQ_OK;
+    // (the call's limit: the kernels here use a slot per block and at most 512 of them, a slot per head would take one each)
     LQ_REQUIRE(range == nullptr || long(B) * H <= kRangeSlots, LQ_ERR_SHAPE,
-               "attention: too many (batch, head) pairs for a kept range");
+               "attention: a kept range is limited to %d (batch, head) pairs, got %ld", kRangeSlots, long(B) * H);
     const int heads = B * H, tiles = (T + 15) / 16;
     constexpr long kSlots = 512;  // two blocks of attention_kernel on each of 256 CUs, which take further items in turn
     const auto blocks = [&](int qt) { return (long(heads) + 7) / 8 * 8 * ((tiles + qt * AT_WAVES - 1) / (qt * AT_WAVES)); };
