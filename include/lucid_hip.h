@@ -472,6 +472,10 @@ int lq_quantize_tensor_dynamic_polls_i8(const float* x, size_t rows, unsigned co
 int lq_dynamic_linear_small_f32(const float* x, int M, int K, const int8_t* w, int N, const float* w_scale,
                                 const int32_t* wsum, const float* bias, int relu, int symmetric, int qmin, int qmax,
                                 int is_signed, float eps, int code_offset, float* out, lq_stream stream);
+/* The same for any K: weight rows of `ldw` bytes (K codes, then zeros: a multiple of 16 up to 6080), 16-byte aligned like x. */
+int lq_dynamic_linear_small_rows_f32(const float* x, int M, int K, const int8_t* w, int ldw, int N, const float* w_scale,
+                                     const int32_t* wsum, const float* bias, int relu, int symmetric, int qmin, int qmax,
+                                     int is_signed, float eps, int code_offset, float* out, lq_stream stream);
 
 /* nnqd.Linear.forward for any activation: x [M, K] float32, per-tensor qparams from its runtime min / max, w [N]
  * rows of `ldw` bytes (K codes, then zeros: a multiple of 16, 16-byte aligned), wsum [N] their sums.  One row is
@@ -496,6 +500,13 @@ int lq_dynamic_mlp2_small_f32(const float* x, int M, int K1, const int8_t* w1, i
                               const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2, int symmetric,
                               int qmin, int qmax, int is_signed, float eps, int code_offset, float* out,
                               lq_stream stream);
+/* The same for any K1 and a hidden width up to 511: weight rows of ldw1 (up to 1024) and ldw2 (up to 512) bytes, codes, then
+ * zeros, multiples of 16. */
+int lq_dynamic_mlp2_small_rows_f32(const float* x, int M, int K1, const int8_t* w1, int ldw1, int N1, const float* w1_scale,
+                                   const int32_t* w1sum, const float* bias1, int relu1, const int8_t* w2, int ldw2, int N2,
+                                   const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2,
+                                   int symmetric, int qmin, int qmax, int is_signed, float eps, int code_offset,
+                                   float* out, lq_stream stream);
 
 /* Dynamic per-row quantization in one pass: for every row of x [rows, cols],
  * min / max of the row (PerChannelMinMaxObserver with ch_axis = 0,

@@ -1101,48 +1101,64 @@ int minmax_launch(const float* x, size_t outer, size_t C, size_t inner, float* m
     return LQ_OK;
 }
 
-// A whole dynamic-quantized Linear on a small activation in one launch
-// (lucid/nn/quantized/dynamic/linear.py:87-99: x.min() / x.max(), calculate_qparams, quantize,
-// dequantize-free integer GEMM, bias): every block takes the tensor's min / max and qparams and
-// quantizes x into LDS itself - x is at most 65536 floats, so repeating that per block costs less
-// than a separate launch and its round trip - but only its own 16 rows, and then computes a
-// 16 x 16 block of the output: its 16 wavefronts split the k steps of v_mfma_i32_16x16x64_i8 (activation fragments from the LDS codes,
-// weight rows from global memory), meet through LDS atomics, and one lane per output applies
-// float(acc - zp * wsum[n]) * (s * w_scale[n]) + bias[n] (and the optional ReLU) in the order of
-// the GEMM's epilogue.  Same bits as lq_quantize_tensor_dynamic_i8 followed by lq_qlinear_i8.
-__global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
-    const float* __restrict__ x, int M, int K, const int8_t* __restrict__ w, int N, const float* __restrict__ w_scale,
-    const int32_t* __restrict__ wsum, const float* __restrict__ bias, int relu, int symmetric, int qmin, int qmax,
-    int is_signed, float eps, float half_range, int off, float* __restrict__ out) {
-    extern __shared__ __attribute__((aligned(16))) int8_t dl_smem[];
-    typedef int dl_v4i __attribute__((ext_vector_type(4)));
+// What the kernels of small dynamic layers share: every block takes the min / max and qparams of all of x (at most 65536
+// floats: repeating that per block costs less than a separate launch and its round trip), quantizes its own 16 rows
+// m0 .. m0+15 into LDS and multiplies them with the 16 weight rows n0 .. n0+15: the 16 wavefronts split the k steps of
+// v_mfma_i32_16x16x64_i8 (activation fragments from the LDS codes, weight rows from global memory) and meet through LDS
+// atomics in `red` [4][64] (red[q * 64 + lane]: activation row m0 + 4 (lane / 16) + q, weight row n0 + lane % 16), which
+// is complete when the function returns.  `ld` bytes separate rows of weight codes and of the codes in LDS: K where that is a
+// multiple of 16, otherwise a multiple of 16 beyond it with zeros in the weight past K (RAGGED).  Quads of x then straddle
+// rows, and every code is placed by itself; what LDS holds past K is multiplied by those zeros.
+struct SmallTile {
+    float s;        // the activation's scale
+    int zp;         // and zero point, as stored
+    float c_ws;     // output lanes (tid < 256): scale, code sum and bias of column n0 + tid % 16
+    int c_wsum;
+    float c_bias;
+    // float(acc - zp * wsum[n]) * (s * w_scale[n]) + bias[n] and the optional ReLU, in the order of the GEMM's epilogue
+    __device__ __forceinline__ float output(int acc, bool corrected, int relu) const {
+        const int corr = (corrected && zp != 0) ? zp * c_wsum : 0;
+        const float f = float(acc - corr);
+        const float sc = s * c_ws;
+        float y = f * sc;
+        y = y + c_bias;
+        const float floor = relu ? 0.0f : -__builtin_inff();
+        return (y < floor) ? floor : y;
+    }
+};
+typedef int dl_v4i __attribute__((ext_vector_type(4)));
+
+template <bool RAGGED>
+__device__ __forceinline__ SmallTile small_tile(const float* __restrict__ x, int M, int K, int ld, int8_t* codes, int* red,
+                                                const int8_t* __restrict__ w, int N, const float* __restrict__ w_scale,
+                                                const int32_t* __restrict__ wsum, const float* __restrict__ bias, int m0,
+                                                int n0, int symmetric, int qmin, int qmax, int is_signed, float eps,
+                                                float half_range, int off) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int8_t* const codes = dl_smem;                                     // [16][K]: the block's rows
-    int* const red = reinterpret_cast<int*>(dl_smem + size_t(16) * K);  // [4][64]
     constexpr int kKeep = 16;
-    const int quads = (M * K) >> 2;
+    const int n = M * K, quads = n >> 2;
     const float4* x4 = reinterpret_cast<const float4*>(x);
     // What does not depend on x is requested first, so that it arrives under the quantization: the
     // wavefront's first weight fragment and the output lane's column parameters.
-    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
     const int ln = lane & 15, lg = lane >> 4;
     // (requested with lane = 4 * row + chunk, so that four neighbouring lanes read 64 contiguous bytes,
     // and handed to the lane that multiplies it - row lane % 16, chunk lane / 16 - by dl_place)
     const int rq = lane >> 2, cq = lane & 3;
-    const int8_t* wrow = w + size_t(n0 + rq < N ? n0 + rq : N - 1) * size_t(K);
+    const int8_t* wrow = w + size_t(n0 + rq < N ? n0 + rq : N - 1) * size_t(ld);
     auto dl_place = [&](dl_v4i f) {
         const int from = (4 * ln + lg) * 4;
         return dl_v4i{__builtin_amdgcn_ds_bpermute(from, f[0]), __builtin_amdgcn_ds_bpermute(from, f[1]),
                       __builtin_amdgcn_ds_bpermute(from, f[2]), __builtin_amdgcn_ds_bpermute(from, f[3])};
     };
-    const int ksteps = (K + 63) >> 6;
-    const bool first_in_k = wave < ksteps && wave * 64 + cq * 16 < K;
+    const int ksteps = (ld + 63) >> 6;
+    const bool first_in_k = wave < ksteps && wave * 64 + cq * 16 < ld;
     const dl_v4i wf_first = first_in_k ? *reinterpret_cast<const dl_v4i*>(wrow + wave * 64 + cq * 16) : dl_v4i{0, 0, 0, 0};
+    SmallTile t;
     const int out_n = n0 + (tid & 15);
     const bool out_lane = tid < 256 && out_n < N;
-    const float c_ws = (out_lane && w_scale) ? w_scale[out_n] : 1.0f;
-    const int c_wsum = (out_lane && wsum) ? wsum[out_n] : 0;
-    const float c_bias = (out_lane && bias) ? bias[out_n] : -0.0f;
+    t.c_ws = (out_lane && w_scale) ? w_scale[out_n] : 1.0f;
+    t.c_wsum = (out_lane && wsum) ? wsum[out_n] : 0;
+    t.c_bias = (out_lane && bias) ? bias[out_n] : -0.0f;
     MinMax m{__builtin_inff(), -__builtin_inff(), 0};
     float4 v[kKeep];
 #pragma unroll
@@ -1150,37 +1166,65 @@ __global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
         const int i = u * 1024 + tid;
         if (i < quads) v[u] = x4[i];
     }
+    const bool in_tail = RAGGED && tid < (n & 3);  // the elements behind the last quad
+    float v_tail = 0.f;
+    if (in_tail) v_tail = x[4 * quads + tid];
     if (tid < 256) red[tid] = 0;
-    // the block's rows m0 .. m0+15 are a contiguous range of quads; rows past M (the last block's padding)
+    // the block's rows m0 .. m0+15 are a contiguous range of elements; rows past M (the last block's padding)
     // feed accumulator rows that are never stored
-    const int q_lo = (m0 * K) >> 2;
-    const int q_hi = ((m0 + 16 < M ? m0 + 16 : M) * K) >> 2;
-    for (int i = q_hi - q_lo + tid; i < 4 * K; i += 1024) reinterpret_cast<unsigned*>(codes)[i] = 0u;
+    const int rows = m0 + 16 < M ? 16 : M - m0;
+    const int q_lo = (m0 * K) >> 2, q_hi = ((m0 + rows) * K) >> 2;
+    for (int i = ((rows * ld) >> 2) + tid; i < 4 * ld; i += 1024) reinterpret_cast<unsigned*>(codes)[i] = 0u;
 #pragma unroll
     for (int u = 0; u < kKeep; ++u)
-        if (u * 1024 + tid < quads) mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
+        if (u * 1024 + tid < quads) mm_update(m, v[u]);
+    if (in_tail) mm_update(m, v_tail);
     m = mm_block_reduce(m);
     // (every thread derives the qparams: cheaper than one thread, a barrier and a read)
     const float qnan = __builtin_nanf("");
     float s, z;
     qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
+    t.s = s, t.zp = int(z) + off;
     const float r = 1.0f / s;
     const QuantizeOp<int8_t> op{x4, reinterpret_cast<Code8x4*>(codes), float(double(qmin)), float(double(qmax)), off};
+    if constexpr (!RAGGED) {
 #pragma unroll
-    for (int u = 0; u < kKeep; ++u) {
-        const int i = u * 1024 + tid;
-        if (i >= q_lo && i < q_hi) op.q[i - q_lo] = op.pack(v[u], s, z, r);
+        for (int u = 0; u < kKeep; ++u) {
+            const int i = u * 1024 + tid;
+            if (i >= q_lo && i < q_hi) op.q[i - q_lo] = op.pack(v[u], s, z, r);
+        }
+    } else {
+        // (element e of the block's range is in row floor((e + 0.5) / K): e < 16 K <= 97 280, so the quotient's rounding, at
+        // most 16 * 2^-22, stays below its distance from an integer, at least 0.5 / 6080)
+        const float per_row = 1.0f / float(K);
+        const int count = rows * K;
+        auto put = [&](int e, int8_t code) {
+            if (e >= 0 && e < count) {
+                const int row = int((float(e) + 0.5f) * per_row);
+                codes[row * ld + (e - row * K)] = code;
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < kKeep; ++u) {
+            const int i = u * 1024 + tid;
+            if (i >= q_lo && i <= q_hi && i < quads) {
+                const Code8x4 c = op.pack(v[u], s, z, r);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) put(4 * i + j - m0 * K, c.v[j]);
+            }
+        }
+        if (in_tail) put(4 * quads + tid - m0 * K, op.pack(splat(v_tail), s, z, r).v[0]);
     }
     lds_barrier();  // (the weights are still on their way)
 
     dl_v4i acc = dl_v4i{0, 0, 0, 0};
     for (int ks = wave; ks < ksteps; ks += 16) {
         const int k = ks * 64 + lg * 16;
-        const bool in_k = k < K;  // K % 16 == 0: a 16-byte chunk is inside or outside as a whole
+        const bool in_k = k < ld;  // ld % 16 == 0: a 16-byte chunk is inside or outside as a whole
         const int kq = ks * 64 + cq * 16;
         const dl_v4i wf = dl_place(ks == wave ? wf_first
-                                              : (kq < K ? *reinterpret_cast<const dl_v4i*>(wrow + kq) : dl_v4i{0, 0, 0, 0}));
-        const dl_v4i af = in_k ? *reinterpret_cast<const dl_v4i*>(codes + size_t(ln) * K + k) : dl_v4i{0, 0, 0, 0};
+                                              : (kq < ld ? *reinterpret_cast<const dl_v4i*>(wrow + kq) : dl_v4i{0, 0, 0, 0}));
+        const dl_v4i af = in_k ? *reinterpret_cast<const dl_v4i*>(codes + size_t(ln) * ld + k) : dl_v4i{0, 0, 0, 0};
         acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, wf, acc, 0, 0, 0);
     }
     if (wave < ksteps) {
@@ -1189,22 +1233,28 @@ __global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
             __hip_atomic_fetch_add(&red[q * 64 + lane], acc[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     __syncthreads();
-    // red[q * 64 + lane]: activation row m0 + 4 (lane / 16) + q, weight row n0 + lane % 16
+    return t;
+}
+
+// A whole dynamic-quantized Linear on a small activation in one launch
+// (lucid/nn/quantized/dynamic/linear.py:87-99: x.min() / x.max(), calculate_qparams, quantize,
+// dequantize-free integer GEMM, bias): a block per 16 x 16 outputs.  Same bits as lq_quantize_tensor_dynamic_i8
+// followed by lq_qlinear_i8.
+template <bool RAGGED>
+__global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
+    const float* __restrict__ x, int M, int K, const int8_t* __restrict__ w, int ld, int N, const float* __restrict__ w_scale,
+    const int32_t* __restrict__ wsum, const float* __restrict__ bias, int relu, int symmetric, int qmin, int qmax,
+    int is_signed, float eps, float half_range, int off, float* __restrict__ out) {
+    extern __shared__ __attribute__((aligned(16))) int8_t dl_smem[];
+    int8_t* const codes = dl_smem;                                      // [16][ld]: the block's rows
+    int* const red = reinterpret_cast<int*>(dl_smem + size_t(16) * ld);  // [4][64]
+    const int tid = threadIdx.x, n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
+    const SmallTile t = small_tile<RAGGED>(x, M, K, ld, codes, red, w, N, w_scale, wsum, bias, m0, n0, symmetric, qmin, qmax,
+                                           is_signed, eps, half_range, off);
     if (tid < 256) {
         const int q = tid >> 6, l = tid & 63;
         const int mm = m0 + 4 * (l >> 4) + q, nn = n0 + (l & 15);
-        if (mm < M && nn < N) {
-            // GEMM epilogue, float32 output form: the zero point enters as an integer, the steps stay separate
-            const int zp = int(z) + off;
-            const int corr = (wsum != nullptr && zp != 0) ? zp * c_wsum : 0;
-            const float f = float(red[tid] - corr);
-            const float sc = s * c_ws;
-            float y = f * sc;
-            y = y + c_bias;
-            const float floor = relu ? 0.0f : -__builtin_inff();
-            y = (y < floor) ? floor : y;
-            out[size_t(mm) * N + nn] = y;
-        }
+        if (mm < M && nn < N) out[size_t(mm) * N + nn] = t.output(red[tid], wsum != nullptr, relu);
     }
 }
 
@@ -1213,110 +1263,52 @@ __global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
 // launches cost three round trips).  Layer 1 runs exactly as dynamic_linear_small_kernel runs it -
 // a block per 16 x 16 tile of the hidden activation, so the 50 k inputs are quantized by 64 CUs
 // at once - with each block's tile (ReLU applied) and its min / max written through to device
-// scope; the block that arrives last (one counter, at most 64 arrivals) then owns the whole
-// hidden activation - 64 KB, one round trip - and does for layer 2 what the separate operators
+// scope; the block that arrives last (one counter, at most kMlpBlocks arrivals) then owns the whole
+// hidden activation - 64 KB there, one round trip - and does for layer 2 what the separate operators
 // do: the tensor's min / max (from the tiles'), calculate_qparams, the codes, the integer GEMM
 // (one wavefront per 16 x 16 output tile), float(acc - zp * wsum[n]) * (s * w_scale[n]) + bias[n],
 // ReLU.  Same bits as two lq_dynamic_linear_small_f32 calls (the ReLU between them folded into
 // the first).  15.7 us for that MLP; with ONE block doing both layers it was 21 us (one CU's
-// vector units quantized all 50 k inputs).  `hid`: [M][N1] float32, then 64 minima and 64 maxima;
-// `counter`: zero between launches (the last block resets it).
+// vector units quantized all 50 k inputs).  `hid`: [M][ld2] float32, then kMlpBlocks minima and as many maxima;
+// `counter`: zero between launches (the last block resets it).  Columns of `hid` from N1 to ld2 hold anything: their codes
+// meet the zeros of layer 2's padded weight rows.  KS2: steps of 64 k that ld2 takes at most.
+constexpr int kMlpBlocks = 128, kMlpMaxHidden = 511;
+template <bool RAGGED, int KS2>
 __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
-    const float* __restrict__ x, int M, int K1, const int8_t* __restrict__ w1, int N1, const float* __restrict__ ws1,
-    const int32_t* __restrict__ wsum1, const float* __restrict__ b1, int relu1, const int8_t* __restrict__ w2, int N2,
+    const float* __restrict__ x, int M, int K1, const int8_t* __restrict__ w1, int ld1, int N1, const float* __restrict__ ws1,
+    const int32_t* __restrict__ wsum1, const float* __restrict__ b1, int relu1, const int8_t* __restrict__ w2, int ld2, int N2,
     const float* __restrict__ ws2, const int32_t* __restrict__ wsum2, const float* __restrict__ b2, int relu2,
     int symmetric, int qmin, int qmax, int is_signed, float eps, float half_range, int off, float* __restrict__ out,
     float* hid, int* counter) {
     extern __shared__ __attribute__((aligned(16))) int8_t mb_smem[];
     __shared__ int s_arrived;
-    typedef int mb_v4i __attribute__((ext_vector_type(4)));
     typedef unsigned mb_v4u __attribute__((ext_vector_type(4)));
     constexpr unsigned kScopeDevice = 16;  // "sc1" cache-policy bit of buffer accesses
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int8_t* const codes = mb_smem;                                      // [16][K1]: the block's rows
-    int* const red = reinterpret_cast<int*>(mb_smem + size_t(16) * K1);  // [4][64]
-    int8_t* const codes2 = mb_smem + size_t(16) * K1 + 1024;             // [64][N1]: the last block's
-    constexpr int kKeep = 16;
+    int8_t* const codes = mb_smem;                                       // [16][ld1]: the block's rows
+    int* const red = reinterpret_cast<int*>(mb_smem + size_t(16) * ld1);  // [4][64]
+    int8_t* const codes2 = mb_smem + size_t(16) * ld1 + 1024;             // [64][ld2]: the last block's
     const float qnan = __builtin_nanf("");
-    const int quads = (M * K1) >> 2;
-    const float4* x4 = reinterpret_cast<const float4*>(x);
     const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
     const int nblocks = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
     const int ln = lane & 15, lg = lane >> 4;
     const int rq = lane >> 2, cq = lane & 3;
-    const int8_t* wrow = w1 + size_t(n0 + rq < N1 ? n0 + rq : N1 - 1) * size_t(K1);
-    auto place = [&](mb_v4i f) {
+    auto place = [&](dl_v4i f) {
         const int from = (4 * ln + lg) * 4;
-        return mb_v4i{__builtin_amdgcn_ds_bpermute(from, f[0]), __builtin_amdgcn_ds_bpermute(from, f[1]),
+        return dl_v4i{__builtin_amdgcn_ds_bpermute(from, f[0]), __builtin_amdgcn_ds_bpermute(from, f[1]),
                       __builtin_amdgcn_ds_bpermute(from, f[2]), __builtin_amdgcn_ds_bpermute(from, f[3])};
     };
-    const size_t hid_bytes = size_t(M) * N1 * 4;
-    const __amdgpu_buffer_rsrc_t hbuf = __builtin_amdgcn_make_buffer_rsrc(hid, 0, int(hid_bytes) + 512, 0x00020000);
-    const int ksteps = (K1 + 63) >> 6;
-    const bool first_in_k = wave < ksteps && wave * 64 + cq * 16 < K1;
-    const mb_v4i wf_first = first_in_k ? *reinterpret_cast<const mb_v4i*>(wrow + wave * 64 + cq * 16) : mb_v4i{0, 0, 0, 0};
-    const int out_n = n0 + (tid & 15);
-    const bool out_lane = tid < 256 && out_n < N1;
-    const float c_ws = (out_lane && ws1) ? ws1[out_n] : 1.0f;
-    const int c_wsum = (out_lane && wsum1) ? wsum1[out_n] : 0;
-    const float c_bias = (out_lane && b1) ? b1[out_n] : -0.0f;
-    MinMax m{__builtin_inff(), -__builtin_inff(), 0};
-    float4 v[kKeep];
-#pragma unroll
-    for (int u = 0; u < kKeep; ++u) {
-        const int i = u * 1024 + tid;
-        if (i < quads) v[u] = x4[i];
-    }
-    if (tid < 256) red[tid] = 0;
-    const int q_lo = (m0 * K1) >> 2;
-    const int q_hi = ((m0 + 16 < M ? m0 + 16 : M) * K1) >> 2;
-    for (int i = q_hi - q_lo + tid; i < 4 * K1; i += 1024) reinterpret_cast<unsigned*>(codes)[i] = 0u;
-#pragma unroll
-    for (int u = 0; u < kKeep; ++u)
-        if (u * 1024 + tid < quads) mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
-    m = mm_block_reduce(m);
-    float s, z;
-    qparams_of(m.nan ? qnan : m.lo, m.nan ? qnan : m.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s, &z);
-    const float r = 1.0f / s;
-    {
-        const QuantizeOp<int8_t> op{x4, reinterpret_cast<Code8x4*>(codes), float(double(qmin)), float(double(qmax)), off};
-#pragma unroll
-        for (int u = 0; u < kKeep; ++u) {
-            const int i = u * 1024 + tid;
-            if (i >= q_lo && i < q_hi) op.q[i - q_lo] = op.pack(v[u], s, z, r);
-        }
-    }
-    lds_barrier();  // (the weights are still on their way)
-    mb_v4i acc = mb_v4i{0, 0, 0, 0};
-    for (int ks = wave; ks < ksteps; ks += 16) {
-        const int k = ks * 64 + lg * 16;
-        const bool in_k = k < K1;
-        const int kq = ks * 64 + cq * 16;
-        const mb_v4i wf = place(ks == wave ? wf_first
-                                           : (kq < K1 ? *reinterpret_cast<const mb_v4i*>(wrow + kq) : mb_v4i{0, 0, 0, 0}));
-        const mb_v4i af = in_k ? *reinterpret_cast<const mb_v4i*>(codes + size_t(ln) * K1 + k) : mb_v4i{0, 0, 0, 0};
-        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, wf, acc, 0, 0, 0);
-    }
-    if (wave < ksteps) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-            __hip_atomic_fetch_add(&red[q * 64 + lane], acc[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    __syncthreads();
+    const size_t hid_bytes = size_t(M) * ld2 * 4;
+    const __amdgpu_buffer_rsrc_t hbuf = __builtin_amdgcn_make_buffer_rsrc(hid, 0, int(hid_bytes) + 8 * kMlpBlocks, 0x00020000);
+    const SmallTile t = small_tile<RAGGED>(x, M, K1, ld1, codes, red, w1, N1, ws1, wsum1, b1, m0, n0, symmetric, qmin, qmax,
+                                           is_signed, eps, half_range, off);
     MinMax hm{__builtin_inff(), -__builtin_inff(), 0};
     if (tid < 256) {
         const int q = tid >> 6, l = tid & 63;
         const int mm = m0 + 4 * (l >> 4) + q, nn = n0 + (l & 15);
         if (mm < M && nn < N1) {
-            const int zp = int(z) + off;
-            const int corr = (wsum1 != nullptr && zp != 0) ? zp * c_wsum : 0;
-            const float f = float(red[tid] - corr);
-            const float sc = s * c_ws;
-            float y = f * sc;
-            y = y + c_bias;
-            const float floor = relu1 ? 0.0f : -__builtin_inff();
-            y = (y < floor) ? floor : y;
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), hbuf, unsigned(mm * N1 + nn) * 4, 0, kScopeDevice);
+            const float y = t.output(red[tid], wsum1 != nullptr, relu1);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), hbuf, unsigned(mm * ld2 + nn) * 4, 0, kScopeDevice);
             mm_update(hm, y);
         }
     }
@@ -1324,7 +1316,8 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     if (tid == 0) {
         const float lo = hm.nan ? qnan : hm.lo, hi = hm.nan ? qnan : hm.hi;
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(lo), hbuf, unsigned(hid_bytes) + bid * 4, 0, kScopeDevice);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(hi), hbuf, unsigned(hid_bytes) + 256 + bid * 4, 0, kScopeDevice);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(hi), hbuf, unsigned(hid_bytes) + 4 * kMlpBlocks + bid * 4, 0,
+                                              kScopeDevice);
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this thread's part of the tile has been written through
     __syncthreads();
@@ -1338,71 +1331,62 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     if (tid < nblocks) {
         slot_lo = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(hbuf, unsigned(hid_bytes) + tid * 4, 0, kScopeDevice));
         slot_hi = __uint_as_float(
-            __builtin_amdgcn_raw_buffer_load_b32(hbuf, unsigned(hid_bytes) + 256 + tid * 4, 0, kScopeDevice));
+            __builtin_amdgcn_raw_buffer_load_b32(hbuf, unsigned(hid_bytes) + 4 * kMlpBlocks + tid * 4, 0, kScopeDevice));
     }
-    const int quads2 = (M * N1) >> 2;  // at most 4096: four per thread
-    mb_v4u h[4];
+    const int quads2 = (M * ld2) >> 2;  // at most KS2 per thread
+    mb_v4u h[KS2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < KS2; ++u) {
         const int i = u * 1024 + tid;
         h[u] = __builtin_amdgcn_raw_buffer_load_b128(hbuf, unsigned(i < quads2 ? i : 0) * 16, 0, kScopeDevice);
     }
-    constexpr int kSteps2 = 4;
     const int rb2 = wave & 3, cb2 = wave >> 2;
     const int n2 = cb2 * 16 + ln, nc2 = n2 < N2 ? n2 : N2 - 1;
-    mb_v4i w2f[kSteps2];
+    dl_v4i w2f[KS2];
     {
         const int r2 = cb2 * 16 + rq;
-        const int8_t* wrow2 = w2 + size_t(r2 < N2 ? r2 : N2 - 1) * size_t(N1) + cq * 16;
+        const int8_t* wrow2 = w2 + size_t(r2 < N2 ? r2 : N2 - 1) * size_t(ld2) + cq * 16;
 #pragma unroll
-        for (int ks = 0; ks < kSteps2; ++ks)
-            w2f[ks] = ks * 64 + cq * 16 < N1 ? *reinterpret_cast<const mb_v4i*>(wrow2 + ks * 64) : mb_v4i{0, 0, 0, 0};
+        for (int ks = 0; ks < KS2; ++ks)
+            w2f[ks] = ks * 64 + cq * 16 < ld2 ? *reinterpret_cast<const dl_v4i*>(wrow2 + ks * 64) : dl_v4i{0, 0, 0, 0};
     }
-    const float c_ws2 = ws2 ? ws2[nc2] : 1.0f;
-    const int c_wsum2 = wsum2 ? wsum2[nc2] : 0;
-    const float c_bias2 = b2 ? b2[nc2] : -0.0f;
-    for (int i = quads2 + tid; i < 16 * N1; i += 1024) reinterpret_cast<unsigned*>(codes2)[i] = 0u;
+    SmallTile t2;
+    t2.c_ws = ws2 ? ws2[nc2] : 1.0f;
+    t2.c_wsum = wsum2 ? wsum2[nc2] : 0;
+    t2.c_bias = b2 ? b2[nc2] : -0.0f;
+    for (int i = quads2 + tid; i < 16 * ld2; i += 1024) reinterpret_cast<unsigned*>(codes2)[i] = 0u;
     MinMax tm{slot_lo, slot_hi, int((slot_lo != slot_lo) | (slot_hi != slot_hi))};
     if (tm.nan) tm.lo = __builtin_inff(), tm.hi = -__builtin_inff();
     tm = mm_block_reduce(tm);
     if (tid == 0) *counter = 0;  // ready for the next launch
     float s2, z2;
     qparams_of(tm.nan ? qnan : tm.lo, tm.nan ? qnan : tm.hi, symmetric, qmin, qmax, is_signed, eps, half_range, &s2, &z2);
+    t2.s = s2, t2.zp = int(z2) + off;
     {
         const float r2 = 1.0f / s2;
         const QuantizeOp<int8_t> op{nullptr, reinterpret_cast<Code8x4*>(codes2), float(double(qmin)), float(double(qmax)), off};
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < KS2; ++u) {
             const int i = u * 1024 + tid;
             if (i < quads2) op.q[i] = op.pack(__builtin_bit_cast(float4, h[u]), s2, z2, r2);
         }
     }
     __syncthreads();
     if (cb2 * 16 < N2 && rb2 * 16 < M) {
-        const int zp = int(z2) + off;
-        mb_v4i acc2 = mb_v4i{0, 0, 0, 0};
+        dl_v4i acc2 = dl_v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int ks = 0; ks < kSteps2; ++ks) {
+        for (int ks = 0; ks < KS2; ++ks) {
             const int k = ks * 64 + lg * 16;
-            if (ks * 64 < N1) {  // uniform
-                const mb_v4i af = k < N1 ? *reinterpret_cast<const mb_v4i*>(codes2 + size_t(16 * rb2 + ln) * N1 + k)
-                                         : mb_v4i{0, 0, 0, 0};
+            if (ks * 64 < ld2) {  // uniform
+                const dl_v4i af = k < ld2 ? *reinterpret_cast<const dl_v4i*>(codes2 + size_t(16 * rb2 + ln) * ld2 + k)
+                                          : dl_v4i{0, 0, 0, 0};
                 acc2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, place(w2f[ks]), acc2, 0, 0, 0);
             }
         }
-        const int corr = (wsum2 != nullptr && zp != 0) ? zp * c_wsum2 : 0;
-        const float sc = s2 * c_ws2;
-        const float floor = relu2 ? 0.0f : -__builtin_inff();
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int mm = 16 * rb2 + 4 * lg + q;
-            if (mm < M && n2 < N2) {
-                const float f = float(acc2[q] - corr);
-                float y = f * sc;
-                y = y + c_bias2;
-                y = (y < floor) ? floor : y;
-                out[size_t(mm) * N2 + n2] = y;
-            }
+            if (mm < M && n2 < N2) out[size_t(mm) * N2 + n2] = t2.output(acc2[q], wsum2 != nullptr, relu2);
         }
     }
 }
@@ -1572,60 +1556,92 @@ int lq_dynamic_mlp2_small_f32(const float* x, int M, int K1, const int8_t* w1, i
                               int qmin, int qmax, int is_signed, float eps, int code_offset, float* out,
                               lq_stream stream) {
     if (M == 0 || N2 == 0) return LQ_OK;
+    LQ_REQUIRE(K1 >= 16 && K1 % 16 == 0 && long(M) * K1 <= 65536 && N1 >= 16 && N1 % 16 == 0 && N1 <= 256,
+               LQ_ERR_NOT_IMPLEMENTED,
+               "dynamic_mlp2_small: takes K1 %% 16 == 0 and a hidden width that is a multiple of 16 up to 256 (got M = %d, "
+               "K1 = %d, N1 = %d); use lq_dynamic_mlp2_small_rows_f32 or two lq_dynamic_linear_f32 calls", M, K1, N1);
+    return lq_dynamic_mlp2_small_rows_f32(x, M, K1, w1, K1, N1, w1_scale, w1sum, bias1, relu1, w2, N1, N2, w2_scale, w2sum,
+                                          bias2, relu2, symmetric, qmin, qmax, is_signed, eps, code_offset, out, stream);
+}
+
+int lq_dynamic_mlp2_small_rows_f32(const float* x, int M, int K1, const int8_t* w1, int ldw1, int N1, const float* w1_scale,
+                                   const int32_t* w1sum, const float* bias1, int relu1, const int8_t* w2, int ldw2, int N2,
+                                   const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2,
+                                   int symmetric, int qmin, int qmax, int is_signed, float eps, int code_offset,
+                                   float* out, lq_stream stream) {
+    if (M == 0 || N2 == 0) return LQ_OK;
     LQ_REQUIRE(x && w1 && w2 && out, LQ_ERR_VALUE, "dynamic_mlp2_small: NULL pointer");
     LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
                "dynamic_mlp2_small: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
-    // a block holds 16 rows of x's codes; the last one also the hidden activation's codes (64 N1 bytes)
-    LQ_REQUIRE(M > 0 && M <= 64 && K1 >= 16 && K1 % 16 == 0 && K1 <= 1024 && long(M) * K1 <= 65536 && N1 >= 16 &&
-                   N1 % 16 == 0 && N1 <= 256 && N2 > 0 && N2 <= 64 && aligned16(x) && aligned16(w1) && aligned16(w2),
+    // a block holds 16 rows of x's codes; the last one also the hidden activation's codes (64 ldw2 bytes)
+    LQ_REQUIRE(M > 0 && M <= 64 && K1 > 0 && ldw1 >= K1 && ldw1 % 16 == 0 && ldw1 <= 1024 && N1 > 0 && N1 <= kMlpMaxHidden &&
+                   ldw2 >= N1 && ldw2 % 16 == 0 && ldw2 <= 512 && N2 > 0 && N2 <= 64 && aligned16(x) && aligned16(w1) &&
+                   aligned16(w2),
                LQ_ERR_NOT_IMPLEMENTED,
-               "dynamic_mlp2_small: takes up to 64 rows, K1 %% 16 == 0 up to 1024, a hidden width that is a multiple of "
-               "16 up to 256 and up to 64 outputs (got M = %d, K1 = %d, N1 = %d, N2 = %d); use two "
-               "lq_dynamic_linear_small_f32 calls", M, K1, N1, N2);
+               "dynamic_mlp2_small: takes up to 64 rows, weight rows of a multiple of 16 bytes (K1 up to 1024, a hidden width "
+               "up to %d), up to 64 outputs and 16-byte aligned operands (got M = %d, K1 = %d in rows of %d, N1 = %d in rows "
+               "of %d, N2 = %d); use two lq_dynamic_linear_f32 calls", kMlpMaxHidden, M, K1, ldw1, N1, ldw2, N2);
     const float half_range = float((double(qmax) - double(qmin)) / 2.0);
     // the hidden activation and the tiles' ranges pass through the stream's split-K scratch
     SkScratch sk;
     const auto lock = scratch_lock(as_stream(stream));
-    const size_t hid_bytes = size_t(M) * N1 * 4;
-    if (int rc = sk_scratch(1, hid_bytes + 512, as_stream(stream), &sk)) return rc;
-    const size_t lds = size_t(16) * K1 + 1024 + size_t(64) * N1;
-    static DeviceOnce attr_once;
-    if (int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(dynamic_mlp2_blocks_kernel), 64 * 1024))
-        return rc;
-    hipLaunchKernelGGL(dynamic_mlp2_blocks_kernel, dim3(unsigned(N1 / 16), unsigned((M + 15) / 16)), dim3(1024), lds,
-                       as_stream(stream), x, M, K1, w1, N1, w1_scale, w1sum, bias1, relu1, w2, N2, w2_scale, w2sum, bias2,
-                       relu2, symmetric, qmin, qmax, is_signed, eps, half_range, code_offset, out,
-                       reinterpret_cast<float*>(sk.slabs), sk.counters);
-    LQ_CHECK_LAUNCH("dynamic_mlp2_small");
-    return LQ_OK;
+    const size_t hid_bytes = size_t(M) * ldw2 * 4;
+    if (int rc = sk_scratch(1, hid_bytes + 8 * kMlpBlocks, as_stream(stream), &sk)) return rc;
+    const size_t lds = size_t(16) * ldw1 + 1024 + size_t(64) * ldw2;
+    static DeviceOnce attr_once[4];
+    auto launch = [&](auto kernel, int form) -> int {
+        if (int rc = allow_dynamic_lds(attr_once[form], reinterpret_cast<const void*>(kernel), 64 * 1024)) return rc;
+        hipLaunchKernelGGL(kernel, dim3(unsigned((N1 + 15) / 16), unsigned((M + 15) / 16)), dim3(1024), lds,
+                           as_stream(stream), x, M, K1, w1, ldw1, N1, w1_scale, w1sum, bias1, relu1, w2, ldw2, N2, w2_scale,
+                           w2sum, bias2, relu2, symmetric, qmin, qmax, is_signed, eps, half_range, code_offset, out,
+                           reinterpret_cast<float*>(sk.slabs), sk.counters);
+        LQ_CHECK_LAUNCH("dynamic_mlp2_small");
+        return LQ_OK;
+    };
+    const bool ragged = ldw1 != K1, wide = ldw2 > 256;
+    return ragged ? (wide ? launch(dynamic_mlp2_blocks_kernel<true, 8>, 0) : launch(dynamic_mlp2_blocks_kernel<true, 4>, 1))
+                  : (wide ? launch(dynamic_mlp2_blocks_kernel<false, 8>, 2) : launch(dynamic_mlp2_blocks_kernel<false, 4>, 3));
 }
 
 int lq_dynamic_linear_small_f32(const float* x, int M, int K, const int8_t* w, int N, const float* w_scale,
                                 const int32_t* wsum, const float* bias, int relu, int symmetric, int qmin, int qmax,
                                 int is_signed, float eps, int code_offset, float* out, lq_stream stream) {
     if (M == 0 || N == 0) return LQ_OK;
+    LQ_REQUIRE(K >= 16 && K % 16 == 0 && K <= 6080, LQ_ERR_NOT_IMPLEMENTED,
+               "dynamic_linear_small: takes K %% 16 == 0 and K <= 6080 (got K = %d); use lq_dynamic_linear_small_rows_f32 or "
+               "lq_quantize_tensor_dynamic_i8 + lq_qlinear_i8", K);
+    return lq_dynamic_linear_small_rows_f32(x, M, K, w, K, N, w_scale, wsum, bias, relu, symmetric, qmin, qmax, is_signed, eps,
+                                            code_offset, out, stream);
+}
+
+int lq_dynamic_linear_small_rows_f32(const float* x, int M, int K, const int8_t* w, int ldw, int N, const float* w_scale,
+                                     const int32_t* wsum, const float* bias, int relu, int symmetric, int qmin, int qmax,
+                                     int is_signed, float eps, int code_offset, float* out, lq_stream stream) {
+    if (M == 0 || N == 0) return LQ_OK;
     LQ_REQUIRE(x && w && out, LQ_ERR_VALUE, "dynamic_linear_small: NULL pointer");
     LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
                "dynamic_linear_small: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
-    // 16 rows of codes (16 K bytes) + 1 KiB of reduction scratch have to fit the 96 KiB of dynamic
-    // LDS the kernel is allowed: K <= 6080
-    LQ_REQUIRE(M > 0 && M <= 64 && K >= 16 && K % 16 == 0 && long(M) * K <= 65536 && K <= 6080 && N > 0 &&
+    // 16 rows of codes (16 ldw bytes) + 1 KiB of reduction scratch have to fit the 96 KiB of dynamic
+    // LDS the kernel is allowed: ldw <= 6080
+    LQ_REQUIRE(M > 0 && M <= 64 && K > 0 && ldw >= K && ldw % 16 == 0 && long(M) * K <= 65536 && ldw <= 6080 && N > 0 &&
                    aligned16(x) && aligned16(w),
                LQ_ERR_NOT_IMPLEMENTED,
-               "dynamic_linear_small: takes up to 64 rows, K %% 16 == 0 and K <= 6080, at most 65536 activations and "
-               "16-byte aligned operands (got M = %d, K = %d); use lq_quantize_tensor_dynamic_i8 + lq_qlinear_i8", M, K);
+               "dynamic_linear_small: takes up to 64 rows, weight rows of a multiple of 16 bytes up to 6080, at most 65536 "
+               "activations and 16-byte aligned operands (got M = %d, K = %d in rows of %d); use "
+               "lq_quantize_tensor_dynamic_i8 + lq_qlinear_i8", M, K, ldw);
     const float half_range = float((double(qmax) - double(qmin)) / 2.0);
     const int tiles = (M + 15) / 16;
-    const size_t lds = size_t(16) * K + 256 * sizeof(int);
-    static DeviceOnce attr_once;
-    if (int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(dynamic_linear_small_kernel), 96 * 1024))
-        return rc;
-    hipLaunchKernelGGL(dynamic_linear_small_kernel, dim3(unsigned((N + 15) / 16), unsigned(tiles)), dim3(1024), lds,
-                       as_stream(stream), x,
-                       M, K, w, N, w_scale, wsum, bias, relu, symmetric, qmin, qmax, is_signed, eps, half_range,
-                       code_offset, out);
-    LQ_CHECK_LAUNCH("dynamic_linear_small");
-    return LQ_OK;
+    const size_t lds = size_t(16) * ldw + 256 * sizeof(int);
+    static DeviceOnce attr_once[2];
+    auto launch = [&](auto kernel, int form) -> int {
+        if (int rc = allow_dynamic_lds(attr_once[form], reinterpret_cast<const void*>(kernel), 96 * 1024)) return rc;
+        hipLaunchKernelGGL(kernel, dim3(unsigned((N + 15) / 16), unsigned(tiles)), dim3(1024), lds, as_stream(stream), x, M, K,
+                           w, ldw, N, w_scale, wsum, bias, relu, symmetric, qmin, qmax, is_signed, eps, half_range,
+                           code_offset, out);
+        LQ_CHECK_LAUNCH("dynamic_linear_small");
+        return LQ_OK;
+    };
+    return ldw != K ? launch(dynamic_linear_small_kernel<true>, 0) : launch(dynamic_linear_small_kernel<false>, 1);
 }
 
 int lq_quantize_rows_dynamic_i8(const float* x, size_t rows, size_t cols, int symmetric, int qmin, int qmax,

@@ -36,7 +36,7 @@ def _one_launch_pays(M: int, K: int, N: int) -> bool:
     up) in two.  Its blocks each take the range of all of x and quantize 16 rows: about 4 us + 0.043 us per
     1000 activations + 2.4 us per 1000 of K, one round of 256 blocks.  Measured: 64 x 784 -> 256 8.0 us,
     7 x 1024 -> 1024 7.2, 16 x 4096 -> 1024 16.5, 32 x 2048 -> 4096 (512 blocks) 22.7, 16 x 4096 -> 11008 48.5."""
-    return (1 < M <= 64 and K % 16 == 0 and 0 < K <= SMALL_LINEAR_MAX_K and M * K <= 65536
+    return (1 < M <= 64 and 0 < K <= SMALL_LINEAR_MAX_K and M * K <= 65536
             and ((M + 15) // 16) * ((N + 15) // 16) <= 256 and 43 * M * K + 2400 * K <= 6_000_000)
 
 
@@ -83,11 +83,18 @@ def _keep(*derived) -> None:
         setattr(lin, name, value)
 
 
+# What the one launch for two layers holds: the first layer's row of codes, the hidden row of the block that runs the second.
+PAIR_MAX_K, PAIR_MAX_HIDDEN = 1024, 511
+
+
 def fused_pair(first, relu_between: bool, second, x):
     """``second(relu(first(x)))`` (or without the ReLU) for two dynamic ``Linear`` layers on a small
     activation as ONE launch (``lq_dynamic_mlp2_small_f32``: the last block of layer 1 to finish
-    reduces the hidden activation's min / max and runs layer 2), or ``None`` when the shapes or
-    operands do not qualify.  Same bits as calling the modules one after the other."""
+    reduces the hidden activation's min / max and runs layer 2; ``lq_dynamic_mlp2_small_rows_f32`` where a weight's
+    rows are no whole 16 bytes or the hidden layer is wide), beyond it as two calls with the ReLU in the
+    first one's epilogue, or ``None`` when the shapes or operands do not qualify.  Same bits as calling the modules one
+    after the other.  Per forward, ReLU between: 91-32-58 of 12 rows in one launch 12.6 us (32 in three calls, which is what
+    their host side takes), 64 rows of 784-496-10 17.9 (33)."""
     if not (isinstance(first, Linear) and isinstance(second, Linear) and isinstance(x, Tensor)):
         return None
     if x.device != "hip" or x.dtype != T.float32 or x._grid is not None or x._range is not None:
@@ -95,30 +102,49 @@ def fused_pair(first, relu_between: bool, second, x):
     K1, N1, N2 = first.in_features, first.out_features, second.out_features
     if x.ndim < 1 or x.shape[-1] != K1 or second.in_features != N1:
         return None
-    M = x.numel // K1
-    if not (0 < M <= 64 and K1 % 16 == 0 and 16 <= K1 <= 1024 and M * K1 <= 65536 and N1 % 16 == 0
-            and 16 <= N1 <= 256 and 0 < N2 <= 64):
+    M = x.numel // K1 if K1 else 0
+    small = 0 < M <= 64 and K1 <= PAIR_MAX_K and 0 < N1 <= PAIR_MAX_HIDDEN and 0 < N2 <= 64
+    rows = small and (K1 % 16 != 0 or N1 % 16 != 0 or N1 > 256)
+    if rows and x.data_ptr % 16:
+        small = False
+    if not small and not relu_between:
         return None
     if first.act_qdtype is not second.act_qdtype:
         return None
     if weight_zero_points(first) is not None or weight_zero_points(second) is not None:
         return None
+    if not small:
+        h = first._one_call(x, M, 1) if M else None
+        return None if h is None else second(h)
     taken1, taken2 = _kernel_operands(first, N1, K1), _kernel_operands(second, N2, N1)
     if taken1 is None or taken2 is None:
         return None
     (w1, scale1, bias1), (w2, scale2, bias2) = taken1, taken2
     wsum1, wsum2 = first._wsum, second._wsum
-    fresh = wsum1 is None or wsum2 is None
-    if fresh:
+    fresh = ()
+    if wsum1 is None or wsum2 is None:
         wsum1, wsum2 = first._weight_sums(), second._weight_sums()
+        fresh = ((first, "_wsum", wsum1), (second, "_wsum", wsum2))
     qd = first.act_qdtype
     y = Tensor.empty((*x.shape[:-1], N2), T.float32, "hip")
-    _C.call("lq_dynamic_mlp2_small_f32", x.data_ptr, M, K1, w1.data_ptr, N1, scale1.data_ptr, wsum1.data_ptr,
-            None if bias1 is None else bias1.data_ptr, int(relu_between),
-            w2.data_ptr, N2, scale2.data_ptr, wsum2.data_ptr, None if bias2 is None else bias2.data_ptr, 0, 0,
-            qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, storage_offset(qd), y.data_ptr, None)
+    b1, b2 = None if bias1 is None else bias1.data_ptr, None if bias2 is None else bias2.data_ptr
+    grid = (0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, storage_offset(qd))
+    if rows:
+        padded = []
+        for lin, w, K in ((first, w1, K1), (second, w2, N1)):
+            rows = (w, K) if K % 16 == 0 else lin._wrows
+            if rows is None:
+                rows = lin._weight_rows()
+                fresh += ((lin, "_wrows", rows),)
+            padded.append(rows)
+        (w1, ld1), (w2, ld2) = padded
+        _C.call("lq_dynamic_mlp2_small_rows_f32", x.data_ptr, M, K1, w1.data_ptr, ld1, N1, scale1.data_ptr, wsum1.data_ptr,
+                b1, int(relu_between), w2.data_ptr, ld2, N2, scale2.data_ptr, wsum2.data_ptr, b2, 0, *grid, y.data_ptr, None)
+    else:
+        _C.call("lq_dynamic_mlp2_small_f32", x.data_ptr, M, K1, w1.data_ptr, N1, scale1.data_ptr, wsum1.data_ptr,
+                b1, int(relu_between), w2.data_ptr, N2, scale2.data_ptr, wsum2.data_ptr, b2, 0, *grid, y.data_ptr, None)
     if fresh:
-        _keep((first, "_wsum", wsum1), (second, "_wsum", wsum2))
+        _keep(*fresh)
     return y
 
 
@@ -167,6 +193,43 @@ class Linear(Module):
         _C.call("lq_d2d_rows", rows.data_ptr, ld, self._buffers["weight_int8"].data_ptr, K, K, N, None)
         return rows, ld
 
+    def _one_call(self, x: Tensor, M: int, relu: int) -> Tensor | None:
+        """min / max, qparams, codes, GEMM, bias and an optional ReLU behind one call (the same bits as the separate
+        operators), or ``None`` where that call does not take the layer."""
+        K, N = self.in_features, self.out_features
+        if (weight_zero_points(self) is not None or not _one_call_takes(M, K)
+                or (taken := _kernel_operands(self, N, K)) is None):
+            return None
+        w, scale, bias = taken
+        wsum, fresh = self._wsum, ()
+        if wsum is None:
+            wsum = self._weight_sums()
+            fresh = ((self, "_wsum", wsum),)
+        qd = self.act_qdtype
+        y = Tensor.empty((*x.shape[:-1], N), T.float32, "hip")
+        grid = (relu, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, storage_offset(qd))
+        b = None if bias is None else bias.data_ptr
+        at, ldw = x.data_ptr if M else None, K
+        if K % 16:
+            if self._wrows is not None:
+                w, ldw = self._wrows
+            else:
+                w, ldw = rows = self._weight_rows()
+                fresh += ((self, "_wrows", rows),)
+        if _one_launch_pays(M, K, N) and (ldw == K or at % 16 == 0):
+            if ldw == K:
+                _C.call("lq_dynamic_linear_small_f32", at, M, K, w.data_ptr, N, scale.data_ptr, wsum.data_ptr, b, *grid,
+                        y.data_ptr, None)
+            else:
+                _C.call("lq_dynamic_linear_small_rows_f32", at, M, K, w.data_ptr, ldw, N, scale.data_ptr, wsum.data_ptr, b,
+                        *grid, y.data_ptr, None)
+        else:
+            _C.call("lq_dynamic_linear_f32", at, M, K, w.data_ptr, ldw, N, scale.data_ptr, wsum.data_ptr, b, *grid,
+                    y.data_ptr if M else None, None)
+        if fresh:
+            _keep(*fresh)
+        return y
+
     def forward(self, x: Tensor, residual: Tensor | None = None, activation: str | None = None,
                 track_range: bool = False) -> Tensor:
         """Beyond Lucid's signature, all inside the GEMM epilogue: ``residual`` is added to
@@ -183,36 +246,12 @@ class Linear(Module):
         if x.shape[-1] != K:
             raise _C.ShapeMismatch(f"expected last dim {K}, got {x.shape}")
         M = x.numel // K
+        if x._range is None and residual is None and activation is None and not track_range:
+            y = self._one_call(x, M, 0)
+            if y is not None:
+                return y
         qd = self.act_qdtype
         off = storage_offset(qd)
-        if (x._range is None and residual is None and activation is None and not track_range
-                and weight_zero_points(self) is None and _one_call_takes(M, K)
-                and (taken := _kernel_operands(self, N, K)) is not None):
-            # min / max, qparams, codes, GEMM and bias behind one call (same bits whichever)
-            w, scale, bias = taken
-            wsum, fresh = self._wsum, ()
-            if wsum is None:
-                wsum = self._weight_sums()
-                fresh = ((self, "_wsum", wsum),)
-            y = Tensor.empty((*x.shape[:-1], N), T.float32, "hip")
-            grid = (0, 0, qd.quant_min, qd.quant_max, int(qd.signed), 1e-8, off)
-            b = None if bias is None else bias.data_ptr
-            if _one_launch_pays(M, K, N):
-                _C.call("lq_dynamic_linear_small_f32", x.data_ptr, M, K, w.data_ptr, N, scale.data_ptr,
-                        wsum.data_ptr, b, *grid, y.data_ptr, None)
-            else:
-                ldw = K
-                if K % 16:
-                    rows = self._wrows
-                    if rows is None:
-                        rows = self._weight_rows()
-                        fresh += ((self, "_wrows", rows),)
-                    w, ldw = rows
-                _C.call("lq_dynamic_linear_f32", x.data_ptr if M else None, M, K, w.data_ptr, ldw, N, scale.data_ptr,
-                        wsum.data_ptr, b, *grid, y.data_ptr if M else None, None)
-            if fresh:
-                _keep(*fresh)
-            return y
         xq = Tensor.empty((M, K), T.int8, "hip")
         small = x._range is None and x.numel <= (1 << 18)
         if small:

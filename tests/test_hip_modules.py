@@ -699,6 +699,82 @@ def test_two_dynamic_linears_in_one_launch(M, K1, N1, N2, relu, kind):
         assert np.array_equal(got.view(np.uint32), exp.view(np.uint32))
 
 
+def _pair(rng, K1, N1, N2, relu=True):
+    l1, l2 = nn.Linear(K1, N1), nn.Linear(N1, N2)
+    for lin, shape in ((l1, (N1, K1)), (l2, (N2, N1))):
+        lin.register_buffer("weight", L.tensor((rng.standard_normal(shape) * 0.05).astype(np.float32)))
+        lin.register_buffer("bias", L.tensor((rng.standard_normal(shape[0]) * 0.05).astype(np.float32)))
+    return Q.quantize_dynamic(nn.Sequential(*([l1, nn.ReLU(), l2] if relu else [l1, l2])))
+
+
+def _same_as_one_after_the_other(model, xd, got):
+    """The operators one by one, through the general quantization and GEMM."""
+    h = xd
+    for m in (model[i] for i in range(len(model))):
+        if type(m) is nnqd.Linear:
+            mn, mx = Q.minmax(h)
+            s, z = Q.calculate_qparams(mn, mx, Q.per_tensor_affine, Q.quint8)
+            codes = Q.quantize(h, s, z, Q.quint8).numpy().astype(np.int16) - 128
+            h = m.forward_quantized(hip(codes.astype(np.int8)), s, z, h.shape[:-1])
+        else:
+            h = m(h)
+    got, want = got.numpy(), h.numpy()
+    assert got.shape == want.shape and np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~np.isnan(got)].view(np.uint32), want[~np.isnan(want)].view(np.uint32))
+
+
+@pytest.mark.parametrize("M,K1,N1,N2", [(1, 1, 1, 1), (1, 98, 48, 3), (12, 91, 32, 58), (3, 549, 33, 13), (64, 1023, 511, 64),
+                                        (17, 640, 45, 17), (16, 1001, 257, 16), (64, 1024, 496, 10), (49, 784, 272, 10),
+                                        (63, 1009, 255, 1), (15, 16, 17, 5)])
+@pytest.mark.parametrize("kind", ["normal", "constant", "nan", "inf"])
+def test_two_dynamic_linears_of_any_sizes_in_one_launch(M, K1, N1, N2, kind):
+    """Rows that are no whole 16 bytes, hidden layers up to 511: one call, the bits of the separate operators."""
+    rng = np.random.default_rng(M + K1 + N1 + N2)
+    model = _pair(rng, K1, N1, N2)
+    x = rng.standard_normal((M, K1)).astype(np.float32)
+    if kind == "constant":
+        x[:] = -0.25
+    elif kind != "normal":
+        x[M - 1, K1 - 1] = np.nan if kind == "nan" else np.inf
+    xd = hip(x)
+    model(xd)
+    with _recorded_calls() as calls:
+        got = model(xd)
+    assert calls == ["lq_dynamic_mlp2_small_rows_f32"]
+    _same_as_one_after_the_other(model, xd, got)
+
+
+@pytest.mark.parametrize("M,K1,N1,N2,row", [(65, 784, 256, 10, 0), (256, 91, 512, 64, 0), (70, 33, 20, 65, 0), (8, 91, 40, 7, 1),
+                                            (64, 2000, 64, 10, 0)])
+def test_the_relu_between_two_dynamic_linears_rides_in_the_first(M, K1, N1, N2, row):
+    """Beyond the one launch, and on rows of an activation that begin at no 16 bytes: two calls, the same bits."""
+    rng = np.random.default_rng(M + K1)
+    model = _pair(rng, K1, N1, N2)
+    xd = hip(rng.standard_normal((M + row, K1)).astype(np.float32)).row_range(row, row + M)
+    model(xd)
+    with _recorded_calls() as calls:
+        got = model(xd)
+    assert len(calls) == 2 and "lq_relu_f32" not in calls
+    _same_as_one_after_the_other(model, xd, got)
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 3, 5), (17, 33, 16), (64, 1023, 100), (10, 6079, 17), (33, 91, 250)])
+@pytest.mark.parametrize("row", [0, 1])
+def test_one_launch_dynamic_linear_of_any_row_length(M, K, N, row):
+    rng = np.random.default_rng(M + K)
+    lin = nn.Linear(K, N)
+    lin.register_buffer("weight", L.tensor((rng.standard_normal((N, K)) * 0.05).astype(np.float32)))
+    model = Q.quantize_dynamic(nn.Sequential(lin))
+    xd = hip((rng.standard_normal((M + row, K)) * 3 - 1).astype(np.float32)).row_range(row, row + M)
+    model(xd)
+    with _recorded_calls() as calls:
+        got = model(xd)
+    # (a view whose rows begin at no 16 bytes takes the two launches)
+    one = xd.data_ptr % 16 == 0 and 43 * M * K + 2400 * K <= 6_000_000
+    assert calls == ["lq_dynamic_linear_small_rows_f32" if one else "lq_dynamic_linear_f32"]
+    _same_as_one_after_the_other(model, xd, got)
+
+
 def test_two_dynamic_linears_keep_separate_launches_when_hooked_or_large():
     """A forward hook has to see each module's own output, and a wide layer is not what the one
     launch takes: the modules then run one after the other."""
