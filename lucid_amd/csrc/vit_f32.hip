@@ -385,7 +385,7 @@ typedef __bf16 sg_v8bf __attribute__((ext_vector_type(8)));
 // v_mfma_f32_32x32x16_bf16 per 16 k, against eight of v_mfma_f32_32x32x2_f32 at four times the
 // cycles each.
 //
-// 128 x 128 x 32 block tile, 4 wavefronts of 64 x 64; the next tile's operands wait in registers
+// 128 x 128 x 32 block tile, 4 wavefronts of 64 x 64; BLOCKS of them per CU; the next tile's operands wait in registers
 // while the current one is multiplied.  LDS: per part 256 rows (A's 128, then W's) of 32
 // bfloat16 = 64 bytes; the 16-byte chunk k of row r sits at chunk k ^ ((r / 4) % 4), which puts
 // the 16 rows of a fragment pass on 16 different bank groups.
@@ -406,68 +406,53 @@ struct PatchForm {
     const float* pos;  // [(1 + per_image), N]
 };
 
+// NU rows of A and as many of W for a thread, RS apart from row `a_row` / `w_row` on: groups of four consecutive k.
 // PATCH 0: a is a plain [M,K] matrix.  1: patch rows with p a power of two and every group of
 // four columns one aligned 16-byte load (no branch and no division in the loop).  2: patch rows
 // of any geometry, element by element.
-template <int PATCH>
-__global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restrict__ a, const float* __restrict__ w,
-                                                          const float* __restrict__ bias, float* __restrict__ out,
-                                                          int M, int N, int K, PatchForm pf) {
-    __shared__ __attribute__((aligned(16))) uint16_t sp[3][SG_ROWS * SG_BK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int m0 = blockIdx.y * SG_BM, n0 = blockIdx.x * SG_BN;
-    // loader: piece tid + 256 u = row (tid + 256 u) / 8 of either operand, four consecutive k at 4 * (tid % 8)
-    const int lrow = tid >> 3, lk = (tid & 7) * 4;
-    const bool vec = (K % 4 == 0) && aligned16(w) && (PATCH != 0 || aligned16(a));
-    size_t patch_at[4];  // PATCH: where the patch of loader row u starts in the image
-    if constexpr (PATCH != 0) {
+// VEC: groups of four k of both operands are whole, aligned 16 bytes (known to the compiler: where the two ways to load meet,
+// the registers of one are copied, and a copy waits for the load).
+template <int PATCH, bool VEC, int RS, int NU>
+struct SgLoader {
+    const float* __restrict__ a;
+    const float* __restrict__ w;
+    int M, N, K, a_row, w_row;
+    const PatchForm& pf;
+    size_t patch_at[NU];  // PATCH: where the patch of row u starts in the image
+    __device__ __forceinline__ SgLoader(const float* a_, const float* w_, int M_, int N_, int K_, int a_row_, int w_row_,
+                                        const PatchForm& pf_)
+        : a(a_), w(w_), M(M_), N(N_), K(K_), a_row(a_row_), w_row(w_row_), pf(pf_) {
+        if constexpr (PATCH != 0) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int row = min(m0 + lrow + 32 * u, M - 1);
-            const int b = row / pf.per_image, i = row - b * pf.per_image;
-            const int gy = i / pf.gw, gx = i - gy * pf.gw;
-            patch_at[u] = (size_t(b) * pf.C * pf.H + size_t(gy) * pf.p) * pf.W + size_t(gx) * pf.p;
+            for (int u = 0; u < NU; ++u) {
+                const int row = min(a_row + RS * u, M - 1);
+                const int b = row / pf.per_image, i = row - b * pf.per_image;
+                const int gy = i / pf.gw, gx = i - gy * pf.gw;
+                patch_at[u] = (size_t(b) * pf.C * pf.H + size_t(gy) * pf.p) * pf.W + size_t(gx) * pf.p;
+            }
         }
     }
-    v16f acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-    float4 ra[4], rb[4];
-    auto fetch_row = [&](const float* base, int row, int rows, int k) {
+    __device__ __forceinline__ float4 any_row(const float* base, int row, int rows, int k) const {
         float4 v = {0.f, 0.f, 0.f, 0.f};
         if (row < rows) {
             const float* p = base + size_t(row) * K + k;
-            if (vec && k + 3 < K) {
-                v = *reinterpret_cast<const float4*>(p);
-            } else {
-                if (k < K) v.x = p[0];
-                if (k + 1 < K) v.y = p[1];
-                if (k + 2 < K) v.z = p[2];
-                if (k + 3 < K) v.w = p[3];
-            }
+            if (k < K) v.x = p[0];
+            if (k + 1 < K) v.y = p[1];
+            if (k + 2 < K) v.z = p[2];
+            if (k + 3 < K) v.w = p[3];
         }
         return v;
-    };
-    // PATCH: column k of a patch row is pixel (c, ph, pw) of the patch.  Loads go to clamped
-    // (always valid) addresses and what lies past M or K is zeroed afterwards, so that the four
-    // loads of a fetch are issued back to back.
-    auto fetch_patches = [&](int k) {
+    }
+    // PATCH: column k of a patch row is pixel (c, ph, pw) of the patch.  Loads go to clamped (always valid) addresses: what
+    // a row past M gives is never stored, what lies past K is zeroed when it is stashed (zeroed here, every load would be
+    // waited for where it is issued).
+    __device__ __forceinline__ void patches(int k, float4 (&ra)[NU]) const {
         if constexpr (PATCH == 1) {
             const int kk = min(k, K - 4);
             const int pw = kk & (pf.p - 1), ph = (kk >> pf.log2p) & (pf.p - 1), c = kk >> (2 * pf.log2p);
             const size_t pixel = (size_t(c) * pf.H + ph) * pf.W + pw;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) ra[u] = *reinterpret_cast<const float4*>(a + patch_at[u] + pixel);
-            if (k >= K) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) ra[u] = float4{0.f, 0.f, 0.f, 0.f};
-            }
+            for (int u = 0; u < NU; ++u) ra[u] = *reinterpret_cast<const float4*>(a + patch_at[u] + pixel);
         } else {
             const int pp = pf.p * pf.p;
             size_t pixel[4];
@@ -479,69 +464,87 @@ __global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restric
                 pixel[e] = (size_t(c) * pf.H + ph) * pf.W + pw;
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < NU; ++u) {
                 const float* p = a + patch_at[u];
                 ra[u] = float4{p[pixel[0]], p[pixel[1]], p[pixel[2]], p[pixel[3]]};
             }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (k >= K) ra[u].x = 0.f;
-                if (k + 1 >= K) ra[u].y = 0.f;
-                if (k + 2 >= K) ra[u].z = 0.f;
-                if (k + 3 >= K) ra[u].w = 0.f;
-            }
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (m0 + lrow + 32 * u >= M) ra[u] = float4{0.f, 0.f, 0.f, 0.f};
-    };
-    // plain rows in the aligned case: the row is clamped instead of tested (a row past the end
-    // only feeds results that are never stored) and a k past the end is zeroed afterwards
-    auto fetch_rows_vec = [&](const float* base, int row0, int rows, int k, float4 (&r)[4]) {
+    }
+    // plain rows in the aligned case
+    __device__ __forceinline__ void rows_vec(const float* base, int row0, int rows, int k, float4 (&r)[NU]) const {
         const int kk = min(k, K - 4);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            r[u] = *reinterpret_cast<const float4*>(base + size_t(min(row0 + 32 * u, rows - 1)) * K + kk);
-        if (k >= K) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) r[u] = float4{0.f, 0.f, 0.f, 0.f};
-        }
-    };
-    auto fetch = [&](int k0) {
-        if constexpr (PATCH != 0) fetch_patches(k0 + lk);
-        if (vec) {
-            if constexpr (PATCH == 0) fetch_rows_vec(a, m0 + lrow, M, k0 + lk, ra);
-            fetch_rows_vec(w, n0 + lrow, N, k0 + lk, rb);
+        for (int u = 0; u < NU; ++u)
+            r[u] = *reinterpret_cast<const float4*>(base + size_t(min(row0 + RS * u, rows - 1)) * K + kk);
+    }
+    __device__ __forceinline__ void operator()(int k, float4 (&ra)[NU], float4 (&rb)[NU]) const {
+        if constexpr (PATCH != 0) patches(k, ra);
+        if constexpr (VEC) {
+            if constexpr (PATCH == 0) rows_vec(a, a_row, M, k, ra);
+            rows_vec(w, w_row, N, k, rb);
         } else {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if constexpr (PATCH == 0) ra[u] = fetch_row(a, m0 + lrow + 32 * u, M, k0 + lk);
-                rb[u] = fetch_row(w, n0 + lrow + 32 * u, N, k0 + lk);
+            for (int u = 0; u < NU; ++u) {
+                if constexpr (PATCH == 0) ra[u] = any_row(a, a_row + RS * u, M, k);
+                rb[u] = any_row(w, w_row + RS * u, N, k);
             }
         }
-    };
-    auto stash_one = [&](int row, float4 v) {
-        uint32_t lo[3], hi[3];
-        at_split3x2(v.x, v.y, lo[0], lo[1], lo[2]);
-        at_split3x2(v.z, v.w, hi[0], hi[1], hi[2]);
-        const int at = sg_index(row, lk);
+    }
+};
+
+// a tile that reaches past K: zeros there
+template <int NU>
+__device__ __forceinline__ void sg_inside(float4 (&r)[NU], int k, int K) {
 #pragma unroll
-        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(&sp[p][at]) = uint2{lo[p], hi[p]};
-    };
-    auto stash = [&] {
+    for (int u = 0; u < NU; ++u) {
+        r[u].x = k < K ? r[u].x : 0.f, r[u].y = k + 1 < K ? r[u].y : 0.f;
+        r[u].z = k + 2 < K ? r[u].z : 0.f, r[u].w = k + 3 < K ? r[u].w : 0.f;
+    }
+}
+
+// four consecutive k of a row, as three parts, into an image of rows of SG_BK bfloat16 per part
+template <int LEN>
+__device__ __forceinline__ void sg_stash(uint16_t (&sp)[3][LEN], int row, int k, float4 v) {
+    uint32_t lo[3], hi[3];
+    at_split3x2(v.x, v.y, lo[0], lo[1], lo[2]);
+    at_split3x2(v.z, v.w, hi[0], hi[1], hi[2]);
+    const int at = sg_index(row, k);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            stash_one(lrow + 32 * u, ra[u]);
-            stash_one(SG_BM + lrow + 32 * u, rb[u]);
-        }
-    };
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(&sp[p][at]) = uint2{lo[p], hi[p]};
+}
+
+template <int PATCH, bool VEC, int BLOCKS>
+__global__ __launch_bounds__(256, BLOCKS) void sgemm_nt_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                               const float* __restrict__ bias, float* __restrict__ out,
+                                                               int M, int N, int K, PatchForm pf) {
+    __shared__ __attribute__((aligned(16))) uint16_t sp[3][SG_ROWS * SG_BK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int m0 = blockIdx.y * SG_BM, n0 = blockIdx.x * SG_BN;
+    // loader: row tid / 8 (+ 32 u) of either operand, four consecutive k at 4 * (tid % 8)
+    const int lrow = tid >> 3, lk = (tid & 7) * 4;
+    const SgLoader<PATCH, VEC, 32, 4> fetch(a, w, M, N, K, m0 + lrow, n0 + lrow, pf);
+    v16f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    float4 ra[4], rb[4];
     const int nk = (K + SG_BK - 1) / SG_BK;
     const int fr = lane & 31, kg = lane >> 5;
-    fetch(0);
+    fetch(lk, ra, rb);
     for (int t = 0; t < nk; ++t) {
-        stash();
-        __syncthreads();
-        if (t + 1 < nk) fetch((t + 1) * SG_BK);
+        if ((t + 1) * SG_BK > K) sg_inside(ra, t * SG_BK + lk, K), sg_inside(rb, t * SG_BK + lk, K);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            sg_stash(sp, lrow + 32 * u, lk, ra[u]);
+            sg_stash(sp, SG_BM + lrow + 32 * u, lk, rb[u]);
+        }
+        lds_barrier();
+        if (t + 1 < nk) fetch((t + 1) * SG_BK + lk, ra, rb);
 #pragma unroll
         for (int ks = 0; ks < SG_BK / 16; ++ks) {
             uint4 fa[2][3], fb[2][3];
@@ -568,7 +571,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restric
             };
             mm(1, 1), mm(0, 2), mm(2, 0), mm(0, 1), mm(1, 0), mm(0, 0);
         }
-        __syncthreads();  // the tile has been read: the next one may be written
+        lds_barrier();  // the tile has been read: the next one may be written (what was requested is still on its way)
     }
     // result layout of the 32x32 MFMA: column = lane % 32, row = 8*(r/4) + 4*(lane/32) + r%4
 #pragma unroll
@@ -617,6 +620,139 @@ __global__ __launch_bounds__(256, 2) void sgemm_nt_kernel(const float* __restric
             }
         }
     }
+}
+
+
+// The same product for few tiles: 32 x 32 outputs per block, K dealt to its four wavefronts in turns of SG_BK, each of which
+// stages its own rows in LDS of its own (no barrier in the loop) and keeps two sums per element (even and odd halves of a
+// turn, so that consecutive MFMAs do not wait for each other); the eight sums are added once, in a fixed order.  A 128 x 128
+// tile is a chain of K / 32 turns of 2.2 us (split, barrier, LDS reads, MFMAs, barrier) however few of them there are:
+// patches of ViT-B/16, K = N = 768, us: 196 rows 55 -> 9, 784 55 -> 17, 1568 61 -> 27, 3136 62 -> 52.  Beyond
+// SG_SMALL_BLOCKS blocks the larger tiles win, whose operands are split less often (4704 rows 69 against 58, 2048 x 2048 x 512
+// 52 against 42).  Root mean square of the error against float64 6.4e-8 of the result's (1.6e-7 for the large tiles, whose
+// sums are longer).
+constexpr int SG_SMALL = 32;
+constexpr long SG_SMALL_BLOCKS = 2600;
+
+template <int PATCH, bool VEC>
+__global__ __launch_bounds__(256, 3) void sgemm_nt_small_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                const float* __restrict__ bias, float* __restrict__ out,
+                                                                int M, int N, int K, PatchForm pf) {
+    __shared__ __attribute__((aligned(16))) union {
+        uint16_t parts[4][3][2 * SG_SMALL * SG_BK];
+        float sums[4][SG_SMALL][SG_SMALL + 4];
+    } lds;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m0 = blockIdx.y * SG_SMALL, n0 = blockIdx.x * SG_SMALL;
+    const int lrow = lane >> 3, lk = (lane & 7) * 4;
+    const SgLoader<PATCH, VEC, 8, 4> fetch(a, w, M, N, K, m0 + lrow, n0 + lrow, pf);
+    uint16_t(&sp)[3][2 * SG_SMALL * SG_BK] = lds.parts[wave];
+    v16f acc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+    const int nk = (K + SG_BK - 1) / SG_BK;
+    const int fr = lane & 31, kg = lane >> 5;
+    float4 ra[4], rb[4];
+    if (wave < nk) fetch(wave * SG_BK + lk, ra, rb);
+    for (int t = wave; t < nk; t += 4) {
+        if ((t + 1) * SG_BK > K) sg_inside(ra, t * SG_BK + lk, K), sg_inside(rb, t * SG_BK + lk, K);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            sg_stash(sp, lrow + 8 * u, lk, ra[u]);
+            sg_stash(sp, SG_SMALL + lrow + 8 * u, lk, rb[u]);
+        }
+        // (the wavefront's own LDS: its instructions execute in order, the fence is for the compiler)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (t + 4 < nk) fetch((t + 4) * SG_BK + lk, ra, rb);
+        uint4 fa[2][3], fb[2][3];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int at = sg_index(fr, 16 * ks + 8 * kg), bt = sg_index(SG_SMALL + fr, 16 * ks + 8 * kg);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                fa[ks][p] = *reinterpret_cast<const uint4*>(&sp[p][at]);
+                fb[ks][p] = *reinterpret_cast<const uint4*>(&sp[p][bt]);
+            }
+        }
+        auto mm = [&](int pa, int pb) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+                acc[ks] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(sg_v8bf, fa[ks][pa]),
+                                                                  __builtin_bit_cast(sg_v8bf, fb[ks][pb]), acc[ks], 0, 0, 0);
+        };
+        mm(1, 1), mm(0, 2), mm(2, 0), mm(0, 1), mm(1, 0), mm(0, 0);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) lds.sums[wave][8 * (r >> 2) + 4 * kg + (r & 3)][fr] = acc[0][r] + acc[1][r];
+    __syncthreads();
+    // row tid / 8, four columns from 4 * (tid % 8)
+    const int row = tid >> 3, col = (tid & 7) * 4, m = m0 + row;
+    if (m < M) {
+        float4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const float4*>(&lds.sums[i][row][col]);
+        const float y[4] = {(v[0].x + v[1].x) + (v[2].x + v[3].x), (v[0].y + v[1].y) + (v[2].y + v[3].y),
+                            (v[0].z + v[1].z) + (v[2].z + v[3].z), (v[0].w + v[1].w) + (v[2].w + v[3].w)};
+        size_t at = size_t(m) * N;
+        const float* pos = nullptr;
+        if constexpr (PATCH != 0) {
+            const int b = m / pf.per_image, t = m - b * pf.per_image;
+            at = (size_t(b) * (pf.per_image + 1) + 1 + t) * N;
+            pos = pf.pos + size_t(1 + t) * N;
+        }
+        float bv[4], pv[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int n = min(n0 + col + e, N - 1);
+            bv[e] = bias ? bias[n] : 0.0f;
+            pv[e] = PATCH != 0 ? pos[n] : 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int n = n0 + col + e;
+            if (n < N) out[at + n] = PATCH != 0 ? (y[e] + bv[e]) + pv[e] : y[e] + bv[e];
+        }
+    }
+    if constexpr (PATCH != 0) {
+        if (blockIdx.y == 0) {
+            // class-token rows: token 0 of every image, this block's columns
+            const int n = n0 + (tid & 31);
+            if (n < N) {
+                const float v = pf.cls[n] + pf.pos[n];
+                for (int b = tid >> 5; b < pf.B; b += 8) out[size_t(b) * (pf.per_image + 1) * N + n] = v;
+            }
+        }
+    }
+}
+
+// (by M and N alone: a matrix and the image whose patches are its rows get the same sums)
+template <int PATCH, bool VEC>
+int launch_sgemm(const float* a, const float* w, const float* bias, float* out, int M, int N, int K, const PatchForm& pf,
+                 hipStream_t st) {
+    const long tiles_m = (long(M) + SG_SMALL - 1) / SG_SMALL, tiles_n = (long(N) + SG_SMALL - 1) / SG_SMALL;
+    if (tiles_m * tiles_n <= SG_SMALL_BLOCKS) {
+        const dim3 grid{unsigned(tiles_n), unsigned(tiles_m)};
+        sgemm_nt_small_kernel<PATCH, VEC><<<grid, 256, 0, st>>>(a, w, bias, out, M, N, K, pf);
+    } else {
+        const dim3 grid{(unsigned(N) + SG_BN - 1) / SG_BN, (unsigned(M) + SG_BM - 1) / SG_BM};
+        const long tiles = long(grid.x) * grid.y;
+        // three blocks per CU (168 registers, up to 4 % slower) where they are one round and two per CU are a second, nearly
+        // empty one: 12 544 rows of ViT-B/16's patches, 588 tiles, 134 -> 106 us; 441 tiles 78 with two, 82 with three
+        if (tiles > 512 && tiles <= 768)
+            sgemm_nt_kernel<PATCH, VEC, 3><<<grid, 256, 0, st>>>(a, w, bias, out, M, N, K, pf);
+        else
+            sgemm_nt_kernel<PATCH, VEC, 2><<<grid, 256, 0, st>>>(a, w, bias, out, M, N, K, pf);
+    }
+    LQ_CHECK_LAUNCH();
+    return LQ_OK;
 }
 
 // ---------------------------------------------------------------- attention
@@ -1418,11 +1554,9 @@ int lq_sgemm_nt_f32(const float* a, const float* w, const float* bias, float* ou
     LQ_REQUIRE(a && w && out, LQ_ERR_VALUE, "sgemm: null pointer");
     LQ_REQUIRE(M >= 0 && N >= 0 && K > 0, LQ_ERR_SHAPE, "sgemm: bad shape (%d, %d, %d)", M, N, K);
     if (M == 0 || N == 0) return LQ_OK;
-    dim3 grid((N + SG_BN - 1) / SG_BN, (M + SG_BM - 1) / SG_BM);
-    LQ_REQUIRE(grid.y < 65536, LQ_ERR_SHAPE, "sgemm: M too large");
-    sgemm_nt_kernel<0><<<grid, 256, 0, as_stream(stream)>>>(a, w, bias, out, M, N, K, PatchForm{});
-    LQ_CHECK_LAUNCH();
-    return LQ_OK;
+    LQ_REQUIRE(M <= 65535 * SG_BM, LQ_ERR_SHAPE, "sgemm: M too large");
+    const bool vec = K % 4 == 0 && aligned16(a) && aligned16(w);
+    return (vec ? launch_sgemm<0, true> : launch_sgemm<0, false>)(a, w, bias, out, M, N, K, PatchForm{}, as_stream(stream));
 }
 
 int lq_patch_embed_f32(const float* img, const float* w, const float* bias, const float* cls, const float* pos,
@@ -1435,18 +1569,16 @@ int lq_patch_embed_f32(const float* img, const float* w, const float* bias, cons
     const size_t rows = size_t(B) * per_image, K = size_t(C) * patch * patch;
     LQ_REQUIRE(rows < (size_t(1) << 31) && K < (size_t(1) << 31), LQ_ERR_SHAPE, "patch_embed: too many patch rows");
     if (B == 0) return LQ_OK;
-    dim3 grid((D + SG_BN - 1) / SG_BN, (unsigned(rows) + SG_BM - 1) / SG_BM);
-    LQ_REQUIRE(grid.y < 65536, LQ_ERR_SHAPE, "patch_embed: too many patch rows");
+    LQ_REQUIRE(rows <= size_t(65535) * SG_BM, LQ_ERR_SHAPE, "patch_embed: too many patch rows");
     int log2p = -1;
     for (int e = 0; e < 15; ++e)
         if ((1 << e) == patch) log2p = e;
     const PatchForm pf{C, H, W, patch, W / patch, per_image, B, log2p, cls, pos};
-    if (log2p >= 2 && W % 4 == 0 && aligned16(img))
-        sgemm_nt_kernel<1><<<grid, 256, 0, as_stream(stream)>>>(img, w, bias, out, int(rows), D, int(K), pf);
-    else
-        sgemm_nt_kernel<2><<<grid, 256, 0, as_stream(stream)>>>(img, w, bias, out, int(rows), D, int(K), pf);
-    LQ_CHECK_LAUNCH();
-    return LQ_OK;
+    const bool vec = K % 4 == 0 && aligned16(w);
+    const auto launch = vec && log2p >= 2 && W % 4 == 0 && aligned16(img) ? launch_sgemm<1, true>
+                        : vec                                             ? launch_sgemm<2, true>
+                                                                          : launch_sgemm<2, false>;
+    return launch(img, w, bias, out, int(rows), D, int(K), pf, as_stream(stream));
 }
 
 int lq_gather_rows_f32(const float* src, size_t src_row_stride, float* dst, size_t rows, size_t cols,

@@ -229,6 +229,24 @@ def test_patch_embedding_of_an_image_that_is_not_16_byte_aligned():
     assert np.array_equal(outs[0], outs[1]) and np.isfinite(outs[0]).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 33, 4), (31, 32, 31), (32, 31, 32), (33, 65, 33), (65, 64, 128), (64, 96, 132),
+                                   (200, 40, 97), (1600, 1664, 36), (1632, 1664, 36), (2689, 1152, 40), (4096, 3073, 68)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_float_gemm_of_any_size(M, N, K, shift):
+    """Both tile sizes (2600 tiles of 32 x 32 are the line; 588 large tiles run three per CU), K of whole and partial turns, rows
+    that are no 16 bytes, operands that begin at none: within the roundings of the additions, each at most
+    2^-24 of the sum of the terms' magnitudes (six per 16 k, the halves and wavefronts, the product's own and the bias)."""
+    rng = np.random.default_rng(M + N + K)
+    flat = [rng.standard_normal(n + shift).astype(np.float32) for n in (M * K, N * K)]
+    bias = rng.standard_normal(N).astype(np.float32)
+    a, w = (L.Tensor(s, L.float32, "hip", buf=hip(f)._buf, offset=4 * shift) for f, s in zip(flat, ((M, K), (N, K))))
+    out, bv = L.tensor(np.full((M, N), np.nan, np.float32), device="hip"), hip(bias)
+    _C.call("lq_sgemm_nt_f32", a.data_ptr, w.data_ptr, bv.data_ptr, out.data_ptr, M, N, K, None)
+    a64, w64 = (f[shift:].reshape(s).astype(np.float64) for f, s in zip(flat, ((M, K), (N, K))))
+    bound = (6 * ((K + 15) // 16) + 12) * 2.0 ** -24 * (np.abs(a64) @ np.abs(w64).T + np.abs(bias))
+    assert (np.abs(out.numpy() - (a64 @ w64.T + bias)) <= bound).all()
+
+
 def test_patch_embedding_refuses_a_ragged_image():
     z = L.Tensor.empty((1, 3, 20, 32), L.float32, "hip")
     o = L.Tensor.empty((1, 3, 8), L.float32, "hip")
