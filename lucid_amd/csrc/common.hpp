@@ -63,6 +63,8 @@ struct SkScratch {
     int32_t* slabs = nullptr;
 };
 int sk_scratch(size_t counters, size_t slab_bytes, hipStream_t st, SkScratch* out);
+// lq_sgemm_nt_f32; `large`: 128 x 128 tiles for a small problem too.
+int sgemm_nt(const float* a, const float* w, const float* bias, float* out, int M, int N, int K, bool large, hipStream_t st);
 // Launches that may be placed at once: the hardware queues of the process, which HIP takes from the environment (four unless
 // GPU_MAX_HW_QUEUES says more).  What a kernel whose blocks wait for each other leaves free for launches like it.
 int hardware_queues();

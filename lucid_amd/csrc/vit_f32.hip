@@ -736,9 +736,9 @@ __global__ __launch_bounds__(256, 3) void sgemm_nt_small_kernel(const float* __r
 // (by M and N alone: a matrix and the image whose patches are its rows get the same sums)
 template <int PATCH, bool VEC>
 int launch_sgemm(const float* a, const float* w, const float* bias, float* out, int M, int N, int K, const PatchForm& pf,
-                 hipStream_t st) {
+                 hipStream_t st, bool large) {
     const long tiles_m = (long(M) + SG_SMALL - 1) / SG_SMALL, tiles_n = (long(N) + SG_SMALL - 1) / SG_SMALL;
-    if (tiles_m * tiles_n <= SG_SMALL_BLOCKS) {
+    if (!large && tiles_m * tiles_n <= SG_SMALL_BLOCKS) {
         const dim3 grid{unsigned(tiles_n), unsigned(tiles_m)};
         sgemm_nt_small_kernel<PATCH, VEC><<<grid, 256, 0, st>>>(a, w, bias, out, M, N, K, pf);
     } else {
@@ -1412,6 +1412,17 @@ unsigned blocks_for(size_t n) { return unsigned((n + 255) / 256); }
 
 }  // namespace
 
+namespace lq {
+int sgemm_nt(const float* a, const float* w, const float* bias, float* out, int M, int N, int K, bool large, hipStream_t st) {
+    LQ_REQUIRE(a && w && out, LQ_ERR_VALUE, "sgemm: null pointer");
+    LQ_REQUIRE(M >= 0 && N >= 0 && K > 0, LQ_ERR_SHAPE, "sgemm: bad shape (%d, %d, %d)", M, N, K);
+    if (M == 0 || N == 0) return LQ_OK;
+    LQ_REQUIRE(M <= 65535 * SG_BM, LQ_ERR_SHAPE, "sgemm: M too large");
+    const bool vec = K % 4 == 0 && aligned16(a) && aligned16(w);
+    return (vec ? launch_sgemm<0, true> : launch_sgemm<0, false>)(a, w, bias, out, M, N, K, PatchForm{}, st, large);
+}
+}  // namespace lq
+
 extern "C" {
 
 int lq_layernorm_f32(const float* x, const float* gamma, const float* beta, float* out, long rows, int cols,
@@ -1551,12 +1562,7 @@ int lq_assemble_tokens_f32(const float* patches, const float* cls, const float* 
 
 int lq_sgemm_nt_f32(const float* a, const float* w, const float* bias, float* out, int M, int N, int K,
                     void* stream) {
-    LQ_REQUIRE(a && w && out, LQ_ERR_VALUE, "sgemm: null pointer");
-    LQ_REQUIRE(M >= 0 && N >= 0 && K > 0, LQ_ERR_SHAPE, "sgemm: bad shape (%d, %d, %d)", M, N, K);
-    if (M == 0 || N == 0) return LQ_OK;
-    LQ_REQUIRE(M <= 65535 * SG_BM, LQ_ERR_SHAPE, "sgemm: M too large");
-    const bool vec = K % 4 == 0 && aligned16(a) && aligned16(w);
-    return (vec ? launch_sgemm<0, true> : launch_sgemm<0, false>)(a, w, bias, out, M, N, K, PatchForm{}, as_stream(stream));
+    return sgemm_nt(a, w, bias, out, M, N, K, false, as_stream(stream));
 }
 
 int lq_patch_embed_f32(const float* img, const float* w, const float* bias, const float* cls, const float* pos,
@@ -1578,7 +1584,7 @@ int lq_patch_embed_f32(const float* img, const float* w, const float* bias, cons
     const auto launch = vec && log2p >= 2 && W % 4 == 0 && aligned16(img) ? launch_sgemm<1, true>
                         : vec                                             ? launch_sgemm<2, true>
                                                                           : launch_sgemm<2, false>;
-    return launch(img, w, bias, out, int(rows), D, int(K), pf, as_stream(stream));
+    return launch(img, w, bias, out, int(rows), D, int(K), pf, as_stream(stream), false);
 }
 
 int lq_gather_rows_f32(const float* src, size_t src_row_stride, float* dst, size_t rows, size_t cols,

@@ -705,8 +705,6 @@ int check_group(const char* who, int K, int gs, int bits) {
 
 extern "C" {
 
-int lq_sgemm_nt_f32(const float* a, const float* w, const float* bias, float* out, int M, int N, int K, void* stream);
-
 int lq_wq_quantize(const float* w, int N, int K, int group_size, int bits, uint32_t* packed, float* scales,
                    float* biases, lq_stream stream) {
     int rc = check_group("wq_quantize", K, group_size, bits);
@@ -765,7 +763,8 @@ int lq_wq_matmul(const float* x, const uint32_t* packed, const float* scales, co
     if (rc) return rc;
     rc = lq_wq_dequantize(packed, scales, biases, N, K, group_size, bits, static_cast<float*>(ws), stream);
     if (rc) return rc;
-    return lq_sgemm_nt_f32(x, static_cast<const float*>(ws), nullptr, out, M, N, K, stream);
+    // (its large tiles whatever the size: a rare route, and the one that the products without a decoded weight are measured against)
+    return sgemm_nt(x, static_cast<const float*>(ws), nullptr, out, M, N, K, true, st);
 }
 
 }  // extern "C"
