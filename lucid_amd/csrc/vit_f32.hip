@@ -26,9 +26,21 @@ namespace {
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
+// The sum over the 64 lanes, in every lane: lane l adds lane l ^ 32's value, then l ^ 16's, 8, 4, 2, 1.  (Rows of 16 lanes are
+// rotated by 8, 4, 2, 1: once a value is the same in lanes that differ in bit 3, lane l + 4 has what lane l ^ 4 has, and so
+// on.  As six ds_bpermute the two sums of a LayerNorm row were a chain of 1200 cycles.)
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    typedef unsigned pair __attribute__((ext_vector_type(2)));
+    pair p = __builtin_bit_cast(pair, __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = __uint_as_float(p.x) + __uint_as_float(p.y);
+    p = __builtin_bit_cast(pair, __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = __uint_as_float(p.x) + __uint_as_float(p.y);
+#define LQ_ROW_ROR(n) __uint_as_float(unsigned(__builtin_amdgcn_update_dpp(0, int(__float_as_uint(v)), 0x120 + n, 0xf, 0xf, false)))
+    v += LQ_ROW_ROR(8);
+    v += LQ_ROW_ROR(4);
+    v += LQ_ROW_ROR(2);
+    v += LQ_ROW_ROR(1);
+#undef LQ_ROW_ROR
     return v;
 }
 
