@@ -733,7 +733,10 @@ typedef struct {
                               join), 20 (the packed route of a convolution with at most four
                               input channels, filter row of at most 256 bytes, no join) =
                               boxes of 16 x 16 output positions x 64 channels with the
-                              filter in registers and the box's input halo in LDS;
+                              filter in registers and the box's input halo in LDS,
+                              23 / 24 / 25 = 32x32 / 64x32 tiles and tiles of 16 rows
+                              (plain GEMM) with K dealt to the wavefronts of a block
+                              (K % 16 == 0, Cin/groups % 64 == 0);
                               next byte 0 = choose, 1 = one block per tile,
                               2 = stream-K work split, 3 = stream-K over the
                               leftover tiles of the last round only; bits 16..30

@@ -110,6 +110,19 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// floor(n / d) for n < 2^31: one multiplication by ceil(2^(31 + l) / d), 2^(l-1) < d <= 2^l
+struct FastDiv {
+    unsigned d, m;
+    int shift;
+    explicit FastDiv(unsigned div) : d(div), m(0), shift(31) {
+        int l = 0;
+        while ((1ull << l) < div) ++l;
+        shift = 31 + l;
+        m = unsigned(((1ull << shift) + div - 1) / div);
+    }
+    __device__ __forceinline__ unsigned operator()(unsigned n) const { return unsigned((uint64_t(n) * m) >> shift); }
+};
+
 __host__ __device__ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // GELU in its erf form, 0.5 x (1 + erf(x / sqrt 2)) (lucid/nn/functional/activations.py:219), erf by Abramowitz & Stegun

@@ -66,6 +66,9 @@ int launch_tile_c11(const GemmArgs&, int, int, int, hipStream_t);
 int launch_tile_c12(const GemmArgs&, int, int, int, hipStream_t);
 int launch_pp_shape(const GemmArgs&, int, hipStream_t);
 int launch_bw_shape(const GemmArgs&, int, hipStream_t);
+int launch_ks_c1(const GemmArgs&, int conv, int groups, hipStream_t);
+int launch_ks_c2(const GemmArgs&, int conv, int groups, hipStream_t);
+int launch_ks_c3(const GemmArgs&, int conv, int groups, hipStream_t);
 bool conv_halo_applies(const GemmArgs&, int conv, int lbox = 8);
 int launch_conv_halo(const GemmArgs&, int conv, int groups, int lbox, hipStream_t);
 bool conv_few_applies(const GemmArgs&, int conv, int groups);
@@ -73,6 +76,19 @@ int launch_conv_few(const GemmArgs&, int conv, int groups, hipStream_t);
 }  // namespace lq
 
 namespace {
+
+// Whether the K-split tiles can run the problem: a k step of a convolution lies inside one tap.
+bool ks_applies(const GemmArgs& g, int conv) { return g.K > 0 && g.K % 16 == 0 && (!conv || (conv == 1 && g.cCg % 64 == 0)); }
+
+// The K-split tile that gives every tile a CU of its own, or 0: see qgemm_ks.hpp for both sides of the line.  (One stage of
+// 128 k is too little to split: 128 x 4096 x 64 in 64 x 32 tiles 3.9 us, in 64 x 64 ones 3.6.)
+int ks_shape(const GemmArgs& g, int conv, int groups) {
+    if (!ks_applies(g, conv)) return 0;
+    const long tn = (long(g.N) + 31) / 32 * groups;
+    if (!conv && g.M <= 16) return 25;
+    if ((long(g.M) + 31) / 32 * tn <= 256) return 23;
+    return (long(g.M) + 63) / 64 * tn <= 256 && g.K >= 128 ? 24 : 0;
+}
 
 int launch_tile_shape(const GemmArgs& g, int conv, int groups, int cfg, int schedule, hipStream_t st) {
     switch (cfg) {
@@ -115,6 +131,14 @@ int launch_tile_shape(const GemmArgs& g, int conv, int groups, int cfg, int sche
         LQ_REQUIRE(conv, LQ_ERR_VALUE, "tile_config %d is for convolutions", cfg);
         LQ_REQUIRE(schedule <= 1, LQ_ERR_VALUE, "tile_config %d runs one block per tile", cfg);
         return launch_conv_few(g, conv, groups, st);
+    case 23:
+    case 24:
+    case 25:
+        // 32 x 32 and 64 x 32 tiles and tiles of 16 rows, K dealt to the wavefronts of a block
+        LQ_REQUIRE(ks_applies(g, conv), LQ_ERR_VALUE, "tile_config %d is for K %% 16 == 0, convolutions of whole 64-channel steps",
+                   cfg);
+        LQ_REQUIRE(schedule <= 1, LQ_ERR_VALUE, "tile_config %d runs one block per tile", cfg);
+        return (cfg == 23 ? launch_ks_c1 : (cfg == 24 ? launch_ks_c2 : launch_ks_c3))(g, conv, groups, st);
     default: return fail(LQ_ERR_VALUE, "unknown tile_config %d", cfg);
     }
 }
@@ -136,6 +160,7 @@ bool pp_applies(const GemmArgs& g, int conv, int groups) {
 // of the CUs without work.
 int heuristic_tile_shape(const GemmArgs& g, int conv, int groups) {
     const long mt128 = (g.M + 127) / 128;
+    if (const int ks = ks_shape(g, conv, groups)) return ks;
     // an image of at most four channels with a block's worth of 16 x 16 boxes for every CU
     if (g.M >= 65536 && conv_few_applies(g, conv, groups)) return 20;
     // far fewer 128 x 128 tiles than CUs (a small batch in the late stages of a network): 64 x 64
@@ -235,7 +260,7 @@ int tune_import_text(const char* text, int* accepted) {
         }
         if (got != kTuneKeyInts + 1) return fail(LQ_ERR_VALUE, "tune_import: malformed line '%s'", line.c_str());
         const int shape = v[kTuneKeyInts] & 0xff;
-        if (shape < 1 || shape > 22) return fail(LQ_ERR_VALUE, "tune_import: tile shape %d in '%s'", shape, line.c_str());
+        if (shape < 1 || shape > 25) return fail(LQ_ERR_VALUE, "tune_import: tile shape %d in '%s'", shape, line.c_str());
         TuneKey key;
         std::memcpy(&key, v, sizeof(key));
         std::lock_guard<std::mutex> lock(g_tune_mu);
@@ -273,6 +298,10 @@ bool autotune_enabled() {
 }
 
 int tuned_tile_shape(const GemmArgs& g, int conv, int groups, hipStream_t st, int* cfg_out) {
+    if (!conv && g.M <= 16 && ks_applies(g, conv)) {  // a stream of the weight: nothing to choose from
+        *cfg_out = ks_shape(g, conv, groups);
+        return LQ_OK;
+    }
     TuneKey key;
     std::memset(&key, 0, sizeof(key));
     key.M = g.M, key.N = g.N, key.K = g.K, key.mode = g.out_mode, key.conv = conv, key.groups = groups;
@@ -319,6 +348,7 @@ int tuned_tile_shape(const GemmArgs& g, int conv, int groups, hipStream_t st, in
         if (long((g.M + 127) / 128) * ((g.N + 127) / 128) * groups < 256) cands[n++] = 9;
         if (conv_halo_applies(g, conv)) cands[n++] = 15;
     } else {
+        if (const int ks = ks_shape(g, conv, groups)) cands[n++] = ks;
         if (g.N <= 64) cands[n++] = 6;
         cands[n++] = 5;
         if (g.K <= 256) cands[n++] = 8;  // one to four k-iterations: latency-bound tiles, four blocks per CU
@@ -849,13 +879,12 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
     const bool vec_ok = g.K % 16 == 0 && g.K > 0 && aligned16(g.a) && aligned16(g.w);
     int path = force_path;  // 0 = choose, 1 = tile, 2 = skinny, 3 = naive
     if (path == 0) {
-        // The small-batch kernels stream the weight once whatever its alignment.  From 17 rows on 64 x 64 tiles
-        // are faster (us, small batch / tiles: 17 x 11008 x 4096 17.2 / 11.0, 64 rows 33.4 / 11.5; 17 x 4096 x
-        // 4096 11.8 / 9.8; 17 x 1024 x 4096 9.0 / 9.5, 64 rows 15.8 / 9.3), but ragged or unaligned operands
-        // have to be copied to padded rows for them, the whole weight too: that pays from 65 rows (333 x 1001
+        // One row is a stream of the weight; aligned rows go to the K-split tiles of 16 rows from two on (see qgemm_ks.hpp), to
+        // those of 32 and 64 and the tile kernel from 17.  Ragged or unaligned operands have to be copied to padded rows for
+        // them, the whole weight too: that pays from 65 rows (333 x 1001
         // x 1000: 1340 -> 11 us against the plain kernel; 100 x 11008 x 5001: 26.4 ms -> 50 us).  A kept range
-        // needs the tile kernel.  Rows shorter than one chunk stay with the plain kernel.
-        path = g.K < 16 ? 3 : (g.M <= (vec_ok ? 16 : 64) && g.range == nullptr ? 2 : 1);
+        // needs the tile kernels.  Rows shorter than one chunk stay with the plain kernel.
+        path = g.K < 16 ? 3 : (g.M <= (vec_ok ? 1 : 64) && g.range == nullptr ? 2 : 1);
         if (path == 1 && !vec_ok) {
             const int ld = (g.K + 63) / 64 * 64;
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;

@@ -242,19 +242,6 @@ __global__ __launch_bounds__(kThreads) void seg_kernel(Op op, size_t inner4, uns
     }
 }
 
-// floor(n / d) for n < 2^31: one multiplication by ceil(2^(31 + l) / d), 2^(l-1) < d <= 2^l
-struct FastDiv {
-    unsigned d, m;
-    int shift;
-    explicit FastDiv(unsigned div) : d(div), m(0), shift(31) {
-        int l = 0;
-        while ((1ull << l) < div) ++l;
-        shift = 31 + l;
-        m = unsigned(((1ull << shift) + div - 1) / div);
-    }
-    __device__ __forceinline__ unsigned operator()(unsigned n) const { return unsigned((uint64_t(n) * m) >> shift); }
-};
-
 // Segments that no block can have to itself (short, or not whole quads; the channel-last layouts among them): quads
 // of consecutive elements whatever segment they are of, with the channel found per quad and carried from element to
 // element.  CHANNELS: most channels a quad can be of - 2 where a segment is at least 4 elements, 4 below.  As

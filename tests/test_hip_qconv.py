@@ -752,3 +752,31 @@ def test_float_input_form_of_quantized_conv1d_and_conv3d():
                                                          L.tensor(np.float32(128.0), device="hip"))(hip(x))._grid)).numpy()
     assert got.shape == want.shape == (B, Cout, D, H, W)
     assert np.abs(got - want).max() <= S * 1.0001 and np.mean(got != want) < 0.02
+
+
+@pytest.mark.parametrize("cfg", [23, 24])
+@pytest.mark.parametrize("B,H,W,Cin,Cout,k,st,pad,dil,groups", [
+    (1, 7, 7, 512, 70, 3, (1, 1), (1, 1, 1, 1), (1, 1), 1), (2, 5, 9, 64, 33, 3, (2, 1), (0, 1, 2, 0), (1, 2), 1),
+    (1, 9, 8, 384, 62, 3, (1, 2), (1, 0, 1, 1), (2, 1), 2), (3, 6, 5, 192, 31, 2, (1, 1), (0, 0, 0, 0), (1, 1), 1),
+    (1, 33, 1, 128, 64, 1, (1, 1), (0, 0, 0, 0), (1, 1), 1), (1, 3, 3, 256, 130, 5, (1, 1), (2, 2, 2, 2), (1, 1), 1),
+])
+def test_k_split_tiles_gather_convolutions(cfg, B, H, W, Cin, Cout, k, st, pad, dil, groups):
+    """Steps of 64 and 128 channels, groups, strides, taps outside the image, images that end inside a tile: the oracle's sums, and
+    codes after a join those of the tile kernel."""
+    rng = np.random.default_rng(H * W + Cin)
+    Cout *= groups
+    x, w = codes(rng, (B, H, W, Cin)), codes(rng, (Cout, k, k, Cin // groups))
+    kw = dict(a_zp=-17, stride=st, pad=pad, dilation=dil, groups=groups, path=IMPLICIT)
+    exp = O.qconv2d(x, w, -17, 1.0, np.ones(Cout, np.float32), stride=st, pad=pad, dilation=dil, groups=groups, out_mode=O.OUT_ACC_I32)
+    xd, wd = hip(x), hip(w)
+    got = _ops.qconv2d_i8(xd, wd, out_mode=_ops.OUT_ACC_I32, tile_config=cfg, **kw).numpy()
+    assert np.array_equal(got, exp)
+    f = np.float32
+    kw.update(a_scale=hip(f(.02)), w_scale=hip(rng.uniform(1e-3, 2e-3, Cout).astype(f)), wsum=_ops.rowsum_i8(wd),
+              bias=hip(rng.standard_normal(Cout).astype(f)), relu=True, out_mode=_ops.OUT_REQUANT_I8, out_scale=hip(f(.03)),
+              out_zp=hip(f(0.)), out_qmin=0, out_qmax=255, out_offset=-128)
+    join = dict(q=hip(codes(rng, exp.shape)), offset=-128, scale=hip(f(.025)), zp=hip(f(131)), relu=True, out_scale=hip(f(.04)),
+                out_zp=hip(f(0.)), out_qmin=0, out_qmax=255, out_offset=-128)
+    for extra in (dict(), dict(join=join)):
+        a, b = (_ops.qconv2d_i8(xd, wd, tile_config=c, **kw, **extra).numpy() for c in (cfg, 9))
+        assert np.array_equal(a, b)

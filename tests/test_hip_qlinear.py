@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import lucid_amd as L
-from lucid_amd import _ops
+from lucid_amd import _C, _ops
 import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -1009,3 +1009,48 @@ def test_matrix_edges_on_tile_boundaries_take_the_fast_epilogue_and_stay_exact()
                                       out_mode=mode, path=TILE, tile_config=cfg).numpy()
                 exp = O.qlinear(a, w, 0, a_scale, w_scale, bias=bias, out_mode=omode)
                 assert np.array_equal(got.view(dt), exp.view(dt)), (M, N, cfg, mode)
+
+
+@pytest.mark.parametrize("cfg", [23, 24, 25])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 16), (2, 31, 48), (15, 33, 112), (16, 4097, 128), (17, 100, 144), (31, 64, 1008),
+                                   (33, 95, 1040), (65, 32, 4608), (64, 130, 64), (3, 8200, 256), (16, 12300, 144), (5, 16500, 80),
+                                   (50, 161, 5104)])
+def test_k_split_tiles(M, N, K, cfg):
+    """32 x 32 and 64 x 32 tiles and the four widths of 16 rows: fewer stages than wavefronts, stages that no wavefront's ring
+    holds at once, a last stage that K does not fill, rows and columns past the edge, every output form: the accumulators exact and
+    the other forms the bits of the tile kernel."""
+    rng = np.random.default_rng(M + N + K)
+    a, w = codes(rng, (M, K)), codes(rng, (N, K))
+    ad, wd = hip(a), hip(w)
+    got = _ops.qlinear_i8(ad, wd, out_mode=_ops.OUT_ACC_I32, path=TILE, tile_config=cfg).numpy()
+    assert np.array_equal(got, a.astype(np.int64) @ w.astype(np.int64).T)
+    f = np.float32
+    common = dict(a_zp=-7, a_scale=hip(rng.uniform(0.01, 0.02, M).astype(f)), w_scale=hip(rng.uniform(1e-3, 2e-3, N).astype(f)),
+                  wsum=_ops.rowsum_i8(wd), bias=hip(rng.standard_normal(N).astype(f)), path=TILE)
+    grid = dict(out_scale=hip(f(0.03)), out_zp=hip(f(120.0)), out_qmin=0, out_qmax=255, out_offset=-128)
+    join = dict(q=hip(codes(rng, (M, N))), offset=-128, scale=hip(f(.025)), zp=hip(f(131)), relu=True, out_scale=hip(f(.04)),
+                out_zp=hip(f(3.)), out_qmin=0, out_qmax=255, out_offset=-128)
+    res = hip(rng.standard_normal((M, N)).astype(f))
+    forms = [dict(out_mode=_ops.OUT_F32, relu=True), dict(out_mode=_ops.OUT_F32, residual=res), dict(out_mode=_ops.OUT_F16, residual=res),
+             dict(out_mode=_ops.OUT_REQUANT_I8, relu=True, **grid), dict(out_mode=_ops.OUT_REQUANT_I8, join=join, **grid),
+             dict(out_mode=_ops.OUT_FAKEQUANT_F32, **grid), dict(out_mode=_ops.OUT_F32, gelu=True)]
+    for form in forms:
+        got, want = (_ops.qlinear_i8(ad, wd, **common, **form, tile_config=c).numpy() for c in (cfg, 9))
+        assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), form
+    kept = []
+    for c in (cfg, 9):
+        rb = L.Tensor.empty((_C.range_buffer_words(),), L.float32, "hip")
+        s, z, lo, hi = (L.Tensor.empty((), L.float32, "hip") for _ in range(4))
+        _ops.qlinear_i8(ad, wd, **common, out_mode=_ops.OUT_F32, gelu=True, range_buf=rb, tile_config=c)
+        _C.call("lq_calc_qparams_from_range", rb.data_ptr, 0, 0, 255, 0, 1e-8, s.data_ptr, z.data_ptr, lo.data_ptr, hi.data_ptr, None)
+        kept.append([v.numpy().tobytes() for v in (s, z, lo, hi)])
+    assert kept[0] == kept[1]
+
+
+def test_few_rows_and_few_tiles_take_the_k_split_tiles():
+    """What the choice by size alone gives, small problems being below what is timed."""
+    rng = np.random.default_rng(0)
+    for (M, N, K), cfg in {(2, 64, 64): 25, (16, 11008, 256): 25, (17, 8192, 64): 23, (33, 4100, 128): 24, (33, 4100, 112): 9, (17, 8193, 128): 9,
+                           (512, 512, 128): 23, (513, 512, 128): 24, (1024, 513, 128): 9}.items():
+        _ops.qlinear_i8(hip(codes(rng, (M, K))), hip(codes(rng, (N, K))), out_mode=_ops.OUT_ACC_I32)
+        assert _C.load().lq_last_tile_config() & 0xff == cfg, (M, N, K)
