@@ -300,19 +300,29 @@ int launch_gemv1(const float* x, const uint32_t* packed, const float* scales, co
 //
 // Every block needs the x of its k range next to its weights (64 bytes of x per k against
 // rows / 2 or rows bytes of codes), and every block converts it again.  So a block takes
-// many rows (eight wavefronts with one to three 16-row tiles each, wq_tiles_per_wave) and a short k range (512),
+// many rows (one to three 16-row tiles per wavefront, wq_form) and a short k range (512 or 1024),
 // keeps that range's fragments in LDS for all its wavefronts, and requests its first weights
 // when it starts.  The k ranges of a row tile are blocks of their own (grid.y); each
 // writes its partial sums to a slab, and the last one to arrive (an arrival counter per row
 // tile, reset by that block) adds the slabs in index order - the result does not depend on
 // the order of arrival - and stores.  One launch, no workspace besides the slabs.
-constexpr int kWqSliceK = 512;  // k per block
-constexpr int kWqWaves = 8;
-// weight rows of a block whose wavefronts take `rb` tiles of 16 each
-constexpr int wq_rows(int rb) { return kWqWaves * rb * 16; }
-// its LDS: 48 KiB of x fragments, the sums of x per group segment, the tables of its rows
-constexpr size_t wq_lds_bytes(int rb, int gs) {
-    return size_t(kWqSliceK / 32) * 3 * 64 * 16 + (kWqSliceK / 32) * 16 * 4 + size_t(2) * wq_rows(rb) * (kWqSliceK / gs + 1) * 4;
+//
+// Handing slabs on is a third of the time where the weight is a few ten MB (16 x 11008 x 4096 int8, 384 rows x 512 k per block: 4.4 us
+// until the first window, 6.8 us for all of them, 2.3 us for the slab to be written through, 4.1 us for the last block of a row tile
+// to fetch eight).  So a block may also take 1024 k in four parts, four of its sixteen wavefronts for each, and add the parts in
+// LDS: half the slabs, and four wavefronts per SIMD to wait with (20.1 -> 18.4 us; int4 18.9 -> 16.8, 16 x 1033 x 4608 int8
+// 9.8 -> 9.2, 4 x 1024 x 1024 int8 8.3 -> 7.0).  All of K in a block needs no slabs, but every block then fetches and splits all
+// of x: 18.9 us, 18.3, 11.0, 5.3.
+
+// a block of one part is eight wavefronts with all of its k range, one of four sixteen with a quarter each
+constexpr int wq_waves(int parts) { return parts == 4 ? 16 : 8; }
+constexpr int wq_slice(int parts) { return parts == 4 ? 1024 : 512; }  // k
+// weight rows, with `rb` tiles of 16 per wavefront
+constexpr int wq_rows(int rb, int parts) { return wq_waves(parts) / parts * rb * 16; }
+// LDS: 48 or 96 KiB of x fragments, the sums of x per group segment, the tables of the rows
+constexpr size_t wq_lds_bytes(int rb, int parts, int gs) {
+    return size_t(wq_slice(parts) / 32) * 3 * 64 * 16 + (wq_slice(parts) / 32) * 16 * 4 +
+           size_t(2) * wq_rows(rb, parts) * (wq_slice(parts) / gs + 1) * 4;
 }
 
 // Where the A fragment of row m, lane quarter qd of instruction block `blk` sits among the block's
@@ -334,20 +344,22 @@ __device__ __forceinline__ float wq_neighbour_sum(float v) {
     return v;
 }
 
-template <int BITS, int SW, int RB, bool PATTERN>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4 : 2, RB <= 2 ? 4 : 2))) void wq_mfma_kernel(
+template <int BITS, int SW, int RB, int KP, bool PATTERN>
+__global__ __launch_bounds__(64 * wq_waves(KP)) __attribute__((amdgpu_waves_per_eu((RB <= 2 && KP == 1) || KP == 4 ? 4 : 2, (RB <= 2 && KP == 1) || KP == 4 ? 4 : 2))) void wq_mfma_kernel(
     const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N, int K,
     int gs_shift, float* out, float* slabs, int* counters) {
     using G = WqGeom<BITS>;
     constexpr int CODES = G::CODES, WK = G::WK, NI = G::NI;
     constexpr int GW = 1 << SW, SEG = WK / GW;  // group segments per window and their length
     constexpr int IPS = NI / GW;                // instructions per segment
-    constexpr int WAVES = kWqWaves, WPS = kWqSliceK / WK;  // windows per block: 4 or 8
-    constexpr int kWqRows = wq_rows(RB);
+    constexpr int THREADS = 64 * wq_waves(KP), SLICE = wq_slice(KP);
+    constexpr int WAVES = wq_waves(KP) / KP, WPW = SLICE / KP / WK;  // wavefronts of a k range; windows of a wavefront: 4 or 8
+    constexpr int WPS = KP * WPW;                               // windows of the block
+    constexpr int kWqRows = wq_rows(RB, KP);
     constexpr int UNITS = WPS * NI * 64;                    // (window, instruction, lane) triples of the block's x
-    constexpr int AHEAD = RB == 1 ? WPS : 2;                // windows of weights a wavefront has requested and not used
+    constexpr int AHEAD = RB == 1 || WPW < 2 ? WPW : 2;                // windows of weights a wavefront has requested and not used
     static_assert(IPS >= 1, "a segment is at least one instruction");
-    static_assert(UNITS % 512 == 0, "");
+    static_assert(UNITS % THREADS == 0, "");
     // Dynamic LDS: the x fragments of the block's windows ([window][instruction][part][lane],
     // 16 bytes each), then the block's rows of scales and of biases for the groups of those
     // windows - each row padded by one float: lanes of a quarter read 16 different rows at the
@@ -360,16 +372,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     // the k ranges of a row tile are neighbours in the grid: they are dispatched together, so the pieces of a
     // weight row (one per k range) are requested at about the same time
     const int tile = blockIdx.y, ks = blockIdx.x, mb = blockIdx.z, slices = gridDim.x;
-    const int n_base = tile * kWqRows + wave * (RB * 16), m0 = mb * 16;
+    const int wc = wave % WAVES, part = wave / WAVES;  // the wavefront's columns and its part of the k range
+    const int n_base = tile * kWqRows + wc * (RB * 16), m0 = mb * 16;
     const int words_per_row = K * BITS / 32, groups_per_row = K >> gs_shift;
     const int windows = (K + WK - 1) / WK;  // the last one may be partial (K is a multiple of 32: whole 16-byte loads)
     const int w0 = ks * WPS;
     const int nw = windows - w0 < WPS ? windows - w0 : WPS;  // at least 1: the host sizes grid.y so
+    const int w_first = part * WPW, w_end = nw < w_first + WPW ? nw : w_first + WPW;  // the wavefront's (none in a short last range)
     // groups of this block's windows, and the row stride of the tables
     const int g0 = (w0 * WK) >> gs_shift;
     const int k_end = (w0 + nw) * WK < K ? (w0 + nw) * WK : K;
     const int ng = ((k_end - 1) >> gs_shift) - g0 + 1;
-    const int gmax = kWqSliceK >> gs_shift, gp = (gmax < 1 ? 1 : gmax) + 1;
+    const int gmax = SLICE >> gs_shift, gp = (gmax < 1 ? 1 : gmax) + 1;
 
     // Every global load of the block is requested before anything is consumed, in the order of
     // consumption (the wait counter retires loads in order): the scale / bias tables (short, from
@@ -377,7 +391,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     // Tables: wq_rows(RB) rows x gcap slots (gcap = the groups of a full k range, 4, 8 or 16), four slots per
     // 16-byte load where the rows allow it (a dword per lane costs the vector cache as many cycles
     // as 16 bytes per lane do).
-    constexpr int kTabVec = kWqRows * 16 / 4 / 512;  // 16-byte loads per thread and table, at 16 groups per k range
+    constexpr int kTabVec = (kWqRows * (SLICE / 32) + 4 * THREADS - 1) / 4 / THREADS;  // 16-byte loads per thread and table, at 16 groups per k range
     const int gcap = gp - 1, gsh = 31 - __builtin_clz(unsigned(gcap));  // a power of two: shifts, no division
     const bool tab_vec = ng == gcap && (groups_per_row & 3) == 0 && aligned16(scales) && aligned16(biases);
     // (No branch between these requests and none that gives a register another value: the compiler would wait for each load
@@ -391,7 +405,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     if (tab_vec) {
 #pragma unroll
         for (int u = 0; u < kTabVec; ++u) {
-            const int i = (threadIdx.x + u * 512) * 4;
+            const int i = (threadIdx.x + u * THREADS) * 4;
             const size_t at = table_at(i < kWqRows * gcap ? i : 0);
             tab_s[u] = *reinterpret_cast<const float4*>(scales + at);
             tab_b[u] = *reinterpret_cast<const float4*>(biases + at);
@@ -399,12 +413,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     }
     // x of the block's windows: a thread takes eight consecutive k of one row (a wavefront reads
     // 2 KiB of a row)
-    constexpr int OCTS = kWqSliceK / 8;  // per row
+    constexpr int OCTS = SLICE / 8;  // per row
     static_assert(16 * OCTS == UNITS, "");
-    float4 raw[UNITS / 512][2];
+    float4 raw[UNITS / THREADS][2];
 #pragma unroll
-    for (int u = 0; u < UNITS / 512; ++u) {
-        const int unit = u * 512 + threadIdx.x, m = m0 + unit / OCTS, kl = (unit % OCTS) * 8;
+    for (int u = 0; u < UNITS / THREADS; ++u) {
+        const int unit = u * THREADS + threadIdx.x, m = m0 + unit / OCTS, kl = (unit % OCTS) * 8;
         // (K is a multiple of 32; what lies past M and K becomes zero below)
         const float* src = x + size_t(m < M ? m : M - 1) * K + (w0 * WK + kl < k_end ? w0 * WK + kl : 0);
         raw[u][0] = *reinterpret_cast<const float4*>(src);
@@ -431,18 +445,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     };
     uint4 ahead[AHEAD][RB];
 #pragma unroll
-    for (int j = 0; j < AHEAD; ++j) fetch(ahead[j], j);
+    for (int j = 0; j < AHEAD; ++j) fetch(ahead[j], w_first + j);
     // The tables go to LDS, then x, split and laid out as fragments by the block itself: a thread
     // finds the (instruction, quarter) that holds its eight k - the exchange of registers is its
     // own inverse.
     uint4* x_lds = wq_lds;
     float* sum_lds = reinterpret_cast<float*>(wq_lds + WPS * NI * 3 * 64);  // of x: [segment][row]
-    float* s_lds = sum_lds + kWqSliceK / 32 * 16;
+    float* s_lds = sum_lds + SLICE / 32 * 16;
     float* b_lds = s_lds + kWqRows * gp;
     if (tab_vec) {
 #pragma unroll
         for (int u = 0; u < kTabVec; ++u) {
-            const int i = (threadIdx.x + u * 512) * 4, row = i >> gsh, g = i & (gcap - 1);
+            const int i = (threadIdx.x + u * THREADS) * 4, row = i >> gsh, g = i & (gcap - 1);
             if (i < kWqRows * gcap) {
                 float* sd = s_lds + row * gp + g;
                 float* bd = b_lds + row * gp + g;
@@ -451,7 +465,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
             }
         }
     } else {  // the last k range of a K that is not a multiple of 512, or rows that vectors cannot take
-        for (int i = threadIdx.x; i < kWqRows * gcap; i += 512) {
+        for (int i = threadIdx.x; i < kWqRows * gcap; i += THREADS) {
             const int row = i >> gsh, g = i & (gcap - 1);
             // (zeros past the row's groups: a partial window's segments past K read them)
             s_lds[row * gp + g] = g < ng ? scales[table_at(i)] : 0.0f;
@@ -460,8 +474,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     }
     {
 #pragma unroll
-        for (int u = 0; u < UNITS / 512; ++u) {
-            const int unit = u * 512 + threadIdx.x, ml = unit / OCTS, kl = (unit % OCTS) * 8;
+        for (int u = 0; u < UNITS / THREADS; ++u) {
+            const int unit = u * THREADS + threadIdx.x, ml = unit / OCTS, kl = (unit % OCTS) * 8;
             const int wi = kl / WK, off = kl % WK, qs = off / CODES, js = (off % CODES) / (32 / BITS);
             int qd, rho;
             wq_source(SW, js, qs, qd, rho);
@@ -495,7 +509,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     v4f y[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) y[rb] = v4f{0.f, 0.f, 0.f, 0.f};
-    const int row_in_tile = wave * (RB * 16) + r;
+    const int row_in_tile = wc * (RB * 16) + r;
     auto window = [&](int wi, const uint4 (&wv)[RB]) {
         uint32_t wd[RB][4];
 #pragma unroll
@@ -554,12 +568,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
         }
     };
 #pragma unroll 1
-    for (int w = 0; w < nw; w += AHEAD)
+    for (int w = w_first; w < w_end; w += AHEAD)
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
-            if (w + j < nw) window(w + j, ahead[j]);
-            if (AHEAD < WPS) fetch(ahead[j], w + j + AHEAD);
+            if (w + j < w_end) window(w + j, ahead[j]);
+            if (AHEAD < WPW) fetch(ahead[j], w + j + AHEAD);
         }
+    if constexpr (KP > 1) {  // the parts of the range meet where x was
+        v4f* const parts = reinterpret_cast<v4f*>(wq_lds) + lane;
+        lds_barrier();
+        if (part > 0) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) parts[((part - 1) * WAVES + wc) * (RB * 64) + rb * 64] = y[rb];
+        }
+        lds_barrier();
+        if (part == 0) {
+#pragma unroll
+            for (int p = 1; p < KP; ++p)
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) y[rb] = y[rb] + parts[((p - 1) * WAVES + wc) * (RB * 64) + rb * 64];
+        }
+    }
 
     // accumulator element t of a lane: row m = 4 * quarter + t, column n = lane % 16
     auto store_out = [&](const v4f (&v)[RB]) {
@@ -574,7 +603,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
         }
     };
     if (slices == 1) {
-        store_out(y);
+        if (part == 0) store_out(y);
         return;
     }
     // slab of (row tile, k range): [wavefront][tile of 16 rows][lane] x 16 bytes, written through to
@@ -584,8 +613,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     typedef unsigned v4u __attribute__((ext_vector_type(4)));
     const size_t tile_index = size_t(mb) * gridDim.y + tile;
     float* first_slab = slabs + tile_index * slices * (kSlabBytes / 4);
-    const unsigned my_off = unsigned((wave * RB) * 64 + lane) * 16;
-    {
+    const unsigned my_off = unsigned((wc * RB) * 64 + lane) * 16;
+    if (part == 0) {
         const __amdgpu_buffer_rsrc_t mine =
             __builtin_amdgcn_make_buffer_rsrc(first_slab + size_t(ks) * (kSlabBytes / 4), 0, kSlabBytes, 0x00020000);
 #pragma unroll
@@ -598,7 +627,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
     if (threadIdx.x == 0)
         s_arrived = __hip_atomic_fetch_add(&counters[tile_index], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(s_arrived) != slices - 1) return;
+    if (__builtin_amdgcn_readfirstlane(s_arrived) != slices - 1 || part > 0) return;
     v4f total[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) total[rb] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -628,45 +657,51 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RB <= 2 ? 4
 }
 
 
-// Tiles of 16 weight rows per wavefront.  One tile spreads a small weight over the most CUs and leaves room for two blocks on
-// one; three need a CU each, and fetch and split x for the fewest blocks.  us of 1 / 2 / 3 tiles, and of two tiles with all
-// weights requested at once and the sums of x on the matrix unit: 16 x 4096 x 4096 int8 groups of 32 (256 / 128 / 88 blocks)
-// 10.0 / 13.1 / 16.1, 13.9; 16 x 11008 x 4096 int8 of 64 (688 / 344 / 232) 20.6 / 20.1 / 18.8, 22.4; the same int4
-// 19.0 / 19.3 / 19.0, 18.8; 64 x 4096 x 4096 int4 of 64 (1024 / 512 / 352) 21.6 / 18.0 / 27.3, 18.7; 16 x 32000 x 4096 int4
-// of 128 (2000 / 1000 / 672) 38.0 / 37.0 / 46.0, 37.6; 5 x 4096 x 11008 int4 of 32 (704 / 352 / 242) 22.9 / 27.2 / 25.1, 26.9;
-// 3 x 300 x 512 int4 of 64 5.1 / 7.7 / 9.6, 6.8.  The costs below follow those, in us behind the first 3.
-int wq_tiles_per_wave(int M, int N, int slices, int sw) {
-    constexpr double kBlock[4] = {0.0, 4.8, 7.7, 14.5};
-    int best = 1;
-    double least = 1e30;
+// Tiles of 16 weight rows per wavefront and parts of a block's k range.  Four parts of 1024 k (a CU per block) with as many
+// tiles as give every block a CU at once; where the blocks are too many for that, one part of 512 k and two tiles, of which a CU
+// has two blocks, one starting or adding slabs while the other streams.  us of 1 / 2 / 3 tiles of four parts, and of one part of
+// two: 16 x 4096 x 4096 int8 groups of 64 (256 / 128 / 88 blocks) 11.6 / 12.0 / 14.8, 13.6 (128); 16 x 11008 x 4096 int8 of 64
+// (688 / 344 / 232) 26.9 / 24.0 / 18.4, 20.5 (344); the same int4 24.0 / 21.6 / 16.8, 19.4; 64 x 4096 x 4096 int4 of 64
+// (1024 / 512 / 352) 30.4 / 22.4 / 25.9, 19.6 (512); 33 x 2048 x 4096 int4 of 32 (384 / 192 / 132) 16.8 / 12.5 / 15.6,
+// 14.1 (192); 3 x 7450 x 7808 int4 of 64 (936 / 472 / 312) 31.2 / 25.3 / 29.6, 25.0 (480); 20 x 388 x 448 int8 of 32
+// 5.9 / 7.9 / 9.6, 9.7.  The costs below follow those, in us behind the first 3.
+struct WqForm {
+    int tiles, parts;
+};
+WqForm wq_form(int M, int N, int K) {
+    constexpr double kBlock[4] = {0.0, 7.5, 9.3, 12.5};
+    auto blocks = [&](int rb, int kp) {
+        return long((M + 15) / 16) * ((N + wq_rows(rb, kp) - 1) / wq_rows(rb, kp)) * ((K + wq_slice(kp) - 1) / wq_slice(kp));
+    };
+    const long two = blocks(2, 1), rest = two % 512;
+    WqForm best{2, 1};
+    double least = double(two / 512) * 17.0 + (rest == 0 ? 0.0 : rest <= 256 ? 11.0 : 17.0);
     for (int rb = 1; rb <= 3; ++rb) {
-        const long blocks = long((M + 15) / 16) * ((N + wq_rows(rb) - 1) / wq_rows(rb)) * slices;
-        // (four groups per window: three tiles of them are more than a block has registers and LDS for)
-        const double cost = double((blocks + 255) / 256) * (kBlock[rb] + (rb == 3 && sw == 2 ? 4.0 : 0.0)) + (rb < 3 ? 2.0 : 0.5);
-        if (cost < least) least = cost, best = rb;
+        const double cost = double((blocks(rb, 4) + 255) / 256) * kBlock[rb];
+        if (cost < least) least = cost, best = WqForm{rb, 4};
     }
     return best;
 }
 
-template <int BITS, int SW, int RB, bool PATTERN>
+template <int BITS, int SW, int RB, int KP, bool PATTERN>
 int launch_wq_mfma_form(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
                         int K, int gs, float* out, hipStream_t st) {
     using G = WqGeom<BITS>;
-    constexpr int WPS = kWqSliceK / G::WK;
+    constexpr int WPS = wq_slice(KP) / G::WK;
     const int mblocks = (M + 15) / 16, windows = (K + G::WK - 1) / G::WK;
-    const int tiles = (N + wq_rows(RB) - 1) / wq_rows(RB), slices = (windows + WPS - 1) / WPS;
+    const int tiles = (N + wq_rows(RB, KP) - 1) / wq_rows(RB, KP), slices = (windows + WPS - 1) / WPS;
     static DeviceOnce attr_once;
-    if (const int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SW, RB, PATTERN>),
-                                         int(wq_lds_bytes(RB, 32))))
+    if (const int rc = allow_dynamic_lds(attr_once, reinterpret_cast<const void*>(wq_mfma_kernel<BITS, SW, RB, KP, PATTERN>),
+                                         int(wq_lds_bytes(RB, KP, 32))))
         return rc;
     SkScratch sk;
     const auto lock = scratch_lock(st);
     if (slices > 1) {
-        const int rc = sk_scratch(size_t(mblocks) * tiles, size_t(mblocks) * tiles * slices * (kWqWaves * RB * 64 * 16), st, &sk);
+        const int rc = sk_scratch(size_t(mblocks) * tiles, size_t(mblocks) * tiles * slices * (wq_waves(KP) / KP * RB * 64 * 16), st, &sk);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL((wq_mfma_kernel<BITS, SW, RB, PATTERN>), dim3(unsigned(slices), unsigned(tiles), unsigned(mblocks)), dim3(512),
-                       wq_lds_bytes(RB, gs), st, x, packed, scales, biases, M, N, K, 31 - __builtin_clz(unsigned(gs)), out,
+    hipLaunchKernelGGL((wq_mfma_kernel<BITS, SW, RB, KP, PATTERN>), dim3(unsigned(slices), unsigned(tiles), unsigned(mblocks)), dim3(64 * wq_waves(KP)),
+                       wq_lds_bytes(RB, KP, gs), st, x, packed, scales, biases, M, N, K, 31 - __builtin_clz(unsigned(gs)), out,
                        reinterpret_cast<float*>(sk.slabs), sk.counters);
     LQ_CHECK_LAUNCH("wq_mfma");
     return LQ_OK;
@@ -675,13 +710,14 @@ int launch_wq_mfma_form(const float* x, const uint32_t* packed, const float* sca
 template <int BITS>
 int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
                    int K, int gs, float* out, hipStream_t st) {
-    const int sw = wq_swap_mode(BITS, gs), rb = wq_tiles_per_wave(M, N, (K + kWqSliceK - 1) / kWqSliceK, sw);
+    const int sw = wq_swap_mode(BITS, gs);
+    const WqForm form = wq_form(M, N, K);
     const bool pattern = BITS == 4 && M > 1 && M <= 64 && K % WqGeom<BITS>::WK == 0;
-#define LQ_WQ_FORM(SWM, RBS)                                                                                       \
-    if (sw == SWM && rb == RBS)                                                                                    \
-        return pattern ? launch_wq_mfma_form<BITS, SWM, RBS, BITS == 4>(x, packed, scales, biases, M, N, K, gs, out, st) \
-                       : launch_wq_mfma_form<BITS, SWM, RBS, false>(x, packed, scales, biases, M, N, K, gs, out, st)
-#define LQ_WQ_FORMS(SWM) LQ_WQ_FORM(SWM, 1); LQ_WQ_FORM(SWM, 2); LQ_WQ_FORM(SWM, 3)
+#define LQ_WQ_FORM(SWM, RBS, KPS)                                                                                            \
+    if (sw == SWM && form.tiles == RBS && form.parts == KPS)                                                                 \
+        return pattern ? launch_wq_mfma_form<BITS, SWM, RBS, KPS, BITS == 4>(x, packed, scales, biases, M, N, K, gs, out, st) \
+                       : launch_wq_mfma_form<BITS, SWM, RBS, KPS, false>(x, packed, scales, biases, M, N, K, gs, out, st)
+#define LQ_WQ_FORMS(SWM) LQ_WQ_FORM(SWM, 2, 1); LQ_WQ_FORM(SWM, 1, 4); LQ_WQ_FORM(SWM, 2, 4); LQ_WQ_FORM(SWM, 3, 4)
     LQ_WQ_FORMS(0);
     LQ_WQ_FORMS(1);
     if constexpr (BITS == 4) {

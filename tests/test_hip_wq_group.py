@@ -96,6 +96,15 @@ def test_small_batch_forms_are_exact_on_exact_inputs(M, N, K, gs, bits):
     assert np.array_equal(y.astype(np.float64), x.astype(np.float64) @ W.dequantize(packed, s, b, gs, bits).astype(np.float64).T)
 
 
+# blocks of 1024 k in four parts, with one, two and three tiles per wavefront, every exchange of registers: a last range that ends
+# inside its first, second and last part, a range alone, rows that end inside a wavefront's tiles
+@pytest.mark.parametrize("M,N,K,gs,bits", [
+    (9, 191, 1312, 32, 8), (3, 8191, 2304, 32, 4), (5, 8190, 2816, 128, 8), (16, 11007, 3328, 32, 4), (12, 12288, 3136, 64, 8),
+    (16, 10999, 3136, 64, 4), (2, 65, 224, 32, 4), (16, 63, 1024, 128, 4), (4, 1, 96, 32, 8)])
+def test_ranges_in_four_parts_are_exact_on_exact_inputs(M, N, K, gs, bits):
+    test_small_batch_forms_are_exact_on_exact_inputs(M, N, K, gs, bits)
+
+
 @pytest.mark.parametrize("M,N,K,gs,bits", SMALL_BATCH_FORMS)
 def test_small_batch_forms_against_float64(M, N, K, gs, bits):
     rng = np.random.default_rng(N)
