@@ -252,6 +252,24 @@ def test_minmax_matches_oracle(shape, ch_axis):
     assert np.array_equal(mx.numpy().reshape(-1), emx)
 
 
+# Channels in many runs: one channel (a single run whatever its shape), runs shared out among the blocks of a channel (even and
+# uneven shares, the last one empty, runs of 64 and of more than a block reads at once), runs that are also split lengthwise.
+@pytest.mark.parametrize("shape,ch_axis", [
+    ((70001, 1), 1), ((5, 1, 7), 1), ((8192, 3, 64), 1), ((1000, 2, 65), 1), ((4099, 1, 3), 1), ((129, 5, 515), 1),
+    ((67, 17, 3136), 1), ((3, 2, 9000), 1), ((33, 1000, 128), 1), ((5, 2047, 4097), 1),
+])
+def test_minmax_of_channels_in_many_runs(shape, ch_axis):
+    rng = np.random.default_rng(shape[0])
+    x = rng.standard_normal(shape).astype(np.float32)
+    for at in (0, -1):  # the extreme at either end of the tensor, then a NaN there
+        for v in (99.0, -99.0, np.nan):
+            y = x.copy()
+            y.reshape(-1)[at] = v
+            mn, mx = Q.minmax(hip(y), ch_axis=ch_axis)
+            emn, emx = O.minmax(y, ch_axis=ch_axis)
+            assert same_f32(mn.numpy().reshape(-1), emn) and same_f32(mx.numpy().reshape(-1), emx)
+
+
 def test_minmax_propagates_nan():
     x = np.arange(3 * 5000, dtype=np.float32).reshape(3, 5000)
     x[1, 4321] = np.nan
