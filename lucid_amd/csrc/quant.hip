@@ -120,6 +120,7 @@ struct QuantizeOp {
     int off;
     __device__ __forceinline__ In load(size_t i) const { return nt_load(&x[i]); }
     static constexpr int kMaxU = 2;  // loads in flight per lane; measured best for 4 B in / 1 B out
+    static constexpr bool kDivides = true;
     __device__ __forceinline__ Vec pack(In v, float4 s, float4 z, float4 r) const {
         const float4 n = rint_div4(v, s, r);
         Vec o;
@@ -151,6 +152,7 @@ struct DequantizeOp {
     using Vec = typename CodeVec<CodeT>::type;
     using In = Vec;
     static constexpr int kMaxU = 8;
+    static constexpr bool kDivides = false;
     const Vec* __restrict__ q;
     float4* __restrict__ out;
     int off;
@@ -173,6 +175,7 @@ struct DequantizeOp {
 struct FakeQuantizeOp {
     using In = float4;
     static constexpr int kMaxU = 4;
+    static constexpr bool kDivides = true;
     const float4* __restrict__ x;
     float4* __restrict__ out;
     float lo, hi;
@@ -243,25 +246,30 @@ __global__ __launch_bounds__(kThreads) void seg_kernel(Op op, size_t inner4, uns
 }
 
 // Segments that no block can have to itself (short, or not whole quads; the channel-last layouts among them): quads
-// of consecutive elements whatever segment they are of, with the channel found per quad and carried from element to
-// element.  CHANNELS: most channels a quad can be of - 2 where a segment is at least 4 elements, 4 below.  As
-// elements on generic_kernel, a lane did a 64-bit division and an IEEE division for each 4 bytes it moved.
-// (The address arithmetic still is what bounds it with 4 channels, memory with 2.)
-template <typename Op, int U, int CHANNELS>
-__global__ __launch_bounds__(kThreads) void flat_kernel(Op op, unsigned n, FastDiv inner, FastDiv C, QParams qp) {
-    const unsigned n4 = n / 4, i0 = blockIdx.x * unsigned(U * kThreads) + threadIdx.x;
+// of consecutive elements whatever segment they are of.  CHANNELS: most channels a quad can be of - 2 where a segment is
+// at least 4 elements, 4 below.
+// SHARED: a thread's quads are `stride` apart, a whole number of rounds of the channels, so that they are all of the same
+// channels at the same places: those, their qparams and reciprocals are found once per U quads.  Groups of `stride`
+// threads take U * stride quads.  Otherwise they are found per quad.
+// (Quantize / dequantize / fake-quantize, us, per quad and shared by four: 5000 x 3000 x 7 along the last axis 166 / 181 / 191 and
+// 93 / 105 / 142, 8192 x 8192 along the last 127 / 135 / 149 and 52 / 72 / 84, where memory takes 52 / 56 / 84 with a channel per row;
+// 4096 x 512 x 8 along the last 25.7 / 29.4 / 32.9 and 15.0 / 16.3 / 22.5, along the middle 18.1 / - / 25.0 and 15.9 / - / 22.6.
+// Two quads per thread: 115 / 125 / 148 for the first; eight: 89 / 108 / 156.)
+template <typename Op, int U, int CHANNELS, bool SHARED>
+__global__ __launch_bounds__(kThreads) void flat_kernel(Op op, unsigned n, FastDiv stride, FastDiv inner, FastDiv C,
+                                                        QParams qp) {
+    const unsigned n4 = n / 4, t = blockIdx.x * unsigned(kThreads) + threadIdx.x;
+    const unsigned step = SHARED ? stride.d : unsigned(kThreads);
+    const unsigned i0 = SHARED ? t + stride(t) * (U - 1) * stride.d : blockIdx.x * unsigned(U * kThreads) + threadIdx.x;
     typename Op::In v[U];
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-        const unsigned i = i0 + j * kThreads;
+        const unsigned i = i0 + j * step;
         v[j] = op.load(i < n4 ? i : n4 - 1);
     }
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-        const unsigned i = i0 + j * kThreads;
-        if (i >= n4) break;
+    float s[4], z[4], r[4];
+    auto find = [&](unsigned i) {
         unsigned seg = inner(i * 4), at = i * 4 - seg * inner.d, c = seg - C(seg) * C.d;
-        float s[4], z[4], r[4];
         if constexpr (CHANNELS == 2) {
             const unsigned next = c + 1 == C.d ? 0 : c + 1, left = inner.d - at;
             const float s0 = qp.scale[c], z0 = qp.zp[c], s1 = qp.scale[next], z1 = qp.zp[next];
@@ -279,6 +287,13 @@ __global__ __launch_bounds__(kThreads) void flat_kernel(Op op, unsigned n, FastD
 #pragma unroll
             for (int e = 0; e < 4; ++e) r[e] = 1.0f / s[e];
         }
+    };
+    if (SHARED && i0 < n4) find(i0);
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const unsigned i = i0 + j * step;
+        if (i >= n4) break;
+        if (!SHARED) find(i);
         op.store(i, v[j], float4{s[0], s[1], s[2], s[3]}, float4{z[0], z[1], z[2], z[3]}, float4{r[0], r[1], r[2], r[3]});
     }
     if (blockIdx.x == 0 && threadIdx.x < n % 4) {
@@ -333,13 +348,30 @@ int launch_elementwise(Op op, size_t outer, size_t C, size_t inner, QParams qp, 
         default: hipLaunchKernelGGL((seg_kernel<Op, 1>), grid, block, 0, st, op, inner4, unsigned(tail), unsigned(chunks), C, qp); break;
         }
     } else if (vec_ok && n >= 4 && n < (size_t(1) << 31) && qp.scale) {
-        constexpr int U = Op::kMaxU < 4 ? Op::kMaxU : 4;
-        const unsigned blocks = unsigned((n / 4 + U * kThreads - 1) / (U * kThreads));
+        // `round`: quads after which the channels come round again.  A stride of whole rounds that is not much more than
+        // a block keeps a thread's quads near each other; where that would be fewer than 16 groups of threads, one group.
+        const size_t quads = n / 4, cols = C * inner, round = cols % 4 == 0 ? cols / 4 : (cols % 2 == 0 ? cols / 2 : cols);
         const FastDiv by_inner{unsigned(inner)}, by_c{unsigned(C)};
-        if (inner >= 4)
-            hipLaunchKernelGGL((flat_kernel<Op, U, 2>), dim3(blocks), dim3(kThreads), 0, st, op, unsigned(n), by_inner, by_c, qp);
-        else
-            hipLaunchKernelGGL((flat_kernel<Op, U, 4>), dim3(blocks), dim3(kThreads), 0, st, op, unsigned(n), by_inner, by_c, qp);
+        auto launch = [&](auto kernel, size_t threads, size_t stride) {
+            hipLaunchKernelGGL(kernel, dim3(unsigned((threads + kThreads - 1) / kThreads)), dim3(kThreads), 0, st, op,
+                               unsigned(n), FastDiv{unsigned(stride)}, by_inner, by_c, qp);
+        };
+        // Found per quad: channels that come round less than twice, and what has two channels to find and nothing to divide by
+        // (dequantize of 5000 x 3000 x 7 along the middle axis: 92.6 us, shared 96.1).
+        if (quads >= 2 * round && (inner < 4 || Op::kDivides)) {
+            constexpr int U = 4;
+            size_t stride = (kThreads + round - 1) / round * round;
+            if (quads < 16 * U * stride) stride = (quads + U * round - 1) / (U * round) * round;
+            const size_t threads = (quads + U * stride - 1) / (U * stride) * stride;
+            if (inner < 4)
+                launch(flat_kernel<Op, U, 4, true>, threads, stride);
+            else if constexpr (Op::kDivides)
+                launch(flat_kernel<Op, U, 2, true>, threads, stride);
+        } else {
+            constexpr int U = Op::kMaxU < 4 ? Op::kMaxU : 4;
+            const size_t threads = (quads + U - 1) / U;
+            inner >= 4 ? launch(flat_kernel<Op, U, 2, false>, threads, 1) : launch(flat_kernel<Op, U, 4, false>, threads, 1);
+        }
     } else {
         size_t blocks = (n + kThreads - 1) / kThreads;
         if (blocks > 262144) blocks = 262144;

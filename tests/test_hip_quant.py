@@ -312,6 +312,29 @@ def test_ragged_segments_bit_exact(shape, ch_axis):
                           bits(O.fake_quantize(x, s, z, qd.quant_min, qd.quant_max, ch_axis=ch_axis)))
 
 
+# Channels that come round often: a thread's quads a block or more apart, in many groups (the last one partial), in one group, with as
+# many rounds as a thread has quads, and with fewer than two.
+@pytest.mark.parametrize("shape", [
+    (40001, 3), (20003, 2, 3), (66000, 1, 2), (2001, 3, 13), (7001, 1, 1), (9000, 7), (5, 1031), (4, 515, 3), (3, 700, 2), (7, 100, 9),
+    (1, 4001), (1, 300, 7), (2, 33, 5), (70000, 4), (1201, 2, 67),
+])
+@pytest.mark.parametrize("qd", ["qint8", "quint8"])
+def test_channels_that_come_round_bit_exact(shape, qd):
+    rng = np.random.default_rng(sum(shape))
+    qdtype = getattr(Q, qd)
+    s, z = _params(rng, shape, 1, qd == "quint8")
+    if qd == "qint8":
+        z = np.zeros_like(z)
+    x = _adversarial(rng, shape, s[0])
+    st, zt = hip(s), hip(z)
+    q = Q.quantize(hip(x), st, zt, qdtype, ch_axis=1)
+    eq = O.quantize(x, s, z, qdtype.quant_min, qdtype.quant_max, ch_axis=1, q_dtype=O.I16 if qd == "quint8" else O.I8)
+    assert np.array_equal(q.numpy(), eq)
+    assert np.array_equal(bits(Q.dequantize(q, st, zt, ch_axis=1).numpy()), bits(O.dequantize(eq, s, z, ch_axis=1)))
+    assert np.array_equal(bits(Q.fake_quantize(hip(x), st, zt, qdtype.quant_min, qdtype.quant_max, ch_axis=1).numpy()),
+                          bits(O.fake_quantize(x, s, z, qdtype.quant_min, qdtype.quant_max, ch_axis=1)))
+
+
 # ------------------------------------------------------------------ full-size properties
 def test_round_trip_properties_at_benchmark_size():
     """4096 x 4096 x 16 float32, per-channel symmetric along dim 0, then
