@@ -516,10 +516,14 @@ int lq_dynamic_mlp2_small_rows_f32(const float* x, int M, int K1, const int8_t* 
  * per-token activation quantization in front of an LLM-shaped Linear.  scale,
  * zp: [rows] out; mn_out, mx_out: optional [rows] out.  cols must be a multiple
  * of 4, at most 16384, x 16-byte aligned (LQ_ERR_NOT_IMPLEMENTED otherwise: use
- * the three calls). */
+ * the call below or the three calls). */
 int lq_quantize_rows_dynamic_i8(const float* x, size_t rows, size_t cols, int symmetric, int qmin, int qmax,
                                 int is_signed, float eps, int code_offset, float* scale, float* zp,
                                 float* mn_out, float* mx_out, int8_t* q, lq_stream stream);
+/* The same for rows of 1 to 16384 floats at any address, their codes one row after the other. */
+int lq_quantize_rows_dynamic_ragged_i8(const float* x, size_t rows, size_t cols, int symmetric, int qmin, int qmax,
+                                       int is_signed, float eps, int code_offset, float* scale, float* zp,
+                                       float* mn_out, float* mx_out, int8_t* q, lq_stream stream);
 
 /* nnqd.Linear takes x.min() / x.max() of its input on every forward
  * (lucid/nn/quantized/dynamic/linear.py:87-89): a full pass over a tensor some

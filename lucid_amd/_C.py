@@ -118,6 +118,7 @@ _SIGNATURES = {
     "lq_quantize_tensor_dynamic_i8": [_vp, _sz, _i, _i, _i, _i, C.c_float, _i, _vp, _vp, _vp, _vp, _vp, _vp],
     "lq_quantize_tensor_dynamic_polls_i8": [_vp, _sz, C.c_uint, C.c_uint, _i, _i, _i, _i, C.c_float, _i, _vp, _vp, _vp, _vp, _vp,
                                             _i, _vp],
+    "lq_quantize_rows_dynamic_ragged_i8": [_vp, _sz, _sz, _i, _i, _i, _i, C.c_float, _i, _vp, _vp, _vp, _vp, _vp, _vp],
     "lq_quantize_rows_dynamic_i8": [_vp, _sz, _sz, _i, _i, _i, _i, C.c_float, _i, _vp, _vp, _vp, _vp, _vp, _vp],
     "lq_dynamic_linear_small_f32": [_vp, _i, _i, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, C.c_float, _i, _vp, _vp],
     "lq_dynamic_linear_small_rows_f32": [_vp, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, C.c_float, _i, _vp, _vp],

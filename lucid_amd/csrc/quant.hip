@@ -5,6 +5,7 @@
 // (lucid/quantization/_functional.py:180, 281, 311-313): IEEE division,
 // round-half-even, add zero point, clamp, cast.  No reciprocal, no FMA.
 #include <mutex>
+#include <type_traits>
 #include "common.hpp"
 #include "qgemm.hpp"
 #include "range_slots.hpp"
@@ -655,26 +656,72 @@ __global__ __launch_bounds__(1024) void quantize_range_kernel(QuantizeOp<int8_t>
         if (at + u * 1024 < quads) op.store(at + u * 1024, v[u], splat(s), splat(z), splat(r));
 }
 
+// Elements e .. e+3 of x[0 .. n), zeros past n.  One unconditional 16-byte load (any float address) from where all
+// four exist: a load under a condition would be waited for before the next one is issued.
+__device__ __forceinline__ float4 load_quad(const float* x, size_t e, size_t n) {
+    float4 v{0.f, 0.f, 0.f, 0.f};
+    if (n < 4) {  // uniform
+        if (e < n) v.x = x[e];
+        if (e + 1 < n) v.y = x[e + 1];
+        if (e + 2 < n) v.z = x[e + 2];
+        return v;
+    }
+    const size_t at = e < n - 4 ? e : n - 4;
+    __builtin_memcpy(&v, x + at, 16);
+    return v;
+}
+// ... and, once it has arrived, the elements in place
+__device__ __forceinline__ float4 place_quad(float4 v, size_t e, size_t n) {
+    if (n < 4 || e + 4 <= n) return v;
+    const size_t d = e - (n - 4);
+    return d == 1 ? float4{v.y, v.z, v.w, 0.f}
+                  : (d == 2 ? float4{v.z, v.w, 0.f, 0.f} : (d == 3 ? float4{v.w, 0.f, 0.f, 0.f} : float4{0.f, 0.f, 0.f, 0.f}));
+}
+__device__ __forceinline__ void mm_update_quad(MinMax& m, float4 v, size_t e, size_t n) {
+    if (e + 4 <= n) {
+        mm_update(m, v.x), mm_update(m, v.y), mm_update(m, v.z), mm_update(m, v.w);
+    } else {
+        if (e < n) mm_update(m, v.x);
+        if (e + 1 < n) mm_update(m, v.y);
+        if (e + 2 < n) mm_update(m, v.z);
+    }
+}
+
 // Dynamic per-row quantization in one pass over x: a block holds one row in registers, takes
 // its min / max (observer.py:634-653 with ch_axis = 0), turns them into the row's qparams
 // (qparams_of) and writes the row's codes with QuantizeOp's arithmetic - the three separate
 // launches' results, bit for bit, with x read once instead of twice.
-template <int R>  // float4 per lane: rows of up to 1024 * R floats
+// RAGGED: rows of any length at any float address, their codes at any byte address.  (1500 rows of 3333 in the four launches of the
+// three calls 24.4 us, 2 of 7386 24.6; in one 10.2 and 10.6, of which the host takes most.)
+template <int R, bool RAGGED>  // quads per lane: rows of up to 1024 * R floats
 __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
-    const float4* __restrict__ x, int quads, int symmetric, int qmin, int qmax, int is_signed, float eps,
+    const float* __restrict__ x, int cols, int symmetric, int qmin, int qmax, int is_signed, float eps,
     float half_range, int off, float* __restrict__ scale, float* __restrict__ zp, float* __restrict__ mn_out,
-    float* __restrict__ mx_out, Code8x4* __restrict__ q) {
+    float* __restrict__ mx_out, int8_t* __restrict__ q) {
     __shared__ float s_sz[2];
     const size_t row = blockIdx.x;
-    const float4* xr = x + row * size_t(quads);
+    const float* xr = x + row * size_t(cols);
     float4 v[R];
     MinMax m{__builtin_inff(), -__builtin_inff(), 0};
+    if constexpr (RAGGED) {
 #pragma unroll
-    for (int u = 0; u < R; ++u) {
-        const int i = u * 256 + int(threadIdx.x);
-        if (i < quads) {
-            v[u] = nt_load(&xr[i]);
-            mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
+        for (int u = 0; u < R; ++u) {
+            const int e = (u * 256 + int(threadIdx.x)) * 4;
+            if (e < cols) v[u] = load_quad(xr, e, cols);
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int e = (u * 256 + int(threadIdx.x)) * 4;
+            if (e < cols) v[u] = place_quad(v[u], e, cols), mm_update_quad(m, v[u], e, cols);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int i = u * 256 + int(threadIdx.x);
+            if (i * 4 < cols) {
+                v[u] = nt_load(&reinterpret_cast<const float4*>(xr)[i]);
+                mm_update(m, v[u].x), mm_update(m, v[u].y), mm_update(m, v[u].z), mm_update(m, v[u].w);
+            }
         }
     }
     m = mm_block_reduce(m);
@@ -692,11 +739,21 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
     __syncthreads();
     const float s = s_sz[0], z = s_sz[1], r = 1.0f / s;
     const QuantizeOp<int8_t> op{nullptr, nullptr, float(double(qmin)), float(double(qmax)), off};
-    Code8x4* qr = q + row * size_t(quads);
+    int8_t* qr = q + row * size_t(cols);
 #pragma unroll
     for (int u = 0; u < R; ++u) {
-        const int i = u * 256 + int(threadIdx.x);
-        if (i < quads) qr[i] = op.pack(v[u], s, z, r);
+        const int e = (u * 256 + int(threadIdx.x)) * 4;
+        if (e >= cols) break;
+        const Code8x4 c = op.pack(v[u], s, z, r);
+        if (!RAGGED) {
+            *reinterpret_cast<Code8x4*>(qr + e) = c;
+        } else if (e + 4 <= cols) {
+            __builtin_memcpy(qr + e, &c, 4);
+        } else {  // (named one by one: an index would put the codes into LDS, at a place found in the dispatch packet)
+            qr[e] = c.v[0];
+            if (e + 1 < cols) qr[e + 1] = c.v[1];
+            if (e + 2 < cols) qr[e + 2] = c.v[2];
+        }
     }
 }
 
@@ -729,37 +786,6 @@ struct DynScratch {
     unsigned long long slot[kExchange];    // low word: the block's minimum, high word: its maximum
     unsigned left;                        // blocks that have read the slots
 };
-
-// Elements e .. e+3 of x[0 .. n), zeros past n.  One unconditional 16-byte load (any float address) from where all
-// four exist: a load under a condition would be waited for before the next one is issued.
-__device__ __forceinline__ float4 load_quad(const float* x, size_t e, size_t n) {
-    float4 v{0.f, 0.f, 0.f, 0.f};
-    if (n < 4) {  // uniform
-        if (e < n) v.x = x[e];
-        if (e + 1 < n) v.y = x[e + 1];
-        if (e + 2 < n) v.z = x[e + 2];
-        return v;
-    }
-    const size_t at = e < n - 4 ? e : n - 4;
-    __builtin_memcpy(&v, x + at, 16);
-    return v;
-}
-// ... and, once it has arrived, the elements in place
-__device__ __forceinline__ float4 place_quad(float4 v, size_t e, size_t n) {
-    if (n < 4 || e + 4 <= n) return v;
-    const size_t d = e - (n - 4);
-    return d == 1 ? float4{v.y, v.z, v.w, 0.f}
-                  : (d == 2 ? float4{v.z, v.w, 0.f, 0.f} : (d == 3 ? float4{v.w, 0.f, 0.f, 0.f} : float4{0.f, 0.f, 0.f, 0.f}));
-}
-__device__ __forceinline__ void mm_update_quad(MinMax& m, float4 v, size_t e, size_t n) {
-    if (e + 4 <= n) {
-        mm_update(m, v.x), mm_update(m, v.y), mm_update(m, v.z), mm_update(m, v.w);
-    } else {
-        if (e < n) mm_update(m, v.x);
-        if (e + 1 < n) mm_update(m, v.y);
-        if (e + 2 < n) mm_update(m, v.z);
-    }
-}
 
 // RAGGED: rows of `cols` elements to rows of `ld` codes (a multiple of 4); the quads are those of the codes, so
 // that every store is one aligned word.  Otherwise one run of n elements.
@@ -1505,6 +1531,36 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
     return LQ_OK;
 }
 
+int quantize_rows(const float* x, size_t rows, size_t cols, bool ragged, int symmetric, int qmin, int qmax, int is_signed,
+                  float eps, int off, float* scale, float* zp, float* mn, float* mx, int8_t* q, hipStream_t st) {
+    if (rows == 0) return LQ_OK;
+    LQ_REQUIRE(x && q && scale && zp, LQ_ERR_VALUE, "quantize_rows_dynamic: NULL pointer");
+    LQ_REQUIRE(qmax > qmin && qmin + off >= -128 && qmax + off <= 127, LQ_ERR_VALUE,
+               "quantize_rows_dynamic: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, off);
+    LQ_REQUIRE(ragged || (cols >= 4 && cols % 4 == 0 && cols <= 16384 && aligned16(x) &&
+                          (reinterpret_cast<uintptr_t>(q) & 3u) == 0),
+               LQ_ERR_NOT_IMPLEMENTED,
+               "quantize_rows_dynamic: rows of %zu floats (a multiple of 4, at most 16384, 16-byte aligned) are what this call "
+               "takes; use lq_quantize_rows_dynamic_ragged_i8, or lq_minmax + lq_calc_qparams + lq_quantize", cols);
+    LQ_REQUIRE(cols >= 1 && cols <= 16384 && rows <= 0x7fffffffull, LQ_ERR_NOT_IMPLEMENTED,
+               "quantize_rows_dynamic: %zu rows of %zu floats (1 to 16384); use lq_minmax + lq_calc_qparams + lq_quantize", rows, cols);
+    const float half_range = float((double(qmax) - double(qmin)) / 2.0);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(rows)), dim3(256), 0, st, x, int(cols), symmetric, qmin, qmax, is_signed, eps,
+                           half_range, off, scale, zp, mn, mx, q);
+    };
+    auto of_length = [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        ragged ? launch(quantize_rows_dynamic_kernel<R, true>) : launch(quantize_rows_dynamic_kernel<R, false>);
+    };
+    if (cols <= 1024) of_length(std::integral_constant<int, 1>{});
+    else if (cols <= 4096) of_length(std::integral_constant<int, 4>{});
+    else if (cols <= 8192) of_length(std::integral_constant<int, 8>{});
+    else of_length(std::integral_constant<int, 16>{});
+    LQ_CHECK_LAUNCH("quantize_rows_dynamic");
+    return LQ_OK;
+}
+
 }  // namespace
 
 namespace lq {
@@ -1682,31 +1738,15 @@ int lq_dynamic_linear_small_rows_f32(const float* x, int M, int K, const int8_t*
 int lq_quantize_rows_dynamic_i8(const float* x, size_t rows, size_t cols, int symmetric, int qmin, int qmax,
                                 int is_signed, float eps, int code_offset, float* scale, float* zp,
                                 float* mn_out, float* mx_out, int8_t* q, lq_stream stream) {
-    if (rows == 0) return LQ_OK;
-    LQ_REQUIRE(x && q && scale && zp, LQ_ERR_VALUE, "quantize_rows_dynamic: NULL pointer");
-    LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
-               "quantize_rows_dynamic: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
-    LQ_REQUIRE(cols >= 4 && cols % 4 == 0 && cols <= 16384 && aligned16(x) &&
-                   (reinterpret_cast<uintptr_t>(q) & 3u) == 0 && rows <= 0x7fffffffull,
-               LQ_ERR_NOT_IMPLEMENTED,
-               "quantize_rows_dynamic: rows of %zu floats (a multiple of 4, at most 16384, 16-byte aligned) "
-               "are what the one-pass kernel takes; use lq_minmax + lq_calc_qparams + lq_quantize", cols);
-    const float half_range = float((double(qmax) - double(qmin)) / 2.0);
-    const int quads = int(cols / 4);
-    hipStream_t st = as_stream(stream);
-    const float4* x4 = reinterpret_cast<const float4*>(x);
-    Code8x4* q4 = reinterpret_cast<Code8x4*>(q);
-#define LQ_ROWS_DYN(R)                                                                                      \
-    hipLaunchKernelGGL(quantize_rows_dynamic_kernel<R>, dim3(unsigned(rows)), dim3(256), 0, st, x4, quads,  \
-                       symmetric, qmin, qmax, is_signed, eps, half_range, code_offset, scale, zp, mn_out,   \
-                       mx_out, q4)
-    if (quads <= 256) LQ_ROWS_DYN(1);
-    else if (quads <= 1024) LQ_ROWS_DYN(4);
-    else if (quads <= 2048) LQ_ROWS_DYN(8);
-    else LQ_ROWS_DYN(16);
-#undef LQ_ROWS_DYN
-    LQ_CHECK_LAUNCH("quantize_rows_dynamic");
-    return LQ_OK;
+    return quantize_rows(x, rows, cols, false, symmetric, qmin, qmax, is_signed, eps, code_offset, scale, zp, mn_out, mx_out, q,
+                         as_stream(stream));
+}
+
+int lq_quantize_rows_dynamic_ragged_i8(const float* x, size_t rows, size_t cols, int symmetric, int qmin, int qmax,
+                                       int is_signed, float eps, int code_offset, float* scale, float* zp,
+                                       float* mn_out, float* mx_out, int8_t* q, lq_stream stream) {
+    return quantize_rows(x, rows, cols, true, symmetric, qmin, qmax, is_signed, eps, code_offset, scale, zp, mn_out, mx_out, q,
+                         as_stream(stream));
 }
 
 int lq_minmax(const float* x, size_t outer, size_t C, size_t inner, float* mn, float* mx,

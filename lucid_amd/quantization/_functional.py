@@ -139,20 +139,21 @@ def quantize_rows_dynamic(x: Tensor, qscheme, qdtype: QDtype, eps: float = 1e-8
         codes = quantize(x, scale, zero_point, qdtype, ch_axis=0)
 
     (``observer.py:634-653``, ``_qparams.py:198-215``, ``_functional.py:164-182``) with ``x``
-    read once.  Rows the one-pass kernel does not take (longer than 16384, not a multiple
-    of 4, int16 storage) go through those three calls."""
+    read once.  Rows the one-pass kernel does not take (longer than 16384, empty ones, int16
+    storage) go through those three calls."""
     _require_hip(x, "quantize_rows_dynamic")
     if x.dtype != T.float32 or x.ndim != 2:
         raise _C.DtypeMismatch(f"quantize_rows_dynamic expects a 2-d float32 tensor, got {x.dtype} {x.shape}")
     rows, cols = x.shape
     storage = T.as_dtype(qdtype.storage)
-    if storage == T.int8 and cols % 4 == 0 and 4 <= cols <= 16384 and x.data_ptr % 16 == 0:
+    whole = cols % 4 == 0 and x.data_ptr % 16 == 0
+    if storage == T.int8 and 1 <= cols <= 16384 and (whole or rows):
         q = Tensor.empty(x.shape, T.int8, "hip")
         scale = Tensor.empty((rows,), T.float32, "hip")
         zp = Tensor.empty((rows,), T.float32, "hip")
-        _C.call("lq_quantize_rows_dynamic_i8", x.data_ptr, rows, cols, int(qscheme.is_symmetric),
-                qdtype.quant_min, qdtype.quant_max, int(qdtype.signed), float(eps), 0, scale.data_ptr,
-                zp.data_ptr, None, None, q.data_ptr, None)
+        _C.call("lq_quantize_rows_dynamic_i8" if whole else "lq_quantize_rows_dynamic_ragged_i8", x.data_ptr, rows,
+                cols, int(qscheme.is_symmetric), qdtype.quant_min, qdtype.quant_max, int(qdtype.signed), float(eps), 0,
+                scale.data_ptr, zp.data_ptr, None, None, q.data_ptr, None)
         return q, scale, zp
     mn, mx = minmax(x, ch_axis=0)
     scale, zp = calculate_qparams(mn, mx, qscheme, qdtype, eps)

@@ -419,6 +419,44 @@ def test_quantize_rows_dynamic_equals_the_three_calls_and_the_oracle(rows, cols,
     assert np.array_equal(q.numpy()[ok], oq[ok])
 
 
+# rows that end inside a quad, shorter than one, at the ends of what a block's registers hold; rows that begin at odd addresses
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (9, 5), (300, 7), (3, 1023), (3, 1025), (4, 4095), (2, 4097), (5, 7386),
+                                       (2, 8191), (2, 8193), (2, 16383), (1, 16385)])
+@pytest.mark.parametrize("scheme", ["sym_i8", "affine_i8"])
+def test_quantize_rows_dynamic_of_ragged_rows(rows, cols, scheme):
+    qs = Q.per_channel_symmetric if scheme == "sym_i8" else Q.per_channel_affine
+    rng = np.random.default_rng(cols)
+    x = (rng.standard_normal((rows, cols)) * 3 + 0.5).astype(np.float32)
+    x[-1, -1] = 77.0  # the last element of all
+    x[0, 0] = -55.0
+    if rows > 3:
+        x[2, -1] = np.nan
+    xt = hip(x)
+    q, s, z = Q.quantize_rows_dynamic(xt, qs, Q.qint8)
+    mn, mx = Q.minmax(xt, ch_axis=0)
+    ws, wz = Q.calculate_qparams(mn, mx, qs, Q.qint8)
+    wq = Q.quantize(xt, ws, wz, Q.qint8, ch_axis=0)
+    assert same_f32(s.numpy(), ws.numpy()) and same_f32(z.numpy(), wz.numpy())
+    ok = ~np.isnan(ws.numpy())
+    assert np.array_equal(q.numpy()[ok], wq.numpy()[ok])
+
+
+def test_quantize_rows_dynamic_at_odd_addresses_writes_its_rows_only():
+    from lucid_amd import _C
+    rows, cols = 3, 1030
+    x = np.random.default_rng(5).standard_normal(rows * cols + 1).astype(np.float32)
+    xt = hip(x)
+    q = hip(np.full(rows * cols + 5, 99, np.int8))
+    s, z, mn, mx = [L.Tensor.empty((rows,), L.float32, "hip") for _ in range(4)]
+    _C.call("lq_quantize_rows_dynamic_ragged_i8", xt.data_ptr + 4, rows, cols, 1, -128, 127, 1, 1e-8, 0, s.data_ptr,
+            z.data_ptr, mn.data_ptr, mx.data_ptr, q.data_ptr + 3, None)
+    r = x[1:].reshape(rows, cols)
+    got = q.numpy()
+    assert (got[:3] == 99).all() and (got[-2:] == 99).all()
+    assert np.array_equal(mn.numpy(), r.min(1)) and np.array_equal(mx.numpy(), r.max(1))
+    assert np.array_equal(got[3:-2].reshape(rows, cols), O.quantize(r, s.numpy(), z.numpy(), -128, 127, ch_axis=0))
+
+
 @pytest.mark.parametrize("n", [0, 1, 3, 4, 1000, 64 * 784, 262144, 50177,
                                122881, 131071, 131072, 131073])  # 16 blocks of 8192, and 17
 @pytest.mark.parametrize("qd", ["quint8", "qint8"])
