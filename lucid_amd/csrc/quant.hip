@@ -774,11 +774,13 @@ __global__ __launch_bounds__(256) void quantize_rows_dynamic_kernel(
 //
 // Rows of `cols` elements go to rows of `ld` codes, zeros past `cols` (what a GEMM of ragged rows wants).
 //
-// 8192 elements 3.4 us, 65536 (8 blocks, the exchange) 5.9.  A slot is read first when most of them have been written, and
-// not at once again: 128 blocks of 1 M elements that polled without a pause took 17 us, in two launches 3.8 + 5.0.  A dynamic
-// Linear behind it, in two launches / in one, us: 333 x 1000 -> 1001 (42 blocks) 16.6 / 13.6; with 128 blocks it is 25.7 / 24.9,
-// with 256 32.7 / 30.7, too little for that much of the device.  Before either: one block on one CU for up to 262144
-// elements (61 us), five launches beyond (1 M elements: 12.3 us).
+// 8192 elements 3.3 us, 65536 (8 blocks, the exchange) 5.7.  A slot is read first when most of them have been written, and
+// not at once again.  In two launches 1 M elements take 7.5 us, 4 M 11.3, 16 M 30.8 (14.8, 22.9 and 41.2 while the codes of the
+// last quads were picked by an index: the array lay in LDS, at a place that every wavefront computed from the dispatch
+// packet, which is read from host memory; 262144 elements in one launch 8.9 -> 5.7).  Blocks that exchange and take that long to
+// start were measured as: a dynamic Linear in two launches / in one 333 x 1000 -> 1001 (42 blocks) 16.6 / 13.6, with 128 blocks
+// 25.7 / 24.9, with 256 32.7 / 30.7, too little for that much of the device.  Before either: one block on one CU for up to
+// 262144 elements (61 us), five launches beyond (1 M elements: 12.3 us).
 constexpr int kDynThreads = 512, kDynQuads = 4, kDynPerBlock = kDynThreads * kDynQuads * 4;
 constexpr int kExchange = 64, kExchangePolls = 4096, kMaxParts = 512;
 constexpr unsigned long long kSlotEmpty = ~0ull;  // NaNs that no range contains: mm_write's NaN is the canonical one
@@ -889,8 +891,10 @@ void quantize_tensor_dynamic_kernel(const float* __restrict__ x, size_t n, unsig
             if (at(u) < size_t(n / cols) * ld) __builtin_memcpy(q + at(u), &w, 4);
         } else if (count[u] == 4) {
             __builtin_memcpy(q + at(u), &c, 4);
-        } else {
-            for (int i = 0; i < count[u]; ++i) q[at(u) + i] = c.v[i];
+        } else {  // (named one by one, as in quantize_rows_dynamic_kernel)
+            if (count[u] > 0) q[at(u)] = c.v[0];
+            if (count[u] > 1) q[at(u) + 1] = c.v[1];
+            if (count[u] > 2) q[at(u) + 2] = c.v[2];
         }
     }
 }
