@@ -507,6 +507,12 @@ int lq_dynamic_mlp2_small_rows_f32(const float* x, int M, int K1, const int8_t* 
                                    const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2,
                                    int symmetric, int qmin, int qmax, int is_signed, float eps, int code_offset,
                                    float* out, lq_stream stream);
+/* The same for any number of rows with M K1 <= 65536, M ldw2 <= 32768 and at most 192 tiles of 16 x 16 hidden values. */
+int lq_dynamic_mlp2_rows_f32(const float* x, int M, int K1, const int8_t* w1, int ldw1, int N1, const float* w1_scale,
+                             const int32_t* w1sum, const float* bias1, int relu1, const int8_t* w2, int ldw2, int N2,
+                             const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2,
+                             int symmetric, int qmin, int qmax, int is_signed, float eps, int code_offset,
+                             float* out, lq_stream stream);
 
 /* Dynamic per-row quantization in one pass: for every row of x [rows, cols],
  * min / max of the row (PerChannelMinMaxObserver with ch_axis = 0,

@@ -125,6 +125,8 @@ _SIGNATURES = {
     "lq_dynamic_linear_f32": [_vp, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, C.c_float, _i, _vp, _vp],
     "lq_dynamic_mlp2_small_f32": [_vp, _i, _i, _vp, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i,
                                   C.c_float, _i, _vp, _vp],
+    "lq_dynamic_mlp2_rows_f32": [_vp, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i,
+                                       C.c_float, _i, _vp, _vp],
     "lq_dynamic_mlp2_small_rows_f32": [_vp, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i,
                                        C.c_float, _i, _vp, _vp],
     "lq_selftest_requant_route": [C.c_float, C.c_float, _i, _i, _i, C.c_ulonglong, C.c_ulonglong, _vp, _vp, _vp],

@@ -1336,8 +1336,11 @@ __global__ __launch_bounds__(1024) void dynamic_linear_small_kernel(
 // the first).  15.7 us for that MLP; with ONE block doing both layers it was 21 us (one CU's
 // vector units quantized all 50 k inputs).  `hid`: [M][ld2] float32, then kMlpBlocks minima and as many maxima;
 // `counter`: zero between launches (the last block resets it).  Columns of `hid` from N1 to ld2 hold anything: their codes
-// meet the zeros of layer 2's padded weight rows.  KS2: steps of 64 k that ld2 takes at most.
-constexpr int kMlpBlocks = 128, kMlpMaxHidden = 511;
+// meet the zeros of layer 2's padded weight rows.  KS2: steps of 64 k that ld2 takes at most, and quads of the hidden
+// activation per thread of the last block: M * ld2 is at most 4096 KS2.  (More than 64 rows, which the last block's wavefronts
+// take 64 at a time, in two calls of two launches 28.5 us, whatever their size: 148 rows of 32-48-15 14.0 in one, 256 of
+// 256-128-64 18.1, 2048 of 32-16-8 24.9.)
+constexpr int kMlpBlocks = 192, kMlpMaxHidden = 511;
 template <bool RAGGED, int KS2>
 __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     const float* __restrict__ x, int M, int K1, const int8_t* __restrict__ w1, int ld1, int N1, const float* __restrict__ ws1,
@@ -1352,7 +1355,7 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int8_t* const codes = mb_smem;                                       // [16][ld1]: the block's rows
     int* const red = reinterpret_cast<int*>(mb_smem + size_t(16) * ld1);  // [4][64]
-    int8_t* const codes2 = mb_smem + size_t(16) * ld1 + 1024;             // [64][ld2]: the last block's
+    int8_t* const codes2 = mb_smem + size_t(16) * ld1 + 1024;             // [M rounded up to 16][ld2]: the last block's
     const float qnan = __builtin_nanf("");
     const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
     const int nblocks = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
@@ -1405,7 +1408,7 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
         const int i = u * 1024 + tid;
         h[u] = __builtin_amdgcn_raw_buffer_load_b128(hbuf, unsigned(i < quads2 ? i : 0) * 16, 0, kScopeDevice);
     }
-    const int rb2 = wave & 3, cb2 = wave >> 2;
+    const int cb2 = wave >> 2;
     const int n2 = cb2 * 16 + ln, nc2 = n2 < N2 ? n2 : N2 - 1;
     dl_v4i w2f[KS2];
     {
@@ -1419,7 +1422,7 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
     t2.c_ws = ws2 ? ws2[nc2] : 1.0f;
     t2.c_wsum = wsum2 ? wsum2[nc2] : 0;
     t2.c_bias = b2 ? b2[nc2] : -0.0f;
-    for (int i = quads2 + tid; i < 16 * ld2; i += 1024) reinterpret_cast<unsigned*>(codes2)[i] = 0u;
+    for (int i = quads2 + tid; i < ((M + 15) >> 4) * 4 * ld2; i += 1024) reinterpret_cast<unsigned*>(codes2)[i] = 0u;
     MinMax tm{slot_lo, slot_hi, int((slot_lo != slot_lo) | (slot_hi != slot_hi))};
     if (tm.nan) tm.lo = __builtin_inff(), tm.hi = -__builtin_inff();
     tm = mm_block_reduce(tm);
@@ -1436,22 +1439,28 @@ __global__ __launch_bounds__(1024) void dynamic_mlp2_blocks_kernel(
             if (i < quads2) op.q[i] = op.pack(__builtin_bit_cast(float4, h[u]), s2, z2, r2);
         }
     }
+    if (cb2 * 16 < N2) {
+#pragma unroll
+        for (int ks = 0; ks < KS2; ++ks) w2f[ks] = place(w2f[ks]);
+    }
     __syncthreads();
-    if (cb2 * 16 < N2 && rb2 * 16 < M) {
-        dl_v4i acc2 = dl_v4i{0, 0, 0, 0};
+    if (cb2 * 16 < N2) {
+        for (int rb2 = wave & 3; rb2 * 16 < M; rb2 += 4) {
+            dl_v4i acc2 = dl_v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int ks = 0; ks < KS2; ++ks) {
-            const int k = ks * 64 + lg * 16;
-            if (ks * 64 < ld2) {  // uniform
-                const dl_v4i af = k < ld2 ? *reinterpret_cast<const dl_v4i*>(codes2 + size_t(16 * rb2 + ln) * ld2 + k)
-                                          : dl_v4i{0, 0, 0, 0};
-                acc2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, place(w2f[ks]), acc2, 0, 0, 0);
+            for (int ks = 0; ks < KS2; ++ks) {
+                const int k = ks * 64 + lg * 16;
+                if (ks * 64 < ld2) {  // uniform
+                    const dl_v4i af = k < ld2 ? *reinterpret_cast<const dl_v4i*>(codes2 + size_t(16 * rb2 + ln) * ld2 + k)
+                                              : dl_v4i{0, 0, 0, 0};
+                    acc2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, w2f[ks], acc2, 0, 0, 0);
+                }
             }
-        }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int mm = 16 * rb2 + 4 * lg + q;
-            if (mm < M && n2 < N2) out[size_t(mm) * N2 + n2] = t2.output(acc2[q], wsum2 != nullptr, relu2);
+            for (int q = 0; q < 4; ++q) {
+                const int mm = 16 * rb2 + 4 * lg + q;
+                if (mm < M && n2 < N2) out[size_t(mm) * N2 + n2] = t2.output(acc2[q], wsum2 != nullptr, relu2);
+            }
         }
     }
 }
@@ -1533,6 +1542,46 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
            : launch(quantize_tensor_dynamic_kernel<true, false>, parts, int(splits));
     LQ_CHECK_LAUNCH("quantize_tensor_parts");
     return LQ_OK;
+}
+
+int dynamic_mlp2(int max_rows, const float* x, int M, int K1, const int8_t* w1, int ldw1, int N1, const float* w1_scale,
+                 const int32_t* w1sum, const float* bias1, int relu1, const int8_t* w2, int ldw2, int N2,
+                 const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2,
+                 int symmetric, int qmin, int qmax, int is_signed, float eps, int code_offset,
+                 float* out, lq_stream stream) {
+    if (M == 0 || N2 == 0) return LQ_OK;
+    LQ_REQUIRE(x && w1 && w2 && out, LQ_ERR_VALUE, "dynamic_mlp2_small: NULL pointer");
+    LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
+               "dynamic_mlp2_small: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
+    // a block holds 16 rows of x's codes; the last one also the hidden activation's codes, in rows of ldw2 bytes
+    LQ_REQUIRE(M > 0 && M <= max_rows && K1 > 0 && ldw1 >= K1 && ldw1 % 16 == 0 && ldw1 <= 1024 && N1 > 0 && N1 <= kMlpMaxHidden &&
+                   ldw2 >= N1 && ldw2 % 16 == 0 && ldw2 <= 512 && N2 > 0 && N2 <= 64 && aligned16(x) && aligned16(w1) &&
+                   aligned16(w2) && long(M) * K1 <= 65536 && long(M) * ldw2 <= 32768 &&
+                   ((M + 15) / 16) * ((N1 + 15) / 16) <= kMlpBlocks,
+               LQ_ERR_NOT_IMPLEMENTED,
+               "dynamic_mlp2_small: takes up to %d rows, weight rows of a multiple of 16 bytes (K1 up to 1024, a hidden width "
+               "up to %d), up to 64 outputs, 65536 inputs, 32768 hidden values in 192 tiles and 16-byte aligned operands (got "
+               "M = %d, K1 = %d in rows of %d, N1 = %d in rows of %d, N2 = %d); use two lq_dynamic_linear_f32 calls", max_rows, kMlpMaxHidden, M, K1, ldw1, N1, ldw2, N2);
+    const float half_range = float((double(qmax) - double(qmin)) / 2.0);
+    // the hidden activation and the tiles' ranges pass through the stream's split-K scratch
+    SkScratch sk;
+    const auto lock = scratch_lock(as_stream(stream));
+    const size_t hid_bytes = size_t(M) * ldw2 * 4;
+    if (int rc = sk_scratch(1, hid_bytes + 8 * kMlpBlocks, as_stream(stream), &sk)) return rc;
+    const size_t lds = size_t(16) * ldw1 + 1024 + size_t((M + 15) / 16 * 16) * ldw2;  // at most 16 + 1 + 32 + 7.5 KiB
+    static DeviceOnce attr_once[4];
+    auto launch = [&](auto kernel, int form) -> int {
+        if (int rc = allow_dynamic_lds(attr_once[form], reinterpret_cast<const void*>(kernel), 64 * 1024)) return rc;
+        hipLaunchKernelGGL(kernel, dim3(unsigned((N1 + 15) / 16), unsigned((M + 15) / 16)), dim3(1024), lds,
+                           as_stream(stream), x, M, K1, w1, ldw1, N1, w1_scale, w1sum, bias1, relu1, w2, ldw2, N2, w2_scale,
+                           w2sum, bias2, relu2, symmetric, qmin, qmax, is_signed, eps, half_range, code_offset, out,
+                           reinterpret_cast<float*>(sk.slabs), sk.counters);
+        LQ_CHECK_LAUNCH("dynamic_mlp2_small");
+        return LQ_OK;
+    };
+    const bool ragged = ldw1 != K1, wide = ldw2 > 256 || M * ldw2 > 16384;
+    return ragged ? (wide ? launch(dynamic_mlp2_blocks_kernel<true, 8>, 0) : launch(dynamic_mlp2_blocks_kernel<true, 4>, 1))
+                  : (wide ? launch(dynamic_mlp2_blocks_kernel<false, 8>, 2) : launch(dynamic_mlp2_blocks_kernel<false, 4>, 3));
 }
 
 int quantize_rows(const float* x, size_t rows, size_t cols, bool ragged, int symmetric, int qmin, int qmax, int is_signed,
@@ -1664,38 +1713,17 @@ int lq_dynamic_mlp2_small_rows_f32(const float* x, int M, int K1, const int8_t* 
                                    const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2,
                                    int symmetric, int qmin, int qmax, int is_signed, float eps, int code_offset,
                                    float* out, lq_stream stream) {
-    if (M == 0 || N2 == 0) return LQ_OK;
-    LQ_REQUIRE(x && w1 && w2 && out, LQ_ERR_VALUE, "dynamic_mlp2_small: NULL pointer");
-    LQ_REQUIRE(qmax > qmin && qmin + code_offset >= -128 && qmax + code_offset <= 127, LQ_ERR_VALUE,
-               "dynamic_mlp2_small: grid [%d,%d] + offset %d does not fit int8", qmin, qmax, code_offset);
-    // a block holds 16 rows of x's codes; the last one also the hidden activation's codes (64 ldw2 bytes)
-    LQ_REQUIRE(M > 0 && M <= 64 && K1 > 0 && ldw1 >= K1 && ldw1 % 16 == 0 && ldw1 <= 1024 && N1 > 0 && N1 <= kMlpMaxHidden &&
-                   ldw2 >= N1 && ldw2 % 16 == 0 && ldw2 <= 512 && N2 > 0 && N2 <= 64 && aligned16(x) && aligned16(w1) &&
-                   aligned16(w2),
-               LQ_ERR_NOT_IMPLEMENTED,
-               "dynamic_mlp2_small: takes up to 64 rows, weight rows of a multiple of 16 bytes (K1 up to 1024, a hidden width "
-               "up to %d), up to 64 outputs and 16-byte aligned operands (got M = %d, K1 = %d in rows of %d, N1 = %d in rows "
-               "of %d, N2 = %d); use two lq_dynamic_linear_f32 calls", kMlpMaxHidden, M, K1, ldw1, N1, ldw2, N2);
-    const float half_range = float((double(qmax) - double(qmin)) / 2.0);
-    // the hidden activation and the tiles' ranges pass through the stream's split-K scratch
-    SkScratch sk;
-    const auto lock = scratch_lock(as_stream(stream));
-    const size_t hid_bytes = size_t(M) * ldw2 * 4;
-    if (int rc = sk_scratch(1, hid_bytes + 8 * kMlpBlocks, as_stream(stream), &sk)) return rc;
-    const size_t lds = size_t(16) * ldw1 + 1024 + size_t(64) * ldw2;
-    static DeviceOnce attr_once[4];
-    auto launch = [&](auto kernel, int form) -> int {
-        if (int rc = allow_dynamic_lds(attr_once[form], reinterpret_cast<const void*>(kernel), 64 * 1024)) return rc;
-        hipLaunchKernelGGL(kernel, dim3(unsigned((N1 + 15) / 16), unsigned((M + 15) / 16)), dim3(1024), lds,
-                           as_stream(stream), x, M, K1, w1, ldw1, N1, w1_scale, w1sum, bias1, relu1, w2, ldw2, N2, w2_scale,
-                           w2sum, bias2, relu2, symmetric, qmin, qmax, is_signed, eps, half_range, code_offset, out,
-                           reinterpret_cast<float*>(sk.slabs), sk.counters);
-        LQ_CHECK_LAUNCH("dynamic_mlp2_small");
-        return LQ_OK;
-    };
-    const bool ragged = ldw1 != K1, wide = ldw2 > 256;
-    return ragged ? (wide ? launch(dynamic_mlp2_blocks_kernel<true, 8>, 0) : launch(dynamic_mlp2_blocks_kernel<true, 4>, 1))
-                  : (wide ? launch(dynamic_mlp2_blocks_kernel<false, 8>, 2) : launch(dynamic_mlp2_blocks_kernel<false, 4>, 3));
+    return dynamic_mlp2(64, x, M, K1, w1, ldw1, N1, w1_scale, w1sum, bias1, relu1, w2, ldw2, N2, w2_scale, w2sum, bias2, relu2,
+                        symmetric, qmin, qmax, is_signed, eps, code_offset, out, stream);
+}
+
+int lq_dynamic_mlp2_rows_f32(const float* x, int M, int K1, const int8_t* w1, int ldw1, int N1, const float* w1_scale,
+                             const int32_t* w1sum, const float* bias1, int relu1, const int8_t* w2, int ldw2, int N2,
+                             const float* w2_scale, const int32_t* w2sum, const float* bias2, int relu2,
+                             int symmetric, int qmin, int qmax, int is_signed, float eps, int code_offset,
+                             float* out, lq_stream stream) {
+    return dynamic_mlp2(2048, x, M, K1, w1, ldw1, N1, w1_scale, w1sum, bias1, relu1, w2, ldw2, N2, w2_scale, w2sum, bias2, relu2,
+                        symmetric, qmin, qmax, is_signed, eps, code_offset, out, stream);
 }
 
 int lq_dynamic_linear_small_f32(const float* x, int M, int K, const int8_t* w, int N, const float* w_scale,

@@ -87,14 +87,22 @@ def _keep(*derived) -> None:
 PAIR_MAX_K, PAIR_MAX_HIDDEN = 1024, 511
 
 
+def _pair_in_one_launch(M: int, K1: int, N1: int, N2: int) -> bool:
+    """Whether ``lq_dynamic_mlp2_rows_f32`` takes the pair: what its blocks (all of x) and the last one of them (all of
+    the hidden activation) keep in registers."""
+    return (M > 0 and 0 < K1 <= PAIR_MAX_K and 0 < N1 <= PAIR_MAX_HIDDEN and 0 < N2 <= 64 and M * K1 <= 65536
+            and (M <= 64 or M * _code_row_bytes(N1) <= 32768 and (M + 15) // 16 * ((N1 + 15) // 16) <= 192))
+
+
 def fused_pair(first, relu_between: bool, second, x):
     """``second(relu(first(x)))`` (or without the ReLU) for two dynamic ``Linear`` layers on a small
     activation as ONE launch (``lq_dynamic_mlp2_small_f32``: the last block of layer 1 to finish
     reduces the hidden activation's min / max and runs layer 2; ``lq_dynamic_mlp2_small_rows_f32`` where a weight's
-    rows are no whole 16 bytes or the hidden layer is wide), beyond it as two calls with the ReLU in the
-    first one's epilogue, or ``None`` when the shapes or operands do not qualify.  Same bits as calling the modules one
+    rows are no whole 16 bytes or the hidden layer is wide; ``lq_dynamic_mlp2_rows_f32`` for more than 64 rows), beyond
+    it as two calls with the ReLU in the first one's epilogue, or ``None`` when the shapes or operands do not qualify.  Same bits as calling the modules one
     after the other.  Per forward, ReLU between: 91-32-58 of 12 rows in one launch 12.6 us (32 in three calls, which is what
-    their host side takes), 64 rows of 784-496-10 17.9 (33)."""
+    their host side takes), 64 rows of 784-496-10 17.9 (33), 148 of
+    32-48-15 14.0, 256 of 256-128-64 18.1, 2048 of 32-16-8 24.9 (28.5 in two calls)."""
     if not (isinstance(first, Linear) and isinstance(second, Linear) and isinstance(x, Tensor)):
         return None
     if x.device != "hip" or x.dtype != T.float32 or x._grid is not None or x._range is not None:
@@ -103,8 +111,8 @@ def fused_pair(first, relu_between: bool, second, x):
     if x.ndim < 1 or x.shape[-1] != K1 or second.in_features != N1:
         return None
     M = x.numel // K1 if K1 else 0
-    small = 0 < M <= 64 and K1 <= PAIR_MAX_K and 0 < N1 <= PAIR_MAX_HIDDEN and 0 < N2 <= 64
-    rows = small and (K1 % 16 != 0 or N1 % 16 != 0 or N1 > 256)
+    small = _pair_in_one_launch(M, K1, N1, N2)
+    rows = small and (M > 64 or K1 % 16 != 0 or N1 % 16 != 0 or N1 > 256)
     if rows and x.data_ptr % 16:
         small = False
     if not small and not relu_between:
@@ -138,8 +146,9 @@ def fused_pair(first, relu_between: bool, second, x):
                 fresh += ((lin, "_wrows", rows),)
             padded.append(rows)
         (w1, ld1), (w2, ld2) = padded
-        _C.call("lq_dynamic_mlp2_small_rows_f32", x.data_ptr, M, K1, w1.data_ptr, ld1, N1, scale1.data_ptr, wsum1.data_ptr,
-                b1, int(relu_between), w2.data_ptr, ld2, N2, scale2.data_ptr, wsum2.data_ptr, b2, 0, *grid, y.data_ptr, None)
+        _C.call("lq_dynamic_mlp2_small_rows_f32" if M <= 64 else "lq_dynamic_mlp2_rows_f32", x.data_ptr, M, K1, w1.data_ptr,
+                ld1, N1, scale1.data_ptr, wsum1.data_ptr, b1, int(relu_between), w2.data_ptr, ld2, N2, scale2.data_ptr,
+                wsum2.data_ptr, b2, 0, *grid, y.data_ptr, None)
     else:
         _C.call("lq_dynamic_mlp2_small_f32", x.data_ptr, M, K1, w1.data_ptr, N1, scale1.data_ptr, wsum1.data_ptr,
                 b1, int(relu_between), w2.data_ptr, N2, scale2.data_ptr, wsum2.data_ptr, b2, 0, *grid, y.data_ptr, None)

@@ -744,7 +744,30 @@ def test_two_dynamic_linears_of_any_sizes_in_one_launch(M, K1, N1, N2, kind):
     _same_as_one_after_the_other(model, xd, got)
 
 
-@pytest.mark.parametrize("M,K1,N1,N2,row", [(65, 784, 256, 10, 0), (256, 91, 512, 64, 0), (70, 33, 20, 65, 0), (8, 91, 40, 7, 1),
+# batches whose hidden activation the last block still holds: 16384 and 32768 values and one row more than the former, 65536
+# inputs, 130 tiles, tiles of one row, batches that are no whole tiles or rounds of its wavefronts
+@pytest.mark.parametrize("M,K1,N1,N2", [(65, 784, 256, 10), (128, 512, 256, 64), (129, 91, 128, 33), (256, 256, 128, 17),
+                                        (255, 33, 64, 1), (65, 1000, 400, 10), (2048, 32, 16, 5), (500, 65, 20, 64),
+                                        (449, 16, 1, 3), (200, 300, 160, 10)])
+@pytest.mark.parametrize("relu", [True, False])
+@pytest.mark.parametrize("kind", ["normal", "nan", "inf"])
+def test_two_dynamic_linears_of_larger_batches_in_one_launch(M, K1, N1, N2, relu, kind):
+    rng = np.random.default_rng(M + K1 + N1 + N2)
+    model = _pair(rng, K1, N1, N2, relu)
+    x = rng.standard_normal((M, K1)).astype(np.float32)
+    if kind != "normal":
+        x[M - 1, K1 - 1] = np.nan if kind == "nan" else np.inf
+    xd = hip(x)
+    model(xd)
+    for _ in range(2):  # the counter of the blocks is zero again behind each
+        with _recorded_calls() as calls:
+            got = model(xd)
+        assert calls == ["lq_dynamic_mlp2_rows_f32"]
+        _same_as_one_after_the_other(model, xd, got)
+
+
+@pytest.mark.parametrize("M,K1,N1,N2,row", [(100, 784, 256, 10, 0), (129, 91, 256, 10, 0), (97, 64, 333, 10, 0),
+                                            (256, 91, 512, 64, 0), (70, 33, 20, 65, 0), (8, 91, 40, 7, 1),
                                             (64, 2000, 64, 10, 0)])
 def test_the_relu_between_two_dynamic_linears_rides_in_the_first(M, K1, N1, N2, row):
     """Beyond the one launch, and on rows of an activation that begin at no 16 bytes: two calls, the same bits."""
