@@ -488,7 +488,7 @@ __device__ __forceinline__ v4i act16(const int8_t* row, int k, int K) {
     return v;
 }
 
-// The tile kernels' global-to-LDS loads do need aligned rows: for more than 64 activation rows both
+// The tile kernels' global-to-LDS loads do need aligned rows: for more than 64 activation rows (16 with a large weight) both
 // operands are copied to rows of `ld` bytes (a multiple of 64: every shape is open to the problem), zeros
 // past K.  A thread moves 16 bytes.  The copy moves 2 (M + N) K bytes beside 2 M N K operations and is bound by
 // memory: at 333 x 1001 x 1000 it is 3.9 us and the product 7 us, where the one-output-per-lane kernel took
@@ -874,6 +874,43 @@ int run_tile_kernel(const GemmArgs& g_in, int conv, int groups, int tile_config,
     return launch_tile_cfg(g, 0, 1, tile_config, st);
 }
 
+// The kernels for up to 64 rows, of any length from 16 on and at any address.
+int run_skinny(const GemmArgs& g, hipStream_t st) {
+    if (g.M == 1 && g.K <= 65536) {
+        // four rows per wavefront; as many wavefronts per block (up to 8) as still leave 256 blocks
+        int waves = 8;
+        while (waves > 1 && (g.N + 4 * waves - 1) / (4 * waves) < 256) waves >>= 1;
+        const unsigned blocks = unsigned((g.N + 4 * waves - 1) / (4 * waves));
+        const size_t lds = size_t((g.K + 4095) / 4096) * 4096;
+        hipLaunchKernelGGL(qgemv1_kernel, dim3(blocks), dim3(waves * 64), lds, st, g);
+        LQ_CHECK_LAUNCH("qgemv1");
+        return LQ_OK;
+    }
+    if (g.M <= 16 && g.K >= 1024) {
+        int R = (g.N + 255) / 256;  // one block per compute unit when the rows allow it
+        R = R < 16 ? 16 : (R > 64 ? 64 : R);
+        const int G = (R + 15) / 16;
+        const dim3 grid16{unsigned((g.N + R - 1) / R)}, block16{1024};
+        switch (G) {
+        case 1: hipLaunchKernelGGL((qgemm_skinny16_kernel<1>), grid16, block16, 0, st, g, R); break;
+        case 2: hipLaunchKernelGGL((qgemm_skinny16_kernel<2>), grid16, block16, 0, st, g, R); break;
+        case 3: hipLaunchKernelGGL((qgemm_skinny16_kernel<3>), grid16, block16, 0, st, g, R); break;
+        default: hipLaunchKernelGGL((qgemm_skinny16_kernel<4>), grid16, block16, 0, st, g, R); break;
+        }
+        LQ_CHECK_LAUNCH("qgemm_skinny16");
+        return LQ_OK;
+    }
+    dim3 grid{unsigned((g.N + 15) / 16)}, block{256};
+    if (g.M <= 16)
+        hipLaunchKernelGGL((qgemm_skinny_kernel<1>), grid, block, 0, st, g);
+    else if (g.M <= 32)
+        hipLaunchKernelGGL((qgemm_skinny_kernel<2>), grid, block, 0, st, g);
+    else
+        hipLaunchKernelGGL((qgemm_skinny_kernel<4>), grid, block, 0, st, g);
+    LQ_CHECK_LAUNCH("qgemm_skinny");
+    return LQ_OK;
+}
+
 int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t st) {
     GemmArgs g = g_in;
     const bool vec_ok = g.K % 16 == 0 && g.K > 0 && aligned16(g.a) && aligned16(g.w);
@@ -881,19 +918,25 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
     if (path == 0) {
         // One row is a stream of the weight; aligned rows go to the K-split tiles of 16 rows from two on (see qgemm_ks.hpp), to
         // those of 32 and 64 and the tile kernel from 17.  Ragged or unaligned operands have to be copied to padded rows for
-        // them, the whole weight too: that pays from 65 rows (333 x 1001
-        // x 1000: 1340 -> 11 us against the plain kernel; 100 x 11008 x 5001: 26.4 ms -> 50 us).  A kept range
-        // needs the tile kernels.  Rows shorter than one chunk stay with the plain kernel.
-        path = g.K < 16 ? 3 : (g.M <= (vec_ok ? 1 : 64) && g.range == nullptr ? 2 : 1);
+        // them, the whole weight too: that pays from 65 rows (333 x 1001 x 1000: 1340 -> 11 us against the plain kernel;
+        // 100 x 11008 x 5001: 26.4 ms -> 50 us), and below that where the skinny kernels' blocks fetch much of the activation
+        // for a large weight.  K x N of them / of copies and tiles, us with the launches: 64 rows 4100 x 4001 25.0 / 19.3, 7386 x
+        // 3036 52.2 / 22.6, 515 x 8000 13.4 / 15.6, 1001 x 1000 10.6 / 11.3; 40 rows 25.6 / 20.1, 39.7 / 22.2, 10.6 / 11.0, 9.1 / 11.4;
+        // 32 rows 17.1 / 20.2, 30.3 / 21.7, 2050 x 11008 31.9 / 21.1; 17 rows 14.7 / 20.5, 25.2 / 20.8, 23.5 / 21.8; 16 rows 21.0 /
+        // 19.6 for 7386 x 3036, 15.0 / 19.3 for 2050 x 11008.
+        // A kept range needs the tile kernels.  Rows shorter than one chunk stay with the plain kernel.
+        const size_t weight = size_t(g.K) * size_t(g.N);
+        const int direct = vec_ok ? 1 : weight < (size_t(8) << 20) ? 64 : weight < size_t(20000000) ? 32 : 16;
+        path = g.K < 16 ? 3 : (g.M <= direct && g.range == nullptr ? 2 : 1);
         if (path == 1 && !vec_ok) {
             const int ld = (g.K + 63) / 64 * 64;
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;
             void* tmp = nullptr;
             const auto lock = scratch_lock(st);
             int rc = call_buffer(4, a_bytes + w_bytes, st, &tmp);
-            if (rc == LQ_ERR_OOM && g.range == nullptr) {  // no room for the copies: the plain kernel needs none
+            if (rc == LQ_ERR_OOM && g.range == nullptr) {  // no room for the copies: the others need none
                 (void)hipGetLastError();
-                return run_gemm(g_in, 3, tile_config, st);
+                return g.M <= 64 ? run_skinny(g, st) : run_gemm(g_in, 3, tile_config, st);
             }
             if (rc) return rc;
             int8_t* pa = static_cast<int8_t*>(tmp);
@@ -903,7 +946,7 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
                                pa, pa + a_bytes);
             LQ_CHECK_LAUNCH("pad_rows");
             g.a = pa, g.w = pa + a_bytes, g.K = ld;
-            return run_tile_kernel(g, 0, 1, tile_config, st);
+            return run_tile_kernel(g, 0, 1, g.M > 64 ? tile_config : 0, st);  // (a shape asked for was never looked at up to 64 rows)
         }
     }
     // only the tile kernel keeps the range of what it writes
@@ -916,38 +959,7 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
         if (rc) return rc;
     } else if (path == 2) {
         LQ_REQUIRE(g.M <= 64, LQ_ERR_SHAPE, "qlinear_i8: skinny path needs M <= 64 (M = %d)", g.M);
-        if (g.M == 1 && g.K <= 65536) {
-            // four rows per wavefront; as many wavefronts per block (up to 8) as still leave 256 blocks
-            int waves = 8;
-            while (waves > 1 && (g.N + 4 * waves - 1) / (4 * waves) < 256) waves >>= 1;
-            const unsigned blocks = unsigned((g.N + 4 * waves - 1) / (4 * waves));
-            const size_t lds = size_t((g.K + 4095) / 4096) * 4096;
-            hipLaunchKernelGGL(qgemv1_kernel, dim3(blocks), dim3(waves * 64), lds, st, g);
-            LQ_CHECK_LAUNCH("qgemv1");
-            return LQ_OK;
-        }
-        if (g.M <= 16 && g.K >= 1024) {
-            int R = (g.N + 255) / 256;  // one block per compute unit when the rows allow it
-            R = R < 16 ? 16 : (R > 64 ? 64 : R);
-            const int G = (R + 15) / 16;
-            const dim3 grid16{unsigned((g.N + R - 1) / R)}, block16{1024};
-            switch (G) {
-            case 1: hipLaunchKernelGGL((qgemm_skinny16_kernel<1>), grid16, block16, 0, st, g, R); break;
-            case 2: hipLaunchKernelGGL((qgemm_skinny16_kernel<2>), grid16, block16, 0, st, g, R); break;
-            case 3: hipLaunchKernelGGL((qgemm_skinny16_kernel<3>), grid16, block16, 0, st, g, R); break;
-            default: hipLaunchKernelGGL((qgemm_skinny16_kernel<4>), grid16, block16, 0, st, g, R); break;
-            }
-            LQ_CHECK_LAUNCH("qgemm_skinny16");
-            return LQ_OK;
-        }
-        dim3 grid{unsigned((g.N + 15) / 16)}, block{256};
-        if (g.M <= 16)
-            hipLaunchKernelGGL((qgemm_skinny_kernel<1>), grid, block, 0, st, g);
-        else if (g.M <= 32)
-            hipLaunchKernelGGL((qgemm_skinny_kernel<2>), grid, block, 0, st, g);
-        else
-            hipLaunchKernelGGL((qgemm_skinny_kernel<4>), grid, block, 0, st, g);
-        LQ_CHECK_LAUNCH("qgemm_skinny");
+        return run_skinny(g, st);
     } else {
         size_t blocks = (size_t(g.M) * g.N + 255) / 256;
         if (blocks > 65536) blocks = 65536;

@@ -55,6 +55,17 @@ def test_accumulators_exact(M, N, K, path):
     assert np.array_equal(acc, O.igemm(a, w))
 
 
+# ragged rows, a weight on both sides of the sizes from which it is copied to padded rows (8 Mi from 33 rows, 20 M from 17)
+@pytest.mark.parametrize("M,N,K", [(16, 4900, 4099), (17, 4870, 4099), (17, 4890, 4099), (32, 4880, 4099), (33, 2046, 4099), (33, 2047, 4099),
+                                   (64, 1001, 8385), (48, 8390, 1003), (64, 2000, 4104)])
+@pytest.mark.parametrize("tile_config", [0, 77])
+def test_ragged_rows_of_a_large_weight_exact(M, N, K, tile_config):
+    rng = np.random.default_rng(M + N + K)
+    a, w = codes(rng, (M, K)), codes(rng, (N, K))
+    acc = _ops.qlinear_i8(hip(a), hip(w), out_mode=_ops.OUT_ACC_I32, tile_config=tile_config).numpy()
+    assert np.array_equal(acc, O.igemm(a, w))
+
+
 @pytest.mark.parametrize("cfg", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12])
 @pytest.mark.parametrize("M,N,K", [(256, 256, 128), (300, 260, 144), (129, 77, 784), (513, 1000, 576),
                                    (2048, 512, 4096), (1, 16, 16), (700, 130, 64)])
