@@ -43,7 +43,10 @@ typedef unsigned v2u __attribute__((ext_vector_type(2)));
 constexpr int kPiece = 1024;  // bytes one wavefront moves into LDS with one instruction
 
 // One launch, two kinds of blocks.  The first `split_blocks`: one thread = eight consecutive k of one
-// row; a block = 16 rows x two stages.  The others: one thread = up to four consecutive groups of one column.
+// row; a block = 16 rows x two stages.  The others: 32 groups of 64 columns, read row by row and turned in LDS.
+// 333 x 11008 x 4096 int4 of 128 10.4 -> 8.8 us, 100 x 11008 x 4096 of 32 21.0 -> 11.5: a thread that took four groups of a column for itself
+// read 16 bytes of a line that the blocks of the next groups, on other XCDs, fetched again.
+constexpr int kSbGroups = 32, kSbColumns = 64;
 template <int BITS>
 __global__ __launch_bounds__(256) void wq_prepare_kernel(const float* __restrict__ x, const float* __restrict__ scales,
                                                          const float* __restrict__ biases, int M, int N, int K,
@@ -51,22 +54,50 @@ __global__ __launch_bounds__(256) void wq_prepare_kernel(const float* __restrict
                                                          int segs, unsigned split_blocks, uint4* __restrict__ parts,
                                                          float* __restrict__ xsum, float2* __restrict__ sb) {
     if (blockIdx.x >= split_blocks) {
+        __shared__ float2 tile[kSbGroups][kSbColumns + 1];
         const int groups = K >> gs_shift;
         const int per = segs == 2 ? 1 : (1 << gs_shift) / 64;  // segments per group
-        const unsigned idx = (blockIdx.x - split_blocks) * 256 + threadIdx.x;
-        const unsigned quad = idx / unsigned(n_pad), n = idx - quad * unsigned(n_pad);
-        const int g0 = int(quad) * 4;
-        float s[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
-        if (n < unsigned(N)) {
+        const unsigned idx = blockIdx.x - split_blocks, across = unsigned(n_pad) / kSbColumns;
+        const int n0 = int(idx % across) * kSbColumns, first = int(idx / across) * kSbGroups;
+        // four groups per lane, and of a row's 32 side by side; the last four of a row where those asked for run past it
+        float4 sv[2], bv[2];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (g0 + e < groups) s[e] = scales[size_t(n) * groups + g0 + e], b[e] = biases[size_t(n) * groups + g0 + e];
+        for (int u = 0; u < 2; ++u) {
+            const int n = n0 + u * 32 + int(threadIdx.x >> 3), g0 = first + int(threadIdx.x & 7) * 4;
+            const size_t row = size_t(n < N ? n : N - 1) * groups;
+            if (groups >= 4) {
+                const size_t from = row + (g0 + 4 <= groups ? g0 : groups - 4);
+                __builtin_memcpy(&sv[u], scales + from, 16);
+                __builtin_memcpy(&bv[u], biases + from, 16);
+            } else {  // uniform
+                sv[u] = float4{scales[row], scales[row + groups / 2], scales[row + groups - 1], 0.f};
+                bv[u] = float4{biases[row], biases[row + groups / 2], biases[row + groups - 1], 0.f};
+            }
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int u = 0; u < 2; ++u) {
+            const int c = u * 32 + int(threadIdx.x >> 3), q0 = int(threadIdx.x & 7) * 4, g0 = first + q0;
+            const bool column = n0 + c < N;
+            const float s4[4] = {sv[u].x, sv[u].y, sv[u].z, sv[u].w}, b4[4] = {bv[u].x, bv[u].y, bv[u].z, bv[u].w};
+            // element e of the load is group `at + e`: what is past the row is zeros
+            const int at = groups < 4 || g0 + 4 <= groups ? g0 : groups - 4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int g = groups < 4 ? (e < groups ? first + e : first + kSbGroups) : at + e, slot = g - first;
+                if (column && slot >= q0 && slot < q0 + 4 && (groups >= 4 || q0 == 0))
+                    tile[slot][c] = float2{kWqUnit<BITS> * s4[e], b4[e] - float(kWqCentre<BITS>) * s4[e]};
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (!column || g0 + e >= groups) tile[q0 + e][c] = float2{0.f, 0.f};
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < kSbGroups * kSbColumns; i += 256) {
+            const int g = i / kSbColumns, c = i % kSbColumns;
+            const float2 v = tile[g][c];
             for (int r = 0; r < per; ++r)
-                if ((g0 + e) * per + r < stages * segs)
-                    sb[size_t((g0 + e) * per + r) * n_pad + n] = float2{kWqUnit<BITS> * s[e], b[e] - float(kWqCentre<BITS>) * s[e]};
+                if ((first + g) * per + r < stages * segs) sb[size_t((first + g) * per + r) * n_pad + n0 + c] = v;
+        }
         return;
     }
     const unsigned pairs = unsigned(stages + 1) / 2;
@@ -351,7 +382,8 @@ int launch_rows(const float* x, const uint32_t* packed, const float* scales, con
     const unsigned split_blocks = unsigned((stages + 1) / 2) * unsigned(mtiles);
     // (groups of the stages, past K too)
     const int sb_groups = SEGS == 2 ? stages * 2 : stages / (GS / 64);
-    const unsigned sb_blocks = unsigned((size_t((sb_groups + 3) / 4) * n_pad + 255) / 256);
+    static_assert(bn % kSbColumns == 0, "");
+    const unsigned sb_blocks = unsigned((sb_groups + kSbGroups - 1) / kSbGroups) * unsigned(n_pad / kSbColumns);
     hipLaunchKernelGGL((wq_prepare_kernel<BITS>), dim3(split_blocks + sb_blocks), dim3(256), 0, st, x, scales, biases, M, N,
                        K, gs_shift, mtiles, bm, n_pad, stages, SEGS, split_blocks, reinterpret_cast<uint4*>(parts),
                        reinterpret_cast<float*>(xsum), reinterpret_cast<float2*>(sb));

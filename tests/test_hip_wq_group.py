@@ -147,6 +147,13 @@ def test_large_batch_matmul_is_exact_on_exact_inputs(M, N, K, gs, bits):
     assert np.array_equal(y, x @ W.dequantize(packed, s, b, gs, bits).T)
 
 
+# scales and biases in tiles of 32 groups x 64 columns: rows of 32, 33, 34, 37, 63 and 65 groups, columns that end inside a tile
+@pytest.mark.parametrize("M,N,K,gs,bits", [(700, 2500, 1024, 32, 4), (700, 2500, 1056, 32, 8), (500, 3009, 1088, 32, 4), (700, 2431, 1184, 32, 4),
+                                           (400, 3000, 4032, 64, 8), (400, 3000, 2080, 32, 8), (333, 3073, 4224, 128, 4)])
+def test_large_batch_matmul_of_many_groups_is_exact_on_exact_inputs(M, N, K, gs, bits):
+    test_large_batch_matmul_is_exact_on_exact_inputs(M, N, K, gs, bits)
+
+
 @pytest.mark.parametrize("bits,gs", [(4, 32), (4, 64), (4, 128), (8, 32), (8, 128)])
 @pytest.mark.parametrize("M,K", [(333, 2048), (80, 4096), (20, 2048 + 32)])  # large batch, small batch, its partial window
 @pytest.mark.parametrize("kind", ["normal", "relu", "mean1"])
