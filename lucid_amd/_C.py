@@ -340,7 +340,7 @@ _STREAM_LAST = None
 def call(name: str, *args):
     """Call an ABI function and raise on a non-zero status.  A ``None`` stream
     argument means the current stream (see ``set_current_stream``)."""
-    fn = getattr(load(), name)
+    fn = getattr(load() if _lib is None else _lib, name)
     if _current_stream is not None and args and args[-1] is None and name in _stream_last():
         args = args[:-1] + (_current_stream,)
     rc = fn(*args)

@@ -99,10 +99,10 @@ def fused_pair(first, relu_between: bool, second, x):
     activation as ONE launch (``lq_dynamic_mlp2_small_f32``: the last block of layer 1 to finish
     reduces the hidden activation's min / max and runs layer 2; ``lq_dynamic_mlp2_small_rows_f32`` where a weight's
     rows are no whole 16 bytes or the hidden layer is wide; ``lq_dynamic_mlp2_rows_f32`` for more than 64 rows), beyond
-    it as two calls with the ReLU in the first one's epilogue, or ``None`` when the shapes or operands do not qualify.  Same bits as calling the modules one
-    after the other.  Per forward, ReLU between: 91-32-58 of 12 rows in one launch 12.6 us (32 in three calls, which is what
-    their host side takes), 64 rows of 784-496-10 17.9 (33), 148 of
-    32-48-15 14.0, 256 of 256-128-64 18.1, 2048 of 32-16-8 24.9 (28.5 in two calls)."""
+    it as two calls with the ReLU in the first one's epilogue, or ``None`` when the shapes or operands do not qualify.
+    Same bits as calling the modules one after the other.  Per forward, ReLU between: 91-32-58 of 12 rows in one launch 12.6
+    us (32 in three calls, which is what their host side takes), 64 rows of 784-496-10 17.9 (33), 148 of 32-48-15 14.0, 256
+    of 256-128-64 18.1, 2048 of 32-16-8 24.9 (28.5 in two calls)."""
     if not (isinstance(first, Linear) and isinstance(second, Linear) and isinstance(x, Tensor)):
         return None
     if x.device != "hip" or x.dtype != T.float32 or x._grid is not None or x._range is not None:
@@ -122,7 +122,7 @@ def fused_pair(first, relu_between: bool, second, x):
     if weight_zero_points(first) is not None or weight_zero_points(second) is not None:
         return None
     if not small:
-        h = first._one_call(x, M, 1) if M else None
+        h = first._one_call(x, M, K1, N1, 1) if M else None
         return None if h is None else second(h)
     taken1, taken2 = _kernel_operands(first, N1, K1), _kernel_operands(second, N2, N1)
     if taken1 is None or taken2 is None:
@@ -202,10 +202,9 @@ class Linear(Module):
         _C.call("lq_d2d_rows", rows.data_ptr, ld, self._buffers["weight_int8"].data_ptr, K, K, N, None)
         return rows, ld
 
-    def _one_call(self, x: Tensor, M: int, relu: int) -> Tensor | None:
+    def _one_call(self, x: Tensor, M: int, K: int, N: int, relu: int) -> Tensor | None:
         """min / max, qparams, codes, GEMM, bias and an optional ReLU behind one call (the same bits as the separate
         operators), or ``None`` where that call does not take the layer."""
-        K, N = self.in_features, self.out_features
         if (weight_zero_points(self) is not None or not _one_call_takes(M, K)
                 or (taken := _kernel_operands(self, N, K)) is None):
             return None
@@ -225,7 +224,7 @@ class Linear(Module):
             else:
                 w, ldw = rows = self._weight_rows()
                 fresh += ((self, "_wrows", rows),)
-        if _one_launch_pays(M, K, N) and (ldw == K or at % 16 == 0):
+        if 1 < M <= 64 and _one_launch_pays(M, K, N) and (ldw == K or at % 16 == 0):
             if ldw == K:
                 _C.call("lq_dynamic_linear_small_f32", at, M, K, w.data_ptr, N, scale.data_ptr, wsum.data_ptr, b, *grid,
                         y.data_ptr, None)
@@ -256,7 +255,7 @@ class Linear(Module):
             raise _C.ShapeMismatch(f"expected last dim {K}, got {x.shape}")
         M = x.numel // K
         if x._range is None and residual is None and activation is None and not track_range:
-            y = self._one_call(x, M, 0)
+            y = self._one_call(x, M, K, N, 0)
             if y is not None:
                 return y
         qd = self.act_qdtype

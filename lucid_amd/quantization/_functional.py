@@ -78,6 +78,19 @@ class _QP:
         return v
 
 
+def _resolve(scale, zero_point, ch_axis, shape):
+    """``(outer, C, inner, scale address, zero point address, on_host, keep)`` of a call.  Device tensors of the right sizes are
+    taken as they are; the class above converts, or refuses, the rest (it costs a call 0.8 us of the host's 7)."""
+    f32 = T.float32
+    if (type(scale) is Tensor and type(zero_point) is Tensor and scale.dtype is f32 and zero_point.dtype is f32
+            and scale.device == "hip" and zero_point.device == "hip"):
+        outer, Cn, inner = _extents(shape, ch_axis)
+        if scale.numel == Cn and zero_point.numel == Cn:
+            return outer, Cn, inner, scale.data_ptr, zero_point.data_ptr, 0, None
+    qp = _QP(scale, zero_point, ch_axis, shape)
+    return qp.outer, qp.C, qp.inner, qp.sp, qp.zp, qp.on_host, qp
+
+
 def _require_hip(t: Tensor, what: str) -> None:
     if not isinstance(t, Tensor):
         raise TypeError(f"{what} expects a Tensor, got {type(t).__name__}")
@@ -96,10 +109,10 @@ def quantize(x: Tensor, scale, zero_point, qdtype: QDtype, ch_axis: int | None =
     storage = T.as_dtype(qdtype.storage)
     if storage not in (T.int8, T.int16):
         raise NotImplementedError(f"quantize to {qdtype!r} (storage {storage.name}) is not on this path")
-    qp = _QP(scale, zero_point, ch_axis, x.shape)
+    outer, Cn, inner, sp, zp, on_host, _keep = _resolve(scale, zero_point, ch_axis, x.shape)
     q = Tensor.empty(x.shape, storage, "hip")
-    _C.call("lq_quantize", x.data_ptr, q.data_ptr, storage.code, 0, qp.outer, qp.C, qp.inner,
-            qp.sp, qp.zp, qp.on_host, qdtype.quant_min, qdtype.quant_max, None)
+    _C.call("lq_quantize", x.data_ptr, q.data_ptr, storage.code, 0, outer, Cn, inner, sp, zp, on_host, qdtype.quant_min,
+            qdtype.quant_max, None)
     return q
 
 
@@ -108,10 +121,9 @@ def dequantize(q: Tensor, scale, zero_point, ch_axis: int | None = None) -> Tens
     _require_hip(q, "dequantize")
     if q.dtype not in (T.int8, T.int16):
         raise _C.DtypeMismatch(f"dequantize expects int8 / int16 codes, got {q.dtype}")
-    qp = _QP(scale, zero_point, ch_axis, q.shape)
+    outer, Cn, inner, sp, zp, on_host, _keep = _resolve(scale, zero_point, ch_axis, q.shape)
     out = Tensor.empty(q.shape, T.float32, "hip")
-    _C.call("lq_dequantize", q.data_ptr, q.dtype.code, 0, out.data_ptr, qp.outer, qp.C, qp.inner,
-            qp.sp, qp.zp, qp.on_host, None)
+    _C.call("lq_dequantize", q.data_ptr, q.dtype.code, 0, out.data_ptr, outer, Cn, inner, sp, zp, on_host, None)
     return out
 
 
@@ -122,10 +134,10 @@ def fake_quantize(x: Tensor, scale, zero_point, quant_min: int, quant_max: int,
     _require_hip(x, "fake_quantize")
     if x.dtype != T.float32:
         raise _C.DtypeMismatch(f"fake_quantize expects float32 input, got {x.dtype}")
-    qp = _QP(scale, zero_point, ch_axis, x.shape)
+    outer, Cn, inner, sp, zp, on_host, _keep = _resolve(scale, zero_point, ch_axis, x.shape)
     out = Tensor.empty(x.shape, T.float32, "hip")
-    _C.call("lq_fake_quantize", x.data_ptr, out.data_ptr, qp.outer, qp.C, qp.inner, qp.sp, qp.zp,
-            qp.on_host, int(quant_min), int(quant_max), None)
+    _C.call("lq_fake_quantize", x.data_ptr, out.data_ptr, outer, Cn, inner, sp, zp, on_host, int(quant_min),
+            int(quant_max), None)
     return out
 
 
