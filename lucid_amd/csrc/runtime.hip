@@ -143,6 +143,10 @@ int workspace(size_t nbytes, hipStream_t stream, void** ptr) {
     return stream_buffer(0, nbytes, size_t(4) << 20, stream, ptr, nullptr);
 }
 
+int call_workspace(size_t nbytes, hipStream_t stream, void** ptr) {
+    return t_capturing_graph ? call_buffer(0, nbytes, stream, ptr) : workspace(nbytes, stream, ptr);
+}
+
 }  // namespace lq
 
 using namespace lq;

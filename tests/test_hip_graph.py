@@ -148,6 +148,41 @@ def test_scratch_growth_after_capture_keeps_the_graph_valid():
     _C.call("lq_stream_destroy", stream)
 
 
+@pytest.mark.parametrize("outer,channels,inner", [(1, 1, 1 << 20), (2048, 16, 64), (30000, 3, 1)])
+def test_partial_ranges_of_a_recorded_call_are_the_graphs_own(outer, channels, inner):
+    """Partial results of a recorded min / max: replays on another stream run beside eager calls on the stream it was
+    recorded on, which use that stream's scratch."""
+    _C.init()
+    rng = np.random.default_rng(channels)
+    shape = (outer, channels, inner)
+    x, z = [L.tensor(rng.standard_normal(shape).astype(np.float32), device="hip") for _ in range(2)]
+    mn, mx, en, ex = [L.Tensor.empty((channels,), L.float32, "hip") for _ in range(4)]
+    streams = [C.c_void_p(), C.c_void_p()]
+    for s in streams:
+        _C.call("lq_stream_create", C.byref(s))
+    gid = C.c_int()
+    _C.call("lq_sync", None)
+    _C.call("lq_graph_begin", streams[0], C.byref(gid))
+    try:
+        _C.call("lq_minmax", x.data_ptr, *shape, mn.data_ptr, mx.data_ptr, streams[0])
+    finally:
+        _C.call("lq_graph_end", streams[0], gid.value)
+    zn, zx = z.numpy().min(axis=(0, 2)), z.numpy().max(axis=(0, 2))
+    for rep in range(3):
+        data = rng.standard_normal(shape).astype(np.float32) * (rep + 1)
+        x.copy_from(data)
+        for _ in range(4):
+            _C.call("lq_minmax", z.data_ptr, *shape, en.data_ptr, ex.data_ptr, streams[0])
+            _C.call("lq_graph_launch", gid.value, streams[1])
+        for s in streams:
+            _C.call("lq_sync", s)
+        assert np.array_equal(mn.numpy(), data.min(axis=(0, 2))) and np.array_equal(mx.numpy(), data.max(axis=(0, 2)))
+        assert np.array_equal(en.numpy(), zn) and np.array_equal(ex.numpy(), zx)
+    _C.call("lq_graph_destroy", gid.value)
+    for s in streams:
+        _C.call("lq_stream_destroy", s)
+
+
 def test_tensor_that_outlives_its_graph_keeps_its_memory():
     """Blocks allocated during capture go back to the pool at destroy only if their owner has
     freed them; a result tensor still alive keeps its block to itself."""
