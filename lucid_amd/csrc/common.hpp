@@ -52,8 +52,8 @@ int workspace(size_t nbytes, hipStream_t stream, void** ptr);
 // Scratch (kinds 4 to 6 and 8) of one call's launches.  While this thread records a graph it is memory of that graph's own:
 // replays may run on any stream, beside each other and beside the stream's eager calls.
 int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr);
-// The same for the general workspace.
-int call_workspace(size_t nbytes, hipStream_t stream, void** ptr);
+// Whether this thread records a graph.
+bool recording_graph();
 // Held by every user of a stream's scratch from before it asks for the buffer until its last launch on it is issued:
 // two threads that use one stream would otherwise interleave launches that hand data to each other, or free
 // a buffer that the other one has outgrown before it is launched on.  One per (device, stream).

@@ -1786,7 +1786,9 @@ int lq_minmax(const float* x, size_t outer, size_t C, size_t inner, float* mn, f
     hipStream_t st = as_stream(stream);
     const auto lock = scratch_lock(st);
     return minmax_launch(x, outer, C, inner, mn, mx, st, ~size_t(0),
-                         [st](size_t nbytes, void** ws) { return call_workspace(nbytes, st, ws); });
+                         [st](size_t nbytes, void** ws) {
+                             return recording_graph() ? call_buffer(5, nbytes, st, ws) : workspace(nbytes, st, ws);
+                         });
 }
 
 int lq_minmax_noalloc(const float* x, size_t outer, size_t C, size_t inner, float* mn, float* mx,

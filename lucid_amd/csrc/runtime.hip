@@ -143,9 +143,7 @@ int workspace(size_t nbytes, hipStream_t stream, void** ptr) {
     return stream_buffer(0, nbytes, size_t(4) << 20, stream, ptr, nullptr);
 }
 
-int call_workspace(size_t nbytes, hipStream_t stream, void** ptr) {
-    return t_capturing_graph ? call_buffer(0, nbytes, stream, ptr) : workspace(nbytes, stream, ptr);
-}
+bool recording_graph() { return t_capturing_graph != 0; }
 
 }  // namespace lq
 
