@@ -928,6 +928,8 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
         const size_t weight = size_t(g.K) * size_t(g.N);
         const int direct = vec_ok ? 1 : weight < (size_t(8) << 20) ? 64 : weight < size_t(20000000) ? 32 : 16;
         path = g.K < 16 ? 3 : (g.M <= direct && g.range == nullptr ? 2 : 1);
+        // (up to 16 rows a shape asked for is not looked at)
+        if (vec_ok && g.M <= 16 && g.range == nullptr) tile_config = 25;
         if (path == 1 && !vec_ok) {
             const int ld = (g.K + 63) / 64 * 64;
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;

@@ -66,6 +66,16 @@ def test_ragged_rows_of_a_large_weight_exact(M, N, K, tile_config):
     assert np.array_equal(acc, O.igemm(a, w))
 
 
+@pytest.mark.parametrize("tile_config", [77, 15, 13, 17, 9 | 0x200, 0x200, 23 | 0x300, 3 << 16])
+@pytest.mark.parametrize("M,N,K", [(2, 33, 48), (16, 130, 1040), (1, 7, 64)])
+def test_up_to_16_rows_are_free_of_tile_config(M, N, K, tile_config):
+    """Shapes are for more rows: an unknown one, one for convolutions or one that K does not suit is no error here."""
+    rng = np.random.default_rng(M + N + K)
+    a, w = codes(rng, (M, K)), codes(rng, (N, K))
+    acc = _ops.qlinear_i8(hip(a), hip(w), out_mode=_ops.OUT_ACC_I32, tile_config=tile_config).numpy()
+    assert np.array_equal(acc, O.igemm(a, w))
+
+
 @pytest.mark.parametrize("cfg", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12])
 @pytest.mark.parametrize("M,N,K", [(256, 256, 128), (300, 260, 144), (129, 77, 784), (513, 1000, 576),
                                    (2048, 512, 4096), (1, 16, 16), (700, 130, 64)])
