@@ -752,7 +752,9 @@ typedef struct {
                               leftover tiles of the last round only; bits 16..30
                               = number of leading 256-column tiles computed with
                               256x256 tiles, the remaining columns as a problem of
-                              their own (0 = no split)                          */
+                              their own (0 = no split).  Not looked at where other
+                              kernels serve the call: force_path 0, no range and up to 16
+                              rows (64 where K % 16 != 0 or an operand is unaligned) */
     const float* residual; /* optional float32 [M, ldr] added after the activation:
                               out = act(y) + residual (x + linear(...), the
                               residual joins of a transformer block,

@@ -928,8 +928,8 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
         const size_t weight = size_t(g.K) * size_t(g.N);
         const int direct = vec_ok ? 1 : weight < (size_t(8) << 20) ? 64 : weight < size_t(20000000) ? 32 : 16;
         path = g.K < 16 ? 3 : (g.M <= direct && g.range == nullptr ? 2 : 1);
-        // (up to 16 rows a shape asked for is not looked at)
-        if (vec_ok && g.M <= 16 && g.range == nullptr) tile_config = 25;
+        // a shape asked for is for calls that have no other kernel
+        if (g.range == nullptr && g.M <= (vec_ok ? 16 : 64)) tile_config = vec_ok ? 25 : 0;
         if (path == 1 && !vec_ok) {
             const int ld = (g.K + 63) / 64 * 64;
             const size_t a_bytes = size_t(g.M) * ld, w_bytes = size_t(g.N) * ld;
@@ -948,7 +948,7 @@ int run_gemm(const GemmArgs& g_in, int force_path, int tile_config, hipStream_t 
                                pa, pa + a_bytes);
             LQ_CHECK_LAUNCH("pad_rows");
             g.a = pa, g.w = pa + a_bytes, g.K = ld;
-            return run_tile_kernel(g, 0, 1, g.M > 64 ? tile_config : 0, st);  // (a shape asked for was never looked at up to 64 rows)
+            return run_tile_kernel(g, 0, 1, tile_config, st);
         }
     }
     // only the tile kernel keeps the range of what it writes

@@ -76,6 +76,22 @@ def test_up_to_16_rows_are_free_of_tile_config(M, N, K, tile_config):
     assert np.array_equal(acc, O.igemm(a, w))
 
 
+@pytest.mark.parametrize("M,K", [(8, 64), (16, 1000), (17, 99), (64, 1000), (65, 250)])
+def test_a_kept_range_follows_tile_config(M, K):
+    """Products that keep the range of their output run on the tiles asked for at any number of rows, aligned or not."""
+    rng = np.random.default_rng(M + K)
+    a, w = codes(rng, (M, K)), codes(rng, (70, K))
+    kw = dict(a_scale=hip(np.float32(0.01)), w_scale=hip(np.full(70, 0.002, np.float32)), out_mode=_ops.OUT_F32)
+    want = _ops.qlinear_i8(hip(a), hip(w), **kw).numpy()
+    rb = L.Tensor.empty((_C.range_buffer_words(),), L.float32, "hip")
+    for cfg in (5, 9):
+        y = _ops.qlinear_i8(hip(a), hip(w), **kw, range_buf=rb, tile_config=cfg).numpy()
+        assert _C.load().lq_last_tile_config() & 0xff == cfg
+        assert np.array_equal(y.view(np.uint32), want.view(np.uint32))
+    with pytest.raises(ValueError, match="tile_config 77"):
+        _ops.qlinear_i8(hip(a), hip(w), **kw, range_buf=rb, tile_config=77)
+
+
 @pytest.mark.parametrize("cfg", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12])
 @pytest.mark.parametrize("M,N,K", [(256, 256, 128), (300, 260, 144), (129, 77, 784), (513, 1000, 576),
                                    (2048, 512, 4096), (1, 16, 16), (700, 130, 64)])
