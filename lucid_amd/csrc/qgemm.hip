@@ -157,17 +157,19 @@ bool pp_applies(const GemmArgs& g, int conv, int groups) {
 // the ping-pong kernel, with the tile width that wastes less of the 256 CUs: the cost of a
 // shape is its rounds of 256 tiles times the tile's area.  Otherwise 128 x 256 tiles keep two
 // blocks per CU busy; narrower tiles when N is small or when the wide ones would leave most
-// of the CUs without work.
-int heuristic_tile_shape(const GemmArgs& g, int conv, int groups) {
+// of the CUs without work.  `shared`: of the shapes whose tiles several blocks can share (schedules 2 and 3).
+int heuristic_tile_shape(const GemmArgs& g, int conv, int groups, bool shared) {
     const long mt128 = (g.M + 127) / 128;
-    if (const int ks = ks_shape(g, conv, groups)) return ks;
-    // an image of at most four channels with a block's worth of 16 x 16 boxes for every CU
-    if (g.M >= 65536 && conv_few_applies(g, conv, groups)) return 20;
+    if (!shared) {
+        if (const int ks = ks_shape(g, conv, groups)) return ks;
+        // an image of at most four channels with a block's worth of 16 x 16 boxes for every CU
+        if (g.M >= 65536 && conv_few_applies(g, conv, groups)) return 20;
+    }
     // far fewer 128 x 128 tiles than CUs (a small batch in the late stages of a network): 64 x 64
     // tiles, four blocks per CU, with 128-byte k steps when K is long (plain and 2-d only)
     if (mt128 * ((g.N + 127) / 128) * groups < 128) return (g.K >= 1024 && conv != 2) ? 10 : 9;
     // (not with a GELU: its vector arithmetic needs a second block on the CU to overlap with)
-    if (pp_applies(g, conv, groups) && g.K >= 512 && !g.gelu) {
+    if (!shared && pp_applies(g, conv, groups) && g.K >= 512 && !g.gelu) {
         const long tm = (g.M + 255) / 256;
         const long t352 = tm * ((g.N + 351) / 352), t256 = tm * ((g.N + 255) / 256);
         // at least half a round of tiles, or the four-wavefront shapes below cover the chip better
@@ -183,6 +185,9 @@ int heuristic_tile_shape(const GemmArgs& g, int conv, int groups) {
     if (g.N <= 128 || mt128 * ((g.N + 255) / 256) * groups < 256) return 5;
     return 4;
 }
+
+// Whether a tile of the shape can be shared between blocks.
+bool can_share_tiles(int cfg) { return cfg <= 12; }
 
 int launch_tile_cfg(const GemmArgs& g, int conv, int groups, int tile_config, hipStream_t st);
 thread_local int t_last_tile_config = 0;  // what the last tile-kernel launch of this thread resolved to
@@ -325,7 +330,7 @@ int tuned_tile_shape(const GemmArgs& g, int conv, int groups, hipStream_t st, in
             return LQ_OK;
         }
     }
-    int fallback = heuristic_tile_shape(g, conv, groups);
+    int fallback = heuristic_tile_shape(g, conv, groups, false);
     *cfg_out = fallback;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     LQ_HIP(hipStreamIsCapturing(st, &capturing));
@@ -436,7 +441,7 @@ int tuned_tile_shape(const GemmArgs& g, int conv, int groups, hipStream_t st, in
     return LQ_OK;
 }
 
-// tile_config: low byte = tile shape (0 = choose, 1..9 = a specific one), next
+// tile_config: low byte = tile shape (0 = choose, 1..25 = a specific one), next
 // byte = schedule (0 = choose, 1 = block per tile, 2 = stream-K, 3 = stream-K over
 // the leftover tiles only), bits 16..30 = number of leading 256-column tiles given to
 // shape 1 with the remaining columns tuned separately (0 = no split).
@@ -450,6 +455,7 @@ int launch_tile_cfg(const GemmArgs& g, int conv, int groups, int tile_config, hi
         if (rc) return rc;
         cfg = tuned & 0xff;
         if (schedule == 0) schedule = (tuned >> 8) & 0xff;
+        if (schedule > 1 && !can_share_tiles(cfg)) cfg = heuristic_tile_shape(g, conv, groups, true);
         a_tiles = tuned >> 16;
     }
     if (a_tiles > 0) {

@@ -86,6 +86,20 @@ def test_gather_exact_at_every_tile_shape(case, cfg):
         assert np.array_equal(got, exp), schedule
 
 
+@pytest.mark.parametrize("schedule", [2, 3])
+@pytest.mark.parametrize("case", TAP_CASES)
+def test_gather_exact_with_a_schedule_alone(case, schedule):
+    """A schedule without a shape: the shape chosen is one that has that schedule."""
+    B, H, W, Cin, Cout, KH, KW, st, pad, dil, groups = case
+    rng = np.random.default_rng(sum(case[:7]))
+    x, w = codes(rng, (B, H, W, Cin)), codes(rng, (Cout, KH, KW, Cin // groups))
+    geo = dict(stride=st, pad=pad, dilation=dil, groups=groups)
+    exp = O.qconv2d(x, w, 91, 1.0, np.ones(Cout, np.float32), out_mode=O.OUT_ACC_I32, **geo)
+    got = _ops.qconv2d_i8(hip(x), hip(w), a_zp=91, out_mode=_ops.OUT_ACC_I32, path=IMPLICIT, tile_config=schedule << 8,
+                          **geo).numpy()
+    assert np.array_equal(got, exp)
+
+
 @pytest.mark.parametrize("cfg", [0, 1, 3, 5, 8, 10, 12])
 @pytest.mark.parametrize("groups,og", [(2, 66), (2, 130), (4, 33), (3, 260), (4, 65)])
 def test_groups_that_begin_between_two_vectors(groups, og, cfg):

@@ -134,6 +134,19 @@ def test_stream_k_schedule_exact(cfg, M, N, K):
     assert np.array_equal(got.view(np.uint16), exp.view(np.uint16))
 
 
+@pytest.mark.parametrize("schedule", [2, 3])
+@pytest.mark.parametrize("M,N,K", [(49, 512, 4608), (17, 40, 1040), (300, 64, 2048), (2048, 2048, 512)])
+def test_schedule_alone_exact(M, N, K, schedule):
+    """A schedule without a shape: the shape chosen is one that has that schedule."""
+    rng = np.random.default_rng(M + N + K)
+    a, w = codes(rng, (M, K)), codes(rng, (N, K))
+    ad, wd, ref = hip(a), hip(w), O.igemm(a, w)
+    for _ in range(2):
+        acc = _ops.qlinear_i8(ad, wd, out_mode=_ops.OUT_ACC_I32, tile_config=schedule << 8).numpy()
+        assert np.array_equal(acc, ref)
+        assert _C.load().lq_last_tile_config() >> 8 == schedule
+
+
 @pytest.mark.parametrize("cfg,M,N,K", [(4, 2048, 11008, 512), (5, 3000, 3000, 256), (6, 4096, 2500, 320),
                                        (3, 4096, 5000, 256), (4, 2100, 11000, 400), (1, 2048, 11008, 192)])
 def test_hybrid_schedule_exact(cfg, M, N, K):
