@@ -303,10 +303,6 @@ bool autotune_enabled() {
 }
 
 int tuned_tile_shape(const GemmArgs& g, int conv, int groups, hipStream_t st, int* cfg_out) {
-    if (!conv && g.M <= 16 && ks_applies(g, conv)) {  // a stream of the weight: nothing to choose from
-        *cfg_out = ks_shape(g, conv, groups);
-        return LQ_OK;
-    }
     TuneKey key;
     std::memset(&key, 0, sizeof(key));
     key.M = g.M, key.N = g.N, key.K = g.K, key.mode = g.out_mode, key.conv = conv, key.groups = groups;
@@ -341,7 +337,9 @@ int tuned_tile_shape(const GemmArgs& g, int conv, int groups, hipStream_t st, in
     // once per timing launch)
     const bool in_place = (g.residual && static_cast<const void*>(g.residual) == g.out) ||
                           (g.join_q && static_cast<const void*>(g.join_q) == g.out);
-    if (!autotune_enabled() || capturing != hipStreamCaptureStatusNone || ops < 5e8 || in_place) return LQ_OK;
+    // up to 16 rows are a stream of the weight: nothing to choose from
+    const bool stream = !conv && g.M <= 16 && ks_applies(g, conv);
+    if (!autotune_enabled() || capturing != hipStreamCaptureStatusNone || ops < 5e8 || in_place || stream) return LQ_OK;
 
     // candidates are whole tile_config values (shape | schedule << 8)
     int cands[24], n = 0;

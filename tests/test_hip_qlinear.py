@@ -971,6 +971,25 @@ def test_tuning_choices_export_and_import():
         _C.call("lq_tune_import", b"lq-tune-1 1 2 3\n", None)
 
 
+@pytest.mark.parametrize("kept", [False, True])
+def test_imported_choices_decide_up_to_16_rows(kept):
+    """A line of the table is followed where the tile kernels were asked for or a range is kept, whatever the rows."""
+    rng = np.random.default_rng(4)
+    M, N, K = (11, 111, 272) if kept else (12, 111, 272)
+    a, w = codes(rng, (M, K)), codes(rng, (N, K))
+    kw = dict(a_scale=hip(np.float32(0.01)), w_scale=hip(np.full(N, 0.002, np.float32)), out_mode=_ops.OUT_F32)
+    want = _ops.qlinear_i8(hip(a), hip(w), **kw).numpy()
+    if kept:
+        kw["range_buf"] = L.Tensor.empty((_C.range_buffer_words(),), L.float32, "hip")
+    else:
+        kw["path"] = TILE
+    key = [M, N, K, _ops.OUT_F32, 0, 1] + [0] * 14 + [32 if kept else 0]  # (the last: a range is kept)
+    _C.call("lq_tune_import", f"lq-tune-1 {' '.join(map(str, key))} {9 | 0x100}\n".encode(), None)
+    got = _ops.qlinear_i8(hip(a), hip(w), **kw).numpy()
+    assert _C.load().lq_last_tile_config() == 9 | 0x100
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_first_calls_from_two_threads():
     """Two threads of a fresh process make their first launches at once (kernel attributes, the
     padding table and the tuner's table are set up on first use): both get right results."""
