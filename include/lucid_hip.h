@@ -112,8 +112,9 @@ int lq_event_elapsed_ms(lq_event start, lq_event stop, float* ms);
  * (a created stream, not the default one), then replay it with one launch -
  * for launch-bound inference loops (a quantized ResNet-50 forward is ~75 short
  * kernels).  Memory allocated during capture stays reserved for the graph until
- * lq_graph_destroy.  The library's scratch of `stream` is part of what is recorded (split-K slabs, partial
- * min / max, convolution patches, decoded or prepared weight-only operands): do not replay a graph beside another that was
+ * lq_graph_destroy, and so do partial results of its calls (split-K slabs and counters, partial min / max, codes, padded
+ * rows).  The rest of the library's scratch of `stream` is part of what is recorded (convolution patches, packed images, raw
+ * accumulators of affine weights, decoded or prepared weight-only operands): do not replay a graph with such calls beside another that was
  * captured on the same stream, or beside eager calls on that stream.  No counterpart in Lucid (its Metal backend batches lazily
  * through MLX instead). */
 int lq_graph_begin(lq_stream stream, int* graph_id);
@@ -489,7 +490,7 @@ int lq_dynamic_linear_f32(const float* x, int M, int K, const int8_t* w, int ldw
 
 /* Two dynamic-quantized Linears in ONE launch: y = L2(act1(L1(x))) with each layer as
  * lq_dynamic_linear_small_f32 computes it (the hidden activation's min / max, qparams and codes
- * included: the blocks of layer 1 pass their tiles and ranges through the stream's scratch and
+ * included: the blocks of layer 1 pass their tiles and ranges through the stream's scratch (in a recording the graph's) and
  * the last of them to arrive runs layer 2) and relu1 / relu2 the optional ReLU behind each.  x [M, K1] float32, w1 [N1, K1], w2 [N2, N1] int8 codes with their
  * per-row scales, code sums and float32 biases (or NULL); out [M, N2] float32.  M <= 64,
  * K1 % 16 == 0 and <= 1024, N1 % 16 == 0 and <= 256, N2 <= 64; anything else

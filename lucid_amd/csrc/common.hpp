@@ -41,9 +41,12 @@ int hip_fail(hipError_t e, const char* what);
 // sums: one buffer per (device, stream, kind), grown on demand and never shrunk, so calls
 // on different streams do not share scratch and calls on one stream are ordered by it.
 // A buffer that is outgrown stays allocated while any captured graph exists (its address
-// may be baked into the graph).  `fresh` reports that the buffer was (re)allocated by
-// this request and holds no defined contents.
-int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, bool* fresh);
+// may be baked into the graph).  `fresh`: the bytes of the buffer where nothing has set it up yet, else 0; the caller
+// does so on the stream in front of its launch.  What is issued on a stream under capture does not count: a
+// replay comes after the eager calls before it, if there ever is one.
+int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, size_t* fresh);
+// The same, but while this thread records a graph a buffer of that graph, kept over the calls that it records on the stream.
+int kept_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, size_t* fresh);
 // kind 0: the general workspace (at least 4 MiB); 1 / 2: stream-K counters / slabs;
 // 3: raw accumulators and operand sums of a layer with affine weights; 4: padded copies of ragged GEMM operands;
 // 5: the range slots of a dynamic quantization; 6: the codes and qparams of a dynamic Linear's activation;
@@ -58,7 +61,7 @@ bool recording_graph();
 // two threads that use one stream would otherwise interleave launches that hand data to each other, or free
 // a buffer that the other one has outgrown before it is launched on.  One per (device, stream).
 std::unique_lock<std::recursive_mutex> scratch_lock(hipStream_t stream);
-// Split-K scratch of one stream (the caller holds its scratch_lock): arrival counters (zero between launches: the finisher of a
+// Split-K scratch of one stream, or of the graph being recorded there (the caller holds its scratch_lock): arrival counters (zero between launches: the finisher of a
 // tile resets its counter) and slabs for the partial results, whose layout the kernel defines.
 struct SkScratch {
     int* counters = nullptr;

@@ -620,9 +620,8 @@ int lq_qconv2d_i8(const lq_qconv2d_args* p, lq_stream stream) {
         const size_t sum_bytes = (M * p->groups * 4 + 255) / 256 * 256;
         const size_t ones_bytes = size_t(p->groups) * K;
         void* tmp = nullptr;
-        bool fresh = false;
         const auto lock = scratch_lock(st);
-        int rc = stream_buffer(3, acc_bytes + sum_bytes + ones_bytes, 0, st, &tmp, &fresh);
+        int rc = stream_buffer(3, acc_bytes + sum_bytes + ones_bytes, 0, st, &tmp, nullptr);
         if (rc) return rc;
         int32_t* acc = static_cast<int32_t*>(tmp);
         int32_t* asum = reinterpret_cast<int32_t*>(static_cast<char*>(tmp) + acc_bytes);
@@ -824,9 +823,8 @@ int lq_qconv3d_i8(const lq_qconv3d_args* p, lq_stream stream) {
         const size_t sum_bytes = (M * p->groups * 4 + 255) / 256 * 256;
         const size_t ones_bytes = size_t(p->groups) * K;
         void* tmp = nullptr;
-        bool fresh = false;
         const auto lock = scratch_lock(st);
-        int rc = stream_buffer(3, acc_bytes + sum_bytes + ones_bytes, 0, st, &tmp, &fresh);
+        int rc = stream_buffer(3, acc_bytes + sum_bytes + ones_bytes, 0, st, &tmp, nullptr);
         if (rc) return rc;
         int32_t* acc = static_cast<int32_t*>(tmp);
         int32_t* asum = reinterpret_cast<int32_t*>(static_cast<char*>(tmp) + acc_bytes);

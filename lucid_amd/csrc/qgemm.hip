@@ -30,22 +30,17 @@
 using namespace lq;
 
 namespace lq {
-// The stream's stream-K scratch, grown to the requested sizes: arrival counters (zero
-// between launches: freshly allocated ones are cleared by a kernel on the stream, which a
-// graph capture records like any other launch) and the accumulator slabs.
+// The stream's stream-K scratch, grown to the requested sizes: arrival counters (zero between launches: new ones are cleared
+// by a kernel on the stream) and the accumulator slabs.  A graph that this thread records has its own of either for each
+// stream, with the clear in front of the first launch that counts on it: replays then share nothing with eager calls.
 int sk_scratch(size_t counters, size_t slab_bytes, hipStream_t st, SkScratch* out) {
     void* c = nullptr;
-    bool fresh = false;
-    int rc = stream_buffer(1, counters * sizeof(int), size_t(65536) * sizeof(int), st, &c, &fresh);
+    size_t fresh = 0;
+    int rc = kept_buffer(1, counters * sizeof(int), size_t(65536) * sizeof(int), st, &c, &fresh);
+    if (!rc) rc = lq_fill_bytes(c, 0, fresh, reinterpret_cast<lq_stream>(st));
     if (rc) return rc;
-    if (fresh) {
-        const size_t bytes = counters * sizeof(int) < size_t(65536) * sizeof(int) ? size_t(65536) * sizeof(int)
-                                                                                : counters * sizeof(int);
-        rc = lq_fill_bytes(c, 0, bytes, reinterpret_cast<lq_stream>(st));
-        if (rc) return rc;
-    }
     void* s = nullptr;
-    rc = stream_buffer(2, slab_bytes, 0, st, &s, nullptr);
+    rc = kept_buffer(2, slab_bytes, 0, st, &s, nullptr);
     if (rc) return rc;
     out->counters = static_cast<int*>(c);
     out->slabs = static_cast<int32_t*>(s);
@@ -1166,10 +1161,9 @@ int lq_qlinear_i8(const lq_qlinear_args* p, lq_stream stream) {
                    "qlinear_i8: K = %d overflows the int32 accumulator with affine weights", p->K);
         hipStream_t st = as_stream(stream);
         void* tmp = nullptr;
-        bool fresh = false;
         const auto lock = scratch_lock(st);
         const size_t acc_bytes = (size_t(p->M) * p->N * 4 + 255) / 256 * 256;
-        int rc = stream_buffer(3, acc_bytes + size_t(p->M) * 4, 0, st, &tmp, &fresh);
+        int rc = stream_buffer(3, acc_bytes + size_t(p->M) * 4, 0, st, &tmp, nullptr);
         if (rc) return rc;
         int32_t* acc = static_cast<int32_t*>(tmp);
         int32_t* asum = reinterpret_cast<int32_t*>(static_cast<char*>(tmp) + acc_bytes);

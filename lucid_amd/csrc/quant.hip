@@ -1501,7 +1501,8 @@ int quantize_tensor(const float* x, size_t n, unsigned cols, unsigned ld, int sy
     if (blocks > 1 && blocks <= size_t(kExchange)) {
         if (const int rc = exchange_blocks(&most)) return rc;
     }
-    bool exchange = blocks <= size_t(most), fresh = false;
+    bool exchange = blocks <= size_t(most);
+    size_t fresh = 0;
     std::unique_lock<std::recursive_mutex> lock;
     if (blocks > 1) {
         lock = scratch_lock(st);

@@ -55,6 +55,7 @@ std::recursive_mutex g_rt_mutex;
 struct StreamBuf {
     void* ptr = nullptr;
     size_t size = 0;
+    bool set_up = false;  // what its first user puts into it has been issued to run
 };
 struct BufKey {
     int dev;
@@ -74,6 +75,7 @@ struct GraphRec {
     hipGraph_t graph = nullptr;      // the captured template, kept until the exec is destroyed
     hipGraphExec_t exec = nullptr;   // null while capturing or after a failed end
     std::vector<std::pair<int, void*>> blocks;  // (device, block) allocated during capture
+    std::map<BufKey, StreamBuf> bufs;           // scratch of the recorded calls, in such blocks
     bool capturing = false;          // between a successful begin and its end / destroy
 };
 std::unordered_map<int, GraphRec> g_graphs;
@@ -93,22 +95,28 @@ void drain_retired() {
 }
 }  // namespace
 
-int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, bool* fresh) {
+int stream_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, size_t* fresh) {
     int dev = 0;
     LQ_HIP(hipGetDevice(&dev));
     LQ_REQUIRE(dev >= 0 && dev < kMaxDevices, LQ_ERR_DEVICE, "device index %d out of range", dev);
     std::lock_guard<std::recursive_mutex> lock(g_rt_mutex);
     StreamBuf& b = g_bufs[BufKey{dev, stream, kind}];
-    if (fresh) *fresh = false;
     if (b.size < nbytes || b.ptr == nullptr) {
         const size_t want = nbytes < min_bytes ? min_bytes : nbytes;
         void* p = nullptr;
         LQ_HIP(hipMalloc(&p, want));  // legal during a relaxed capture; no synchronisation here
         if (b.ptr) g_retired.push_back(b.ptr);
-        b.ptr = p;
-        b.size = want;
-        if (fresh) *fresh = true;
+        b = StreamBuf{p, want, false};
         drain_retired();
+    }
+    if (fresh) {
+        *fresh = b.set_up ? 0 : b.size;
+        if (!b.set_up) {
+            // (what goes into a recording runs with its replays, after eager calls of the stream that come before them)
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            if (stream) LQ_HIP(hipStreamIsCapturing(stream, &capturing));  // (see lq_stream_is_capturing)
+            b.set_up = capturing == hipStreamCaptureStatusNone;
+        }
     }
     *ptr = b.ptr;
     return LQ_OK;
@@ -137,6 +145,26 @@ int call_buffer(int kind, size_t nbytes, hipStream_t stream, void** ptr) {
     // pinned to the graph by the allocator, and given back with it
     const int rc = lq_alloc(ptr, nbytes);
     return rc ? rc : lq_free(*ptr);
+}
+
+int kept_buffer(int kind, size_t nbytes, size_t min_bytes, hipStream_t stream, void** ptr, size_t* fresh) {
+    if (!t_capturing_graph) return stream_buffer(kind, nbytes, min_bytes, stream, ptr, fresh);
+    int dev = 0;
+    LQ_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::recursive_mutex> lock(g_rt_mutex);
+    StreamBuf& b = g_graphs[t_capturing_graph].bufs[BufKey{dev, stream, kind}];
+    const bool grown = b.size < nbytes || b.ptr == nullptr;
+    if (grown) {
+        const size_t want = nbytes < min_bytes ? min_bytes : nbytes;
+        void* p = nullptr;
+        int rc = lq_alloc(&p, want);  // pinned to the graph, and given back with it
+        if (!rc) rc = lq_free(p);
+        if (rc) return rc;
+        b = StreamBuf{p, want, true};
+    }
+    if (fresh) *fresh = grown ? b.size : 0;
+    *ptr = b.ptr;
+    return LQ_OK;
 }
 
 int workspace(size_t nbytes, hipStream_t stream, void** ptr) {

@@ -183,6 +183,122 @@ def test_partial_ranges_of_a_recorded_call_are_the_graphs_own(outer, channels, i
         _C.call("lq_stream_destroy", s)
 
 
+@pytest.mark.parametrize("recorder", ["graph", "hip"])
+def test_arrival_counters_of_a_first_call_that_is_recorded(recorder):
+    """A product that splits K is recorded before its stream was ever used: the clear of the arrival counters is part of
+    what is recorded, and eager calls on that stream come before any replay.  Recorded by the library, counters and partial
+    sums are the graph's own; recorded by the program itself, the stream's."""
+    _C.init()
+    rng = np.random.default_rng(1)
+    M, N, K, gs = 16, 512, 4096, 64
+    x = L.tensor(rng.standard_normal((M, K)).astype(np.float32), device="hip")
+    packed = L.tensor(rng.integers(0, 2**32, (N, K // 4), dtype=np.uint32).view(np.int32), device="hip")
+    sc, bi = [L.tensor(rng.standard_normal((N, K // gs)).astype(np.float32), device="hip") for _ in range(2)]
+    hip, unset = _C.load(), np.full((M, N), np.nan, np.float32)
+
+    def matmul(out, stream):
+        _C.call("lq_wq_matmul", x.data_ptr, packed.data_ptr, sc.data_ptr, bi.data_ptr, M, N, K, gs, 8, out.data_ptr, stream)
+
+    outs = [L.tensor(unset, device="hip") for _ in range(4)]
+    matmul(outs[3], None)
+    want = outs[3].numpy()
+    stream = C.c_void_p()
+    _C.call("lq_stream_create", C.byref(stream))
+    _C.call("lq_sync", None)
+    graphs = []
+    for i in (0, 1):
+        if recorder == "graph":
+            gid, used = C.c_int(), _stats()[0]
+            _C.call("lq_graph_begin", stream, C.byref(gid))
+            matmul(outs[i], stream)
+            _C.call("lq_graph_end", stream, gid)
+            graphs.append(gid)
+            assert _stats()[0] - used >= 4 * 65536 + 4 * M * N * 4  # counters, the partial sums of four ranges of K
+        else:
+            graph, run = C.c_void_p(), C.c_void_p()
+            assert hip.hipStreamBeginCapture(stream, 2) == 0  # relaxed
+            matmul(outs[i], stream)
+            assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+            graphs.append((graph, run))
+    for rep in range(3):
+        for i in (None, 1, 0):
+            out = outs[2 if i is None else i]
+            out.copy_from(unset)
+            _C.call("lq_sync", None)
+            if i is None:
+                matmul(out, stream)
+            elif recorder == "graph":
+                _C.call("lq_graph_launch", graphs[i], stream)
+            else:
+                assert hip.hipGraphLaunch(graphs[i][1], stream) == 0
+            _C.call("lq_sync", stream)
+            assert np.array_equal(out.numpy(), want), (rep, i)
+    for g in graphs:
+        if recorder == "graph":
+            _C.call("lq_graph_destroy", g)
+        else:
+            hip.hipGraphExecDestroy(g[1]), hip.hipGraphDestroy(g[0])
+    _C.call("lq_stream_destroy", stream)
+
+
+@pytest.mark.parametrize("call", ["wq_matmul", "mlp2"])
+def test_split_sums_of_a_recorded_call_are_the_graphs_own(call):
+    """Counters, partial sums and a hidden activation of a recorded call: replays on another stream run beside eager calls
+    on the stream it was recorded on."""
+    _C.init()
+    rng = np.random.default_rng(3)
+    M, K, N, H = 128, 400, 24, 130
+
+    def dev(a):
+        return L.tensor(a, device="hip")
+
+    xs = [dev((rng.standard_normal((M, K if call == "mlp2" else 4096)) * f).astype(np.float32)) for f in (1, 9)]
+    outs = [L.Tensor.empty((M, 512), L.float32, "hip") for _ in range(4)]
+    if call == "mlp2":
+        w1, w2 = np.zeros((H, 400), np.int8), np.zeros((N, 144), np.int8)  # rows of 16 bytes, zeros past the codes
+        w1[:, :K], w2[:, :H] = rng.integers(-127, 128, (H, K)), rng.integers(-127, 128, (N, H))
+        ops = [dev(v) for v in (w1, rng.uniform(1e-3, 1e-2, H).astype(np.float32), w1.sum(1, dtype=np.int32),
+                                w2, rng.uniform(1e-3, 1e-2, N).astype(np.float32), w2.sum(1, dtype=np.int32))]
+
+        def run(x, out, stream):
+            p = [t.data_ptr for t in ops]
+            _C.call("lq_dynamic_mlp2_rows_f32", x.data_ptr, M, K, p[0], 400, H, p[1], p[2], None, 1, p[3], 144, N, p[4], p[5],
+                    None, 0, 0, 0, 255, 0, 1e-8, -128, out.data_ptr, stream)
+    else:
+        ops = [dev(rng.integers(0, 2**32, (512, 1024), dtype=np.uint32).view(np.int32)),
+               *[dev(rng.standard_normal((512, 64)).astype(np.float32)) for _ in range(2)]]
+
+        def run(x, out, stream):
+            _C.call("lq_wq_matmul", x.data_ptr, *[t.data_ptr for t in ops], 16, 512, 4096, 64, 8, out.data_ptr, stream)
+
+    size = M * N if call == "mlp2" else 16 * 512
+    for i in (0, 1):
+        run(xs[i], outs[2 + i], None)
+    want = [outs[2 + i].numpy().ravel()[:size] for i in (0, 1)]
+    assert not np.array_equal(*want)
+    streams = [C.c_void_p(), C.c_void_p()]
+    for s in streams:
+        _C.call("lq_stream_create_nonblocking", C.byref(s))
+    run(xs[1], outs[1], streams[0])
+    _C.call("lq_sync", streams[0])
+    gid = C.c_int()
+    _C.call("lq_graph_begin", streams[0], C.byref(gid))
+    run(xs[0], outs[0], streams[0])
+    _C.call("lq_graph_end", streams[0], gid)
+    for rep in range(20):
+        for _ in range(10):
+            _C.call("lq_graph_launch", gid, streams[1])
+            run(xs[1], outs[1], streams[0])
+        for s in streams:
+            _C.call("lq_sync", s)
+        for i in (0, 1):
+            assert np.array_equal(outs[i].numpy().ravel()[:size], want[i]), (rep, i)
+    _C.call("lq_graph_destroy", gid)
+    for s in streams:
+        _C.call("lq_stream_destroy", s)
+
+
 def test_tensor_that_outlives_its_graph_keeps_its_memory():
     """Blocks allocated during capture go back to the pool at destroy only if their owner has
     freed them; a result tensor still alive keeps its block to itself."""

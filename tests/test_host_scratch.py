@@ -6,9 +6,9 @@ import re
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lucid_amd", "csrc")
-USE = re.compile(r"\b(workspace|stream_buffer|call_buffer|sk_scratch)\(")
+USE = re.compile(r"\b(workspace|stream_buffer|kept_buffer|call_buffer|sk_scratch)\(")
 # what defines the buffers (a caller of sk_scratch holds the lock for it), and the start-up call of one thread
-DEFINES = {("runtime.hip", "stream_buffer"), ("runtime.hip", "call_buffer"), ("runtime.hip", "workspace"),
+DEFINES = {("runtime.hip", "stream_buffer"), ("runtime.hip", "kept_buffer"), ("runtime.hip", "call_buffer"), ("runtime.hip", "workspace"),
            ("runtime.hip", "lq_init"), ("qgemm.hip", "sk_scratch")}
 
 
