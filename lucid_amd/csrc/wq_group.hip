@@ -660,26 +660,36 @@ __global__ __launch_bounds__(64 * wq_waves(KP)) __attribute__((amdgpu_waves_per_
 
 
 // Tiles of 16 weight rows per wavefront and parts of a block's k range.  Four parts of 1024 k (a CU per block) with as many
-// tiles as give every block a CU at once; where the blocks are too many for that, one part of 512 k and two tiles, of which a CU
-// has two blocks, one starting or adding slabs while the other streams.  us of 1 / 2 / 3 tiles of four parts, and of one part of
-// two: 16 x 4096 x 4096 int8 groups of 64 (256 / 128 / 88 blocks) 11.6 / 12.0 / 14.8, 13.6 (128); 16 x 11008 x 4096 int8 of 64
-// (688 / 344 / 232) 26.9 / 24.0 / 18.4, 20.5 (344); the same int4 24.0 / 21.6 / 16.8, 19.4; 64 x 4096 x 4096 int4 of 64
-// (1024 / 512 / 352) 30.4 / 22.4 / 25.9, 19.6 (512); 33 x 2048 x 4096 int4 of 32 (384 / 192 / 132) 16.8 / 12.5 / 15.6,
-// 14.1 (192); 3 x 7450 x 7808 int4 of 64 (936 / 472 / 312) 31.2 / 25.3 / 29.6, 25.0 (480); 20 x 388 x 448 int8 of 32
-// 5.9 / 7.9 / 9.6, 9.7.  The costs below follow those, in us behind the first 3.
+// tiles as give every block a CU at once; where the blocks are too many for that, one part of 512 k, of which a CU
+// has two blocks, one starting or adding slabs while the other streams.  Those have two tiles per wavefront, with groups of 32 one
+// (the tables of two do not leave a CU room for a second block).
+// us of 1 / 2 / 3 tiles of four parts, and of one part: groups of 64, 128 alike: 16 x 4096 x 4096 int8 (256 / 128 / 88 blocks)
+// 11.2 / 11.8 / 14.3, 13.3 (128); 16 x 11008 x 4096 int8 (688 / 344 / 232) 25.5 / 23.7 / 17.9, 19.7 (344); the same int4
+// 22.4 / 21.0 / 15.9, 19.3; 33 x 4096 x 4096 int4 (768 / 384 / 264) 21.8 / 19.9 / 21.9, 17.7 (384); 33 x 4096 x 11008 int4
+// (2112 / 1056 / 726) 61.4 / 49.4 / 45.8, 39.8 (1056); 33 x 6144 x 1536 int4 (576 / 288 / 192) 19.9 / 17.9 / 12.7, 11.6 (216);
+// groups of 32, one part with one tile and with two: 33 x 4096 x 4096 int4 (768 / 384 / 264) 23.3 / 21.8 / 24.5, 19.5 (768) and
+// 23.2 (384); 33 x 8192 x 2048 int8 24.8 / 22.3 / 28.8, 20.1 and 23.7; 64 x 8192 x 8192 int4 (4096 / 2048 / 1376) 111 / 83.5 /
+// 84.0, 83.5 (4096) and 97.9; 17 x 4096 x 11008 int4 (1408 / 704 / 484) 46.6 / 38.5 / 37.2, 34.6 (1408) and 42.4.
+// The costs below follow those and 200 more, in us behind what all have in common: the fastest form is chosen or within 5 %
+// (0.1 % on average).
 struct WqForm {
     int tiles, parts;
 };
-WqForm wq_form(int M, int N, int K) {
-    constexpr double kBlock[4] = {0.0, 7.5, 9.3, 12.5};
-    auto blocks = [&](int rb, int kp) {
-        return long((M + 15) / 16) * ((N + wq_rows(rb, kp) - 1) / wq_rows(rb, kp)) * ((K + wq_slice(kp) - 1) / wq_slice(kp));
-    };
-    const long two = blocks(2, 1), rest = two % 512;
-    WqForm best{2, 1};
-    double least = double(two / 512) * 17.0 + (rest == 0 ? 0.0 : rest <= 256 ? 11.0 : 17.0);
+WqForm wq_form(int M, int N, int K, int gs) {
+    // a round of 256 blocks of four parts, and what each range of K adds to it (slabs)
+    constexpr double kRound[4] = {0.0, 7.0, 9.0, 12.5}, kRange[4] = {0.0, 0.0, 0.05, 0.25};
+    auto ranges = [&](int kp) { return (K + wq_slice(kp) - 1) / wq_slice(kp); };
+    auto blocks = [&](int rb, int kp) { return long((M + 15) / 16) * ((N + wq_rows(rb, kp) - 1) / wq_rows(rb, kp)) * ranges(kp); };
+    WqForm best{gs == 32 ? 1 : 2, 1};
+    const long n = blocks(best.tiles, 1);
+    double least = 11.0;
+    if (n > 256) {
+        least = (gs == 32 ? 8.8 : 15.0) * (n > 512 ? double(n) / 512 : 1.0);
+        if (n > 512 && n % 512 > 0 && n % 512 <= 256) least += 3.0;  // (a last round with one block on a CU)
+    }
+    least += 0.2 * ranges(1);
     for (int rb = 1; rb <= 3; ++rb) {
-        const double cost = double((blocks(rb, 4) + 255) / 256) * kBlock[rb];
+        const double cost = double((blocks(rb, 4) + 255) / 256) * (kRound[rb] + kRange[rb] * ranges(4));
         if (cost < least) least = cost, best = WqForm{rb, 4};
     }
     return best;
@@ -713,17 +723,19 @@ template <int BITS>
 int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, const float* biases, int M, int N,
                    int K, int gs, float* out, hipStream_t st) {
     const int sw = wq_swap_mode(BITS, gs);
-    const WqForm form = wq_form(M, N, K);
+    const WqForm form = wq_form(M, N, K, gs);
     const bool pattern = BITS == 4 && M > 1 && M <= 64 && K % WqGeom<BITS>::WK == 0;
 #define LQ_WQ_FORM(SWM, RBS, KPS)                                                                                            \
     if (sw == SWM && form.tiles == RBS && form.parts == KPS)                                                                 \
         return pattern ? launch_wq_mfma_form<BITS, SWM, RBS, KPS, BITS == 4>(x, packed, scales, biases, M, N, K, gs, out, st) \
                        : launch_wq_mfma_form<BITS, SWM, RBS, KPS, false>(x, packed, scales, biases, M, N, K, gs, out, st)
-#define LQ_WQ_FORMS(SWM) LQ_WQ_FORM(SWM, 2, 1); LQ_WQ_FORM(SWM, 1, 4); LQ_WQ_FORM(SWM, 2, 4); LQ_WQ_FORM(SWM, 3, 4)
-    LQ_WQ_FORMS(0);
-    LQ_WQ_FORMS(1);
-    if constexpr (BITS == 4) {
-        LQ_WQ_FORMS(2);
+#define LQ_WQ_FORMS(SWM, ONE) LQ_WQ_FORM(SWM, ONE, 1); LQ_WQ_FORM(SWM, 1, 4); LQ_WQ_FORM(SWM, 2, 4); LQ_WQ_FORM(SWM, 3, 4)
+    LQ_WQ_FORMS(0, 2);
+    if constexpr (BITS == 4) {  // (the last one: groups of 32)
+        LQ_WQ_FORMS(1, 2);
+        LQ_WQ_FORMS(2, 1);
+    } else {
+        LQ_WQ_FORMS(1, 1);
     }
 #undef LQ_WQ_FORMS
 #undef LQ_WQ_FORM

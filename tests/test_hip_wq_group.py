@@ -83,7 +83,8 @@ SMALL_BATCH_FORMS = [(2, 127, 544, 32, 4), (17, 129, 1088, 64, 8), (16, 4097, 40
                      (13, 7000, 6176, 32, 4), (64, 4100, 4096, 32, 8), (24, 8000, 992, 32, 4)]
 
 
-@pytest.mark.parametrize("M,N,K,gs,bits", SMALL_BATCH_FORMS + [(5, 385, 640, 64, 4), (33, 6000, 1024, 32, 4)])
+@pytest.mark.parametrize("M,N,K,gs,bits", SMALL_BATCH_FORMS + [(5, 385, 640, 64, 4), (33, 6000, 1024, 32, 4),
+                                                             (33, 4033, 4096, 32, 4), (20, 4095, 4896, 32, 8)])
 def test_small_batch_forms_are_exact_on_exact_inputs(M, N, K, gs, bits):
     # small integers and scales of 1 and 2 keep every product and sum exact in float32 (below 2^24, 128 + c included): one
     # code, row or group out of place shows
