@@ -80,7 +80,8 @@ bool ks_applies(const GemmArgs& g, int conv) { return g.K > 0 && g.K % 16 == 0 &
 int ks_shape(const GemmArgs& g, int conv, int groups) {
     if (!ks_applies(g, conv)) return 0;
     const long tn = (long(g.N) + 31) / 32 * groups;
-    if (!conv && g.M <= 16) return 25;
+    // (64 columns per tile: a kept range of more than a million columns would need more slots than there are, wider tiles do not)
+    if (!conv && g.M <= 16) return g.range != nullptr && (long(g.N) + 63) / 64 > kRangeSlots ? 0 : 25;
     if ((long(g.M) + 31) / 32 * tn <= 256) return 23;
     return (long(g.M) + 63) / 64 * tn <= 256 && g.K >= 128 ? 24 : 0;
 }

@@ -92,6 +92,20 @@ def test_a_kept_range_follows_tile_config(M, K):
         _ops.qlinear_i8(hip(a), hip(w), **kw, range_buf=rb, tile_config=77)
 
 
+@pytest.mark.parametrize("M,N", [(2, (1 << 20) + 33), (16, 1 << 20)])
+def test_a_kept_range_of_a_million_columns(M, N):
+    """Tiles of 64 columns have a range slot each up to 2^20 columns; what is wider runs on wider tiles."""
+    rng = np.random.default_rng(N)
+    a, w = codes(rng, (M, 16)), codes(rng, (N, 16))
+    rb = L.Tensor.empty((_C.range_buffer_words(),), L.float32, "hip")
+    y = _ops.qlinear_i8(hip(a), hip(w), a_scale=hip(np.float32(0.01)), w_scale=hip(np.full(N, 0.002, np.float32)),
+                        out_mode=_ops.OUT_F32, range_buf=rb).numpy()
+    assert np.array_equal(y, O.igemm(a, w).astype(np.float32) * (np.float32(0.01) * np.float32(0.002)))
+    r = rb.numpy()
+    n, half = int(r[:1].view(np.uint32)[0]), (r.size - 4) // 2
+    assert r[4:4 + n].min() == y.min() and r[4 + half:4 + half + n].max() == y.max()
+
+
 @pytest.mark.parametrize("cfg", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12])
 @pytest.mark.parametrize("M,N,K", [(256, 256, 128), (300, 260, 144), (129, 77, 784), (513, 1000, 576),
                                    (2048, 512, 4096), (1, 16, 16), (700, 130, 64)])
