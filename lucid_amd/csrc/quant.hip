@@ -1090,7 +1090,8 @@ int minmax_launch(const float* x, size_t outer, size_t C, size_t inner, float* m
     }
     LQ_REQUIRE(x, LQ_ERR_VALUE, "minmax: x is NULL");
     LQ_REQUIRE(C <= 0x3fffffffull, LQ_ERR_SHAPE, "minmax: too many channels (%zu)", C);
-    if (C == 1) inner *= outer, outer = 1;  // one run, whatever its shape
+    const bool folded = C == 1 && outer > 1;
+    if (folded) inner *= outer, outer = 1;  // one run, whatever its shape
 
     if (inner < 64 && C > 1) {
         const size_t cols = C * inner;
@@ -1128,7 +1129,13 @@ int minmax_launch(const float* x, size_t outer, size_t C, size_t inner, float* m
     }
 
     // contiguous runs: aim for ~2048 blocks, each with at least 4096 elements; side by side in a run first, then
-    // each with a share of the runs
+    // each with a share of the runs where that pays for the second launch.  That launch takes the host 3.5 us; a block that has a
+    // channel to itself takes 0.2 (lines in its L2) to 0.6 us per round trip.  us of one block per channel / shares, tensors in the
+    // L2, then not: several runs per trip: 6 channels 115 x 93 (6 trips) 5.0 / 8.3, 6 x 512 x 64 (8) 6.2 / 7.8 and 7.8 / 7.3, 6 x 768 x 64
+    // (12) 9.5 / 8.3 and 10.4 / 7.4; 300 channels 1024 x 64 (16) 17.0 / 17.3, 1536 x 64 (24) 23.9 / 22.6; 480 and more have the
+    // memory busy by themselves: 655 x 443 x 64 13.6 / 15.7, 480 x 640 x 200 41 / 45.  Runs of more than 512, one after the other: 16
+    // channels 3 x 2801 (9) 6.4 / 8.4, 20 channels 6 x 1500 (12) 7.4 / 7.8 and 8.7 / 8.2, 8 x 1500 (16) 9.5 / 8.7, 1000 channels
+    // 6 x 1500 11.4 / 12.0.  One channel of 32768 in many runs 5.1 / 8.0 and 9.6 / 7.5, 65536 6.9 / 8.3 and 17.6 / 7.5.
     size_t run_splits = 1, splits = 1;
     if (C < 2048) {
         const size_t want = 2048 / C;
@@ -1138,6 +1145,22 @@ int minmax_launch(const float* x, size_t outer, size_t C, size_t inner, float* m
         if (parts > most) parts = most;
         if (parts > outer) parts = outer;
         if (parts < 1) parts = 1;
+        if (run_splits == 1) {
+            size_t trips = 0, few = 0;  // of a block alone; up to how many it stays alone
+            if (inner <= 2 * kThreads) {
+                size_t lanes = 1;
+                while (lanes * 4 < inner) lanes *= 2;
+                const size_t runs = kThreads / lanes;
+                trips = outer / (4 * runs) + (outer % (4 * runs) + runs - 1) / runs;
+                few = C < 250 ? 9 : C < 400 ? 16 : trips;
+            } else {
+                const size_t quads = (inner + 3) / 4;
+                trips = outer * (quads / (4 * kThreads) + (quads % (4 * kThreads) + kThreads - 1) / kThreads);
+                few = 12;
+            }
+            if (trips <= few) parts = 1;
+        }
+        if (folded && inner <= 32768) run_splits = parts = 1;
         splits = run_splits * parts;
     }
     float *pmin = mn, *pmax = mx;

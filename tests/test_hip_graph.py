@@ -183,6 +183,34 @@ def test_partial_ranges_of_a_recorded_call_are_the_graphs_own(outer, channels, i
         _C.call("lq_stream_destroy", s)
 
 
+@pytest.mark.parametrize("outer,channels,inner,alone", [
+    (75, 1, 432, True), (8192, 1, 4, True), (8193, 1, 4, False),               # one channel of 32768 elements and more
+    (115, 6, 93, True), (288, 6, 93, True), (290, 6, 93, False), (131, 215, 64, True),  # runs side by side
+    (512, 300, 93, True), (520, 300, 93, False), (443, 655, 64, True), (450, 480, 300, True),
+    (3, 16, 2801, True), (4, 16, 2801, True), (5, 16, 2801, False), (6, 1000, 1500, True), (7, 1000, 1500, False)])
+def test_min_max_of_few_elements_per_channel_takes_one_launch(outer, channels, inner, alone):
+    """Where one block per channel is no slower than its shares and a second launch it needs no partial results: a recorded
+    call then takes no memory.  Values on both sides of each line."""
+    _C.init()
+    rng = np.random.default_rng(outer)
+    data = rng.standard_normal((outer, channels, inner)).astype(np.float32)
+    x, (mn, mx) = L.tensor(data, device="hip"), [L.Tensor.empty((channels,), L.float32, "hip") for _ in range(2)]
+    stream, gid = C.c_void_p(), C.c_int()
+    _C.call("lq_stream_create", C.byref(stream))
+    _C.call("lq_sync", None)
+    used = _stats()[0]
+    _C.call("lq_graph_begin", stream, C.byref(gid))
+    _C.call("lq_minmax", x.data_ptr, outer, channels, inner, mn.data_ptr, mx.data_ptr, stream)
+    _C.call("lq_graph_end", stream, gid.value)
+    assert (_stats()[0] == used) == alone
+    for _ in range(2):
+        _C.call("lq_graph_launch", gid.value, stream)
+        _C.call("lq_sync", stream)
+        assert np.array_equal(mn.numpy(), data.min(axis=(0, 2))) and np.array_equal(mx.numpy(), data.max(axis=(0, 2)))
+    _C.call("lq_graph_destroy", gid.value)
+    _C.call("lq_stream_destroy", stream)
+
+
 @pytest.mark.parametrize("recorder", ["graph", "hip"])
 def test_arrival_counters_of_a_first_call_that_is_recorded(recorder):
     """A product that splits K is recorded before its stream was ever used: the clear of the arrival counters is part of
