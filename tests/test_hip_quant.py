@@ -441,6 +441,21 @@ def test_quantize_rows_dynamic_of_ragged_rows(rows, cols, scheme):
     assert np.array_equal(q.numpy()[ok], wq.numpy()[ok])
 
 
+@pytest.mark.parametrize("rows,cols,one", [(99_999, 31, True), (100_000, 31, False), (100_000, 32, True), (100_000, 33, True),
+                                           (120_001, 3, False), (100_000, 4, True)])
+def test_many_short_ragged_rows_take_the_three_calls(rows, cols, one, monkeypatch):
+    """A block per row is slower than the three calls there; the same values either way."""
+    from lucid_amd import _C
+    x = (np.random.default_rng(cols).standard_normal((rows, cols)) * 3).astype(np.float32)
+    xt, names, call = hip(x), [], _C.call
+    monkeypatch.setattr(_C, "call", lambda name, *a: (names.append(name), call(name, *a))[1])
+    q, s, z = Q.quantize_rows_dynamic(xt, Q.per_channel_affine, Q.qint8)
+    assert any("rows_dynamic" in n for n in names) == one
+    ws, wz = O.calc_qparams(x.min(1), x.max(1), False, -128, 127, True)
+    assert same_f32(s.numpy(), ws) and same_f32(z.numpy(), wz)
+    assert np.array_equal(q.numpy(), O.quantize(x, ws, wz, -128, 127, ch_axis=0))
+
+
 def test_quantize_rows_dynamic_at_odd_addresses_writes_its_rows_only():
     from lucid_amd import _C
     rows, cols = 3, 1030
