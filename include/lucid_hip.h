@@ -615,7 +615,10 @@ int lq_conv2d_f32(const float* x, const float* w, const float* bias, float* out,
 /* out[M,N] = a[M,K] . w[N,K]^T + bias[N] in float32 (IBackend::linear, CpuBackend.h:4525);
  * bias may be null.  Products are formed from three-way bfloat16 splits of both operands
  * (six part products, float32 accumulation): 2^-24 relative accuracy per product, as a
- * float32 multiply-add, at the rate of the bfloat16 matrix instruction. */
+ * float32 multiply-add, at the rate of the bfloat16 matrix instruction.  The order in which a row's products are
+ * added depends on the size and the alignment (tiles of 32 x 32 up to 2600 of them, of 128 x 128 beyond; 2000 where
+ * K % 4 != 0, 1500 where a or w is not 16-byte aligned): the same row can differ by roundings between a batch on one
+ * side of that line and one on the other. */
 int lq_sgemm_nt_f32(const float* a, const float* w, const float* bias, float* out, int M, int N, int K,
                     lq_stream stream);
 

@@ -641,10 +641,13 @@ __global__ __launch_bounds__(256, BLOCKS) void sgemm_nt_kernel(const float* __re
 // tile is a chain of K / 32 turns of 2.2 us (split, barrier, LDS reads, MFMAs, barrier) however few of them there are:
 // patches of ViT-B/16, K = N = 768, us: 196 rows 55 -> 9, 784 55 -> 17, 1568 61 -> 27, 3136 62 -> 52.  Beyond
 // SG_SMALL_BLOCKS blocks the larger tiles win, whose operands are split less often (4704 rows 69 against 58, 2048 x 2048 x 512
-// 52 against 42).  Root mean square of the error against float64 6.4e-8 of the result's (1.6e-7 for the large tiles, whose
+// 52 against 42).  Operands that are no whole, aligned 16 bytes are read float by float, more often here: us of small / large tiles,
+// 2592 tiles 2301 x 1147 x 1155 139 / 108, 2304 x 770 82.5 / 77.5, 2025 x 3001 272 / 264, 2000 x 770 75 / 77, 1600 x 1155 94 / 107; at
+// addresses between 16 bytes rows of K = 768 and 3072 are slower still: 1920 x 768 90 / 74, 1600 x 3072 300 / 256, 1536 x 768 70 / 72
+// (K = 1156 as 1155).  Root mean square of the error against float64 6.4e-8 of the result's (1.6e-7 for the large tiles, whose
 // sums are longer).
 constexpr int SG_SMALL = 32;
-constexpr long SG_SMALL_BLOCKS = 2600;
+constexpr long SG_SMALL_BLOCKS = 2600, SG_SMALL_RAGGED = 2000, SG_SMALL_UNALIGNED = 1500;
 
 template <int PATCH, bool VEC>
 __global__ __launch_bounds__(256, 3) void sgemm_nt_small_kernel(const float* __restrict__ a, const float* __restrict__ w,
@@ -745,12 +748,13 @@ __global__ __launch_bounds__(256, 3) void sgemm_nt_small_kernel(const float* __r
     }
 }
 
-// (by M and N alone: a matrix and the image whose patches are its rows get the same sums)
+// (by M, N, K and whether operands are aligned: a matrix and the image whose patches are its rows get the same sums)
 template <int PATCH, bool VEC>
 int launch_sgemm(const float* a, const float* w, const float* bias, float* out, int M, int N, int K, const PatchForm& pf,
                  hipStream_t st, bool large) {
     const long tiles_m = (long(M) + SG_SMALL - 1) / SG_SMALL, tiles_n = (long(N) + SG_SMALL - 1) / SG_SMALL;
-    if (!large && tiles_m * tiles_n <= SG_SMALL_BLOCKS) {
+    const long most = VEC ? SG_SMALL_BLOCKS : K % 4 != 0 ? SG_SMALL_RAGGED : SG_SMALL_UNALIGNED;
+    if (!large && tiles_m * tiles_n <= most) {
         const dim3 grid{unsigned(tiles_n), unsigned(tiles_m)};
         sgemm_nt_small_kernel<PATCH, VEC><<<grid, 256, 0, st>>>(a, w, bias, out, M, N, K, pf);
     } else {

@@ -247,6 +247,18 @@ def test_float_gemm_of_any_size(M, N, K, shift):
     assert (np.abs(out.numpy() - (a64 @ w64.T + bias)) <= bound).all()
 
 
+@pytest.mark.parametrize("M,N,K,shift", [(2300, 1147, 1155, 0), (1990, 1027, 259, 0), (1600, 1152, 256, 1), (2300, 1147, 36, 1)])
+def test_float_gemm_of_unaligned_rows_leaves_the_small_tiles_sooner(M, N, K, shift):
+    """More than 2000 tiles of 32 x 32 (1500 at addresses between 16 bytes): the sums are those of the large tiles, which a
+    problem of more rows takes anyway.  M and N are below the line of aligned rows."""
+    rng = np.random.default_rng(K)
+    a, w = (hip(rng.standard_normal(n + shift).astype(np.float32)) for n in (4000 * K, N * K))
+    outs = [L.Tensor.empty((m, N), L.float32, "hip") for m in (M, 4000)]
+    for o in outs:
+        _C.call("lq_sgemm_nt_f32", a.data_ptr + 4 * shift, w.data_ptr + 4 * shift, None, o.data_ptr, o.shape[0], N, K, None)
+    assert -(-M // 32) * -(-N // 32) <= 2600 and np.array_equal(outs[0].numpy(), outs[1].numpy()[:M])
+
+
 def test_patch_embedding_refuses_a_ragged_image():
     z = L.Tensor.empty((1, 3, 20, 32), L.float32, "hip")
     o = L.Tensor.empty((1, 3, 8), L.float32, "hip")
