@@ -761,7 +761,8 @@ int launch_sgemm(const float* a, const float* w, const float* bias, float* out, 
         const dim3 grid{(unsigned(N) + SG_BN - 1) / SG_BN, (unsigned(M) + SG_BM - 1) / SG_BM};
         const long tiles = long(grid.x) * grid.y;
         // three blocks per CU (168 registers, up to 4 % slower) where they are one round and two per CU are a second, nearly
-        // empty one: 12 544 rows of ViT-B/16's patches, 588 tiles, 134 -> 106 us; 441 tiles 78 with two, 82 with three
+        // empty one: 12 544 rows of ViT-B/16's patches, 588 tiles, 134 -> 106 us; 441 tiles 78 with two, 82 with three.  (Float by float
+        // too, where two to six registers go to scratch: 588 tiles with K = 770 165 us, with two 175; 520 x 333 73 and 79.)
         if (tiles > 512 && tiles <= 768)
             sgemm_nt_kernel<PATCH, VEC, 3><<<grid, 256, 0, st>>>(a, w, bias, out, M, N, K, pf);
         else

@@ -230,7 +230,8 @@ def test_patch_embedding_of_an_image_that_is_not_16_byte_aligned():
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 33, 4), (31, 32, 31), (32, 31, 32), (33, 65, 33), (65, 64, 128), (64, 96, 132),
-                                   (200, 40, 97), (1600, 1664, 36), (1632, 1664, 36), (2689, 1152, 40), (4096, 3073, 68)])
+                                   (200, 40, 97), (1600, 1664, 36), (1632, 1664, 36), (2689, 1152, 40), (4096, 3073, 68),
+                                   (2660, 3457, 68), (3000, 3200, 33)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_float_gemm_of_any_size(M, N, K, shift):
     """Both tile sizes (2600 tiles of 32 x 32 are the line; 588 large tiles run three per CU), K of whole and partial turns, rows
@@ -257,6 +258,25 @@ def test_float_gemm_of_unaligned_rows_leaves_the_small_tiles_sooner(M, N, K, shi
     for o in outs:
         _C.call("lq_sgemm_nt_f32", a.data_ptr + 4 * shift, w.data_ptr + 4 * shift, None, o.data_ptr, o.shape[0], N, K, None)
     assert -(-M // 32) * -(-N // 32) <= 2600 and np.array_equal(outs[0].numpy(), outs[1].numpy()[:M])
+
+
+@pytest.mark.parametrize("B,C,H,W,p,D", [(33, 1, 40, 40, 4, 2561), (27, 3, 33, 33, 3, 2560), (34, 1, 60, 60, 6, 2500)])
+def test_patch_embedding_on_tiles_that_run_three_per_cu(B, C, H, W, p, D):
+    """513 to 768 tiles of 128 x 128 (pixels by aligned quads, one by one, and beside an aligned weight): within the roundings
+    of the additions, as for the float GEMM, with one more for the position."""
+    rng = np.random.default_rng(D)
+    n, K = (H // p) * (W // p), C * p * p
+    assert 512 < -(-B * n // 128) * -(-D // 128) <= 768
+    img = rng.standard_normal((B, C, H, W)).astype(np.float32)
+    w, bias, cls, pos = (rng.standard_normal(s).astype(np.float32) for s in ((D, K), (D,), (D,), (n + 1, D)))
+    out = L.tensor(np.full((B, n + 1, D), np.nan, np.float32), device="hip")
+    held = [hip(v) for v in (img, w, bias, cls, pos)]
+    _C.call("lq_patch_embed_f32", *[t.data_ptr for t in held], out.data_ptr, B, C, H, W, p, D, None)
+    rows, got = V.patch_rows(img, p).astype(np.float64), out.numpy()
+    exact = (rows @ w.T.astype(np.float64)).reshape(B, n, D) + bias + pos[1:].astype(np.float64)
+    size = (np.abs(rows) @ np.abs(w).T.astype(np.float64)).reshape(B, n, D) + np.abs(bias) + np.abs(pos[1:])
+    assert (np.abs(got[:, 1:] - exact) <= (6 * ((K + 15) // 16) + 13) * 2.0 ** -24 * size).all()
+    assert np.array_equal(got[:, 0], np.broadcast_to(cls + pos[0], (B, D)))
 
 
 def test_patch_embedding_refuses_a_ragged_image():
