@@ -390,10 +390,10 @@ __global__ __launch_bounds__(64 * wq_waves(KP)) __attribute__((amdgpu_waves_per_
     // Every global load of the block is requested before anything is consumed, in the order of
     // consumption (the wait counter retires loads in order): the scale / bias tables (short, from
     // the L2), x, the weights.
-    // Tables: wq_rows(RB) rows x gcap slots (gcap = the groups of a full k range, 4, 8 or 16), four slots per
+    // Tables: kWqRows rows x gcap slots (gcap = the groups of a full k range of 512 or 1024: 4, 8, 16 or 32), four slots per
     // 16-byte load where the rows allow it (a dword per lane costs the vector cache as many cycles
     // as 16 bytes per lane do).
-    constexpr int kTabVec = (kWqRows * (SLICE / 32) + 4 * THREADS - 1) / 4 / THREADS;  // 16-byte loads per thread and table, at 16 groups per k range
+    constexpr int kTabVec = (kWqRows * (SLICE / 32) + 4 * THREADS - 1) / 4 / THREADS;  // 16-byte loads per thread and table, in groups of 32
     const int gcap = gp - 1, gsh = 31 - __builtin_clz(unsigned(gcap));  // a power of two: shifts, no division
     const bool tab_vec = ng == gcap && (groups_per_row & 3) == 0 && aligned16(scales) && aligned16(biases);
     // (No branch between these requests and none that gives a register another value: the compiler would wait for each load
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(64 * wq_waves(KP)) __attribute__((amdgpu_waves_per_
                 bd[0] = tab_b[u].x, bd[1] = tab_b[u].y, bd[2] = tab_b[u].z, bd[3] = tab_b[u].w;
             }
         }
-    } else {  // the last k range of a K that is not a multiple of 512, or rows that vectors cannot take
+    } else {  // the last k range of a K that is not a multiple of the block's, or rows that vectors cannot take
         for (int i = threadIdx.x; i < kWqRows * gcap; i += THREADS) {
             const int row = i >> gsh, g = i & (gcap - 1);
             // (zeros past the row's groups: a partial window's segments past K read them)
@@ -794,8 +794,8 @@ int lq_wq_matmul(const float* x, const uint32_t* packed, const float* scales, co
     LQ_REQUIRE(x && packed && scales && biases && out, LQ_ERR_VALUE, "wq_matmul: NULL pointer");
     hipStream_t st = as_stream(stream);
     if (aligned16(x) && aligned16(packed)) {
-        // one row is a stream of the weight; more rows go to the matrix cores: 16 rows x 512 k of
-        // wq_rows(1 .. 3) columns per block, or (wq_gemm.hip) tiles over all of K
+        // one row is a stream of the weight; more rows go to the matrix cores: 16 rows x 512 or 1024 k of
+        // wq_rows(tiles, parts) columns per block, or (wq_gemm.hip) tiles over all of K
         if (M == 1 && wq_gemv1_lds(K, bits) <= size_t(kGemv1MaxLds))
             return bits == 4 ? launch_gemv1<4>(x, packed, scales, biases, N, K, group_size, out, st)
                              : launch_gemv1<8>(x, packed, scales, biases, N, K, group_size, out, st);
