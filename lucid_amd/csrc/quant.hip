@@ -358,8 +358,11 @@ int launch_elementwise(Op op, size_t outer, size_t C, size_t inner, QParams qp, 
                                unsigned(n), FastDiv{unsigned(stride)}, by_inner, by_c, qp);
         };
         // Found per quad: channels that come round less than twice, and what has two channels to find and nothing to divide by
-        // (dequantize of 5000 x 3000 x 7 along the middle axis: 92.6 us, shared 96.1).
-        if (quads >= 2 * round && (inner < 4 || Op::kDivides)) {
+        // (dequantize of 5000 x 3000 x 7 along the middle axis: 92.6 us, shared 96.1).  So does a quantization of so few that a CU has
+        // less than three blocks either way: it takes two quads per thread by itself, four would halve the blocks (us, per quad /
+        // shared, replayed from a graph: 300 x 39 x 28 3.1 / 3.5, 1777 x 20 x 2 3.0 / 3.3, 796 x 63 x 10 3.1 / 3.4; 143 x 3027 x 2 and 1215 x
+        // 49 x 15 3.6 and 3.5 either way, 132 x 5645 x 2 4.5 / 4.2).
+        if (quads >= 2 * round && (inner < 4 || Op::kDivides) && (Op::kMaxU >= 4 || quads >= 768 * kThreads)) {
             constexpr int U = 4;
             size_t stride = (kThreads + round - 1) / round * round;
             if (quads < 16 * U * stride) stride = (quads + U * round - 1) / (U * round) * round;

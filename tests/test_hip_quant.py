@@ -317,6 +317,7 @@ def test_ragged_segments_bit_exact(shape, ch_axis):
 @pytest.mark.parametrize("shape", [
     (40001, 3), (20003, 2, 3), (66000, 1, 2), (2001, 3, 13), (7001, 1, 1), (9000, 7), (5, 1031), (4, 515, 3), (3, 700, 2), (7, 100, 9),
     (1, 4001), (1, 300, 7), (2, 33, 5), (70000, 4), (1201, 2, 67),
+    (262145, 3), (262143, 3), (400001, 2), (60001, 2, 7), (13, 1009, 67), (5, 26215, 6), (2, 65543, 7), (800001, 1, 1),  # 768 x 1024 elements and more
 ])
 @pytest.mark.parametrize("qd", ["qint8", "quint8"])
 def test_channels_that_come_round_bit_exact(shape, qd):
