@@ -18,7 +18,10 @@
 // 197 x 768 x 3072 8.7 / 5.6, 60 x 92 x 6624 12.4 / 6.4; 64 x 32 tiles: 784 x 512 x 4608 12.5 / 9.0, 1568 x 256 x 2304
 // 8.7 / 7.0.  Two tiles per CU are slower than four wavefronts on larger ones: 392 x 512 x 1024 in 208 tiles 5.4 / 4.1,
 // 3136 x 128 x 1152 in 392 tiles 7.3 / 7.9.  16-row tiles against the kernel whose wavefronts load fragments straight into registers: 16 x
-// 11008 x 4096 10.9 / 9.5, 16 x 4096 x 4096 7.8 / 5.7, 16 x 1024 x 4096 6.9 / 3.8, 2 x 12000 x 1024 5.6 / 4.9.
+// 11008 x 4096 10.9 / 9.5, 16 x 4096 x 4096 7.8 / 5.7, 16 x 1024 x 4096 6.9 / 3.8, 2 x 12000 x 1024 5.6 / 4.9.  Several rounds of tiles of 64
+// columns, which have one stage each and nothing on its way during the products (other blocks of the CU have): 16 x 14336 x 4096
+// 16.7 / 14.7, 16 x 16384 x 4096 17.1 / 15.7, 16 x 32000 x 4096 32.6 / 29.9 (weights in the last-level cache 25.2 / 20.4), 2 x 32000 x 4096
+// 30.4 / 29.0, 16 x 151936 x 4096 142 / 111, 16 x 65536 x 1024 23.3 / 16.0.
 #pragma once
 #include "qgemm_tile.hpp"
 
