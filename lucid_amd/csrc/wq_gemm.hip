@@ -45,20 +45,42 @@ constexpr int kPiece = 1024;  // bytes one wavefront moves into LDS with one ins
 // One launch, two kinds of blocks.  The first `split_blocks`: one thread = eight consecutive k of one
 // row; a block = 16 rows x two stages.  The others: 32 groups of 64 columns, read row by row and turned in LDS.
 // 333 x 11008 x 4096 int4 of 128 10.4 -> 8.8 us, 100 x 11008 x 4096 of 32 21.0 -> 11.5: a thread that took four groups of a column for itself
-// read 16 bytes of a line that the blocks of the next groups, on other XCDs, fetched again.
-constexpr int kSbGroups = 32, kSbColumns = 64;
+// read 16 bytes of a line that the blocks of the next groups, on other XCDs, fetched again.  Few groups are not worth the turn, a row is
+// a line or two: there a thread takes up to four consecutive groups of a column as before (the whole call, turned / not: 88 x 10080 x
+// 640 int4 of 128 15.0 / 13.7, 198 x 5378 x 384 of 32 14.9 / 13.6, 351 x 4212 x 512 of 32 17.8 / 17.1; equal at 24 groups).
+constexpr int kSbGroups = 32, kSbColumns = 64, kSbFew = 24;
 template <int BITS>
 __global__ __launch_bounds__(256) void wq_prepare_kernel(const float* __restrict__ x, const float* __restrict__ scales,
                                                          const float* __restrict__ biases, int M, int N, int K,
                                                          int gs_shift, int mtiles, int bm, int n_pad, int stages,
                                                          int segs, unsigned split_blocks, uint4* __restrict__ parts,
                                                          float* __restrict__ xsum, float2* __restrict__ sb) {
+    if (blockIdx.x >= split_blocks && stages * segs < kSbFew * (segs == 2 ? 1 : (1 << gs_shift) / 64)) {
+        const int groups = K >> gs_shift;
+        const int per = segs == 2 ? 1 : (1 << gs_shift) / 64;  // segments per group
+        const unsigned idx = (blockIdx.x - split_blocks) * 256 + threadIdx.x;
+        const unsigned quad = idx / unsigned(n_pad), n = idx - quad * unsigned(n_pad);
+        const int g0 = int(quad) * 4;
+        float s[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
+        if (n < unsigned(N)) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (g0 + e < groups) s[e] = scales[size_t(n) * groups + g0 + e], b[e] = biases[size_t(n) * groups + g0 + e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            for (int r = 0; r < per; ++r)
+                if ((g0 + e) * per + r < stages * segs)
+                    sb[size_t((g0 + e) * per + r) * n_pad + n] = float2{kWqUnit<BITS> * s[e], b[e] - float(kWqCentre<BITS>) * s[e]};
+        return;
+    }
     if (blockIdx.x >= split_blocks) {
         __shared__ float2 tile[kSbGroups][kSbColumns + 1];
         const int groups = K >> gs_shift;
         const int per = segs == 2 ? 1 : (1 << gs_shift) / 64;  // segments per group
         const unsigned idx = blockIdx.x - split_blocks, across = unsigned(n_pad) / kSbColumns;
         const int n0 = int(idx % across) * kSbColumns, first = int(idx / across) * kSbGroups;
+        const int all = stages * segs / per, here = all - first < kSbGroups ? all - first : kSbGroups;  // groups, past K too
         // four groups per lane, and of a row's 32 side by side; the last four of a row where those asked for run past it
         float4 sv[2], bv[2];
 #pragma unroll
@@ -84,15 +106,15 @@ __global__ __launch_bounds__(256) void wq_prepare_kernel(const float* __restrict
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int g = groups < 4 ? (e < groups ? first + e : first + kSbGroups) : at + e, slot = g - first;
-                if (column && slot >= q0 && slot < q0 + 4 && (groups >= 4 || q0 == 0))
+                if (column && slot >= q0 && slot < q0 + 4 && slot < here && (groups >= 4 || q0 == 0))
                     tile[slot][c] = float2{kWqUnit<BITS> * s4[e], b4[e] - float(kWqCentre<BITS>) * s4[e]};
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (!column || g0 + e >= groups) tile[q0 + e][c] = float2{0.f, 0.f};
+                if (q0 + e < here && (!column || g0 + e >= groups)) tile[q0 + e][c] = float2{0.f, 0.f};
         }
         __syncthreads();
-        for (int i = threadIdx.x; i < kSbGroups * kSbColumns; i += 256) {
+        for (int i = threadIdx.x; i < here * kSbColumns; i += 256) {
             const int g = i / kSbColumns, c = i % kSbColumns;
             const float2 v = tile[g][c];
             for (int r = 0; r < per; ++r)
@@ -383,7 +405,8 @@ int launch_rows(const float* x, const uint32_t* packed, const float* scales, con
     // (groups of the stages, past K too)
     const int sb_groups = SEGS == 2 ? stages * 2 : stages / (GS / 64);
     static_assert(bn % kSbColumns == 0, "");
-    const unsigned sb_blocks = unsigned((sb_groups + kSbGroups - 1) / kSbGroups) * unsigned(n_pad / kSbColumns);
+    const unsigned sb_blocks = sb_groups < kSbFew ? unsigned((size_t((sb_groups + 3) / 4) * n_pad + 255) / 256)
+                                                  : unsigned((sb_groups + kSbGroups - 1) / kSbGroups) * unsigned(n_pad / kSbColumns);
     hipLaunchKernelGGL((wq_prepare_kernel<BITS>), dim3(split_blocks + sb_blocks), dim3(256), 0, st, x, scales, biases, M, N,
                        K, gs_shift, mtiles, bm, n_pad, stages, SEGS, split_blocks, reinterpret_cast<uint4*>(parts),
                        reinterpret_cast<float*>(xsum), reinterpret_cast<float2*>(sb));

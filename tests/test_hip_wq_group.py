@@ -106,6 +106,13 @@ def test_ranges_in_four_parts_are_exact_on_exact_inputs(M, N, K, gs, bits):
     test_small_batch_forms_are_exact_on_exact_inputs(M, N, K, gs, bits)
 
 
+# the large-batch kernel's table of scales: few groups (a thread per column), as many as are turned in LDS, one more, one less
+@pytest.mark.parametrize("M,N,K,gs,bits", [(80, 6161, 736, 32, 4), (80, 6161, 768, 32, 4), (80, 6161, 800, 32, 8), (70, 7003, 1472, 64, 4),
+                                           (70, 7003, 1536, 64, 8), (300, 2049, 2816, 128, 4), (300, 2049, 3072, 128, 8), (90, 9000, 32, 32, 4)])
+def test_large_batch_scales_of_few_groups_are_exact_on_exact_inputs(M, N, K, gs, bits):
+    test_large_batch_matmul_is_exact_on_exact_inputs(M, N, K, gs, bits)
+
+
 @pytest.mark.parametrize("M,N,K,gs,bits", SMALL_BATCH_FORMS)
 def test_small_batch_forms_against_float64(M, N, K, gs, bits):
     rng = np.random.default_rng(N)
