@@ -508,11 +508,16 @@ __global__ __launch_bounds__(64 * wq_waves(KP)) __attribute__((amdgpu_waves_per_
     }
     lds_barrier();  // (the weights are still on their way)
 
-    v4f y[RB];
+    // (one part of one tile, which has all its windows at once: four sums, a quarter as long; error of 51 x 92 x 3072 int8 against
+    // float64 1.33e-7 of the result with one sum, 1.25e-7 in four parts, 1.24e-7 so.  128 + c have more to round than that: one sum.)
+    constexpr int SUMS = KP == 1 && RB == 1 && !PATTERN ? 4 : 1;
+    v4f ys[SUMS][RB];
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) y[rb] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < SUMS; ++i)
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) ys[i][rb] = v4f{0.f, 0.f, 0.f, 0.f};
     const int row_in_tile = wc * (RB * 16) + r;
-    auto window = [&](int wi, const uint4 (&wv)[RB]) {
+    auto window = [&](int wi, const uint4 (&wv)[RB], v4f (&y)[RB]) {
         uint32_t wd[RB][4];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
@@ -573,9 +578,11 @@ __global__ __launch_bounds__(64 * wq_waves(KP)) __attribute__((amdgpu_waves_per_
     for (int w = w_first; w < w_end; w += AHEAD)
 #pragma unroll
         for (int j = 0; j < AHEAD; ++j) {
-            if (w + j < w_end) window(w + j, ahead[j]);
+            if (w + j < w_end) window(w + j, ahead[j], ys[j % SUMS]);
             if (AHEAD < WPW) fetch(ahead[j], w + j + AHEAD);
         }
+    v4f(&y)[RB] = ys[0];
+    if constexpr (SUMS == 4) y[0] = (ys[0][0] + ys[1][0]) + (ys[2][0] + ys[3][0]);
     if constexpr (KP > 1) {  // the parts of the range meet where x was
         v4f* const parts = reinterpret_cast<v4f*>(wq_lds) + lane;
         lds_barrier();
@@ -661,37 +668,47 @@ __global__ __launch_bounds__(64 * wq_waves(KP)) __attribute__((amdgpu_waves_per_
 
 // Tiles of 16 weight rows per wavefront and parts of a block's k range.  Four parts of 1024 k (a CU per block) with as many
 // tiles as give every block a CU at once; where the blocks are too many for that, one part of 512 k, of which a CU
-// has two blocks, one starting or adding slabs while the other streams.  Those have two tiles per wavefront, with groups of 32 one
-// (the tables of two do not leave a CU room for a second block).
-// us of 1 / 2 / 3 tiles of four parts, and of one part: groups of 64, 128 alike: 16 x 4096 x 4096 int8 (256 / 128 / 88 blocks)
-// 11.2 / 11.8 / 14.3, 13.3 (128); 16 x 11008 x 4096 int8 (688 / 344 / 232) 25.5 / 23.7 / 17.9, 19.7 (344); the same int4
-// 22.4 / 21.0 / 15.9, 19.3; 33 x 4096 x 4096 int4 (768 / 384 / 264) 21.8 / 19.9 / 21.9, 17.7 (384); 33 x 4096 x 11008 int4
-// (2112 / 1056 / 726) 61.4 / 49.4 / 45.8, 39.8 (1056); 33 x 6144 x 1536 int4 (576 / 288 / 192) 19.9 / 17.9 / 12.7, 11.6 (216);
-// groups of 32, one part with one tile and with two: 33 x 4096 x 4096 int4 (768 / 384 / 264) 23.3 / 21.8 / 24.5, 19.5 (768) and
-// 23.2 (384); 33 x 8192 x 2048 int8 24.8 / 22.3 / 28.8, 20.1 and 23.7; 64 x 8192 x 8192 int4 (4096 / 2048 / 1376) 111 / 83.5 /
-// 84.0, 83.5 (4096) and 97.9; 17 x 4096 x 11008 int4 (1408 / 704 / 484) 46.6 / 38.5 / 37.2, 34.6 (1408) and 42.4.
-// The costs below follow those and 200 more, in us behind what all have in common: the fastest form is chosen or within 5 %
-// (0.1 % on average).
+// has two blocks, one starting or adding slabs while the other streams: with two tiles per wavefront, in groups of 32 one (the tables of
+// two do not leave a CU room for a second block).  One part of one tile is also the better one where K is no multiple of 1024 and
+// half of the second range would be empty, and where K is short.
+// us of 1 / 2 / 3 tiles of four parts, then of one part of one and of two: groups of 64, 128 alike: 16 x 11008 x 4096 int8 (688 / 344 / 232
+// blocks) 25.5 / 23.7 / 17.9, - / 19.7 (344); the same int4 22.4 / 21.0 / 15.9, - / 19.3; 33 x 4096 x 4096 int4 (768 / 384 / 264) 21.8 / 19.9 / 21.9,
+// - / 17.7 (384); 33 x 4096 x 11008 int4 (2112 / 1056 / 726) 61.4 / 49.4 / 45.8, - / 39.8 (1056); 38 x 2767 x 1536 int4 (264 / 132 / 90) 14.2 / 9.9 /
+// 12.1, 8.7 (198) / 10.9; 31 x 10765 x 320 int8 (338 / 170 / 114) 9.5 / 7.1 / 8.4, 6.0 (170) / 7.5; 4 x 3092 x 3904 int8 (196 / 100 / 68) 9.4 / 11.5 /
+// 14.2, 10.0 (200) / 12.8; 51 x 92 x 3072 int8 (24 / 12 / 12) 8.5 / 10.7 / 13.1, 8.0 (24) / 10.9;
+// groups of 32: 33 x 4096 x 4096 int4 (768 / 384 / 264) 23.3 / 21.8 / 24.5, 19.5 (768) / 23.2 (384); 33 x 8192 x 2048 int8 24.8 / 22.3 / 28.8, 20.1
+// / 23.7; 64 x 8192 x 8192 int4 (4096 / 2048 / 1376) 111 / 83.5 / 84.0, 83.5 (4096) / 97.9; 33 x 3529 x 1280 int8 (336 / 168 / 114) 16.0 / 11.6 / 15.5,
+// 9.3 (252) / 12.7; 62 x 3817 x 3360 int4 34.1 / 27.1 / 34.5, 28.5 / 33.8.
+// The costs below follow 1850 shapes timed in every form (2 to 64 rows, and more where this kernel takes them; 64 to 16384 columns, K
+// from 32 to 12288), in us behind what all have in common: what they choose is the fastest or within 3 % but for 49 shapes, 0.3 % off
+// on average and 13 % at most.
 struct WqForm {
     int tiles, parts;
 };
 WqForm wq_form(int M, int N, int K, int gs) {
-    // a round of 256 blocks of four parts, and what each range of K adds to it (slabs)
-    constexpr double kRound[4] = {0.0, 7.0, 9.0, 12.5}, kRange[4] = {0.0, 0.0, 0.05, 0.25};
     auto ranges = [&](int kp) { return (K + wq_slice(kp) - 1) / wq_slice(kp); };
     auto blocks = [&](int rb, int kp) { return long((M + 15) / 16) * ((N + wq_rows(rb, kp) - 1) / wq_rows(rb, kp)) * ranges(kp); };
-    WqForm best{gs == 32 ? 1 : 2, 1};
-    const long n = blocks(best.tiles, 1);
-    double least = 11.0;
-    if (n > 256) {
-        least = (gs == 32 ? 8.8 : 15.0) * (n > 512 ? double(n) / 512 : 1.0);
-        if (n > 512 && n % 512 > 0 && n % 512 <= 256) least += 3.0;  // (a last round with one block on a CU)
-    }
-    least += 0.2 * ranges(1);
-    for (int rb = 1; rb <= 3; ++rb) {
-        const double cost = double((blocks(rb, 4) + 255) / 256) * (kRound[rb] + kRange[rb] * ranges(4));
-        if (cost < least) least = cost, best = WqForm{rb, 4};
-    }
+    // handing slabs on: the last block fetches eight at a time
+    auto slabs = [&](int kp) { return ranges(kp) == 1 ? 0.0 : 1.5 + 1.5 * ((ranges(kp) + 7) / 8); };
+    WqForm best{1, 4};
+    double least = 1e30;
+    auto take = [&](int rb, int kp, double cost) {
+        if (cost < least) least = cost, best = WqForm{rb, kp};
+    };
+    // one part: alone on a CU, or two blocks at once, of which the last round of 512 may leave one
+    const double short1 = 0.35 + 0.65 * (K < 512 ? K : 512) / 512;
+    auto one_part = [&](int rb, double alone, double round) {
+        const long n = blocks(rb, 1);
+        const double last = n > 512 && n % 512 > 0 && n % 512 <= 256 ? 2.4 : 0.0;
+        take(rb, 1, (n <= 256 ? alone : round * (n > 512 ? double(n) / 512 : 1.0) + last) * short1 + slabs(1));
+    };
+    one_part(1, gs == 32 ? 6.8 : 6.3, gs == 32 ? 9.3 : 10.1);
+    if (gs > 32) one_part(2, ranges(1) == 1 ? 9.5 : 11.0, 15.3);
+    // four parts: rounds of 256 blocks, and what each range of K adds to one
+    constexpr double kRound[4] = {0.0, 6.3, 9.0, 11.8}, kRange[4] = {0.0, 0.08, 0.06, 0.2};
+    const double short4 = 0.62 + 0.38 * (K < 1024 ? K : 1024) / 1024;
+    for (int rb = 1; rb <= 3; ++rb)
+        take(rb, 4, double((blocks(rb, 4) + 255) / 256) * (kRound[rb] * short4 + kRange[rb] * ranges(4)) + slabs(4));
     return best;
 }
 
@@ -729,13 +746,13 @@ int launch_wq_mfma(const float* x, const uint32_t* packed, const float* scales, 
     if (sw == SWM && form.tiles == RBS && form.parts == KPS)                                                                 \
         return pattern ? launch_wq_mfma_form<BITS, SWM, RBS, KPS, BITS == 4>(x, packed, scales, biases, M, N, K, gs, out, st) \
                        : launch_wq_mfma_form<BITS, SWM, RBS, KPS, false>(x, packed, scales, biases, M, N, K, gs, out, st)
-#define LQ_WQ_FORMS(SWM, ONE) LQ_WQ_FORM(SWM, ONE, 1); LQ_WQ_FORM(SWM, 1, 4); LQ_WQ_FORM(SWM, 2, 4); LQ_WQ_FORM(SWM, 3, 4)
-    LQ_WQ_FORMS(0, 2);
-    if constexpr (BITS == 4) {  // (the last one: groups of 32)
-        LQ_WQ_FORMS(1, 2);
-        LQ_WQ_FORMS(2, 1);
-    } else {
-        LQ_WQ_FORMS(1, 1);
+#define LQ_WQ_FORMS(SWM) LQ_WQ_FORM(SWM, 1, 1); LQ_WQ_FORM(SWM, 1, 4); LQ_WQ_FORM(SWM, 2, 4); LQ_WQ_FORM(SWM, 3, 4)
+    LQ_WQ_FORMS(0);
+    LQ_WQ_FORM(0, 2, 1);
+    LQ_WQ_FORMS(1);
+    if constexpr (BITS == 4) {  // (the last swap mode of either width: groups of 32)
+        LQ_WQ_FORM(1, 2, 1);
+        LQ_WQ_FORMS(2);
     }
 #undef LQ_WQ_FORMS
 #undef LQ_WQ_FORM

@@ -106,6 +106,18 @@ def test_ranges_in_four_parts_are_exact_on_exact_inputs(M, N, K, gs, bits):
     test_small_batch_forms_are_exact_on_exact_inputs(M, N, K, gs, bits)
 
 
+# one and two tiles of one part, one to three of four: for each exchange of registers and with whole windows and a partial one, beyond
+# what the shapes above take
+@pytest.mark.parametrize("M,N,K,gs,bits", [
+    (2, 63, 1792, 32, 4), (2, 11532, 1056, 32, 4), (2, 7194, 4128, 32, 4), (2, 7724, 4224, 32, 4), (3, 99, 1088, 64, 4),
+    (4, 53, 1536, 64, 4), (2, 10185, 4288, 64, 4), (2, 9921, 4352, 64, 4), (2, 105, 704, 64, 4), (2, 11146, 1088, 64, 4),
+    (2, 10990, 1152, 64, 4), (2, 11185, 2624, 64, 4), (2, 9516, 3200, 64, 4), (2, 9929, 4224, 128, 4), (2, 150, 512, 128, 4),
+    (2, 11401, 2688, 128, 4), (2, 52, 1536, 32, 8), (2, 11095, 1088, 32, 8), (2, 10017, 4224, 64, 8), (3, 63, 640, 64, 8),
+    (2, 11140, 1088, 64, 8), (38, 2767, 1536, 64, 4)])
+def test_every_small_batch_form_is_exact_on_exact_inputs(M, N, K, gs, bits):
+    test_small_batch_forms_are_exact_on_exact_inputs(M, N, K, gs, bits)
+
+
 # the large-batch kernel's table of scales: few groups (a thread per column), as many as are turned in LDS, one more, one less
 @pytest.mark.parametrize("M,N,K,gs,bits", [(80, 6161, 736, 32, 4), (80, 6161, 768, 32, 4), (80, 6161, 800, 32, 8), (70, 7003, 1472, 64, 4),
                                            (70, 7003, 1536, 64, 8), (300, 2049, 2816, 128, 4), (300, 2049, 3072, 128, 8), (90, 9000, 32, 32, 4)])
